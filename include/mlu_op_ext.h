@@ -84,6 +84,16 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtSetSparseConvExtendedModes(mluOpHandle_t han
  * all but one of such pairs.  Off by default. */
 mluOpStatus_t MLUOP_WIN_API mluOpExtSetDistinctPairsPromise(mluOpHandle_t handle, int promised);
 
+/* The pair counts of a rulebook on the host.  The convolution operators take indice_num as a host
+ * array, so a caller has to bring the counts mluOpGetIndicePairs left in device memory over; a copy
+ * waits for the whole queue.  The last kernel of a rulebook also stores them into pinned memory of
+ * the handle: this call waits for them there and fills indice_num[0 .. kernel_volume).  For the last
+ * 32 rulebooks of the handle; NOT_SUPPORTED for a pair tensor it did not build, that was built under
+ * graph capture or has more than 343 offsets (copy the counts then).  No counterpart in the
+ * reference. */
+mluOpStatus_t MLUOP_WIN_API mluOpExtGetIndicePairsHostCounts(mluOpHandle_t handle, const void *indice_pairs,
+                                                             int kernel_volume, int64_t indice_num[]);
+
 /* Row maps kept across calls.  mluOpIndiceConvolutionForward and ...BackwardData turn the pair
  * lists into a [K, rows] map (partner row of every result row at every offset, or -1) on every
  * call: the reference API (mlu_op.h:10321-10448, :9625-9773) hands them nothing else to keep.

@@ -66,7 +66,10 @@ mluOpStatus_t MLUOP_WIN_API mluOpCreate(mluOpHandle_t *handle) {
   ctx->cu_count = prop.multiProcessorCount;
   ctx->lds_bytes = (int)prop.sharedMemPerBlock;
   void *pinned = nullptr;
-  const size_t pinned_bytes = 64 + sizeof(mluOpContext::RulebookReport) * mluOpContext::kRulebookNotes;
+  const size_t reports_bytes = sizeof(unsigned long long) * mluOpContext::kRulebookNotes;
+  const size_t readback_bytes = sizeof(unsigned long long) * mluOpContext::kReadbackWords;
+  const size_t pinned_bytes = 64 + reports_bytes + readback_bytes +
+                              sizeof(unsigned long long) * mluOpContext::kRulebookNotes * mluOpContext::kCountWords;
   err = hipHostMalloc(&pinned, pinned_bytes, hipHostMallocDefault);
   if (err != hipSuccess) {
     MLUOP_LOG(ERROR) << "[mluOpCreate] hipHostMalloc failed: " << hipGetErrorString(err);
@@ -75,15 +78,10 @@ mluOpStatus_t MLUOP_WIN_API mluOpCreate(mluOpHandle_t *handle) {
   }
   ctx->pinned_scalar = static_cast<int32_t *>(pinned);
   memset(pinned, 0, pinned_bytes);
-  err = hipEventCreateWithFlags(&ctx->readback_event, hipEventDisableTiming | hipEventReleaseToSystem);
-  if (err != hipSuccess) {
-    MLUOP_LOG(ERROR) << "[mluOpCreate] hipEventCreateWithFlags failed: " << hipGetErrorString(err);
-    (void)hipHostFree(pinned);
-    delete ctx;
-    return MLUOP_STATUS_INTERNAL_ERROR;
-  }
-  ctx->rulebook_reports =
-      reinterpret_cast<mluOpContext::RulebookReport *>(static_cast<char *>(pinned) + 64);
+  char *behind = static_cast<char *>(pinned) + 64;
+  ctx->rulebook_reports = reinterpret_cast<unsigned long long *>(behind);
+  ctx->readback_words = reinterpret_cast<unsigned long long *>(behind + reports_bytes);
+  ctx->count_words = reinterpret_cast<unsigned long long *>(behind + reports_bytes + readback_bytes);
   // Stamps and tickets only have to differ from what earlier calls, of this handle or of
   // another, left in memory: start somewhere no other handle starts.
   ctx->next_stamp = ((unsigned long long)std::chrono::steady_clock::now().time_since_epoch().count()
@@ -113,7 +111,6 @@ mluOpStatus_t MLUOP_WIN_API mluOpDestroy(mluOpHandle_t handle) {
       (void)hipGetLastError();
   }
   if (handle->pinned_scalar != nullptr) (void)hipHostFree(handle->pinned_scalar);
-  if (handle->readback_event != nullptr) (void)hipEventDestroy(handle->readback_event);
   handle->timer.destroy();
   delete handle;
   return MLUOP_STATUS_SUCCESS;
@@ -262,6 +259,35 @@ const char *MLUOP_WIN_API mluOpGetErrorString(mluOpStatus_t status) {
 }  // extern "C"
 
 namespace mluop {
+
+hipError_t waitForWord(hipStream_t queue, const unsigned long long *word, unsigned long long stamp,
+                       int32_t *value) {
+  using Clock = std::chrono::steady_clock;
+  auto arrived = [&] {
+    const unsigned long long w = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+    if ((w >> 32) != (stamp & 0xffffffffull)) return false;
+    *value = (int32_t)(uint32_t)w;
+    return true;
+  };
+  Clock::time_point look_again{};
+  for (unsigned long long spins = 0;; ++spins) {
+    if (arrived()) return hipSuccess;
+    __builtin_ia32_pause();
+    if (spins % 4096 != 4095) continue;
+    // every millisecond: is the queue still at work at all?
+    const Clock::time_point now = Clock::now();
+    if (look_again == Clock::time_point{}) look_again = now + std::chrono::milliseconds(1);
+    if (now < look_again) continue;
+    look_again = now + std::chrono::milliseconds(1);
+    const hipError_t err = hipStreamQuery(queue);
+    if (err == hipErrorNotReady) {
+      (void)hipGetLastError();
+      continue;
+    }
+    if (err != hipSuccess) return err;
+    return arrived() ? hipSuccess : hipErrorUnknown;
+  }
+}
 
 bool logEnabled() {
   static const bool enabled = [] {

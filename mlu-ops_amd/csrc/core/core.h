@@ -33,7 +33,8 @@ struct mluOpContext {
   mluOpQuantizeRoundMode_t round_mode = MLUOP_ROUND_HALF_TO_EVEN;
   mluOpAtomicsMode_t atomics_mode = MLUOP_ATOMICS_NOT_ALLOWED;
   int32_t *pinned_scalar = nullptr;  // 64-byte pinned host slot for read-backs
-  hipEvent_t readback_event = nullptr;  // recorded behind a kernel that stores into the slot
+  // What kernels leave for the host while they run (pinned): stamped words, see waitForWord.
+  unsigned long long *readback_words = nullptr;
   mluop::KernelTimer timer;          // per-kernel event timing, off by default
   // Modes the reference rejects (inverse convolution, filters_grad written in its
   // tagged layout): off unless mluOpExtSetSparseConvExtendedModes switched them on.
@@ -57,19 +58,20 @@ struct mluOpContext {
   // convolution operators read the slot, without waiting for anything, to choose their way
   // through the pair lists.  A note is a hint about speed only: what the kernels rely on is
   // checked on the device in every call.
-  struct RulebookReport {       // pinned host memory, written by the device
-    unsigned long long stamp;   // the note's stamp, stored after the flag
-    unsigned int rows_in_order;
-    unsigned int unused;
-  };
   struct RulebookNote {
     const void *pairs = nullptr;
     int K = 0, L = 0;
     unsigned long long stamp = 0;
+    bool counts_on_file = false;  // its last kernel stores the pair counts into count_words
   };
   static constexpr int kRulebookNotes = 32;
+  // Pair counts of a rulebook reach the host through stamped words, kCountWords a note
+  // (kernels of up to 7 x 7 x 7; larger ones are copied).
+  static constexpr int kCountWords = 343;
+  static constexpr int kReadbackWords = 8;
   RulebookNote rulebook_notes[kRulebookNotes];
-  RulebookReport *rulebook_reports = nullptr;  // kRulebookNotes slots behind pinned_scalar
+  unsigned long long *rulebook_reports = nullptr;  // kRulebookNotes stamped words behind pinned_scalar
+  unsigned long long *count_words = nullptr;   // kRulebookNotes x kCountWords behind those
   int next_rulebook_note = 0;
   unsigned long long next_stamp = 1;   // also the source of per-call tickets
 
@@ -158,6 +160,13 @@ class LogMessage {
   const char *level_;
   std::ostringstream ss_;
 };
+
+// Waits until a kernel on `queue` has stored a word with the low half of `stamp` above its
+// value into pinned memory, and returns the value through `value`.  The word is looked at
+// directly (a wait for an event or the queue costs the runtime's wake-up, 10 us and more, on
+// top); a queue that is through or in error without having stored it ends the wait.
+hipError_t waitForWord(hipStream_t queue, const unsigned long long *word, unsigned long long stamp,
+                       int32_t *value);
 
 }  // namespace mluop
 

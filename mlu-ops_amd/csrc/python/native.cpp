@@ -1,0 +1,633 @@
+// The host side of the Python package in native code: tensors in, tensors out, one call per
+// operator.  A call sets its descriptors, asks for the workspace size, allocates outputs and
+// workspace from torch's caching allocator and enqueues the operator through the C API; the
+// sparse layers' autograd node lives here as well, so that neither direction of a layer runs
+// interpreter code.  What bounds a small layer is this path: with ctypes calls, Python
+// descriptors and a Python autograd function a training step of one layer took 290-360 us of
+// host time around 90-130 us of kernels.
+//
+// The library is bound at run time (bind) to the very file the ctypes side loaded, so both
+// share its handles.
+#include <torch/extension.h>
+
+#include <ATen/hip/HIPContext.h>
+#include <c10/hip/HIPStream.h>
+#include <dlfcn.h>
+
+#include <map>
+#include <mutex>
+#include <optional>
+#include <stdexcept>
+#include <string>
+#include <utility>
+#include <vector>
+
+#include "mlu_op.h"
+#include "mlu_op_ext.h"
+
+namespace py = pybind11;
+
+namespace {
+
+// ---- the library ---------------------------------------------------------------------------
+
+#define MLUOP_NATIVE_FUNCTIONS(X)                          \
+  X(mluOpCreate)                                           \
+  X(mluOpSetQueue)                                         \
+  X(mluOpGetErrorString)                                   \
+  X(mluOpCreateTensorDescriptor)                           \
+  X(mluOpSetTensorDescriptor_v2)                           \
+  X(mluOpSetTensorDescriptorOnchipDataType)                \
+  X(mluOpDestroyTensorDescriptor)                          \
+  X(mluOpCreateSparseConvolutionDescriptor)                \
+  X(mluOpSetSparseConvolutionDescriptor)                   \
+  X(mluOpGetSparseConvolutionNumActOut)                    \
+  X(mluOpDestroySparseConvolutionDescriptor)               \
+  X(mluOpGetIndicePairsWorkspaceSize)                      \
+  X(mluOpGetIndicePairs)                                   \
+  X(mluOpGetIndiceConvolutionForwardWorkspaceSize)         \
+  X(mluOpIndiceConvolutionForward)                         \
+  X(mluOpGetIndiceConvolutionBackwardDataWorkspaceSize)    \
+  X(mluOpIndiceConvolutionBackwardData)                    \
+  X(mluOpGetIndiceConvolutionBackwardFilterWorkspaceSize)  \
+  X(mluOpIndiceConvolutionBackwardFilter)                  \
+  X(mluOpGetVoxelizationWorkspaceSize)                     \
+  X(mluOpVoxelization)                                     \
+  X(mluOpGetDynamicPointToVoxelForwardWorkspaceSize)       \
+  X(mluOpDynamicPointToVoxelForward)                       \
+  X(mluOpGetDynamicPointToVoxelBackwardWorkspaceSize)      \
+  X(mluOpDynamicPointToVoxelBackward)                      \
+  X(mluOpExtSetSparseConvExtendedModes)                    \
+  X(mluOpExtSetDistinctPairsPromise)                       \
+  X(mluOpExtGetIndicePairsHostCounts)                      \
+  X(mluOpExtUseRowMap)
+
+struct Library {
+#define X(name) decltype(&::name) name = nullptr;
+  MLUOP_NATIVE_FUNCTIONS(X)
+#undef X
+};
+Library api;
+
+void bind(const std::string &path) {
+  void *so = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
+  if (so == nullptr) throw std::runtime_error(std::string("cannot load ") + path + ": " + dlerror());
+#define X(name)                                                                         \
+  api.name = reinterpret_cast<decltype(&::name)>(dlsym(so, #name));                     \
+  if (api.name == nullptr) throw std::runtime_error(path + " does not export " #name);
+  MLUOP_NATIVE_FUNCTIONS(X)
+#undef X
+}
+
+// A status other than success; Python sees it as mluop_hip.MluOpError.
+struct StatusError : std::runtime_error {
+  StatusError(int status, const char *what)
+      : std::runtime_error(std::string(what) + " returned " +
+                           api.mluOpGetErrorString(static_cast<mluOpStatus_t>(status))),
+        status(status), call(what) {}
+  int status;
+  std::string call;
+};
+
+inline void check(mluOpStatus_t status, const char *what) {
+  if (status != MLUOP_STATUS_SUCCESS) throw StatusError(status, what);
+}
+
+class TensorDesc {
+ public:
+  TensorDesc(mluOpTensorLayout_t layout, mluOpDataType_t dtype, at::IntArrayRef dims) {
+    check(api.mluOpCreateTensorDescriptor(&d_), "mluOpCreateTensorDescriptor");
+    const mluOpStatus_t st =
+        api.mluOpSetTensorDescriptor_v2(d_, layout, dtype, static_cast<int>(dims.size()), dims.data());
+    if (st != MLUOP_STATUS_SUCCESS) {
+      api.mluOpDestroyTensorDescriptor(d_);
+      check(st, "mluOpSetTensorDescriptor_v2");
+    }
+  }
+  ~TensorDesc() { api.mluOpDestroyTensorDescriptor(d_); }
+  TensorDesc(const TensorDesc &) = delete;
+  TensorDesc &operator=(const TensorDesc &) = delete;
+  operator mluOpTensorDescriptor_t() const { return d_; }
+
+ private:
+  mluOpTensorDescriptor_t d_ = nullptr;
+};
+
+mluOpDataType_t dtypeCode(at::ScalarType t) {
+  switch (t) {
+    case at::kHalf: return MLUOP_DTYPE_HALF;
+    case at::kFloat: return MLUOP_DTYPE_FLOAT;
+    case at::kBFloat16: return MLUOP_DTYPE_BFLOAT16;
+    case at::kInt: return MLUOP_DTYPE_INT32;
+    default: throw py::key_error(std::string(c10::toString(t)));
+  }
+}
+
+// ---- buffers -------------------------------------------------------------------------------
+
+// Outputs and workspaces of one operator call.  In the package's guard mode (bands of a
+// pattern around every buffer, checked after the call) they come from the Python functions
+// that keep the bands; otherwise straight from the allocator.  Never used with the GIL held.
+class Buffers {
+ public:
+  Buffers(bool guarded, at::Device device) : guarded_(guarded), device_(device) {}
+
+  at::Tensor output(at::IntArrayRef shape, at::ScalarType dtype, const char *what,
+                    std::optional<int> fill = std::nullopt) const {
+    if (guarded_) {
+      py::gil_scoped_acquire gil;
+      py::tuple dims(shape.size());
+      for (size_t i = 0; i < shape.size(); ++i) dims[i] = shape[i];
+      py::object filled = py::none();
+      if (fill) filled = py::int_(*fill);
+      return package().attr("_output")(dims, py::cast(dtype), py::cast(device_), what, filled).cast<at::Tensor>();
+    }
+    const auto options = at::TensorOptions().dtype(dtype).device(device_);
+    return fill ? at::full(shape, *fill, options) : at::empty(shape, options);
+  }
+  at::Tensor workspace(size_t bytes) const {
+    if (guarded_) {
+      py::gil_scoped_acquire gil;
+      return package().attr("_workspace")(bytes, py::cast(device_)).cast<at::Tensor>();
+    }
+    return at::empty({static_cast<int64_t>(bytes > 0 ? bytes : 1)},
+                     at::TensorOptions().dtype(at::kByte).device(device_));
+  }
+  void done(const char *call) const {
+    if (!guarded_) return;
+    py::gil_scoped_acquire gil;
+    package().attr("_guards_intact")(call);
+  }
+
+ private:
+  static py::module_ package() { return py::module_::import("mluop_hip"); }
+  bool guarded_;
+  at::Device device_;
+};
+
+// ---- operators -----------------------------------------------------------------------------
+
+using Ints = std::vector<int>;
+using Counts = std::vector<int64_t>;
+
+struct Rulebook3 {
+  at::Tensor pairs, out_indices, indice_num;
+  int64_t num_act_out = 0;
+  Counts counts;
+};
+
+// Sets and destroys the descriptor of one rulebook call.
+class ConvDesc {
+ public:
+  ConvDesc(int batch, const Ints &pad, const Ints &stride, const Ints &dilation, const Ints &input_space,
+           const Ints &filter_space, const Ints &output_space, bool sub_m) {
+    for (const Ints *v : {&pad, &stride, &dilation, &input_space, &filter_space, &output_space})
+      if (v->size() != 3) throw py::value_error("spaces, padding, stride and dilation have three values each");
+    check(api.mluOpCreateSparseConvolutionDescriptor(&d_), "mluOpCreateSparseConvolutionDescriptor");
+    const mluOpStatus_t st = api.mluOpSetSparseConvolutionDescriptor(
+        d_, 5, batch, pad.data(), stride.data(), dilation.data(), input_space.data(), filter_space.data(),
+        output_space.data(), sub_m ? 1 : 0, 0, 0);
+    if (st != MLUOP_STATUS_SUCCESS) {
+      api.mluOpDestroySparseConvolutionDescriptor(d_);
+      check(st, "mluOpSetSparseConvolutionDescriptor");
+    }
+  }
+  ~ConvDesc() { api.mluOpDestroySparseConvolutionDescriptor(d_); }
+  ConvDesc(const ConvDesc &) = delete;
+  ConvDesc &operator=(const ConvDesc &) = delete;
+  operator mluOpSparseConvolutionDescriptor_t() const { return d_; }
+
+ private:
+  mluOpSparseConvolutionDescriptor_t d_ = nullptr;
+};
+
+// `for_layer`: out_indices is cut to the active rows (and its tail left as allocated), and the
+// counts come back on the host.
+Rulebook3 indicePairs(mluOpHandle_t handle, const Buffers &buffers, const at::Tensor &indices, int batch,
+                      const Ints &input_space, const Ints &filter_space, const Ints &output_space, const Ints &pad,
+                      const Ints &stride, const Ints &dilation, bool sub_m, std::optional<int64_t> out_rows,
+                      std::optional<at::Tensor> out_indices, bool for_layer) {
+  const int64_t L = indices.size(0);
+  int64_t K = 1;
+  for (int k : filter_space) K *= k;
+  if (!out_rows) {
+    int64_t volume = batch;
+    for (int o : output_space) volume *= o;
+    out_rows = sub_m ? L : std::min(volume, K * L);
+  }
+  Rulebook3 r;
+  r.pairs = buffers.output({K, 2, L}, at::kInt, "indice_pairs");
+  if (out_indices) {
+    r.out_indices = *out_indices;
+    out_rows = out_indices->size(0);
+  } else {
+    // the operator writes the first num_act_out rows only; the rest keep this initial -1
+    r.out_indices = buffers.output({*out_rows, 4}, at::kInt, "out_indices",
+                                   for_layer ? std::nullopt : std::optional<int>(-1));
+  }
+  r.indice_num = buffers.output({K}, at::kInt, "indice_num");
+  const ConvDesc conv(batch, pad, stride, dilation, input_space, filter_space, output_space, sub_m);
+  const TensorDesc d_in(MLUOP_LAYOUT_ARRAY, MLUOP_DTYPE_INT32, {L, 4});
+  const TensorDesc d_pairs(MLUOP_LAYOUT_ARRAY, MLUOP_DTYPE_INT32, {K, 2, L});
+  const TensorDesc d_out(MLUOP_LAYOUT_ARRAY, MLUOP_DTYPE_INT32, {*out_rows, 4});
+  const TensorDesc d_num(MLUOP_LAYOUT_ARRAY, MLUOP_DTYPE_INT32, {K});
+  size_t bytes = 0;
+  check(api.mluOpGetIndicePairsWorkspaceSize(handle, conv, d_in, d_pairs, d_out, d_num, &bytes),
+        "mluOpGetIndicePairsWorkspaceSize");
+  const at::Tensor ws = buffers.workspace(bytes);
+  check(api.mluOpGetIndicePairs(handle, conv, d_in, indices.data_ptr(), ws.data_ptr(), bytes, d_pairs,
+                                r.pairs.data_ptr(), d_out, r.out_indices.data_ptr(), d_num, r.indice_num.data_ptr()),
+        "mluOpGetIndicePairs");
+  r.num_act_out = L;
+  if (!sub_m) {
+    int n = 0;
+    check(api.mluOpGetSparseConvolutionNumActOut(conv, &n), "mluOpGetSparseConvolutionNumActOut");
+    r.num_act_out = n;
+  }
+  if (for_layer) {
+    r.counts.assign(K, 0);
+    const bool empty = L == 0 || K == 0 || *out_rows == 0;
+    if (!empty && api.mluOpExtGetIndicePairsHostCounts(handle, r.pairs.data_ptr(), static_cast<int>(K),
+                                                       r.counts.data()) != MLUOP_STATUS_SUCCESS) {
+      const at::Tensor host = r.indice_num.cpu();
+      const int32_t *n = host.data_ptr<int32_t>();
+      r.counts.assign(n, n + K);
+    }
+    r.out_indices = r.out_indices.narrow(0, 0, r.num_act_out);
+  }
+  buffers.done("mluOpGetIndicePairs");
+  return r;
+}
+
+at::Tensor convForward(mluOpHandle_t handle, const Buffers &buffers, const at::Tensor &features,
+                       const at::Tensor &filters, mluOpTensorLayout_t layout, const at::Tensor &pairs,
+                       const Counts &counts, int64_t num_act_out, bool sub_m, int64_t inverse,
+                       const void *row_map) {
+  const mluOpDataType_t code = dtypeCode(features.scalar_type());
+  const int64_t co = filters.size(layout == MLUOP_LAYOUT_ARRAY ? 4 : 0);
+  at::Tensor out = buffers.output({num_act_out, co}, features.scalar_type(), "features_out");
+  const TensorDesc d_x(MLUOP_LAYOUT_ARRAY, code, features.sizes());
+  const TensorDesc d_w(layout, code, filters.sizes());
+  const TensorDesc d_pairs(MLUOP_LAYOUT_ARRAY, MLUOP_DTYPE_INT32, pairs.sizes());
+  const TensorDesc d_out(MLUOP_LAYOUT_ARRAY, code, out.sizes());
+  size_t bytes = 0;
+  check(api.mluOpGetIndiceConvolutionForwardWorkspaceSize(handle, d_x, d_w, d_pairs, d_out, counts.data(),
+                                                          num_act_out, inverse, sub_m, &bytes),
+        "mluOpGetIndiceConvolutionForwardWorkspaceSize");
+  const at::Tensor ws = buffers.workspace(bytes);
+  if (row_map != nullptr) check(api.mluOpExtUseRowMap(handle, row_map), "mluOpExtUseRowMap");
+  check(api.mluOpIndiceConvolutionForward(handle, d_x, features.data_ptr(), d_w, filters.data_ptr(), d_pairs,
+                                          pairs.data_ptr(), counts.data(), num_act_out, inverse, sub_m,
+                                          ws.data_ptr(), bytes, d_out, out.data_ptr()),
+        "mluOpIndiceConvolutionForward");
+  buffers.done("mluOpIndiceConvolutionForward");
+  return out;
+}
+
+at::Tensor convBackwardData(mluOpHandle_t handle, const Buffers &buffers, const at::Tensor &output_grad,
+                            const at::Tensor &filters, mluOpTensorLayout_t layout, const at::Tensor &pairs,
+                            const Counts &counts, bool sub_m, int64_t ci, int64_t inverse, int64_t rows,
+                            const void *row_map) {
+  const mluOpDataType_t code = dtypeCode(output_grad.scalar_type());
+  at::Tensor dx = buffers.output({rows, ci}, output_grad.scalar_type(), "input_grad");
+  const TensorDesc d_dy(MLUOP_LAYOUT_ARRAY, code, output_grad.sizes());
+  const TensorDesc d_w(layout, code, filters.sizes());
+  const TensorDesc d_pairs(MLUOP_LAYOUT_ARRAY, MLUOP_DTYPE_INT32, pairs.sizes());
+  const TensorDesc d_dx(MLUOP_LAYOUT_ARRAY, code, dx.sizes());
+  size_t bytes = 0;
+  check(api.mluOpGetIndiceConvolutionBackwardDataWorkspaceSize(handle, d_dy, d_w, d_pairs, d_dx, counts.data(),
+                                                               inverse, &bytes),
+        "mluOpGetIndiceConvolutionBackwardDataWorkspaceSize");
+  const at::Tensor ws = buffers.workspace(bytes);
+  if (row_map != nullptr) check(api.mluOpExtUseRowMap(handle, row_map), "mluOpExtUseRowMap");
+  check(api.mluOpIndiceConvolutionBackwardData(handle, d_dy, output_grad.data_ptr(), d_w, filters.data_ptr(),
+                                               d_pairs, pairs.data_ptr(), counts.data(), inverse, sub_m,
+                                               ws.data_ptr(), bytes, d_dx, dx.data_ptr()),
+        "mluOpIndiceConvolutionBackwardData");
+  buffers.done("mluOpIndiceConvolutionBackwardData");
+  return dx;
+}
+
+at::Tensor convBackwardFilter(mluOpHandle_t handle, const Buffers &buffers, const at::Tensor &features,
+                              const at::Tensor &output_grad, const at::Tensor &pairs, const Counts &counts,
+                              const Counts &filter_space, bool sub_m, int64_t inverse, bool onchip_float,
+                              mluOpTensorLayout_t layout) {
+  const mluOpDataType_t code = dtypeCode(features.scalar_type());
+  const int64_t ci = features.size(1), co = output_grad.size(1);
+  Counts shape;
+  if (layout == MLUOP_LAYOUT_NDHWC || layout == MLUOP_LAYOUT_NHWC) {
+    shape.push_back(co);
+    shape.insert(shape.end(), filter_space.begin(), filter_space.end());
+    shape.push_back(ci);
+  } else if (layout == MLUOP_LAYOUT_NCDHW || layout == MLUOP_LAYOUT_NCHW) {
+    shape = {co, ci};
+    shape.insert(shape.end(), filter_space.begin(), filter_space.end());
+  } else {
+    shape = filter_space;
+    shape.push_back(ci);
+    shape.push_back(co);
+  }
+  at::Tensor dw = buffers.output(shape, features.scalar_type(), "filters_grad");
+  const TensorDesc d_x(MLUOP_LAYOUT_ARRAY, code, features.sizes());
+  const TensorDesc d_dy(MLUOP_LAYOUT_ARRAY, code, output_grad.sizes());
+  const TensorDesc d_pairs(MLUOP_LAYOUT_ARRAY, MLUOP_DTYPE_INT32, pairs.sizes());
+  const TensorDesc d_dw(layout, code, dw.sizes());
+  if (onchip_float)
+    check(api.mluOpSetTensorDescriptorOnchipDataType(d_dw, MLUOP_DTYPE_FLOAT),
+          "mluOpSetTensorDescriptorOnchipDataType");
+  size_t bytes = 0;
+  check(api.mluOpGetIndiceConvolutionBackwardFilterWorkspaceSize(handle, d_x, d_dy, d_pairs, d_dw, counts.data(),
+                                                                 inverse, sub_m, &bytes),
+        "mluOpGetIndiceConvolutionBackwardFilterWorkspaceSize");
+  const at::Tensor ws = buffers.workspace(bytes);
+  check(api.mluOpIndiceConvolutionBackwardFilter(handle, d_x, features.data_ptr(), d_dy, output_grad.data_ptr(),
+                                                 d_pairs, pairs.data_ptr(), counts.data(), inverse, sub_m,
+                                                 ws.data_ptr(), bytes, d_dw, dw.data_ptr()),
+        "mluOpIndiceConvolutionBackwardFilter");
+  buffers.done("mluOpIndiceConvolutionBackwardFilter");
+  return dw;
+}
+
+// ---- handles of the layers -----------------------------------------------------------------
+
+// One library handle per (device, stream), made on first use and kept for the life of the
+// process; its mutex keeps the calls of one operator together when several threads use one
+// stream.
+struct StreamHandle {
+  mluOpHandle_t handle = nullptr;
+  std::mutex mutex;
+};
+
+StreamHandle &streamHandle() {
+  static std::mutex mutex;
+  static auto *handles = new std::map<std::pair<int, hipStream_t>, StreamHandle>();
+  const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream();
+  std::lock_guard<std::mutex> lock(mutex);
+  StreamHandle &h = (*handles)[{static_cast<int>(stream.device_index()), stream.stream()}];
+  if (h.handle == nullptr) {
+    check(api.mluOpCreate(&h.handle), "mluOpCreate");
+    check(api.mluOpSetQueue(h.handle, reinterpret_cast<mluOpQueue_t>(stream.stream())), "mluOpSetQueue");
+    // SparseInverseConv3d runs the operators with inverse = 1
+    check(api.mluOpExtSetSparseConvExtendedModes(h.handle, 1), "mluOpExtSetSparseConvExtendedModes");
+  }
+  return h;
+}
+
+// ---- the layers' autograd node -------------------------------------------------------------
+
+// What the three convolution operators need of a rulebook.  `row_maps` holds, by pair column,
+// the map buffers a caller shares between calls (undefined tensors: none).
+struct LayerRulebook : torch::CustomClassHolder {
+  at::Tensor pairs;
+  Counts counts, filter_space;
+  int64_t num_act_out = 0;
+  bool sub_m = false, distinct = false;
+  at::Tensor row_maps[2];
+
+  const void *rowMap(int column) const {
+    return row_maps[column].defined() ? row_maps[column].data_ptr() : nullptr;
+  }
+};
+using LayerRulebookPtr = c10::intrusive_ptr<LayerRulebook>;
+
+struct IndiceConv : torch::autograd::Function<IndiceConv> {
+  static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &features,
+                            const at::Tensor &weight, const LayerRulebookPtr &rb, bool inverse, bool guarded) {
+    const at::Tensor x = features.contiguous(), w = weight.contiguous();
+    ctx->save_for_backward({x, w});
+    ctx->saved_data["rulebook"] = c10::IValue::make_capsule(rb);
+    ctx->saved_data["inverse"] = inverse;
+    ctx->saved_data["guarded"] = guarded;
+    StreamHandle &h = streamHandle();
+    const std::lock_guard<std::mutex> lock(h.mutex);
+    check(api.mluOpExtSetDistinctPairsPromise(h.handle, rb->distinct), "mluOpExtSetDistinctPairsPromise");
+    const Buffers buffers(guarded, x.device());
+    // an inverse layer runs the partner layer's rulebook backwards: one output row per input
+    // row of the partner
+    return inverse ? convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts,
+                                 rb->pairs.size(2), false, 1, rb->rowMap(0))
+                   : convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts,
+                                 rb->num_act_out, rb->sub_m, 0, rb->rowMap(1));
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx,
+                                                 torch::autograd::variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const at::Tensor &x = saved[0], &w = saved[1];
+    const auto rb = c10::static_intrusive_pointer_cast<LayerRulebook>(ctx->saved_data["rulebook"].toCapsule());
+    const bool inverse = ctx->saved_data["inverse"].toBool();
+    torch::autograd::variable_list out(5);
+    if (!grads[0].defined()) return out;
+    const at::Tensor dy = grads[0].contiguous();
+    StreamHandle &h = streamHandle();
+    const std::lock_guard<std::mutex> lock(h.mutex);
+    check(api.mluOpExtSetDistinctPairsPromise(h.handle, rb->distinct), "mluOpExtSetDistinctPairsPromise");
+    const Buffers buffers(ctx->saved_data["guarded"].toBool(), x.device());
+    const bool sub_m = !inverse && rb->sub_m;
+    if (ctx->needs_input_grad(0))
+      out[0] = convBackwardData(h.handle, buffers, dy, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts, sub_m,
+                                x.size(1), inverse, x.size(0), rb->rowMap(inverse ? 1 : 0));
+    if (ctx->needs_input_grad(1))
+      out[1] = convBackwardFilter(h.handle, buffers, x, dy, rb->pairs, rb->counts, rb->filter_space, sub_m, inverse,
+                                  true, MLUOP_LAYOUT_ARRAY);
+    return out;
+  }
+};
+
+// ---- point operators -----------------------------------------------------------------------
+
+std::vector<at::Tensor> voxelization(mluOpHandle_t handle, const Buffers &buffers, const at::Tensor &points,
+                                     const at::Tensor &voxel_size, const at::Tensor &coors_range, int64_t max_points,
+                                     int64_t max_voxels, bool deterministic) {
+  const at::Tensor voxels = buffers.output({max_voxels, max_points, points.size(1)}, at::kFloat, "voxels");
+  const at::Tensor coors = buffers.output({max_voxels, 3}, at::kInt, "coors");
+  const at::Tensor npv = buffers.output({max_voxels}, at::kInt, "num_points_per_voxel");
+  const at::Tensor num = at::zeros({1}, at::TensorOptions().dtype(at::kInt).device(points.device()));
+  const mluOpTensorLayout_t array = MLUOP_LAYOUT_ARRAY;
+  const TensorDesc d_points(array, MLUOP_DTYPE_FLOAT, points.sizes());
+  const TensorDesc d_vs(array, MLUOP_DTYPE_FLOAT, {3});
+  const TensorDesc d_cr(array, MLUOP_DTYPE_FLOAT, {6});
+  const TensorDesc d_voxels(array, MLUOP_DTYPE_FLOAT, voxels.sizes());
+  const TensorDesc d_coors(array, MLUOP_DTYPE_INT32, coors.sizes());
+  const TensorDesc d_npv(array, MLUOP_DTYPE_INT32, npv.sizes());
+  const TensorDesc d_num(array, MLUOP_DTYPE_INT32, {1});
+  size_t bytes = 0;
+  check(api.mluOpGetVoxelizationWorkspaceSize(handle, d_points, d_vs, d_cr, static_cast<int32_t>(max_points),
+                                              static_cast<int32_t>(max_voxels), 3, deterministic, d_voxels, d_coors,
+                                              d_npv, d_num, &bytes),
+        "mluOpGetVoxelizationWorkspaceSize");
+  const at::Tensor ws = buffers.workspace(bytes);
+  check(api.mluOpVoxelization(handle, d_points, points.data_ptr(), d_vs, voxel_size.data_ptr(), d_cr,
+                              coors_range.data_ptr(), static_cast<int32_t>(max_points),
+                              static_cast<int32_t>(max_voxels), 3, deterministic, ws.data_ptr(), bytes, d_voxels,
+                              voxels.data_ptr(), d_coors, coors.data_ptr(), d_npv, npv.data_ptr(), d_num,
+                              num.data_ptr()),
+        "mluOpVoxelization");
+  buffers.done("mluOpVoxelization");
+  return {voxels, coors, npv, num};
+}
+
+std::vector<at::Tensor> scatterForward(mluOpHandle_t handle, const Buffers &buffers, const at::Tensor &feats,
+                                       const at::Tensor &coors, mluOpReduceMode_t mode, int64_t rows) {
+  const int64_t n = feats.size(0), c = feats.size(1);
+  const at::Tensor voxel_feats = buffers.output({rows, c}, at::kFloat, "voxel_feats");
+  const at::Tensor voxel_coors = buffers.output({rows, 3}, at::kInt, "voxel_coors");
+  const at::Tensor p2v = buffers.output({n}, at::kInt, "point2voxel_map");
+  const at::Tensor count = buffers.output({rows}, at::kInt, "voxel_points_count");
+  const at::Tensor num = at::zeros({1}, at::TensorOptions().dtype(at::kInt).device(feats.device()));
+  const mluOpTensorLayout_t array = MLUOP_LAYOUT_ARRAY;
+  const TensorDesc d_feats(array, MLUOP_DTYPE_FLOAT, feats.sizes());
+  const TensorDesc d_coors(array, MLUOP_DTYPE_INT32, coors.sizes());
+  const TensorDesc d_vf(array, MLUOP_DTYPE_FLOAT, voxel_feats.sizes());
+  const TensorDesc d_vc(array, MLUOP_DTYPE_INT32, voxel_coors.sizes());
+  const TensorDesc d_p2v(array, MLUOP_DTYPE_INT32, p2v.sizes());
+  const TensorDesc d_count(array, MLUOP_DTYPE_INT32, count.sizes());
+  const TensorDesc d_num(array, MLUOP_DTYPE_INT32, {1});
+  size_t bytes = 0;
+  check(api.mluOpGetDynamicPointToVoxelForwardWorkspaceSize(handle, d_feats, d_coors, &bytes),
+        "mluOpGetDynamicPointToVoxelForwardWorkspaceSize");
+  const at::Tensor ws = buffers.workspace(bytes);
+  check(api.mluOpDynamicPointToVoxelForward(handle, mode, d_feats, feats.data_ptr(), d_coors, coors.data_ptr(),
+                                            ws.data_ptr(), bytes, d_vf, voxel_feats.data_ptr(), d_vc,
+                                            voxel_coors.data_ptr(), d_p2v, p2v.data_ptr(), d_count, count.data_ptr(),
+                                            d_num, num.data_ptr()),
+        "mluOpDynamicPointToVoxelForward");
+  buffers.done("mluOpDynamicPointToVoxelForward");
+  return {voxel_feats, voxel_coors, p2v, count, num};
+}
+
+at::Tensor scatterBackward(mluOpHandle_t handle, const Buffers &buffers, const at::Tensor &grad,
+                           const at::Tensor &feats, const at::Tensor &voxel_feats, const at::Tensor &p2v,
+                           const at::Tensor &count, const at::Tensor &num, mluOpReduceMode_t mode) {
+  const int64_t n = feats.size(0), c = feats.size(1), m = grad.size(0);
+  const at::Tensor grad_feats = buffers.output({n, c}, at::kFloat, "grad_feats");
+  const mluOpTensorLayout_t array = MLUOP_LAYOUT_ARRAY;
+  const TensorDesc d_grad(array, MLUOP_DTYPE_FLOAT, {m, c});
+  const TensorDesc d_feats(array, MLUOP_DTYPE_FLOAT, {n, c});
+  const TensorDesc d_vf(array, MLUOP_DTYPE_FLOAT, {m, c});
+  const TensorDesc d_p2v(array, MLUOP_DTYPE_INT32, {n});
+  const TensorDesc d_count(array, MLUOP_DTYPE_INT32, {m});
+  const TensorDesc d_num(array, MLUOP_DTYPE_INT32, {1});
+  size_t bytes = 0;
+  check(api.mluOpGetDynamicPointToVoxelBackwardWorkspaceSize(handle, mode, d_grad, d_feats, d_vf, d_p2v, d_count,
+                                                             d_num, &bytes),
+        "mluOpGetDynamicPointToVoxelBackwardWorkspaceSize");
+  const at::Tensor ws = buffers.workspace(bytes);
+  check(api.mluOpDynamicPointToVoxelBackward(handle, mode, d_grad, grad.data_ptr(), d_feats, feats.data_ptr(), d_vf,
+                                             voxel_feats.data_ptr(), d_p2v, p2v.data_ptr(), d_count,
+                                             count.data_ptr(), d_num, num.data_ptr(), ws.data_ptr(), bytes, d_feats,
+                                             grad_feats.data_ptr()),
+        "mluOpDynamicPointToVoxelBackward");
+  buffers.done("mluOpDynamicPointToVoxelBackward");
+  return grad_feats;
+}
+
+inline mluOpHandle_t asHandle(uintptr_t h) { return reinterpret_cast<mluOpHandle_t>(h); }
+
+}  // namespace
+
+PYBIND11_MODULE(_native, m) {
+  using NoGil = py::gil_scoped_release;
+  m.doc() = "Native host path of mluop_hip: operators and the sparse layers' autograd node over the C API.";
+
+  static py::exception<StatusError> unused(m, "StatusError", PyExc_RuntimeError);
+  py::register_exception_translator([](std::exception_ptr p) {
+    try {
+      if (p) std::rethrow_exception(p);
+    } catch (const StatusError &e) {
+      const py::object type = py::module_::import("mluop_hip").attr("MluOpError");
+      const py::object error = type(e.status, e.call);
+      PyErr_SetObject(type.ptr(), error.ptr());
+    }
+  });
+
+  m.def("bind", &bind, "Binds the C API to the library at this path.");
+  m.def("stream_handle", [] { return reinterpret_cast<uintptr_t>(streamHandle().handle); },
+        "The library handle of the current device and stream.");
+
+  m.def("get_indice_pairs",
+        [](uintptr_t handle, bool guarded, const at::Tensor &indices, int batch, const Ints &input_space,
+           const Ints &filter_space, const Ints &output_space, const Ints &pad, const Ints &stride,
+           const Ints &dilation, bool sub_m, std::optional<int64_t> out_rows, std::optional<at::Tensor> out_indices,
+           bool for_layer) {
+          Rulebook3 r;
+          {
+            NoGil released;
+            r = indicePairs(asHandle(handle), Buffers(guarded, indices.device()), indices, batch, input_space,
+                            filter_space, output_space, pad, stride, dilation, sub_m, out_rows, std::move(out_indices),
+                            for_layer);
+          }
+          py::object num = for_layer ? py::cast(r.counts) : py::cast(r.indice_num);
+          return py::make_tuple(r.pairs, r.out_indices, num, r.num_act_out);
+        });
+  m.def("indice_conv_forward",
+        [](uintptr_t handle, bool guarded, const at::Tensor &features, const at::Tensor &filters, int layout,
+           const at::Tensor &pairs, const Counts &counts, int64_t num_act_out, bool sub_m, int64_t inverse,
+           uintptr_t row_map) {
+          NoGil released;
+          return convForward(asHandle(handle), Buffers(guarded, features.device()), features, filters,
+                             static_cast<mluOpTensorLayout_t>(layout), pairs, counts, num_act_out, sub_m, inverse,
+                             reinterpret_cast<const void *>(row_map));
+        });
+  m.def("indice_conv_backward_data",
+        [](uintptr_t handle, bool guarded, const at::Tensor &output_grad, const at::Tensor &filters, int layout,
+           const at::Tensor &pairs, const Counts &counts, bool sub_m, int64_t ci, int64_t inverse, int64_t rows,
+           uintptr_t row_map) {
+          NoGil released;
+          return convBackwardData(asHandle(handle), Buffers(guarded, output_grad.device()), output_grad, filters,
+                                  static_cast<mluOpTensorLayout_t>(layout), pairs, counts, sub_m, ci, inverse, rows,
+                                  reinterpret_cast<const void *>(row_map));
+        });
+  m.def("indice_conv_backward_filter",
+        [](uintptr_t handle, bool guarded, const at::Tensor &features, const at::Tensor &output_grad,
+           const at::Tensor &pairs, const Counts &counts, const Counts &filter_space, bool sub_m, int64_t inverse,
+           bool onchip_float, int layout) {
+          NoGil released;
+          return convBackwardFilter(asHandle(handle), Buffers(guarded, features.device()), features, output_grad,
+                                    pairs, counts, filter_space, sub_m, inverse, onchip_float,
+                                    static_cast<mluOpTensorLayout_t>(layout));
+        });
+  m.def("voxelization",
+        [](uintptr_t handle, bool guarded, const at::Tensor &points, const at::Tensor &voxel_size,
+           const at::Tensor &coors_range, int64_t max_points, int64_t max_voxels, bool deterministic) {
+          NoGil released;
+          return voxelization(asHandle(handle), Buffers(guarded, points.device()), points, voxel_size, coors_range,
+                              max_points, max_voxels, deterministic);
+        });
+  m.def("dynamic_point_to_voxel_forward",
+        [](uintptr_t handle, bool guarded, const at::Tensor &feats, const at::Tensor &coors, int mode, int64_t rows) {
+          NoGil released;
+          return scatterForward(asHandle(handle), Buffers(guarded, feats.device()), feats, coors,
+                                static_cast<mluOpReduceMode_t>(mode), rows);
+        });
+  m.def("dynamic_point_to_voxel_backward",
+        [](uintptr_t handle, bool guarded, const at::Tensor &grad, const at::Tensor &feats,
+           const at::Tensor &voxel_feats, const at::Tensor &p2v, const at::Tensor &count, const at::Tensor &num,
+           int mode) {
+          NoGil released;
+          return scatterBackward(asHandle(handle), Buffers(guarded, feats.device()), grad, feats, voxel_feats, p2v,
+                                 count, num, static_cast<mluOpReduceMode_t>(mode));
+        });
+
+  py::class_<LayerRulebook, LayerRulebookPtr>(m, "LayerRulebook")
+      .def(py::init([](const at::Tensor &pairs, Counts counts, int64_t num_act_out, Counts filter_space, bool sub_m,
+                       bool distinct) {
+        auto rb = c10::make_intrusive<LayerRulebook>();
+        rb->pairs = pairs;
+        rb->counts = std::move(counts);
+        rb->num_act_out = num_act_out;
+        rb->filter_space = std::move(filter_space);
+        rb->sub_m = sub_m;
+        rb->distinct = distinct;
+        return rb;
+      }))
+      .def("set_row_map", [](LayerRulebook &rb, int column, std::optional<at::Tensor> map) {
+        if (column != 0 && column != 1) throw py::index_error("a pair has two columns");
+        rb.row_maps[column] = map ? *map : at::Tensor();
+      });
+  m.def("indice_conv", [](const at::Tensor &features, const at::Tensor &weight, const LayerRulebookPtr &rulebook,
+                          bool inverse, bool guarded) {
+    NoGil released;
+    return IndiceConv::apply(features, weight, rulebook, inverse, guarded);
+  });
+}

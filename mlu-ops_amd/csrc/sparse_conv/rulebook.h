@@ -27,16 +27,26 @@ struct RulebookGeom {
   bool sub_m;
 };
 
-// Where the last kernel of a rulebook reports (pinned host memory, written from the device):
-// whether the input rows were strictly ascending in (n, d, h, w) order, then the stamp that
-// tells the host the report is the one it waits for.  Null words: no report.
+// Where the last kernel of a rulebook reports (pinned host memory, written from the device), in
+// words that carry the low half of the stamp above their value, so that a reader sees by
+// itself whether a word is this rulebook's.  Null pointers: no report.
 struct RulebookReportTarget {
-  unsigned long long *stamp_word = nullptr;
-  unsigned int *order_word = nullptr;
+  // were the input rows strictly ascending in (n, d, h, w) order?
+  unsigned long long *order_word = nullptr;
   // A value no earlier rulebook of any handle used (never 0); also marks this call's words
   // in the workspace, so it is set whether or not a report is wanted.
   unsigned long long stamp = 0;
+  // word k: the number of pairs of offset k
+  unsigned long long *count_words = nullptr;
 };
+
+// A value with the low half of a stamp above it, as the device stores it for the host.
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+inline unsigned long long stampedWord(unsigned long long stamp, int value) {
+  return (stamp << 32) | (unsigned int)value;
+}
 
 // Bytes of device workspace the kernel set needs for this geometry.
 size_t rulebookWorkspaceBytes(const RulebookGeom &g);
@@ -47,13 +57,13 @@ hipError_t launchSubmRulebook(const LaunchCtx &lc, const RulebookGeom &g, const 
                               int32_t *indice_num, const RulebookReportTarget &report);
 
 // Enqueues regular (strided / dilated) rulebook construction.  The kernel that numbers the
-// output cells stores their count into `host_num_act_out` (pinned host memory) and
-// `count_ready` is recorded behind it: the caller waits for that event before reading the
-// count, while the kernel that writes the pair lists may still be running.
+// output cells stores their count, stamped, into `host_num_act_out` (pinned host memory): the
+// caller waits for that word, while the kernel that writes the pair lists may still be
+// running.
 hipError_t launchRegularRulebook(const LaunchCtx &lc, const RulebookGeom &g,
                                  const int32_t *indices, void *workspace, int32_t *indice_pairs,
                                  int32_t *out_indices, int32_t *indice_num,
-                                 int32_t *host_num_act_out, hipEvent_t count_ready,
+                                 unsigned long long *host_num_act_out,
                                  const RulebookReportTarget &report);
 
 }  // namespace sparse_conv

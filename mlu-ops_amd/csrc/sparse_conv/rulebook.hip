@@ -133,11 +133,19 @@ __device__ __forceinline__ void noteRowOrder(const int32_t *indices, int j, int4
 }
 
 // The rulebook's report to the host: the flag first, then the stamp the host looks for.
+// The number of pairs of offset k, for the device and for the host.
+__device__ __forceinline__ void fileCount(int k, int count, int32_t *indice_num,
+                                          const RulebookReportTarget &report) {
+  indice_num[k] = count;
+  if (report.count_words != nullptr)
+    __hip_atomic_store(report.count_words + k, stampedWord(report.stamp, count), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __device__ __forceinline__ void fileReport(bool rows_in_order, const RulebookReportTarget &report) {
-  if (report.stamp_word == nullptr) return;
-  *report.order_word = rows_in_order ? 1u : 0u;
-  __threadfence_system();
-  __hip_atomic_store(report.stamp_word, report.stamp, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (report.order_word == nullptr) return;
+  __hip_atomic_store(report.order_word, stampedWord(report.stamp, rows_in_order ? 1 : 0), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Up to three ranges of 32-bit words, each set to its own value (16-byte stores: every
@@ -1156,7 +1164,8 @@ __global__ __launch_bounds__(kBlock) void rbRankAndDecode(GeomDev g,
                                                           size_t n_words,
                                                           const int32_t *block_count,
                                                           bool scanned, int32_t *num_act_out,
-                                                          int32_t *host_num_act_out,
+                                                          unsigned long long *host_num_act_out,
+                                                          unsigned long long stamp,
                                                           uint32_t *word_rank,
                                                           int32_t *out_indices, bool aligned,
                                                           int out_rows) {
@@ -1194,10 +1203,12 @@ __global__ __launch_bounds__(kBlock) void rbRankAndDecode(GeomDev g,
   // the count of output cells, for the device and (pinned memory) for the host
   if (!scanned && blockIdx.x == gridDim.x - 1 && threadIdx.x == kBlock - 1) {
     *num_act_out = rank + mine;
-    __hip_atomic_store(host_num_act_out, rank + mine, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(host_num_act_out, stampedWord(stamp, rank + mine), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
   }
   if (scanned && blockIdx.x == 0 && threadIdx.x == 0)
-    __hip_atomic_store(host_num_act_out, *num_act_out, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(host_num_act_out, stampedWord(stamp, *num_act_out), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
   if (w < n_words) word_rank[w] = (uint32_t)rank;
   auto put = [&](size_t cell64, int r) {
     if (r >= out_rows) return;
@@ -1301,7 +1312,7 @@ __global__ __launch_bounds__(kPlaceBlock) void rbPlacePairs(int L, Staging st,
         in_col[r] = r;
         in_col[L + r] = r;
       }
-      if (blockIdx.x == 0 && tid == 0) indice_num[k] = L;
+      if (blockIdx.x == 0 && tid == 0) fileCount(k, L, indice_num, report);
       return;
     }
     mirror_in = pairs + (size_t)(K - 1 - k) * 2 * L;
@@ -1390,8 +1401,8 @@ __global__ __launch_bounds__(kPlaceBlock) void rbPlacePairs(int L, Staging st,
     before += total;
   }
   if (blockIdx.x == gridDim.x - 1 && tid == 0) {
-    indice_num[k] = before;
-    if (mirror) indice_num[gridDim.y - 1 - k] = before;
+    fileCount(k, before, indice_num, report);
+    if (mirror) fileCount(gridDim.y - 1 - k, before, indice_num, report);
   }
 }
 
@@ -1621,7 +1632,7 @@ hipError_t launchSubmRulebook(const LaunchCtx &lc, const RulebookGeom &g, const 
 hipError_t launchRegularRulebook(const LaunchCtx &lc, const RulebookGeom &g,
                                  const int32_t *indices, void *workspace, int32_t *indice_pairs,
                                  int32_t *out_indices, int32_t *indice_num,
-                                 int32_t *host_num_act_out, hipEvent_t count_ready,
+                                 unsigned long long *host_num_act_out,
                                  const RulebookReportTarget &report) {
   const Workspace ws = carve(g, workspace);
   const GeomDev d = toDev(g);
@@ -1690,10 +1701,8 @@ hipError_t launchRegularRulebook(const LaunchCtx &lc, const RulebookGeom &g,
   lc.begin("rbRankAndDecode");
   rbRankAndDecode<<<ws.n_bitmap_blocks, kBlock, 0, lc.stream>>>(d, ws.bitmap, ws.n_words, ws.block_sum,
                                                              scanned, ws.num_act_out, host_num_act_out,
-                                                             ws.word_rank, out_indices, al_out, g.out_rows);
+                                                             report.stamp, ws.word_rank, out_indices, al_out, g.out_rows);
   lc.end();
-  hipError_t err = hipEventRecord(count_ready, lc.stream);
-  if (err != hipSuccess) return err;
   lc.begin("rbPlacePairs");
   const int per_group = placeChunksPerGroup(ws.n_wave, g.K);
   const int place_groups = (ws.n_wave + kPlaceWaves * per_group - 1) / (kPlaceWaves * per_group);

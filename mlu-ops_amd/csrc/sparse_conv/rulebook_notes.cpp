@@ -16,9 +16,11 @@ RulebookReportTarget openRulebookNote(mluOpContext *handle, const void *pairs, i
   note.K = K;
   note.L = L;
   note.stamp = handle->next_stamp++;
-  // the device ORs its flags into a cleared word and stores the stamp last
-  handle->rulebook_reports[slot].stamp = 0;
-  handle->rulebook_reports[slot].rows_in_order = 0;
+  note.counts_on_file = false;
+  // no word of another rulebook passes for one of this
+  unsigned long long *const report = handle->rulebook_reports + slot;
+  const unsigned long long empty = stampedWord(~note.stamp, 0);
+  __atomic_store_n(report, empty, __ATOMIC_RELAXED);
   RulebookReportTarget t;
   t.stamp = note.stamp;
   // A captured rulebook files no report in host memory: nothing runs now, so no report of
@@ -27,8 +29,25 @@ RulebookReportTarget openRulebookNote(mluOpContext *handle, const void *pairs, i
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(handle->queue, &capturing) != hipSuccess) (void)hipGetLastError();
   if (capturing == hipStreamCaptureStatusNone) {
-    t.stamp_word = &handle->rulebook_reports[slot].stamp;
-    t.order_word = &handle->rulebook_reports[slot].rows_in_order;
+    t.order_word = report;
+    if (K <= mluOpContext::kCountWords) {
+      t.count_words = handle->count_words + (size_t)slot * mluOpContext::kCountWords;
+      for (int k = 0; k < K; ++k) __atomic_store_n(t.count_words + k, empty, __ATOMIC_RELAXED);
+      note.counts_on_file = true;
+    }
+  }
+  return t;
+}
+
+RulebookReportTarget rulebookReport(const mluOpContext *handle, const void *pairs, int K) {
+  RulebookReportTarget t;
+  for (int slot = 0; slot < mluOpContext::kRulebookNotes; ++slot) {
+    const mluOpContext::RulebookNote &note = handle->rulebook_notes[slot];
+    if (note.pairs != pairs || note.K != K || !note.counts_on_file) continue;
+    t.stamp = note.stamp;
+    t.order_word = handle->rulebook_reports + slot;
+    t.count_words = handle->count_words + (size_t)slot * mluOpContext::kCountWords;
+    break;
   }
   return t;
 }
@@ -44,13 +63,13 @@ void consultRulebookNotes(mluOpContext *handle, int row_column, ConvProblem *p) 
       p->list_trust = ListTrust::kInOrder;
       return;
     }
-    const volatile mluOpContext::RulebookReport *report = &handle->rulebook_reports[slot];
-    if (__atomic_load_n(&report->stamp, __ATOMIC_ACQUIRE) != note.stamp) {
+    const unsigned long long report = __atomic_load_n(handle->rulebook_reports + slot, __ATOMIC_ACQUIRE);
+    if (report >> 32 != (note.stamp & 0xffffffffull)) {
       // not arrived (or never sent: a captured rulebook files none)
       p->list_trust = ListTrust::kUnknown;
       return;
     }
-    p->list_trust = report->rows_in_order != 0 ? ListTrust::kInOrder : ListTrust::kNone;
+    p->list_trust = (uint32_t)report != 0 ? ListTrust::kInOrder : ListTrust::kNone;
     return;
   }
 }

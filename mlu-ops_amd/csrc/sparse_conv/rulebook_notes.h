@@ -13,6 +13,10 @@ namespace sparse_conv {
 // kernel reports to.
 RulebookReportTarget openRulebookNote(mluOpContext *handle, const void *pairs, int K, int L);
 
+// Where the rulebook this handle wrote to `pairs` reports to (count_words null: no counts of
+// such a rulebook are on file).
+RulebookReportTarget rulebookReport(const mluOpContext *handle, const void *pairs, int K);
+
 // Sets p->list_trust and p->ticket for a forward / backward-data launch whose result rows
 // are named by pair column `row_column`.  Column 0 of a rulebook this handle built ascends by
 // construction; column 1 does when the report says the input rows were in cell order.  A

@@ -126,6 +126,7 @@ SIGNATURES = {
     "mluOpExtSetKernelChoice": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int]),
     "mluOpExtSetSparseConvExtendedModes": (ctypes.c_int, [_vp, ctypes.c_int]),
     "mluOpExtSetDistinctPairsPromise": (ctypes.c_int, [_vp, ctypes.c_int]),
+    "mluOpExtGetIndicePairsHostCounts": (ctypes.c_int, [_vp, _vp, ctypes.c_int, _i64p]),
     "mluOpExtGetRowMapSize": (ctypes.c_int, [_vp, ctypes.c_int64, ctypes.POINTER(ctypes.c_size_t)]),
     "mluOpExtBuildRowMap": (ctypes.c_int, [_vp, _vp, _vp, ctypes.POINTER(ctypes.c_int64), ctypes.c_int64,
                                            ctypes.c_int64, ctypes.c_int, _vp, ctypes.c_size_t,
@@ -159,6 +160,22 @@ def lib():
     return _lib
 
 
+_native_module = None
+
+
+def native():
+    """The compiled host path (csrc/python/native.cpp), bound to the library lib() returns.  Raises if it
+    has not been built."""
+    global _native_module
+    if _native_module is None:
+        _torch()
+        lib()
+        from . import _native
+        _native.bind(LIB_PATH)
+        _native_module = _native
+    return _native_module
+
+
 class MluOpError(RuntimeError):
     def __init__(self, status, what):
         self.status = status
@@ -179,11 +196,20 @@ def _int_array(values, ctype=ctypes.c_int):
 class Handle:
     """mluOpHandle_t bound to the current device; `queue` is a raw hipStream_t."""
 
+    _owned = True
+
     def __init__(self, queue=None):
         self.ptr = _vp()
         check(lib().mluOpCreate(ctypes.byref(self.ptr)), "mluOpCreate")
         if queue is not None:
             self.set_queue(queue)
+
+    @classmethod
+    def borrowed(cls, address):
+        """A view of a handle that somebody else owns (close() leaves it alone)."""
+        h = cls.__new__(cls)
+        h.ptr, h._owned = _vp(address), False
+        return h
 
     def set_queue(self, queue):
         check(lib().mluOpSetQueue(self.ptr, _vp(queue)), "mluOpSetQueue")
@@ -222,7 +248,8 @@ class Handle:
 
     def close(self):
         if self.ptr:
-            lib().mluOpDestroy(self.ptr)
+            if self._owned:
+                lib().mluOpDestroy(self.ptr)
             self.ptr = _vp()
 
     def __del__(self):
@@ -335,6 +362,11 @@ GUARD_PATTERN = 0xA5
 _guard_state = threading.local()   # .bands: (whole buffer, payload bytes, what) of this thread's next call
 
 
+def _guarded():
+    """Whether the native path takes its buffers from _output and _workspace below."""
+    return GUARD_BYTES > 0 or WORKSPACE_SKEW > 0
+
+
 def _bands():
     if not hasattr(_guard_state, "bands"):
         _guard_state.bands = []
@@ -411,52 +443,23 @@ def _guards_intact(call):
 
 
 def get_indice_pairs(handle, indices, batch, input_space, filter_space, output_space, pad, stride,
-                     dilation, sub_m, out_rows=None, out_indices=None):
+                     dilation, sub_m, out_rows=None, out_indices=None, for_layer=False):
     """Builds the rulebook for `indices` (int32 [L, 4] device tensor).
 
     Returns (indice_pairs [K,2,L], out_indices [out_rows,4], indice_num [K] device int32,
     num_act_out).  In submanifold mode num_act_out is L.  Rows of out_indices from
     num_act_out on are -1: this wrapper allocates the tensor that way, the operator leaves
-    them alone (the reference decodes num_act_out rows, normal_get_indice_pairs.cpp:1143-1150)."""
-    torch = _torch()
-    L = indices.shape[0]
-    K = 1
-    for k in filter_space:
-        K *= int(k)
-    if out_rows is None:
-        if sub_m:
-            out_rows = L
-        else:
-            vol = batch
-            for o in output_space:
-                vol *= int(o)
-            out_rows = min(vol, K * L)
-    dev = indices.device
-    pairs = _output((K, 2, L), torch.int32, dev, "indice_pairs")
-    # the operator writes the first num_act_out rows only; the rest keep this initial -1
-    if out_indices is None:
-        out_indices = _output((out_rows, 4), torch.int32, dev, "out_indices", fill=-1)
-    else:
-        out_rows = out_indices.shape[0]
-    indice_num = _output((K,), torch.int32, dev, "indice_num")
-    desc = SparseConvDescriptor(batch, pad, stride, dilation, input_space, filter_space,
-                                output_space, sub_m)
-    d_in = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [L, 4])
-    d_pairs = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [K, 2, L])
-    d_out = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [out_rows, 4])
-    d_num = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [K])
-    size = ctypes.c_size_t(0)
-    check(lib().mluOpGetIndicePairsWorkspaceSize(handle.ptr, desc.ptr, d_in.ptr, d_pairs.ptr,
-                                                 d_out.ptr, d_num.ptr, ctypes.byref(size)),
-          "mluOpGetIndicePairsWorkspaceSize")
-    ws = _workspace(size.value, dev)
-    check(lib().mluOpGetIndicePairs(handle.ptr, desc.ptr, d_in.ptr, indices.data_ptr(),
-                                    ws.data_ptr(), size.value, d_pairs.ptr, pairs.data_ptr(),
-                                    d_out.ptr, out_indices.data_ptr(), d_num.ptr,
-                                    indice_num.data_ptr()), "mluOpGetIndicePairs")
-    _guards_intact("mluOpGetIndicePairs")
-    num_act_out = L if sub_m else desc.num_act_out()
-    return pairs, out_indices, indice_num, num_act_out
+    them alone (the reference decodes num_act_out rows, normal_get_indice_pairs.cpp:1143-1150).
+
+    `for_layer=True` is the form the convolution operators go on with: out_indices cut to its
+    num_act_out rows and indice_num as host ints, waited for without draining the queue."""
+    return native().get_indice_pairs(handle.ptr.value, _guarded(), indices, batch, _ints(input_space),
+                                     _ints(filter_space), _ints(output_space), _ints(pad), _ints(stride),
+                                     _ints(dilation), bool(sub_m), out_rows, out_indices, for_layer)
+
+
+def _ints(values):
+    return [int(v) for v in values]
 
 
 def _host_counts(indice_num):
@@ -494,6 +497,10 @@ class RowMap:
         """The next forward / backward-data call on the handle uses this map."""
         check(lib().mluOpExtUseRowMap(self.handle.ptr, self.buffer.data_ptr()), "mluOpExtUseRowMap")
 
+    def address(self):
+        """Where the map lies: what a call that is to use it announces to the library."""
+        return self.buffer.data_ptr()
+
     def close(self):
         if self.buffer is not None and self.handle.ptr:
             lib().mluOpExtForgetRowMap(self.handle.ptr, self.buffer.data_ptr())
@@ -510,60 +517,18 @@ def indice_conv_forward(handle, features, filters, filters_layout, indice_pairs,
                         num_act_out, sub_m, inverse=0, row_map=None):
     """features [L,Ci], filters 5-D in `filters_layout`, indice_num_host: K python ints.
     `row_map`: a usable RowMap built for this pair tensor and direction."""
-    torch = _torch()
-    code = torch_dtype_code(features.dtype)
-    K, _, L = indice_pairs.shape
-    if filters_layout == LAYOUT_ARRAY:
-        co = filters.shape[4]
-    else:
-        co = filters.shape[0]
-    out = _output((num_act_out, co), features.dtype, features.device, "features_out")
-    d_feat = _descriptor(LAYOUT_ARRAY, code, list(features.shape))
-    d_filt = _descriptor(filters_layout, code, list(filters.shape))
-    d_pairs = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [K, 2, L])
-    d_out = _descriptor(LAYOUT_ARRAY, code, [num_act_out, co])
-    counts = _host_counts(indice_num_host)
-    size = ctypes.c_size_t(0)
-    check(lib().mluOpGetIndiceConvolutionForwardWorkspaceSize(
-        handle.ptr, d_feat.ptr, d_filt.ptr, d_pairs.ptr, d_out.ptr, counts, num_act_out, inverse,
-        int(sub_m), ctypes.byref(size)), "mluOpGetIndiceConvolutionForwardWorkspaceSize")
-    ws = _workspace(size.value, features.device)
-    if row_map is not None:
-        row_map.announce()
-    check(lib().mluOpIndiceConvolutionForward(
-        handle.ptr, d_feat.ptr, features.data_ptr(), d_filt.ptr, filters.data_ptr(), d_pairs.ptr,
-        indice_pairs.data_ptr(), counts, num_act_out, inverse, int(sub_m), ws.data_ptr(),
-        size.value, d_out.ptr, out.data_ptr()), "mluOpIndiceConvolutionForward")
-    _guards_intact("mluOpIndiceConvolutionForward")
-    return out
+    return native().indice_conv_forward(handle.ptr.value, _guarded(), features, filters, filters_layout, indice_pairs,
+                                        _ints(indice_num_host), num_act_out, bool(sub_m), int(inverse),
+                                        0 if row_map is None else row_map.address())
 
 
 def indice_conv_backward_data(handle, output_grad, filters, filters_layout, indice_pairs,
                               indice_num_host, sub_m, ci, inverse=0, rows=None, row_map=None):
     """input_grad [rows, ci]; rows = indice_pairs.shape[2] unless the convolution is an inverse one."""
-    torch = _torch()
-    code = torch_dtype_code(output_grad.dtype)
-    K, _, L = indice_pairs.shape
-    rows = L if rows is None else int(rows)
-    dx = _output((rows, ci), output_grad.dtype, output_grad.device, "input_grad")
-    d_dy = _descriptor(LAYOUT_ARRAY, code, list(output_grad.shape))
-    d_filt = _descriptor(filters_layout, code, list(filters.shape))
-    d_pairs = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [K, 2, L])
-    d_dx = _descriptor(LAYOUT_ARRAY, code, [rows, ci])
-    counts = _host_counts(indice_num_host)
-    size = ctypes.c_size_t(0)
-    check(lib().mluOpGetIndiceConvolutionBackwardDataWorkspaceSize(
-        handle.ptr, d_dy.ptr, d_filt.ptr, d_pairs.ptr, d_dx.ptr, counts, inverse,
-        ctypes.byref(size)), "mluOpGetIndiceConvolutionBackwardDataWorkspaceSize")
-    ws = _workspace(size.value, output_grad.device)
-    if row_map is not None:
-        row_map.announce()
-    check(lib().mluOpIndiceConvolutionBackwardData(
-        handle.ptr, d_dy.ptr, output_grad.data_ptr(), d_filt.ptr, filters.data_ptr(), d_pairs.ptr,
-        indice_pairs.data_ptr(), counts, inverse, int(sub_m), ws.data_ptr(), size.value, d_dx.ptr,
-        dx.data_ptr()), "mluOpIndiceConvolutionBackwardData")
-    _guards_intact("mluOpIndiceConvolutionBackwardData")
-    return dx
+    rows = indice_pairs.shape[2] if rows is None else int(rows)
+    return native().indice_conv_backward_data(handle.ptr.value, _guarded(), output_grad, filters, filters_layout,
+                                              indice_pairs, _ints(indice_num_host), bool(sub_m), ci, int(inverse),
+                                              rows, 0 if row_map is None else row_map.address())
 
 
 def indice_conv_backward_filter(handle, features, output_grad, indice_pairs, indice_num_host,
@@ -571,34 +536,9 @@ def indice_conv_backward_filter(handle, features, output_grad, indice_pairs, ind
                                 grad_layout=LAYOUT_ARRAY):
     """Returns filters_grad laid out [kd, kh, kw, Ci, Co]; with the handle's extended modes on,
     grad_layout NDHWC gives [Co, kd, kh, kw, Ci] and NCDHW [Co, Ci, kd, kh, kw]."""
-    torch = _torch()
-    code = torch_dtype_code(features.dtype)
-    K, _, L = indice_pairs.shape
-    ci, co = features.shape[1], output_grad.shape[1]
-    if grad_layout in (LAYOUT_NDHWC, LAYOUT_NHWC):
-        shape = (co,) + tuple(filter_space) + (ci,)
-    elif grad_layout in (LAYOUT_NCDHW, LAYOUT_NCHW):
-        shape = (co, ci) + tuple(filter_space)
-    else:
-        shape = tuple(filter_space) + (ci, co)
-    dw = _output(shape, features.dtype, features.device, "filters_grad")
-    d_x = _descriptor(LAYOUT_ARRAY, code, list(features.shape))
-    d_dy = _descriptor(LAYOUT_ARRAY, code, list(output_grad.shape))
-    d_pairs = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [K, 2, L])
-    d_dw = _descriptor(grad_layout, code, list(dw.shape),
-                            onchip_dtype=DTYPE_FLOAT if onchip_float else None)
-    counts = _host_counts(indice_num_host)
-    size = ctypes.c_size_t(0)
-    check(lib().mluOpGetIndiceConvolutionBackwardFilterWorkspaceSize(
-        handle.ptr, d_x.ptr, d_dy.ptr, d_pairs.ptr, d_dw.ptr, counts, inverse, int(sub_m),
-        ctypes.byref(size)), "mluOpGetIndiceConvolutionBackwardFilterWorkspaceSize")
-    ws = _workspace(size.value, features.device)
-    check(lib().mluOpIndiceConvolutionBackwardFilter(
-        handle.ptr, d_x.ptr, features.data_ptr(), d_dy.ptr, output_grad.data_ptr(), d_pairs.ptr,
-        indice_pairs.data_ptr(), counts, inverse, int(sub_m), ws.data_ptr(), size.value, d_dw.ptr,
-        dw.data_ptr()), "mluOpIndiceConvolutionBackwardFilter")
-    _guards_intact("mluOpIndiceConvolutionBackwardFilter")
-    return dw
+    return native().indice_conv_backward_filter(handle.ptr.value, _guarded(), features, output_grad, indice_pairs,
+                                                _ints(indice_num_host), _ints(filter_space), bool(sub_m),
+                                                int(inverse), bool(onchip_float), grad_layout)
 
 
 NO_ALLOC_SCRATCH_BYTES = 16 * 1024 * 1024  # MLUOP_EXT_NO_ALLOC_SCRATCH_BYTES
@@ -624,39 +564,17 @@ def indice_conv_backward_filter_no_alloc(handle, features, output_grad, indice_p
     return filters_grad
 
 
+_REDUCE_MODES = {"max": REDUCE_DMAX, "mean": REDUCE_DMEAN, "sum": REDUCE_DSUM}
+
+
 def voxelization(handle, points, voxel_size, coors_range, max_points, max_voxels, deterministic=True):
     """Hard voxelization of `points` [N, F] (float32 device tensor; x, y, z first).
 
     voxel_size [3] and coors_range [6] are float32 device tensors.  Returns (voxels
     [max_voxels, max_points, F], coors [max_voxels, 3] int32 (z, y, x), num_points_per_voxel
     [max_voxels] int32, voxel_num [1] int32), all on the device."""
-    torch = _torch()
-    n, f = points.shape
-    dev = points.device
-    voxels = _output((max_voxels, max_points, f), torch.float32, dev, "voxels")
-    coors = _output((max_voxels, 3), torch.int32, dev, "coors")
-    npv = _output((max_voxels,), torch.int32, dev, "num_points_per_voxel")
-    voxel_num = torch.zeros((1,), dtype=torch.int32, device=dev)
-    d_points = _descriptor(LAYOUT_ARRAY, DTYPE_FLOAT, [n, f])
-    d_vs = _descriptor(LAYOUT_ARRAY, DTYPE_FLOAT, [3])
-    d_cr = _descriptor(LAYOUT_ARRAY, DTYPE_FLOAT, [6])
-    d_voxels = _descriptor(LAYOUT_ARRAY, DTYPE_FLOAT, [max_voxels, max_points, f])
-    d_coors = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [max_voxels, 3])
-    d_npv = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [max_voxels])
-    d_num = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [1])
-    size = ctypes.c_size_t(0)
-    check(lib().mluOpGetVoxelizationWorkspaceSize(
-        handle.ptr, d_points.ptr, d_vs.ptr, d_cr.ptr, max_points, max_voxels, 3, bool(deterministic),
-        d_voxels.ptr, d_coors.ptr, d_npv.ptr, d_num.ptr, ctypes.byref(size)),
-        "mluOpGetVoxelizationWorkspaceSize")
-    ws = _workspace(size.value, dev)
-    check(lib().mluOpVoxelization(
-        handle.ptr, d_points.ptr, points.data_ptr(), d_vs.ptr, voxel_size.data_ptr(), d_cr.ptr,
-        coors_range.data_ptr(), max_points, max_voxels, 3, bool(deterministic), ws.data_ptr(), size.value,
-        d_voxels.ptr, voxels.data_ptr(), d_coors.ptr, coors.data_ptr(), d_npv.ptr, npv.data_ptr(), d_num.ptr,
-        voxel_num.data_ptr()), "mluOpVoxelization")
-    _guards_intact("mluOpVoxelization")
-    return voxels, coors, npv, voxel_num
+    return tuple(native().voxelization(handle.ptr.value, _guarded(), points, voxel_size, coors_range, max_points,
+                                       max_voxels, bool(deterministic)))
 
 
 def dynamic_point_to_voxel_forward(handle, feats, coors, reduce_type="max", rows=None):
@@ -665,61 +583,14 @@ def dynamic_point_to_voxel_forward(handle, feats, coors, reduce_type="max", rows
     feats [N, C] float32 and coors [N, 3] int32 are device tensors; coors is modified in place
     (rows with a negative coordinate become -1,-1,-1).  Returns (voxel_feats [rows, C], voxel_coors
     [rows, 3], point2voxel_map [N], voxel_points_count [rows], voxel_num [1]); rows defaults to N."""
-    torch = _torch()
-    n, c = feats.shape
-    m = n if rows is None else int(rows)
-    dev = feats.device
-    voxel_feats = _output((m, c), torch.float32, dev, "voxel_feats")
-    voxel_coors = _output((m, 3), torch.int32, dev, "voxel_coors")
-    p2v = _output((n,), torch.int32, dev, "point2voxel_map")
-    count = _output((m,), torch.int32, dev, "voxel_points_count")
-    voxel_num = torch.zeros((1,), dtype=torch.int32, device=dev)
-    mode = {"max": REDUCE_DMAX, "mean": REDUCE_DMEAN, "sum": REDUCE_DSUM}[reduce_type]
-    d_feats = _descriptor(LAYOUT_ARRAY, DTYPE_FLOAT, [n, c])
-    d_coors = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [n, 3])
-    d_vf = _descriptor(LAYOUT_ARRAY, DTYPE_FLOAT, [m, c])
-    d_vc = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [m, 3])
-    d_p2v = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [n])
-    d_cnt = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [m])
-    d_num = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [1])
-    size = ctypes.c_size_t(0)
-    check(lib().mluOpGetDynamicPointToVoxelForwardWorkspaceSize(handle.ptr, d_feats.ptr, d_coors.ptr,
-                                                                ctypes.byref(size)),
-          "mluOpGetDynamicPointToVoxelForwardWorkspaceSize")
-    ws = _workspace(size.value, dev)
-    check(lib().mluOpDynamicPointToVoxelForward(
-        handle.ptr, mode, d_feats.ptr, feats.data_ptr(), d_coors.ptr, coors.data_ptr(), ws.data_ptr(),
-        size.value, d_vf.ptr, voxel_feats.data_ptr(), d_vc.ptr, voxel_coors.data_ptr(), d_p2v.ptr,
-        p2v.data_ptr(), d_cnt.ptr, count.data_ptr(), d_num.ptr, voxel_num.data_ptr()),
-        "mluOpDynamicPointToVoxelForward")
-    _guards_intact("mluOpDynamicPointToVoxelForward")
-    return voxel_feats, voxel_coors, p2v, count, voxel_num
+    return tuple(native().dynamic_point_to_voxel_forward(handle.ptr.value, _guarded(), feats, coors,
+                                                         _REDUCE_MODES[reduce_type],
+                                                         feats.shape[0] if rows is None else int(rows)))
 
 
 def dynamic_point_to_voxel_backward(handle, grad_voxel_feats, feats, voxel_feats, point2voxel_map,
                                     voxel_points_count, voxel_num, reduce_type="max"):
     """Gradient of `dynamic_point_to_voxel_forward(..., "max")` with respect to feats: [N, C]."""
-    torch = _torch()
-    n, c = feats.shape
-    m = grad_voxel_feats.shape[0]
-    grad_feats = _output((n, c), torch.float32, feats.device, "grad_feats")
-    mode = {"max": REDUCE_DMAX, "mean": REDUCE_DMEAN, "sum": REDUCE_DSUM}[reduce_type]
-    d_g = _descriptor(LAYOUT_ARRAY, DTYPE_FLOAT, [m, c])
-    d_feats = _descriptor(LAYOUT_ARRAY, DTYPE_FLOAT, [n, c])
-    d_vf = _descriptor(LAYOUT_ARRAY, DTYPE_FLOAT, [m, c])
-    d_p2v = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [n])
-    d_cnt = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [m])
-    d_num = _descriptor(LAYOUT_ARRAY, DTYPE_INT32, [1])
-    d_out = _descriptor(LAYOUT_ARRAY, DTYPE_FLOAT, [n, c])
-    size = ctypes.c_size_t(0)
-    check(lib().mluOpGetDynamicPointToVoxelBackwardWorkspaceSize(
-        handle.ptr, mode, d_g.ptr, d_feats.ptr, d_vf.ptr, d_p2v.ptr, d_cnt.ptr, d_num.ptr, ctypes.byref(size)),
-        "mluOpGetDynamicPointToVoxelBackwardWorkspaceSize")
-    ws = _workspace(size.value, feats.device)
-    check(lib().mluOpDynamicPointToVoxelBackward(
-        handle.ptr, mode, d_g.ptr, grad_voxel_feats.data_ptr(), d_feats.ptr, feats.data_ptr(), d_vf.ptr,
-        voxel_feats.data_ptr(), d_p2v.ptr, point2voxel_map.data_ptr(), d_cnt.ptr,
-        voxel_points_count.data_ptr(), d_num.ptr, voxel_num.data_ptr(), ws.data_ptr(), size.value, d_out.ptr,
-        grad_feats.data_ptr()), "mluOpDynamicPointToVoxelBackward")
-    _guards_intact("mluOpDynamicPointToVoxelBackward")
-    return grad_feats
+    return native().dynamic_point_to_voxel_backward(handle.ptr.value, _guarded(), grad_voxel_feats, feats, voxel_feats,
+                                                    point2voxel_map, voxel_points_count, voxel_num,
+                                                    _REDUCE_MODES[reduce_type])

@@ -16,19 +16,18 @@ import math
 
 import torch
 
-from . import (LAYOUT_ARRAY, RowMap, get_indice_pairs, indice_conv_backward_data, indice_conv_backward_filter,
-               indice_conv_forward, make_handle_on_current_stream, regular_output_space, voxelization)
+from . import Handle, RowMap, _guarded, get_indice_pairs, native, regular_output_space, voxelization
 
 _handles = {}
 
 
 def _handle():
-    """One library handle per (device, stream): a handle is used from one stream at a time."""
-    key = (torch.cuda.current_device(), torch.cuda.current_stream().cuda_stream)
-    if key not in _handles:
-        _handles[key] = make_handle_on_current_stream()
-        _handles[key].set_extended_modes(True)  # SparseInverseConv3d runs the operators with inverse = 1
-    return _handles[key]
+    """The library handle of the current device and stream (made by the native path, which keeps one for
+    each: a handle is used from one stream at a time)."""
+    address = native().stream_handle()
+    if address not in _handles:
+        _handles[address] = Handle.borrowed(address)
+    return _handles[address]
 
 
 _share_row_maps = False
@@ -64,6 +63,19 @@ class Rulebook:
         self.sub_m = sub_m
         self.out_space = tuple(out_space)
         self._row_maps = {}
+        self._for_operators = None
+
+    def for_operators(self, needs_grad, inverse):
+        """What the native operators take of this rulebook, with the shared row maps it is to use."""
+        if self._for_operators is None:
+            self._for_operators = native().LayerRulebook(self.pairs, self.indice_num, self.num_act_out,
+                                                         list(self.filter_space), self.sub_m, self.distinct)
+        if _share_row_maps or self._row_maps:
+            handle = _handle()
+            for column in (0, 1):
+                m = self.row_map(handle, column) if needs_grad or column == (0 if inverse else 1) else None
+                self._for_operators.set_row_map(column, None if m is None else m.buffer)
+        return self._for_operators
 
     def row_map(self, handle, row_column):
         """The [K, rows] row map of this rulebook for one direction (row_column 1: rows are the
@@ -78,6 +90,7 @@ class Rulebook:
             rows, source_rows = (self.num_act_out, L) if row_column == 1 else (L, self.num_act_out)
             # the coordinates are known to be distinct and the handle carries that promise: the
             # build need not count lost pairs, which would make the host wait for the stream
+            handle.promise_distinct_pairs(True)
             m = RowMap(handle, self.pairs, self.indice_num, rows, source_rows, row_column, verify=False)
             self._row_maps[key] = m if m.usable else None
         return self._row_maps[key]
@@ -112,45 +125,13 @@ class SparseTensor:
         return out.permute(0, 4, 1, 2, 3).contiguous()
 
 
-class _IndiceConv(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, features, weight, rulebook, inverse=False):
-        handle = _handle()
-        features = features.contiguous()
-        weight = weight.contiguous()
-        handle.promise_distinct_pairs(rulebook.distinct)
-        if inverse:
-            # the partner layer's rulebook backwards: one output row per input row of the partner
-            out = indice_conv_forward(handle, features, weight, LAYOUT_ARRAY, rulebook.pairs, rulebook.indice_num,
-                                      rulebook.pairs.shape[2], False, inverse=1,
-                                      row_map=rulebook.row_map(handle, 0))
-        else:
-            out = indice_conv_forward(handle, features, weight, LAYOUT_ARRAY, rulebook.pairs,
-                                      rulebook.indice_num, rulebook.num_act_out, rulebook.sub_m,
-                                      row_map=rulebook.row_map(handle, 1))
-        ctx.save_for_backward(features, weight)
-        ctx.rulebook = rulebook
-        ctx.inverse = inverse
-        return out
+class _IndiceConv:
+    """The layers' differentiable convolution; its autograd node is native (csrc/python/native.cpp)."""
 
     @staticmethod
-    def backward(ctx, grad_out):
-        features, weight = ctx.saved_tensors
-        rb = ctx.rulebook
-        handle = _handle()
-        handle.promise_distinct_pairs(rb.distinct)
-        grad_out = grad_out.contiguous()
-        grad_features = grad_weight = None
-        inverse, sub_m = (1, False) if ctx.inverse else (0, rb.sub_m)
-        if ctx.needs_input_grad[0]:
-            grad_features = indice_conv_backward_data(handle, grad_out, weight, LAYOUT_ARRAY, rb.pairs,
-                                                      rb.indice_num, sub_m, features.shape[1], inverse=inverse,
-                                                      rows=features.shape[0],
-                                                      row_map=rb.row_map(handle, 1 if ctx.inverse else 0))
-        if ctx.needs_input_grad[1]:
-            grad_weight = indice_conv_backward_filter(handle, features, grad_out, rb.pairs, rb.indice_num,
-                                                      rb.filter_space, sub_m, inverse=inverse)
-        return grad_features, grad_weight, None, None
+    def apply(features, weight, rulebook, inverse=False):
+        needs_grad = torch.is_grad_enabled() and (features.requires_grad or weight.requires_grad)
+        return native().indice_conv(features, weight, rulebook.for_operators(needs_grad, inverse), inverse, _guarded())
 
 
 def _mfma_channels(c):
@@ -196,11 +177,11 @@ class _ConvBase(torch.nn.Module):
         else:
             out_space = regular_output_space(x.spatial_shape, self.kernel_size, self.padding, self.stride,
                                              self.dilation)
+        # the operators take indice_num as host ints: one wait per rulebook
         pairs, out_indices, num, n_out = get_indice_pairs(
             _handle(), x.indices, x.batch_size, x.spatial_shape, self.kernel_size, out_space, self.padding,
-            self.stride, self.dilation, self.sub_m)
-        # the operators take indice_num as host int64: one device-to-host copy per rulebook
-        rb = Rulebook(pairs, out_indices[:n_out], num.cpu().tolist(), n_out, self.kernel_size, self.sub_m,
+            self.stride, self.dilation, self.sub_m, for_layer=True)
+        rb = Rulebook(pairs, out_indices, num, n_out, self.kernel_size, self.sub_m,
                       out_space, in_indices=x.indices, in_space=x.spatial_shape, distinct=x.distinct)
         if self.indice_key is not None:
             x.rulebooks[self.indice_key] = rb
