@@ -60,6 +60,9 @@ __device__ __forceinline__ void requestToLds(const void *global, uint32_t lds_ad
 }
 constexpr int kMaxInlineK = 128;
 
+// What a lane without a row of its own loads: a row of zeros in device memory.
+__device__ __attribute__((aligned(256))) unsigned char kZeroRow[512];  // never written
+
 // Pair counts per offset, passed by value for the common small kernel volumes.
 struct OffsetCounts {
   int n[kMaxInlineK];
@@ -292,46 +295,92 @@ __global__ __launch_bounds__(256) void gatherConvSimt(const typename E::storage 
 // for float):
 // packed[(((k*(C/16) + nb)*(Q/CHUNK) + kb)*64 + lane)*VEC + e]
 //   = B(k, q = kb*CHUNK + VEC*(lane/16) + e, c = nb*16 + lane%16), zero for q >= Q
-// (16 reduction channels of a 2-byte type fill half a fragment).
+// (16 reduction channels of a 2-byte type fill half a fragment) and for columns beyond the
+// filter's own: a filter of q x c channels runs on the instance of the next padded size.
 // One launch for the two independent preparations of the MFMA path: blocks
 // below fill_blocks set the row map to -1 (16-byte stores), the others repack
 // the filter.
+// Channels of a filter B(k, q, c) as they are, and as the kernel instance counts them.
+struct FilterShape {
+  int q, c;
+  int q_padded, c_padded;
+};
+
 template <typename E>
-__global__ __launch_bounds__(256) void fillMapPackFilter(int32_t *map, size_t map_elems,
-                                                         int fill_blocks,
-                                                         const typename E::storage *W, int64_t sK,
-                                                         int64_t sQ, int64_t sC, int K, int Q,
-                                                         int C, typename E::storage *packed,
-                                                         RunIf run_if) {
-  if (notWanted(run_if)) return;
-  if ((int)blockIdx.x < fill_blocks) {
-    const size_t quads = map_elems / 4;
-    int4 *dst = reinterpret_cast<int4 *>(map);
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < quads;
-         i += (size_t)fill_blocks * 256)
-      dst[i] = make_int4(-1, -1, -1, -1);
-    if (blockIdx.x == 0 && threadIdx.x < (map_elems & 3)) map[quads * 4 + threadIdx.x] = -1;
-    return;
-  }
-  const int pack_blocks = gridDim.x - fill_blocks;
+__device__ __forceinline__ void packFilter(const typename E::storage *W, int64_t sK, int64_t sQ, int64_t sC, int K,
+                                           const FilterShape &shape, typename E::storage *packed, int block,
+                                           int blocks) {
   constexpr int VEC = E::kVec, CHUNK = E::kChunk;
-  const int chunks = (Q + CHUNK - 1) / CHUNK;  // Q below one fragment is padded with zeros
-  const size_t total = (size_t)K * (C / 16) * chunks * 64;
-  for (size_t t = (size_t)(blockIdx.x - fill_blocks) * 256 + threadIdx.x; t < total;
-       t += (size_t)pack_blocks * 256) {
+  const int chunks = (shape.q_padded + CHUNK - 1) / CHUNK;
+  const int groups = shape.c_padded / 16;
+  const size_t total = (size_t)K * groups * chunks * 64;
+  for (size_t t = (size_t)block * 256 + threadIdx.x; t < total; t += (size_t)blocks * 256) {
     const int lane = (int)(t & 63);
     size_t rest = t >> 6;
     const int kb = (int)(rest % chunks);
     rest /= chunks;
-    const int nb = (int)(rest % (C / 16));
-    const int k = (int)(rest / (C / 16));
+    const int nb = (int)(rest % groups);
+    const int k = (int)(rest / groups);
     const int c = nb * 16 + (lane & 15);
     const int qb = kb * CHUNK + VEC * (lane >> 4);
 #pragma unroll
     for (int e = 0; e < VEC; ++e)
-      packed[t * VEC + e] =
-          qb + e < Q ? W[(size_t)k * sK + (size_t)(qb + e) * sQ + (size_t)c * sC] : typename E::storage(0);
+      packed[t * VEC + e] = qb + e < shape.q && c < shape.c
+                                ? W[(size_t)k * sK + (size_t)(qb + e) * sQ + (size_t)c * sC]
+                                : typename E::storage(0);
   }
+}
+
+// Rows of `bytes` bytes copied to rows of `padded_bytes` (zeros behind), by the first `blocks`
+// workgroups of a launch.
+struct PadRows {
+  const char *from;
+  char *to;
+  int bytes, padded_bytes;
+  int rows;
+  int blocks;
+};
+
+// Element: what the row length is a multiple of.
+template <typename ELEM>
+__device__ __forceinline__ void padRows(const PadRows &pad) {
+  const int pieces = pad.padded_bytes / 16;
+  const size_t total = (size_t)pad.rows * pieces;
+  constexpr int N = 16 / (int)sizeof(ELEM);
+  for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < total; t += (size_t)pad.blocks * 256) {
+    const size_t row = t / pieces;
+    const int at = (int)(t % pieces) * 16;
+    const ELEM *src = reinterpret_cast<const ELEM *>(pad.from + row * pad.bytes + at);
+    ELEM v[N];
+#pragma unroll
+    for (int e = 0; e < N; ++e) v[e] = at + e * (int)sizeof(ELEM) < pad.bytes ? src[e] : ELEM(0);
+    *reinterpret_cast<uint4 *>(pad.to + row * pad.padded_bytes + at) = *reinterpret_cast<const uint4 *>(v);
+  }
+}
+
+template <typename E>
+__global__ __launch_bounds__(256) void fillMapPackFilter(PadRows pad, int32_t *map, size_t map_elems,
+                                                         int fill_blocks,
+                                                         const typename E::storage *W, int64_t sK,
+                                                         int64_t sQ, int64_t sC, int K,
+                                                         FilterShape shape,
+                                                         typename E::storage *packed, RunIf run_if) {
+  if (notWanted(run_if)) return;
+  if ((int)blockIdx.x < pad.blocks) {
+    padRows<typename E::storage>(pad);
+    return;
+  }
+  const int block = (int)blockIdx.x - pad.blocks;
+  if (block < fill_blocks) {
+    const size_t quads = map_elems / 4;
+    int4 *dst = reinterpret_cast<int4 *>(map);
+    for (size_t i = (size_t)block * 256 + threadIdx.x; i < quads; i += (size_t)fill_blocks * 256)
+      dst[i] = make_int4(-1, -1, -1, -1);
+    if (block == 0 && threadIdx.x < (map_elems & 3)) map[quads * 4 + threadIdx.x] = -1;
+    return;
+  }
+  packFilter<E>(W, sK, sQ, sC, K, shape, packed, block - fill_blocks,
+                (int)gridDim.x - pad.blocks - fill_blocks);
 }
 
 // ---- where a gather kernel finds the pairs of its tile -------------------------------
@@ -375,7 +424,7 @@ struct SegmentSource {
 // bits.  It is slow and runs only when a pair tensor was changed
 // after the library had seen it in order.
 template <typename E, int NT>
-__device__ __forceinline__ void scanAllPairsForTile(const typename E::storage *A, int Q,
+__device__ __forceinline__ void scanAllPairsForTile(const typename E::storage *A, int Q, int row_bytes,
                                                     const SegmentSource &src, int K, int r_begin,
                                                     int r_end, int C, int col0, float *acc,
                                                     int acc_stride) {
@@ -399,7 +448,8 @@ __device__ __forceinline__ void scanAllPairsForTile(const typename E::storage *A
         const int from = __ffsll((long long)m) - 1;
         m &= m - 1;
         const int rr = __shfl(r, from, kWave) - r_begin;
-        const typename E::storage *a = A + (size_t)__shfl(g, from, kWave) * Q;
+        const typename E::storage *a = reinterpret_cast<const typename E::storage *>(
+            reinterpret_cast<const char *>(A) + (size_t)__shfl(g, from, kWave) * row_bytes);
         for (int c = lane; c < C; c += kWave) {
           const typename E::storage *w = W + (size_t)k * src.sK + (size_t)(col0 + c) * src.sC;
           float dot = 0.f;
@@ -427,32 +477,19 @@ constexpr int kCutPairsPerThread = 4;
 
 template <typename E>
 __global__ __launch_bounds__(256) void packFilterCutPairLists(
-    const typename E::storage *W, int64_t sK, int64_t sQ, int64_t sC, int K, int Q, int C,
+    PadRows pad, const typename E::storage *W, int64_t sK, int64_t sQ, int64_t sC, int K, FilterShape shape,
     typename E::storage *packed, int pack_blocks, const int32_t *pairs, int L, OffsetCounts inl,
     OffsetBlocks blocks, int row_col, int src_col, int R, int n_src, int tile_shift, int n_tiles,
     int32_t *cuts, unsigned long long *verdict, unsigned long long ticket) {
-  if ((int)blockIdx.x < pack_blocks) {
-    constexpr int VEC = E::kVec, CHUNK = E::kChunk;
-    const int chunks = (Q + CHUNK - 1) / CHUNK;
-    const size_t total = (size_t)K * (C / 16) * chunks * 64;
-    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < total;
-         t += (size_t)pack_blocks * 256) {
-      const int lane = (int)(t & 63);
-      size_t rest = t >> 6;
-      const int kb = (int)(rest % chunks);
-      rest /= chunks;
-      const int nb = (int)(rest % (C / 16));
-      const int k = (int)(rest / (C / 16));
-      const int c = nb * 16 + (lane & 15);
-      const int qb = kb * CHUNK + VEC * (lane >> 4);
-#pragma unroll
-      for (int e = 0; e < VEC; ++e)
-        packed[t * VEC + e] =
-            qb + e < Q ? W[(size_t)k * sK + (size_t)(qb + e) * sQ + (size_t)c * sC] : typename E::storage(0);
-    }
+  if ((int)blockIdx.x < pad.blocks) {
+    padRows<typename E::storage>(pad);
     return;
   }
-  const int b = (int)blockIdx.x - pack_blocks;
+  if ((int)blockIdx.x - pad.blocks < pack_blocks) {
+    packFilter<E>(W, sK, sQ, sC, K, shape, packed, (int)blockIdx.x - pad.blocks, pack_blocks);
+    return;
+  }
+  const int b = (int)blockIdx.x - pad.blocks - pack_blocks;
   int lo = 0, hi = K - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -543,8 +580,37 @@ constexpr int mfmaBatchBlocks(int elem_bytes, int Q, int C) {
   return g < 1 ? 1 : (g > 4 ? 4 : g);
 }
 
-// Workgroup = TR result rows x C columns (column group blockIdx.y of the ldc
-// result columns), WAVES multiplying waves and as many fetching waves.
+// The rows a gather kernel reads and writes, in their own channel counts: an instance is
+// compiled for padded counts, reads nothing behind a row's own bytes (a piece of 16 bytes that
+// is not there is zero) and writes the result's own columns only.
+struct ConvRows {
+  int q;          // reduction channels
+  int row_bytes;  // bytes from one gathered row to the next: a multiple of 16, all of them readable
+  int c;          // result columns
+  int c_padded;   // result columns of the packed filter
+};
+
+// `VALS` consecutive result values of one row from column `col` on, as many as the row has.
+template <typename E, int VALS>
+__device__ __forceinline__ void storeColumns(typename E::storage *row, int col, int columns,
+                                             const typename E::storage (&v)[VALS]) {
+  typedef typename E::storage S;
+  constexpr int BYTES = VALS * (int)sizeof(S);
+  static_assert(BYTES == 8 || BYTES == 16, "one store");
+  if (col + VALS <= columns && columns % VALS == 0) {
+    if constexpr (BYTES == 8)
+      *reinterpret_cast<uint2 *>(row + col) = *reinterpret_cast<const uint2 *>(v);
+    else
+      *reinterpret_cast<uint4 *>(row + col) = *reinterpret_cast<const uint4 *>(v);
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < VALS; ++e)
+    if (col + e < columns) row[col + e] = v[e];
+}
+
+// Workgroup = TR result rows x C columns (column group blockIdx.y of the
+// result's columns), WAVES multiplying waves and as many fetching waves.
 // Multiplying wave w owns columns [w*16*NB, (w+1)*16*NB) of the
 // fp32 accumulator tile in LDS, so no two waves ever touch the same accumulator
 // element and every element sees its contributions in ascending offset order.
@@ -574,8 +640,8 @@ constexpr int mfmaBatchBlocks(int elem_bytes, int Q, int C) {
 template <typename E, int Q, int C, typename SRC>
 __global__ __launch_bounds__(mfmaThreads(C)) __attribute__((amdgpu_waves_per_eu(mfmaWavesPerSimd((int)sizeof(typename E::storage), Q, C),
                                    mfmaWavesPerSimd((int)sizeof(typename E::storage), Q, C))))
-void gatherConvMfma(const typename E::storage *A, const typename E::storage *packedW,
-                    SRC source, int R, int K, int ldc, typename E::storage *result) {
+void gatherConvMfma(const typename E::storage *A, ConvRows rows, const typename E::storage *packedW,
+                    SRC source, int R, int K, typename E::storage *result) {
   typedef typename E::vec8 vec8;
   typedef typename E::storage S;
   constexpr int NB = mfmaColBlocksPerWave(C);
@@ -641,18 +707,19 @@ void gatherConvMfma(const typename E::storage *A, const typename E::storage *pac
     if (!in_order && source.leave_if_unordered) return;
     if (!in_order) {
       __syncthreads();
-      scanAllPairsForTile<E, NT>(A, Q, source, K, r0, r0 + TR < R ? r0 + TR : R, C, blockIdx.y * C,
-                                 s_acc, ACC_STRIDE);
+      const int columns = rows.c - (int)blockIdx.y * C;
+      scanAllPairsForTile<E, NT>(A, rows.q, rows.row_bytes, source, K, r0, r0 + TR < R ? r0 + TR : R,
+                                 columns < C ? columns : C, blockIdx.y * C, s_acc, ACC_STRIDE);
     }
   }
 
   // per-lane constants of the multiply phase
   const char *a_bytes = reinterpret_cast<const char *>(A);
-  // the workgroup owns result columns [blockIdx.y*C, (blockIdx.y+1)*C) of ldc
+  // the workgroup owns result columns [blockIdx.y*C, (blockIdx.y+1)*C)
   const int col_group = blockIdx.y;
   const char *b_base = reinterpret_cast<const char *>(packedW) +
                        ((size_t)(col_group * GROUPS + wave * NB) * KB * 64 + lane) * 16;
-  const uint32_t kBytesPerOffset = (uint32_t)(ldc / 16) * KB * 64 * 16;  // packed W[k]
+  const uint32_t kBytesPerOffset = (uint32_t)(rows.c_padded / 16) * KB * 64 * 16;  // packed W[k]
   const int pair = lane & 15;
   const int quad = lane >> 4;
   char *acc_lane = reinterpret_cast<char *>(s_acc) + (wave * 16 * NB + 4 * quad) * 4;
@@ -791,8 +858,10 @@ void gatherConvMfma(const typename E::storage *A, const typename E::storage *pac
             int ci = round * STEP + p / PPR;
             ci = ci < total ? ci : total - 1;
             const uint32_t src = s_ent[ci] >> 8;
-            piece[i] = *reinterpret_cast<const u32x4 *>(a_bytes + (size_t)src * ROW_BYTES +
-                                                        (p % PPR) * 16);
+            const int at = (p % PPR) * 16;
+            piece[i] = *reinterpret_cast<const u32x4 *>(
+                at < rows.row_bytes ? a_bytes + (size_t)src * rows.row_bytes + at
+                                    : reinterpret_cast<const char *>(kZeroRow));
           }
           if (round > 0) __syncthreads();  // the multiplying waves have left the stage
 #pragma unroll
@@ -905,16 +974,12 @@ void gatherConvMfma(const typename E::storage *A, const typename E::storage *pac
     S tmp[VALS];
 #pragma unroll
     for (int e = 0; e < VALS; ++e) E::store(&tmp[e], s_acc[rr * ACC_STRIDE + c0 + e]);
-    *reinterpret_cast<uint4 *>(result + (size_t)(r0 + rr) * ldc + col_group * C + c0) =
-        *reinterpret_cast<const uint4 *>(tmp);
+    storeColumns<E>(result + (size_t)(r0 + rr) * rows.c, col_group * C + c0, rows.c, tmp);
   }
   if constexpr (!SRC::kSegments) {
     if (tid == 0 && blockIdx.y == 0) source.filled[blockIdx.x] = slots;
   }
 }
-
-// What a lane without a row of its own loads: a row of zeros in device memory.
-__device__ __attribute__((aligned(256))) unsigned char kZeroRow[512];  // never written
 
 // ---- MFMA gather convolution, one free-running wavefront per tile ---------------------
 //
@@ -945,8 +1010,8 @@ constexpr bool waveKernelShape(int elem_bytes, int Q, int C) {
 }
 template <typename E, int Q, int C>
 __global__ __launch_bounds__(64) void gatherConvWave(
-    const typename E::storage *A, const typename E::storage *packedW, SegmentSource source, int R,
-    int K, typename E::storage *result) {
+    const typename E::storage *A, ConvRows conv, const typename E::storage *packedW, SegmentSource source,
+    int R, int K, typename E::storage *result) {
   typedef typename E::vec8 vec8;
   typedef typename E::storage S;
   constexpr int NB = C / 16;                            // column blocks
@@ -1000,13 +1065,14 @@ __global__ __launch_bounds__(64) void gatherConvWave(
       S tmp[VALS];
 #pragma unroll
       for (int e = 0; e < VALS; ++e) E::store(&tmp[e], s_acc[rr * ACC_STRIDE + c0 + e]);
-      *reinterpret_cast<uint4 *>(result + (size_t)(r0 + rr) * C + c0) = *reinterpret_cast<const uint4 *>(tmp);
+      storeColumns<E>(result + (size_t)(r0 + rr) * conv.c, c0, conv.c, tmp);
     }
   };
   if (verdict == source.ticket) {
     if (source.leave_if_unordered) return;
     // lists out of order: every pair of every offset is looked at
-    scanAllPairsForTile<E, 64>(A, Q, source, K, r0, r0 + TR < R ? r0 + TR : R, C, 0, s_acc, ACC_STRIDE);
+    scanAllPairsForTile<E, 64>(A, conv.q, conv.row_bytes, source, K, r0, r0 + TR < R ? r0 + TR : R,
+                               conv.c, 0, s_acc, ACC_STRIDE);
     write_out();
     return;
   }
@@ -1090,8 +1156,8 @@ __global__ __launch_bounds__(64) void gatherConvWave(
       int g = pair_src[pslot];
       if (pair >= n || (unsigned)g >= (unsigned)source.n_src) g = 0;
       // (a lane beyond the row's channels reads the row of zeros)
-      const char *from = quad * 16 < ROW_BYTES ? a_bytes + (size_t)g * ROW_BYTES + quad * 16
-                                               : reinterpret_cast<const char *>(kZeroRow);
+      const char *from = quad * 16 < conv.row_bytes ? a_bytes + (size_t)g * conv.row_bytes + quad * 16
+                                                    : reinterpret_cast<const char *>(kZeroRow);
       rows[rslot][0] = *reinterpret_cast<const u32x4 *>(from);
     } else {
 #pragma unroll
@@ -1099,7 +1165,10 @@ __global__ __launch_bounds__(64) void gatherConvWave(
         const int e = lane / PPR + EPL * h;  // which pair's row this lane fetches a piece of
         int g = __shfl(pair_src[pslot], e & 15, kWave);
         if (e >= n || (unsigned)g >= (unsigned)source.n_src) g = 0;
-        rows[rslot][h] = *reinterpret_cast<const u32x4 *>(a_bytes + (size_t)g * ROW_BYTES + (lane % PPR) * 16);
+        const int at = (lane % PPR) * 16;
+        rows[rslot][h] = *reinterpret_cast<const u32x4 *>(
+            at < conv.row_bytes ? a_bytes + (size_t)g * conv.row_bytes + at
+                                : reinterpret_cast<const char *>(kZeroRow));
       }
     }
     const char *bk = b_base + (size_t)k * kBytesPerOffset;
@@ -1174,63 +1243,125 @@ __global__ __launch_bounds__(64) void gatherConvWave(
 //
 // When most rows of a tile have a partner at most offsets, compacting pairs buys
 // little and the fp32 accumulate in LDS (a 16-byte read-modify-write per lane and
-// 16 result columns, on arbitrary rows: bank conflicts) is what the kernel above
-// spends its time on.  Here a tile is 128 result rows (256 below 128 channels), a wave
-// of eight owns G = 1 (2) groups of 16 of them and all result columns, and accumulates
-// them in registers over all offsets: no accumulator traffic at all.  The partner rows of an offset come from global memory straight into the
-// operand registers of the lane that multiplies them (lane (row, quarter) loads 16
-// bytes of its row per reduction chunk, one offset ahead), so no wave waits for
-// another one's rows.  What the waves of a workgroup share is the offset's filter: its
-// fragments travel from global memory into one of two LDS buffers (16 bytes per lane
-// straight into LDS, one offset ahead, every wave a share of them) and every wave reads
-// all of them from there, once per offset for all its row groups.  One barrier per
-// offset hands the buffers over; it waits for LDS traffic only, and each wave waits for
-// its own loads itself (__syncthreads() would make every wave wait for all loads in
-// flight, the requests for the offset after included).  A lane whose row has no
-// partner at the offset reads a row of zeros; a row group none of whose rows has one
-// is skipped, and a wave without any skips the offset.
+// 16 result columns, on arbitrary rows: bank conflicts) is what the kernels above
+// spend their time on.  Here a wave owns two groups of 16 result rows and all result
+// columns, and accumulates them in registers over all offsets: no accumulator traffic
+// at all.
+//
+// Rows are buffer loads: the row map holds byte offsets, a lane without a partner holds one
+// behind the tensor's end, and the hardware answers it with zeros without going to memory.  The
+// rows of the wave's next offsets travel while the current one is multiplied.
+// Filter.  The waves share an offset's filter: its fragments travel from global memory into a
+// ring of two LDS buffers, a phase of one or two offsets at a time, and every wave reads all of
+// them from there, once per offset for both its row groups.  One barrier per phase hands a
+// buffer over; it waits for LDS traffic only, and each wave waits for its own requests itself
+// (__syncthreads() would make every wave wait for all loads in flight).
+//
+// What bounds it differs with the row length, and so does the way of the rows (us for forward
+// at 80 k rows, 27 offsets, half the slots filled; in brackets one path for all lengths: 4 row
+// groups' filters read from LDS per offset by 4 waves, rows by plain loads):
+//   up to 64 bytes (16 channels: 37 us [42]): the loop itself.  Rows come straight into the
+//     operand registers (lane (row, quarter) loads 16 bytes), whole phases of two offsets are in
+//     flight, and nothing is skipped: a group without rows multiplies zeros.
+//   up to 128 bytes (64 channels: 88 us [101]): operand-order loads touch 16 rows of 64 bytes
+//     each, which the CU's address unit takes at a third of the rate of whole rows.  So rows come
+//     row by row into registers, go through LDS (pieces permuted so that operand reads meet no
+//     bank twice), and every request is spread between the multiplies.
+//   above (128 channels: 199 us [230]): the multiplies (130 us at the matrix cores' rate if
+//     nothing were skipped), and LDS, which carries the filter; rows through LDS as well measure
+//     217 us.  So rows go in operand order again, a chunk requested right behind its last use,
+//     in eight waves per filter copy, and a wave multiplies only the groups that have a row
+//     at the offset.
 constexpr int kDenseChunk = 27;      // offsets whose row-map slice is resident in LDS at once
 constexpr int kDenseMapBatch = 14;   // loads in flight per thread while a tile's row map is read
-constexpr int kDenseWaves = 8;
-// Row groups per wave: with two sets of partner rows a wave stays within 128 registers, four
-// waves a SIMD.  (Four waves of twice the groups measured the same at 64 and 128 columns and
-// 12 % slower at 16 and 32, where a wave has little to multiply between two barriers.)
-constexpr int denseGroups(int Q, int C) { return (C >= 128 || Q >= 128) ? 1 : 2; }
-constexpr int denseTileRows(int Q, int C) { return kDenseWaves * denseGroups(Q, C) * 16; }
+constexpr uint32_t kNoRow = 0x80000000u;  // byte offset of a partner that is not there
+
+// How an instance splits its work, from what a CU has: 160 KiB of LDS and 512 registers a lane
+// and SIMD.  Short rows: as many workgroups as registers and LDS allow.  Rows above 128 bytes: one
+// workgroup of eight waves, since two ring buffers of 64 KiB leave no room for a second.
+enum class DenseRows { kByPhase, kStaged, kInPlace };  // how rows reach the operand registers
+struct DensePlan {
+  int waves;        // per workgroup
+  int groups;       // row groups (of 16) per wave
+  int per_cu;       // workgroups a CU
+  int offsets;      // offsets per phase
+  DenseRows rows;
+};
+constexpr DensePlan densePlan(int elem_bytes, int Q, int C) {
+  const int nb = C / 16, kb = (Q * elem_bytes + 63) / 64;
+  const int row_bytes = Q * elem_bytes;
+  if (row_bytes <= 64) {
+    DensePlan p = {4, 2, 4, 2, DenseRows::kByPhase};
+    const int room = 160 * 1024 / 4 - kDenseChunk * 4 * p.groups * 16 * 4 - 1024;
+    if (p.groups * 4 * (nb + 2 * 2) + 4 * nb + 40 > 128) p.per_cu = 2;
+    if (p.per_cu == 4 && room < 4 * nb * kb * 1024) p.per_cu = 2;
+    return p;
+  }
+  if (row_bytes <= 128) {
+    DensePlan p = {4, 2, 2, 2, DenseRows::kStaged};
+    const int rows = p.waves * p.groups * 16;
+    const int room = 160 * 1024 / p.per_cu - kDenseChunk * rows * 4 - rows * row_bytes - 1024;
+    if (room < 4 * nb * kb * 1024) p.offsets = 1;
+    return p;
+  }
+  DensePlan p = {8, 2, 1, 2, DenseRows::kInPlace};
+  const int room = 160 * 1024 - kDenseChunk * p.waves * p.groups * 16 * 4 - 1024;
+  if (room < 4 * nb * kb * 1024) p.offsets = 1;
+  return p;
+}
+constexpr int denseWavesPerSimd(int elem_bytes, int Q, int C) {
+  const DensePlan p = densePlan(elem_bytes, Q, C);
+  return p.waves * p.per_cu / 4;
+}
+constexpr int denseTileRows(int elem_bytes, int Q, int C) {
+  return densePlan(elem_bytes, Q, C).waves * densePlan(elem_bytes, Q, C).groups * 16;
+}
+// Where piece `piece` of a staged row lies in its row's bytes: rows lie a multiple of the bank
+// width apart, and the 16 rows whose same piece is read at once have to meet all banks.
+constexpr int denseRowSwizzle(int row_bytes, int row) {
+  return row_bytes >= 256 ? (row & 15) : ((row >> 1) & 7);
+}
+
+// The gathered tensor as a buffer of `bytes` (below 2^31) for loads that answer zero behind it.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rowsBuffer(const void *base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
+}
 
 template <typename E, int Q, int C, typename SRC>
-__global__ __launch_bounds__(64 * kDenseWaves) __attribute__((amdgpu_waves_per_eu(4, 4))) void gatherConvDense(
-    const typename E::storage *A, const typename E::storage *packedW, SRC source, int R,
-    int K, int ldc, typename E::storage *result) {
+__global__ __launch_bounds__(64 * densePlan((int)sizeof(typename E::storage), Q, C).waves)
+    __attribute__((amdgpu_waves_per_eu(denseWavesPerSimd((int)sizeof(typename E::storage), Q, C),
+                                       denseWavesPerSimd((int)sizeof(typename E::storage), Q, C))))
+void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows conv,
+                     const typename E::storage *packedW, SRC source, int R, int K,
+                     typename E::storage *result) {
   typedef typename E::vec8 vec8;
   typedef typename E::storage S;
-  constexpr int WAVES = kDenseWaves;
-  constexpr int G = denseGroups(Q, C);
-  constexpr int TR = denseTileRows(Q, C);
+  constexpr DensePlan PLAN = densePlan((int)sizeof(S), Q, C);
+  constexpr int WAVES = PLAN.waves;
+  constexpr bool kStaged = PLAN.rows == DenseRows::kStaged;
+  constexpr int G = PLAN.groups;
+  constexpr int TR = WAVES * G * 16;
+  constexpr int NT = WAVES * 64;
   constexpr int NB = C / 16;                 // 16-column blocks, all of them in every wave
   constexpr int KC = kDenseChunk;
   constexpr int KB = (Q + E::kChunk - 1) / E::kChunk;
-  // 16 channels of a 2-byte type: half a fragment, the lanes of the other half read zeros
-  constexpr bool kHalfFragment = Q % E::kChunk != 0;
   constexpr int ROW_BYTES = Q * (int)sizeof(S);
   constexpr int FRAGS = NB * KB;             // 1 KiB filter fragments per offset
   constexpr int W_BYTES = FRAGS * 1024;
-  constexpr int FPW = (FRAGS + WAVES - 1) / WAVES;
-  // Offsets multiplied between two barriers: two where a filter is 4 KiB at most (a wave then
-  // has little to multiply per offset, and the second set of rows fits the registers): 16 and
-  // 32 column layers 7 % faster; at 64 x 64 the rows of two offsets spill.
-  constexpr int OPP = W_BYTES <= 4096 ? 2 : 1;
-  constexpr int POOL = 2 * OPP * W_BYTES;
-  static_assert((Q % E::kChunk == 0 || (KB == 1 && Q % E::kVec == 0)) && C % 16 == 0,
-                "whole fragments, or part of a single one");
-  static_assert(G >= 1 && G <= 4, "one code path per set of row groups");
+  constexpr int OPP = PLAN.offsets;          // offsets per phase
+  constexpr int BUF_FRAGS = OPP * FRAGS;
+  constexpr int FPW = (BUF_FRAGS + WAVES - 1) / WAVES;
+  // kStaged: loads of 1 KiB per row group, and rows per load
+  constexpr int LPG = kStaged ? 16 * ROW_BYTES / 1024 : 1;
+  constexpr int RPL = kStaged ? 1024 / ROW_BYTES : 1;
+  static_assert(KC <= 32, "a chunk's offsets in one mask");
 
-  __shared__ __attribute__((aligned(1024))) char s_w[POOL];
-  __shared__ int s_map[KC][TR];   // partner row of (offset in chunk, tile row) or -1
-  __shared__ int s_list[KC];      // offsets of the chunk that have a pair in this tile
+  __shared__ __attribute__((aligned(1024))) char s_w[2 * BUF_FRAGS * 1024];
+  __shared__ __attribute__((aligned(1024))) char s_rows[kStaged ? TR * ROW_BYTES : 16];
+  __shared__ uint32_t s_map[KC][TR];  // where the partner row of (offset in chunk, tile row) begins, or kNoRow
   __shared__ int s_has[KC];
   __shared__ int s_first[KC];
-  __shared__ int s_count;
+  __shared__ uint32_t s_offsets;      // offsets of the chunk that have a pair in this tile
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1243,11 +1374,10 @@ __global__ __launch_bounds__(64 * kDenseWaves) __attribute__((amdgpu_waves_per_e
   }
   if (r0 >= R) {
     if constexpr (!SRC::kSegments) {
-      if (tid == 0 && blockIdx.y == 0) source.filled[blockIdx.x] = 0;
+      if (tid == 0) source.filled[blockIdx.x] = 0;
     }
     return;
   }
-  const int col_group = blockIdx.y;
   if constexpr (SRC::kSegments) {
     if (*source.verdict == source.ticket && source.leave_if_unordered) return;
     if (*source.verdict == source.ticket) {
@@ -1255,15 +1385,16 @@ __global__ __launch_bounds__(64 * kDenseWaves) __attribute__((amdgpu_waves_per_e
       // time, every pair looked at by every workgroup
       float *acc = reinterpret_cast<float *>(&s_map[0][0]);
       constexpr int CP = 16;  // columns per pass
-      static_assert(CP <= KC && C % CP == 0, "a pass of columns fits the row map");
+      static_assert(CP <= KC, "a pass of columns fits the row map");
       const int r_end = r0 + TR < R ? r0 + TR : R;
-      for (int c0 = 0; c0 < C; c0 += CP) {
-        for (int i = tid; i < TR * CP; i += WAVES * 64) acc[i] = 0.f;
+      for (int c0 = 0; c0 < conv.c; c0 += CP) {
+        for (int i = tid; i < TR * CP; i += NT) acc[i] = 0.f;
         __syncthreads();
-        scanAllPairsForTile<E, WAVES * 64>(A, Q, source, K, r0, r_end, CP, col_group * C + c0, acc, CP);
-        for (int i = tid; i < TR * CP; i += WAVES * 64) {
+        const int columns = conv.c - c0 < CP ? conv.c - c0 : CP;
+        scanAllPairsForTile<E, NT>(A, conv.q, conv.row_bytes, source, K, r0, r_end, columns, c0, acc, CP);
+        for (int i = tid; i < TR * CP; i += NT) {
           const int rr = i / CP, c = i % CP;
-          if (r0 + rr < R) E::store(result + (size_t)(r0 + rr) * ldc + col_group * C + c0 + c, acc[i]);
+          if (r0 + rr < R && c < columns) E::store(result + (size_t)(r0 + rr) * conv.c + c0 + c, acc[i]);
         }
         __syncthreads();
       }
@@ -1272,13 +1403,20 @@ __global__ __launch_bounds__(64 * kDenseWaves) __attribute__((amdgpu_waves_per_e
   }
   const int pair = lane & 15;
   const int quad = lane >> 4;
-  const char *a_lane = reinterpret_cast<const char *>(A) + quad * 16;
-  const char *zero_lane = reinterpret_cast<const char *>(kZeroRow) + quad * 16;
-  const char *w_base = reinterpret_cast<const char *>(packedW) +
-                       (size_t)col_group * FRAGS * 1024 + lane * 16;
-  const size_t kBytesPerOffset = (size_t)(ldc / 16) * KB * 1024;
+  const __amdgpu_buffer_rsrc_t a_rows = rowsBuffer(A, a_size);
+  const char *w_base = reinterpret_cast<const char *>(packedW) + lane * 16;
   const uint32_t w_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)s_w;
   const int row_first = wave * (G * 16) + pair;  // this lane's row in its wave's first group
+  // Which 16 bytes of a row a lane asks for: its quarter, or in staged loads the piece that
+  // belongs where the lane writes.  Behind the row's own bytes: nowhere (zeros).
+  uint32_t piece_at[LPG];
+#pragma unroll
+  for (int j = 0; j < LPG; ++j) {
+    const int row = j * RPL + lane / (64 / RPL);
+    const int piece = kStaged ? (lane % (64 / RPL)) ^ denseRowSwizzle(ROW_BYTES, row) : quad;
+    piece_at[j] = piece * 16 < conv.row_bytes ? (uint32_t)piece * 16u : kNoRow;
+  }
+  char *const rows_lds = s_rows + wave * (G * 16) * (kStaged ? ROW_BYTES : 0);
 
   float4v acc[G][NB];
 #pragma unroll
@@ -1286,7 +1424,6 @@ __global__ __launch_bounds__(64 * kDenseWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[g][nb] = float4v{0.f, 0.f, 0.f, 0.f};
   int slots = 0;  // filled map slots this thread staged
-  constexpr int NT = WAVES * 64;
 
   for (int kc = 0; kc < K; kc += KC) {
     const int kn = (K - kc) < KC ? (K - kc) : KC;
@@ -1302,7 +1439,7 @@ __global__ __launch_bounds__(64 * kDenseWaves) __attribute__((amdgpu_waves_per_e
         s_first[tid] = first;
         s_has[tid] = count;
       }
-      for (int i = tid; i < kn * TR; i += NT) (&s_map[0][0])[i] = -1;
+      for (int i = tid; i < kn * TR; i += NT) (&s_map[0][0])[i] = kNoRow;
       __syncthreads();
       // a thread per (offset, pair of the piece): the partner goes to the result row's
       // position.  A thread's loads of one batch are all requested before the first is
@@ -1326,7 +1463,7 @@ __global__ __launch_bounds__(64 * kDenseWaves) __attribute__((amdgpu_waves_per_e
           }
 #pragma unroll
           for (int u = 0; u < kDenseMapBatch; ++u)
-            if (at[u] >= 0) s_map[at[u]][(own[u] - r0) & (TR - 1)] = partner[u];
+            if (at[u] >= 0) s_map[at[u]][(own[u] - r0) & (TR - 1)] = (uint32_t)partner[u] * (uint32_t)conv.row_bytes;
         }
       }
     } else {
@@ -1346,7 +1483,7 @@ __global__ __launch_bounds__(64 * kDenseWaves) __attribute__((amdgpu_waves_per_e
 #pragma unroll
         for (int u = 0; u < kDenseMapBatch; ++u) {
           const int slot = base + u * NT;  // (a wave stays inside one offset)
-          if (slot < kn * TR) s_map[slot / TR][slot % TR] = v[u];
+          if (slot < kn * TR) s_map[slot / TR][slot % TR] = v[u] >= 0 ? (uint32_t)v[u] * (uint32_t)conv.row_bytes : kNoRow;
           const unsigned long long m = __ballot(v[u] >= 0);
           if (m != 0ull && lane == 0) s_has[slot / TR] = 1;
           slots += v[u] >= 0;
@@ -1357,123 +1494,338 @@ __global__ __launch_bounds__(64 * kDenseWaves) __attribute__((amdgpu_waves_per_e
     if (wave == 0) {
       const bool has = lane < kn && s_has[lane < kn ? lane : 0] != 0;
       const unsigned long long m = __ballot(has);
-      if (has) s_list[__popcll(m & ((1ull << lane) - 1ull))] = lane;
-      if (lane == 0) s_count = __popcll(m);
+      if (lane == 0) s_offsets = (uint32_t)m;
     }
     __syncthreads();
-    const int items = s_count;
-    if (items == 0) continue;
-
-    // The partner rows of one offset, into the registers of the lanes that multiply them
-    // (a lane without a partner reads zeros); returns which of the wave's row groups have
-    // a partner at all.
-    auto load_rows = [&](int item, vec8 (&rows)[G][KB]) -> int {
-      const int kk = s_list[item];
-      int present = 0;
+    const uint32_t offsets = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_offsets);
+    if (offsets == 0) continue;
+    // A phase: the OPP lowest offsets of `left` (fewer at the end), which are taken out of it.
+    auto next_phase = [](uint32_t &left) -> uint32_t {
+      uint32_t rest = left;
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const int src = s_map[kk][row_first + g * 16];
-        const bool mine = src >= 0;
-        const bool read = mine && (!kHalfFragment || quad * E::kVec < Q);
-        const char *row = read ? a_lane + (size_t)src * ROW_BYTES : zero_lane;
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb)
-          rows[g][kb] = *reinterpret_cast<const vec8 *>(row + kb * 64);
-        if (__ballot(mine) != 0ull) present |= 1 << g;
-      }
-      return present;
+      for (int o = 0; o < OPP; ++o) rest &= rest - 1;
+      const uint32_t phase = left & ~rest;
+      left = rest;
+      return phase;
     };
-    // The filter fragments of one offset into a buffer: fragment f by wave f % WAVES.
-    auto request_filter = [&](int item, int buffer) {
-      const char *wk = w_base + (size_t)(kc + s_list[item]) * kBytesPerOffset;
-      const uint32_t buf = w_lds + buffer * W_BYTES;
+    // Fragment f of a phase's filters (its offsets in ascending order), as bytes of the packed
+    // filter.  Behind the phase's last offset: fragments of some other one, which nobody reads.
+    auto fragment_of = [&](uint32_t phase, int f) -> const char * {
+      uint32_t left = phase;
+#pragma unroll
+      for (int o = 1; o < OPP; ++o)
+        if (f >= o * FRAGS && (left & (left - 1)) != 0) left &= left - 1;
+      const int k = left != 0 ? __builtin_ctz(left) : 0;
+      return w_base + ((size_t)(kc + k) * FRAGS + f % FRAGS) * 1024;
+    };
+    // The filters of a phase's offsets into half `half` of the ring: fragment f by wave f % WAVES.
+    auto filters_to_lds = [&](uint32_t phase, int half) {
 #pragma unroll
       for (int t = 0; t < FPW; ++t) {
         const int f = wave + t * WAVES;
-        if (FRAGS % WAVES != 0 && f >= FRAGS) break;
-        requestToLds(wk + f * 1024, buf + f * 1024);
+        if (BUF_FRAGS % WAVES == 0 || f < BUF_FRAGS)
+          requestToLds(fragment_of(phase, f), w_lds + (half * BUF_FRAGS + f) * 1024);
       }
     };
-    // acc[g] += rows[g] x filter for the two row groups from G0 on that MASK names
-    auto multiply = [&](auto g0_tag, auto mask_tag, const vec8 (&rows)[G][KB], const char *wbuf) {
-      constexpr int G0 = decltype(g0_tag)::value;
+    if constexpr (PLAN.rows == DenseRows::kByPhase) {
+      // Rows in one of two sets of registers, filters in one of two ring buffers.
+      vec8 rows_a[OPP][G], rows_b[OPP][G];
+      auto request_phase = [&](uint32_t phase, int half, vec8 (&rows)[OPP][G]) {
+        filters_to_lds(phase, half);
+        uint32_t left = phase;
+#pragma unroll
+        for (int o = 0; o < OPP; ++o) {
+          const bool there = left != 0;
+          const int kk = there ? __builtin_ctz(left) : 0;
+          left &= left - 1;
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+            const uint32_t at = there ? s_map[kk][row_first + g * 16] : kNoRow;
+            rows[o][g] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(
+                                                      a_rows, __builtin_elementwise_add_sat(at, piece_at[0]), 0, 0));
+          }
+        }
+      };
+      // Everything this wave has requested is there.  The rows pass through an empty statement
+      // that the compiler must take for their last writer: it then places its own wait for their
+      // loads here, and not in front of their first use, behind the next phase's requests, which
+      // it would wait for as well.
+      auto landed = [&](vec8 (&rows)[OPP][G]) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int o = 0; o < OPP; ++o)
+#pragma unroll
+          for (int g = 0; g < G; ++g) asm volatile("" : "+v"(rows[o][g]));
+      };
+      auto multiply_phase = [&](int half, const vec8 (&rows)[OPP][G]) {
+        const char *filters = s_w + half * BUF_FRAGS * 1024 + lane * 16;
+#pragma unroll
+        for (int o = 0; o < OPP; ++o)
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            const vec8 w = *reinterpret_cast<const vec8 *>(filters + o * W_BYTES + nb * 1024);
+#pragma unroll
+            for (int g = 0; g < G; ++g) acc[g][nb] = E::mfma(w, rows[o][g], acc[g][nb]);
+          }
+      };
+      uint32_t left = offsets;
+      uint32_t phase = next_phase(left);
+      request_phase(phase, 0, rows_a);
+      landed(rows_a);
+      ldsBarrier();
+      while (true) {
+        phase = next_phase(left);
+        if (phase != 0) request_phase(phase, 1, rows_b);
+        multiply_phase(0, rows_a);
+        if (phase == 0) break;
+        landed(rows_b);
+        ldsBarrier();
+        phase = next_phase(left);
+        if (phase != 0) request_phase(phase, 0, rows_a);
+        multiply_phase(1, rows_b);
+        if (phase == 0) break;
+        landed(rows_a);
+        ldsBarrier();
+      }
+    } else if constexpr (PLAN.rows == DenseRows::kInPlace) {
+    // offsets at which the wave's first / second row group has a partner
+    uint32_t has_first = 0, has_second = 0;
+#pragma unroll 9
+    for (int kk = 0; kk < kn; ++kk) {
+      if (__ballot(s_map[kk][row_first] != kNoRow) != 0ull) has_first |= 1u << kk;
+      if (__ballot(s_map[kk][row_first + 16] != kNoRow) != 0ull) has_second |= 1u << kk;
+    }
+    has_first = (uint32_t)__builtin_amdgcn_readfirstlane((int)has_first);
+    has_second = (uint32_t)__builtin_amdgcn_readfirstlane((int)has_second);
+
+    // The wave's way through a phase: first the offsets at which both its groups have rows, then
+    // those of the first group alone, then the second's; each in ascending order.
+    struct Way {
+      uint32_t both, first, second;
+    };
+    auto way_through = [&](uint32_t phase) -> Way {
+      return Way{phase & has_first & has_second, phase & has_first & ~has_second, phase & has_second & ~has_first};
+    };
+    // The offset whose rows are requested next: one in front of the one that is multiplied.
+    uint32_t ahead_left = offsets;
+    Way ahead = {0, 0, 0};
+    auto next_ahead = [&]() -> int {
+      while ((ahead.both | ahead.first | ahead.second) == 0) {
+        if (ahead_left == 0) return -1;
+        ahead = way_through(next_phase(ahead_left));
+      }
+      const uint32_t from = ahead.both != 0 ? ahead.both : (ahead.first != 0 ? ahead.first : ahead.second);
+      const uint32_t taken = from & (0u - from);
+      ahead.both &= ~taken;  // (an offset is in one of the three masks)
+      ahead.first &= ~taken;
+      ahead.second &= ~taken;
+      return __builtin_ctz(taken);
+    };
+    // where this lane's rows of offset kk (none: -1) begin
+    auto locate_rows = [&](int kk, uint32_t (&at)[G]) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        at[g] = s_map[kk < 0 ? 0 : kk][row_first + g * 16];
+        at[g] = kk < 0 ? kNoRow : at[g];
+      }
+    };
+    // 16 bytes of a row: reduction chunk kb, this lane's quarter; zeros where the row ends before
+    auto load_chunk = [&](uint32_t at, int kb) -> vec8 {
+      const uint32_t piece = (uint32_t)(kb * 64 + quad * 16);
+      const uint32_t from = piece < (uint32_t)conv.row_bytes ? at + quad * 16 : kNoRow;
+      return __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(a_rows, from, kb * 64, 0));
+    };
+
+    vec8 rows[G][KB];
+    // one offset: the fragments at `wbuf` times the rows of the groups in MASK, while the rows of
+    // the wave's next offset are requested chunk by chunk behind their last use
+    auto multiply = [&](auto mask_tag, const char *wbuf) {
       constexpr int MASK = decltype(mask_tag)::value;
+      uint32_t at[G];
+      locate_rows(next_ahead(), at);
+      vec8 w[2][NB];
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) w[0][nb] = *reinterpret_cast<const vec8 *>(wbuf + nb * KB * 1024);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        if (kb + 1 < KB) {
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb)
+            w[(kb + 1) & 1][nb] = *reinterpret_cast<const vec8 *>(wbuf + (nb * KB + kb + 1) * 1024);
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          if ((MASK >> g) & 1) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[g][nb] = E::mfma(w[kb & 1][nb], rows[g][kb], acc[g][nb]);
+          }
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) rows[g][kb] = load_chunk(at[g], kb);
+        asm volatile("" ::: "memory");  // the requests stay here, an offset ahead of their use
+      }
+    };
+
+    uint32_t phases_left = offsets;
+    uint32_t phase = next_phase(phases_left);
+    filters_to_lds(phase, 0);
+    {
+      uint32_t at[G];
+      locate_rows(next_ahead(), at);
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          const vec8 wf = *reinterpret_cast<const vec8 *>(wbuf + (nb * KB + kb) * 1024 + lane * 16);
-          if constexpr ((MASK & 1) != 0) acc[G0][nb] = E::mfma(wf, rows[G0][kb], acc[G0][nb]);
-          if constexpr ((MASK & 2) != 0 && G0 + 1 < G)
-            acc[G0 + 1][nb] = E::mfma(wf, rows[G0 + 1][kb], acc[G0 + 1][nb]);
-        }
-    };
-    auto multiply_present = [&](int present, const vec8 (&rows)[G][KB], const char *wbuf) {
-      typedef std::integral_constant<int, 1> one;
-      typedef std::integral_constant<int, 2> two;
-      typedef std::integral_constant<int, 3> both;
-      {
-        typedef std::integral_constant<int, 0> first;
-        const int bits = present & 3;
-        if (bits == 3) multiply(first(), both(), rows, wbuf);
-        else if (bits == 1) multiply(first(), one(), rows, wbuf);
-        else if (bits == 2) multiply(first(), two(), rows, wbuf);
-      }
-      if constexpr (G == 4) {
-        typedef std::integral_constant<int, 2> first;
-        const int bits = (present >> 2) & 3;
-        if (bits == 3) multiply(first(), both(), rows, wbuf);
-        else if (bits == 1) multiply(first(), one(), rows, wbuf);
-        else if (bits == 2) multiply(first(), two(), rows, wbuf);
-      }
-    };
-    // Waits for everything this wave has requested.  The rows pass through an empty
-    // statement that the compiler must take for their last writer: it then places its own
-    // wait for their loads here, where it costs nothing, and not in front of their first
-    // use, behind the requests for the offsets after, which it would wait for as well.
-    auto landed = [&](vec8 (&rows)[OPP][G][KB]) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        for (int g = 0; g < G; ++g) rows[g][kb] = load_chunk(at[g], kb);
+    }
+    // (the filters are older than the rows)
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G * KB) : "memory");
+    ldsBarrier();
+    int half = 0;
+    while (true) {
+      // (every wave has left the other half of the ring)
+      const uint32_t phase_after = next_phase(phases_left);
+      if (phase_after != 0) filters_to_lds(phase_after, half ^ 1);
+      Way way = way_through(phase);
+      const bool took_part = (way.both | way.first | way.second) != 0;
+      const char *ring = s_w + half * OPP * W_BYTES + lane * 16;
+      auto filter_of = [&](int k) { return ring + __popc(phase & ((1u << k) - 1u)) * W_BYTES; };
+      for (; way.both != 0; way.both &= way.both - 1)
+        multiply(std::integral_constant<int, 3>(), filter_of(__builtin_ctz(way.both)));
+      for (; way.first != 0; way.first &= way.first - 1)
+        multiply(std::integral_constant<int, 1>(), filter_of(__builtin_ctz(way.first)));
+      for (; way.second != 0; way.second &= way.second - 1)
+        multiply(std::integral_constant<int, 2>(), filter_of(__builtin_ctz(way.second)));
+      if (phase_after == 0) break;
+      // the filters requested in front of this phase are older than the rows requested in it
+      if (took_part)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G * KB) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      ldsBarrier();
+      phase = phase_after;
+      half ^= 1;
+    }
+    } else {
+    // Where the rows of a phase's offsets begin, for this lane's share of the loads (a KiB each: whole
+    // lines of whole rows); behind the tensor where the phase has no such offset.
+    auto locate_rows = [&](uint32_t phase, uint32_t (&at)[OPP][G][LPG]) {
+      uint32_t left = phase;
 #pragma unroll
-      for (int o = 0; o < OPP; ++o)
+      for (int o = 0; o < OPP; ++o) {
+        const uint32_t nowhere = left != 0 ? 0u : kNoRow;
+        const int kk = left != 0 ? __builtin_ctz(left) : 0;
+        left &= left - 1;
 #pragma unroll
         for (int g = 0; g < G; ++g)
 #pragma unroll
-          for (int kb = 0; kb < KB; ++kb) asm volatile("" : "+v"(rows[o][g][kb]));
-    };
-    // requests rows and filters of the OPP offsets from `item` on into `rows` and LDS buffer
-    // `buffer`; an offset past the last one repeats the last (its rows are not multiplied)
-    auto request_phase = [&](int item, int buffer, vec8 (&rows)[OPP][G][KB], int (&present)[OPP]) {
-#pragma unroll
-      for (int o = 0; o < OPP; ++o) {
-        const bool there = item + o < items;
-        const int it = there ? item + o : items - 1;
-        const int got = load_rows(it, rows[o]);
-        present[o] = there ? got : 0;
-        request_filter(it, buffer * OPP + o);
+          for (int j = 0; j < LPG; ++j)
+            at[o][g][j] = s_map[kk][wave * (G * 16) + g * 16 + j * RPL + lane / (64 / RPL)] | nowhere;
       }
     };
-    // The OPP offsets from `item` on with the rows in `cur`, while the rows and the filters of
-    // the next ones travel.  Everything requested here has landed when the barrier is
-    // passed, and every wave has left the buffers that the phase after the next writes to.
-    auto phase = [&](int item, const int (&present)[OPP], const vec8 (&cur)[OPP][G][KB],
-                     vec8 (&nxt)[OPP][G][KB], int (&present_next)[OPP]) {
-      const int buffer = (item / OPP) & 1;
-      if (item + OPP < items) request_phase(item + OPP, buffer ^ 1, nxt, present_next);
+    auto request_row = [&](uint32_t at, int j) -> u32x4 {
+      return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                           a_rows, __builtin_elementwise_add_sat(at, piece_at[j]), 0, 0));
+    };
+    auto request_filter = [&](uint32_t phase, int t) -> u32x4 {
+      return *reinterpret_cast<const u32x4 *>(fragment_of(phase, (wave + t * WAVES) % BUF_FRAGS));
+    };
+    auto store_filter = [&](u32x4 v, int t, int half) {
+      *reinterpret_cast<u32x4 *>(s_w + (half * BUF_FRAGS + (wave + t * WAVES) % BUF_FRAGS) * 1024 + lane * 16) = v;
+    };
+    // One phase: its rows in `set` go through the wave's place in LDS into operand registers, and
+    // `set` is requested again for the phase after the next, as are the filters.  The requests are
+    // spread between the multiplies: made together they keep all waves waiting for the CU's
+    // address unit at the same time, with nothing left to multiply.  No load and no multiply
+    // depends on what the wave has to do: a wave without rows at an offset multiplies zeros,
+    // and the number of loads in flight is the same on every way through the loop, so that
+    // the compiler waits for exactly the ones it needs.
+    u32x4 filters[FPW];
+    auto take_phase = [&](uint32_t after_that, int half, u32x4 (&set)[OPP][G][LPG]) {
+      // steps of up to four column blocks of one chunk; a step's fragments are read while the
+      // step before is multiplied
+      constexpr int NS = NB < 4 ? NB : 4, PER = NB / NS, STEPS = KB * PER;
+      uint32_t at[OPP][G][LPG];
+      locate_rows(after_that, at);
 #pragma unroll
-      for (int o = 0; o < OPP; ++o)
-        multiply_present(present[o], cur[o], s_w + (buffer * OPP + o) * W_BYTES);
-      landed(nxt);
+      for (int o = 0; o < OPP; ++o) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+          for (int j = 0; j < LPG; ++j)
+            *reinterpret_cast<u32x4 *>(rows_lds + (g * LPG + j) * 1024 + lane * 16) = set[o][g][j];
+        const char *const wbuf = s_w + (half * BUF_FRAGS + o * FRAGS) * 1024 + lane * 16;
+        vec8 rows[2][G], w[2][NS];
+        auto read_step = [&](int step) {
+          const int kb = step / PER, nb0 = step % PER * NS;
+          if (step % PER == 0) {
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+              rows[kb & 1][g] = *reinterpret_cast<const vec8 *>(
+                  rows_lds + (g * 16 + pair) * ROW_BYTES + (((kb * 4 + quad) ^ denseRowSwizzle(ROW_BYTES, pair)) * 16));
+          }
+#pragma unroll
+          for (int i = 0; i < NS; ++i)
+            w[step & 1][i] = *reinterpret_cast<const vec8 *>(wbuf + ((nb0 + i) * KB + kb) * 1024);
+        };
+        read_step(0);
+#pragma unroll
+        for (int step = 0; step < STEPS; ++step) {
+          if (step + 1 < STEPS) read_step(step + 1);
+          // this step's share of the requests
+#pragma unroll
+          for (int x = 0; x < G * LPG; ++x)
+            if (x * STEPS / (G * LPG) == step) set[o][x / LPG][x % LPG] = request_row(at[o][x / LPG][x % LPG], x % LPG);
+#pragma unroll
+          for (int t = 0; t < FPW; ++t)
+            if (t * (OPP * STEPS) / FPW == o * STEPS + step) {
+              store_filter(filters[t], t, half ^ 1);
+              filters[t] = request_filter(after_that, t);
+            }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < NS; ++i)
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+              float4v &sum = acc[g][step % PER * NS + i];
+              sum = E::mfma(w[step & 1][i], rows[(step / PER) & 1][g], sum);
+            }
+        }
+      }
       ldsBarrier();
     };
 
-    vec8 rows_a[OPP][G][KB], rows_b[OPP][G][KB];
-    int present_a[OPP], present_b[OPP];
-    request_phase(0, 0, rows_a, present_a);
-    landed(rows_a);
-    ldsBarrier();
-    for (int i = 0; i < items; i += 2 * OPP) {
-      phase(i, present_a, rows_a, rows_b, present_b);
-      if (i + OPP < items) phase(i + OPP, present_b, rows_b, rows_a, present_a);
+    u32x4 rows_a[OPP][G][LPG], rows_b[OPP][G][LPG];
+    uint32_t left = offsets;
+    uint32_t p0 = next_phase(left), p1 = next_phase(left), p2 = 0;
+    {
+      auto request_phase = [&](uint32_t phase, u32x4 (&set)[OPP][G][LPG]) {
+        uint32_t at[OPP][G][LPG];
+        locate_rows(phase, at);
+#pragma unroll
+        for (int x = 0; x < OPP * G * LPG; ++x)
+          set[x / (G * LPG)][x / LPG % G][x % LPG] = request_row(at[x / (G * LPG)][x / LPG % G][x % LPG], x % LPG);
+      };
+#pragma unroll
+      for (int t = 0; t < FPW; ++t) filters[t] = request_filter(p0, t);
+      request_phase(p0, rows_a);
+#pragma unroll
+      for (int t = 0; t < FPW; ++t) store_filter(filters[t], t, 0);
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int t = 0; t < FPW; ++t) filters[t] = request_filter(p1, t);
+      request_phase(p1, rows_b);
+      ldsBarrier();
+    }
+    // (two phases a trip and one way out of the loop, at the price of an empty phase at the end of an
+    // odd number of them: with a second way out the compiler waits for all loads at the loop's head)
+    do {
+      p2 = next_phase(left);
+      take_phase(p2, 0, rows_a);
+      p0 = next_phase(left);
+      take_phase(p0, 1, rows_b);
+      p1 = p0;
+      p0 = p2;
+    } while (p0 != 0);
     }
   }
   // lane holds result columns 16*nb + 4*quad + (0..3) of row 16*g + pair of its wave's rows
@@ -1483,14 +1835,10 @@ __global__ __launch_bounds__(64 * kDenseWaves) __attribute__((amdgpu_waves_per_e
     if (r >= R) continue;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-      S *dst = result + (size_t)r * ldc + col_group * C + nb * 16 + quad * 4;
       S tmp[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) E::store(&tmp[e], acc[g][nb][e]);
-      if constexpr (sizeof(S) == 2)
-        *reinterpret_cast<uint2 *>(dst) = *reinterpret_cast<const uint2 *>(tmp);
-      else
-        *reinterpret_cast<uint4 *>(dst) = *reinterpret_cast<const uint4 *>(tmp);
+      storeColumns<E>(result + (size_t)r * conv.c, nb * 16 + quad * 4, conv.c, tmp);
     }
   }
   if constexpr (!SRC::kSegments) {
@@ -1501,7 +1849,7 @@ __global__ __launch_bounds__(64 * kDenseWaves) __attribute__((amdgpu_waves_per_e
     for (int d = 32; d > 0; d >>= 1) wave_slots += __shfl_xor(wave_slots, d, kWave);
     if (lane == 0) s_has[wave] = wave_slots;
     __syncthreads();
-    if (tid == 0 && blockIdx.y == 0) {
+    if (tid == 0) {
       int all = 0;
       for (int w = 0; w < WAVES; ++w) all += s_has[w];
       source.filled[blockIdx.x] = all;
@@ -1865,10 +2213,39 @@ __device__ __forceinline__ SlicePlace sliceOfWorkgroup(const SliceOrder &order, 
 // writes two runs of 32 consecutive pairs, which no two lanes share a bank in
 // (with a row's pieces spread over eight lanes the same stores hit 8 banks and
 // took 28 cycles each).  Wave w multiplies the 16-row blocks w, w+4, ... of dW[k]
-// against all column blocks.
+// against all column blocks.  Rows are `rows.ci` and `rows.co` channels long: the channels
+// behind them, up to CI and CO, are zeros.
+
+// The channels of the feature and gradient rows, at most the CI and CO of the instance.
+struct FilterGradRows {
+  int ci, co;
+};
+
+// Elements [c0, c0 + 16 bytes) of a row of `channels`, zeros behind its end.  (Rows need no
+// alignment: the memory path takes 16 bytes from any address.)
+template <typename S>
+__device__ __forceinline__ u32x4 rowPiece(const S *row, int c0, int channels) {
+  constexpr int EPP = 16 / (int)sizeof(S);
+  u32x4 piece = {0u, 0u, 0u, 0u};
+  if (c0 + EPP <= channels) {
+    __builtin_memcpy(&piece, row + c0, 16);
+  } else {
+#pragma unroll
+    for (int e = 0; e < EPP; ++e) {
+      if (c0 + e < channels) {
+        if constexpr (sizeof(S) == 2)
+          piece[e >> 1] |= (uint32_t)reinterpret_cast<const u16 *>(row)[c0 + e] << ((e & 1) * 16);
+        else
+          piece[e] = reinterpret_cast<const uint32_t *>(row)[c0 + e];
+      }
+    }
+  }
+  return piece;
+}
+
 template <typename E, int CI, int CO>
 __global__ __launch_bounds__(256) void backwardFilterMfma(
-    const typename E::storage *X, const typename E::storage *dY, const int32_t *pairs, int L,
+    const typename E::storage *X, const typename E::storage *dY, FilterGradRows rows, const int32_t *pairs, int L,
     int x_col, int n_in, int n_out, int K, SliceTable tab, SliceOrder order, int total_slices,
     int slice_len, float *partial) {
   typedef typename E::vec8 vec8;
@@ -1921,8 +2298,7 @@ __global__ __launch_bounds__(256) void backwardFilterMfma(
       if (XU >= 4 || u < XU) {
         const int row = s_in[local + (u & 1) * 32 + (lane >> 1)];
         if (row >= 0)
-          xr[i] = *reinterpret_cast<const u32x4 *>(X + (size_t)row * CI +
-                                                   ((u >> 1) * 2 + (lane & 1)) * EPP);
+          xr[i] = rowPiece(X + (size_t)row * rows.ci, ((u >> 1) * 2 + (lane & 1)) * EPP, rows.ci);
       }
     }
 #pragma unroll
@@ -1932,8 +2308,7 @@ __global__ __launch_bounds__(256) void backwardFilterMfma(
       if (YU >= 4 || u < YU) {
         const int row = s_out[local + (u & 1) * 32 + (lane >> 1)];
         if (row >= 0)
-          yr[i] = *reinterpret_cast<const u32x4 *>(dY + (size_t)row * CO +
-                                                   ((u >> 1) * 2 + (lane & 1)) * EPP);
+          yr[i] = rowPiece(dY + (size_t)row * rows.co, ((u >> 1) * 2 + (lane & 1)) * EPP, rows.co);
       }
     }
   };
@@ -2026,7 +2401,8 @@ __global__ __launch_bounds__(256) void backwardFilterMfma(
   }
 }
 
-// The same product for 2-byte elements and 32 to 128 channels on both sides, with the
+// The same product for 2-byte elements, 17 to 128 channels on both sides and rows of whole
+// 16-byte pieces (an LDS request takes one), with the
 // transposition done by the LDS read itself.  The gathered rows go from global memory
 // straight into LDS as they are ([pair][channel], 16 bytes per lane, a pair without a
 // valid row reads a row of zeros), one step of 64 (or 32) pairs ahead into the other of two
@@ -2047,7 +2423,7 @@ constexpr int filterRowSwizzle(int row_bytes, int pair) {
 
 template <typename E, int CI, int CO, int SP>
 __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
-    const typename E::storage *X, const typename E::storage *dY, const int32_t *pairs, int L,
+    const typename E::storage *X, const typename E::storage *dY, FilterGradRows rows, const int32_t *pairs, int L,
     int x_col, int n_in, int n_out, int K, SliceTable tab, SliceOrder order, int total_slices,
     int slice_len, float *partial) {
   typedef typename E::vec8 vec8;
@@ -2118,8 +2494,10 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
       const int row_bytes = is_x ? RBX : RBY;
       const int byte = (wave + (is_x ? u : u - XM) * 4) * 1024 + lane * 16;
       const int piece = ((byte % row_bytes) / 16) ^ filterRowSwizzle(row_bytes, byte / row_bytes);
-      const char *rows = reinterpret_cast<const char *>(is_x ? (const void *)X : (const void *)dY);
-      loads.from[u] = (live && row[u] >= 0 ? rows + (size_t)row[u] * row_bytes : zero_row) + piece * 16;
+      const char *from = reinterpret_cast<const char *>(is_x ? (const void *)X : (const void *)dY);
+      const int length = (is_x ? rows.ci : rows.co) * 2;  // bytes; zeros behind them
+      loads.from[u] =
+          (live && row[u] >= 0 && piece * 16 < length ? from + (size_t)row[u] * length : zero_row) + piece * 16;
     }
   };
   auto request = [&](const StepLoads &loads, int u, int buffer) {
@@ -2232,7 +2610,7 @@ constexpr int kSliceSumWaves = 16;
 template <typename E>
 __global__ __launch_bounds__(64 * kSliceSumWaves) void sliceSum(const float *partial,
                                                                 SliceTable tab, int slice_len,
-                                                                int tile_elems, int Co,
+                                                                int tile_elems, int tile_co, FilterGradRows rows,
                                                                 GradLayout lay,
                                                                 typename E::storage *dW) {
   constexpr int W = kSliceSumWaves;
@@ -2266,8 +2644,10 @@ __global__ __launch_bounds__(64 * kSliceSumWaves) void sliceSum(const float *par
 #pragma unroll
       for (int i = 0; i < W; i += 2 * span) t[i] += t[i + span];
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
-      E::store(dW + gradOffset(lay, k, (e + v) / Co, (e + v) % Co), t[0][v]);
+    for (int v = 0; v < 4; ++v) {
+      const int ci = (e + v) / tile_co, co = (e + v) % tile_co;
+      if (ci < rows.ci && co < rows.co) E::store(dW + gradOffset(lay, k, ci, co), t[0][v]);
+    }
   }
 }
 
@@ -2287,7 +2667,7 @@ template <typename E>
 __global__ __launch_bounds__(64 * kSliceSumWaves) void sliceSumFlat(const float *partial,
                                                                     SliceTable tab, SumGrid grid,
                                                                     int K, int slice_len,
-                                                                    int tile_elems, int Co,
+                                                                    int tile_elems, int tile_co, FilterGradRows rows,
                                                                     GradLayout lay,
                                                                     typename E::storage *dW) {
   constexpr int W = kSliceSumWaves;
@@ -2318,8 +2698,10 @@ __global__ __launch_bounds__(64 * kSliceSumWaves) void sliceSumFlat(const float 
 #pragma unroll
       for (int i = 0; i < W; i += 2 * span) t[i] += t[i + span];
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
-      E::store(dW + gradOffset(lay, k, (e + v) / Co, (e + v) % Co), t[0][v]);
+    for (int v = 0; v < 4; ++v) {
+      const int ci = (e + v) / tile_co, co = (e + v) % tile_co;
+      if (ci < rows.ci && co < rows.co) E::store(dW + gradOffset(lay, k, ci, co), t[0][v]);
+    }
     return;
   }
   const int e = (chunk * 64 + lane) * 4;
@@ -2347,8 +2729,10 @@ __global__ __launch_bounds__(64 * kSliceSumWaves) void sliceSumFlat(const float 
 #pragma unroll
       for (int i = 0; i < W; i += 2 * span) t[i] += t[i + span];
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
-      E::store(dW + gradOffset(lay, k, (e + v) / Co, (e + v) % Co), t[0][v]);
+    for (int v = 0; v < 4; ++v) {
+      const int ci = (e + v) / tile_co, co = (e + v) % tile_co;
+      if (ci < rows.ci && co < rows.co) E::store(dW + gradOffset(lay, k, ci, co), t[0][v]);
+    }
   }
 }
 
@@ -2373,19 +2757,24 @@ inline int gridFor(size_t n, int cap = 8192) {
 // workgroups on (or as the handle's kernel choice says; the two kernels give the same bits).
 constexpr int kFlatSumFromBlocks = 2048;
 
-// fp16/bf16: 16x16x32 MFMA; float: 16x16x4 MFMA; reduction channels in {16, 32, 64, 128}.
-bool mfmaShapeOk(ElemType t, int Q, int C) {
-  (void)t;  // 16 channels of a 2-byte type run as half-filled fragments
-  const bool q_ok = (Q == 16 || Q == 32 || Q == 64 || Q == 128);
-  const bool c_ok = (C == 16 || C == 32 || C == 64 || C == 128);
-  return q_ok && c_ok;
-}
+// The matrix-core kernels are compiled for 16, 32, 64 and 128 channels (fp16/bf16: 16x16x32
+// MFMA, 16 channels as half-filled fragments; float: 16x16x4); a tensor of up to 128 channels
+// runs on the next of these.
+int paddedChannels(int c) { return c <= 16 ? 16 : (c <= 32 ? 32 : (c <= 64 ? 64 : 128)); }
+bool mfmaShapeOk(int Q, int C) { return Q >= 1 && Q <= 128 && C >= 1 && C <= 128; }
+
+// They read rows in 16-byte pieces.  Rows of another length (4 or 5 point features, 12 channels
+// of a 2-byte type) are copied to padded rows in the workspace first, by workgroups of the
+// launch that prepares the filter.
+int paddedRowBytes(ElemType t, int channels) { return (channels * (int)elemSize(t) + 15) / 16 * 16; }
+bool rowsNeedPadding(ElemType t, int channels) { return channels * (int)elemSize(t) % 16 != 0; }
 
 struct GatherDims {
   int R;       // result rows
   int n_src;   // rows of the gathered tensor
   int Q;       // reduction channels
   int C;       // result channels
+  int q_padded, c_padded;  // of the matrix-core instance
   int row_col, src_col;
   bool filter_forward;  // B(k, q, c) = W(k, ci = q, co = c); otherwise its transpose
 };
@@ -2398,6 +2787,8 @@ GatherDims gatherDims(const ConvProblem &p, GatherDirection dir) {
   } else {
     d.Q = p.Co; d.C = p.Ci;
   }
+  d.q_padded = paddedChannels(d.Q);
+  d.c_padded = paddedChannels(d.C);
   // The result rows are the pair column the operator writes through: column 1
   // for forward, column 0 for backward data, and the other way round for an
   // inverse convolution, which runs its partner's rulebook backwards.
@@ -2429,6 +2820,7 @@ struct GatherWorkspace {
   float *pool = nullptr;
   int32_t *map = nullptr;
   void *packed = nullptr;
+  void *padded_rows = nullptr;  // the gathered tensor with rows of whole 16-byte pieces
   size_t bytes = 0;
 };
 
@@ -2479,11 +2871,12 @@ GatherWorkspace carveGather(const ConvProblem &p, const GatherDims &d, void *bas
   ws.pool_row = reinterpret_cast<int32_t *>(take(repair_blocks * kRepairPoolRows * 4));
   ws.pool = reinterpret_cast<float *>(take(repair_blocks * kRepairPoolRows * d.C * 4));
   ws.map = reinterpret_cast<int32_t *>(take((size_t)p.K * ws.map_rows * 4));
-  if (mfmaShapeOk(p.dtype, d.Q, d.C)) {
+  if (mfmaShapeOk(d.Q, d.C)) {
     // reduction channels are padded to whole 16-byte fragments (32 for the 2-byte types)
     const size_t chunk = 64 / elemSize(p.dtype);
-    const size_t q_padded = ((size_t)d.Q + chunk - 1) / chunk * chunk;
-    ws.packed = take((size_t)p.K * q_padded * d.C * elemSize(p.dtype));
+    const size_t q_padded = ((size_t)d.q_padded + chunk - 1) / chunk * chunk;
+    ws.packed = take((size_t)p.K * q_padded * d.c_padded * elemSize(p.dtype));
+    if (rowsNeedPadding(p.dtype, d.Q)) ws.padded_rows = take((size_t)d.n_src * paddedRowBytes(p.dtype, d.Q));
   }
   ws.bytes = off + kBaseAlign;
   return ws;
@@ -2525,7 +2918,7 @@ hipError_t prepareCounts(const LaunchCtx &lc, const ConvProblem &p, OffsetCounts
 // 64-column halves over 128-row tiles: twice the entries in every block for
 // the same accumulator size, at the price of gathering each row twice.
 int mfmaTileCols(const ConvProblem &p, const GatherDims &d) {
-  if (d.C != 128) return d.C;
+  if (d.c_padded != 128) return d.c_padded;
   double pairs = 0;
   for (int k = 0; k < p.K; ++k) pairs += (double)p.indice_num[k];
   const double per_tile_offset = pairs * mfmaTileRows(128) / ((double)d.R * p.K);
@@ -2537,72 +2930,69 @@ int mfmaGridX(int R, int tile_cols) {
   const int tr = mfmaTileRows(tile_cols);
   return ((R + tr - 1) / tr + 7) / 8 * 8;
 }
-int denseGridX(int R, int Q, int C) {
-  const int rows = denseTileRows(Q, C);
-  return ((R + rows - 1) / rows + 7) / 8 * 8;
-}
+int denseGridX(int R, int tile_rows) { return ((R + tile_rows - 1) / tile_rows + 7) / 8 * 8; }
 
 template <typename E, int Q, int C, typename SRC>
-void launchMfmaInstance(const LaunchCtx &lc, const void *A, const void *packed,
-                        const SRC &source, int R, int K, int ldc, void *result) {
+void launchMfmaInstance(const LaunchCtx &lc, const void *A, const ConvRows &rows, const void *packed,
+                        const SRC &source, int R, int K, void *result) {
   constexpr int NT = mfmaThreads(C);
-  const dim3 grid(mfmaGridX(R, C), ldc / C);
+  const dim3 grid(mfmaGridX(R, C), (rows.c + C - 1) / C);
   lc.begin("gatherConvMfma");
   gatherConvMfma<E, Q, C, SRC><<<grid, NT, 0, lc.stream>>>(
-      static_cast<const typename E::storage *>(A),
-      static_cast<const typename E::storage *>(packed), source, R, K, ldc,
+      static_cast<const typename E::storage *>(A), rows,
+      static_cast<const typename E::storage *>(packed), source, R, K,
       static_cast<typename E::storage *>(result));
   lc.end();
 }
 
-// `tile_cols` result columns per workgroup out of C: a narrower tile has more
-// rows, so sparse rulebooks fill their 16-pair blocks better.
+// `tile_cols` result columns per workgroup: a narrower tile has more rows, so sparse
+// rulebooks fill their 16-pair blocks better.
 template <typename E, int Q, typename SRC>
-void launchMfmaByC(const LaunchCtx &lc, int C, int tile_cols, const void *A, const void *packed,
+void launchMfmaByC(const LaunchCtx &lc, int tile_cols, const void *A, const ConvRows &rows, const void *packed,
                    const SRC &source, int R, int K, void *result) {
   switch (tile_cols) {
-    case 16: launchMfmaInstance<E, Q, 16, SRC>(lc, A, packed, source, R, K, C, result); break;
-    case 32: launchMfmaInstance<E, Q, 32, SRC>(lc, A, packed, source, R, K, C, result); break;
-    case 64: launchMfmaInstance<E, Q, 64, SRC>(lc, A, packed, source, R, K, C, result); break;
-    case 128: launchMfmaInstance<E, Q, 128, SRC>(lc, A, packed, source, R, K, C, result); break;
+    case 16: launchMfmaInstance<E, Q, 16, SRC>(lc, A, rows, packed, source, R, K, result); break;
+    case 32: launchMfmaInstance<E, Q, 32, SRC>(lc, A, rows, packed, source, R, K, result); break;
+    case 64: launchMfmaInstance<E, Q, 64, SRC>(lc, A, rows, packed, source, R, K, result); break;
+    case 128: launchMfmaInstance<E, Q, 128, SRC>(lc, A, rows, packed, source, R, K, result); break;
     default: break;
   }
 }
 
 template <typename E, typename SRC>
-void launchMfma(const LaunchCtx &lc, int Q, int C, int tile_cols, const void *A, const void *packed,
-                const SRC &source, int R, int K, void *result) {
-  switch (Q) {
-    case 16: launchMfmaByC<E, 16, SRC>(lc, C, tile_cols, A, packed, source, R, K, result); break;
-    case 32: launchMfmaByC<E, 32, SRC>(lc, C, tile_cols, A, packed, source, R, K, result); break;
-    case 64: launchMfmaByC<E, 64, SRC>(lc, C, tile_cols, A, packed, source, R, K, result); break;
-    case 128: launchMfmaByC<E, 128, SRC>(lc, C, tile_cols, A, packed, source, R, K, result); break;
+void launchMfma(const LaunchCtx &lc, int q_padded, int tile_cols, const void *A, const ConvRows &rows,
+                const void *packed, const SRC &source, int R, int K, void *result) {
+  switch (q_padded) {
+    case 16: launchMfmaByC<E, 16, SRC>(lc, tile_cols, A, rows, packed, source, R, K, result); break;
+    case 32: launchMfmaByC<E, 32, SRC>(lc, tile_cols, A, rows, packed, source, R, K, result); break;
+    case 64: launchMfmaByC<E, 64, SRC>(lc, tile_cols, A, rows, packed, source, R, K, result); break;
+    case 128: launchMfmaByC<E, 128, SRC>(lc, tile_cols, A, rows, packed, source, R, K, result); break;
     default: break;
   }
 }
 
 template <typename E, int Q, int C>
-void launchWaveInstance(const LaunchCtx &lc, const void *A, const void *packed,
+void launchWaveInstance(const LaunchCtx &lc, const void *A, const ConvRows &rows, const void *packed,
                         const SegmentSource &source, int R, int K, void *result) {
   if constexpr (waveKernelShape((int)sizeof(typename E::storage), Q, C)) {
     const int grid = ((R + kWaveTileRows - 1) / kWaveTileRows + 7) / 8 * 8;
     lc.begin("gatherConvWave");
     gatherConvWave<E, Q, C><<<grid, 64, 0, lc.stream>>>(
-        static_cast<const typename E::storage *>(A), static_cast<const typename E::storage *>(packed),
+        static_cast<const typename E::storage *>(A), rows, static_cast<const typename E::storage *>(packed),
         source, R, K, static_cast<typename E::storage *>(result));
     lc.end();
   }
 }
 
 template <typename E>
-void launchWave(const LaunchCtx &lc, int Q, int C, const void *A, const void *packed,
+void launchWave(const LaunchCtx &lc, int q_padded, const void *A, const ConvRows &rows, const void *packed,
                 const SegmentSource &source, int R, int K, void *result) {
 #define WAVE_CASE(q)                                                                      \
   case q:                                                                                 \
-    if (C == 16) launchWaveInstance<E, q, 16>(lc, A, packed, source, R, K, result);       \
-    else launchWaveInstance<E, q, 32>(lc, A, packed, source, R, K, result);               \
+    if (rows.c_padded == 16) launchWaveInstance<E, q, 16>(lc, A, rows, packed, source, R, K, result); \
+    else launchWaveInstance<E, q, 32>(lc, A, rows, packed, source, R, K, result);         \
     break;
-  switch (Q) {
+  switch (q_padded) {
     WAVE_CASE(16)
     WAVE_CASE(32)
     WAVE_CASE(64)
@@ -2617,16 +3007,15 @@ bool useWaveKernel(const LaunchCtx &lc, ElemType t, int Q, int C) {
   return waveKernelShape((int)elemSize(t), Q, C);
 }
 
-// The register-accumulating kernel takes 16 to 128 result columns and 16 to 128 reduction
-// channels (16 channels of a 2-byte type as half a fragment).
-bool denseShapeOk(ElemType t, int Q, int C) {
-  // fp32 rows of 128 channels leave no room for two sets of partner rows and the fragments
-  if (t == ElemType::kFloat && Q > 64) return false;
-  return (C == 16 || C == 32 || C == 64 || C == 128) && (Q == 16 || Q == 32 || Q == 64 || Q == 128);
+// The register-accumulating kernel addresses the gathered tensor with 32-bit byte offsets.
+bool denseShapeOk(const ConvProblem &p, const GatherDims &d) {
+  // (fp32 rows of more than 64 channels leave no room for two row groups a wave)
+  if (p.dtype == ElemType::kFloat && d.Q > 64) return false;
+  return (uint64_t)d.n_src * (uint64_t)paddedRowBytes(p.dtype, d.Q) < (uint64_t)kNoRow;
 }
 
 bool useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d) {
-  if (!denseShapeOk(p.dtype, d.Q, d.C)) return false;
+  if (!denseShapeOk(p, d)) return false;
   if (lc.choices.dense_tiles >= 0) return lc.choices.dense_tiles == 1;
   // What the kernel costs goes with the (tile, offset) pieces that hold a pair at all, what
   // the pair-list kernels cost with the pairs.  Measured on 150000 rows, 3x3x3, fp16, as the
@@ -2654,37 +3043,40 @@ bool useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims 
   // (the largest count is the centre offset of a submanifold convolution: left out)
   const double mean_rest = p.K > 1 ? (pairs - largest) / (p.K - 1) : 0.0;
   const bool sheets = mean_rest > 0 && second >= 1.5 * mean_rest;
-  if (d.C <= 32) return fill >= (sheets ? 0.04 : 0.35);
-  if (d.C == 64) return fill >= (sheets ? 0.15 : 0.38);
+  if (d.c_padded <= 32) return fill >= (sheets ? 0.04 : 0.35);
+  if (d.c_padded == 64) return fill >= (sheets ? 0.15 : 0.38);
   return fill >= (sheets ? 0.04 : 0.25);
 }
 
 template <typename E, int Q, int C, typename SRC>
-void launchDenseInstance(const LaunchCtx &lc, const void *A, const void *packed, const SRC &source,
-                         int R, int K, void *result) {
-  const dim3 grid(denseGridX(R, Q, C), 1);
+void launchDenseInstance(const LaunchCtx &lc, const void *A, uint32_t a_size, const ConvRows &rows, const void *packed,
+                         const SRC &source, int R, int K, void *result) {
   lc.begin("gatherConvDense");
-  gatherConvDense<E, Q, C, SRC><<<grid, 64 * kDenseWaves, 0, lc.stream>>>(
-      static_cast<const typename E::storage *>(A), static_cast<const typename E::storage *>(packed),
-      source, R, K, C, static_cast<typename E::storage *>(result));
+  constexpr int kElem = (int)sizeof(typename E::storage);
+  gatherConvDense<E, Q, C, SRC><<<denseGridX(R, denseTileRows(kElem, Q, C)), 64 * densePlan(kElem, Q, C).waves, 0,
+                                  lc.stream>>>(
+      static_cast<const typename E::storage *>(A), a_size, rows, static_cast<const typename E::storage *>(packed),
+      source, R, K, static_cast<typename E::storage *>(result));
   lc.end();
 }
 
 template <typename E, typename SRC>
-void launchDense(const LaunchCtx &lc, int Q, int C, const void *A, const void *packed,
+void launchDense(const LaunchCtx &lc, int q_padded, const void *A, int n_src, const ConvRows &rows, const void *packed,
                  const SRC &source, int R, int K, void *result) {
-  constexpr bool is_float = std::is_same<E, FloatElem>::value;
-#define DENSE_BY_C(q)                                                                           \
-  if (C == 16) launchDenseInstance<E, q, 16, SRC>(lc, A, packed, source, R, K, result);         \
-  else if (C == 32) launchDenseInstance<E, q, 32, SRC>(lc, A, packed, source, R, K, result);    \
-  else if (C == 64) launchDenseInstance<E, q, 64, SRC>(lc, A, packed, source, R, K, result);    \
-  else launchDenseInstance<E, q, 128, SRC>(lc, A, packed, source, R, K, result);
-  switch (Q) {
+  const uint32_t a_size = (uint32_t)n_src * (uint32_t)rows.row_bytes;
+#define DENSE_BY_C(q)                                                                                     \
+  switch (rows.c_padded) {                                                                                \
+    case 16: launchDenseInstance<E, q, 16, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break;  \
+    case 32: launchDenseInstance<E, q, 32, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break;  \
+    case 64: launchDenseInstance<E, q, 64, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break;  \
+    default: launchDenseInstance<E, q, 128, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break; \
+  }
+  switch (q_padded) {
     case 16: DENSE_BY_C(16) break;
     case 32: DENSE_BY_C(32) break;
     case 64: DENSE_BY_C(64) break;
     case 128:
-      if constexpr (!is_float) { DENSE_BY_C(128) }
+      if constexpr (!std::is_same<E, FloatElem>::value) { DENSE_BY_C(128) }
       break;
     default: break;
   }
@@ -2742,6 +3134,13 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
   // B(k, q, c): forward q = ci, c = co; backward data q = co, c = ci.
   const int64_t sQ = d.filter_forward ? f.stride_ci : f.stride_co;
   const int64_t sC = d.filter_forward ? f.stride_co : f.stride_ci;
+  const FilterShape shape = {d.Q, d.C, d.q_padded, d.c_padded};
+  const bool pad_rows = use_mfma && rowsNeedPadding(p.dtype, d.Q);
+  const ConvRows rows_of = {d.Q, pad_rows ? paddedRowBytes(p.dtype, d.Q) : d.Q * (int)sizeof(S), d.C, d.c_padded};
+  const void *rows_from = pad_rows ? ws.padded_rows : gathered;
+  const PadRows pad = {static_cast<const char *>(gathered), static_cast<char *>(ws.padded_rows), d.Q * (int)sizeof(S),
+                       rows_of.row_bytes, pad_rows ? d.n_src : 0, pad_rows ? gridFor((size_t)d.n_src, 1024) : 0};
+  const size_t frags = (size_t)p.K * (d.c_padded / 16) * ((d.q_padded + E::kChunk - 1) / E::kChunk) * 64;
   const bool single_chunk = p.row_map == nullptr && ws.map_rows >= d.R && lc.choices.small_map_chunks != 1;
   // Pair lists whose order nobody has reported yet: the call starts on them all the same,
   // and the row-map kernels are enqueued behind, each of them told to return at once unless
@@ -2753,8 +3152,8 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     // Pair lists in order (as far as the caller knows: the first kernel checks): the
     // gather kernel reads them cut by tile, no row map.
     const bool dense = useDenseKernel(lc, p, d);
-    const int tile_cols = dense ? d.C : mfmaTileCols(p, d);
-    const int tile_rows = dense ? denseTileRows(d.Q, d.C) : mfmaTileRows(tile_cols);
+    const int tile_cols = dense ? d.c_padded : mfmaTileCols(p, d);
+    const int tile_rows = dense ? denseTileRows((int)sizeof(S), d.q_padded, d.c_padded) : mfmaTileRows(tile_cols);
     int tile_shift = 0;
     while ((1 << tile_shift) < tile_rows) ++tile_shift;
     const int n_tiles = (d.R + tile_rows - 1) / tile_rows;
@@ -2765,11 +3164,10 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
       const int per_block = 256 * kCutPairsPerThread;
       if (k < p.K) list_blocks += inl.n[k] > 0 ? (inl.n[k] + per_block - 1) / per_block : 1;
     }
-    const size_t frags = (size_t)p.K * (d.C / 16) * ((d.Q + E::kChunk - 1) / E::kChunk) * 64;
     const int pack_blocks = gridFor(frags, 512);
     lc.begin("packFilterCutPairLists");
-    packFilterCutPairLists<E><<<pack_blocks + list_blocks, 256, 0, lc.stream>>>(
-        static_cast<const S *>(f.base), f.stride_k, sQ, sC, p.K, d.Q, d.C, static_cast<S *>(ws.packed),
+    packFilterCutPairLists<E><<<pad.blocks + pack_blocks + list_blocks, 256, 0, lc.stream>>>(
+        pad, static_cast<const S *>(f.base), f.stride_k, sQ, sC, p.K, shape, static_cast<S *>(ws.packed),
         pack_blocks, p.indice_pairs, p.L, inl, ob, d.row_col, d.src_col, d.R, d.n_src, tile_shift,
         n_tiles, ws.cuts, ws.verdict, p.ticket);
     lc.end();
@@ -2790,11 +3188,11 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     src.sC = sC;
     src.counts = inl;
     if (dense)
-      launchDense<E, SegmentSource>(lc, d.Q, d.C, gathered, ws.packed, src, d.R, p.K, result);
-    else if (tile_cols == d.C && useWaveKernel(lc, p.dtype, d.Q, d.C))
-      launchWave<E>(lc, d.Q, d.C, gathered, ws.packed, src, d.R, p.K, result);
+      launchDense<E, SegmentSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, src, d.R, p.K, result);
+    else if (tile_cols == d.c_padded && useWaveKernel(lc, p.dtype, d.q_padded, d.c_padded))
+      launchWave<E>(lc, d.q_padded, rows_from, rows_of, ws.packed, src, d.R, p.K, result);
     else
-      launchMfma<E, SegmentSource>(lc, d.Q, d.C, tile_cols, gathered, ws.packed, src, d.R, p.K, result);
+      launchMfma<E, SegmentSource>(lc, d.q_padded, tile_cols, rows_from, rows_of, ws.packed, src, d.R, p.K, result);
     if (!speculate || lc.choices.lists_on_trust == 1) return;
   }
   // What follows runs always, or (behind lists taken on trust) only when they failed the check.
@@ -2805,7 +3203,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
   int chunk_rows = own_map ? ws.map_rows : d.R;
   if (own_map && lc.choices.small_map_chunks == 1 && chunk_rows > kRepairPoolRows) chunk_rows = kRepairPoolRows;
   const bool dense = use_mfma && useDenseKernel(lc, p, d);
-  const int tile_cols = use_mfma && !dense ? mfmaTileCols(p, d) : d.C;
+  const int tile_cols = use_mfma && !dense ? mfmaTileCols(p, d) : d.c_padded;
   for (int row_base = 0; row_base < d.R; row_base += chunk_rows) {
     const int rows = d.R - row_base < chunk_rows ? d.R - row_base : chunk_rows;
     const size_t map_elems = (size_t)p.K * rows;
@@ -2816,24 +3214,25 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     if (use_mfma) {
       // the filter is repacked with the first chunk's map fill (the list kernels' first
       // launch has done it already where they ran)
-      const size_t frags = (size_t)p.K * (d.C / 16) * ((d.Q + E::kChunk - 1) / E::kChunk) * 64;
       const int fill_blocks = own_map ? gridFor(map_elems / 4 + 1, 2048) : 0;
       const int pack_blocks = row_base == 0 && !lists ? gridFor(frags, 512) : 0;
+      PadRows pad_now = pad;
+      if (pack_blocks == 0) pad_now.blocks = 0;
       if (fill_blocks + pack_blocks > 0) {
         lc.begin("fillMapPackFilter");
-        fillMapPackFilter<E><<<fill_blocks + pack_blocks, 256, 0, lc.stream>>>(
-            ws.map, map_elems, fill_blocks, static_cast<const S *>(f.base), f.stride_k, sQ, sC, p.K,
-            d.Q, d.C, static_cast<S *>(ws.packed), run_if);
+        fillMapPackFilter<E><<<pad_now.blocks + fill_blocks + pack_blocks, 256, 0, lc.stream>>>(
+            pad_now, ws.map, map_elems, fill_blocks, static_cast<const S *>(f.base), f.stride_k, sQ, sC, p.K,
+            shape, static_cast<S *>(ws.packed), run_if);
         lc.end();
       }
       if (own_map) n_accepted = launchScatterRowMap(lc, p, d, ws, inl, max_count, row_base, rows, run_if);
       const MapSource map = {entries, ws.filled, run_if};
       if (dense) {
-        n_filled = denseGridX(rows, d.Q, d.C);
-        launchDense<E, MapSource>(lc, d.Q, d.C, gathered, ws.packed, map, rows, p.K, result_rows);
+        n_filled = denseGridX(rows, denseTileRows((int)sizeof(S), d.q_padded, d.c_padded));
+        launchDense<E, MapSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K, result_rows);
       } else {
         n_filled = mfmaGridX(rows, tile_cols);
-        launchMfma<E, MapSource>(lc, d.Q, d.C, tile_cols, gathered, ws.packed, map, rows, p.K, result_rows);
+        launchMfma<E, MapSource>(lc, d.q_padded, tile_cols, rows_from, rows_of, ws.packed, map, rows, p.K, result_rows);
       }
     } else {
       if (own_map) {
@@ -2871,8 +3270,7 @@ struct FilterGradWorkspace {
 };
 
 bool filterMfmaShapeOk(const ConvProblem &p) {
-  auto ok = [](int c) { return c == 16 || c == 32 || c == 64 || c == 128; };
-  return ok(p.Ci) && ok(p.Co) && p.K <= kMaxInlineK;
+  return mfmaShapeOk(p.Ci, p.Co) && p.K <= kMaxInlineK;
 }
 
 // Slices the MFMA kernels cut the pair lists into at most: kFilterMaxSlices (fewer for many
@@ -2904,11 +3302,14 @@ FilterGradWorkspace carveFilterGrad(const ConvProblem &p, void *base) {
   };
   if (p.K > kMaxInlineK) ws.dev_counts = reinterpret_cast<int32_t *>(take((size_t)p.K * 4));
   ws.splits = filterGradSplits(p);
-  size_t tiles = ws.splits > 1 ? (size_t)ws.splits * p.K : 0;
-  // the MFMA path writes at most filterMaxSlices + K partial tiles
-  if (filterMfmaShapeOk(p) && (size_t)filterMaxSlices(p) + p.K > tiles)
-    tiles = (size_t)filterMaxSlices(p) + p.K;
-  if (tiles > 0) ws.partial = reinterpret_cast<float *>(take(tiles * p.Ci * p.Co * 4));
+  size_t elems = ws.splits > 1 ? (size_t)ws.splits * p.K * p.Ci * p.Co : 0;
+  // the MFMA path writes at most filterMaxSlices + K partial tiles of padded channels
+  if (filterMfmaShapeOk(p)) {
+    const size_t tiles = (size_t)filterMaxSlices(p) + p.K;
+    const size_t mfma_elems = tiles * paddedChannels(p.Ci) * paddedChannels(p.Co);
+    if (mfma_elems > elems) elems = mfma_elems;
+  }
+  if (elems > 0) ws.partial = reinterpret_cast<float *>(take(elems * 4));
   ws.bytes = off + kBaseAlign;
   return ws;
 }
@@ -2929,33 +3330,26 @@ void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const S
                               const SliceOrder &order, int slice_len, int total_slices, float *partial, const void *features,
                               const void *output_grad, void *filters_grad) {
   typedef typename E::storage S;
-  constexpr bool kTransposingReads = sizeof(S) == 2 && CI >= 32 && CO >= 32;
+  constexpr bool kTransposingShape = sizeof(S) == 2 && CI >= 32 && CO >= 32;
+  const bool transposing = kTransposingShape && lc.choices.filter_stores != 1 &&
+                           !rowsNeedPadding(p.dtype, p.Ci) && !rowsNeedPadding(p.dtype, p.Co);
+  const FilterGradRows rows = {p.Ci, p.Co};
   const int grid = (total_slices + 7) / 8 * 8;
-  lc.begin(kTransposingReads && lc.choices.filter_stores != 1 ? "backwardFilterMfmaTr" : "backwardFilterMfma");
+  lc.begin(transposing ? "backwardFilterMfmaTr" : "backwardFilterMfma");
   if (total_slices > 0) {
-    if constexpr (kTransposingReads) {
-      if (lc.choices.filter_stores != 1) {
-        // Steps of 32 pairs halve the row buffers: below 128 x 128 channels more workgroups
-        // share a CU then, which pays when the slices are long (network 64 x 64: 101 -> 88 us;
-        // on slices of a few steps the shorter steps only add barriers: config 4 23.7 -> 25.3 us).
-        const bool short_steps = CI + CO < 256 && slice_len >= 2048;
-        auto kernel = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32> : backwardFilterMfmaTr<E, CI, CO, 64>;
-        kernel<<<grid, 256, 0, lc.stream>>>(
-            static_cast<const S *>(features), static_cast<const S *>(output_grad), p.indice_pairs,
-            p.L, p.inverse ? 1 : 0, p.inverse ? p.num_out : p.L, p.inverse ? p.L : p.num_out, p.K,
-            tab, order, total_slices, slice_len, partial);
-      } else {
-        backwardFilterMfma<E, CI, CO><<<grid, 256, 0, lc.stream>>>(
-            static_cast<const S *>(features), static_cast<const S *>(output_grad), p.indice_pairs,
-            p.L, p.inverse ? 1 : 0, p.inverse ? p.num_out : p.L, p.inverse ? p.L : p.num_out, p.K,
-            tab, order, total_slices, slice_len, partial);
-      }
-    } else {
-      backwardFilterMfma<E, CI, CO><<<grid, 256, 0, lc.stream>>>(
-          static_cast<const S *>(features), static_cast<const S *>(output_grad), p.indice_pairs,
-          p.L, p.inverse ? 1 : 0, p.inverse ? p.num_out : p.L, p.inverse ? p.L : p.num_out, p.K,
-          tab, order, total_slices, slice_len, partial);
+    auto kernel = backwardFilterMfma<E, CI, CO>;
+    if constexpr (kTransposingShape) {
+      // Steps of 32 pairs halve the row buffers: below 128 x 128 channels more workgroups
+      // share a CU then, which pays when the slices are long (network 64 x 64: 101 -> 88 us;
+      // on slices of a few steps the shorter steps only add barriers: config 4 23.7 -> 25.3 us).
+      const bool short_steps = CI + CO < 256 && slice_len >= 2048;
+      if (transposing)
+        kernel = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32> : backwardFilterMfmaTr<E, CI, CO, 64>;
     }
+    kernel<<<grid, 256, 0, lc.stream>>>(
+        static_cast<const S *>(features), static_cast<const S *>(output_grad), rows, p.indice_pairs, p.L,
+        p.inverse ? 1 : 0, p.inverse ? p.num_out : p.L, p.inverse ? p.L : p.num_out, p.K, tab, order,
+        total_slices, slice_len, partial);
   }
   lc.end();
   // Many offsets of few slices each: the flat grid, on which such an offset takes a
@@ -2973,10 +3367,10 @@ void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const S
   lc.begin("sliceSum");
   if (flat)
     sliceSumFlat<E><<<blocks, 64 * kSliceSumWaves, 0, lc.stream>>>(
-        partial, tab, sg, p.K, slice_len, CI * CO, CO, gradLayout(p), static_cast<S *>(filters_grad));
+        partial, tab, sg, p.K, slice_len, CI * CO, CO, rows, gradLayout(p), static_cast<S *>(filters_grad));
   else
     sliceSum<E><<<dim3(kChunks, p.K), 64 * kSliceSumWaves, 0, lc.stream>>>(
-        partial, tab, slice_len, CI * CO, CO, gradLayout(p), static_cast<S *>(filters_grad));
+        partial, tab, slice_len, CI * CO, CO, rows, gradLayout(p), static_cast<S *>(filters_grad));
   lc.end();
 }
 
@@ -2984,7 +3378,7 @@ template <typename E, int CI>
 void launchFilterMfmaByCo(const LaunchCtx &lc, const ConvProblem &p, const SliceTable &tab,
                           const SliceOrder &order, int slice_len, int total_slices, float *partial, const void *features,
                           const void *output_grad, void *filters_grad) {
-  switch (p.Co) {
+  switch (paddedChannels(p.Co)) {
     case 16: launchFilterMfmaInstance<E, CI, 16>(lc, p, tab, order, slice_len, total_slices, partial, features, output_grad, filters_grad); break;
     case 32: launchFilterMfmaInstance<E, CI, 32>(lc, p, tab, order, slice_len, total_slices, partial, features, output_grad, filters_grad); break;
     case 64: launchFilterMfmaInstance<E, CI, 64>(lc, p, tab, order, slice_len, total_slices, partial, features, output_grad, filters_grad); break;
@@ -3014,7 +3408,7 @@ void launchFilterMfma(const LaunchCtx &lc, const ConvProblem &p, const FilterGra
     // A slice has fixed costs (the first rows' round trip, a Ci x Co fp32 tile written and summed
     // again): few pairs are not cut finer than this, at the price of idle CUs (config 5b, 128 x
     // 128, 400 000 pairs: 56 -> 46 us at 1024; config 2, 32 x 32, 205 000 pairs: 22.5 -> 19 us at 512).
-    const int least = p.Ci * p.Co >= 128 * 128 ? 1024 : 512;
+    const int least = paddedChannels(p.Ci) * paddedChannels(p.Co) >= 128 * 128 ? 1024 : 512;
     if (slice_len < least) slice_len = least;
     int first = 0;
     for (int k = 0; k < kMaxInlineK; ++k) {
@@ -3040,7 +3434,7 @@ void launchFilterMfma(const LaunchCtx &lc, const ConvProblem &p, const FilterGra
           order.offset[placed++] = (uint8_t)k;
           ++next[k];
         }
-    switch (p.Ci) {
+    switch (paddedChannels(p.Ci)) {
       case 16: launchFilterMfmaByCo<E, 16>(lc, p, tab, order, slice_len, first, ws.partial, features, output_grad, filters_grad); break;
       case 32: launchFilterMfmaByCo<E, 32>(lc, p, tab, order, slice_len, first, ws.partial, features, output_grad, filters_grad); break;
       case 64: launchFilterMfmaByCo<E, 64>(lc, p, tab, order, slice_len, first, ws.partial, features, output_grad, filters_grad); break;
@@ -3099,7 +3493,7 @@ hipError_t launchGatherConv(const LaunchCtx &lc, const ConvProblem &p, GatherDir
   // into 24 bits of a list entry.
   const bool ptr_ok =
       ((reinterpret_cast<uintptr_t>(gathered) | reinterpret_cast<uintptr_t>(result)) & 15u) == 0;
-  const bool use_mfma = mfmaShapeOk(p.dtype, d.Q, d.C) && ptr_ok && d.n_src <= (1 << 24) &&
+  const bool use_mfma = mfmaShapeOk(d.Q, d.C) && ptr_ok && d.n_src <= (1 << 24) &&
                         lc.choices.gather_simt != 1;
   switch (p.dtype) {
     case ElemType::kHalf:
