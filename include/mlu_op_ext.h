@@ -94,6 +94,14 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtSetDistinctPairsPromise(mluOpHandle_t handle
 mluOpStatus_t MLUOP_WIN_API mluOpExtGetIndicePairsHostCounts(mluOpHandle_t handle, const void *indice_pairs,
                                                              int kernel_volume, int64_t indice_num[]);
 
+/* The number of voxels of the handle's last mluOpVoxelization on the host.  Its last kernel stores the
+ * number into pinned memory of the handle while it writes the voxels: this call waits for it there,
+ * where a copy of voxel_num waits for the whole queue.  NOT_SUPPORTED if `voxel_num` is not what the
+ * last call wrote, or that call was captured into a graph (copy the number then).  No counterpart in
+ * the reference. */
+mluOpStatus_t MLUOP_WIN_API mluOpExtGetVoxelizationHostCount(mluOpHandle_t handle, const void *voxel_num,
+                                                             int32_t *count);
+
 /* Row maps kept across calls.  mluOpIndiceConvolutionForward and ...BackwardData turn the pair
  * lists into a [K, rows] map (partner row of every result row at every offset, or -1) on every
  * call: the reference API (mlu_op.h:10321-10448, :9625-9773) hands them nothing else to keep.

@@ -73,6 +73,12 @@ struct mluOpContext {
   unsigned long long *rulebook_reports = nullptr;  // kRulebookNotes stamped words behind pinned_scalar
   unsigned long long *count_words = nullptr;   // kRulebookNotes x kCountWords behind those
   int next_rulebook_note = 0;
+  // Where the last voxelization leaves its number of voxels for the host (mluOpExtGetVoxelizationHostCount).
+  struct VoxelCount {
+    const void *voxel_num = nullptr;
+    unsigned long long *word = nullptr;
+    unsigned long long stamp = 0;
+  } voxel_count;
   unsigned long long next_stamp = 1;   // also the source of per-call tickets
 
   // What the kernel launchers need: the stream, and the timer while it is on.

@@ -60,6 +60,7 @@ namespace {
   X(mluOpExtSetSparseConvExtendedModes)                    \
   X(mluOpExtSetDistinctPairsPromise)                       \
   X(mluOpExtGetIndicePairsHostCounts)                      \
+  X(mluOpExtGetVoxelizationHostCount)                      \
   X(mluOpExtUseRowMap)
 
 struct Library {
@@ -442,7 +443,10 @@ std::vector<at::Tensor> voxelization(mluOpHandle_t handle, const Buffers &buffer
   const at::Tensor voxels = buffers.output({max_voxels, max_points, points.size(1)}, at::kFloat, "voxels");
   const at::Tensor coors = buffers.output({max_voxels, 3}, at::kInt, "coors");
   const at::Tensor npv = buffers.output({max_voxels}, at::kInt, "num_points_per_voxel");
-  const at::Tensor num = at::zeros({1}, at::TensorOptions().dtype(at::kInt).device(points.device()));
+  // (a call that keeps nothing enqueues nothing)
+  const at::Tensor num = max_points == 0 || max_voxels == 0
+                             ? at::zeros({1}, points.options().dtype(at::kInt))
+                             : at::empty({1}, points.options().dtype(at::kInt));
   const mluOpTensorLayout_t array = MLUOP_LAYOUT_ARRAY;
   const TensorDesc d_points(array, MLUOP_DTYPE_FLOAT, points.sizes());
   const TensorDesc d_vs(array, MLUOP_DTYPE_FLOAT, {3});
@@ -465,6 +469,22 @@ std::vector<at::Tensor> voxelization(mluOpHandle_t handle, const Buffers &buffer
         "mluOpVoxelization");
   buffers.done("mluOpVoxelization");
   return {voxels, coors, npv, num};
+}
+
+// The same for a layer: cut to the voxels found, whose number the host takes from pinned memory.
+std::vector<at::Tensor> voxelizationCut(bool guarded, const at::Tensor &points, const at::Tensor &voxel_size,
+                                        const at::Tensor &coors_range, int64_t max_points, int64_t max_voxels) {
+  StreamHandle &h = streamHandle();
+  const std::lock_guard<std::mutex> lock(h.mutex);
+  std::vector<at::Tensor> r = voxelization(h.handle, Buffers(guarded, points.device()), points, voxel_size,
+                                           coors_range, max_points, max_voxels, true);
+  int32_t found = 0;
+  if (max_points == 0 || max_voxels == 0 ||
+      api.mluOpExtGetVoxelizationHostCount(h.handle, r[3].data_ptr(), &found) != MLUOP_STATUS_SUCCESS)
+    found = r[3].item<int32_t>();
+  r.pop_back();
+  for (at::Tensor &t : r) t = t.narrow(0, 0, found);
+  return r;
 }
 
 std::vector<at::Tensor> scatterForward(mluOpHandle_t handle, const Buffers &buffers, const at::Tensor &feats,
@@ -593,6 +613,16 @@ PYBIND11_MODULE(_native, m) {
           NoGil released;
           return voxelization(asHandle(handle), Buffers(guarded, points.device()), points, voxel_size, coors_range,
                               max_points, max_voxels, deterministic);
+        });
+  m.def("voxelization_cut",
+        [](bool guarded, const at::Tensor &points, const at::Tensor &voxel_size, const at::Tensor &coors_range,
+           int64_t max_points, int64_t max_voxels) {
+          std::vector<at::Tensor> r;
+          {
+            NoGil released;
+            r = voxelizationCut(guarded, points, voxel_size, coors_range, max_points, max_voxels);
+          }
+          return py::make_tuple(r[0], r[1], r[2]);
         });
   m.def("dynamic_point_to_voxel_forward",
         [](uintptr_t handle, bool guarded, const at::Tensor &feats, const at::Tensor &coors, int mode, int64_t rows) {

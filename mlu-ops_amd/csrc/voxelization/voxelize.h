@@ -19,22 +19,20 @@ struct VoxelizeShape {
   int max_voxels;
 };
 
-// Most points one call accepts (the hash table has twice as many slots and is
-// indexed with 32 bits).
+// Most points one call accepts (a bucket's table has up to three slots a point,
+// counted in 32 bits).
 constexpr int64_t kMaxPoints = (int64_t)1 << 28;
 
-// Bytes of device workspace: the per-point arrays and the cell table, plus
-// `library_bytes` for the sort and the scan (from libraryWorkspaceBytes).
-size_t voxelizeWorkspaceBytes(const VoxelizeShape &s, size_t library_bytes);
+// Bytes of device workspace: the per-point arrays and the cell tables.
+size_t voxelizeWorkspaceBytes(const VoxelizeShape &s);
 
-// Counters the sort and the scan want at this size.
-hipError_t libraryWorkspaceBytes(const VoxelizeShape &s, hipStream_t stream, size_t *bytes);
-
-// Enqueues the whole operator: outputs zero-filled, then written.
+// Enqueues the whole operator: outputs zero-filled, then written.  The number of voxels also goes,
+// below the low half of `stamp`, into `host_voxel_num` (pinned host memory; null: nowhere).
 hipError_t launchVoxelize(const LaunchCtx &lc, const VoxelizeShape &s, const float *points,
                           const float *voxel_size, const float *coors_range, void *workspace,
                           size_t workspace_bytes, float *voxels, int32_t *coors,
-                          int32_t *num_points_per_voxel, int32_t *voxel_num);
+                          int32_t *num_points_per_voxel, int32_t *voxel_num, unsigned long long *host_voxel_num,
+                          unsigned long long stamp);
 
 }  // namespace voxelization
 }  // namespace mluop

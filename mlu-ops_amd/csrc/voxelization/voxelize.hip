@@ -7,24 +7,26 @@
 // cell (kernels/voxelization/voxelization_kernel.mlu, KernelPoint2Voxel), then
 // numbers the voxels with a single core
 // (kernels/voxelization/voxelization.cpp:45-53).  Here the same result comes
-// from grouping instead of searching:
-//   1 voxCellSlots   cell of every point; the 64-bit cell id is entered into an
-//                    open-addressing table, whose slot number names the cell
-//   2 radix sort     (slot, point index) pairs, packed into 64-bit words, by slot, least significant
-//                    digit first and therefore stable: every cell's points end
-//                    up adjacent and in point order
-//   3 voxMarkFirst   the first point of every cell (the point at the head of the cell's
-//                    run) raises its flag in an array over the points
-//   4 prefix sums over the flags: the voxel number of a cell is the number of first
-//                    points in front of its own, which is the sequential numbering of the
-//                    reference
-//   5 voxAssign      in sorted order: position in the cell = sorted position - head of the
-//                    run, voxel number from the bitmap; copies points and coordinates,
-//                    counts points per voxel
-// Integer atomics only (table insertion, per-voxel counts): the outputs are
-// the same bits on every run.
+// from one stable partition of the points and a table in LDS:
+//   1 voxCountBuckets  the cell of every point, hashed to one of up to 2048 buckets; points per
+//                      (tile, bucket).  Workgroups behind the tiles clear the outputs.
+//   2 voxScanColumns   those counters become prefix sums down the tiles
+//   3 voxPartition     the points, packed with their cells, grouped by bucket in point order
+//   4 voxRankInCells   a workgroup takes a bucket in point order: its cells go into a hash table in
+//                      LDS, which gives every point its rank in its cell and its cell's first point
+//   5 voxRankFirsts    bitmap of the cells' first points with prefix sums: the voxel number of a cell
+//                      is the number of first points in front of its own
+//   6 voxAssign        in point order: copies points and coordinates, writes the counts
+// Integer atomics only (LDS counts and table insertion): the outputs are the same bits on
+// every run.
+//
+// What bounds it: random access.  A cell table in device memory costs a 128-byte line each way for
+// every point (58 us for 1.2 M points), a full sort by cell another 70 us in nine launches.  With the
+// buckets only the partition's stores and the ranks' way back to point order are scattered, and
+// every other pass streams.
+// Measured, 1.2 M points in 2048 buckets: 77 us for the six launches (12, 5, 22, 21, 7, 9), 200 us with
+// cell table and sort; 23 k points: 33 us against 68 us, where launches and latency count.
 #include <hip/hip_runtime.h>
-#include <cstring>
 
 #include "core/device_sort.h"
 
@@ -34,7 +36,8 @@ namespace mluop {
 namespace voxelization {
 namespace {
 
-constexpr unsigned long long kEmptyKey = ~0ull;
+typedef unsigned long long u64;
+
 constexpr int kBlock = 256;
 
 inline int gridFor(size_t n, int cap = 1 << 20) {
@@ -45,46 +48,43 @@ inline int gridFor(size_t n, int cap = 1 << 20) {
 
 size_t alignUp(size_t v) { return (v + 255) & ~(size_t)255; }
 
-uint32_t tableSlots(int64_t num_points) {
-  uint32_t cap = 1024;
-  while ((int64_t)cap < 2 * num_points) cap <<= 1;
-  return cap;
-}
+// ---- partition into buckets --------------------------------------------------------------
 
-int bitsFor(uint32_t cap) {  // slot numbers 0..cap (cap itself marks "no cell")
-  int b = 1;
-  while ((1ull << b) <= cap) ++b;
+constexpr int kTileThreads = 512;
+constexpr int kTileWaves = kTileThreads / 64;
+constexpr int kWaveChunks = 4;                               // chunks of 64 points a wave takes in a row
+constexpr int kRound = kTileThreads * kWaveChunks;           // points of a tile's round
+constexpr int kMaxBuckets = 2048;
+constexpr int kMaxTiles = 1024;
+constexpr uint32_t kNoBucket = 0xffffffffu;
+
+// Buckets of about 500 points: a bucket is one workgroup's work and half of its LDS table, while a
+// small cloud still gives many workgroups something to do.
+int bucketsFor(int64_t n) {
+  int b = 64;
+  while (b < kMaxBuckets && (int64_t)b * 600 < n) b <<= 1;
   return b;
 }
 
-// Up to five regions of 32-bit words filled by one launch.
-constexpr int kFillRegions = 5;
-struct FillRegions {
-  uint32_t *base[kFillRegions];
-  size_t words[kFillRegions];
-  uint32_t value[kFillRegions];
-};
+// A tile takes `rounds` rounds of points one after the other, so that there are at most kMaxTiles
+// rows of counters.
+int roundsFor(int64_t n) {
+  const int64_t all = (n + kRound - 1) / kRound;
+  return (int)((all + kMaxTiles - 1) / kMaxTiles);
+}
 
-__global__ __launch_bounds__(kBlock) void voxFillRegions(FillRegions r) {
-#pragma unroll
-  for (int g = 0; g < kFillRegions; ++g) {
-    // words in front of the first 16-byte boundary, 16-byte stores, words behind the last
-    size_t head = ((16 - (reinterpret_cast<uintptr_t>(r.base[g]) & 15)) & 15) / 4;
-    head = head < r.words[g] ? head : r.words[g];
-    uint32_t *body = r.base[g] + head;
-    const size_t body_words = r.words[g] - head;
-    const size_t quads = body_words / 4;
-    const uint32_t value = r.value[g];
-    const uint4 v = make_uint4(value, value, value, value);
-    uint4 *dst = reinterpret_cast<uint4 *>(body);
-    for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < quads;
-         i += (size_t)gridDim.x * kBlock)
-      dst[i] = v;
-    if (blockIdx.x == 0) {
-      if (threadIdx.x < head) r.base[g][threadIdx.x] = value;
-      if (threadIdx.x < (body_words & 3)) body[quads * 4 + threadIdx.x] = value;
-    }
-  }
+int tilesFor(int64_t n) {
+  const int64_t tile = (int64_t)kRound * roundsFor(n);
+  return (int)((n + tile - 1) / tile);
+}
+
+__device__ inline u64 mix64(u64 k) {
+  k ^= k >> 33;
+  k *= 0xff51afd7ed558ccdull;
+  k ^= k >> 33;
+  k *= 0xc4ceb9fe1a85ec53ull;
+  k ^= k >> 33;
+  return k;
 }
 
 // Cells along one axis: the float quotient rounded half away from zero.
@@ -99,15 +99,6 @@ __device__ inline int cellIndex(float p, float lo, float size, int cells) {
   if (!(f >= 0.f && f < 2147483648.f)) return -1;
   const int c = (int)f;
   return c < cells ? c : -1;
-}
-
-__device__ inline uint32_t mix64(unsigned long long k) {
-  k ^= k >> 33;
-  k *= 0xff51afd7ed558ccdull;
-  k ^= k >> 33;
-  k *= 0xc4ceb9fe1a85ec53ull;
-  k ^= k >> 33;
-  return (uint32_t)k;
 }
 
 // The cell (z, y, x) of a point, or cz < 0 outside the grid.
@@ -132,125 +123,453 @@ __device__ inline Cell cellOfPoint(const float *__restrict__ p, const float *__r
   return c;
 }
 
-__global__ __launch_bounds__(kBlock) void voxCellSlots(
-    const float *__restrict__ points, const float *__restrict__ voxel_size,
-    const float *__restrict__ range, int64_t n, int num_features, unsigned long long *keys,
-    uint32_t cap, unsigned long long *slot_and_point) {
-  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const Cell c = cellOfPoint(points + i * num_features, voxel_size, range);
-  const int cz = c.cz, cy = c.cy, cx = c.cx, gy = c.gy, gx = c.gx;
-  // (table slot in the low half, point index in the high half: sorted as one 64-bit key by
-  // the slot's bits, the point travels with it)
-  const unsigned long long point_half = (unsigned long long)i << 32;
-  if (cz < 0) {
-    slot_and_point[i] = point_half | cap;
+__device__ inline u64 cellKey(const Cell &c) {
+  return ((u64)c.cz * (u64)c.gy + c.cy) * (u64)c.gx + c.cx;
+}
+
+// A grid of fewer than 2^32 - 1 cells (the same for every thread) has 32-bit keys; in a larger
+// one the cell of a partitioned point is worked out again from the point.
+__device__ inline bool smallGrid(u64 cells) { return cells < 0xffffffffull; }
+
+// Up to four regions of 32-bit words cleared by one launch.
+constexpr int kClearRegions = 4;
+struct ClearRegions {
+  uint32_t *base[kClearRegions];
+  size_t words[kClearRegions];
+};
+
+__device__ void clearRegions(const ClearRegions &r, int block, int blocks) {
+#pragma unroll
+  for (int g = 0; g < kClearRegions; ++g) {
+    // words in front of the first 16-byte boundary, 16-byte stores, words behind the last
+    size_t head = ((16 - (reinterpret_cast<uintptr_t>(r.base[g]) & 15)) & 15) / 4;
+    head = head < r.words[g] ? head : r.words[g];
+    uint32_t *body = r.base[g] + head;
+    const size_t body_words = r.words[g] - head;
+    const size_t quads = body_words / 4;
+    uint4 *dst = reinterpret_cast<uint4 *>(body);
+    for (size_t i = (size_t)block * blockDim.x + threadIdx.x; i < quads; i += (size_t)blocks * blockDim.x)
+      dst[i] = make_uint4(0, 0, 0, 0);
+    if (block == 0) {
+      if (threadIdx.x < head) r.base[g][threadIdx.x] = 0;
+      if (threadIdx.x < (body_words & 3)) body[quads * 4 + threadIdx.x] = 0;
+    }
+  }
+}
+
+// tagged[i] = bucket of point i (kNoBucket outside the grid) above the low half of its cell key;
+// hist[tile][bucket] = points of the tile in the bucket.
+__global__ __launch_bounds__(kTileThreads) void voxCountBuckets(
+    const float *__restrict__ points, const float *__restrict__ voxel_size, const float *__restrict__ range,
+    int64_t n, int num_features, int buckets, int rounds, int tiles, u64 *__restrict__ tagged,
+    uint32_t *__restrict__ hist, ClearRegions clear) {
+  __shared__ uint32_t s_count[kMaxBuckets];
+  if ((int)blockIdx.x >= tiles) {
+    clearRegions(clear, blockIdx.x - tiles, gridDim.x - tiles);
     return;
   }
-  const unsigned long long key =
-      ((unsigned long long)cz * (unsigned long long)gy + cy) * (unsigned long long)gx + cx;
-  uint32_t slot = mix64(key) & (cap - 1);
-  // At most half of the slots are ever taken, so an empty one is always reached.
-  // A grid of fewer than 2^32 - 1 cells (the same for every thread) keeps 32-bit
-  // keys in the first half of the table: 32-bit compare-and-swap is several times
-  // faster than the 64-bit one.
-  if (c.cells < 0xffffffffull) {
-    uint32_t *keys32 = reinterpret_cast<uint32_t *>(keys);
-    const uint32_t key32 = (uint32_t)key;
-    while (true) {
-      const uint32_t seen = atomicCAS(&keys32[slot], 0xffffffffu, key32);
-      if (seen == 0xffffffffu || seen == key32) break;
-      slot = (slot + 1) & (cap - 1);
+  for (int b = threadIdx.x; b < buckets; b += kTileThreads) s_count[b] = 0;
+  __syncthreads();
+  const int64_t begin = (int64_t)blockIdx.x * rounds * kRound;
+  for (int j = 0; j < rounds * kWaveChunks; ++j) {
+    const int64_t i = begin + (int64_t)j * kTileThreads + threadIdx.x;
+    if (i >= n) break;
+    const Cell c = cellOfPoint(points + i * num_features, voxel_size, range);
+    u64 tag = (u64)kNoBucket << 32;
+    if (c.cz >= 0) {
+      const u64 key = cellKey(c);
+      const uint32_t bucket = (uint32_t)mix64(key) & (uint32_t)(buckets - 1);
+      tag = (u64)bucket << 32 | (uint32_t)key;
+      atomicAdd(&s_count[bucket], 1u);
     }
-  } else {
-    while (true) {
-      const unsigned long long seen = atomicCAS(&keys[slot], kEmptyKey, key);
-      if (seen == kEmptyKey || seen == key) break;
-      slot = (slot + 1) & (cap - 1);
-    }
+    tagged[i] = tag;
   }
-  slot_and_point[i] = point_half | slot;
+  __syncthreads();
+  for (int b = threadIdx.x; b < buckets; b += kTileThreads) hist[(size_t)blockIdx.x * buckets + b] = s_count[b];
 }
 
-// is_first[f] = 1 <=> point f is the first of its cell (the array was cleared by the fill; a
-// plain store per cell: a bitmap would take an atomic per cell, four times as long).
-__global__ __launch_bounds__(kBlock) void voxMarkFirst(const unsigned long long *__restrict__ sorted,
-                                                       int64_t n, uint32_t cap, uint32_t *is_first) {
-  const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (p >= n) return;
-  const unsigned long long mine = sorted[p];
-  const uint32_t s = (uint32_t)mine;
-  if (s == cap) return;
-  if (p == 0 || (uint32_t)sorted[p - 1] != s) is_first[(uint32_t)(mine >> 32)] = 1u;
-}
-
-// First sorted position whose slot is `s`, which lies in front of position `from` (whose slot
-// is `s` as well): doubling steps backwards, then a binary search.
-__device__ inline int64_t headBefore(const unsigned long long *__restrict__ sorted, int64_t from, uint32_t s) {
-  int64_t hi = from;  // sorted[hi] holds slot s
-  int64_t step = 1;
-  int64_t lo = hi - step;
-  while (lo >= 0 && (uint32_t)sorted[lo] == s) {
-    hi = lo;
-    step *= 2;
-    lo = hi - step;
-  }
-  if (lo < 0) {
-    if ((uint32_t)sorted[0] == s) return 0;
-    lo = 0;
-  }
-  // sorted[lo] is another slot's, sorted[hi] this one's, the run starts in (lo, hi]
-  while (hi - lo > 1) {
-    const int64_t mid = lo + (hi - lo) / 2;
-    if ((uint32_t)sorted[mid] == s)
-      hi = mid;
-    else
-      lo = mid;
-  }
-  return hi;
-}
-
-// Thread p takes the point at sorted position p.  The head of its cell's run is the nearest
-// position at or in front of p where the slot changes: found among the lanes of the wave by a
-// running maximum, and looked up behind the wave only by the lanes of a run that began earlier.
-__global__ __launch_bounds__(kBlock) void voxAssign(
-    const float *__restrict__ points, const float *__restrict__ voxel_size,
-    const float *__restrict__ range, const unsigned long long *__restrict__ sorted,
-    const uint32_t *__restrict__ is_first,
-    const uint32_t *__restrict__ voxel_of_first, int64_t n, uint32_t cap, int num_features, int max_points,
-    int max_voxels, float *voxels, int32_t *coors, int32_t *num_points_per_voxel, int32_t *voxel_num) {
-  const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  const int lane = threadIdx.x & 63;
-  if (p == 0) {
-    uint32_t cells = 0;
-    if (n > 0) cells = voxel_of_first[n - 1] + is_first[n - 1];
-    *voxel_num = cells < (uint32_t)max_voxels ? (int32_t)cells : max_voxels;
-  }
-  const bool live = p < n;
-  const unsigned long long mine = live ? sorted[p] : (unsigned long long)cap;
-  const uint32_t s = (uint32_t)mine;
-  const uint32_t before = (live && p > 0) ? (uint32_t)sorted[p - 1] : cap;
-  const bool starts = live && s != cap && (p == 0 || before != s);
-  // nearest run start at or below this lane, inside the wave (-1: none)
-  long long head = starts ? (long long)p : -1;
+// hist[0..tiles)[bucket] -> exclusive prefix sums down the column, its sum to totals[bucket].  A
+// workgroup takes 32 columns (128-byte rows), 32 groups of threads share the tiles.
+constexpr int kColumns = 32;
+constexpr int kColumnGroups = 32;
+__global__ __launch_bounds__(kColumns *kColumnGroups) void voxScanColumns(uint32_t *__restrict__ hist, int tiles,
+                                                                          int buckets,
+                                                                          uint32_t *__restrict__ totals) {
+  __shared__ uint32_t s_sum[kColumnGroups][kColumns];
+  const int c = threadIdx.x % kColumns, g = threadIdx.x / kColumns;
+  const int per = (tiles + kColumnGroups - 1) / kColumnGroups;  // at most 32 (kMaxTiles)
+  const int t0 = g * per, t1 = t0 + per < tiles ? t0 + per : tiles;
+  uint32_t *column = hist + blockIdx.x * kColumns + c;
+  uint32_t v[kMaxTiles / kColumnGroups];
+  uint32_t sum = 0;
 #pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const long long up = __shfl_up(head, d, 64);
-    if (lane >= d && up > head) head = up;
+  for (int u = 0; u < kMaxTiles / kColumnGroups; ++u) {
+    v[u] = t0 + u < t1 ? column[(size_t)(t0 + u) * buckets] : 0u;
   }
-  if (!live || s == cap) return;
-  if (head < 0) head = headBefore(sorted, p - lane, s);  // (position p - lane holds slot s too)
-  const int64_t r = p - head;
-  if (r >= max_points) return;
-  const uint32_t f = (uint32_t)(sorted[head] >> 32);
-  const uint32_t v = voxel_of_first[f];  // first points in front of f
+#pragma unroll
+  for (int u = 0; u < kMaxTiles / kColumnGroups; ++u) sum += v[u];
+  s_sum[g][c] = sum;
+  __syncthreads();
+  uint32_t run = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < kColumnGroups; ++w) {
+    const uint32_t s = s_sum[w][c];
+    run += w < g ? s : 0u;
+    total += s;
+  }
+#pragma unroll
+  for (int u = 0; u < kMaxTiles / kColumnGroups; ++u) {
+    if (t0 + u < t1) column[(size_t)(t0 + u) * buckets] = run;
+    run += v[u];
+  }
+  if (g == 0) totals[blockIdx.x * kColumns + c] = total;
+}
+
+// Exclusive prefix sums of totals[0..buckets) into s_first, by the whole workgroup.
+template <int THREADS>
+__device__ inline void bucketStarts(const uint32_t *__restrict__ totals, int buckets, uint32_t *s_first,
+                                    uint32_t *s_wave) {
+  constexpr int kPer = kMaxBuckets / THREADS;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  uint32_t v[kPer], sum = 0;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    v[u] = tid * kPer + u < buckets ? totals[tid * kPer + u] : 0u;
+    sum += v[u];
+  }
+  const uint32_t incl = device_sort::waveInclusiveSum(sum);
+  if (lane == 63) s_wave[wave] = incl;
+  __syncthreads();
+  uint32_t run = incl - sum;
+  for (int w = 0; w < wave; ++w) run += s_wave[w];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    if (tid * kPer + u < buckets) s_first[tid * kPer + u] = run;
+    run += v[u];
+  }
+}
+
+// grouped[] = (point index above the low half of the cell key), by bucket, points of a bucket in
+// their order.  A wave owns 256 consecutive points and takes them 64 at a time; lanes of one
+// bucket find each other with a ballot per bucket bit.
+__global__ __launch_bounds__(kTileThreads) void voxPartition(const u64 *__restrict__ tagged, int64_t n, int buckets,
+                                                             int bucket_bits, int rounds,
+                                                             const uint32_t *__restrict__ hist,
+                                                             const uint32_t *__restrict__ totals,
+                                                             u64 *__restrict__ grouped,
+                                                             uint32_t *__restrict__ bucket_start) {
+  __shared__ uint16_t s_count[kTileWaves][kMaxBuckets];  // points of a bucket per wave, then in the waves before
+  __shared__ uint32_t s_first[kMaxBuckets];              // where the next point of a bucket goes
+  __shared__ uint32_t s_wave[kTileWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  bucketStarts<kTileThreads>(totals, buckets, s_first, s_wave);
+  __syncthreads();
+  if (blockIdx.x == 0)
+    for (int b = tid; b < buckets; b += kTileThreads) bucket_start[b] = s_first[b];
+  for (int b = tid; b < buckets; b += kTileThreads) s_first[b] += hist[(size_t)blockIdx.x * buckets + b];
+  volatile uint16_t *mine = s_count[wave];
+  const u64 below = (1ull << lane) - 1ull;
+  for (int round = 0; round < rounds; ++round) {
+    for (int b = tid; b < buckets; b += kTileThreads)
+#pragma unroll
+      for (int w = 0; w < kTileWaves; ++w) s_count[w][b] = 0;
+    __syncthreads();
+    const int64_t base = ((int64_t)blockIdx.x * rounds + round) * kRound + (int64_t)wave * (64 * kWaveChunks);
+    u64 tag[kWaveChunks];
+    uint32_t place[kWaveChunks];
+#pragma unroll
+    for (int j = 0; j < kWaveChunks; ++j) {
+      const int64_t i = base + j * 64 + lane;
+      tag[j] = i < n ? tagged[i] : (u64)kNoBucket << 32;
+    }
+#pragma unroll
+    for (int j = 0; j < kWaveChunks; ++j) {
+      const uint32_t bucket = (uint32_t)(tag[j] >> 32);
+      const bool valid = bucket != kNoBucket;
+      u64 peers = __ballot(valid);
+      for (int b = 0; b < bucket_bits; ++b) {
+        const bool bit = (bucket >> b) & 1u;
+        const u64 with = __ballot(bit);
+        peers &= bit ? with : ~with;
+      }
+      const int leader = valid ? __ffsll((long long)peers) - 1 : lane;
+      uint32_t before = 0;  // points of the bucket in the wave's earlier chunks
+      if (valid && lane == leader) {
+        before = mine[bucket];
+        mine[bucket] = (uint16_t)(before + (uint32_t)__popcll(peers));
+      }
+      before = __shfl(before, leader, 64);
+      place[j] = before + (uint32_t)__popcll(peers & below);
+    }
+    __syncthreads();
+    // the waves' counts of a bucket become the counts of the waves before
+    uint32_t round_total[kMaxBuckets / kTileThreads];
+#pragma unroll
+    for (int u = 0; u < kMaxBuckets / kTileThreads; ++u) {
+      const int b = tid + u * kTileThreads;
+      uint32_t run = 0;
+      if (b < buckets) {
+#pragma unroll
+        for (int w = 0; w < kTileWaves; ++w) {
+          const uint32_t c = s_count[w][b];
+          s_count[w][b] = (uint16_t)run;
+          run += c;
+        }
+      }
+      round_total[u] = run;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kWaveChunks; ++j) {
+      const uint32_t bucket = (uint32_t)(tag[j] >> 32);
+      if (bucket != kNoBucket) {
+        const uint32_t i = (uint32_t)(base + j * 64 + lane);
+        grouped[(size_t)s_first[bucket] + s_count[wave][bucket] + place[j]] = (u64)i << 32 | (uint32_t)tag[j];
+      }
+    }
+    if (round + 1 == rounds) break;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kMaxBuckets / kTileThreads; ++u) {
+      const int b = tid + u * kTileThreads;
+      if (b < buckets) s_first[b] += round_total[u];
+    }
+  }
+}
+
+// ---- ranks inside the cells of a bucket --------------------------------------------------
+
+constexpr int kRankThreads = 512;
+constexpr int kRankWaves = kRankThreads / 64;
+constexpr int kLdsSlots = 2048;  // an LDS table serves a bucket of up to half as many points
+constexpr uint32_t kIsFirst = 0x80000000u;
+
+// Cells of a bucket in LDS (32-bit keys).
+struct LdsTable {
+  uint32_t *keys, *counts, *firsts;
+  uint32_t slots;  // a power of two
+  typedef uint32_t Key;
+  static constexpr Key kEmpty = 0xffffffffu;
+  __device__ static void cleared() {}
+};
+// The same in device memory, for buckets of more points than the LDS table serves and for grids
+// whose keys need 64 bits.
+struct WideTable {
+  u64 *keys;
+  uint32_t *counts, *firsts;
+  uint32_t slots;
+  typedef u64 Key;
+  static constexpr Key kEmpty = ~0ull;
+  // (plain stores of empty keys, then compare-and-swap by the other waves of the workgroup)
+  __device__ static void cleared() { __threadfence(); }
+};
+
+// Takes the bucket's points in order, kRankThreads at a time.  A wave's points of one cell are put
+// in order by ballots; the waves add theirs to the cell's count one after the other.  Points of a
+// cell that is full already are dropped in front of all that, so that a cell with very many points
+// (padding at one coordinate) costs a table lookup a point.
+template <typename TABLE>
+__device__ void rankBucket(const TABLE &t, const u64 *__restrict__ entries, uint32_t count,
+                           const float *__restrict__ points, const float *__restrict__ voxel_size,
+                           const float *__restrict__ range, int num_features, bool small_grid, uint32_t max_points,
+                           volatile uint16_t *s_owner, uint32_t *__restrict__ state, uint32_t *__restrict__ first_of) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (uint32_t s = tid; s < t.slots; s += kRankThreads) {
+    t.keys[s] = TABLE::kEmpty;
+    t.counts[s] = 0;
+  }
+  TABLE::cleared();
+  __syncthreads();
+  u64 next = (uint32_t)tid < count ? entries[tid] : 0;
+  for (uint32_t base = 0; base < count; base += kRankThreads) {
+    const u64 entry = next;
+    const uint32_t i = base + tid;
+    if (i + kRankThreads < count) next = entries[i + kRankThreads];
+    bool live = i < count;
+    const uint32_t idx = (uint32_t)(entry >> 32);
+    uint32_t slot = 0;
+    if (live) {
+      u64 key = (uint32_t)entry;
+      if (!small_grid) key = cellKey(cellOfPoint(points + (size_t)idx * num_features, voxel_size, range));
+      slot = (uint32_t)(mix64(key) >> 32) & (t.slots - 1);
+      // (there are more slots than points, so an empty one is always reached)
+      while (true) {
+        const typename TABLE::Key seen = atomicCAS(&t.keys[slot], TABLE::kEmpty, (typename TABLE::Key)key);
+        if (seen == TABLE::kEmpty || seen == (typename TABLE::Key)key) break;
+        slot = (slot + 1) & (t.slots - 1);
+      }
+      live = t.counts[slot] < max_points;
+    }
+    if (!__syncthreads_or(live)) continue;
+    // A lane that reads its own number back is alone in its wave with the slot, or the last of its
+    // group to write; the groups of all other lanes are gone through one by one.
+    if (live) s_owner[slot & (kLdsSlots - 1)] = (uint16_t)tid;
+    const bool shares = live && s_owner[slot & (kLdsSlots - 1)] != (uint16_t)tid;
+    uint32_t rank = 0, group = 1;
+    int leader = lane;
+    u64 open = __ballot(shares);
+    while (open != 0) {
+      const uint32_t s = __shfl(slot, __ffsll((long long)open) - 1, 64);
+      const bool in = live && slot == s;
+      const u64 same = __ballot(in);
+      if (in) {
+        rank = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+        group = (uint32_t)__popcll(same);
+        leader = __ffsll((long long)same) - 1;
+      }
+      open &= ~same;
+    }
+    uint32_t before = 0;
+    for (int w = 0; w < kRankWaves; ++w) {
+      if (wave == w && live && rank == 0) {
+        before = t.counts[slot];
+        t.counts[slot] = before + group;
+        if (before == 0) t.firsts[slot] = idx;
+      }
+      __syncthreads();
+    }
+    rank += __shfl(before, leader, 64);
+    if (live && rank > 0 && rank < max_points) {
+      state[idx] = rank;
+      first_of[idx] = t.firsts[slot];
+    }
+  }
+  __syncthreads();
+  for (uint32_t s = tid; s < t.slots; s += kRankThreads) {
+    const uint32_t c = t.counts[s];
+    if (c != 0) state[t.firsts[s]] = kIsFirst | (c < max_points ? c : max_points);
+  }
+}
+
+// state[i] (cleared before): kIsFirst | points the cell keeps, for the first point of a cell; the
+// rank in the cell for another point it keeps, whose first_of[i] is the first one; 0 otherwise.
+__global__ __launch_bounds__(kRankThreads) void voxRankInCells(
+    const float *__restrict__ points, const float *__restrict__ voxel_size, const float *__restrict__ range,
+    int num_features, uint32_t max_points, const u64 *__restrict__ grouped, const uint32_t *__restrict__ bucket_start,
+    const uint32_t *__restrict__ totals, u64 *wide_keys, uint32_t *wide_counts, uint32_t *wide_firsts,
+    uint32_t *__restrict__ state, uint32_t *__restrict__ first_of) {
+  __shared__ uint32_t s_keys[kLdsSlots], s_counts[kLdsSlots], s_firsts[kLdsSlots];
+  __shared__ uint16_t s_owner[kLdsSlots];
+  const uint32_t count = totals[blockIdx.x];
+  if (count == 0) return;
+  const uint32_t start = bucket_start[blockIdx.x];
+  const bool small_grid =
+      smallGrid((u64)axisCells(range[2], range[5], voxel_size[2]) * (u64)axisCells(range[1], range[4], voxel_size[1]) *
+                (u64)axisCells(range[0], range[3], voxel_size[0]));
+  if (small_grid && count <= kLdsSlots / 2) {
+    LdsTable t = {s_keys, s_counts, s_firsts, 64};
+    while (t.slots < 2 * count) t.slots <<= 1;
+    rankBucket(t, grouped + start, count, points, voxel_size, range, num_features, true, max_points, s_owner, state,
+               first_of);
+  } else {
+    // the bucket's share of the region: the largest power of two within three slots a point
+    const size_t at = 3 * (size_t)start;
+    WideTable t = {wide_keys + at, wide_counts + at, wide_firsts + at, 1u << (31 - __clz(3 * count))};
+    rankBucket(t, grouped + start, count, points, voxel_size, range, num_features, small_grid, max_points, s_owner,
+               state, first_of);
+  }
+}
+
+// ---- voxel numbers -----------------------------------------------------------------------
+
+// A tile of 4096 points: 64 words of its bitmap of first points, the number of first points of the
+// tile in front of each word, and their number in the tile.
+constexpr int kFirstsTile = 4096;
+__global__ __launch_bounds__(kBlock) void voxRankFirsts(const uint32_t *__restrict__ state, int64_t n,
+                                                        u64 *__restrict__ first_bits,
+                                                        uint32_t *__restrict__ word_firsts,
+                                                        uint32_t *__restrict__ tile_firsts) {
+  __shared__ u64 s_bits[kFirstsTile / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t base = (int64_t)blockIdx.x * kFirstsTile + (int64_t)wave * 1024;
+  uint32_t v[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int64_t i = base + j * 64 + lane;
+    v[j] = i < n ? state[i] : 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const u64 bits = __ballot((v[j] & kIsFirst) != 0);
+    if (lane == 0) s_bits[wave * 16 + j] = bits;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const u64 bits = s_bits[lane];
+    const uint32_t c = (uint32_t)__popcll(bits);
+    const uint32_t incl = device_sort::waveInclusiveSum(c);
+    first_bits[(size_t)blockIdx.x * 64 + lane] = bits;
+    word_firsts[(size_t)blockIdx.x * 64 + lane] = incl - c;
+    if (lane == 63) tile_firsts[blockIdx.x] = incl;
+    if (lane == 0 && blockIdx.x + 1 == gridDim.x) tile_firsts[gridDim.x] = 0;  // becomes the sum of all in a scan
+  }
+}
+
+// Point i of the cloud.  Up to kSumTiles tiles every workgroup sums up the tiles' counts itself, which
+// takes less than a launch of its own does; more are scanned before (`scanned`: tile_firsts holds
+// prefix sums, and one word behind them the sum of all).
+constexpr int kSumTiles = 1024;
+__global__ __launch_bounds__(kBlock) void voxAssign(
+    const float *__restrict__ points, const float *__restrict__ voxel_size, const float *__restrict__ range, int64_t n,
+    int num_features, const uint32_t *__restrict__ state, const uint32_t *__restrict__ first_of,
+    const u64 *__restrict__ first_bits, const uint32_t *__restrict__ word_firsts,
+    const uint32_t *__restrict__ tile_firsts, int tiles, bool scanned, bool quads, int max_points, int max_voxels,
+    float *__restrict__ voxels, int32_t *__restrict__ coors, int32_t *__restrict__ num_points_per_voxel,
+    int32_t *__restrict__ voxel_num, u64 *host_voxel_num, u64 stamp) {
+  __shared__ uint32_t s_tile[kSumTiles];
+  __shared__ uint32_t s_wave[kBlock / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t i = (int64_t)blockIdx.x * kBlock + tid;
+  const uint32_t st = i < n ? state[i] : 0u;
+  uint32_t all = 0;
+  if (scanned) {
+    if (blockIdx.x == 0 && tid == 0) all = tile_firsts[tiles];
+  } else {
+    constexpr int kPer = kSumTiles / kBlock;
+    uint32_t v[kPer], sum = 0;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      v[u] = tid * kPer + u < tiles ? tile_firsts[tid * kPer + u] : 0u;
+      sum += v[u];
+    }
+    const uint32_t incl = device_sort::waveInclusiveSum(sum);
+    if (lane == 63) s_wave[wave] = incl;
+    __syncthreads();
+    uint32_t run = incl - sum;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; ++w) {
+      run += w < wave ? s_wave[w] : 0u;
+      all += s_wave[w];
+    }
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      s_tile[tid * kPer + u] = run;
+      run += v[u];
+    }
+    __syncthreads();
+  }
+  if (blockIdx.x == 0 && tid == 0) {
+    const int32_t kept = all < (uint32_t)max_voxels ? (int32_t)all : max_voxels;
+    *voxel_num = kept;
+    if (host_voxel_num != nullptr)
+      __hip_atomic_store(host_voxel_num, stamp << 32 | (uint32_t)kept, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  if (st == 0) return;
+  const bool is_first = (st & kIsFirst) != 0;
+  const uint32_t f = is_first ? (uint32_t)i : first_of[i];
+  const uint32_t r = is_first ? 0u : st;
+  const uint32_t tile = f / kFirstsTile, word = f >> 6;
+  const uint32_t v = (scanned ? tile_firsts[tile] : s_tile[tile]) + word_firsts[word] +
+                     (uint32_t)__popcll(first_bits[word] & ((1ull << (f & 63)) - 1ull));
   if (v >= (uint32_t)max_voxels) return;
-  const uint32_t i = (uint32_t)(mine >> 32);
   const float *src = points + (size_t)i * num_features;
   float *dst = voxels + ((size_t)v * max_points + r) * num_features;
-  for (int k = 0; k < num_features; ++k) dst[k] = src[k];
-  atomicAdd(&num_points_per_voxel[v], 1);
-  if (r == 0) {
+  if (quads)
+    *reinterpret_cast<float4 *>(dst) = *reinterpret_cast<const float4 *>(src);
+  else
+    for (int k = 0; k < num_features; ++k) dst[k] = src[k];
+  if (is_first) {
+    num_points_per_voxel[v] = (int32_t)(st & ~kIsFirst);
     const Cell c = cellOfPoint(src, voxel_size, range);
     coors[3 * (size_t)v] = c.cz;
     coors[3 * (size_t)v + 1] = c.cy;
@@ -259,19 +578,17 @@ __global__ __launch_bounds__(kBlock) void voxAssign(
 }
 
 struct Workspace {
-  unsigned long long *pairs_a, *pairs_b;  // table slot | point index << 32
-  uint32_t *is_first, *voxel_of_first;
-  unsigned long long *keys;
-  void *library;
+  u64 *tagged, *grouped, *first_bits, *wide_keys;
+  uint32_t *state, *first_of, *hist, *totals, *bucket_start, *word_firsts, *tile_firsts, *wide_counts, *wide_firsts;
   size_t total;
 };
 
-Workspace carve(void *base, const VoxelizeShape &s, size_t library_bytes) {
+Workspace carve(void *base, const VoxelizeShape &s) {
   const size_t n = (size_t)s.num_points;
-  const uint32_t cap = tableSlots(s.num_points);
-  // Blocks start at the caller's pointer rounded up to 256 bytes (64-bit keys, packed sort
-  // keys and the sort's counters need their alignment whatever the caller
-  // passes); the reported size includes that slack.  A null base only measures.
+  const size_t firsts_tiles = (n + kFirstsTile - 1) / kFirstsTile;
+  // Blocks start at the caller's pointer rounded up to 256 bytes (64-bit words need their
+  // alignment whatever the caller passes); the reported size includes that slack.  A null base
+  // only measures.
   char *p = base ? reinterpret_cast<char *>(alignUp(reinterpret_cast<uintptr_t>(base))) : nullptr;
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -279,96 +596,103 @@ Workspace carve(void *base, const VoxelizeShape &s, size_t library_bytes) {
     off += alignUp(bytes);
     return q;
   };
+  auto words = [&](size_t count) { return reinterpret_cast<uint32_t *>(take(4 * count)); };
+  auto longs = [&](size_t count) { return reinterpret_cast<u64 *>(take(8 * count)); };
   Workspace w;
-  w.pairs_a = reinterpret_cast<unsigned long long *>(take(8 * n));
-  w.pairs_b = reinterpret_cast<unsigned long long *>(take(8 * n));
-  w.is_first = reinterpret_cast<uint32_t *>(take(4 * n));
-  w.voxel_of_first = reinterpret_cast<uint32_t *>(take(4 * n));
-  w.keys = reinterpret_cast<unsigned long long *>(take(8 * (size_t)cap));
-  w.library = take(library_bytes);
+  w.tagged = longs(n);
+  w.grouped = longs(n);
+  w.state = words(n);
+  w.first_of = words(n);
+  w.hist = words((size_t)tilesFor(s.num_points) * bucketsFor(s.num_points));
+  w.totals = words(kMaxBuckets);
+  w.bucket_start = words(kMaxBuckets);
+  w.first_bits = longs(firsts_tiles * 64);
+  w.word_firsts = words(firsts_tiles * 64);
+  w.tile_firsts = words(firsts_tiles + 8);
+  w.wide_keys = longs(3 * n);
+  w.wide_counts = words(3 * n);
+  w.wide_firsts = words(3 * n);
   w.total = off + 256;
   return w;
 }
 
-
 }  // namespace
 
-size_t voxelizeWorkspaceBytes(const VoxelizeShape &s, size_t library_bytes) {
-  return carve(nullptr, s, library_bytes).total;
-}
-
-hipError_t libraryWorkspaceBytes(const VoxelizeShape &s, hipStream_t stream, size_t *bytes) {
-  (void)stream;
-  *bytes = device_sort::workspaceBytes((size_t)s.num_points);
-  return hipSuccess;
-}
+size_t voxelizeWorkspaceBytes(const VoxelizeShape &s) { return carve(nullptr, s).total; }
 
 hipError_t launchVoxelize(const LaunchCtx &lc, const VoxelizeShape &s, const float *points,
                           const float *voxel_size, const float *coors_range, void *workspace,
                           size_t workspace_bytes, float *voxels, int32_t *coors,
-                          int32_t *num_points_per_voxel, int32_t *voxel_num) {
+                          int32_t *num_points_per_voxel, int32_t *voxel_num, unsigned long long *host_voxel_num,
+                          unsigned long long stamp) {
   const int64_t n = s.num_points;
-  const uint32_t cap = tableSlots(n);
-  size_t library_bytes = 0;
-  hipError_t e = libraryWorkspaceBytes(s, lc.stream, &library_bytes);
-  if (e != hipSuccess) return e;
-  const Workspace w = carve(workspace, s, library_bytes);
+  const Workspace w = carve(workspace, s);
   if (w.total > workspace_bytes) return hipErrorInvalidValue;
+  const int buckets = bucketsFor(n), rounds = roundsFor(n), tiles = tilesFor(n);
+  int bucket_bits = 0;
+  while ((1 << bucket_bits) < buckets) ++bucket_bits;
 
-  // outputs start from zero (reference kernels/voxelization/voxelization.cpp:283-309),
-  // the cell table from "empty" and the flags of first points from none raised
-  FillRegions fr;
-  fr.base[0] = reinterpret_cast<uint32_t *>(voxels);
-  fr.words[0] = (size_t)s.max_voxels * s.max_points * s.num_features;
-  fr.base[1] = reinterpret_cast<uint32_t *>(coors);
-  fr.words[1] = (size_t)s.max_voxels * 3;
-  fr.base[2] = reinterpret_cast<uint32_t *>(num_points_per_voxel);
-  fr.words[2] = (size_t)s.max_voxels;
-  fr.base[3] = reinterpret_cast<uint32_t *>(w.keys);
-  fr.words[3] = (size_t)cap * 2;
-  fr.base[4] = w.is_first;
-  fr.words[4] = (size_t)n;
+  // outputs start from zero (reference kernels/voxelization/voxelization.cpp:283-309), and no
+  // point has a place yet
+  ClearRegions clear;
+  clear.base[0] = reinterpret_cast<uint32_t *>(voxels);
+  clear.words[0] = (size_t)s.max_voxels * s.max_points * s.num_features;
+  clear.base[1] = reinterpret_cast<uint32_t *>(coors);
+  clear.words[1] = (size_t)s.max_voxels * 3;
+  clear.base[2] = reinterpret_cast<uint32_t *>(num_points_per_voxel);
+  clear.words[2] = (size_t)s.max_voxels;
+  clear.base[3] = w.state;
+  clear.words[3] = (size_t)n;
   size_t most = 0;
-  for (int g = 0; g < kFillRegions; ++g) {
-    fr.value[g] = g == 3 ? 0xffffffffu : 0u;
-    most = fr.words[g] > most ? fr.words[g] : most;
+  for (int g = 0; g < kClearRegions; ++g) most = clear.words[g] > most ? clear.words[g] : most;
+  const size_t clear_blocks = most / (4 * kTileThreads) + 1;
+  hipError_t e;
+  lc.begin("voxCountBuckets");
+  voxCountBuckets<<<tiles + (int)(clear_blocks < 1024 ? clear_blocks : 1024), kTileThreads, 0, lc.stream>>>(
+      points, voxel_size, coors_range, n, s.num_features, buckets, rounds, tiles, w.tagged, w.hist, clear);
+  lc.end();
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+
+  lc.begin("voxScanColumns");
+  voxScanColumns<<<buckets / kColumns, kColumns * kColumnGroups, 0, lc.stream>>>(w.hist, tiles, buckets, w.totals);
+  lc.end();
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+
+  lc.begin("voxPartition");
+  voxPartition<<<tiles, kTileThreads, 0, lc.stream>>>(w.tagged, n, buckets, bucket_bits, rounds, w.hist, w.totals,
+                                                      w.grouped, w.bucket_start);
+  lc.end();
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+
+  lc.begin("voxRankInCells");
+  voxRankInCells<<<buckets, kRankThreads, 0, lc.stream>>>(points, voxel_size, coors_range, s.num_features,
+                                                         (uint32_t)s.max_points, w.grouped, w.bucket_start, w.totals,
+                                                         w.wide_keys, w.wide_counts, w.wide_firsts, w.state,
+                                                         w.first_of);
+  lc.end();
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+
+  const int firsts_tiles = (int)((n + kFirstsTile - 1) / kFirstsTile);
+  const bool scanned = firsts_tiles > kSumTiles;
+  lc.begin("voxRankFirsts");
+  voxRankFirsts<<<firsts_tiles, kBlock, 0, lc.stream>>>(w.state, n, w.first_bits, w.word_firsts, w.tile_firsts);
+  lc.end();
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  if (scanned) {
+    lc.begin("scanCounters");
+    device_sort::scanCounters<<<1, device_sort::kScanThreads, 0, lc.stream>>>(w.tile_firsts,
+                                                                             (size_t)firsts_tiles + 1);
+    lc.end();
+    if ((e = hipGetLastError()) != hipSuccess) return e;
   }
-  lc.begin("voxFillRegions");
-  voxFillRegions<<<gridFor(most / 4 + 1, 4096), kBlock, 0, lc.stream>>>(fr);
-  lc.end();
-  if ((e = hipGetLastError()) != hipSuccess) return e;
 
-  const int blocks = gridFor((size_t)n);
-  lc.begin("voxCellSlots");
-  voxCellSlots<<<blocks, kBlock, 0, lc.stream>>>(points, voxel_size, coors_range, n,
-                                                  s.num_features, w.keys, cap, w.pairs_a);
-  lc.end();
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-
-  // points grouped by table slot, the points of a slot in their input order
-  lc.begin("radixSortPairs");
-  bool in_b = false;
-  e = device_sort::sortKeys<unsigned long long>(lc.stream, w.library, w.pairs_a, w.pairs_b, (size_t)n,
-                                                bitsFor(cap), &in_b);
-  lc.end();
-  if (e != hipSuccess) return e;
-  const unsigned long long *sorted = in_b ? w.pairs_b : w.pairs_a;
-
-  lc.begin("voxMarkFirst");
-  voxMarkFirst<<<blocks, kBlock, 0, lc.stream>>>(sorted, n, cap, w.is_first);
-  lc.end();
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-
-  // first points in front of every point
-  lc.begin("exclusiveScan");
-  e = device_sort::prefixSums(lc.stream, w.library, w.is_first, w.voxel_of_first, (size_t)n, false);
-  lc.end();
-  if (e != hipSuccess) return e;
-
+  const bool quads = s.num_features == 4 &&
+                     ((reinterpret_cast<uintptr_t>(points) | reinterpret_cast<uintptr_t>(voxels)) & 15) == 0;
   lc.begin("voxAssign");
-  voxAssign<<<blocks, kBlock, 0, lc.stream>>>(points, voxel_size, coors_range, sorted, w.is_first, w.voxel_of_first, n, cap, s.num_features,
-                                               s.max_points, s.max_voxels, voxels, coors,
-                                               num_points_per_voxel, voxel_num);
+  voxAssign<<<gridFor((size_t)n), kBlock, 0, lc.stream>>>(
+      points, voxel_size, coors_range, n, s.num_features, w.state, w.first_of, w.first_bits, w.word_firsts,
+      w.tile_firsts, firsts_tiles, scanned, quads, s.max_points, s.max_voxels, voxels, coors, num_points_per_voxel,
+      voxel_num, host_voxel_num, stamp);
   lc.end();
   return hipGetLastError();
 }

@@ -126,6 +126,7 @@ SIGNATURES = {
     "mluOpExtSetKernelChoice": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int]),
     "mluOpExtSetSparseConvExtendedModes": (ctypes.c_int, [_vp, ctypes.c_int]),
     "mluOpExtSetDistinctPairsPromise": (ctypes.c_int, [_vp, ctypes.c_int]),
+    "mluOpExtGetVoxelizationHostCount": (ctypes.c_int, [_vp, _vp, ctypes.POINTER(ctypes.c_int32)]),
     "mluOpExtGetIndicePairsHostCounts": (ctypes.c_int, [_vp, _vp, ctypes.c_int, _i64p]),
     "mluOpExtGetRowMapSize": (ctypes.c_int, [_vp, ctypes.c_int64, ctypes.POINTER(ctypes.c_size_t)]),
     "mluOpExtBuildRowMap": (ctypes.c_int, [_vp, _vp, _vp, ctypes.POINTER(ctypes.c_int64), ctypes.c_int64,

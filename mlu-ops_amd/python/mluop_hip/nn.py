@@ -16,7 +16,7 @@ import math
 
 import torch
 
-from . import Handle, RowMap, _guarded, get_indice_pairs, native, regular_output_space, voxelization
+from . import Handle, RowMap, _guarded, get_indice_pairs, native, regular_output_space
 
 _handles = {}
 
@@ -283,7 +283,7 @@ class SparseSequential(torch.nn.Sequential):
 class Voxelization(torch.nn.Module):
     """Hard voxelization of one point cloud [N, F] (x, y, z first), the module mmcv puts in front of
     its sparse encoder: returns (voxels [V, max_num_points, F], coors [V, 3] as (z, y, x),
-    num_points_per_voxel [V]) cut to the V voxels found.  Reading V costs one device-to-host copy."""
+    num_points_per_voxel [V]) cut to the V voxels found (the host waits for V, not for the voxels)."""
 
     def __init__(self, voxel_size, point_cloud_range, max_num_points, max_voxels):
         super().__init__()
@@ -299,10 +299,8 @@ class Voxelization(torch.nn.Module):
 
     @torch.no_grad()
     def forward(self, points):
-        voxels, coors, npv, num = voxelization(_handle(), points.contiguous().float(), self.voxel_size,
-                                               self.point_cloud_range, self.max_num_points, self.max_voxels)
-        v = int(num.item())
-        return voxels[:v], coors[:v], npv[:v]
+        return native().voxelization_cut(_guarded(), points.contiguous().float(), self.voxel_size,
+                                         self.point_cloud_range, self.max_num_points, self.max_voxels)
 
 
 def mean_voxel_features(voxels, num_points_per_voxel):
