@@ -68,7 +68,10 @@ struct mluOpContext {
   // Pair counts of a rulebook reach the host through stamped words, kCountWords a note
   // (kernels of up to 7 x 7 x 7; larger ones are copied).
   static constexpr int kCountWords = 343;
-  static constexpr int kReadbackWords = 8;
+  // (word 0: output rows of a rulebook; 1..7: numbers of voxels; from kAxisWords: largest coordinates)
+  static constexpr int kReadbackWords = 16;
+  static constexpr int kVoxelWords = 7;
+  static constexpr int kAxisWords = 8;
   RulebookNote rulebook_notes[kRulebookNotes];
   unsigned long long *rulebook_reports = nullptr;  // kRulebookNotes stamped words behind pinned_scalar
   unsigned long long *count_words = nullptr;   // kRulebookNotes x kCountWords behind those

@@ -152,6 +152,6 @@ mluOpStatus_t MLUOP_WIN_API mluOpDynamicPointToVoxelBackward(
                             static_cast<const float *>(voxel_feats),
                             static_cast<const int32_t *>(point2voxel_map),
                             static_cast<const int32_t *>(voxel_num),
-                            static_cast<int32_t *>(workspace), static_cast<float *>(grad_feats)));
+                            workspace, workspace_size, static_cast<float *>(grad_feats)));
   return MLUOP_STATUS_SUCCESS;
 }

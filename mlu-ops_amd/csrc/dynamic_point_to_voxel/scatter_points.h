@@ -19,25 +19,23 @@ struct ScatterShape {
   bool reduce_max;   // max, else mean
 };
 
-// Per-point arrays only; the sort's counters come on top (libraryWorkspaceBytes).
-size_t scatterWorkspaceBytes(const ScatterShape &s, size_t library_bytes);
-hipError_t libraryWorkspaceBytes(const ScatterShape &s, hipStream_t stream, size_t *bytes);
+size_t scatterWorkspaceBytes(const ScatterShape &s);
 
-// Enqueues the operator.  It synchronises the stream once to read the largest
-// coordinate of every axis back into `pinned_host` (three ints of pinned host
-// memory), which sizes the radix sorts.
+// Enqueues the operator.  It waits once for the largest coordinate of every axis, which the first
+// kernels store below the low half of `stamp` into `host_words` (three words of pinned host
+// memory) and which sizes the radix sorts.
 hipError_t launchScatterPoints(const LaunchCtx &lc, const ScatterShape &s, const float *feats,
                                int32_t *coors, void *workspace, size_t workspace_bytes,
-                               int32_t *pinned_host, float *voxel_feats, int32_t *voxel_coors,
-                               int32_t *point2voxel_map, int32_t *voxel_points_count,
+                               unsigned long long *host_words, unsigned long long stamp, float *voxel_feats,
+                               int32_t *voxel_coors, int32_t *point2voxel_map, int32_t *voxel_points_count,
                                int32_t *voxel_num);
 
-// Backward of the max reduction: `from` is [voxel_rows, num_features] ints of workspace.
+// Backward of the max reduction: `workspace` holds voxel_rows * num_features ints at least.
 hipError_t launchScatterPointsBackward(const LaunchCtx &lc, int num_points, int num_features,
                                        int voxel_rows, const float *grad_voxel_feats,
                                        const float *feats, const float *voxel_feats,
                                        const int32_t *point2voxel_map, const int32_t *voxel_num,
-                                       int32_t *from, float *grad_feats);
+                                       void *workspace, size_t workspace_bytes, float *grad_feats);
 
 }  // namespace dynamic_point_to_voxel
 }  // namespace mluop

@@ -494,7 +494,8 @@ std::vector<at::Tensor> scatterForward(mluOpHandle_t handle, const Buffers &buff
   const at::Tensor voxel_coors = buffers.output({rows, 3}, at::kInt, "voxel_coors");
   const at::Tensor p2v = buffers.output({n}, at::kInt, "point2voxel_map");
   const at::Tensor count = buffers.output({rows}, at::kInt, "voxel_points_count");
-  const at::Tensor num = at::zeros({1}, at::TensorOptions().dtype(at::kInt).device(feats.device()));
+  // (a call on nothing enqueues nothing)
+  const at::Tensor num = n == 0 || c == 0 ? at::zeros({1}, coors.options()) : at::empty({1}, coors.options());
   const mluOpTensorLayout_t array = MLUOP_LAYOUT_ARRAY;
   const TensorDesc d_feats(array, MLUOP_DTYPE_FLOAT, feats.sizes());
   const TensorDesc d_coors(array, MLUOP_DTYPE_INT32, coors.sizes());

@@ -10,11 +10,11 @@
 // from one stable partition of the points and a table in LDS:
 //   1 voxCountBuckets  the cell of every point, hashed to one of up to 2048 buckets; points per
 //                      (tile, bucket).  Workgroups behind the tiles clear the outputs.
-//   2 voxScanColumns   those counters become prefix sums down the tiles
-//   3 voxPartition     the points, packed with their cells, grouped by bucket in point order
+//   2 scanColumns      those counters become prefix sums down the tiles
+//   3 partitionTiles   the points, packed with their cells, grouped by bucket in point order
 //   4 voxRankInCells   a workgroup takes a bucket in point order: its cells go into a hash table in
 //                      LDS, which gives every point its rank in its cell and its cell's first point
-//   5 voxRankFirsts    bitmap of the cells' first points with prefix sums: the voxel number of a cell
+//   5 rankFlags        bitmap of the cells' first points with prefix sums: the voxel number of a cell
 //                      is the number of first points in front of its own
 //   6 voxAssign        in point order: copies points and coordinates, writes the counts
 // Integer atomics only (LDS counts and table insertion): the outputs are the same bits on
@@ -36,9 +36,9 @@ namespace mluop {
 namespace voxelization {
 namespace {
 
-typedef unsigned long long u64;
+using device_sort::u64;
 
-constexpr int kBlock = 256;
+constexpr int kBlock = device_sort::kFlagThreads;
 
 inline int gridFor(size_t n, int cap = 1 << 20) {
   size_t b = (n + kBlock - 1) / kBlock;
@@ -50,32 +50,17 @@ size_t alignUp(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // ---- partition into buckets --------------------------------------------------------------
 
-constexpr int kTileThreads = 512;
-constexpr int kTileWaves = kTileThreads / 64;
-constexpr int kWaveChunks = 4;                               // chunks of 64 points a wave takes in a row
-constexpr int kRound = kTileThreads * kWaveChunks;           // points of a tile's round
-constexpr int kMaxBuckets = 2048;
-constexpr int kMaxTiles = 1024;
-constexpr uint32_t kNoBucket = 0xffffffffu;
+using device_sort::kMaxDigits;
+using device_sort::kNoDigit;
+using device_sort::kRound;
+using device_sort::kTileThreads;
 
 // Buckets of about 500 points: a bucket is one workgroup's work and half of its LDS table, while a
 // small cloud still gives many workgroups something to do.
 int bucketsFor(int64_t n) {
   int b = 64;
-  while (b < kMaxBuckets && (int64_t)b * 600 < n) b <<= 1;
+  while (b < kMaxDigits && (int64_t)b * 600 < n) b <<= 1;
   return b;
-}
-
-// A tile takes `rounds` rounds of points one after the other, so that there are at most kMaxTiles
-// rows of counters.
-int roundsFor(int64_t n) {
-  const int64_t all = (n + kRound - 1) / kRound;
-  return (int)((all + kMaxTiles - 1) / kMaxTiles);
-}
-
-int tilesFor(int64_t n) {
-  const int64_t tile = (int64_t)kRound * roundsFor(n);
-  return (int)((n + tile - 1) / tile);
 }
 
 __device__ inline u64 mix64(u64 k) {
@@ -157,13 +142,13 @@ __device__ void clearRegions(const ClearRegions &r, int block, int blocks) {
   }
 }
 
-// tagged[i] = bucket of point i (kNoBucket outside the grid) above the low half of its cell key;
+// tagged[i] = bucket of point i (kNoDigit outside the grid) above the low half of its cell key;
 // hist[tile][bucket] = points of the tile in the bucket.
 __global__ __launch_bounds__(kTileThreads) void voxCountBuckets(
     const float *__restrict__ points, const float *__restrict__ voxel_size, const float *__restrict__ range,
     int64_t n, int num_features, int buckets, int rounds, int tiles, u64 *__restrict__ tagged,
     uint32_t *__restrict__ hist, ClearRegions clear) {
-  __shared__ uint32_t s_count[kMaxBuckets];
+  __shared__ uint32_t s_count[kMaxDigits];
   if ((int)blockIdx.x >= tiles) {
     clearRegions(clear, blockIdx.x - tiles, gridDim.x - tiles);
     return;
@@ -171,11 +156,11 @@ __global__ __launch_bounds__(kTileThreads) void voxCountBuckets(
   for (int b = threadIdx.x; b < buckets; b += kTileThreads) s_count[b] = 0;
   __syncthreads();
   const int64_t begin = (int64_t)blockIdx.x * rounds * kRound;
-  for (int j = 0; j < rounds * kWaveChunks; ++j) {
+  for (int j = 0; j < rounds * device_sort::kWaveChunks; ++j) {
     const int64_t i = begin + (int64_t)j * kTileThreads + threadIdx.x;
     if (i >= n) break;
     const Cell c = cellOfPoint(points + i * num_features, voxel_size, range);
-    u64 tag = (u64)kNoBucket << 32;
+    u64 tag = (u64)kNoDigit << 32;
     if (c.cz >= 0) {
       const u64 key = cellKey(c);
       const uint32_t bucket = (uint32_t)mix64(key) & (uint32_t)(buckets - 1);
@@ -188,154 +173,16 @@ __global__ __launch_bounds__(kTileThreads) void voxCountBuckets(
   for (int b = threadIdx.x; b < buckets; b += kTileThreads) hist[(size_t)blockIdx.x * buckets + b] = s_count[b];
 }
 
-// hist[0..tiles)[bucket] -> exclusive prefix sums down the column, its sum to totals[bucket].  A
-// workgroup takes 32 columns (128-byte rows), 32 groups of threads share the tiles.
-constexpr int kColumns = 32;
-constexpr int kColumnGroups = 32;
-__global__ __launch_bounds__(kColumns *kColumnGroups) void voxScanColumns(uint32_t *__restrict__ hist, int tiles,
-                                                                          int buckets,
-                                                                          uint32_t *__restrict__ totals) {
-  __shared__ uint32_t s_sum[kColumnGroups][kColumns];
-  const int c = threadIdx.x % kColumns, g = threadIdx.x / kColumns;
-  const int per = (tiles + kColumnGroups - 1) / kColumnGroups;  // at most 32 (kMaxTiles)
-  const int t0 = g * per, t1 = t0 + per < tiles ? t0 + per : tiles;
-  uint32_t *column = hist + blockIdx.x * kColumns + c;
-  uint32_t v[kMaxTiles / kColumnGroups];
-  uint32_t sum = 0;
-#pragma unroll
-  for (int u = 0; u < kMaxTiles / kColumnGroups; ++u) {
-    v[u] = t0 + u < t1 ? column[(size_t)(t0 + u) * buckets] : 0u;
-  }
-#pragma unroll
-  for (int u = 0; u < kMaxTiles / kColumnGroups; ++u) sum += v[u];
-  s_sum[g][c] = sum;
-  __syncthreads();
-  uint32_t run = 0, total = 0;
-#pragma unroll
-  for (int w = 0; w < kColumnGroups; ++w) {
-    const uint32_t s = s_sum[w][c];
-    run += w < g ? s : 0u;
-    total += s;
-  }
-#pragma unroll
-  for (int u = 0; u < kMaxTiles / kColumnGroups; ++u) {
-    if (t0 + u < t1) column[(size_t)(t0 + u) * buckets] = run;
-    run += v[u];
-  }
-  if (g == 0) totals[blockIdx.x * kColumns + c] = total;
-}
-
-// Exclusive prefix sums of totals[0..buckets) into s_first, by the whole workgroup.
-template <int THREADS>
-__device__ inline void bucketStarts(const uint32_t *__restrict__ totals, int buckets, uint32_t *s_first,
-                                    uint32_t *s_wave) {
-  constexpr int kPer = kMaxBuckets / THREADS;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  uint32_t v[kPer], sum = 0;
-#pragma unroll
-  for (int u = 0; u < kPer; ++u) {
-    v[u] = tid * kPer + u < buckets ? totals[tid * kPer + u] : 0u;
-    sum += v[u];
-  }
-  const uint32_t incl = device_sort::waveInclusiveSum(sum);
-  if (lane == 63) s_wave[wave] = incl;
-  __syncthreads();
-  uint32_t run = incl - sum;
-  for (int w = 0; w < wave; ++w) run += s_wave[w];
-#pragma unroll
-  for (int u = 0; u < kPer; ++u) {
-    if (tid * kPer + u < buckets) s_first[tid * kPer + u] = run;
-    run += v[u];
-  }
-}
-
-// grouped[] = (point index above the low half of the cell key), by bucket, points of a bucket in
-// their order.  A wave owns 256 consecutive points and takes them 64 at a time; lanes of one
-// bucket find each other with a ballot per bucket bit.
-__global__ __launch_bounds__(kTileThreads) void voxPartition(const u64 *__restrict__ tagged, int64_t n, int buckets,
-                                                             int bucket_bits, int rounds,
-                                                             const uint32_t *__restrict__ hist,
-                                                             const uint32_t *__restrict__ totals,
-                                                             u64 *__restrict__ grouped,
-                                                             uint32_t *__restrict__ bucket_start) {
-  __shared__ uint16_t s_count[kTileWaves][kMaxBuckets];  // points of a bucket per wave, then in the waves before
-  __shared__ uint32_t s_first[kMaxBuckets];              // where the next point of a bucket goes
-  __shared__ uint32_t s_wave[kTileWaves];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  bucketStarts<kTileThreads>(totals, buckets, s_first, s_wave);
-  __syncthreads();
-  if (blockIdx.x == 0)
-    for (int b = tid; b < buckets; b += kTileThreads) bucket_start[b] = s_first[b];
-  for (int b = tid; b < buckets; b += kTileThreads) s_first[b] += hist[(size_t)blockIdx.x * buckets + b];
-  volatile uint16_t *mine = s_count[wave];
-  const u64 below = (1ull << lane) - 1ull;
-  for (int round = 0; round < rounds; ++round) {
-    for (int b = tid; b < buckets; b += kTileThreads)
-#pragma unroll
-      for (int w = 0; w < kTileWaves; ++w) s_count[w][b] = 0;
-    __syncthreads();
-    const int64_t base = ((int64_t)blockIdx.x * rounds + round) * kRound + (int64_t)wave * (64 * kWaveChunks);
-    u64 tag[kWaveChunks];
-    uint32_t place[kWaveChunks];
-#pragma unroll
-    for (int j = 0; j < kWaveChunks; ++j) {
-      const int64_t i = base + j * 64 + lane;
-      tag[j] = i < n ? tagged[i] : (u64)kNoBucket << 32;
-    }
-#pragma unroll
-    for (int j = 0; j < kWaveChunks; ++j) {
-      const uint32_t bucket = (uint32_t)(tag[j] >> 32);
-      const bool valid = bucket != kNoBucket;
-      u64 peers = __ballot(valid);
-      for (int b = 0; b < bucket_bits; ++b) {
-        const bool bit = (bucket >> b) & 1u;
-        const u64 with = __ballot(bit);
-        peers &= bit ? with : ~with;
-      }
-      const int leader = valid ? __ffsll((long long)peers) - 1 : lane;
-      uint32_t before = 0;  // points of the bucket in the wave's earlier chunks
-      if (valid && lane == leader) {
-        before = mine[bucket];
-        mine[bucket] = (uint16_t)(before + (uint32_t)__popcll(peers));
-      }
-      before = __shfl(before, leader, 64);
-      place[j] = before + (uint32_t)__popcll(peers & below);
-    }
-    __syncthreads();
-    // the waves' counts of a bucket become the counts of the waves before
-    uint32_t round_total[kMaxBuckets / kTileThreads];
-#pragma unroll
-    for (int u = 0; u < kMaxBuckets / kTileThreads; ++u) {
-      const int b = tid + u * kTileThreads;
-      uint32_t run = 0;
-      if (b < buckets) {
-#pragma unroll
-        for (int w = 0; w < kTileWaves; ++w) {
-          const uint32_t c = s_count[w][b];
-          s_count[w][b] = (uint16_t)run;
-          run += c;
-        }
-      }
-      round_total[u] = run;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kWaveChunks; ++j) {
-      const uint32_t bucket = (uint32_t)(tag[j] >> 32);
-      if (bucket != kNoBucket) {
-        const uint32_t i = (uint32_t)(base + j * 64 + lane);
-        grouped[(size_t)s_first[bucket] + s_count[wave][bucket] + place[j]] = (u64)i << 32 | (uint32_t)tag[j];
-      }
-    }
-    if (round + 1 == rounds) break;
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < kMaxBuckets / kTileThreads; ++u) {
-      const int b = tid + u * kTileThreads;
-      if (b < buckets) s_first[b] += round_total[u];
-    }
-  }
-}
+// The points by bucket: (point index above the low half of the cell key), points of a bucket in
+// their order.
+struct BucketedPoints {
+  typedef u64 Item;
+  const u64 *tagged;
+  u64 *grouped;
+  __device__ Item load(int64_t i) const { return tagged[i]; }
+  __device__ uint32_t digit(Item t) const { return (uint32_t)(t >> 32); }
+  __device__ void store(size_t to, Item t, int64_t i) const { grouped[to] = (u64)i << 32 | (uint32_t)t; }
+};
 
 // ---- ranks inside the cells of a bucket --------------------------------------------------
 
@@ -472,82 +319,23 @@ __global__ __launch_bounds__(kRankThreads) void voxRankInCells(
 
 // ---- voxel numbers -----------------------------------------------------------------------
 
-// A tile of 4096 points: 64 words of its bitmap of first points, the number of first points of the
-// tile in front of each word, and their number in the tile.
-constexpr int kFirstsTile = 4096;
-__global__ __launch_bounds__(kBlock) void voxRankFirsts(const uint32_t *__restrict__ state, int64_t n,
-                                                        u64 *__restrict__ first_bits,
-                                                        uint32_t *__restrict__ word_firsts,
-                                                        uint32_t *__restrict__ tile_firsts) {
-  __shared__ u64 s_bits[kFirstsTile / 64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t base = (int64_t)blockIdx.x * kFirstsTile + (int64_t)wave * 1024;
-  uint32_t v[16];
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int64_t i = base + j * 64 + lane;
-    v[j] = i < n ? state[i] : 0u;
-  }
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const u64 bits = __ballot((v[j] & kIsFirst) != 0);
-    if (lane == 0) s_bits[wave * 16 + j] = bits;
-  }
-  __syncthreads();
-  if (wave == 0) {
-    const u64 bits = s_bits[lane];
-    const uint32_t c = (uint32_t)__popcll(bits);
-    const uint32_t incl = device_sort::waveInclusiveSum(c);
-    first_bits[(size_t)blockIdx.x * 64 + lane] = bits;
-    word_firsts[(size_t)blockIdx.x * 64 + lane] = incl - c;
-    if (lane == 63) tile_firsts[blockIdx.x] = incl;
-    if (lane == 0 && blockIdx.x + 1 == gridDim.x) tile_firsts[gridDim.x] = 0;  // becomes the sum of all in a scan
-  }
-}
+struct FirstPoints {
+  const uint32_t *state;
+  __device__ bool flagged(int64_t i) const { return (state[i] & kIsFirst) != 0; }
+};
 
-// Point i of the cloud.  Up to kSumTiles tiles every workgroup sums up the tiles' counts itself, which
-// takes less than a launch of its own does; more are scanned before (`scanned`: tile_firsts holds
-// prefix sums, and one word behind them the sum of all).
-constexpr int kSumTiles = 1024;
+// Point i of the cloud.
 __global__ __launch_bounds__(kBlock) void voxAssign(
     const float *__restrict__ points, const float *__restrict__ voxel_size, const float *__restrict__ range, int64_t n,
     int num_features, const uint32_t *__restrict__ state, const uint32_t *__restrict__ first_of,
-    const u64 *__restrict__ first_bits, const uint32_t *__restrict__ word_firsts,
-    const uint32_t *__restrict__ tile_firsts, int tiles, bool scanned, bool quads, int max_points, int max_voxels,
+    device_sort::FlagRanks firsts, bool quads, int max_points, int max_voxels,
     float *__restrict__ voxels, int32_t *__restrict__ coors, int32_t *__restrict__ num_points_per_voxel,
     int32_t *__restrict__ voxel_num, u64 *host_voxel_num, u64 stamp) {
-  __shared__ uint32_t s_tile[kSumTiles];
-  __shared__ uint32_t s_wave[kBlock / 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ device_sort::FlagSums s_sums;
+  const int tid = threadIdx.x;
   const int64_t i = (int64_t)blockIdx.x * kBlock + tid;
   const uint32_t st = i < n ? state[i] : 0u;
-  uint32_t all = 0;
-  if (scanned) {
-    if (blockIdx.x == 0 && tid == 0) all = tile_firsts[tiles];
-  } else {
-    constexpr int kPer = kSumTiles / kBlock;
-    uint32_t v[kPer], sum = 0;
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      v[u] = tid * kPer + u < tiles ? tile_firsts[tid * kPer + u] : 0u;
-      sum += v[u];
-    }
-    const uint32_t incl = device_sort::waveInclusiveSum(sum);
-    if (lane == 63) s_wave[wave] = incl;
-    __syncthreads();
-    uint32_t run = incl - sum;
-#pragma unroll
-    for (int w = 0; w < kBlock / 64; ++w) {
-      run += w < wave ? s_wave[w] : 0u;
-      all += s_wave[w];
-    }
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      s_tile[tid * kPer + u] = run;
-      run += v[u];
-    }
-    __syncthreads();
-  }
+  const uint32_t all = s_sums.add(firsts);
   if (blockIdx.x == 0 && tid == 0) {
     const int32_t kept = all < (uint32_t)max_voxels ? (int32_t)all : max_voxels;
     *voxel_num = kept;
@@ -558,9 +346,7 @@ __global__ __launch_bounds__(kBlock) void voxAssign(
   const bool is_first = (st & kIsFirst) != 0;
   const uint32_t f = is_first ? (uint32_t)i : first_of[i];
   const uint32_t r = is_first ? 0u : st;
-  const uint32_t tile = f / kFirstsTile, word = f >> 6;
-  const uint32_t v = (scanned ? tile_firsts[tile] : s_tile[tile]) + word_firsts[word] +
-                     (uint32_t)__popcll(first_bits[word] & ((1ull << (f & 63)) - 1ull));
+  const uint32_t v = s_sums.before(firsts, f);
   if (v >= (uint32_t)max_voxels) return;
   const float *src = points + (size_t)i * num_features;
   float *dst = voxels + ((size_t)v * max_points + r) * num_features;
@@ -578,14 +364,14 @@ __global__ __launch_bounds__(kBlock) void voxAssign(
 }
 
 struct Workspace {
-  u64 *tagged, *grouped, *first_bits, *wide_keys;
-  uint32_t *state, *first_of, *hist, *totals, *bucket_start, *word_firsts, *tile_firsts, *wide_counts, *wide_firsts;
+  u64 *tagged, *grouped, *wide_keys;
+  uint32_t *state, *first_of, *counters, *bucket_start, *wide_counts, *wide_firsts;
+  device_sort::FlagRanks firsts;
   size_t total;
 };
 
 Workspace carve(void *base, const VoxelizeShape &s) {
   const size_t n = (size_t)s.num_points;
-  const size_t firsts_tiles = (n + kFirstsTile - 1) / kFirstsTile;
   // Blocks start at the caller's pointer rounded up to 256 bytes (64-bit words need their
   // alignment whatever the caller passes); the reported size includes that slack.  A null base
   // only measures.
@@ -603,12 +389,11 @@ Workspace carve(void *base, const VoxelizeShape &s) {
   w.grouped = longs(n);
   w.state = words(n);
   w.first_of = words(n);
-  w.hist = words((size_t)tilesFor(s.num_points) * bucketsFor(s.num_points));
-  w.totals = words(kMaxBuckets);
-  w.bucket_start = words(kMaxBuckets);
-  w.first_bits = longs(firsts_tiles * 64);
-  w.word_firsts = words(firsts_tiles * 64);
-  w.tile_firsts = words(firsts_tiles + 8);
+  w.counters = words(device_sort::counterWords(s.num_points, bucketsFor(s.num_points)));
+  w.bucket_start = words(kMaxDigits);
+  w.firsts.bits = longs(device_sort::flagBitmapWords(s.num_points));
+  w.firsts.before_word = words(device_sort::flagBitmapWords(s.num_points));
+  w.firsts.tiles = words(device_sort::flagTileWords(s.num_points));
   w.wide_keys = longs(3 * n);
   w.wide_counts = words(3 * n);
   w.wide_firsts = words(3 * n);
@@ -626,9 +411,10 @@ hipError_t launchVoxelize(const LaunchCtx &lc, const VoxelizeShape &s, const flo
                           int32_t *num_points_per_voxel, int32_t *voxel_num, unsigned long long *host_voxel_num,
                           unsigned long long stamp) {
   const int64_t n = s.num_points;
-  const Workspace w = carve(workspace, s);
+  Workspace w = carve(workspace, s);
   if (w.total > workspace_bytes) return hipErrorInvalidValue;
-  const int buckets = bucketsFor(n), rounds = roundsFor(n), tiles = tilesFor(n);
+  const int buckets = bucketsFor(n), rounds = device_sort::roundsFor(n), tiles = device_sort::tilesFor(n);
+  uint32_t *totals = w.counters, *hist = w.counters + kMaxDigits;
   int bucket_bits = 0;
   while ((1 << bucket_bits) < buckets) ++bucket_bits;
 
@@ -649,49 +435,41 @@ hipError_t launchVoxelize(const LaunchCtx &lc, const VoxelizeShape &s, const flo
   hipError_t e;
   lc.begin("voxCountBuckets");
   voxCountBuckets<<<tiles + (int)(clear_blocks < 1024 ? clear_blocks : 1024), kTileThreads, 0, lc.stream>>>(
-      points, voxel_size, coors_range, n, s.num_features, buckets, rounds, tiles, w.tagged, w.hist, clear);
+      points, voxel_size, coors_range, n, s.num_features, buckets, rounds, tiles, w.tagged, hist, clear);
   lc.end();
   if ((e = hipGetLastError()) != hipSuccess) return e;
 
-  lc.begin("voxScanColumns");
-  voxScanColumns<<<buckets / kColumns, kColumns * kColumnGroups, 0, lc.stream>>>(w.hist, tiles, buckets, w.totals);
+  lc.begin("scanColumns");
+  device_sort::scanColumns<<<buckets / device_sort::kColumns, device_sort::kColumns * device_sort::kColumnGroups, 0,
+                             lc.stream>>>(hist, tiles, buckets, totals);
   lc.end();
   if ((e = hipGetLastError()) != hipSuccess) return e;
 
-  lc.begin("voxPartition");
-  voxPartition<<<tiles, kTileThreads, 0, lc.stream>>>(w.tagged, n, buckets, bucket_bits, rounds, w.hist, w.totals,
-                                                      w.grouped, w.bucket_start);
+  lc.begin("partitionTiles");
+  device_sort::partitionTiles<<<tiles, kTileThreads, 0, lc.stream>>>(BucketedPoints{w.tagged, w.grouped}, n, buckets,
+                                                                     bucket_bits, rounds, hist, totals,
+                                                                     w.bucket_start);
   lc.end();
   if ((e = hipGetLastError()) != hipSuccess) return e;
 
   lc.begin("voxRankInCells");
   voxRankInCells<<<buckets, kRankThreads, 0, lc.stream>>>(points, voxel_size, coors_range, s.num_features,
-                                                         (uint32_t)s.max_points, w.grouped, w.bucket_start, w.totals,
+                                                         (uint32_t)s.max_points, w.grouped, w.bucket_start, totals,
                                                          w.wide_keys, w.wide_counts, w.wide_firsts, w.state,
                                                          w.first_of);
   lc.end();
   if ((e = hipGetLastError()) != hipSuccess) return e;
 
-  const int firsts_tiles = (int)((n + kFirstsTile - 1) / kFirstsTile);
-  const bool scanned = firsts_tiles > kSumTiles;
-  lc.begin("voxRankFirsts");
-  voxRankFirsts<<<firsts_tiles, kBlock, 0, lc.stream>>>(w.state, n, w.first_bits, w.word_firsts, w.tile_firsts);
+  lc.begin("rankFlags");
+  e = device_sort::rank(lc.stream, FirstPoints{w.state}, n, &w.firsts);
   lc.end();
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  if (scanned) {
-    lc.begin("scanCounters");
-    device_sort::scanCounters<<<1, device_sort::kScanThreads, 0, lc.stream>>>(w.tile_firsts,
-                                                                             (size_t)firsts_tiles + 1);
-    lc.end();
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
+  if (e != hipSuccess) return e;
 
   const bool quads = s.num_features == 4 &&
                      ((reinterpret_cast<uintptr_t>(points) | reinterpret_cast<uintptr_t>(voxels)) & 15) == 0;
   lc.begin("voxAssign");
   voxAssign<<<gridFor((size_t)n), kBlock, 0, lc.stream>>>(
-      points, voxel_size, coors_range, n, s.num_features, w.state, w.first_of, w.first_bits, w.word_firsts,
-      w.tile_firsts, firsts_tiles, scanned, quads, s.max_points, s.max_voxels, voxels, coors, num_points_per_voxel,
+      points, voxel_size, coors_range, n, s.num_features, w.state, w.first_of, w.firsts, quads, s.max_points, s.max_voxels, voxels, coors, num_points_per_voxel,
       voxel_num, host_voxel_num, stamp);
   lc.end();
   return hipGetLastError();
