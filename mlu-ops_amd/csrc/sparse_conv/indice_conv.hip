@@ -1629,11 +1629,14 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
         at[g] = kk < 0 ? kNoRow : at[g];
       }
     };
-    // 16 bytes of a row: reduction chunk kb, this lane's quarter; zeros where the row ends before
+    // 16 bytes of a row: reduction chunk kb, this lane's quarter; zeros where the row ends before.
+    // (The chunk is part of the lane's own offset, not of the scalar one: the hardware compares the
+    // lane's offset with the tensor's length less the scalar offset, and a tensor of one short row
+    // is shorter than the last chunk's place in it.)
     auto load_chunk = [&](uint32_t at, int kb) -> vec8 {
       const uint32_t piece = (uint32_t)(kb * 64 + quad * 16);
-      const uint32_t from = piece < (uint32_t)conv.row_bytes ? at + quad * 16 : kNoRow;
-      return __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(a_rows, from, kb * 64, 0));
+      const uint32_t from = piece < (uint32_t)conv.row_bytes ? at + piece : kNoRow;
+      return __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(a_rows, from, 0, 0));
     };
 
     vec8 rows[G][KB];
