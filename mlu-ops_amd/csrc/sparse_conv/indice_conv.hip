@@ -82,6 +82,9 @@ struct HalfElem {
   static constexpr int kVec = 8, kChunk = 32;
   static __device__ __forceinline__ float load(const storage *p) { return (float)*p; }
   static __device__ __forceinline__ void store(storage *p, float v) { *p = (_Float16)v; }
+  static __device__ __forceinline__ bool finite(storage v) {
+    return (__builtin_bit_cast(u16, v) & 0x7c00u) != 0x7c00u;
+  }
   static __device__ __forceinline__ float4v mfma(vec8 a, vec8 b, float4v c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
@@ -103,6 +106,7 @@ struct BFloat16Elem {
     u += 0x7fffu + ((u >> 16) & 1u);  // round to nearest even
     *p = (u16)(u >> 16);
   }
+  static __device__ __forceinline__ bool finite(storage v) { return (v & 0x7f80u) != 0x7f80u; }
   static __device__ __forceinline__ float4v mfma(vec8 a, vec8 b, float4v c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
@@ -114,6 +118,9 @@ struct FloatElem {
   static constexpr int kVec = 4, kChunk = 16;
   static __device__ __forceinline__ float load(const storage *p) { return *p; }
   static __device__ __forceinline__ void store(storage *p, float v) { *p = v; }
+  static __device__ __forceinline__ bool finite(storage v) {
+    return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u;
+  }
   // Four 16x16x4 steps; step s pairs element s of both fragments, i.e. channel
   // 4*kq + s in MFMA reduction slot kq: a permutation of the chunk's 16 channels.
   static __device__ __forceinline__ float4v mfma(vec8 a, vec8 b, float4v c) {
@@ -290,6 +297,12 @@ __global__ __launch_bounds__(256) void gatherConvSimt(const typename E::storage 
 
 // ---- MFMA gather convolution ---------------------------------------------------
 
+// Channels of a filter B(k, q, c) as they are, and as the kernel instance counts them.
+struct FilterShape {
+  int q, c;
+  int q_padded, c_padded;
+};
+
 // Filter repacked into MFMA operand fragments of 16 bytes per lane (VEC elements,
 // CHUNK reduction channels per fragment; 8 and 32 for the 2-byte types, 4 and 16
 // for float):
@@ -297,23 +310,20 @@ __global__ __launch_bounds__(256) void gatherConvSimt(const typename E::storage 
 //   = B(k, q = kb*CHUNK + VEC*(lane/16) + e, c = nb*16 + lane%16), zero for q >= Q
 // (16 reduction channels of a 2-byte type fill half a fragment) and for columns beyond the
 // filter's own: a filter of q x c channels runs on the instance of the next padded size.
-// One launch for the two independent preparations of the MFMA path: blocks
-// below fill_blocks set the row map to -1 (16-byte stores), the others repack
-// the filter.
-// Channels of a filter B(k, q, c) as they are, and as the kernel instance counts them.
-struct FilterShape {
-  int q, c;
-  int q_padded, c_padded;
-};
-
+// Behind the fragments lie K + 1 words.  Word k holds the call's ticket (a value no earlier call
+// used, so nothing has to be cleared), which word K repeats, if the filter of offset k holds an
+// infinity or a NaN: a kernel that multiplies rows of zeros takes such an offset apart, since zero
+// times infinity is a NaN.
 template <typename E>
 __device__ __forceinline__ void packFilter(const typename E::storage *W, int64_t sK, int64_t sQ, int64_t sC, int K,
-                                           const FilterShape &shape, typename E::storage *packed, int block,
-                                           int blocks) {
+                                           const FilterShape &shape, typename E::storage *packed,
+                                           unsigned long long ticket, int block, int blocks) {
   constexpr int VEC = E::kVec, CHUNK = E::kChunk;
   const int chunks = (shape.q_padded + CHUNK - 1) / CHUNK;
   const int groups = shape.c_padded / 16;
   const size_t total = (size_t)K * groups * chunks * 64;
+  unsigned long long *const nonfinite = reinterpret_cast<unsigned long long *>(packed + total * VEC);
+  if (block == 0 && threadIdx.x == 0) nonfinite[K] = ticket;
   for (size_t t = (size_t)block * 256 + threadIdx.x; t < total; t += (size_t)blocks * 256) {
     const int lane = (int)(t & 63);
     size_t rest = t >> 6;
@@ -323,11 +333,16 @@ __device__ __forceinline__ void packFilter(const typename E::storage *W, int64_t
     const int k = (int)(rest / groups);
     const int c = nb * 16 + (lane & 15);
     const int qb = kb * CHUNK + VEC * (lane >> 4);
+    bool finite = true;
 #pragma unroll
-    for (int e = 0; e < VEC; ++e)
-      packed[t * VEC + e] = qb + e < shape.q && c < shape.c
-                                ? W[(size_t)k * sK + (size_t)(qb + e) * sQ + (size_t)c * sC]
-                                : typename E::storage(0);
+    for (int e = 0; e < VEC; ++e) {
+      const typename E::storage v = qb + e < shape.q && c < shape.c
+                                        ? W[(size_t)k * sK + (size_t)(qb + e) * sQ + (size_t)c * sC]
+                                        : typename E::storage(0);
+      finite = finite && E::finite(v);
+      packed[t * VEC + e] = v;
+    }
+    if (!finite) nonfinite[k] = ticket;
   }
 }
 
@@ -358,13 +373,17 @@ __device__ __forceinline__ void padRows(const PadRows &pad) {
   }
 }
 
+// One launch for the independent preparations of the MFMA path on a row map: the first pad.blocks
+// workgroups copy the gathered rows to padded ones, the next fill_blocks set the row map to -1
+// (16-byte stores), the others repack the filter.
 template <typename E>
 __global__ __launch_bounds__(256) void fillMapPackFilter(PadRows pad, int32_t *map, size_t map_elems,
                                                          int fill_blocks,
                                                          const typename E::storage *W, int64_t sK,
                                                          int64_t sQ, int64_t sC, int K,
                                                          FilterShape shape,
-                                                         typename E::storage *packed, RunIf run_if) {
+                                                         typename E::storage *packed,
+                                                         unsigned long long ticket, RunIf run_if) {
   if (notWanted(run_if)) return;
   if ((int)blockIdx.x < pad.blocks) {
     padRows<typename E::storage>(pad);
@@ -379,7 +398,7 @@ __global__ __launch_bounds__(256) void fillMapPackFilter(PadRows pad, int32_t *m
     if (block == 0 && threadIdx.x < (map_elems & 3)) map[quads * 4 + threadIdx.x] = -1;
     return;
   }
-  packFilter<E>(W, sK, sQ, sC, K, shape, packed, block - fill_blocks,
+  packFilter<E>(W, sK, sQ, sC, K, shape, packed, ticket, block - fill_blocks,
                 (int)gridDim.x - pad.blocks - fill_blocks);
 }
 
@@ -486,7 +505,7 @@ __global__ __launch_bounds__(256) void packFilterCutPairLists(
     return;
   }
   if ((int)blockIdx.x - pad.blocks < pack_blocks) {
-    packFilter<E>(W, sK, sQ, sC, K, shape, packed, (int)blockIdx.x - pad.blocks, pack_blocks);
+    packFilter<E>(W, sK, sQ, sC, K, shape, packed, ticket, (int)blockIdx.x - pad.blocks, pack_blocks);
     return;
   }
   const int b = (int)blockIdx.x - pad.blocks - pack_blocks;
@@ -1272,6 +1291,9 @@ __global__ __launch_bounds__(64) void gatherConvWave(
 //     217 us.  So rows go in operand order again, a chunk requested right behind its last use,
 //     in eight waves per filter copy, and a wave multiplies only the groups that have a row
 //     at the offset.
+// All of them multiply rows of zeros for the partners that are not there, which is nothing as long
+// as the filter is finite.  An offset whose filter is not (packFilter says so) is taken out of the
+// walk and multiplied by itself, its products added to the rows that have a partner there only.
 constexpr int kDenseChunk = 27;      // offsets whose row-map slice is resident in LDS at once
 constexpr int kDenseMapBatch = 14;   // loads in flight per thread while a tile's row map is read
 constexpr uint32_t kNoRow = 0x80000000u;  // byte offset of a partner that is not there
@@ -1361,7 +1383,9 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
   __shared__ uint32_t s_map[KC][TR];  // where the partner row of (offset in chunk, tile row) begins, or kNoRow
   __shared__ int s_has[KC];
   __shared__ int s_first[KC];
+  __shared__ int s_finite[KC];        // the offset's filter holds no infinity and no NaN
   __shared__ uint32_t s_offsets;      // offsets of the chunk that have a pair in this tile
+  __shared__ uint32_t s_apart;        // those of them whose filter is not finite (not among s_offsets)
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1405,6 +1429,8 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
   const int quad = lane >> 4;
   const __amdgpu_buffer_rsrc_t a_rows = rowsBuffer(A, a_size);
   const char *w_base = reinterpret_cast<const char *>(packedW) + lane * 16;
+  const unsigned long long *const nonfinite =
+      reinterpret_cast<const unsigned long long *>(reinterpret_cast<const char *>(packedW) + (size_t)K * W_BYTES);
   const uint32_t w_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)s_w;
   const int row_first = wave * (G * 16) + pair;  // this lane's row in its wave's first group
   // Which 16 bytes of a row a lane asks for: its quarter, or in staged loads the piece that
@@ -1438,6 +1464,7 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
         count = count < 0 ? 0 : (count > TR ? TR : count);
         s_first[tid] = first;
         s_has[tid] = count;
+        s_finite[tid] = nonfinite[kc + tid] != nonfinite[K];
       }
       for (int i = tid; i < kn * TR; i += NT) (&s_map[0][0])[i] = kNoRow;
       __syncthreads();
@@ -1467,7 +1494,10 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
         }
       }
     } else {
-      if (tid < kn) s_has[tid] = 0;
+      if (tid < kn) {
+        s_has[tid] = 0;
+        s_finite[tid] = nonfinite[kc + tid] != nonfinite[K];
+      }
       __syncthreads();
       for (int base = tid; base < kn * TR; base += NT * kDenseMapBatch) {
         int v[kDenseMapBatch];
@@ -1493,11 +1523,41 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
     __syncthreads();
     if (wave == 0) {
       const bool has = lane < kn && s_has[lane < kn ? lane : 0] != 0;
-      const unsigned long long m = __ballot(has);
-      if (lane == 0) s_offsets = (uint32_t)m;
+      const bool finite = s_finite[lane < kn ? lane : 0] != 0;
+      const unsigned long long m = __ballot(has && finite), apart = __ballot(has && !finite);
+      if (lane == 0) {
+        s_offsets = (uint32_t)m;
+        s_apart = (uint32_t)apart;
+      }
     }
     __syncthreads();
     const uint32_t offsets = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_offsets);
+    for (uint32_t left = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_apart); left != 0; left &= left - 1) {
+      const int kk = __builtin_ctz(left);
+      int own = lane;  // (nothing of this rare loop is worked out ahead of it and held in registers)
+      asm volatile("" : "+v"(own));
+      const char *const filter = reinterpret_cast<const char *>(packedW) + own * 16 + (size_t)(kc + kk) * W_BYTES;
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const uint32_t at = s_map[kk][wave * (G * 16) + g * 16 + (own & 15)];
+        vec8 row[KB];
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          const uint32_t piece = (uint32_t)(kb * 64 + (own >> 4) * 16);
+          row[kb] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(
+                                                 a_rows, piece < (uint32_t)conv.row_bytes ? at + piece : kNoRow, 0, 0));
+        }
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          float4v product = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int kb = 0; kb < KB; ++kb)
+            product = E::mfma(*reinterpret_cast<const vec8 *>(filter + (nb * KB + kb) * 1024), row[kb], product);
+          if (at != kNoRow) acc[g][nb] += product;  // (a lane's results are of its own row)
+          asm volatile("" ::: "memory");            // one block's fragments in registers at a time
+        }
+      }
+    }
     if (offsets == 0) continue;
     // A phase: the OPP lowest offsets of `left` (fewer at the end), which are taken out of it.
     auto next_phase = [](uint32_t &left) -> uint32_t {
@@ -1509,13 +1569,14 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
       return phase;
     };
     // Fragment f of a phase's filters (its offsets in ascending order), as bytes of the packed
-    // filter.  Behind the phase's last offset: fragments of some other one, which nobody reads.
+    // filter.  Behind the phase's last offset: fragments of another offset of the walk, which are
+    // multiplied by zeros if at all.
     auto fragment_of = [&](uint32_t phase, int f) -> const char * {
       uint32_t left = phase;
 #pragma unroll
       for (int o = 1; o < OPP; ++o)
         if (f >= o * FRAGS && (left & (left - 1)) != 0) left &= left - 1;
-      const int k = left != 0 ? __builtin_ctz(left) : 0;
+      const int k = __builtin_ctz(left != 0 ? left : offsets);
       return w_base + ((size_t)(kc + k) * FRAGS + f % FRAGS) * 1024;
     };
     // The filters of a phase's offsets into half `half` of the ring: fragment f by wave f % WAVES.
@@ -2878,7 +2939,7 @@ GatherWorkspace carveGather(const ConvProblem &p, const GatherDims &d, void *bas
     // reduction channels are padded to whole 16-byte fragments (32 for the 2-byte types)
     const size_t chunk = 64 / elemSize(p.dtype);
     const size_t q_padded = ((size_t)d.q_padded + chunk - 1) / chunk * chunk;
-    ws.packed = take((size_t)p.K * q_padded * d.c_padded * elemSize(p.dtype));
+    ws.packed = take((size_t)p.K * q_padded * d.c_padded * elemSize(p.dtype) + ((size_t)p.K + 1) * 8);
     if (rowsNeedPadding(p.dtype, d.Q)) ws.padded_rows = take((size_t)d.n_src * paddedRowBytes(p.dtype, d.Q));
   }
   ws.bytes = off + kBaseAlign;
@@ -3067,12 +3128,13 @@ template <typename E, typename SRC>
 void launchDense(const LaunchCtx &lc, int q_padded, const void *A, int n_src, const ConvRows &rows, const void *packed,
                  const SRC &source, int R, int K, void *result) {
   const uint32_t a_size = (uint32_t)n_src * (uint32_t)rows.row_bytes;
-#define DENSE_BY_C(q)                                                                                     \
-  switch (rows.c_padded) {                                                                                \
-    case 16: launchDenseInstance<E, q, 16, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break;  \
-    case 32: launchDenseInstance<E, q, 32, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break;  \
-    case 64: launchDenseInstance<E, q, 64, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break;  \
-    default: launchDenseInstance<E, q, 128, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break; \
+#define DENSE_INSTANCE(q, c) launchDenseInstance<E, q, c, SRC>(lc, A, a_size, rows, packed, source, R, K, result)
+#define DENSE_BY_C(q)                       \
+  switch (rows.c_padded) {                  \
+    case 16: DENSE_INSTANCE(q, 16); break;  \
+    case 32: DENSE_INSTANCE(q, 32); break;  \
+    case 64: DENSE_INSTANCE(q, 64); break;  \
+    default: DENSE_INSTANCE(q, 128); break; \
   }
   switch (q_padded) {
     case 16: DENSE_BY_C(16) break;
@@ -3084,6 +3146,7 @@ void launchDense(const LaunchCtx &lc, int q_padded, const void *A, int n_src, co
     default: break;
   }
 #undef DENSE_BY_C
+#undef DENSE_INSTANCE
 }
 
 // Row maps are built on the flat grid from this many workgroups of the per-offset grid on.
@@ -3151,10 +3214,10 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
   // instead).  Worth it only where the row map is a single chunk of four launches.
   const bool speculate = p.list_trust == ListTrust::kUnknown && single_chunk && lc.choices.lists_on_trust != 0;
   const bool lists = use_mfma && listsUsable(p, d) && (p.list_trust == ListTrust::kInOrder || speculate);
+  const bool dense = use_mfma && useDenseKernel(lc, p, d);
   if (lists) {
     // Pair lists in order (as far as the caller knows: the first kernel checks): the
     // gather kernel reads them cut by tile, no row map.
-    const bool dense = useDenseKernel(lc, p, d);
     const int tile_cols = dense ? d.c_padded : mfmaTileCols(p, d);
     const int tile_rows = dense ? denseTileRows((int)sizeof(S), d.q_padded, d.c_padded) : mfmaTileRows(tile_cols);
     int tile_shift = 0;
@@ -3205,7 +3268,6 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
   // gather kernel for those rows, checked for lost pairs, and filled again for the next rows.
   int chunk_rows = own_map ? ws.map_rows : d.R;
   if (own_map && lc.choices.small_map_chunks == 1 && chunk_rows > kRepairPoolRows) chunk_rows = kRepairPoolRows;
-  const bool dense = use_mfma && useDenseKernel(lc, p, d);
   const int tile_cols = use_mfma && !dense ? mfmaTileCols(p, d) : d.c_padded;
   for (int row_base = 0; row_base < d.R; row_base += chunk_rows) {
     const int rows = d.R - row_base < chunk_rows ? d.R - row_base : chunk_rows;
@@ -3225,7 +3287,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
         lc.begin("fillMapPackFilter");
         fillMapPackFilter<E><<<pad_now.blocks + fill_blocks + pack_blocks, 256, 0, lc.stream>>>(
             pad_now, ws.map, map_elems, fill_blocks, static_cast<const S *>(f.base), f.stride_k, sQ, sC, p.K,
-            shape, static_cast<S *>(ws.packed), run_if);
+            shape, static_cast<S *>(ws.packed), p.ticket, run_if);
         lc.end();
       }
       if (own_map) n_accepted = launchScatterRowMap(lc, p, d, ws, inl, max_count, row_base, rows, run_if);
