@@ -252,6 +252,15 @@ __global__ __launch_bounds__(256) void gatherConvSimt(const typename E::storage 
     if (tid < TR) s_src[tid] = v;
     if (tid < 64) slots += __popcll(__ballot(v >= 0));
     if (!__syncthreads_or(v >= 0)) continue;
+    // A row without a partner takes the sums it had: zero times a filter that is not finite is a NaN.
+    bool has[2];
+    float before[2][4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      has[i] = s_src[ty * 2 + i] >= 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) before[i][j] = acc[i][j];
+    }
     for (int q0 = 0; q0 < Q; q0 += QC) {
 #pragma unroll
       for (int i = 0; i < TR * QC / 256; ++i) {
@@ -281,6 +290,10 @@ __global__ __launch_bounds__(256) void gatherConvSimt(const typename E::storage 
       }
       __syncthreads();
     }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = has[i] ? acc[i][j] : before[i][j];
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {

@@ -13,6 +13,7 @@ KERNELS = {
     "dense": ({"dense_tiles": True}, "gatherConvDense"),
     "pairs": ({"dense_tiles": False, "wave_per_tile": False}, "gatherConvMfma"),
     "wave": ({"dense_tiles": False}, "gatherConvWave"),
+    "simt": ({"gather_simt": True}, "gatherConvSimt"),
 }
 
 
@@ -78,6 +79,13 @@ def test_matrix_core_kernels(gpu_handle, kernel, dtype_name, ci, co, rows, space
 def test_wave_kernel(gpu_handle):
     for rows, space in CLOUDS:
         run(gpu_handle, "wave", "float16", 32, 32, rows, space, "cell", 0, np.inf)
+
+
+@pytest.mark.parametrize("dtype_name", ["float32", "float16", "bfloat16"])
+def test_generic_kernel(gpu_handle, dtype_name):
+    for rows, space in CLOUDS:
+        for ci, co in ((5, 70), (33, 130)):
+            run(gpu_handle, "simt", dtype_name, ci, co, rows, space, "mixed", 0, np.inf)
 
 
 @pytest.mark.parametrize("kernel", ["dense", "pairs"])
