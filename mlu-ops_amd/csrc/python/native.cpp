@@ -61,7 +61,10 @@ namespace {
   X(mluOpExtSetDistinctPairsPromise)                       \
   X(mluOpExtGetIndicePairsHostCounts)                      \
   X(mluOpExtGetVoxelizationHostCount)                      \
-  X(mluOpExtUseRowMap)
+  X(mluOpExtGetRowMapSize)                                 \
+  X(mluOpExtBuildRowMap)                                   \
+  X(mluOpExtUseRowMap)                                     \
+  X(mluOpExtForgetRowMap)
 
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -357,6 +360,23 @@ at::Tensor convBackwardFilter(mluOpHandle_t handle, const Buffers &buffers, cons
 struct StreamHandle {
   mluOpHandle_t handle = nullptr;
   std::mutex mutex;
+
+  // A row map's buffer is about to be freed: from any thread, whatever it holds.  The handle drops
+  // its record before the next map is built or used on it.
+  void forgetRowMap(const void *map) {
+    const std::lock_guard<std::mutex> lock(forget_mutex_);
+    forget_.push_back(map);
+  }
+  // (with `mutex` held)
+  void dropForgottenRowMaps() {
+    const std::lock_guard<std::mutex> lock(forget_mutex_);
+    for (const void *map : forget_) (void)api.mluOpExtForgetRowMap(handle, map);
+    forget_.clear();
+  }
+
+ private:
+  std::mutex forget_mutex_;
+  std::vector<const void *> forget_;
 };
 
 StreamHandle &streamHandle() {
@@ -376,39 +396,89 @@ StreamHandle &streamHandle() {
 
 // ---- the layers' autograd node -------------------------------------------------------------
 
-// What the three convolution operators need of a rulebook.  `row_maps` holds, by pair column,
-// the map buffers a caller shares between calls (undefined tensors: none).
+// What the three convolution operators need of a rulebook, with the row maps its calls share.  A
+// library handle knows only the maps that were built on it, so there is one for each handle the
+// rulebook is used on (one per stream) and pair column that names result rows (1: the layer's
+// outputs, 0: its inputs).  They live as long as this object, which a pending backward pass holds.
 struct LayerRulebook : torch::CustomClassHolder {
   at::Tensor pairs;
   Counts counts, filter_space;
   int64_t num_act_out = 0;
   bool sub_m = false, distinct = false;
-  at::Tensor row_maps[2];
 
-  const void *rowMap(int column) const {
-    return row_maps[column].defined() ? row_maps[column].data_ptr() : nullptr;
+  ~LayerRulebook() override {
+    for (const auto &[key, map] : row_maps_)
+      if (map.defined()) key.first->forgetRowMap(map.data_ptr());
   }
+
+  // The map for a call on `h` (whose mutex is held), built on first use; null: the operator builds
+  // its own, since the coordinates may repeat or there is nothing to map.  The handle carries the
+  // promise of distinct pairs, so the build need not count lost ones and wait for the stream.
+  const void *rowMap(StreamHandle &h, const Buffers &buffers, int column) {
+    if (!distinct) return nullptr;
+    h.dropForgottenRowMaps();
+    const Key key{&h, column};
+    {
+      const std::lock_guard<std::mutex> lock(maps_mutex_);
+      const auto found = row_maps_.find(key);
+      // (a handle keeps so many records: the oldest are gone when there were more)
+      if (found != row_maps_.end() && api.mluOpExtUseRowMap(h.handle, found->second.data_ptr()) == MLUOP_STATUS_SUCCESS) {
+        check(api.mluOpExtUseRowMap(h.handle, nullptr), "mluOpExtUseRowMap");
+        return found->second.data_ptr();
+      }
+    }
+    const int64_t L = pairs.size(2);
+    const int64_t rows = column == 1 ? num_act_out : L, source_rows = column == 1 ? L : num_act_out;
+    if (rows == 0 || source_rows == 0 || pairs.size(0) == 0) return nullptr;
+    const TensorDesc d_pairs(MLUOP_LAYOUT_ARRAY, MLUOP_DTYPE_INT32, pairs.sizes());
+    size_t bytes = 0;
+    check(api.mluOpExtGetRowMapSize(d_pairs, rows, &bytes), "mluOpExtGetRowMapSize");
+    const at::Tensor map = buffers.output({static_cast<int64_t>(bytes)}, at::kByte, "row map");
+    check(api.mluOpExtBuildRowMap(h.handle, d_pairs, pairs.data_ptr(), counts.data(), rows, source_rows, column,
+                                  map.data_ptr(), bytes, nullptr),
+          "mluOpExtBuildRowMap");
+    buffers.done("mluOpExtBuildRowMap");
+    const std::lock_guard<std::mutex> lock(maps_mutex_);
+    row_maps_[key] = map;
+    return map.data_ptr();
+  }
+
+  // (handle, column) of the maps there are
+  std::vector<std::pair<uintptr_t, int>> rowMaps() {
+    const std::lock_guard<std::mutex> lock(maps_mutex_);
+    std::vector<std::pair<uintptr_t, int>> keys;
+    for (const auto &[key, map] : row_maps_) keys.emplace_back(reinterpret_cast<uintptr_t>(key.first->handle), key.second);
+    return keys;
+  }
+
+ private:
+  using Key = std::pair<StreamHandle *, int>;
+  std::mutex maps_mutex_;  // never held while anything else is waited for
+  std::map<Key, at::Tensor> row_maps_;
 };
 using LayerRulebookPtr = c10::intrusive_ptr<LayerRulebook>;
 
 struct IndiceConv : torch::autograd::Function<IndiceConv> {
   static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &features,
-                            const at::Tensor &weight, const LayerRulebookPtr &rb, bool inverse, bool guarded) {
+                            const at::Tensor &weight, const LayerRulebookPtr &rb, bool inverse, bool share_row_maps,
+                            bool guarded) {
     const at::Tensor x = features.contiguous(), w = weight.contiguous();
     ctx->save_for_backward({x, w});
     ctx->saved_data["rulebook"] = c10::IValue::make_capsule(rb);
     ctx->saved_data["inverse"] = inverse;
+    ctx->saved_data["share_row_maps"] = share_row_maps;
     ctx->saved_data["guarded"] = guarded;
     StreamHandle &h = streamHandle();
     const std::lock_guard<std::mutex> lock(h.mutex);
     check(api.mluOpExtSetDistinctPairsPromise(h.handle, rb->distinct), "mluOpExtSetDistinctPairsPromise");
     const Buffers buffers(guarded, x.device());
+    const void *map = share_row_maps ? rb->rowMap(h, buffers, inverse ? 0 : 1) : nullptr;
     // an inverse layer runs the partner layer's rulebook backwards: one output row per input
     // row of the partner
     return inverse ? convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts,
-                                 rb->pairs.size(2), false, 1, rb->rowMap(0))
+                                 rb->pairs.size(2), false, 1, map)
                    : convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts,
-                                 rb->num_act_out, rb->sub_m, 0, rb->rowMap(1));
+                                 rb->num_act_out, rb->sub_m, 0, map);
   }
 
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx,
@@ -417,7 +487,7 @@ struct IndiceConv : torch::autograd::Function<IndiceConv> {
     const at::Tensor &x = saved[0], &w = saved[1];
     const auto rb = c10::static_intrusive_pointer_cast<LayerRulebook>(ctx->saved_data["rulebook"].toCapsule());
     const bool inverse = ctx->saved_data["inverse"].toBool();
-    torch::autograd::variable_list out(5);
+    torch::autograd::variable_list out(6);
     if (!grads[0].defined()) return out;
     const at::Tensor dy = grads[0].contiguous();
     StreamHandle &h = streamHandle();
@@ -425,9 +495,12 @@ struct IndiceConv : torch::autograd::Function<IndiceConv> {
     check(api.mluOpExtSetDistinctPairsPromise(h.handle, rb->distinct), "mluOpExtSetDistinctPairsPromise");
     const Buffers buffers(ctx->saved_data["guarded"].toBool(), x.device());
     const bool sub_m = !inverse && rb->sub_m;
-    if (ctx->needs_input_grad(0))
+    if (ctx->needs_input_grad(0)) {
+      const void *map =
+          ctx->saved_data["share_row_maps"].toBool() ? rb->rowMap(h, buffers, inverse ? 1 : 0) : nullptr;
       out[0] = convBackwardData(h.handle, buffers, dy, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts, sub_m,
-                                x.size(1), inverse, x.size(0), rb->rowMap(inverse ? 1 : 0));
+                                x.size(1), inverse, x.size(0), map);
+    }
     if (ctx->needs_input_grad(1))
       out[1] = convBackwardFilter(h.handle, buffers, x, dy, rb->pairs, rb->counts, rb->filter_space, sub_m, inverse,
                                   true, MLUOP_LAYOUT_ARRAY);
@@ -652,13 +725,10 @@ PYBIND11_MODULE(_native, m) {
         rb->distinct = distinct;
         return rb;
       }))
-      .def("set_row_map", [](LayerRulebook &rb, int column, std::optional<at::Tensor> map) {
-        if (column != 0 && column != 1) throw py::index_error("a pair has two columns");
-        rb.row_maps[column] = map ? *map : at::Tensor();
-      });
+      .def("row_maps", &LayerRulebook::rowMaps, "(handle, pair column) of the row maps its calls have built.");
   m.def("indice_conv", [](const at::Tensor &features, const at::Tensor &weight, const LayerRulebookPtr &rulebook,
-                          bool inverse, bool guarded) {
+                          bool inverse, bool share_row_maps, bool guarded) {
     NoGil released;
-    return IndiceConv::apply(features, weight, rulebook, inverse, guarded);
+    return IndiceConv::apply(features, weight, rulebook, inverse, share_row_maps, guarded);
   });
 }

@@ -16,7 +16,7 @@ import math
 
 import torch
 
-from . import Handle, RowMap, _guarded, get_indice_pairs, native, regular_output_space
+from . import Handle, _guarded, get_indice_pairs, native, regular_output_space
 
 _handles = {}
 
@@ -62,38 +62,20 @@ class Rulebook:
         self.filter_space = tuple(filter_space)
         self.sub_m = sub_m
         self.out_space = tuple(out_space)
-        self._row_maps = {}
         self._for_operators = None
 
-    def for_operators(self, needs_grad, inverse):
-        """What the native operators take of this rulebook, with the shared row maps it is to use."""
+    def for_operators(self):
+        """What the native operators take of this rulebook; it holds the row maps they share."""
         if self._for_operators is None:
             self._for_operators = native().LayerRulebook(self.pairs, self.indice_num, self.num_act_out,
                                                          list(self.filter_space), self.sub_m, self.distinct)
-        if _share_row_maps or self._row_maps:
-            handle = _handle()
-            for column in (0, 1):
-                m = self.row_map(handle, column) if needs_grad or column == (0 if inverse else 1) else None
-                self._for_operators.set_row_map(column, None if m is None else m.buffer)
         return self._for_operators
 
-    def row_map(self, handle, row_column):
-        """The [K, rows] row map of this rulebook for one direction (row_column 1: rows are the
-        layer's outputs; 0: its inputs), built on first use and shared by every layer and pass that
-        uses the rulebook.  None when the coordinates are not known to be distinct, or when the
-        build found pairs that share a slot: the operators then build their own map per call."""
-        if not (self.distinct and _share_row_maps):
-            return None
-        key = (handle.ptr.value, row_column)   # the library records a map with the handle that built it
-        if key not in self._row_maps:
-            L = self.pairs.shape[2]
-            rows, source_rows = (self.num_act_out, L) if row_column == 1 else (L, self.num_act_out)
-            # the coordinates are known to be distinct and the handle carries that promise: the
-            # build need not count lost pairs, which would make the host wait for the stream
-            handle.promise_distinct_pairs(True)
-            m = RowMap(handle, self.pairs, self.indice_num, rows, source_rows, row_column, verify=False)
-            self._row_maps[key] = m if m.usable else None
-        return self._row_maps[key]
+    @property
+    def _row_maps(self):
+        """{(handle address, pair column that names the result rows): True} of the row maps built so far (with
+        `share_row_maps` on, for coordinates known to be distinct; on first use, one per handle and direction)."""
+        return {} if self._for_operators is None else dict.fromkeys(self._for_operators.row_maps(), True)
 
 
 class SparseTensor:
@@ -130,8 +112,7 @@ class _IndiceConv:
 
     @staticmethod
     def apply(features, weight, rulebook, inverse=False):
-        needs_grad = torch.is_grad_enabled() and (features.requires_grad or weight.requires_grad)
-        return native().indice_conv(features, weight, rulebook.for_operators(needs_grad, inverse), inverse, _guarded())
+        return native().indice_conv(features, weight, rulebook.for_operators(), inverse, _share_row_maps, _guarded())
 
 
 def _triple(v):

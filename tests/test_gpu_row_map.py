@@ -230,3 +230,70 @@ def test_layers_with_known_distinct_coordinates_share_maps(gpu_handle):
     # the tensor that was not declared distinct ran its first stage without maps (the strided
     # layer's output never repeats a coordinate, so the stage behind it has them either way)
     assert len(x_a.rulebooks["a"]._row_maps) == 0 and len(x_b.rulebooks["a"]._row_maps) == 2
+
+
+def layer_and_tensor(spnn, seed, dtype="float16"):
+    import torch
+    idx = torch.from_numpy(random_voxels(np.random.default_rng(seed), 1, (12, 16, 16), 2000)).cuda()
+    torch.manual_seed(seed)
+    layer = spnn.SubMConv3d(16, 32, 3, indice_key="a").cuda().to(getattr(torch, dtype))
+    feats = torch.randn(idx.shape[0], 16, device="cuda").to(getattr(torch, dtype))
+    return layer, feats, idx
+
+
+def test_shared_maps_serve_every_stream_of_a_rulebook(gpu_handle):
+    """One rulebook, forward on one stream, forward on another, then both backward passes: each finds
+    the map of its own stream's handle."""
+    import torch
+    from mluop_hip import nn as spnn
+    layer, feats, idx = layer_and_tensor(spnn, 71)
+    plain_x = feats.clone().requires_grad_(True)
+    plain = layer(spnn.SparseTensor(plain_x, idx, (12, 16, 16), 1, distinct=True)).features
+    plain.float().square().sum().backward()
+    plain_w = layer.weight.grad.clone()
+    torch.cuda.synchronize()
+
+    spnn.share_row_maps(True)
+    try:
+        t = spnn.SparseTensor(feats, idx, (12, 16, 16), 1, distinct=True)
+        layer(t)                       # the rulebook is there before either stream uses it
+        torch.cuda.synchronize()
+        streams, outs, xs = [torch.cuda.Stream(), torch.cuda.Stream()], [], []
+        for s in streams:
+            with torch.cuda.stream(s):
+                x = feats.clone().requires_grad_(True)
+                outs.append(layer(t.replace_features(x)).features)
+                xs.append(x)
+        torch.cuda.synchronize()
+        for s, out, x in zip(streams, outs, xs):
+            layer.weight.grad = None
+            with torch.cuda.stream(s):
+                out.float().square().sum().backward()
+            torch.cuda.synchronize()
+            assert torch.equal(out, plain) and torch.equal(x.grad, plain_x.grad)
+            assert torch.equal(layer.weight.grad, plain_w)
+    finally:
+        spnn.share_row_maps(False)
+
+
+def test_shared_maps_live_as_long_as_the_backward_pass(gpu_handle):
+    """The sparse tensor, and with it the rulebook, may be gone when the gradient is asked for."""
+    import gc
+    import torch
+    from mluop_hip import nn as spnn
+    layer, feats, idx = layer_and_tensor(spnn, 72)
+
+    def gradient(share):
+        spnn.share_row_maps(share)
+        try:
+            x = feats.clone().requires_grad_(True)
+            out = layer(spnn.SparseTensor(x, idx, (12, 16, 16), 1, distinct=True)).features
+            gc.collect()
+            out.float().square().sum().backward()
+            torch.cuda.synchronize()
+            return out.detach(), x.grad
+        finally:
+            spnn.share_row_maps(False)
+
+    for a, b in zip(gradient(False), gradient(True)):
+        assert torch.equal(a, b)
