@@ -355,8 +355,10 @@ at::Tensor convBackwardFilter(mluOpHandle_t handle, const Buffers &buffers, cons
 // ---- handles of the layers -----------------------------------------------------------------
 
 // One library handle per (device, stream), made on first use and kept for the life of the
-// process; its mutex keeps the calls of one operator together when several threads use one
-// stream.
+// process.  Several threads may use one stream and so one handle: every operator below that is
+// called on it holds its mutex (OperatorLock) from its first look at the handle to the last word
+// it waits for, since the calls in between share the handle's stamps, pinned words and settings.
+// (A handle that a caller made is the caller's to use from one thread at a time.)
 struct StreamHandle {
   mluOpHandle_t handle = nullptr;
   std::mutex mutex;
@@ -379,20 +381,50 @@ struct StreamHandle {
   std::vector<const void *> forget_;
 };
 
+struct StreamHandles {
+  std::mutex mutex;
+  std::map<std::pair<int, hipStream_t>, StreamHandle> by_stream;  // (entries stay where they are)
+  std::map<mluOpHandle_t, StreamHandle *> by_handle;
+};
+StreamHandles &streamHandles() {
+  static auto *all = new StreamHandles();
+  return *all;
+}
+
+// That of the current device and stream.
 StreamHandle &streamHandle() {
-  static std::mutex mutex;
-  static auto *handles = new std::map<std::pair<int, hipStream_t>, StreamHandle>();
   const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream();
-  std::lock_guard<std::mutex> lock(mutex);
-  StreamHandle &h = (*handles)[{static_cast<int>(stream.device_index()), stream.stream()}];
+  StreamHandles &all = streamHandles();
+  const std::lock_guard<std::mutex> lock(all.mutex);
+  StreamHandle &h = all.by_stream[{static_cast<int>(stream.device_index()), stream.stream()}];
   if (h.handle == nullptr) {
-    check(api.mluOpCreate(&h.handle), "mluOpCreate");
-    check(api.mluOpSetQueue(h.handle, reinterpret_cast<mluOpQueue_t>(stream.stream())), "mluOpSetQueue");
+    mluOpHandle_t made = nullptr;
+    check(api.mluOpCreate(&made), "mluOpCreate");
+    check(api.mluOpSetQueue(made, reinterpret_cast<mluOpQueue_t>(stream.stream())), "mluOpSetQueue");
     // SparseInverseConv3d runs the operators with inverse = 1
-    check(api.mluOpExtSetSparseConvExtendedModes(h.handle, 1), "mluOpExtSetSparseConvExtendedModes");
+    check(api.mluOpExtSetSparseConvExtendedModes(made, 1), "mluOpExtSetSparseConvExtendedModes");
+    all.by_handle[made] = &h;
+    h.handle = made;
   }
   return h;
 }
+
+// Held for one operator on `handle`, without the GIL (a buffer in guard mode takes it).
+class OperatorLock {
+ public:
+  explicit OperatorLock(StreamHandle &h) : lock_(h.mutex) {}
+  explicit OperatorLock(mluOpHandle_t handle) {
+    StreamHandles &all = streamHandles();
+    std::unique_lock<std::mutex> look(all.mutex);
+    const auto found = all.by_handle.find(handle);
+    if (found == all.by_handle.end()) return;
+    look.unlock();
+    lock_ = std::unique_lock<std::mutex>(found->second->mutex);
+  }
+
+ private:
+  std::unique_lock<std::mutex> lock_;
+};
 
 // ---- the layers' autograd node -------------------------------------------------------------
 
@@ -469,7 +501,7 @@ struct IndiceConv : torch::autograd::Function<IndiceConv> {
     ctx->saved_data["share_row_maps"] = share_row_maps;
     ctx->saved_data["guarded"] = guarded;
     StreamHandle &h = streamHandle();
-    const std::lock_guard<std::mutex> lock(h.mutex);
+    const OperatorLock lock(h);
     check(api.mluOpExtSetDistinctPairsPromise(h.handle, rb->distinct), "mluOpExtSetDistinctPairsPromise");
     const Buffers buffers(guarded, x.device());
     const void *map = share_row_maps ? rb->rowMap(h, buffers, inverse ? 0 : 1) : nullptr;
@@ -491,7 +523,7 @@ struct IndiceConv : torch::autograd::Function<IndiceConv> {
     if (!grads[0].defined()) return out;
     const at::Tensor dy = grads[0].contiguous();
     StreamHandle &h = streamHandle();
-    const std::lock_guard<std::mutex> lock(h.mutex);
+    const OperatorLock lock(h);
     check(api.mluOpExtSetDistinctPairsPromise(h.handle, rb->distinct), "mluOpExtSetDistinctPairsPromise");
     const Buffers buffers(ctx->saved_data["guarded"].toBool(), x.device());
     const bool sub_m = !inverse && rb->sub_m;
@@ -548,7 +580,7 @@ std::vector<at::Tensor> voxelization(mluOpHandle_t handle, const Buffers &buffer
 std::vector<at::Tensor> voxelizationCut(bool guarded, const at::Tensor &points, const at::Tensor &voxel_size,
                                         const at::Tensor &coors_range, int64_t max_points, int64_t max_voxels) {
   StreamHandle &h = streamHandle();
-  const std::lock_guard<std::mutex> lock(h.mutex);
+  const OperatorLock lock(h);
   std::vector<at::Tensor> r = voxelization(h.handle, Buffers(guarded, points.device()), points, voxel_size,
                                            coors_range, max_points, max_voxels, true);
   int32_t found = 0;
@@ -647,6 +679,7 @@ PYBIND11_MODULE(_native, m) {
           Rulebook3 r;
           {
             NoGil released;
+            const OperatorLock lock(asHandle(handle));
             r = indicePairs(asHandle(handle), Buffers(guarded, indices.device()), indices, batch, input_space,
                             filter_space, output_space, pad, stride, dilation, sub_m, out_rows, std::move(out_indices),
                             for_layer);
@@ -659,6 +692,7 @@ PYBIND11_MODULE(_native, m) {
            const at::Tensor &pairs, const Counts &counts, int64_t num_act_out, bool sub_m, int64_t inverse,
            uintptr_t row_map) {
           NoGil released;
+          const OperatorLock lock(asHandle(handle));
           return convForward(asHandle(handle), Buffers(guarded, features.device()), features, filters,
                              static_cast<mluOpTensorLayout_t>(layout), pairs, counts, num_act_out, sub_m, inverse,
                              reinterpret_cast<const void *>(row_map));
@@ -668,6 +702,7 @@ PYBIND11_MODULE(_native, m) {
            const at::Tensor &pairs, const Counts &counts, bool sub_m, int64_t ci, int64_t inverse, int64_t rows,
            uintptr_t row_map) {
           NoGil released;
+          const OperatorLock lock(asHandle(handle));
           return convBackwardData(asHandle(handle), Buffers(guarded, output_grad.device()), output_grad, filters,
                                   static_cast<mluOpTensorLayout_t>(layout), pairs, counts, sub_m, ci, inverse, rows,
                                   reinterpret_cast<const void *>(row_map));
@@ -677,6 +712,7 @@ PYBIND11_MODULE(_native, m) {
            const at::Tensor &pairs, const Counts &counts, const Counts &filter_space, bool sub_m, int64_t inverse,
            bool onchip_float, int layout) {
           NoGil released;
+          const OperatorLock lock(asHandle(handle));
           return convBackwardFilter(asHandle(handle), Buffers(guarded, features.device()), features, output_grad,
                                     pairs, counts, filter_space, sub_m, inverse, onchip_float,
                                     static_cast<mluOpTensorLayout_t>(layout));
@@ -685,6 +721,7 @@ PYBIND11_MODULE(_native, m) {
         [](uintptr_t handle, bool guarded, const at::Tensor &points, const at::Tensor &voxel_size,
            const at::Tensor &coors_range, int64_t max_points, int64_t max_voxels, bool deterministic) {
           NoGil released;
+          const OperatorLock lock(asHandle(handle));
           return voxelization(asHandle(handle), Buffers(guarded, points.device()), points, voxel_size, coors_range,
                               max_points, max_voxels, deterministic);
         });
@@ -701,6 +738,7 @@ PYBIND11_MODULE(_native, m) {
   m.def("dynamic_point_to_voxel_forward",
         [](uintptr_t handle, bool guarded, const at::Tensor &feats, const at::Tensor &coors, int mode, int64_t rows) {
           NoGil released;
+          const OperatorLock lock(asHandle(handle));
           return scatterForward(asHandle(handle), Buffers(guarded, feats.device()), feats, coors,
                                 static_cast<mluOpReduceMode_t>(mode), rows);
         });
@@ -709,6 +747,7 @@ PYBIND11_MODULE(_native, m) {
            const at::Tensor &voxel_feats, const at::Tensor &p2v, const at::Tensor &count, const at::Tensor &num,
            int mode) {
           NoGil released;
+          const OperatorLock lock(asHandle(handle));
           return scatterBackward(asHandle(handle), Buffers(guarded, feats.device()), grad, feats, voxel_feats, p2v,
                                  count, num, static_cast<mluOpReduceMode_t>(mode));
         });
