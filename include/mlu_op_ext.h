@@ -88,17 +88,21 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtSetDistinctPairsPromise(mluOpHandle_t handle
  * array, so a caller has to bring the counts mluOpGetIndicePairs left in device memory over; a copy
  * waits for the whole queue.  The last kernel of a rulebook also stores them into pinned memory of
  * the handle: this call waits for them there and fills indice_num[0 .. kernel_volume).  For the last
- * 32 rulebooks of the handle; NOT_SUPPORTED for a pair tensor it did not build, that was built under
- * graph capture or has more than 343 offsets (copy the counts then).  No counterpart in the
- * reference. */
+ * 32 rulebooks of the handle.  `indice_pairs` names a rulebook by its address: the answer is for the
+ * one this handle last built there.  NOT_SUPPORTED if it built none with so many offsets there, built
+ * it under graph capture or with more than 343 offsets, or if an operator of this handle has written
+ * into the tensor since (copy the counts then).  What others write there, or that the memory was
+ * freed and given out again, the handle cannot see: ask while the tensor is the rulebook, as for the
+ * operators that take both.  No counterpart in the reference. */
 mluOpStatus_t MLUOP_WIN_API mluOpExtGetIndicePairsHostCounts(mluOpHandle_t handle, const void *indice_pairs,
                                                              int kernel_volume, int64_t indice_num[]);
 
 /* The number of voxels of the handle's last mluOpVoxelization on the host.  Its last kernel stores the
  * number into pinned memory of the handle while it writes the voxels: this call waits for it there,
- * where a copy of voxel_num waits for the whole queue.  NOT_SUPPORTED if `voxel_num` is not what the
- * last call wrote, or that call was captured into a graph (copy the number then).  No counterpart in
- * the reference. */
+ * where a copy of voxel_num waits for the whole queue.  NOT_SUPPORTED if `voxel_num` is not the address
+ * that call was given, an operator of this handle has written there since, or the call was captured
+ * into a graph (copy the number then).  The answer is what that call found, whatever others have
+ * written to the address since.  No counterpart in the reference. */
 mluOpStatus_t MLUOP_WIN_API mluOpExtGetVoxelizationHostCount(mluOpHandle_t handle, const void *voxel_num,
                                                              int32_t *count);
 

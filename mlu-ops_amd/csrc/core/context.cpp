@@ -258,6 +258,17 @@ const char *MLUOP_WIN_API mluOpGetErrorString(mluOpStatus_t status) {
 
 }  // extern "C"
 
+void mluOpContext::forgetNotesIn(const void *out, size_t bytes) {
+  const uintptr_t lo = reinterpret_cast<uintptr_t>(out), hi = lo + bytes;
+  auto meets = [&](const void *at, size_t size) {
+    const uintptr_t p = reinterpret_cast<uintptr_t>(at);
+    return at != nullptr && p < hi && lo < p + size;
+  };
+  for (RulebookNote &n : rulebook_notes)
+    if (meets(n.pairs, (size_t)n.K * 2 * (size_t)n.L * sizeof(int32_t))) n.pairs = nullptr;
+  if (meets(voxel_count.voxel_num, sizeof(int32_t))) voxel_count.voxel_num = nullptr;
+}
+
 namespace mluop {
 
 hipError_t waitForWord(hipStream_t queue, const unsigned long long *word, unsigned long long stamp,

@@ -84,6 +84,10 @@ struct mluOpContext {
   } voxel_count;
   unsigned long long next_stamp = 1;   // also the source of per-call tickets
 
+  // An operator of this handle is about to write [out, out + bytes): what was noted about a pair
+  // tensor or a number of voxels in there describes memory that was handed out again, and is dropped.
+  void forgetNotesIn(const void *out, size_t bytes);
+
   // What the kernel launchers need: the stream, and the timer while it is on.
   mluop::KernelChoices kernel_choices;
   mluop::LaunchCtx launchCtx() {

@@ -145,6 +145,8 @@ mluOpStatus_t MLUOP_WIN_API mluOpDynamicPointToVoxelBackward(
   if (need > 0) {
     PARAM_CHECK(api, workspace != NULL);
   }
+  handle->forgetNotesIn(grad_feats, grad_feats_desc->total_tensor_size);
+  handle->forgetNotesIn(workspace, workspace_size);
   HIP_CHECK_RETURN(api, mluop::dynamic_point_to_voxel::launchScatterPointsBackward(
                             handle->launchCtx(), n, c, rows,
                             static_cast<const float *>(grad_voxel_feats),

@@ -293,8 +293,8 @@ mluOpStatus_t MLUOP_WIN_API mluOpIndiceConvolutionBackwardFilter(
     c.finish(0.003);
   }
   DEVICE_HANDLE_CHECK(api, handle);
-  mluop::sparse_conv::forgetRulebookNotesIn(handle, filters_grad, filters_grad_desc->total_tensor_size);
-  mluop::sparse_conv::forgetRulebookNotesIn(handle, workspace, workspace_size);
+  handle->forgetNotesIn(filters_grad, filters_grad_desc->total_tensor_size);
+  handle->forgetNotesIn(workspace, workspace_size);
   HIP_CHECK_RETURN(api, mluop::sparse_conv::launchBackwardFilter(handle->launchCtx(), p, features,
                                                                 output_grad, workspace,
                                                                 filters_grad));
@@ -348,6 +348,7 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtIndiceConvolutionBackwardFilterNoAlloc(
                      << " was not found when the handle was created.";
     return MLUOP_STATUS_NOT_INITIALIZED;
   }
+  handle->forgetNotesIn(filters_grad, filters_grad_desc->total_tensor_size);
   // the handle's kernel choices, but no event pairs: the per-kernel timer creates events on demand
   const mluop::LaunchCtx lc(handle->queue, nullptr, &handle->kernel_choices);
   HIP_CHECK_RETURN(api, mluop::sparse_conv::launchBackwardFilter(lc, p, features, output_grad,

@@ -87,6 +87,7 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtBuildRowMap(mluOpHandle_t handle,
   }
   DEVICE_HANDLE_CHECK(api, handle);
 
+  handle->forgetNotesIn(row_map, size);
   // forget what this buffer held before
   auto &maps = handle->row_maps;
   for (size_t i = 0; i < maps.size();) {

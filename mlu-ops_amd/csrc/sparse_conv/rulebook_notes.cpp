@@ -6,9 +6,8 @@ namespace mluop {
 namespace sparse_conv {
 
 RulebookReportTarget openRulebookNote(mluOpContext *handle, const void *pairs, int K, int L) {
-  // an older note about the same address describes a tensor that is being overwritten
-  for (auto &n : handle->rulebook_notes)
-    if (n.pairs == pairs) n.pairs = nullptr;
+  // older notes about this memory describe tensors that are being overwritten
+  handle->forgetNotesIn(pairs, (size_t)K * 2 * (size_t)L * sizeof(int32_t));
   const int slot = handle->next_rulebook_note;
   handle->next_rulebook_note = (slot + 1) % mluOpContext::kRulebookNotes;
   mluOpContext::RulebookNote &note = handle->rulebook_notes[slot];
@@ -71,14 +70,6 @@ void consultRulebookNotes(mluOpContext *handle, int row_column, ConvProblem *p) 
     }
     p->list_trust = (uint32_t)report != 0 ? ListTrust::kInOrder : ListTrust::kNone;
     return;
-  }
-}
-
-void forgetRulebookNotesIn(mluOpContext *handle, const void *out, size_t bytes) {
-  const char *lo = static_cast<const char *>(out);
-  for (auto &n : handle->rulebook_notes) {
-    const char *at = static_cast<const char *>(n.pairs);
-    if (at != nullptr && at >= lo && at < lo + bytes) n.pairs = nullptr;
   }
 }
 
