@@ -23,7 +23,7 @@
 //
 // What bounds it: rows of features read and written at random places (dpvReduce moves 100 MB in 32 us
 // at 400 k points of 32 features), and launches that each start cold, the sort's nine most of all.
-// Measured there: 105 us forward, 70 us backward; 165 and 88 us with four passes of 8 bits, separate
+// Measured there: 105 us forward, 72 us backward; 165 and 88 us with four passes of 8 bits, separate
 // fills, one feature a thread and atomic minima.
 #include <hip/hip_runtime.h>
 
@@ -263,44 +263,115 @@ __global__ __launch_bounds__(kBlock) void dpvReduce(const float *__restrict__ fe
 
 // ---- backward of the max reduction ----
 //
-// The gradient of (voxel, feature) goes to the lowest point whose feature equals the maximum.  The
-// points of every voxel are listed first (in any order, with an integer atomic a point); then the
-// threads of a voxel go through its points once, reading and writing every row once.
-// (An atomic minimum for every feature of every point, over an array that is filled first and read
-// once more behind, takes 88 us at 400 k points of 32 features; it needs no lists, and stays for
-// workspaces too small for them.)
+// The gradient of (voxel, feature) goes to the lowest point whose feature equals the maximum.
+// Rows of many features: the points of every voxel are listed first, in any order; then the threads
+// of a voxel go through its points once, reading and writing every row once.  A voxel of more than
+// kListed points has no list, and no thread walks it: its points look for themselves, with an
+// atomic minimum for every feature that equals the maximum, and write their rows in a launch of
+// their own, which finds nothing to do where there is no such voxel.  Where voxels have more points
+// than that on average nothing is listed at all.
+// Rows of few features: the atomic minimum for every point (see below), which needs no lists.
 
 __device__ inline bool inVoxel(int v, const int32_t *voxel_num, int rows) { return v >= 0 && v < min(*voxel_num, rows); }
 
-__global__ __launch_bounds__(kBlock) void dpvBackwardClearCounts(uint32_t *counts, int rows, uint32_t *listed) {
+constexpr uint32_t kListed = 32;              // points of a voxel that has a list
+constexpr uint32_t kUnlisted = 0x80000000u;   // starts[v]: this and the number of the voxel among those without one
+
+// So few voxels that each can go without a list (`unlisted_most` of them can).
+__device__ inline bool nothingListed(int voxels, uint32_t unlisted_most) { return voxels <= (int)unlisted_most; }
+
+// What the launches hand on beside the arrays, in device memory.
+struct ListTotals {
+  uint32_t listed;    // points in lists
+  uint32_t unlisted;  // voxels without one
+};
+
+__global__ __launch_bounds__(kBlock) void dpvBackwardClearCounts(uint32_t *counts, int rows, ListTotals *totals) {
   const int v = blockIdx.x * kBlock + threadIdx.x;
   if (v < rows) counts[v] = 0;
-  if (v == 0) *listed = 0;
+  if (v == 0) *totals = ListTotals{0, 0};
 }
 
-__global__ __launch_bounds__(kBlock) void dpvBackwardCount(const int32_t *__restrict__ point2voxel_map,
-                                                           const int32_t *__restrict__ voxel_num, int n, int rows,
-                                                           uint32_t *counts, uint32_t *__restrict__ arrival) {
-  const int x = blockIdx.x * kBlock + threadIdx.x;
-  if (x >= n) return;
-  const int v = point2voxel_map[x];
-  if (inVoxel(v, voxel_num, rows)) arrival[x] = atomicAdd(&counts[v], 1u);
+// counts[v] = points of voxel v, arrival[x] = points of its voxel counted before point x.  The points
+// of a workgroup are counted in LDS first, so that a voxel costs one atomic a workgroup however many
+// of its points are there (atomics on one word take 11 ns each).
+constexpr int kCountThreads = 512;
+constexpr int kCountPer = 4;
+constexpr int kCountSlots = 2 * kCountThreads * kCountPer;
+__global__ __launch_bounds__(kCountThreads) void dpvBackwardCount(const int32_t *__restrict__ point2voxel_map,
+                                                                  const int32_t *__restrict__ voxel_num, int n,
+                                                                  int rows, uint32_t unlisted_most, uint32_t *counts,
+                                                                  uint32_t *__restrict__ arrival) {
+  __shared__ uint32_t s_voxel[kCountSlots], s_count[kCountSlots];
+  constexpr uint32_t kEmpty = 0xffffffffu;
+  const int tid = threadIdx.x;
+  const int first = blockIdx.x * (kCountThreads * kCountPer) + tid;
+  const int voxels = min(*voxel_num, rows);
+  if (nothingListed(voxels, unlisted_most)) return;
+  int v[kCountPer];
+#pragma unroll
+  for (int u = 0; u < kCountPer; ++u) {
+    const int x = first + u * kCountThreads;
+    v[u] = x < n ? point2voxel_map[x] : -1;
+  }
+  for (int s = tid; s < kCountSlots; s += kCountThreads) {
+    s_voxel[s] = kEmpty;
+    s_count[s] = 0;
+  }
+  __syncthreads();
+  uint32_t slot[kCountPer], before[kCountPer];
+#pragma unroll
+  for (int u = 0; u < kCountPer; ++u) {
+    if (v[u] >= voxels) v[u] = -1;
+    if (v[u] < 0) continue;
+    uint32_t at = ((uint32_t)v[u] * 0x9e3779b1u) / (0xffffffffu / kCountSlots + 1);
+    // (twice as many slots as points: an empty one is always reached)
+    while (true) {
+      const uint32_t seen = atomicCAS(&s_voxel[at], kEmpty, (uint32_t)v[u]);
+      if (seen == kEmpty || seen == (uint32_t)v[u]) break;
+      at = (at + 1) & (kCountSlots - 1);
+    }
+    slot[u] = at;
+    before[u] = atomicAdd(&s_count[at], 1u);
+  }
+  __syncthreads();
+  for (int s = tid; s < kCountSlots; s += kCountThreads)
+    if (s_voxel[s] != kEmpty) s_count[s] = atomicAdd(&counts[s_voxel[s]], s_count[s]);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kCountPer; ++u)
+    if (v[u] >= 0) arrival[first + u * kCountThreads] = s_count[slot[u]] + before[u];
 }
 
 // starts[v] = where the list of voxel v starts (the lists lie in no particular order: one atomic a
-// workgroup hands out the space, 8 ns each since they all go to one word).
+// workgroup hands out the space, 8 ns each since they all go to one word), or its number among the
+// voxels without one.
 constexpr int kPlaceThreads = 1024;
 constexpr int kPlacePer = 4;
-__global__ __launch_bounds__(kPlaceThreads) void dpvBackwardPlaces(const uint32_t *__restrict__ counts, int rows,
-                                                                   uint32_t *listed, uint32_t *__restrict__ starts) {
+__global__ __launch_bounds__(kPlaceThreads) void dpvBackwardPlaces(const uint32_t *__restrict__ counts,
+                                                                   const int32_t *__restrict__ voxel_num, int rows,
+                                                                   uint32_t unlisted_most, ListTotals *totals,
+                                                                   uint32_t *__restrict__ starts) {
+  // a workgroup's points in lists, and above them its voxels without one
+  constexpr int kShift = 18;
+  static_assert(kPlaceThreads * kPlacePer * kListed < 1u << kShift && kPlaceThreads * kPlacePer < 1 << (32 - kShift),
+                "both sums in one word");
   __shared__ uint32_t s_wave[kPlaceThreads / 64];
-  __shared__ uint32_t s_base;
+  __shared__ uint32_t s_listed, s_unlisted;
   const int tid = threadIdx.x, wave = tid >> 6;
   const int first = (blockIdx.x * kPlaceThreads + tid) * kPlacePer;
+  const int voxels = min(*voxel_num, rows);
+  if (nothingListed(voxels, unlisted_most)) {
+    for (int u = 0; u < kPlacePer; ++u)
+      if (first + u < rows) starts[first + u] = kUnlisted | (uint32_t)(first + u);
+    if (first == 0) totals->unlisted = (uint32_t)max(voxels, 0);
+    return;
+  }
   uint32_t c[kPlacePer], sum = 0;
 #pragma unroll
   for (int u = 0; u < kPlacePer; ++u) {
     c[u] = first + u < rows ? counts[first + u] : 0u;
+    if (c[u] > kListed) c[u] = 1u << kShift;
     sum += c[u];
   }
   const uint32_t incl = device_sort::waveInclusiveSum(sum);
@@ -309,37 +380,55 @@ __global__ __launch_bounds__(kPlaceThreads) void dpvBackwardPlaces(const uint32_
   if (tid == 0) {
     uint32_t all = 0;
     for (int w = 0; w < kPlaceThreads / 64; ++w) all += s_wave[w];
-    s_base = all == 0 ? 0u : atomicAdd(listed, all);
+    const uint32_t listed = all & ((1u << kShift) - 1u), unlisted = all >> kShift;
+    s_listed = listed == 0 ? 0u : atomicAdd(&totals->listed, listed);
+    s_unlisted = unlisted == 0 ? 0u : atomicAdd(&totals->unlisted, unlisted);
   }
   __syncthreads();
-  uint32_t at = s_base + incl - sum;
-  for (int w = 0; w < wave; ++w) at += s_wave[w];
+  uint32_t in_front = incl - sum;
+  for (int w = 0; w < wave; ++w) in_front += s_wave[w];
 #pragma unroll
   for (int u = 0; u < kPlacePer; ++u) {
-    if (first + u < rows) starts[first + u] = at;
-    at += c[u];
+    if (first + u < rows)
+      starts[first + u] = c[u] >> kShift != 0 ? kUnlisted | (s_unlisted + (in_front >> kShift))
+                                              : s_listed + (in_front & ((1u << kShift) - 1u));
+    in_front += c[u];
   }
 }
 
+// The first `list_blocks` workgroups write the lists, the others from[voxel without a list, feature] = n.
 __global__ __launch_bounds__(kBlock) void dpvBackwardList(const int32_t *__restrict__ point2voxel_map,
                                                           const int32_t *__restrict__ voxel_num, int n, int rows,
+                                                          int num_features, int list_blocks,
                                                           const uint32_t *__restrict__ starts,
                                                           const uint32_t *__restrict__ arrival,
-                                                          uint32_t *__restrict__ points) {
+                                                          uint32_t *__restrict__ points,
+                                                          const ListTotals *__restrict__ totals,
+                                                          int32_t *__restrict__ from) {
+  if ((int)blockIdx.x >= list_blocks) {
+    const size_t words = (size_t)totals->unlisted * num_features;
+    for (size_t i = (size_t)(blockIdx.x - list_blocks) * kBlock + threadIdx.x; i < words;
+         i += (size_t)(gridDim.x - list_blocks) * kBlock)
+      from[i] = n;
+    return;
+  }
   const int x = blockIdx.x * kBlock + threadIdx.x;
   if (x >= n) return;
   const int v = point2voxel_map[x];
-  if (inVoxel(v, voxel_num, rows)) points[starts[v] + arrival[x]] = (uint32_t)x;
+  if (!inVoxel(v, voxel_num, rows)) return;
+  const uint32_t start = starts[v];
+  if ((start & kUnlisted) == 0) points[start + arrival[x]] = (uint32_t)x;
 }
 
-// Thread t takes VEC features of voxel t / (C / VEC), and of the point of that number if it is in no
-// voxel.  Up to four points of a voxel are held at once and their rows written whole.
+// Thread t takes VEC features of the listed voxel t / (C / VEC), and of the point of that number if it
+// is in no voxel or in one without a list.  Up to four points of a voxel are held at once and their
+// rows written whole.
 template <int VEC>
 __global__ __launch_bounds__(kBlock) void dpvBackwardVoxels(
     const float *__restrict__ grad_voxel_feats, const float *__restrict__ feats,
     const float *__restrict__ voxel_feats, const int32_t *__restrict__ point2voxel_map,
     const int32_t *__restrict__ voxel_num, int n, int num_features, int rows, const uint32_t *__restrict__ counts,
-    const uint32_t *__restrict__ starts, const uint32_t *__restrict__ points, float *grad_feats) {
+    const uint32_t *__restrict__ starts, const uint32_t *__restrict__ points, int32_t *from, float *grad_feats) {
   typedef Floats<VEC> F;
   constexpr int kHeld = 4;
   const uint32_t lanes = (uint32_t)num_features / VEC;
@@ -350,11 +439,20 @@ __global__ __launch_bounds__(kBlock) void dpvBackwardVoxels(
   F zero;
 #pragma unroll
   for (int k = 0; k < VEC; ++k) zero.x[k] = 0.f;
-  if (!inVoxel(point2voxel_map[v], voxel_num, rows))
+  const int own = point2voxel_map[v];
+  if (!inVoxel(own, voxel_num, rows)) {
     *reinterpret_cast<F *>(grad_feats + (size_t)v * num_features + c) = zero;
+  } else if (const uint32_t place = starts[own]; (place & kUnlisted) != 0) {
+    const F mine = *reinterpret_cast<const F *>(feats + (size_t)v * num_features + c);
+    const F top = *reinterpret_cast<const F *>(voxel_feats + (size_t)own * num_features + c);
+    int32_t *const best = from + (size_t)(place & ~kUnlisted) * num_features + c;
+#pragma unroll
+    for (int k = 0; k < VEC; ++k)
+      if (mine.x[k] == top.x[k]) atomicMin(best + k, (int32_t)v);
+  }
   if (v >= (uint32_t)min(*voxel_num, rows)) return;
   const uint32_t count = counts[v];
-  if (count == 0) return;
+  if (count == 0 || count > kListed) return;
   const uint32_t begin = starts[v], stop = begin + count;
   const F top = *reinterpret_cast<const F *>(voxel_feats + (size_t)v * num_features + c);
   const F g = *reinterpret_cast<const F *>(grad_voxel_feats + (size_t)v * num_features + c);
@@ -390,6 +488,31 @@ __global__ __launch_bounds__(kBlock) void dpvBackwardVoxels(
 #pragma unroll
     for (int k = 0; k < VEC; ++k)
       if (best[k] < (uint32_t)n) grad_feats[(size_t)best[k] * num_features + c + k] = g.x[k];
+  }
+}
+
+// The rows of the points of voxels without a list.
+template <int VEC>
+__global__ __launch_bounds__(kBlock) void dpvBackwardUnlisted(
+    const float *__restrict__ grad_voxel_feats, const int32_t *__restrict__ point2voxel_map,
+    const int32_t *__restrict__ voxel_num, int n, int num_features, int rows, const uint32_t *__restrict__ starts,
+    const ListTotals *__restrict__ totals, const int32_t *__restrict__ from, float *__restrict__ grad_feats) {
+  typedef Floats<VEC> F;
+  if (totals->unlisted == 0) return;
+  const uint32_t lanes = (uint32_t)num_features / VEC, all = (uint32_t)n * lanes;
+  for (uint32_t t = blockIdx.x * kBlock + threadIdx.x; t < all; t += gridDim.x * kBlock) {
+    const uint32_t x = t / lanes;
+    const int c = (int)(t - x * lanes) * VEC;
+    const int v = point2voxel_map[x];
+    if (!inVoxel(v, voxel_num, rows)) continue;
+    const uint32_t place = starts[v];
+    if ((place & kUnlisted) == 0) continue;
+    const int32_t *const best = from + (size_t)(place & ~kUnlisted) * num_features + c;
+    const F g = *reinterpret_cast<const F *>(grad_voxel_feats + (size_t)v * num_features + c);
+    F out;
+#pragma unroll
+    for (int k = 0; k < VEC; ++k) out.x[k] = best[k] == (int32_t)x ? g.x[k] : 0.f;
+    *reinterpret_cast<F *>(grad_feats + (size_t)x * num_features + c) = out;
   }
 }
 
@@ -435,6 +558,14 @@ int featureLanes(int num_features, std::initializer_list<const void *> tensors) 
   if (num_features % 2 == 0 && low % 8 == 0) return 2;
   return 1;
 }
+
+// From this many features in all and a point on the backward pass lists points.  A list costs the same
+// for a point of any number of features, an atomic minimum a feature: at 400 k points lists take 65 us
+// against 72 to 81 with 32 features and 94 against 164 to 190 with 64 (the larger figures with a voxel
+// row for every point), and no less than the minima with 24 (60) and 16 (52 against 39); at 50 k
+// points, where launches count, 26 against 14 with 32 features and 32 against 22 with 64.
+constexpr int kFeaturesForLists = 32;
+constexpr size_t kAllFeaturesForLists = 8000000;
 
 struct Workspace {
   u64 *keys_a, *keys_b;
@@ -590,26 +721,41 @@ hipError_t launchScatterPointsBackward(const LaunchCtx &lc, int num_points, int 
                                        void *workspace, size_t workspace_bytes, float *grad_feats) {
   const int n = num_points, rows = voxel_rows;
   hipError_t e = hipSuccess;
-  if (workspace_bytes >= 4 * ((size_t)2 * rows + n)) {
+  // [counts, starts: a row each][points][totals][from: a row for every voxel without a list]
+  const size_t unlisted_most = (size_t)n / (kListed + 1);
+  const size_t list_words = 2 * (size_t)rows + n + sizeof(ListTotals) / 4 + unlisted_most * num_features;
+  if (num_features >= kFeaturesForLists && (size_t)n * num_features >= kAllFeaturesForLists &&
+      workspace_bytes >= 4 * list_words) {
     uint32_t *counts = static_cast<uint32_t *>(workspace), *starts = counts + rows, *points = starts + rows;
-    // (free words: the first of the lists until they are written, the gradients until the last kernel)
-    uint32_t *listed = points, *arrival = reinterpret_cast<uint32_t *>(grad_feats);
+    ListTotals *totals = reinterpret_cast<ListTotals *>(points + n);
+    int32_t *from = reinterpret_cast<int32_t *>(totals + 1);
+    // (free words: the gradients until the last kernels)
+    uint32_t *arrival = reinterpret_cast<uint32_t *>(grad_feats);
+    const int list_blocks = gridFor((size_t)n);
     lc.begin("dpvBackwardLists");
-    dpvBackwardClearCounts<<<gridFor((size_t)rows), kBlock, 0, lc.stream>>>(counts, rows, listed);
-    dpvBackwardCount<<<gridFor((size_t)n), kBlock, 0, lc.stream>>>(point2voxel_map, voxel_num, n, rows, counts,
-                                                                   arrival);
-    dpvBackwardPlaces<<<rows / (kPlaceThreads * kPlacePer) + 1, kPlaceThreads, 0, lc.stream>>>(counts, rows, listed,
-                                                                                               starts);
-    dpvBackwardList<<<gridFor((size_t)n), kBlock, 0, lc.stream>>>(point2voxel_map, voxel_num, n, rows, starts, arrival,
-                                                                  points);
+    dpvBackwardClearCounts<<<gridFor((size_t)rows), kBlock, 0, lc.stream>>>(counts, rows, totals);
+    dpvBackwardCount<<<(n + kCountThreads * kCountPer - 1) / (kCountThreads * kCountPer), kCountThreads, 0,
+                       lc.stream>>>(point2voxel_map, voxel_num, n, rows, (uint32_t)unlisted_most, counts, arrival);
+    dpvBackwardPlaces<<<rows / (kPlaceThreads * kPlacePer) + 1, kPlaceThreads, 0, lc.stream>>>(
+        counts, voxel_num, rows, (uint32_t)unlisted_most, totals, starts);
+    dpvBackwardList<<<list_blocks + gridFor(unlisted_most * num_features, 256), kBlock, 0, lc.stream>>>(
+        point2voxel_map, voxel_num, n, rows, num_features, list_blocks, starts, arrival, points, totals, from);
     lc.end();
     if ((e = hipGetLastError()) != hipSuccess) return e;
     const int vec = featureLanes(num_features, {feats, voxel_feats, grad_voxel_feats, grad_feats});
+    const size_t threads = (size_t)n * (num_features / vec);
     auto voxels = vec == 4 ? dpvBackwardVoxels<4> : vec == 2 ? dpvBackwardVoxels<2> : dpvBackwardVoxels<1>;
     lc.begin("dpvBackwardVoxels");
-    voxels<<<gridFor((size_t)n * (num_features / vec)), kBlock, 0, lc.stream>>>(
-        grad_voxel_feats, feats, voxel_feats, point2voxel_map, voxel_num, n, num_features, rows, counts, starts, points,
-        grad_feats);
+    voxels<<<gridFor(threads), kBlock, 0, lc.stream>>>(grad_voxel_feats, feats, voxel_feats, point2voxel_map,
+                                                       voxel_num, n, num_features, rows, counts, starts, points, from,
+                                                       grad_feats);
+    lc.end();
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    if (unlisted_most == 0) return hipSuccess;
+    auto unlisted = vec == 4 ? dpvBackwardUnlisted<4> : vec == 2 ? dpvBackwardUnlisted<2> : dpvBackwardUnlisted<1>;
+    lc.begin("dpvBackwardUnlisted");
+    unlisted<<<gridFor(threads, 2048), kBlock, 0, lc.stream>>>(grad_voxel_feats, point2voxel_map, voxel_num, n,
+                                                               num_features, rows, starts, totals, from, grad_feats);
     lc.end();
     return hipGetLastError();
   }

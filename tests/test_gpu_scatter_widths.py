@@ -29,3 +29,50 @@ def test_forward_and_backward(gpu_handle, c, n, span):
         torch.cuda.synchronize()
         want = dpv.backward(g[:rows], feats, vf.cpu().numpy(), p2v.cpu().numpy(), int(num.item()))
         assert np.array_equal(grad.cpu().numpy(), want), rows
+
+
+def crowded(rng, n, crowds):
+    """Coordinates of n points: a voxel of each size in `crowds`, the rest in voxels of a few points."""
+    cell = np.repeat(np.arange(len(crowds)), crowds)[:n]
+    cell = np.concatenate([cell, rng.integers(1000, 1000 + n, n - cell.size)])
+    cell[rng.random(n) < 0.02] = -1
+    rng.shuffle(cell)
+    return np.where(cell[:, None] < 0, -1, np.stack([cell // 10000, cell // 100 % 100, cell % 100], 1)).astype(np.int32)
+
+
+def check_backward(gpu_handle, rng, feats, coors):
+    import torch
+    import mluop_hip
+    g = rng.standard_normal(feats.shape).astype(np.float32)
+    tf, tc = torch.from_numpy(feats).cuda(), torch.from_numpy(coors).cuda()
+    vf, vc, p2v, cnt, num = mluop_hip.dynamic_point_to_voxel_forward(gpu_handle, tf, tc.clone(), "max")
+    grad = mluop_hip.dynamic_point_to_voxel_backward(gpu_handle, torch.from_numpy(g).cuda(), tf, vf, p2v, cnt, num)
+    torch.cuda.synchronize()
+    assert np.array_equal(grad.cpu().numpy(), dpv.backward(g, feats, vf.cpu().numpy(), p2v.cpu().numpy(), int(num.item())))
+
+
+@pytest.mark.parametrize("c", [3, 32, 65])
+@pytest.mark.parametrize("n,crowds", [(33, [33]), (2049, [2049]), (6000, [3000]), (20000, [12000, 33, 32])])
+def test_backward_with_crowded_voxels(gpu_handle, c, n, crowds):
+    rng = np.random.default_rng(c + n)
+    coors = crowded(rng, n, crowds)
+    for feats in (rng.standard_normal((n, c)).astype(np.float32), np.zeros((n, c), np.float32)):
+        feats[rng.random(n) < 0.01] = np.nan
+        check_backward(gpu_handle, rng, feats, coors)
+
+
+@pytest.mark.parametrize("c,n,crowds", [
+    (32, 250_000, [33, 32, 31, 34, 1, 2, 4, 5, 100_000]),     # lists beside one voxel without, and around the limit
+    (33, 245_000, [40] * 3000),                               # one feature a thread; most points without a list
+    (34, 240_000, [31] * 3000),                               # two; most in long lists
+    (64, 125_001, []),                                        # short lists only
+    (128, 62_500, [62_500]),                                  # so few voxels that nothing is listed
+    (32, 250_000, [250] * 900),
+])
+def test_backward_of_many_wide_features(gpu_handle, c, n, crowds):
+    """Sizes at which the points are listed: voxels on both sides of the longest list."""
+    rng = np.random.default_rng(c + n)
+    coors = crowded(rng, n, crowds)
+    feats = rng.integers(-8, 9, (n, c)).astype(np.float32)   # ties in every longer list
+    feats[rng.random(n) < 0.01] = np.nan
+    check_backward(gpu_handle, rng, feats, coors)
