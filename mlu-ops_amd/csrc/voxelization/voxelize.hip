@@ -23,9 +23,11 @@
 // What bounds it: random access.  A cell table in device memory costs a 128-byte line each way for
 // every point (58 us for 1.2 M points), a full sort by cell another 70 us in nine launches.  With the
 // buckets only the partition's stores and the ranks' way back to point order are scattered, and
-// every other pass streams.
-// Measured, 1.2 M points in 2048 buckets: 77 us for the six launches (12, 5, 22, 21, 7, 9), 200 us with
-// cell table and sort; 23 k points: 33 us against 68 us, where launches and latency count.
+// every other pass streams.  One crowded cell (zero-padded clouds) is one workgroup's work: 1.3 us for
+// every 512 of its points, a table lookup each.
+// Measured, 1.2 M points in 2048 buckets: 75 us for the six launches (13, 7, 24, 25, 6, 11), 198 us with
+// cell table and sort; 23 k points: 29 us against 72 us, where launches and latency count; 4 M points
+// 182 against 552 us, 8 M 359 against 1111; 120 k points, half of them in one cell, 175 against 753.
 #include <hip/hip_runtime.h>
 
 #include "core/device_sort.h"
@@ -55,8 +57,8 @@ using device_sort::kNoDigit;
 using device_sort::kRound;
 using device_sort::kTileThreads;
 
-// Buckets of about 500 points: a bucket is one workgroup's work and half of its LDS table, while a
-// small cloud still gives many workgroups something to do.
+// Buckets of about 500 points: a bucket is one workgroup's work, while a small cloud still gives many
+// workgroups something to do.  From 1.2 million points on the buckets grow.
 int bucketsFor(int64_t n) {
   int b = 64;
   while (b < kMaxDigits && (int64_t)b * 600 < n) b <<= 1;
@@ -186,72 +188,83 @@ struct BucketedPoints {
 
 // ---- ranks inside the cells of a bucket --------------------------------------------------
 
-constexpr int kRankThreads = 512;
-constexpr int kRankWaves = kRankThreads / 64;
-constexpr int kLdsSlots = 2048;  // an LDS table serves a bucket of up to half as many points
 constexpr uint32_t kIsFirst = 0x80000000u;
 
-// Cells of a bucket in LDS (32-bit keys).
+// Cells of a bucket in LDS (32-bit keys).  FILLS: the bucket has more points than the table has
+// slots to spare, and so perhaps more cells.
+template <bool FILLS>
 struct LdsTable {
   uint32_t *keys, *counts, *firsts;
   uint32_t slots;  // a power of two
+  uint32_t *used;  // slots taken so far (FILLS)
+  static constexpr bool kFills = FILLS;
   typedef uint32_t Key;
   static constexpr Key kEmpty = 0xffffffffu;
   __device__ static void cleared() {}
 };
-// The same in device memory, for buckets of more points than the LDS table serves and for grids
-// whose keys need 64 bits.
+// The same in device memory, for buckets of more cells than the LDS table holds and for grids whose
+// keys need 64 bits.
 struct WideTable {
   u64 *keys;
   uint32_t *counts, *firsts;
   uint32_t slots;
   typedef u64 Key;
   static constexpr Key kEmpty = ~0ull;
+  uint32_t *used;
+  static constexpr bool kFills = false;
   // (plain stores of empty keys, then compare-and-swap by the other waves of the workgroup)
   __device__ static void cleared() { __threadfence(); }
 };
 
-// Takes the bucket's points in order, kRankThreads at a time.  A wave's points of one cell are put
+// Takes the bucket's points in order, THREADS at a time.  A wave's points of one cell are put
 // in order by ballots; the waves add theirs to the cell's count one after the other.  Points of a
 // cell that is full already are dropped in front of all that, so that a cell with very many points
-// (padding at one coordinate) costs a table lookup a point.
-template <typename TABLE>
-__device__ void rankBucket(const TABLE &t, const u64 *__restrict__ entries, uint32_t count,
+// (padding at one coordinate) costs a table lookup a point.  False (for all threads): the bucket has
+// more cells than the table takes; whoever starts again writes the same ranks again.
+template <int THREADS, int SLOTS, typename TABLE>
+__device__ __forceinline__ bool rankBucket(const TABLE &t, const u64 *__restrict__ entries, uint32_t count,
                            const float *__restrict__ points, const float *__restrict__ voxel_size,
                            const float *__restrict__ range, int num_features, bool small_grid, uint32_t max_points,
                            volatile uint16_t *s_owner, uint32_t *__restrict__ state, uint32_t *__restrict__ first_of) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (uint32_t s = tid; s < t.slots; s += kRankThreads) {
+  if (TABLE::kFills && tid == 0) *t.used = 0;
+  for (uint32_t s = tid; s < t.slots; s += THREADS) {
     t.keys[s] = TABLE::kEmpty;
     t.counts[s] = 0;
   }
   TABLE::cleared();
   __syncthreads();
   u64 next = (uint32_t)tid < count ? entries[tid] : 0;
-  for (uint32_t base = 0; base < count; base += kRankThreads) {
+  for (uint32_t base = 0; base < count; base += THREADS) {
     const u64 entry = next;
     const uint32_t i = base + tid;
-    if (i + kRankThreads < count) next = entries[i + kRankThreads];
+    if (i + THREADS < count) next = entries[i + THREADS];
     bool live = i < count;
     const uint32_t idx = (uint32_t)(entry >> 32);
     uint32_t slot = 0;
+    bool too_many = false;
     if (live) {
       u64 key = (uint32_t)entry;
       if (!small_grid) key = cellKey(cellOfPoint(points + (size_t)idx * num_features, voxel_size, range));
       slot = (uint32_t)(mix64(key) >> 32) & (t.slots - 1);
-      // (there are more slots than points, so an empty one is always reached)
+      // (there are more slots than points, or at least THREADS empty ones in front of every round, so
+      // an empty one is always reached)
       while (true) {
         const typename TABLE::Key seen = atomicCAS(&t.keys[slot], TABLE::kEmpty, (typename TABLE::Key)key);
+        if (TABLE::kFills && seen == TABLE::kEmpty) too_many = atomicAdd(t.used, 1u) + THREADS >= t.slots;
         if (seen == TABLE::kEmpty || seen == (typename TABLE::Key)key) break;
         slot = (slot + 1) & (t.slots - 1);
       }
       live = t.counts[slot] < max_points;
     }
+    if constexpr (TABLE::kFills) {
+      if (__syncthreads_or(too_many)) return false;
+    }
     if (!__syncthreads_or(live)) continue;
     // A lane that reads its own number back is alone in its wave with the slot, or the last of its
     // group to write; the groups of all other lanes are gone through one by one.
-    if (live) s_owner[slot & (kLdsSlots - 1)] = (uint16_t)tid;
-    const bool shares = live && s_owner[slot & (kLdsSlots - 1)] != (uint16_t)tid;
+    if (live) s_owner[slot & (SLOTS - 1)] = (uint16_t)tid;
+    const bool shares = live && s_owner[slot & (SLOTS - 1)] != (uint16_t)tid;
     uint32_t rank = 0, group = 1;
     int leader = lane;
     u64 open = __ballot(shares);
@@ -267,7 +280,7 @@ __device__ void rankBucket(const TABLE &t, const u64 *__restrict__ entries, uint
       open &= ~same;
     }
     uint32_t before = 0;
-    for (int w = 0; w < kRankWaves; ++w) {
+    for (int w = 0; w < (THREADS / 64); ++w) {
       if (wave == w && live && rank == 0) {
         before = t.counts[slot];
         t.counts[slot] = before + group;
@@ -282,42 +295,61 @@ __device__ void rankBucket(const TABLE &t, const u64 *__restrict__ entries, uint
     }
   }
   __syncthreads();
-  for (uint32_t s = tid; s < t.slots; s += kRankThreads) {
+  for (uint32_t s = tid; s < t.slots; s += THREADS) {
     const uint32_t c = t.counts[s];
     if (c != 0) state[t.firsts[s]] = kIsFirst | (c < max_points ? c : max_points);
   }
+  return true;
 }
 
 // state[i] (cleared before): kIsFirst | points the cell keeps, for the first point of a cell; the
 // rank in the cell for another point it keeps, whose first_of[i] is the first one; 0 otherwise.
-__global__ __launch_bounds__(kRankThreads) void voxRankInCells(
+// A bucket of any number of points is ranked in LDS as long as its cells fit there, which those of a
+// crowded cell do; the table in device memory takes several times as long.
+template <int THREADS, int SLOTS>
+__global__ __launch_bounds__(THREADS) void voxRankInCells(
     const float *__restrict__ points, const float *__restrict__ voxel_size, const float *__restrict__ range,
     int num_features, uint32_t max_points, const u64 *__restrict__ grouped, const uint32_t *__restrict__ bucket_start,
     const uint32_t *__restrict__ totals, u64 *wide_keys, uint32_t *wide_counts, uint32_t *wide_firsts,
     uint32_t *__restrict__ state, uint32_t *__restrict__ first_of) {
-  __shared__ uint32_t s_keys[kLdsSlots], s_counts[kLdsSlots], s_firsts[kLdsSlots];
-  __shared__ uint16_t s_owner[kLdsSlots];
+  __shared__ uint32_t s_keys[SLOTS], s_counts[SLOTS], s_firsts[SLOTS];
+  __shared__ uint16_t s_owner[SLOTS];
+  __shared__ uint32_t s_used;
   const uint32_t count = totals[blockIdx.x];
   if (count == 0) return;
   const uint32_t start = bucket_start[blockIdx.x];
   const bool small_grid =
       smallGrid((u64)axisCells(range[2], range[5], voxel_size[2]) * (u64)axisCells(range[1], range[4], voxel_size[1]) *
                 (u64)axisCells(range[0], range[3], voxel_size[0]));
-  if (small_grid && count <= kLdsSlots / 2) {
-    LdsTable t = {s_keys, s_counts, s_firsts, 64};
-    while (t.slots < 2 * count) t.slots <<= 1;
-    rankBucket(t, grouped + start, count, points, voxel_size, range, num_features, true, max_points, s_owner, state,
-               first_of);
-  } else {
-    // the bucket's share of the region: the largest power of two within three slots a point
-    const size_t at = 3 * (size_t)start;
-    WideTable t = {wide_keys + at, wide_counts + at, wide_firsts + at, 1u << (31 - __clz(3 * count))};
-    rankBucket(t, grouped + start, count, points, voxel_size, range, num_features, small_grid, max_points, s_owner,
-               state, first_of);
+  if (small_grid) {
+    if (__builtin_expect(count <= SLOTS / 2, 1)) {
+      LdsTable<false> t = {s_keys, s_counts, s_firsts, 64, nullptr};
+      while (t.slots < 2 * count) t.slots <<= 1;
+      rankBucket<THREADS, SLOTS>(t, grouped + start, count, points, voxel_size, range, num_features, true, max_points,
+                                 s_owner, state, first_of);
+      return;
+    }
+    const LdsTable<true> t = {s_keys, s_counts, s_firsts, SLOTS, &s_used};
+    if (rankBucket<THREADS, SLOTS>(t, grouped + start, count, points, voxel_size, range, num_features, true, max_points,
+                                   s_owner, state, first_of))
+      return;
   }
+  // the bucket's share of the region: the largest power of two within three slots a point
+  const size_t at = 3 * (size_t)start;
+  const WideTable t = {wide_keys + at, wide_counts + at, wide_firsts + at, 1u << (31 - __clz(3 * count)), nullptr};
+  rankBucket<THREADS, SLOTS>(t, grouped + start, count, points, voxel_size, range, num_features, small_grid, max_points,
+                             s_owner, state, first_of);
 }
 
 // ---- voxel numbers -----------------------------------------------------------------------
+
+// Points a bucket has on average, above which a larger table in LDS is the better one although fewer
+// workgroups share a CU (us for voxRankInCells with 2048, 4096 and 8192 slots, points strewn over all
+// cells: 2.0 million points 37, 41, -; 2.4: 54, 49, -; 3.0: 68, 54, -; 4.0: 318, 74, 86; 6.0: -, 153,
+// 121).  The largest takes 7168 cells, buckets of 14.6 million points; from there on more and more
+// buckets go to device memory (12 million points: 330 us in LDS, 2240 us there).
+constexpr int64_t kPointsForLargerTable = 1100;
+constexpr int64_t kPointsForLargestTable = 2400;
 
 struct FirstPoints {
   const uint32_t *state;
@@ -452,11 +484,15 @@ hipError_t launchVoxelize(const LaunchCtx &lc, const VoxelizeShape &s, const flo
   lc.end();
   if ((e = hipGetLastError()) != hipSuccess) return e;
 
+  const int64_t per_bucket = n / buckets;
+  const bool largest = per_bucket > kPointsForLargestTable;
+  auto rank = largest                                ? voxRankInCells<1024, 8192>
+              : per_bucket > kPointsForLargerTable ? voxRankInCells<512, 4096>
+                                                   : voxRankInCells<512, 2048>;
   lc.begin("voxRankInCells");
-  voxRankInCells<<<buckets, kRankThreads, 0, lc.stream>>>(points, voxel_size, coors_range, s.num_features,
-                                                         (uint32_t)s.max_points, w.grouped, w.bucket_start, totals,
-                                                         w.wide_keys, w.wide_counts, w.wide_firsts, w.state,
-                                                         w.first_of);
+  rank<<<buckets, largest ? 1024 : 512, 0, lc.stream>>>(points, voxel_size, coors_range, s.num_features,
+                                                (uint32_t)s.max_points, w.grouped, w.bucket_start, totals, w.wide_keys,
+                                                w.wide_counts, w.wide_firsts, w.state, w.first_of);
   lc.end();
   if ((e = hipGetLastError()) != hipSuccess) return e;
 
