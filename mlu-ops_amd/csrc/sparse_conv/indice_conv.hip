@@ -310,10 +310,12 @@ __global__ __launch_bounds__(256) void gatherConvSimt(const typename E::storage 
 
 // ---- MFMA gather convolution ---------------------------------------------------
 
-// Channels of a filter B(k, q, c) as they are, and as the kernel instance counts them.
+// Channels of a filter B(k, q, c) as they are, and in fragments of the kernel instance (whose numbers
+// are powers of two).  `whole`: the fragments hold nothing else.
 struct FilterShape {
   int q, c;
-  int q_padded, c_padded;
+  int chunk_bits, group_bits;  // 1 << chunk_bits fragments a column, 1 << group_bits columns of 16
+  bool whole;
 };
 
 // Filter repacked into MFMA operand fragments of 16 bytes per lane (VEC elements,
@@ -332,28 +334,31 @@ __device__ __forceinline__ void packFilter(const typename E::storage *W, int64_t
                                            const FilterShape &shape, typename E::storage *packed,
                                            unsigned long long ticket, int block, int blocks) {
   constexpr int VEC = E::kVec, CHUNK = E::kChunk;
-  const int chunks = (shape.q_padded + CHUNK - 1) / CHUNK;
-  const int groups = shape.c_padded / 16;
-  const size_t total = (size_t)K * groups * chunks * 64;
-  unsigned long long *const nonfinite = reinterpret_cast<unsigned long long *>(packed + total * VEC);
+  const uint32_t total = (uint32_t)K << (shape.group_bits + shape.chunk_bits + 6);  // (below 2^24 for 4096 offsets)
+  unsigned long long *const nonfinite = reinterpret_cast<unsigned long long *>(packed + (size_t)total * VEC);
   if (block == 0 && threadIdx.x == 0) nonfinite[K] = ticket;
-  for (size_t t = (size_t)block * 256 + threadIdx.x; t < total; t += (size_t)blocks * 256) {
+  for (uint32_t t = block * 256 + threadIdx.x; t < total; t += blocks * 256) {
     const int lane = (int)(t & 63);
-    size_t rest = t >> 6;
-    const int kb = (int)(rest % chunks);
-    rest /= chunks;
-    const int nb = (int)(rest % groups);
-    const int k = (int)(rest / groups);
+    const uint32_t fragment = t >> 6;
+    const int kb = (int)(fragment & ((1u << shape.chunk_bits) - 1u));
+    const int nb = (int)(fragment >> shape.chunk_bits & ((1u << shape.group_bits) - 1u));
+    const int k = (int)(fragment >> (shape.chunk_bits + shape.group_bits));
     const int c = nb * 16 + (lane & 15);
     const int qb = kb * CHUNK + VEC * (lane >> 4);
+    const typename E::storage *const from = W + k * sK + qb * sQ + c * sC;
+    typename E::storage v[VEC];
+    if (shape.whole) {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) v[e] = from[e * sQ];
+    } else {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) v[e] = qb + e < shape.q && c < shape.c ? from[e * sQ] : typename E::storage(0);
+    }
     bool finite = true;
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
-      const typename E::storage v = qb + e < shape.q && c < shape.c
-                                        ? W[(size_t)k * sK + (size_t)(qb + e) * sQ + (size_t)c * sC]
-                                        : typename E::storage(0);
-      finite = finite && E::finite(v);
-      packed[t * VEC + e] = v;
+      finite = finite && E::finite(v[e]);
+      packed[(size_t)t * VEC + e] = v[e];
     }
     if (!finite) nonfinite[k] = ticket;
   }
@@ -1035,14 +1040,16 @@ void gatherConvMfma(const typename E::storage *A, ConvRows rows, const typename 
 // Measured against the kernel above on 120 000 rows with 2.2 pairs a row: 32 -> 32
 // channels 26 us against 32 us; at 64 result columns (two waves a tile, 32 columns
 // each) it loses, 43 us against 41 us, and is not used.
+// WHOLE: rows and results of exactly Q and C channels, with their lengths as constants (the same
+// layers with lengths from the arguments: 16 -> 16 channels 30.8 against 28.6 us, 32 -> 32 35 against 32).
 constexpr int kWaveTileRows = 128;
 constexpr bool waveKernelShape(int elem_bytes, int Q, int C) {
   const int chunk = elem_bytes == 4 ? 16 : 32;
   return C <= 32 && Q * elem_bytes <= 256 && ((Q + chunk - 1) / chunk) * (C / 16) <= 8;
 }
-template <typename E, int Q, int C>
+template <typename E, int Q, int C, bool WHOLE>
 __global__ __launch_bounds__(64) void gatherConvWave(
-    const typename E::storage *A, ConvRows conv, const typename E::storage *packedW, SegmentSource source,
+    const typename E::storage *A, ConvRows lengths, const typename E::storage *packedW, SegmentSource source,
     int R, int K, typename E::storage *result) {
   typedef typename E::vec8 vec8;
   typedef typename E::storage S;
@@ -1052,6 +1059,7 @@ __global__ __launch_bounds__(64) void gatherConvWave(
   constexpr int TR = kWaveTileRows;
   constexpr int ACC_STRIDE = C + 4;
   constexpr int ROW_BYTES = Q * (int)sizeof(S);
+  const ConvRows conv = WHOLE ? ConvRows{Q, ROW_BYTES, C, C} : lengths;
   constexpr int STAGE_STRIDE = ROW_BYTES + 16;
   constexpr int PPR = ROW_BYTES / 16;                   // 16-byte pieces per row
   constexpr int RL = (16 * PPR + 63) / 64;              // wave-loads per unit of rows
@@ -2291,7 +2299,9 @@ __device__ __forceinline__ SlicePlace sliceOfWorkgroup(const SliceOrder &order, 
 // (with a row's pieces spread over eight lanes the same stores hit 8 banks and
 // took 28 cycles each).  Wave w multiplies the 16-row blocks w, w+4, ... of dW[k]
 // against all column blocks.  Rows are `rows.ci` and `rows.co` channels long: the channels
-// behind them, up to CI and CO, are zeros.
+// behind them, up to CI and CO, are zeros.  WHOLE: rows of exactly CI and CO channels, with their
+// lengths as constants (64 x 64 channels in fp32: 43 us, 46 with lengths from the arguments; the
+// kernel behind this one, fp16: 64 x 64 14.6 against 15.2, 128 x 128 28.0 against 30.2).
 
 // The channels of the feature and gradient rows, at most the CI and CO of the instance.
 struct FilterGradRows {
@@ -2320,9 +2330,9 @@ __device__ __forceinline__ u32x4 rowPiece(const S *row, int c0, int channels) {
   return piece;
 }
 
-template <typename E, int CI, int CO>
+template <typename E, int CI, int CO, bool WHOLE>
 __global__ __launch_bounds__(256) void backwardFilterMfma(
-    const typename E::storage *X, const typename E::storage *dY, FilterGradRows rows, const int32_t *pairs, int L,
+    const typename E::storage *X, const typename E::storage *dY, FilterGradRows lengths, const int32_t *pairs, int L,
     int x_col, int n_in, int n_out, int K, SliceTable tab, SliceOrder order, int total_slices,
     int slice_len, float *partial) {
   typedef typename E::vec8 vec8;
@@ -2336,6 +2346,7 @@ __global__ __launch_bounds__(256) void backwardFilterMfma(
   constexpr int YT = YP / 256 > 0 ? YP / 256 : 1;
   constexpr int XU = XP / 64;  // staging units (32 pairs x 2 pieces) of X per step
   constexpr int YU = YP / 64;
+  const FilterGradRows rows = WHOLE ? FilterGradRows{CI, CO} : lengths;
   static_assert(SP == 64 && (CI / EPP) % 2 == 0 && (CO / EPP) % 2 == 0, "unit = 32 pairs x 2 pieces");
   constexpr int CBW = (CI / 16 + 3) / 4;  // row blocks per wave
   constexpr int COB = CO / 16;
@@ -2498,9 +2509,9 @@ constexpr int filterRowSwizzle(int row_bytes, int pair) {
                           : 0;
 }
 
-template <typename E, int CI, int CO, int SP>
+template <typename E, int CI, int CO, int SP, bool WHOLE>
 __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
-    const typename E::storage *X, const typename E::storage *dY, FilterGradRows rows, const int32_t *pairs, int L,
+    const typename E::storage *X, const typename E::storage *dY, FilterGradRows lengths, const int32_t *pairs, int L,
     int x_col, int n_in, int n_out, int K, SliceTable tab, SliceOrder order, int total_slices,
     int slice_len, float *partial) {
   typedef typename E::vec8 vec8;
@@ -2512,6 +2523,7 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
   // two chunks of row indices: with 128 channels on both sides the buffers leave 16 KiB of
   // half a CU's LDS
   constexpr int kIndexChunk = 512;
+  const FilterGradRows rows = WHOLE ? FilterGradRows{CI, CO} : lengths;
   constexpr int kChunkSteps = kIndexChunk / SP;
   constexpr int RBX = CI * 2, RBY = CO * 2;     // bytes per row
   constexpr int XN = SP * RBX / 1024;           // 1 KiB wave-loads per step
@@ -3054,7 +3066,9 @@ void launchWaveInstance(const LaunchCtx &lc, const void *A, const ConvRows &rows
   if constexpr (waveKernelShape((int)sizeof(typename E::storage), Q, C)) {
     const int grid = ((R + kWaveTileRows - 1) / kWaveTileRows + 7) / 8 * 8;
     lc.begin("gatherConvWave");
-    gatherConvWave<E, Q, C><<<grid, 64, 0, lc.stream>>>(
+    const bool whole = rows.q == Q && rows.c == C;
+    auto kernel = whole ? gatherConvWave<E, Q, C, true> : gatherConvWave<E, Q, C, false>;
+    kernel<<<grid, 64, 0, lc.stream>>>(
         static_cast<const typename E::storage *>(A), rows, static_cast<const typename E::storage *>(packed),
         source, R, K, static_cast<typename E::storage *>(result));
     lc.end();
@@ -3213,13 +3227,16 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
   // B(k, q, c): forward q = ci, c = co; backward data q = co, c = ci.
   const int64_t sQ = d.filter_forward ? f.stride_ci : f.stride_co;
   const int64_t sC = d.filter_forward ? f.stride_co : f.stride_ci;
-  const FilterShape shape = {d.Q, d.C, d.q_padded, d.c_padded};
+  const int chunks = (d.q_padded + E::kChunk - 1) / E::kChunk, groups = d.c_padded / 16;
+  FilterShape shape = {d.Q, d.C, 0, 0, d.Q == chunks * E::kChunk && d.C == d.c_padded};
+  while (1 << shape.chunk_bits < chunks) ++shape.chunk_bits;
+  while (1 << shape.group_bits < groups) ++shape.group_bits;
   const bool pad_rows = use_mfma && rowsNeedPadding(p.dtype, d.Q);
   const ConvRows rows_of = {d.Q, pad_rows ? paddedRowBytes(p.dtype, d.Q) : d.Q * (int)sizeof(S), d.C, d.c_padded};
   const void *rows_from = pad_rows ? ws.padded_rows : gathered;
   const PadRows pad = {static_cast<const char *>(gathered), static_cast<char *>(ws.padded_rows), d.Q * (int)sizeof(S),
                        rows_of.row_bytes, pad_rows ? d.n_src : 0, pad_rows ? gridFor((size_t)d.n_src, 1024) : 0};
-  const size_t frags = (size_t)p.K * (d.c_padded / 16) * ((d.q_padded + E::kChunk - 1) / E::kChunk) * 64;
+  const size_t frags = (size_t)p.K * groups * chunks * 64;
   const bool single_chunk = p.row_map == nullptr && ws.map_rows >= d.R && lc.choices.small_map_chunks != 1;
   // Pair lists whose order nobody has reported yet: the call starts on them all the same,
   // and the row-map kernels are enqueued behind, each of them told to return at once unless
@@ -3415,14 +3432,20 @@ void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const S
   const int grid = (total_slices + 7) / 8 * 8;
   lc.begin(transposing ? "backwardFilterMfmaTr" : "backwardFilterMfma");
   if (total_slices > 0) {
-    auto kernel = backwardFilterMfma<E, CI, CO>;
+    const bool whole = p.Ci == CI && p.Co == CO;
+    auto kernel = backwardFilterMfma<E, CI, CO, false>;
+    if constexpr (!kTransposingShape) {
+      if (whole) kernel = backwardFilterMfma<E, CI, CO, true>;
+    }
     if constexpr (kTransposingShape) {
       // Steps of 32 pairs halve the row buffers: below 128 x 128 channels more workgroups
       // share a CU then, which pays when the slices are long (network 64 x 64: 101 -> 88 us;
       // on slices of a few steps the shorter steps only add barriers: config 4 23.7 -> 25.3 us).
       const bool short_steps = CI + CO < 256 && slice_len >= 2048;
-      if (transposing)
-        kernel = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32> : backwardFilterMfmaTr<E, CI, CO, 64>;
+      if (transposing && whole)
+        kernel = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32, true> : backwardFilterMfmaTr<E, CI, CO, 64, true>;
+      else if (transposing)
+        kernel = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32, false> : backwardFilterMfmaTr<E, CI, CO, 64, false>;
     }
     kernel<<<grid, 256, 0, lc.stream>>>(
         static_cast<const S *>(features), static_cast<const S *>(output_grad), rows, p.indice_pairs, p.L,
