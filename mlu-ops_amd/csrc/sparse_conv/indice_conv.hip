@@ -3109,12 +3109,21 @@ bool useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims 
   if (!denseShapeOk(p, d)) return false;
   if (lc.choices.dense_tiles >= 0) return lc.choices.dense_tiles == 1;
   // What the kernel costs goes with the (tile, offset) pieces that hold a pair at all, what
-  // the pair-list kernels cost with the pairs.  Measured on 150000 rows, 3x3x3, fp16, as the
-  // share of all (row, offset) slots that hold a pair from which the kernel wins:
-  //   result columns   voxels strewn uniformly   scenes (filled sheets and walls)
-  //   16, 32           0.35 (0.27: 45 us against 40 us, 0.51: 50 against 60)   0.04 (30 against 32)
-  //   64               0.38 (0.27: 86 against 77, 0.51: 104 against 119)      0.15 (67 against 73)
-  //   128              0.25 (175 against 183)                                  0.04 (88 against 98)
+  // the pair-list kernels cost with the pairs.  Measured on 150000 rows, 3x3x3, as the share of all
+  // (row, offset) slots that hold a pair from which the kernel wins, with us of the pair-list kernels
+  // against us of this one around it:
+  //   reduction -> result channels     voxels strewn uniformly               scenes (filled sheets and walls)
+  //   fp16   16 -> 16                  0.18 (0.15: 24/26, 0.27: 31/26)       0.045 (0.04: 18/19, 0.05: 23/19)
+  //          32 -> 32                  0.18 (0.15: 28/31, 0.27: 36/30)       0.045 (0.04: 20/21, 0.05: 27/20)
+  //          16, 32 -> 64              0.14 (0.13: 39/41, 0.18: 47/41)       0.06  (0.05: 31/29, 0.10: 46/32)
+  //          64 -> 64                  0.25 (0.22: 59/63, 0.27: 66/62)       0.09  (0.07: 39/47, 0.10: 52/48)
+  //          64 -> 128                 0.22 (0.18: 79/84, 0.27: 98/83)       0.05  (0.04: 51/56, 0.05: 59/54)
+  //          128 -> 128                0.27 (0.22: 132/149, 0.31: 165/150)   0.055 (0.04: 67/75, 0.07: 91/91)
+  //   fp32   16 -> 16, 32              0.3  (0.22: 46/54, 0.4: 66/54)        0.05  (0.04: 26/31, 0.07: 49/38)
+  //          32 -> 32                  0.4  (0.31: 81/95, 0.5: 114/95)       0.065 (0.05: 46/57, 0.10: 95/72)
+  //          32 -> 64                  0.5  (0.4: 138/160, 0.5: 160/159)     0.15  (0.11: 111/125, 0.17: 138/129)
+  //          64 -> 64                  -    (0.5: 275/338)                   0.2   (0.17: 231/242, 0.27: 294/245)
+  //          64 -> 128                 -    (0.5: 485/636)                   -     (0.27: 462/450, 0.33: 471/505)
   // On strewn voxels every piece holds a few pairs; in a scene the pairs of an offset sit in
   // few pieces.  The host only knows the pair counts: sheets and walls show there as offsets
   // with far more pairs than the average offset (in-plane neighbours), which strewn voxels
@@ -3134,9 +3143,13 @@ bool useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims 
   // (the largest count is the centre offset of a submanifold convolution: left out)
   const double mean_rest = p.K > 1 ? (pairs - largest) / (p.K - 1) : 0.0;
   const bool sheets = mean_rest > 0 && second >= 1.5 * mean_rest;
-  if (d.c_padded <= 32) return fill >= (sheets ? 0.04 : 0.35);
-  if (d.c_padded == 64) return fill >= (sheets ? 0.15 : 0.38);
-  return fill >= (sheets ? 0.04 : 0.25);
+  if (p.dtype != ElemType::kFloat) {
+    if (sheets) return fill >= (d.q_padded >= 64 && d.c_padded == 64 ? 0.085 : 0.05);
+    return fill >= (d.q_padded <= 32 ? 0.17 : 0.27);
+  }
+  if (d.c_padded <= 32) return fill >= (sheets ? 0.06 : 0.35);
+  if (d.c_padded == 64) return fill >= (sheets ? 0.18 : 0.5);
+  return sheets && d.q_padded <= 32 && fill >= 0.2;
 }
 
 template <typename E, int Q, int C, typename SRC>
