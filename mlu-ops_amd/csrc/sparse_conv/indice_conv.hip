@@ -13,16 +13,20 @@
 // is owned by exactly one workgroup, which walks the K offsets in order and adds
 // the contribution of the (at most one) gathered row per offset.  No atomics,
 // no inter-workgroup reduction, so results are reproducible run to run.  The
-// owner of a row finds its gathered rows through a dense row map
+// owner of a row finds its gathered rows through the pair lists, cut by tile of
+// result rows, where they are in order, or through a dense row map
 // map[k][row] -> gathered row or -1, rebuilt from indice_pairs on every call.
 //
-// Two implementations of the gather convolution:
-//  * gatherConvMfma  fp16/bf16, channel counts that tile into 16x16x32 MFMA
-//    blocks.  A workgroup owns up to 256 result rows; per offset the rows that
-//    have a partner are compacted with wave ballots into blocks of 16, so MFMA
-//    work follows the number of pairs, not K x rows.  Each wave owns a column
-//    slice of the fp32 accumulator tile in LDS.
-//  * gatherConvSimt  any type and channel count (fp32 always), LDS-tiled FMA.
+// Kernels of the gather convolution (fp16, bf16 and fp32 alike):
+//  * gatherConvMfma   up to 128 channels on both sides, in MFMA blocks of 16 pairs.  Per offset the
+//    rows of a tile that have a partner are compacted, so MFMA work follows the number of
+//    pairs, not K x rows.  Each wave owns a column slice of the fp32 accumulator tile in LDS.
+//  * gatherConvWave   the same for results of up to 32 columns, one wavefront a tile.
+//  * gatherConvDense  rulebooks whose (tile, offset) pieces are well filled: accumulators in
+//    registers, all rows of a tile multiplied at every offset that has a pair there.
+//  * gatherConvSimt   any channel count, LDS-tiled FMA.
+// A row takes nothing from the filter of an offset at which it has no pair, in any of them, also
+// where that filter is not finite.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -3098,7 +3102,8 @@ bool useWaveKernel(const LaunchCtx &lc, ElemType t, int Q, int C) {
   return waveKernelShape((int)elemSize(t), Q, C);
 }
 
-// The register-accumulating kernel addresses the gathered tensor with 32-bit byte offsets.
+// The register-accumulating kernel addresses the gathered tensor with 32-bit byte offsets: tensors of
+// 2 GiB and more take the pair-list kernels.
 bool denseShapeOk(const ConvProblem &p, const GatherDims &d) {
   // (fp32 rows of more than 64 channels leave no room for two row groups a wave)
   if (p.dtype == ElemType::kFloat && d.Q > 64) return false;

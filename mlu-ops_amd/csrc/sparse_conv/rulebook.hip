@@ -132,8 +132,7 @@ __device__ __forceinline__ void noteRowOrder(const int32_t *indices, int j, int4
   if (j > 0 && !coordBelow(loadCoord(indices, j - 1, aligned), c)) *rows_in_order = 0;
 }
 
-// The rulebook's report to the host: the flag first, then the stamp the host looks for.
-// The number of pairs of offset k, for the device and for the host.
+// The number of pairs of offset k, for the device and (stamped words, one an offset) for the host.
 __device__ __forceinline__ void fileCount(int k, int count, int32_t *indice_num,
                                           const RulebookReportTarget &report) {
   indice_num[k] = count;
@@ -142,6 +141,7 @@ __device__ __forceinline__ void fileCount(int k, int count, int32_t *indice_num,
                        __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// The rulebook's report to the host, a stamped word: were the input rows in cell order?
 __device__ __forceinline__ void fileReport(bool rows_in_order, const RulebookReportTarget &report) {
   if (report.order_word == nullptr) return;
   __hip_atomic_store(report.order_word, stampedWord(report.stamp, rows_in_order ? 1 : 0), __ATOMIC_RELAXED,

@@ -204,8 +204,8 @@ def test_points_to_voxels_to_submanifold_layer(gpu_handle):
 
 
 def test_small_channel_counts_are_padded_for_the_matrix_cores(gpu_handle):
-    """5 -> 12 channels (padded to 16 -> 16 inside the layer): values and gradients against the
-    rulebook-driven float64 formula."""
+    """5 -> 12 channels (on the kernels' instances for 16 -> 16, which read and write the rows as they are):
+    values and gradients against the rulebook-driven float64 formula."""
     import torch
     from mluop_hip import nn as spnn
     rng = np.random.default_rng(24)

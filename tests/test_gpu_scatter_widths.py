@@ -1,5 +1,8 @@
-"""Point scatter with features taken one, two and four at a time by a thread, voxels on both sides of
-the points a thread holds at once, and a backward pass with and without room for the point lists."""
+"""Point scatter with features taken one, two and four at a time by a thread; a backward pass by atomic
+minima, and by lists of points with voxels on both sides of the longest list and of the points a
+thread holds at once, with and without room for the lists."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -22,7 +25,7 @@ def test_forward_and_backward(gpu_handle, c, n, span):
         assert_same(run_gpu(gpu_handle, mode, feats, coors), dpv.forward(mode, feats, coors))
     g = rng.standard_normal((n, c)).astype(np.float32)
     tf, tc = torch.from_numpy(feats).cuda(), torch.from_numpy(coors).cuda()
-    for rows in (n, (n + 1) // 2):   # (half the rows: less workspace, and points of voxels without a row)
+    for rows in (n, (n + 1) // 2):   # (half the rows: points of voxels without a row)
         vf, vc, p2v, cnt, num = mluop_hip.dynamic_point_to_voxel_forward(gpu_handle, tf, tc.clone(), "max", rows)
         grad = mluop_hip.dynamic_point_to_voxel_backward(gpu_handle, torch.from_numpy(g[:rows]).cuda(), tf, vf, p2v,
                                                          cnt, num)
@@ -76,3 +79,37 @@ def test_backward_of_many_wide_features(gpu_handle, c, n, crowds):
     feats = rng.integers(-8, 9, (n, c)).astype(np.float32)   # ties in every longer list
     feats[rng.random(n) < 0.01] = np.nan
     check_backward(gpu_handle, rng, feats, coors)
+
+
+@pytest.mark.parametrize("rows", [1000, 100_000])
+def test_backward_with_no_more_workspace_than_it_must_have(gpu_handle, rows):
+    """rows x features words: room for the lists beside many rows, not beside few."""
+    import torch
+    import mluop_hip as m
+    n, c = 250_000, 32
+    rng = np.random.default_rng(rows)
+    coors = crowded(rng, n, [100, 40, 3])
+    feats = rng.integers(-8, 9, (n, c)).astype(np.float32)
+    g = torch.from_numpy(rng.standard_normal((rows, c)).astype(np.float32)).cuda()
+    tf = torch.from_numpy(feats).cuda()
+    vf, vc, p2v, cnt, num = m.dynamic_point_to_voxel_forward(gpu_handle, tf, torch.from_numpy(coors).cuda(), "max", rows)
+
+    def desc(dtype, *dims):
+        return m.TensorDescriptor(m.LAYOUT_ARRAY, dtype, dims)
+    wide, points, lines, line = (desc(m.DTYPE_FLOAT, rows, c), desc(m.DTYPE_FLOAT, n, c), desc(m.DTYPE_INT32, n),
+                                 desc(m.DTYPE_INT32, rows))
+    one = desc(m.DTYPE_INT32, 1)
+    guard = torch.full((rows * c + 64,), 0x5a5a5a5a, dtype=torch.int32, device="cuda")   # 64 words behind the workspace
+    grad = torch.empty((n, c), device="cuda")
+    gpu_handle.set_kernel_timing(True)
+    m.check(m.lib().mluOpDynamicPointToVoxelBackward(
+        gpu_handle.ptr, m.REDUCE_DMAX, wide.ptr, g.data_ptr(), points.ptr, tf.data_ptr(), wide.ptr, vf.data_ptr(), lines.ptr,
+        p2v.data_ptr(), line.ptr, cnt.data_ptr(), one.ptr, num.data_ptr(), ctypes.c_void_p(guard.data_ptr()), rows * c * 4,
+        points.ptr, grad.data_ptr()))
+    listed = any(k == "dpvBackwardLists" for k, _ in gpu_handle.kernel_timings())
+    gpu_handle.set_kernel_timing(False)
+    torch.cuda.synchronize()
+    assert listed == (rows == 100_000)
+    assert bool((guard[rows * c:] == 0x5a5a5a5a).all())
+    want = dpv.backward(g.cpu().numpy(), feats, vf.cpu().numpy(), p2v.cpu().numpy(), min(int(num.item()), rows))
+    assert np.array_equal(grad.cpu().numpy(), want)
