@@ -34,13 +34,14 @@ _share_row_maps = False
 
 
 def share_row_maps(enable):
-    """Layers and passes that use one rulebook share its row maps (built once per rulebook and
-    direction, without the verifying count since the coordinates are known to be distinct)
-    instead of rebuilding them in every operator call.  Pays when a rulebook serves many calls
-    (a fixed scene, deep stages: the config-4 forward takes 0.036 ms instead of 0.047 ms); with a
-    new rulebook per step and two layers per stage it saves one map build in four (measured on
-    the 11-layer encoder: 6.29-6.35 ms a step against 6.32-6.38 ms) and holds K x rows x 8 bytes
-    per rulebook, hence off by default."""
+    """Layers and passes that use one rulebook share its row maps (built once per rulebook, direction
+    and stream, without the verifying count since the coordinates are known to be distinct)
+    instead of rebuilding them in every operator call or reading the pair lists.  Pays when a
+    rulebook serves many calls (a fixed scene: the forward of a 64 -> 64 layer on 120 000 rows takes
+    0.033 ms with a kept map, 0.036 ms on the pair lists and 0.042 ms with a map per call); with a
+    new rulebook per step and two layers per stage the pair lists are faster (the 11-layer encoder:
+    3.6 ms a step, 3.8 ms with shared maps), and the maps hold K x rows x 8 bytes per rulebook,
+    hence off by default."""
     global _share_row_maps
     _share_row_maps = bool(enable)
 
