@@ -36,6 +36,7 @@ typedef enum {
   MLUOP_EXT_KERNEL_FILTER_STORES = 6,   /* 1: backward filter transposes its operands with element-sized
                                            LDS stores also for 2-byte types of 32 to 128 channels, where
                                            transposing LDS reads are the default */
+  MLUOP_EXT_KERNEL_TALL_TILES = 8,      /* gather kernel with tall tiles of result rows */
   MLUOP_EXT_KERNEL_LISTS_ON_TRUST = 7   /* forward on a rulebook of this handle whose report (were the input
                                            rows in cell order?) has not reached the host yet, as under graph
                                            capture or without any wait between the two calls.  -1: start on

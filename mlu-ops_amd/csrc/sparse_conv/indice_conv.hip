@@ -1022,6 +1022,391 @@ void gatherConvMfma(const typename E::storage *A, ConvRows rows, const typename 
   }
 }
 
+constexpr uint32_t kNoRow = 0x80000000u;  // byte offset of a partner that is not there
+
+// The gathered tensor as a buffer of `bytes` (below 2^31) for loads that answer zero behind it.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rowsBuffer(const void *base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
+}
+
+// ---- MFMA gather convolution, tall tiles -------------------------------------------------
+//
+// What a thinly filled offset costs a tile is its filter: every (tile, offset) piece that holds a pair
+// loads W[k] from L2 (16 KB for 64 columns of 128 channels of a 2-byte type, 12.8 GB in all at
+// 5x5x5, 400 000 rows, 128 -> 128, where the kernel above takes 715 us) for as many pairs as the tile's
+// rows have there.  Here a tile has 256 result rows by 64 columns, two workgroups a CU, which is what
+// LDS holds fp32 sums for when nothing else of the tile lies there whole: the entries of up to
+// max_blocks blocks of 16 pairs and two rounds of gathered rows.  The rest travels in registers:
+//   fetching waves     request the rows of round r + ahead and write those of round r to LDS, their
+//                      pieces of 16 bytes permuted by row, so that the 16 rows of a block meet all banks;
+//   multiplying waves  own 16 result columns each: per block the operand fragments from the staged
+//                      rows, W[k] from registers (requested `ahead` rounds before), and a 16-byte
+//                      read-modify-write of every pair's sums.  The sums of a round are updated while
+//                      the next round's rows are read: both are chains of LDS round trips.
+// One barrier a round.  The arithmetic and its order are those of gatherConvMfma, bit for bit.
+// 715 -> 460 us at the shape above; 120 000 rows, 3x3x3, 64 -> 64: 35 -> 30.  What bounds it there: a tile's first
+// rows arrive 4.7 us after its start (cuts, pairs and rows are three dependent loads), a round of two
+// blocks takes about 0.4 us, and the launch lasts as long as its heaviest tile (28 us, mean 16).
+// Rounds are padded to whole trips of the loops, which have one way out each: with a second one the
+// compiler waits for all loads in flight at the loop's head.
+struct TallPlan {
+  int per_cu;      // workgroups a CU
+  int blocks;      // blocks of 16 pairs a round
+  int ahead;       // rounds whose rows and filters travel in registers
+  int max_blocks;  // blocks whose entries are in LDS at once
+};
+constexpr int kTallCols = 64;
+constexpr int kTallWaves = 4;  // multiplying waves, and as many fetching ones
+constexpr int kTallThreads = 2 * kTallWaves * 64;
+// Two workgroups of 256 rows share a CU, but for rows of 512 bytes, of which the second would leave
+// no room for a round.
+constexpr int tallRows(int row_bytes) { return row_bytes >= 512 ? 512 : 256; }
+constexpr TallPlan tallPlan(int row_bytes) {
+  const int rows = tallRows(row_bytes);
+  TallPlan p = {rows == 256 ? 2 : 1, 1, 4, 0};
+  p.blocks = (rows == 256 ? 4096 : 8192) / (16 * row_bytes);
+  const int left = 160 * 1024 / p.per_cu - (rows + 1) * kTallCols * 4 - 2 * p.blocks * 16 * row_bytes - 256;
+  p.max_blocks = left / 98 / (p.ahead * p.blocks) * (p.ahead * p.blocks);
+  return p;
+}
+// Where 16-byte piece `piece` of staged row `row` lies: piece ^ this.
+constexpr int tallRowSwizzle(int row_bytes, int row) {
+  return row_bytes >= 256 ? (row & 15) : (row_bytes >= 128 ? ((row >> 1) & 7) : ((row >> 2) & 3));
+}
+
+template <typename E, int Q, int C, int TR, typename SRC>
+__global__ __launch_bounds__(kTallThreads)
+    __attribute__((amdgpu_waves_per_eu(2 * tallPlan(Q * (int)sizeof(typename E::storage)).per_cu,
+                                       2 * tallPlan(Q * (int)sizeof(typename E::storage)).per_cu)))
+void gatherConvTall(const typename E::storage *A, uint32_t a_size, ConvRows rows, const typename E::storage *packedW,
+                    SRC source, int R, int K, typename E::storage *result) {
+  typedef typename E::vec8 vec8;
+  typedef typename E::storage S;
+  constexpr int ROW_BYTES = Q * (int)sizeof(S);
+  constexpr TallPlan PLAN = tallPlan(ROW_BYTES);
+  constexpr int NT = kTallThreads;
+  constexpr int FW = kTallWaves;
+  constexpr int NB = C / 16 / kTallWaves;    // column blocks of a multiplying wave
+  constexpr int KB = ROW_BYTES / 64;         // operand fragments per row
+  constexpr int G = PLAN.blocks;
+  constexpr int U = PLAN.ahead;
+  constexpr int MAXB = PLAN.max_blocks;
+  constexpr int ROUND = G * 16 * ROW_BYTES;
+  constexpr int NI = ROUND / 1024 / FW;      // loads of a fetching wave per round
+  constexpr int PPR = ROW_BYTES / 16;
+  constexpr int GROUPS = C / 16;
+  constexpr int ALLW = NT / 64;
+  constexpr int NSEG = TR / 64;
+  constexpr int KPW = 32 / ALLW;             // offsets of a row map a wave reads at once
+  static_assert(ROUND % (1024 * FW) == 0 && NI >= 1, "a round splits evenly over the fetching waves");
+  static_assert(MAXB >= TR / 16, "an offset's pairs fit");
+
+  __shared__ __attribute__((aligned(1024))) char s_stage[2 * ROUND];
+  __shared__ __attribute__((aligned(256))) float s_acc[(TR + 1) * C];
+  __shared__ uint32_t s_src[MAXB * 16];  // where the gathered row begins; kNoRow: no pair
+  __shared__ u16 s_row[MAXB * 16];       // result row in the tile; TR: no pair
+  __shared__ u16 s_k[MAXB];              // offset of a block
+  __shared__ int s_count[SRC::kSegments ? 1 : KPW * ALLW];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool fetcher = wave >= kTallWaves;
+  const int tiles_per_xcd = gridDim.x >> 3;  // neighbouring tiles on one XCD, as above
+  const int tile = (blockIdx.x & 7) * tiles_per_xcd + (blockIdx.x >> 3);
+  const int r0 = tile * TR;
+  if constexpr (!SRC::kSegments) {
+    if (notWanted(source.run_if)) return;
+  }
+  if (r0 >= R) {
+    if constexpr (!SRC::kSegments) {
+      if (tid == 0 && blockIdx.y == 0) source.filled[blockIdx.x] = 0;
+    }
+    return;
+  }
+  int slots = 0;  // filled map slots of this tile
+  // lane l: the piece of offset kc + l
+  int first = 0, count = 0;
+  auto look_up = [&](int kc) {
+    if constexpr (SRC::kSegments) {
+      const int k_mine = kc + lane < K ? kc + lane : K - 1;
+      const int32_t *const cut = source.cuts + (size_t)k_mine * source.cut_stride + tile;
+      first = cut[0];
+      count = cut[1] - first;
+      count = count < 0 ? 0 : (count > TR ? TR : count);
+      if (kc + lane >= K || source.counts.n[k_mine] <= 0) count = 0;
+    }
+  };
+  // (requested ahead of the clearing, which takes as long)
+  bool in_order = true;
+  unsigned long long verdict = 0;
+  if constexpr (SRC::kSegments) verdict = *source.verdict;
+  look_up(0);
+  for (int i = tid; i < (TR + 1) * C / 4; i += NT) reinterpret_cast<float4v *>(s_acc)[i] = float4v{0.f, 0.f, 0.f, 0.f};
+  const int col_group = blockIdx.y;
+  if constexpr (SRC::kSegments) {
+    in_order = verdict != source.ticket;
+    if (!in_order && source.leave_if_unordered) return;
+    if (!in_order) {
+      __syncthreads();
+      const int columns = rows.c - col_group * C;
+      scanAllPairsForTile<E, NT>(A, rows.q, rows.row_bytes, source, K, r0, r0 + TR < R ? r0 + TR : R,
+                                 columns < C ? columns : C, col_group * C, s_acc, C);
+    }
+  }
+
+  const int pair = lane & 15;
+  const int quad = lane >> 4;
+  const __amdgpu_buffer_rsrc_t a_rows = rowsBuffer(A, a_size);
+  const char *const b_base = reinterpret_cast<const char *>(packedW) +
+                             ((size_t)(col_group * GROUPS + (wave & 3) * NB) * KB * 64 + lane) * 16;
+  const uint32_t bytes_per_offset = (uint32_t)(rows.c_padded / 16) * KB * 1024;  // packed W[k]
+
+  for (int kc = 0; kc < (in_order ? K : 0);) {
+    // A: the entries of as many offsets as the lists have room for
+    if (kc > 0) look_up(kc);
+    // (row map: its slots of kMapOffsets offsets, wave w those of the offsets w, w + ALLW, ...)
+    int partners[KPW][NSEG];
+    if constexpr (!SRC::kSegments) {
+#pragma unroll
+      for (int j = 0; j < KPW; ++j) {
+        const int k = kc + wave + j * ALLW < K ? kc + wave + j * ALLW : K - 1;
+#pragma unroll
+        for (int seg = 0; seg < NSEG; ++seg) {
+          const int r = r0 + seg * 64 + lane;
+          partners[j][seg] = source.map[(size_t)k * R + (r < R ? r : R - 1)];
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < KPW; ++j)
+#pragma unroll
+        for (int seg = 0; seg < NSEG; ++seg) asm volatile("" : "+v"(partners[j][seg]));
+#pragma unroll
+      for (int j = 0; j < KPW; ++j) {
+        int c = 0;
+#pragma unroll
+        for (int seg = 0; seg < NSEG; ++seg) {
+          if (kc + wave + j * ALLW >= K || r0 + seg * 64 + lane >= R) partners[j][seg] = -1;
+          c += __popcll(__ballot(partners[j][seg] >= 0));
+        }
+        if (lane == 0) s_count[wave + j * ALLW] = c;
+      }
+      __syncthreads();
+      count = lane < KPW * ALLW ? s_count[lane < KPW * ALLW ? lane : 0] : 0;
+    }
+    constexpr int kAtOnce = SRC::kSegments ? 64 : KPW * ALLW;  // offsets looked up
+    const int blk_end = waveInclusiveScan((count + 15) >> 4);
+    const int taken = __popcll(__ballot(blk_end <= MAXB && lane < kAtOnce && kc + lane < K));
+    const int n_blocks = __builtin_amdgcn_readlane(blk_end, taken - 1);
+    const int n_rounds = ((n_blocks + G - 1) / G + U - 1) / U * U;
+    const int blk_first = blk_end - ((count + 15) >> 4);
+    if constexpr (!SRC::kSegments) {
+      slots += __builtin_amdgcn_readlane(waveInclusiveScan(count), taken - 1);
+      // no pair, where none is written behind the next barrier
+      for (int e = tid; e < n_rounds * G * 16; e += NT) {
+        s_src[e] = kNoRow;
+        s_row[e] = (u16)TR;
+        if ((e & 15) == 0) s_k[e >> 4] = (u16)(kc + taken - 1);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < KPW; ++j) {
+        const int kk = wave + j * ALLW;
+        int at = __shfl(blk_first, kk, kWave) * 16;
+        const int last = __shfl(blk_end, kk, kWave);
+        if (kk >= taken) continue;
+        for (int b = at / 16 + lane; b < last; b += kWave) s_k[b] = (u16)(kc + kk);
+#pragma unroll
+        for (int seg = 0; seg < NSEG; ++seg) {
+          const unsigned long long m = __ballot(partners[j][seg] >= 0);
+          if (partners[j][seg] >= 0) {
+            const int e = at + __popcll(m & ((1ull << lane) - 1ull));
+            s_src[e] = (uint32_t)partners[j][seg] * (uint32_t)rows.row_bytes;
+            s_row[e] = (u16)(seg * 64 + lane);
+          }
+          at += __popcll(m);
+        }
+      }
+    } else {
+    // block b belongs to the first lane whose blocks end behind it
+    constexpr int PER = (MAXB * 16 + NT - 1) / NT;  // entries a thread
+    int own_row[PER], partner[PER], k_of[PER];
+    bool there[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int b = (tid + u * NT) >> 4;
+      int at = 0;
+#pragma unroll
+      for (int step = 32; step > 0; step >>= 1)
+        if (__shfl(blk_end, at + step - 1, kWave) <= b) at += step;
+      at = at < taken ? at : taken - 1;
+      const int i = (b - __shfl(blk_first, at, kWave)) * 16 + (lane & 15);
+      const int pairs_there = __shfl(count, at, kWave);  // (outside the condition: all lanes take part)
+      const bool live = b < n_blocks && i < pairs_there;
+      int p = __shfl(first, at, kWave) + (live ? i : 0);
+      p = p < 0 ? 0 : (p < source.L ? p : source.L - 1);
+      const int32_t *const list = source.pairs + (size_t)(kc + at) * 2 * source.L;
+      own_row[u] = list[(size_t)source.row_col * source.L + p];
+      partner[u] = list[(size_t)source.src_col * source.L + p];
+      there[u] = live;
+      k_of[u] = kc + at;
+    }
+#pragma unroll
+    for (int u = 0; u < PER; ++u) asm volatile("" : "+v"(own_row[u]), "+v"(partner[u]));
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int e = tid + u * NT;
+      if (e < MAXB * 16) {
+        s_src[e] = there[u] ? (uint32_t)partner[u] * (uint32_t)rows.row_bytes : kNoRow;
+        s_row[e] = there[u] ? (u16)((own_row[u] - r0) & (TR - 1)) : (u16)TR;
+        if ((lane & 15) == 0) s_k[e >> 4] = (u16)k_of[u];
+      }
+    }
+    }
+    kc += taken;
+    __syncthreads();
+    if (n_blocks == 0) continue;
+    // B
+    if (fetcher) {
+      const int ftid = tid - kTallWaves * 64;
+      u32x4 piece[U][NI];
+      auto request_round = [&](int round, u32x4 (&to)[NI]) {
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          const int slot = ftid + j * 64 * FW;
+          const uint32_t from = s_src[round * G * 16 + slot / PPR];
+          const uint32_t at = slot % PPR * 16 < rows.row_bytes ? (uint32_t)(slot % PPR * 16) : kNoRow;
+          to[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                a_rows, __builtin_elementwise_add_sat(from, at), 0, 0));
+        }
+      };
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        request_round(j, piece[j]);
+        asm volatile("" ::: "memory");  // (in this order: the loop below waits for the oldest)
+      }
+      for (int r = 0; r < n_rounds; r += U) {
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+          char *const stage = s_stage + ((r + j) & 1) * ROUND;
+#pragma unroll
+          for (int i = 0; i < NI; ++i) {
+            const int slot = ftid + i * 64 * FW;
+            const int row = slot / PPR;
+            *reinterpret_cast<u32x4 *>(stage + row * ROW_BYTES +
+                                       ((slot % PPR) ^ tallRowSwizzle(ROW_BYTES, row & 15)) * 16) = piece[j][i];
+          }
+          request_round(r + j + U < n_rounds ? r + j + U : n_rounds - 1, piece[j]);
+          ldsBarrier();  // round r + j is there, and nobody reads the round before any more
+        }
+      }
+    } else {
+      vec8 w[U][G][KB][NB];
+      // filters of a round whose blocks have the offsets ks
+      auto request_filters = [&](const int (&ks)[G], vec8 (&to)[G][KB][NB]) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const char *const bk = b_base + (size_t)__builtin_amdgcn_readfirstlane(ks[g]) * bytes_per_offset;
+#pragma unroll
+          for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) to[g][kb][nb] = *reinterpret_cast<const vec8 *>(bk + (nb * KB + kb) * 1024);
+        }
+      };
+      auto offsets_of = [&](int round, int (&ks)[G]) {
+        const int r = round < n_rounds ? round : n_rounds - 1;
+#pragma unroll
+        for (int g = 0; g < G; ++g) ks[g] = s_k[r * G + g];
+      };
+      auto rows_of = [&](int round, int (&own)[G]) {
+        const int r = round < n_rounds ? round : n_rounds - 1;
+#pragma unroll
+        for (int g = 0; g < G; ++g) own[g] = s_row[(r * G + g) * 16 + pair];
+      };
+      int ks[G], own[G], own_next[G];
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        offsets_of(j, ks);
+        request_filters(ks, w[j]);
+        asm volatile("" ::: "memory");
+      }
+      offsets_of(U, ks);
+      float4v prod[G][NB];
+      // the products of the round before go to their sums while this round's rows are read from LDS:
+      // one block after the other, since blocks of different offsets may meet in a row
+      auto add_block = [&](int g) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          // lane holds result columns 4 * piece + (0..3) of its pair
+          const int piece = (wave * NB + nb) * 4 + quad;
+          float4v *const sum = reinterpret_cast<float4v *>(s_acc) + own[g] * (C / 4) + (piece ^ (own[g] & 15));
+          float4v old = *sum;
+          old += prod[g][nb];
+          *sum = old;
+        }
+      };
+#pragma unroll
+      for (int g = 0; g < G; ++g) own[g] = TR;
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) prod[g][nb] = float4v{0.f, 0.f, 0.f, 0.f};
+      rows_of(0, own_next);
+      for (int r = 0; r < n_rounds; r += U) {
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+          ldsBarrier();
+          const char *const stage = s_stage + ((r + j) & 1) * ROUND;
+          vec8 a[G][KB];
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+              a[g][kb] = *reinterpret_cast<const vec8 *>(stage + (g * 16 + pair) * ROW_BYTES +
+                                                         (((kb * 4 + quad) ^ tallRowSwizzle(ROW_BYTES, pair)) * 16));
+            add_block(g);
+          }
+#pragma unroll
+          for (int g = 0; g < G; ++g) own[g] = own_next[g];
+          rows_of(r + j + 1, own_next);
+#pragma unroll
+          for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+              prod[g][nb] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+              for (int kb = 0; kb < KB; ++kb) prod[g][nb] = E::mfma(w[j][g][kb][nb], a[g][kb], prod[g][nb]);
+            }
+          request_filters(ks, w[j]);
+          offsets_of(r + j + U + 1, ks);
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g) add_block(g);
+    }
+    __syncthreads();
+  }
+  __syncthreads();
+  constexpr int VALS = 16 / (int)sizeof(S);
+  for (int i = tid; i < TR * C / VALS; i += NT) {
+    const int rr = i / (C / VALS);
+    const int c0 = (i % (C / VALS)) * VALS;
+    if (r0 + rr >= R) break;
+    S tmp[VALS];
+#pragma unroll
+    for (int q = 0; q < VALS / 4; ++q) {
+      const int piece = c0 / 4 + q;
+      const float4v v = reinterpret_cast<const float4v *>(s_acc)[rr * (C / 4) + (in_order ? piece ^ (rr & 15) : piece)];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) E::store(&tmp[q * 4 + e], v[e]);
+    }
+    storeColumns<E>(result + (size_t)(r0 + rr) * rows.c, col_group * C + c0, rows.c, tmp);
+  }
+  if constexpr (!SRC::kSegments) {
+    if (tid == 0 && blockIdx.y == 0) source.filled[blockIdx.x] = slots;
+  }
+}
+
 // ---- MFMA gather convolution, one free-running wavefront per tile ---------------------
 //
 // The kernel above spends a tile's life waiting: cut positions, then pairs, then
@@ -1321,7 +1706,6 @@ __global__ __launch_bounds__(64) void gatherConvWave(
 // walk and multiplied by itself, its products added to the rows that have a partner there only.
 constexpr int kDenseChunk = 27;      // offsets whose row-map slice is resident in LDS at once
 constexpr int kDenseMapBatch = 14;   // loads in flight per thread while a tile's row map is read
-constexpr uint32_t kNoRow = 0x80000000u;  // byte offset of a partner that is not there
 
 // How an instance splits its work, from what a CU has: 160 KiB of LDS and 512 registers a lane
 // and SIMD.  Short rows: as many workgroups as registers and LDS allow.  Rows above 128 bytes: one
@@ -1367,11 +1751,6 @@ constexpr int denseTileRows(int elem_bytes, int Q, int C) {
 // width apart, and the 16 rows whose same piece is read at once have to meet all banks.
 constexpr int denseRowSwizzle(int row_bytes, int row) {
   return row_bytes >= 256 ? (row & 15) : ((row >> 1) & 7);
-}
-
-// The gathered tensor as a buffer of `bytes` (below 2^31) for loads that answer zero behind it.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rowsBuffer(const void *base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
 }
 
 template <typename E, int Q, int C, typename SRC>
@@ -3097,6 +3476,41 @@ void launchWave(const LaunchCtx &lc, int q_padded, const void *A, const ConvRows
 #undef WAVE_CASE
 }
 
+// Workgroups along x of the tall-tile kernel: tiles rounded up to a multiple of the XCD count.
+int tallGridX(int R, int tile_rows) { return ((R + tile_rows - 1) / tile_rows + 7) / 8 * 8; }
+
+template <typename E, int Q, typename SRC>
+void launchTallInstance(const LaunchCtx &lc, const void *A, uint32_t a_size, const ConvRows &rows, const void *packed,
+                        const SRC &source, int R, int K, void *result) {
+  constexpr int TR = tallRows(Q * (int)sizeof(typename E::storage));
+  const dim3 grid(tallGridX(R, TR), (rows.c + kTallCols - 1) / kTallCols);
+  lc.begin("gatherConvTall");
+  gatherConvTall<E, Q, kTallCols, TR, SRC><<<grid, kTallThreads, 0, lc.stream>>>(
+      static_cast<const typename E::storage *>(A), a_size, rows, static_cast<const typename E::storage *>(packed), source,
+      R, K, static_cast<typename E::storage *>(result));
+  lc.end();
+}
+
+// Channels of the instance for rows of q_padded channels (16 channels of a 2-byte type are half a fragment,
+// packed like a whole one).
+int tallQ(ElemType t, int q_padded) { return t != ElemType::kFloat && q_padded < 32 ? 32 : q_padded; }
+
+template <typename E, typename SRC>
+void launchTall(const LaunchCtx &lc, int q, const void *A, int n_src, const ConvRows &rows, const void *packed,
+                const SRC &source, int R, int K, void *result) {
+  const uint32_t a_size = (uint32_t)n_src * (uint32_t)rows.row_bytes;
+  switch (q) {
+    case 16:
+      if constexpr (std::is_same<E, FloatElem>::value)
+        launchTallInstance<E, 16, SRC>(lc, A, a_size, rows, packed, source, R, K, result);
+      break;
+    case 32: launchTallInstance<E, 32, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break;
+    case 64: launchTallInstance<E, 64, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break;
+    case 128: launchTallInstance<E, 128, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break;
+    default: break;
+  }
+}
+
 bool useWaveKernel(const LaunchCtx &lc, ElemType t, int Q, int C) {
   if (lc.choices.wave_per_tile == 0) return false;
   return waveKernelShape((int)elemSize(t), Q, C);
@@ -3108,6 +3522,34 @@ bool denseShapeOk(const ConvProblem &p, const GatherDims &d) {
   // (fp32 rows of more than 64 channels leave no room for two row groups a wave)
   if (p.dtype == ElemType::kFloat && d.Q > 64) return false;
   return (uint64_t)d.n_src * (uint64_t)paddedRowBytes(p.dtype, d.Q) < (uint64_t)kNoRow;
+}
+
+bool useTallKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d, bool lists) {
+  // (rows are addressed with 32-bit byte offsets; results of up to 32 columns have kernels of their own)
+  if (d.c_padded < 64 || (uint64_t)d.n_src * (uint64_t)paddedRowBytes(p.dtype, d.Q) >= (uint64_t)kNoRow) return false;
+  if (lc.choices.tall_tiles >= 0) return lc.choices.tall_tiles == 1;
+  // What a tile of 256 rows saves is filters (one for the pairs of 256 rows instead of 128) and the second,
+  // partly filled round of tiles; what it costs is that a CU's two tiles are long chains, so few rows
+  // leave CUs idle, and that many pairs a tile do not fit its lists at once.  us of gatherConvMfma
+  // against this kernel, 3x3x3 unless noted:
+  //   fp16  64 -> 64, rows strewn              8 k 11/11,  60 k 13.6/13.4, 200 k 37/28;  5x5x5 60 k 31/20, 200 k 110/59
+  //        128 -> 128, in boxes               12 k 17/18,  60 k 42/29,     200 k 149/104; 5x5x5 200 k 506/311
+  //         64 -> 64, strided, 97 k rows of a scene, 0.196 filled: 61/64; 36 k, 0.204: 29/41
+  //   fp32  64 -> 128, strided, strewn         60 k 180/92, 120 k 331/158; 64 -> 64, 12 k 15/17, 60 k 23/22
+  //        128 -> 128 (tiles of 512 rows)      60 k 133/91 in boxes, 12 k 42/56; 128 -> 64 with one pair a row,
+  //                                            150 k rows: 62/78
+  //   row map, fp16 64 -> 64 150 k 1.2 times as fast, 30 k 0.9; 5x5x5 (whose map is read twice) 150 k 0.85
+  double pairs = 0;
+  for (int k = 0; k < p.K; ++k) pairs += (double)p.indice_num[k];
+  const double fill = pairs / ((double)d.R * p.K);
+  const double work = (double)d.R * (d.c_padded / 64);
+  if (fill >= (p.K <= 8 ? 0.25 : 0.16)) return false;
+  const bool long_rows = d.q_padded * (int)elemSize(p.dtype) > 256;
+  if (lists) {
+    if (long_rows) return work >= 85000 && pairs >= 1.1 * d.R;
+    return p.K > 32 || work >= 45000;
+  }
+  return !long_rows && p.K <= 32 && d.q_padded >= 64 && work >= (d.c_padded == 128 ? 50000 : 80000);
 }
 
 bool useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d) {
@@ -3263,11 +3705,14 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
   const bool speculate = p.list_trust == ListTrust::kUnknown && single_chunk && lc.choices.lists_on_trust != 0;
   const bool lists = use_mfma && listsUsable(p, d) && (p.list_trust == ListTrust::kInOrder || speculate);
   const bool dense = use_mfma && useDenseKernel(lc, p, d);
+  const bool tall = use_mfma && !dense && useTallKernel(lc, p, d, lists);
+  const int tall_q = tallQ(p.dtype, d.q_padded);
   if (lists) {
     // Pair lists in order (as far as the caller knows: the first kernel checks): the
     // gather kernel reads them cut by tile, no row map.
     const int tile_cols = dense ? d.c_padded : mfmaTileCols(p, d);
-    const int tile_rows = dense ? denseTileRows((int)sizeof(S), d.q_padded, d.c_padded) : mfmaTileRows(tile_cols);
+    const int tile_rows = dense ? denseTileRows((int)sizeof(S), d.q_padded, d.c_padded)
+                                : (tall ? tallRows(tall_q * (int)sizeof(S)) : mfmaTileRows(tile_cols));
     int tile_shift = 0;
     while ((1 << tile_shift) < tile_rows) ++tile_shift;
     const int n_tiles = (d.R + tile_rows - 1) / tile_rows;
@@ -3303,6 +3748,8 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     src.counts = inl;
     if (dense)
       launchDense<E, SegmentSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, src, d.R, p.K, result);
+    else if (tall)
+      launchTall<E, SegmentSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, src, d.R, p.K, result);
     else if (tile_cols == d.c_padded && useWaveKernel(lc, p.dtype, d.q_padded, d.c_padded))
       launchWave<E>(lc, d.q_padded, rows_from, rows_of, ws.packed, src, d.R, p.K, result);
     else
@@ -3343,6 +3790,9 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
       if (dense) {
         n_filled = denseGridX(rows, denseTileRows((int)sizeof(S), d.q_padded, d.c_padded));
         launchDense<E, MapSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K, result_rows);
+      } else if (tall) {
+        n_filled = tallGridX(rows, tallRows(tall_q * (int)sizeof(S)));
+        launchTall<E, MapSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K, result_rows);
       } else {
         n_filled = mfmaGridX(rows, tile_cols);
         launchMfma<E, MapSource>(lc, d.q_padded, tile_cols, rows_from, rows_of, ws.packed, map, rows, p.K, result_rows);
