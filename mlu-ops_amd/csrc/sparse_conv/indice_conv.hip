@@ -29,6 +29,7 @@
 // where that filter is not finite.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <type_traits>
 
@@ -2620,7 +2621,8 @@ __global__ __launch_bounds__(256) void reduceFilterPartials(const float *partial
 // offset in slice order (no float atomics, the same bits on every run).
 struct SliceTable {
   int n[kMaxInlineK];      // pairs of the offset
-  int first[kMaxInlineK];  // partial tiles in front of the offset's first slice
+  int first[kMaxInlineK];  // partial tiles in front of the offset's first one
+  int tiles[kMaxInlineK];  // partial tiles of the offset
 };
 
 constexpr int kFilterStepPairs = 64;     // pairs multiplied per barrier
@@ -2631,6 +2633,8 @@ constexpr int kFilterMaxSlices = 1024;   // about four workgroups per CU
 // 149 at 1024; the 27-offset network layers: 183 -> 165 us at 128 channels, 89 -> 77 at 64).
 constexpr int kFilterMaxSlicesManyOffsets = 768;
 constexpr int kFilterFewOffsets = 32;
+constexpr int kFilterWalkChunk = 256;  // pairs a walk takes at a time
+constexpr int kFilterShares = 8;       // shares of every list: the XCDs
 
 // The order in which the workgroups take the slices: by the share of its offset's list that
 // lies in front of a slice, so that the workgroups running at one time are at about the same
@@ -2670,6 +2674,78 @@ __device__ __forceinline__ SlicePlace sliceOfWorkgroup(const SliceOrder &order, 
   at.k = s_place[0];
   at.slice = s_place[1];
   return at;
+}
+
+struct FilterWalk {
+  int k, share, walker;
+};
+
+// Walks: with many pairs slices are so long that the workgroups of an XCD are spread over far more rows than
+// its L2 holds, and a row comes from memory again for most of its offsets (248 636 rows, 2.85 M pairs, 128 x 128
+// channels: 704 MB for tensors of 127 MB, at the rate a copy reaches).  Every list is then cut into
+// `shares` equal shares, share s walked by workgroups of XCD s % 8: an offset's `walkers` take its chunks of
+// kFilterWalkChunk pairs in turn, so that all workgroups of the XCD go through the share's rows together.
+// 163 -> 130 us there, 64 x 64 channels 74 -> 65, 32 x 32 53 -> 50.
+// `order` names the offsets of one share's workgroups.
+__device__ __forceinline__ FilterWalk walkOfWorkgroup(const SliceOrder &order, int per_share, int shares) {
+  __shared__ int s_place[2];
+  const int i = (int)blockIdx.x >> 3;
+  const int entry = i % per_share;
+  if (threadIdx.x < 64) {
+    const int k = order.offset[entry];
+    int earlier = 0;
+    for (int j = threadIdx.x; j < entry; j += 64) earlier += order.offset[j] == k;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) earlier += __shfl_xor(earlier, d, kWave);
+    if (threadIdx.x == 0) {
+      s_place[0] = k;
+      s_place[1] = earlier;
+    }
+  }
+  __syncthreads();
+  return FilterWalk{s_place[0], (i / per_share) * 8 + ((int)blockIdx.x & 7), s_place[1]};
+}
+
+// The pairs of a workgroup: pair t of `length` (whole steps of kFilterStepPairs) at position at(t) of the
+// offset's list, if that lies in front of `end`.
+struct FilterRun {
+  int k;     // -1: nothing to do
+  int tile;  // partial tile the products go to
+  int begin, end, stride, length;
+  __device__ __forceinline__ int at(int t) const {
+    return begin + t / kFilterWalkChunk * stride + t % kFilterWalkChunk;
+  }
+};
+
+__device__ __forceinline__ FilterRun runOfWorkgroup(const SliceTable &tab, const SliceOrder &order, int entries,
+                                                    int slice_len, int shares) {
+  FilterRun run;
+  if (shares > 0) {
+    const FilterWalk walk = walkOfWorkgroup(order, entries, shares);
+    const int n = tab.n[walk.k], walkers = tab.tiles[walk.k] / shares;
+    run.k = walk.k;
+    run.tile = tab.first[walk.k] + walk.share * walkers + walk.walker;
+    run.begin = (int)((long long)n * walk.share / shares) + walk.walker * kFilterWalkChunk;
+    run.end = (int)((long long)n * (walk.share + 1) / shares);
+    run.stride = walkers * kFilterWalkChunk;
+  } else {
+    const SlicePlace at = sliceOfWorkgroup(order, entries);
+    run.k = at.k;
+    if (at.k < 0) return run;
+    const int n = tab.n[at.k];
+    run.tile = tab.first[at.k] + at.slice;
+    run.begin = at.slice * slice_len;
+    run.end = run.begin + slice_len < n ? run.begin + slice_len : n;
+    run.stride = kFilterWalkChunk;
+  }
+  run.length = 0;  // (a walk behind the end of a short share still stores its tile, of zeros)
+  if (run.begin < run.end) {
+    const int before = (run.end - run.begin - 1) / run.stride;  // chunks in front of the last one
+    const int last = run.end - (run.begin + before * run.stride);
+    run.length = before * kFilterWalkChunk + ((last < kFilterWalkChunk ? last : kFilterWalkChunk) + kFilterStepPairs - 1) /
+                                                 kFilterStepPairs * kFilterStepPairs;
+  }
+  return run;
 }
 
 // Both operands are needed with the pair index running along the MFMA's K
@@ -2717,7 +2793,7 @@ template <typename E, int CI, int CO, bool WHOLE>
 __global__ __launch_bounds__(256) void backwardFilterMfma(
     const typename E::storage *X, const typename E::storage *dY, FilterGradRows lengths, const int32_t *pairs, int L,
     int x_col, int n_in, int n_out, int K, SliceTable tab, SliceOrder order, int total_slices,
-    int slice_len, float *partial) {
+    int slice_len, int shares, float *partial) {
   typedef typename E::vec8 vec8;
   typedef typename E::storage S;
   constexpr int SP = kFilterStepPairs;
@@ -2741,13 +2817,9 @@ __global__ __launch_bounds__(256) void backwardFilterMfma(
   __shared__ int s_in[kFilterIndexChunk];
   __shared__ int s_out[kFilterIndexChunk];
 
-  const SlicePlace at = sliceOfWorkgroup(order, total_slices);
-  if (at.k < 0) return;
-  const int k = at.k;
-  const int n = tab.n[k];
-  const int p_begin = at.slice * slice_len;
-  if (p_begin >= n) return;
-  const int p_end = p_begin + slice_len < n ? p_begin + slice_len : n;
+  const FilterRun run = runOfWorkgroup(tab, order, total_slices, slice_len, shares);
+  if (run.k < 0) return;
+  const int k = run.k;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -2816,15 +2888,15 @@ __global__ __launch_bounds__(256) void backwardFilterMfma(
     }
   };
 
-  for (int c_begin = p_begin; c_begin < p_end; c_begin += kFilterIndexChunk) {
-    const int c_len = p_end - c_begin < kFilterIndexChunk ? p_end - c_begin : kFilterIndexChunk;
-    const int c_pad = (c_len + SP - 1) / SP * SP;
+  for (int c_begin = 0; c_begin < run.length; c_begin += kFilterIndexChunk) {
+    const int c_len = run.length - c_begin < kFilterIndexChunk ? run.length - c_begin : kFilterIndexChunk;
     __syncthreads();  // the previous chunk's indices are no longer read
-    for (int t = tid; t < c_pad; t += 256) {
+    for (int t = tid; t < c_len; t += 256) {
       int i = -1, o = -1;
-      if (t < c_len) {
-        i = in_col[c_begin + t];
-        o = out_col[c_begin + t];
+      const int p = run.at(c_begin + t);
+      if (p < run.end) {
+        i = in_col[p];
+        o = out_col[p];
         if ((unsigned)i >= (unsigned)n_in || (unsigned)o >= (unsigned)n_out) i = o = -1;
       }
       s_in[t] = i;
@@ -2832,11 +2904,11 @@ __global__ __launch_bounds__(256) void backwardFilterMfma(
     }
     __syncthreads();
     fetch_step(0);
-    for (int local = 0; local < c_pad; local += SP) {
+    for (int local = 0; local < c_len; local += SP) {
       __syncthreads();  // every wave has read the previous step's operands
       store_step();
       __syncthreads();
-      if (local + SP < c_pad) fetch_step(local + SP);
+      if (local + SP < c_len) fetch_step(local + SP);
 #pragma unroll
       for (int kb = 0; kb < SP / E::kChunk; ++kb) {
         vec8 bfr[COB];
@@ -2858,7 +2930,7 @@ __global__ __launch_bounds__(256) void backwardFilterMfma(
     }
   }
   // lane holds rows 4*(lane/16)+v, column lane%16 of every 16 x 16 block
-  float *tile = partial + (size_t)(tab.first[k] + at.slice) * CI * CO;
+  float *tile = partial + (size_t)run.tile * CI * CO;
 #pragma unroll
   for (int a = 0; a < CBW; ++a) {
     const int cb = wave + a * 4;
@@ -2896,7 +2968,7 @@ template <typename E, int CI, int CO, int SP, bool WHOLE>
 __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
     const typename E::storage *X, const typename E::storage *dY, FilterGradRows lengths, const int32_t *pairs, int L,
     int x_col, int n_in, int n_out, int K, SliceTable tab, SliceOrder order, int total_slices,
-    int slice_len, float *partial) {
+    int slice_len, int shares, float *partial) {
   typedef typename E::vec8 vec8;
   typedef typename E::storage S;
   typedef short v4i16 __attribute__((ext_vector_type(4)));
@@ -2905,7 +2977,7 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
   static_assert(CI % 32 == 0 && CO % 32 == 0 && CI <= 128 && CO <= 128, "two row and column blocks per wave pair");
   // two chunks of row indices: with 128 channels on both sides the buffers leave 16 KiB of
   // half a CU's LDS
-  constexpr int kIndexChunk = 512;
+  constexpr int kIndexChunk = kFilterWalkChunk;
   const FilterGradRows rows = WHOLE ? FilterGradRows{CI, CO} : lengths;
   constexpr int kChunkSteps = kIndexChunk / SP;
   constexpr int RBX = CI * 2, RBY = CO * 2;     // bytes per row
@@ -2919,13 +2991,9 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
   __shared__ int s_in[2][kIndexChunk];   // row indices of a chunk of pairs, and of the chunk after
   __shared__ int s_out[2][kIndexChunk];
 
-  const SlicePlace at = sliceOfWorkgroup(order, total_slices);
-  if (at.k < 0) return;
-  const int k = at.k;
-  const int n = tab.n[k];
-  const int p_begin = at.slice * slice_len;
-  if (p_begin >= n) return;
-  const int p_end = p_begin + slice_len < n ? p_begin + slice_len : n;
+  const FilterRun run = runOfWorkgroup(tab, order, total_slices, slice_len, shares);
+  if (run.k < 0) return;
+  const int k = run.k;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -3002,9 +3070,9 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
   auto fetch_indices = [&](int chunk) {
 #pragma unroll
     for (int u = 0; u < IPT; ++u) {
-      const int at = p_begin + chunk * kIndexChunk + u * 256 + tid;
+      const int at = run.at(chunk * kIndexChunk + u * 256 + tid);
       int i = -1, o = -1;
-      if (at < p_end) {
+      if (at < run.end) {
         i = in_col[at];
         o = out_col[at];
       }
@@ -3022,7 +3090,7 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
     }
   };
 
-  const int steps = (p_end - p_begin + SP - 1) / SP;
+  const int steps = run.length / SP;
   fetch_indices(0);
   store_indices(0);
   __syncthreads();
@@ -3063,14 +3131,14 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
     ldsBarrier();
   }
   // lane holds rows 4*(lane/16)+v, column lane%16 of every 16 x 16 block
-  float *tile = partial + (size_t)(tab.first[k] + at.slice) * CI * CO;
+  float *const sums = partial + (size_t)run.tile * CI * CO;
 #pragma unroll
   for (int a = 0; a < AB; ++a)
 #pragma unroll
     for (int b = 0; b < BB; ++b)
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        tile[(size_t)((wa * AB + a) * 16 + 4 * (lane >> 4) + v) * CO + (wb * BB + b) * 16 + (lane & 15)] =
+        sums[(size_t)((wa * AB + a) * 16 + 4 * (lane >> 4) + v) * CO + (wb * BB + b) * 16 + (lane & 15)] =
             acc[a][b][v];
 }
 
@@ -3091,7 +3159,7 @@ __global__ __launch_bounds__(64 * kSliceSumWaves) void sliceSum(const float *par
   const int lane = threadIdx.x & 63;
   const int g = threadIdx.x >> 6;
   const int e = (blockIdx.x * 64 + lane) * 4;  // tile_elems is a multiple of 256
-  const int slices = (tab.n[k] + slice_len - 1) / slice_len;
+  const int slices = tab.tiles[k];
   float4v acc[8];
 #pragma unroll
   for (int u = 0; u < 8; ++u) acc[u] = float4v{0.f, 0.f, 0.f, 0.f};
@@ -3154,7 +3222,7 @@ __global__ __launch_bounds__(64 * kSliceSumWaves) void sliceSumFlat(const float 
   const int chunk = blockIdx.x - grid.first[k];
   const int lane = threadIdx.x & 63;
   const int g = threadIdx.x >> 6;
-  const int slices = (tab.n[k] + slice_len - 1) / slice_len;
+  const int slices = tab.tiles[k];
   const float *tiles = partial + (size_t)tab.first[k] * tile_elems;
   if (slices <= kThinSlices) {
     const int e = ((chunk * W + g) * 64 + lane) * 4;
@@ -3888,16 +3956,40 @@ GradLayout gradLayout(const ConvProblem &p) {
   return g;
 }
 
+// Rows whose operands the backward filter can transpose with LDS reads.
+bool transposingReads(const LaunchCtx &lc, const ConvProblem &p) {
+  return p.dtype != ElemType::kFloat && p.Ci > 16 && p.Co > 16 && lc.choices.filter_stores != 1 &&
+         !rowsNeedPadding(p.dtype, p.Ci) && !rowsNeedPadding(p.dtype, p.Co);
+}
+
+// Workgroups of the walks (sliceOfWorkgroup), 0: slices.  As many as are resident at a time, so that all
+// of them are at about the same rows: 512 at 128 x 128 channels, 768 with 128 on one side, and from 1.5 M
+// pairs on, where a second round no longer shows, 1024.  Fewer pairs leave walks of a few steps.  us with the
+// sums, slices against walks of 512 / 768 / 1024 workgroups, scenes, 3x3x3, fp16:
+//   128 x 128   0.50 M pairs 44/44/-/54   0.72 M 69/64/-/70   2.0 M 129/103/-/110   2.85 M 180/145/-/146
+//    96 x 96    1.6 M 118/100/108/95      3.0 M 205/163/174/148
+//    64 x 128   0.57 M 36/36/36/39        0.78 M 53/43/41/46  2.0 M 87/109/79/74    3.0 M 111/159/110/94
+//    64 x 64    0.50 M 26/27/-/25         0.84 M 36/38/-/36   1.05 M 36/41/-/33     2.0 M 66/94/-/56
+//    32 x 32    0.50 M 20/22/-/19         0.84 M 28/31/-/25   2.0 M 56/76/-/45
+int filterWalkers(const ConvProblem &p, long long pairs) {
+  if (p.K > kFilterFewOffsets) return 0;
+  const int channels = paddedChannels(p.Ci) + paddedChannels(p.Co);
+  if (pairs < (channels == 256 ? 600000 : (channels >= 192 ? 700000 : 800000))) return 0;
+  int want = kFilterMaxSlices;
+  if (pairs < 1500000 && channels >= 192) want = channels == 256 ? 512 : 768;
+  if (want > filterMaxSlices(p)) want = filterMaxSlices(p);  // (a capped workspace)
+  return want / kFilterShares < p.K ? 0 : want;
+}
+
 template <typename E, int CI, int CO>
 void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const SliceTable &tab,
-                              const SliceOrder &order, int slice_len, int total_slices, float *partial, const void *features,
+                              const SliceOrder &order, int slice_len, int shares, int total_slices, float *partial, const void *features,
                               const void *output_grad, void *filters_grad) {
   typedef typename E::storage S;
   constexpr bool kTransposingShape = sizeof(S) == 2 && CI >= 32 && CO >= 32;
-  const bool transposing = kTransposingShape && lc.choices.filter_stores != 1 &&
-                           !rowsNeedPadding(p.dtype, p.Ci) && !rowsNeedPadding(p.dtype, p.Co);
+  const bool transposing = kTransposingShape && transposingReads(lc, p);
   const FilterGradRows rows = {p.Ci, p.Co};
-  const int grid = (total_slices + 7) / 8 * 8;
+  const int grid = shares > 0 ? shares * total_slices : (total_slices + 7) / 8 * 8;
   lc.begin(transposing ? "backwardFilterMfmaTr" : "backwardFilterMfma");
   if (total_slices > 0) {
     const bool whole = p.Ci == CI && p.Co == CO;
@@ -3910,15 +4002,20 @@ void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const S
       // share a CU then, which pays when the slices are long (network 64 x 64: 101 -> 88 us;
       // on slices of a few steps the shorter steps only add barriers: config 4 23.7 -> 25.3 us).
       const bool short_steps = CI + CO < 256 && slice_len >= 2048;
-      if (transposing && whole)
-        kernel = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32, true> : backwardFilterMfmaTr<E, CI, CO, 64, true>;
-      else if (transposing)
-        kernel = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32, false> : backwardFilterMfmaTr<E, CI, CO, 64, false>;
+      auto tr = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32, false> : backwardFilterMfmaTr<E, CI, CO, 64, false>;
+      if (whole)
+        tr = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32, true> : backwardFilterMfmaTr<E, CI, CO, 64, true>;
+      if (transposing)
+        tr<<<grid, 256, 0, lc.stream>>>(
+            static_cast<const S *>(features), static_cast<const S *>(output_grad), rows, p.indice_pairs, p.L,
+            p.inverse ? 1 : 0, p.inverse ? p.num_out : p.L, p.inverse ? p.L : p.num_out, p.K, tab, order,
+            total_slices, slice_len, shares, partial);
     }
-    kernel<<<grid, 256, 0, lc.stream>>>(
-        static_cast<const S *>(features), static_cast<const S *>(output_grad), rows, p.indice_pairs, p.L,
-        p.inverse ? 1 : 0, p.inverse ? p.num_out : p.L, p.inverse ? p.L : p.num_out, p.K, tab, order,
-        total_slices, slice_len, partial);
+    if (!transposing)
+      kernel<<<grid, 256, 0, lc.stream>>>(
+          static_cast<const S *>(features), static_cast<const S *>(output_grad), rows, p.indice_pairs, p.L,
+          p.inverse ? 1 : 0, p.inverse ? p.num_out : p.L, p.inverse ? p.L : p.num_out, p.K, tab, order,
+          total_slices, slice_len, shares, partial);
   }
   lc.end();
   // Many offsets of few slices each: the flat grid, on which such an offset takes a
@@ -3927,7 +4024,7 @@ void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const S
   SumGrid sg;
   int blocks = 0;
   for (int k = 0; k < p.K; ++k) {
-    const int sl = (tab.n[k] + slice_len - 1) / slice_len;
+    const int sl = tab.tiles[k];
     sg.first[k] = blocks;
     blocks += sl <= kThinSlices ? (kChunks + kSliceSumWaves - 1) / kSliceSumWaves : kChunks;
   }
@@ -3945,13 +4042,13 @@ void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const S
 
 template <typename E, int CI>
 void launchFilterMfmaByCo(const LaunchCtx &lc, const ConvProblem &p, const SliceTable &tab,
-                          const SliceOrder &order, int slice_len, int total_slices, float *partial, const void *features,
+                          const SliceOrder &order, int slice_len, int shares, int total_slices, float *partial, const void *features,
                           const void *output_grad, void *filters_grad) {
   switch (paddedChannels(p.Co)) {
-    case 16: launchFilterMfmaInstance<E, CI, 16>(lc, p, tab, order, slice_len, total_slices, partial, features, output_grad, filters_grad); break;
-    case 32: launchFilterMfmaInstance<E, CI, 32>(lc, p, tab, order, slice_len, total_slices, partial, features, output_grad, filters_grad); break;
-    case 64: launchFilterMfmaInstance<E, CI, 64>(lc, p, tab, order, slice_len, total_slices, partial, features, output_grad, filters_grad); break;
-    case 128: launchFilterMfmaInstance<E, CI, 128>(lc, p, tab, order, slice_len, total_slices, partial, features, output_grad, filters_grad); break;
+    case 16: launchFilterMfmaInstance<E, CI, 16>(lc, p, tab, order, slice_len, shares, total_slices, partial, features, output_grad, filters_grad); break;
+    case 32: launchFilterMfmaInstance<E, CI, 32>(lc, p, tab, order, slice_len, shares, total_slices, partial, features, output_grad, filters_grad); break;
+    case 64: launchFilterMfmaInstance<E, CI, 64>(lc, p, tab, order, slice_len, shares, total_slices, partial, features, output_grad, filters_grad); break;
+    case 128: launchFilterMfmaInstance<E, CI, 128>(lc, p, tab, order, slice_len, shares, total_slices, partial, features, output_grad, filters_grad); break;
     default: break;
   }
 }
@@ -3979,35 +4076,58 @@ void launchFilterMfma(const LaunchCtx &lc, const ConvProblem &p, const FilterGra
     // 128, 400 000 pairs: 56 -> 46 us at 1024; config 2, 32 x 32, 205 000 pairs: 22.5 -> 19 us at 512).
     const int least = paddedChannels(p.Ci) * paddedChannels(p.Co) >= 128 * 128 ? 1024 : 512;
     if (slice_len < least) slice_len = least;
+    // Walks instead of slices, and the workgroups an offset's share of its list is walked by: one each,
+    // the others to the offsets whose walks are longest.
+    int walkers[kMaxInlineK];
+    const int per_share = filterWalkers(p, total) / kFilterShares;
+    const int shares = per_share > 0 ? kFilterShares : 0;
+    for (int k = 0; k < p.K; ++k) walkers[k] = inl.n[k] > 0 ? 1 : 0;
+    for (int left = per_share - p.K; left > 0; --left) {
+      int longest = 0;
+      for (int k = 1; k < p.K; ++k)
+        if ((long long)inl.n[k] * walkers[longest] > (long long)inl.n[longest] * walkers[k]) longest = k;
+      ++walkers[longest];
+    }
     int first = 0;
     for (int k = 0; k < kMaxInlineK; ++k) {
       const int n = k < p.K ? inl.n[k] : 0;
-      const int slices = (n + slice_len - 1) / slice_len;
       tab.n[k] = n;
       tab.first[k] = first;
-      first += slices;
+      tab.tiles[k] = shares == 0 ? (n + slice_len - 1) / slice_len : (k < p.K ? walkers[k] * shares : 0);
+      first += tab.tiles[k];
     }
-    // slices in the order of the share of their offset's list in front of them, in `steps`
-    // steps of that share (as many as the longest list has slices)
+    const int entries = shares > 0 ? first / shares : first;
     SliceOrder order;
-    int steps = 1, next[kMaxInlineK], count[kMaxInlineK];
-    for (int k = 0; k < p.K; ++k) {
-      next[k] = 0;
-      count[k] = (tab.n[k] + slice_len - 1) / slice_len;
-      if (count[k] > steps) steps = count[k];
-    }
     int placed = 0;
-    for (int t = 0; t < steps; ++t)
-      for (int k = 0; k < p.K; ++k)
-        while (next[k] < count[k] && (long long)next[k] * steps < (long long)(t + 1) * count[k]) {
-          order.offset[placed++] = (uint8_t)k;
-          ++next[k];
-        }
+    if (shares > 0) {
+      // the longest walks of a share first
+      int by_length[kMaxInlineK];
+      for (int k = 0; k < p.K; ++k) by_length[k] = k;
+      std::stable_sort(by_length, by_length + p.K, [&](int a, int b) {
+        return (long long)inl.n[a] * walkers[b] > (long long)inl.n[b] * walkers[a];
+      });
+      for (int i = 0; i < p.K; ++i)
+        for (int w = 0; w < walkers[by_length[i]]; ++w) order.offset[placed++] = (uint8_t)by_length[i];
+    } else {
+      // slices in the order of the share of their offset's list in front of them, in `steps`
+      // steps of that share (as many as the longest list has slices)
+      int steps = 1, next[kMaxInlineK];
+      for (int k = 0; k < p.K; ++k) {
+        next[k] = 0;
+        if (tab.tiles[k] > steps) steps = tab.tiles[k];
+      }
+      for (int t = 0; t < steps; ++t)
+        for (int k = 0; k < p.K; ++k)
+          while (next[k] < tab.tiles[k] && (long long)next[k] * steps < (long long)(t + 1) * tab.tiles[k]) {
+            order.offset[placed++] = (uint8_t)k;
+            ++next[k];
+          }
+    }
     switch (paddedChannels(p.Ci)) {
-      case 16: launchFilterMfmaByCo<E, 16>(lc, p, tab, order, slice_len, first, ws.partial, features, output_grad, filters_grad); break;
-      case 32: launchFilterMfmaByCo<E, 32>(lc, p, tab, order, slice_len, first, ws.partial, features, output_grad, filters_grad); break;
-      case 64: launchFilterMfmaByCo<E, 64>(lc, p, tab, order, slice_len, first, ws.partial, features, output_grad, filters_grad); break;
-      case 128: launchFilterMfmaByCo<E, 128>(lc, p, tab, order, slice_len, first, ws.partial, features, output_grad, filters_grad); break;
+      case 16: launchFilterMfmaByCo<E, 16>(lc, p, tab, order, slice_len, shares, entries, ws.partial, features, output_grad, filters_grad); break;
+      case 32: launchFilterMfmaByCo<E, 32>(lc, p, tab, order, slice_len, shares, entries, ws.partial, features, output_grad, filters_grad); break;
+      case 64: launchFilterMfmaByCo<E, 64>(lc, p, tab, order, slice_len, shares, entries, ws.partial, features, output_grad, filters_grad); break;
+      case 128: launchFilterMfmaByCo<E, 128>(lc, p, tab, order, slice_len, shares, entries, ws.partial, features, output_grad, filters_grad); break;
       default: break;
     }
   }
