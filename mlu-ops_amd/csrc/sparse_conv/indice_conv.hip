@@ -1700,7 +1700,7 @@ __global__ __launch_bounds__(64) void gatherConvWave(
 //   above (128 channels: 199 us [230]): the multiplies (130 us at the matrix cores' rate if
 //     nothing were skipped), and LDS, which carries the filter; rows through LDS as well measure
 //     217 us.  So rows go in operand order again, a chunk requested right behind its last use,
-//     in eight waves per filter copy, and a wave multiplies only the groups that have a row
+//     and a wave multiplies only the groups that have a row
 //     at the offset.
 // All of them multiply rows of zeros for the partners that are not there, which is nothing as long
 // as the filter is finite.  An offset whose filter is not (packFilter says so) is taken out of the
@@ -1709,8 +1709,14 @@ constexpr int kDenseChunk = 27;      // offsets whose row-map slice is resident 
 constexpr int kDenseMapBatch = 14;   // loads in flight per thread while a tile's row map is read
 
 // How an instance splits its work, from what a CU has: 160 KiB of LDS and 512 registers a lane
-// and SIMD.  Short rows: as many workgroups as registers and LDS allow.  Rows above 128 bytes: one
-// workgroup of eight waves, since two ring buffers of 64 KiB leave no room for a second.
+// and SIMD.  Short rows: as many workgroups as registers and LDS allow.  Rows above 128 bytes: two
+// workgroups of four waves, of which one multiplies while the other builds its row map and waits for its
+// first rows (8.7 of a tile's 42 us at 128 -> 128 channels, with one workgroup of eight waves a CU); the ring
+// then holds one offset a phase at 128 columns instead of two, and every 128 rows load the filters again,
+// which costs more from about 220 000 rows on (`wide`: eight waves).  us, eight waves against twice four:
+//   fp16 128 -> 128   8 k rows 47/39, 30 k 52/42, 80 k 96/87, 150 k 161/147, 250 k 214/222
+//        128 -> 64    8 k 32/27, 80 k 70/71, 150 k 135/114, 250 k 171/161;  128 -> 32  30 k 42/28, 250 k 158/147
+//   fp32  64 -> 64    8 k 105/68, 30 k 114/70, 80 k 182/162, 150 k 280/271;  64 -> 128  30 k 218/127, 150 k 549/537
 enum class DenseRows { kByPhase, kStaged, kInPlace };  // how rows reach the operand registers
 struct DensePlan {
   int waves;        // per workgroup
@@ -1719,7 +1725,7 @@ struct DensePlan {
   int offsets;      // offsets per phase
   DenseRows rows;
 };
-constexpr DensePlan densePlan(int elem_bytes, int Q, int C) {
+constexpr DensePlan densePlan(int elem_bytes, int Q, int C, bool wide) {
   const int nb = C / 16, kb = (Q * elem_bytes + 63) / 64;
   const int row_bytes = Q * elem_bytes;
   if (row_bytes <= 64) {
@@ -1736,17 +1742,17 @@ constexpr DensePlan densePlan(int elem_bytes, int Q, int C) {
     if (room < 4 * nb * kb * 1024) p.offsets = 1;
     return p;
   }
-  DensePlan p = {8, 2, 1, 2, DenseRows::kInPlace};
-  const int room = 160 * 1024 - kDenseChunk * p.waves * p.groups * 16 * 4 - 1024;
+  DensePlan p = wide ? DensePlan{8, 2, 1, 2, DenseRows::kInPlace} : DensePlan{4, 2, 2, 2, DenseRows::kInPlace};
+  const int room = 160 * 1024 / p.per_cu - kDenseChunk * p.waves * p.groups * 16 * 4 - 1024;
   if (room < 4 * nb * kb * 1024) p.offsets = 1;
   return p;
 }
-constexpr int denseWavesPerSimd(int elem_bytes, int Q, int C) {
-  const DensePlan p = densePlan(elem_bytes, Q, C);
+constexpr int denseWavesPerSimd(int elem_bytes, int Q, int C, bool wide) {
+  const DensePlan p = densePlan(elem_bytes, Q, C, wide);
   return p.waves * p.per_cu / 4;
 }
-constexpr int denseTileRows(int elem_bytes, int Q, int C) {
-  return densePlan(elem_bytes, Q, C).waves * densePlan(elem_bytes, Q, C).groups * 16;
+constexpr int denseTileRows(int elem_bytes, int Q, int C, bool wide) {
+  return densePlan(elem_bytes, Q, C, wide).waves * densePlan(elem_bytes, Q, C, wide).groups * 16;
 }
 // Where piece `piece` of a staged row lies in its row's bytes: rows lie a multiple of the bank
 // width apart, and the 16 rows whose same piece is read at once have to meet all banks.
@@ -1754,16 +1760,16 @@ constexpr int denseRowSwizzle(int row_bytes, int row) {
   return row_bytes >= 256 ? (row & 15) : ((row >> 1) & 7);
 }
 
-template <typename E, int Q, int C, typename SRC>
-__global__ __launch_bounds__(64 * densePlan((int)sizeof(typename E::storage), Q, C).waves)
-    __attribute__((amdgpu_waves_per_eu(denseWavesPerSimd((int)sizeof(typename E::storage), Q, C),
-                                       denseWavesPerSimd((int)sizeof(typename E::storage), Q, C))))
+template <typename E, int Q, int C, typename SRC, bool WIDE>
+__global__ __launch_bounds__(64 * densePlan((int)sizeof(typename E::storage), Q, C, WIDE).waves)
+    __attribute__((amdgpu_waves_per_eu(denseWavesPerSimd((int)sizeof(typename E::storage), Q, C, WIDE),
+                                       denseWavesPerSimd((int)sizeof(typename E::storage), Q, C, WIDE))))
 void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows conv,
                      const typename E::storage *packedW, SRC source, int R, int K,
                      typename E::storage *result) {
   typedef typename E::vec8 vec8;
   typedef typename E::storage S;
-  constexpr DensePlan PLAN = densePlan((int)sizeof(S), Q, C);
+  constexpr DensePlan PLAN = densePlan((int)sizeof(S), Q, C, WIDE);
   constexpr int WAVES = PLAN.waves;
   constexpr bool kStaged = PLAN.rows == DenseRows::kStaged;
   constexpr int G = PLAN.groups;
@@ -3667,23 +3673,37 @@ bool useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims 
   return sheets && d.q_padded <= 32 && fill >= 0.2;
 }
 
+// Whether the kernel takes its wide tiles (densePlan).
+bool denseWide(const ConvProblem &p, const GatherDims &d, int rows) {
+  return d.q_padded * (int)elemSize(p.dtype) > 128 && d.c_padded == 128 && rows >= 220000;
+}
+
 template <typename E, int Q, int C, typename SRC>
-void launchDenseInstance(const LaunchCtx &lc, const void *A, uint32_t a_size, const ConvRows &rows, const void *packed,
-                         const SRC &source, int R, int K, void *result) {
+void launchDenseInstance(const LaunchCtx &lc, bool wide, const void *A, uint32_t a_size, const ConvRows &rows,
+                         const void *packed, const SRC &source, int R, int K, void *result) {
   lc.begin("gatherConvDense");
   constexpr int kElem = (int)sizeof(typename E::storage);
-  gatherConvDense<E, Q, C, SRC><<<denseGridX(R, denseTileRows(kElem, Q, C)), 64 * densePlan(kElem, Q, C).waves, 0,
-                                  lc.stream>>>(
-      static_cast<const typename E::storage *>(A), a_size, rows, static_cast<const typename E::storage *>(packed),
-      source, R, K, static_cast<typename E::storage *>(result));
+  auto launch = [&](auto wide_tag) {
+    constexpr bool WIDE = decltype(wide_tag)::value;
+    gatherConvDense<E, Q, C, SRC, WIDE><<<denseGridX(R, denseTileRows(kElem, Q, C, WIDE)), 64 * densePlan(kElem, Q, C, WIDE).waves,
+                                          0, lc.stream>>>(
+        static_cast<const typename E::storage *>(A), a_size, rows, static_cast<const typename E::storage *>(packed),
+        source, R, K, static_cast<typename E::storage *>(result));
+  };
+  if constexpr (Q * kElem > 128 && C == 128) {
+    if (wide) launch(std::true_type());
+    else launch(std::false_type());
+  } else {
+    launch(std::false_type());
+  }
   lc.end();
 }
 
 template <typename E, typename SRC>
-void launchDense(const LaunchCtx &lc, int q_padded, const void *A, int n_src, const ConvRows &rows, const void *packed,
+void launchDense(const LaunchCtx &lc, int q_padded, bool wide, const void *A, int n_src, const ConvRows &rows, const void *packed,
                  const SRC &source, int R, int K, void *result) {
   const uint32_t a_size = (uint32_t)n_src * (uint32_t)rows.row_bytes;
-#define DENSE_INSTANCE(q, c) launchDenseInstance<E, q, c, SRC>(lc, A, a_size, rows, packed, source, R, K, result)
+#define DENSE_INSTANCE(q, c) launchDenseInstance<E, q, c, SRC>(lc, wide, A, a_size, rows, packed, source, R, K, result)
 #define DENSE_BY_C(q)                       \
   switch (rows.c_padded) {                  \
     case 16: DENSE_INSTANCE(q, 16); break;  \
@@ -3779,7 +3799,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     // Pair lists in order (as far as the caller knows: the first kernel checks): the
     // gather kernel reads them cut by tile, no row map.
     const int tile_cols = dense ? d.c_padded : mfmaTileCols(p, d);
-    const int tile_rows = dense ? denseTileRows((int)sizeof(S), d.q_padded, d.c_padded)
+    const int tile_rows = dense ? denseTileRows((int)sizeof(S), d.q_padded, d.c_padded, denseWide(p, d, d.R))
                                 : (tall ? tallRows(tall_q * (int)sizeof(S)) : mfmaTileRows(tile_cols));
     int tile_shift = 0;
     while ((1 << tile_shift) < tile_rows) ++tile_shift;
@@ -3815,7 +3835,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     src.sC = sC;
     src.counts = inl;
     if (dense)
-      launchDense<E, SegmentSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, src, d.R, p.K, result);
+      launchDense<E, SegmentSource>(lc, d.q_padded, denseWide(p, d, d.R), rows_from, d.n_src, rows_of, ws.packed, src, d.R, p.K, result);
     else if (tall)
       launchTall<E, SegmentSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, src, d.R, p.K, result);
     else if (tile_cols == d.c_padded && useWaveKernel(lc, p.dtype, d.q_padded, d.c_padded))
@@ -3856,8 +3876,9 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
       if (own_map) n_accepted = launchScatterRowMap(lc, p, d, ws, inl, max_count, row_base, rows, run_if);
       const MapSource map = {entries, ws.filled, run_if};
       if (dense) {
-        n_filled = denseGridX(rows, denseTileRows((int)sizeof(S), d.q_padded, d.c_padded));
-        launchDense<E, MapSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K, result_rows);
+        const bool wide = denseWide(p, d, rows);
+        n_filled = denseGridX(rows, denseTileRows((int)sizeof(S), d.q_padded, d.c_padded, wide));
+        launchDense<E, MapSource>(lc, d.q_padded, wide, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K, result_rows);
       } else if (tall) {
         n_filled = tallGridX(rows, tallRows(tall_q * (int)sizeof(S)));
         launchTall<E, MapSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K, result_rows);
