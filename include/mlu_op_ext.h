@@ -85,6 +85,12 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtSetSparseConvExtendedModes(mluOpHandle_t han
  * all but one of such pairs.  Off by default. */
 mluOpStatus_t MLUOP_WIN_API mluOpExtSetDistinctPairsPromise(mluOpHandle_t handle, int promised);
 
+/* Whether mluOpGetIndicePairs sets the slots of indice_pairs behind each offset's indice_num pairs to -1 (the
+ * default, and what the reference does).  0: it leaves them as they are, which saves most of a sparse
+ * rulebook's writes; for callers who, like the indice-convolution operators, read no further than
+ * indice_num.  Holds for the handle until changed. */
+mluOpStatus_t MLUOP_WIN_API mluOpExtSetPairTails(mluOpHandle_t handle, int fill);
+
 /* The pair counts of a rulebook on the host.  The convolution operators take indice_num as a host
  * array, so a caller has to bring the counts mluOpGetIndicePairs left in device memory over; a copy
  * waits for the whole queue.  The last kernel of a rulebook also stores them into pinned memory of

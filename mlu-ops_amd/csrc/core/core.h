@@ -43,6 +43,8 @@ struct mluOpContext {
   // (mluOpExtSetDistinctPairsPromise): forward and backward data then skip the
   // check that finds and adds such pairs.
   bool distinct_pairs_promised = false;
+  // rulebooks set the pair slots behind each offset's pairs to -1 (mluOpExtSetPairTails)
+  bool fill_pair_tails = true;
   // Row maps built by mluOpExtBuildRowMap with no pair lost, and the one announced for the
   // next forward / backward-data call (mluOpExtUseRowMap).
   struct RowMapRecord {

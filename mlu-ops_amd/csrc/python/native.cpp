@@ -59,6 +59,7 @@ namespace {
   X(mluOpDynamicPointToVoxelBackward)                      \
   X(mluOpExtSetSparseConvExtendedModes)                    \
   X(mluOpExtSetDistinctPairsPromise)                       \
+  X(mluOpExtSetPairTails)                                  \
   X(mluOpExtGetIndicePairsHostCounts)                      \
   X(mluOpExtGetVoxelizationHostCount)                      \
   X(mluOpExtGetRowMapSize)                                 \
@@ -210,7 +211,7 @@ class ConvDesc {
 Rulebook3 indicePairs(mluOpHandle_t handle, const Buffers &buffers, const at::Tensor &indices, int batch,
                       const Ints &input_space, const Ints &filter_space, const Ints &output_space, const Ints &pad,
                       const Ints &stride, const Ints &dilation, bool sub_m, std::optional<int64_t> out_rows,
-                      std::optional<at::Tensor> out_indices, bool for_layer) {
+                      std::optional<at::Tensor> out_indices, bool for_layer, bool tails) {
   const int64_t L = indices.size(0);
   int64_t K = 1;
   for (int k : filter_space) K *= k;
@@ -239,9 +240,12 @@ Rulebook3 indicePairs(mluOpHandle_t handle, const Buffers &buffers, const at::Te
   check(api.mluOpGetIndicePairsWorkspaceSize(handle, conv, d_in, d_pairs, d_out, d_num, &bytes),
         "mluOpGetIndicePairsWorkspaceSize");
   const at::Tensor ws = buffers.workspace(bytes);
-  check(api.mluOpGetIndicePairs(handle, conv, d_in, indices.data_ptr(), ws.data_ptr(), bytes, d_pairs,
-                                r.pairs.data_ptr(), d_out, r.out_indices.data_ptr(), d_num, r.indice_num.data_ptr()),
-        "mluOpGetIndicePairs");
+  if (!tails) check(api.mluOpExtSetPairTails(handle, 0), "mluOpExtSetPairTails");
+  const mluOpStatus_t built =
+      api.mluOpGetIndicePairs(handle, conv, d_in, indices.data_ptr(), ws.data_ptr(), bytes, d_pairs,
+                              r.pairs.data_ptr(), d_out, r.out_indices.data_ptr(), d_num, r.indice_num.data_ptr());
+  if (!tails) check(api.mluOpExtSetPairTails(handle, 1), "mluOpExtSetPairTails");
+  check(built, "mluOpGetIndicePairs");
   r.num_act_out = L;
   if (!sub_m) {
     int n = 0;
@@ -675,14 +679,14 @@ PYBIND11_MODULE(_native, m) {
         [](uintptr_t handle, bool guarded, const at::Tensor &indices, int batch, const Ints &input_space,
            const Ints &filter_space, const Ints &output_space, const Ints &pad, const Ints &stride,
            const Ints &dilation, bool sub_m, std::optional<int64_t> out_rows, std::optional<at::Tensor> out_indices,
-           bool for_layer) {
+           bool for_layer, bool tails) {
           Rulebook3 r;
           {
             NoGil released;
             const OperatorLock lock(asHandle(handle));
             r = indicePairs(asHandle(handle), Buffers(guarded, indices.device()), indices, batch, input_space,
                             filter_space, output_space, pad, stride, dilation, sub_m, out_rows, std::move(out_indices),
-                            for_layer);
+                            for_layer, tails);
           }
           py::object num = for_layer ? py::cast(r.counts) : py::cast(r.indice_num);
           return py::make_tuple(r.pairs, r.out_indices, num, r.num_act_out);

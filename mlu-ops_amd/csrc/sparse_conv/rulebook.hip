@@ -73,6 +73,7 @@ struct GeomDev {
   int dil[3];
   int K;
   int L;
+  bool fill_tails;        // pair slots behind an offset's pairs become -1
   FastDiv by_stride[3];
   FastDiv by_out_volume;  // out[0] * out[1] * out[2]
   FastDiv by_out_plane;   // out[1] * out[2]
@@ -259,7 +260,7 @@ __global__ __launch_bounds__(kBlock) void rbSubmInsert(GeomDev g, const int32_t 
     // Every pair slot starts as -1; the kernel that places the pairs overwrites the slots in
     // front of each offset's pair count.  Plain stores that nobody waits for, under the
     // table's atomics.
-    for (int k = 0; k < g.K; ++k) {
+    for (int k = 0; k < (g.fill_tails ? g.K : 0); ++k) {
       pairs[(size_t)k * 2 * g.L + j] = -1;
       pairs[((size_t)k * 2 + 1) * g.L + j] = -1;
     }
@@ -501,7 +502,7 @@ __global__ __launch_bounds__(kBlock) void rbProbeCount(GeomDev g,
       markCells<kGroup>(cell, bitmap);
       // every pair slot of this row and these offsets starts out as -1; the kernel that
       // places the pairs overwrites the front of each list afterwards
-      if (active) {
+      if (active && g.fill_tails) {
         for (int k = k0; k < k0 + kGroup && k < k_hi; ++k) {
           pairs[(size_t)(2 * k) * g.L + j] = -1;
           pairs[(size_t)(2 * k + 1) * g.L + j] = -1;
@@ -538,7 +539,7 @@ __global__ __launch_bounds__(kBlock) void rbProbeStrided(GeomDev g, const int32_
     if (blockIdx.y == 0) noteRowOrder(indices, j, c, aligned, rows_in_order);
     // every pair slot of this row starts out as -1 for the slice's offsets; the kernel that
     // places the pairs overwrites the front of each list afterwards
-    for (int k = k_lo; k < k_hi; ++k) {
+    for (int k = k_lo; k < (g.fill_tails ? k_hi : 0); ++k) {
       pairs[(size_t)(2 * k) * g.L + j] = -1;
       pairs[(size_t)(2 * k + 1) * g.L + j] = -1;
     }
@@ -705,7 +706,7 @@ __device__ __forceinline__ void sortedProbe(const GeomDev &g, const UnitStrideOf
   int4 c = make_int4(0, 0, 0, 0);
   if (active) {
     c = loadCoord(indices, j, aligned);
-    for (int k = KW * t_lo; k < k_end; ++k) {
+    for (int k = KW * t_lo; k < (g.fill_tails ? k_end : 0); ++k) {
       pairs[(size_t)(2 * k) * g.L + j] = -1;
       pairs[(size_t)(2 * k + 1) * g.L + j] = -1;
       if (sc.mirror) {
@@ -1513,6 +1514,7 @@ GeomDev toDev(const RulebookGeom &g) {
   d.by_out_width = makeFastDiv(g.out_space[2]);
   d.K = g.K;
   d.L = g.L;
+  d.fill_tails = g.fill_tails;
   return d;
 }
 

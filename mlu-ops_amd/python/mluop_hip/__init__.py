@@ -126,6 +126,7 @@ SIGNATURES = {
     "mluOpExtSetKernelChoice": (ctypes.c_int, [_vp, ctypes.c_int, ctypes.c_int]),
     "mluOpExtSetSparseConvExtendedModes": (ctypes.c_int, [_vp, ctypes.c_int]),
     "mluOpExtSetDistinctPairsPromise": (ctypes.c_int, [_vp, ctypes.c_int]),
+    "mluOpExtSetPairTails": (ctypes.c_int, [_vp, ctypes.c_int]),
     "mluOpExtGetVoxelizationHostCount": (ctypes.c_int, [_vp, _vp, ctypes.POINTER(ctypes.c_int32)]),
     "mluOpExtGetIndicePairsHostCounts": (ctypes.c_int, [_vp, _vp, ctypes.c_int, _i64p]),
     "mluOpExtGetRowMapSize": (ctypes.c_int, [_vp, ctypes.c_int64, ctypes.POINTER(ctypes.c_size_t)]),
@@ -444,7 +445,7 @@ def _guards_intact(call):
 
 
 def get_indice_pairs(handle, indices, batch, input_space, filter_space, output_space, pad, stride,
-                     dilation, sub_m, out_rows=None, out_indices=None, for_layer=False):
+                     dilation, sub_m, out_rows=None, out_indices=None, for_layer=False, tails=True):
     """Builds the rulebook for `indices` (int32 [L, 4] device tensor).
 
     Returns (indice_pairs [K,2,L], out_indices [out_rows,4], indice_num [K] device int32,
@@ -453,10 +454,13 @@ def get_indice_pairs(handle, indices, batch, input_space, filter_space, output_s
     them alone (the reference decodes num_act_out rows, normal_get_indice_pairs.cpp:1143-1150).
 
     `for_layer=True` is the form the convolution operators go on with: out_indices cut to its
-    num_act_out rows and indice_num as host ints, waited for without draining the queue."""
+    num_act_out rows and indice_num as host ints, waited for without draining the queue.
+
+    `tails=False` leaves the slots of indice_pairs behind each offset's pairs as allocated instead of -1
+    (mluOpExtSetPairTails), for callers who read no further than indice_num."""
     return native().get_indice_pairs(handle.ptr.value, _guarded(), indices, batch, _ints(input_space),
                                      _ints(filter_space), _ints(output_space), _ints(pad), _ints(stride),
-                                     _ints(dilation), bool(sub_m), out_rows, out_indices, for_layer)
+                                     _ints(dilation), bool(sub_m), out_rows, out_indices, for_layer, tails)
 
 
 def _ints(values):

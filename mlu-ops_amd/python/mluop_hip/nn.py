@@ -47,7 +47,8 @@ def share_row_maps(enable):
 
 
 class Rulebook:
-    """indice_pairs [K,2,L] (device), indice_num as host ints, out_indices, num_act_out."""
+    """indice_pairs [K,2,L] (device; what lies behind an offset's indice_num pairs is not defined),
+    indice_num as host ints, out_indices, num_act_out."""
 
     def __init__(self, pairs, out_indices, indice_num_host, num_act_out, filter_space, sub_m, out_space,
                  in_indices=None, in_space=None, distinct=False):
@@ -154,7 +155,7 @@ class _ConvBase(torch.nn.Module):
         # the operators take indice_num as host ints: one wait per rulebook
         pairs, out_indices, num, n_out = get_indice_pairs(
             _handle(), x.indices, x.batch_size, x.spatial_shape, self.kernel_size, out_space, self.padding,
-            self.stride, self.dilation, self.sub_m, for_layer=True)
+            self.stride, self.dilation, self.sub_m, for_layer=True, tails=False)
         rb = Rulebook(pairs, out_indices, num, n_out, self.kernel_size, self.sub_m,
                       out_space, in_indices=x.indices, in_space=x.spatial_shape, distinct=x.distinct)
         if self.indice_key is not None:
