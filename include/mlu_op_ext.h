@@ -91,6 +91,10 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtSetDistinctPairsPromise(mluOpHandle_t handle
  * indice_num.  Holds for the handle until changed. */
 mluOpStatus_t MLUOP_WIN_API mluOpExtSetPairTails(mluOpHandle_t handle, int fill);
 
+/* mluOpIndiceConvolutionForward stores negative results as zero (NaN stays NaN) while this is on: the ReLU
+ * behind a layer without a pass of its own over the result.  Off for a new handle; holds until changed. */
+mluOpStatus_t MLUOP_WIN_API mluOpExtSetForwardRelu(mluOpHandle_t handle, int enable);
+
 /* The pair counts of a rulebook on the host.  The convolution operators take indice_num as a host
  * array, so a caller has to bring the counts mluOpGetIndicePairs left in device memory over; a copy
  * waits for the whole queue.  The last kernel of a rulebook also stores them into pinned memory of

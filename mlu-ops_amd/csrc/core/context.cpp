@@ -207,6 +207,12 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtSetSparseConvExtendedModes(mluOpHandle_t han
   return MLUOP_STATUS_SUCCESS;
 }
 
+mluOpStatus_t MLUOP_WIN_API mluOpExtSetForwardRelu(mluOpHandle_t handle, int enable) {
+  PARAM_CHECK("[mluOpExtSetForwardRelu]", handle != NULL);
+  handle->forward_relu = enable != 0;
+  return MLUOP_STATUS_SUCCESS;
+}
+
 mluOpStatus_t MLUOP_WIN_API mluOpExtSetPairTails(mluOpHandle_t handle, int fill) {
   PARAM_CHECK("[mluOpExtSetPairTails]", handle != NULL);
   handle->fill_pair_tails = fill != 0;

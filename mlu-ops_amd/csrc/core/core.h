@@ -45,6 +45,8 @@ struct mluOpContext {
   bool distinct_pairs_promised = false;
   // rulebooks set the pair slots behind each offset's pairs to -1 (mluOpExtSetPairTails)
   bool fill_pair_tails = true;
+  // forward convolutions store negative results as zero (mluOpExtSetForwardRelu)
+  bool forward_relu = false;
   // Row maps built by mluOpExtBuildRowMap with no pair lost, and the one announced for the
   // next forward / backward-data call (mluOpExtUseRowMap).
   struct RowMapRecord {

@@ -60,6 +60,7 @@ namespace {
   X(mluOpExtSetSparseConvExtendedModes)                    \
   X(mluOpExtSetDistinctPairsPromise)                       \
   X(mluOpExtSetPairTails)                                  \
+  X(mluOpExtSetForwardRelu)                                \
   X(mluOpExtGetIndicePairsHostCounts)                      \
   X(mluOpExtGetVoxelizationHostCount)                      \
   X(mluOpExtGetRowMapSize)                                 \
@@ -494,16 +495,32 @@ struct LayerRulebook : torch::CustomClassHolder {
 };
 using LayerRulebookPtr = c10::intrusive_ptr<LayerRulebook>;
 
+// The handle's forward convolutions store negative results as zero while this is there.
+class ReluOn {
+ public:
+  ReluOn(mluOpHandle_t handle, bool on) : handle_(on ? handle : nullptr) {
+    if (on) check(api.mluOpExtSetForwardRelu(handle, 1), "mluOpExtSetForwardRelu");
+  }
+  ~ReluOn() {
+    if (handle_ != nullptr) api.mluOpExtSetForwardRelu(handle_, 0);
+  }
+  ReluOn(const ReluOn &) = delete;
+  ReluOn &operator=(const ReluOn &) = delete;
+
+ private:
+  mluOpHandle_t handle_;
+};
+
 struct IndiceConv : torch::autograd::Function<IndiceConv> {
   static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &features,
                             const at::Tensor &weight, const LayerRulebookPtr &rb, bool inverse, bool share_row_maps,
-                            bool guarded) {
+                            bool guarded, bool relu) {
     const at::Tensor x = features.contiguous(), w = weight.contiguous();
-    ctx->save_for_backward({x, w});
     ctx->saved_data["rulebook"] = c10::IValue::make_capsule(rb);
     ctx->saved_data["inverse"] = inverse;
     ctx->saved_data["share_row_maps"] = share_row_maps;
     ctx->saved_data["guarded"] = guarded;
+    ctx->saved_data["relu"] = relu;
     StreamHandle &h = streamHandle();
     const OperatorLock lock(h);
     check(api.mluOpExtSetDistinctPairsPromise(h.handle, rb->distinct), "mluOpExtSetDistinctPairsPromise");
@@ -511,10 +528,16 @@ struct IndiceConv : torch::autograd::Function<IndiceConv> {
     const void *map = share_row_maps ? rb->rowMap(h, buffers, inverse ? 0 : 1) : nullptr;
     // an inverse layer runs the partner layer's rulebook backwards: one output row per input
     // row of the partner
-    return inverse ? convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts,
-                                 rb->pairs.size(2), false, 1, map)
-                   : convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts,
-                                 rb->num_act_out, rb->sub_m, 0, map);
+    const ReluOn on(h.handle, relu);
+    const at::Tensor out = inverse ? convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts,
+                                                 rb->pairs.size(2), false, 1, map)
+                                   : convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts,
+                                                 rb->num_act_out, rb->sub_m, 0, map);
+    if (relu)
+      ctx->save_for_backward({x, w, out});
+    else
+      ctx->save_for_backward({x, w});
+    return out;
   }
 
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx,
@@ -523,9 +546,11 @@ struct IndiceConv : torch::autograd::Function<IndiceConv> {
     const at::Tensor &x = saved[0], &w = saved[1];
     const auto rb = c10::static_intrusive_pointer_cast<LayerRulebook>(ctx->saved_data["rulebook"].toCapsule());
     const bool inverse = ctx->saved_data["inverse"].toBool();
-    torch::autograd::variable_list out(6);
+    torch::autograd::variable_list out(7);
     if (!grads[0].defined()) return out;
-    const at::Tensor dy = grads[0].contiguous();
+    // behind a ReLU in the store: the gradient that the ReLU would have passed on
+    const bool relu = ctx->saved_data["relu"].toBool();
+    const at::Tensor dy = (relu ? at::threshold_backward(grads[0], saved[2], 0) : grads[0]).contiguous();
     StreamHandle &h = streamHandle();
     const OperatorLock lock(h);
     check(api.mluOpExtSetDistinctPairsPromise(h.handle, rb->distinct), "mluOpExtSetDistinctPairsPromise");
@@ -770,8 +795,8 @@ PYBIND11_MODULE(_native, m) {
       }))
       .def("row_maps", &LayerRulebook::rowMaps, "(handle, pair column) of the row maps its calls have built.");
   m.def("indice_conv", [](const at::Tensor &features, const at::Tensor &weight, const LayerRulebookPtr &rulebook,
-                          bool inverse, bool share_row_maps, bool guarded) {
+                          bool inverse, bool share_row_maps, bool guarded, bool relu) {
     NoGil released;
-    return IndiceConv::apply(features, weight, rulebook, inverse, share_row_maps, guarded);
+    return IndiceConv::apply(features, weight, rulebook, inverse, share_row_maps, guarded, relu);
   });
 }

@@ -137,6 +137,11 @@ struct FloatElem {
   }
 };
 
+// A result's last step: negative sums become zero where the caller asked for it (a NaN stays one).  The
+// ReLU behind a layer by itself reads and writes the whole result again: 11 of them took 97 of 1085 us
+// of an 11-layer network's call.
+__device__ __forceinline__ float activated(float v, bool relu) { return relu && v < 0.f ? 0.f : v; }
+
 // ---- row map ---------------------------------------------------------------
 
 // A launch that is enqueued before anyone knows whether it is needed: it runs when `word` is
@@ -239,7 +244,7 @@ __global__ __launch_bounds__(256) void gatherConvSimt(const typename E::storage 
                                                       int64_t sQ, int64_t sC, const int32_t *map,
                                                       int R, int K, OffsetCounts inl,
                                                       const int32_t *dev_counts, int C,
-                                                      int32_t *filled,
+                                                      int32_t *filled, bool relu,
                                                       typename E::storage *result) {
   constexpr int TR = 32, TC = 64, QC = 32;
   int slots = 0;  // filled map slots of this tile (first wave, uniform)
@@ -307,7 +312,7 @@ __global__ __launch_bounds__(256) void gatherConvSimt(const typename E::storage 
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int c = c0 + tx * 4 + j;
-      if (c < C) E::store(result + (size_t)r * C + c, acc[i][j]);
+      if (c < C) E::store(result + (size_t)r * C + c, activated(acc[i][j], relu));
     }
   }
   if (tid == 0 && blockIdx.y == 0) filled[blockIdx.x] = slots;
@@ -630,6 +635,7 @@ struct ConvRows {
   int row_bytes;  // bytes from one gathered row to the next: a multiple of 16, all of them readable
   int c;          // result columns
   int c_padded;   // result columns of the packed filter
+  bool relu;      // negative results become zero
 };
 
 // `VALS` consecutive result values of one row from column `col` on, as many as the row has.
@@ -1015,7 +1021,7 @@ void gatherConvMfma(const typename E::storage *A, ConvRows rows, const typename 
     if (r0 + rr >= R) break;
     S tmp[VALS];
 #pragma unroll
-    for (int e = 0; e < VALS; ++e) E::store(&tmp[e], s_acc[rr * ACC_STRIDE + c0 + e]);
+    for (int e = 0; e < VALS; ++e) E::store(&tmp[e], activated(s_acc[rr * ACC_STRIDE + c0 + e], rows.relu));
     storeColumns<E>(result + (size_t)(r0 + rr) * rows.c, col_group * C + c0, rows.c, tmp);
   }
   if constexpr (!SRC::kSegments) {
@@ -1399,7 +1405,7 @@ void gatherConvTall(const typename E::storage *A, uint32_t a_size, ConvRows rows
       const int piece = c0 / 4 + q;
       const float4v v = reinterpret_cast<const float4v *>(s_acc)[rr * (C / 4) + (in_order ? piece ^ (rr & 15) : piece)];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) E::store(&tmp[q * 4 + e], v[e]);
+      for (int e = 0; e < 4; ++e) E::store(&tmp[q * 4 + e], activated(v[e], rows.relu));
     }
     storeColumns<E>(result + (size_t)(r0 + rr) * rows.c, col_group * C + c0, rows.c, tmp);
   }
@@ -1449,7 +1455,7 @@ __global__ __launch_bounds__(64) void gatherConvWave(
   constexpr int TR = kWaveTileRows;
   constexpr int ACC_STRIDE = C + 4;
   constexpr int ROW_BYTES = Q * (int)sizeof(S);
-  const ConvRows conv = WHOLE ? ConvRows{Q, ROW_BYTES, C, C} : lengths;
+  const ConvRows conv = WHOLE ? ConvRows{Q, ROW_BYTES, C, C, lengths.relu} : lengths;
   constexpr int STAGE_STRIDE = ROW_BYTES + 16;
   constexpr int PPR = ROW_BYTES / 16;                   // 16-byte pieces per row
   constexpr int RL = (16 * PPR + 63) / 64;              // wave-loads per unit of rows
@@ -1494,7 +1500,7 @@ __global__ __launch_bounds__(64) void gatherConvWave(
       if (r0 + rr >= R) break;
       S tmp[VALS];
 #pragma unroll
-      for (int e = 0; e < VALS; ++e) E::store(&tmp[e], s_acc[rr * ACC_STRIDE + c0 + e]);
+      for (int e = 0; e < VALS; ++e) E::store(&tmp[e], activated(s_acc[rr * ACC_STRIDE + c0 + e], conv.relu));
       storeColumns<E>(result + (size_t)(r0 + rr) * conv.c, c0, conv.c, tmp);
     }
   };
@@ -1829,7 +1835,7 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
         scanAllPairsForTile<E, NT>(A, conv.q, conv.row_bytes, source, K, r0, r_end, columns, c0, acc, CP);
         for (int i = tid; i < TR * CP; i += NT) {
           const int rr = i / CP, c = i % CP;
-          if (r0 + rr < R && c < columns) E::store(result + (size_t)(r0 + rr) * conv.c + c0 + c, acc[i]);
+          if (r0 + rr < R && c < columns) E::store(result + (size_t)(r0 + rr) * conv.c + c0 + c, activated(acc[i], conv.relu));
         }
         __syncthreads();
       }
@@ -2312,7 +2318,7 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
     for (int nb = 0; nb < NB; ++nb) {
       S tmp[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) E::store(&tmp[e], acc[g][nb][e]);
+      for (int e = 0; e < 4; ++e) E::store(&tmp[e], activated(acc[g][nb][e], conv.relu));
       storeColumns<E>(result + (size_t)r * conv.c, nb * 16 + quad * 4, conv.c, tmp);
     }
   }
@@ -2362,7 +2368,7 @@ __global__ __launch_bounds__(256) void repairLostPairs(
     int64_t sC, const int32_t *pairs, int L, int row_col, int src_col, int R, int n_src, int K,
     int row_base, OffsetCounts inl, const int32_t *dev_counts, int32_t *map,
     const int32_t *filled, int n_filled, const int32_t *accepted, int n_accepted, int C,
-    RepairScratch scratch, typename E::storage *result, RunIf run_if) {
+    RepairScratch scratch, bool relu, typename E::storage *result, RunIf run_if) {
   if (notWanted(run_if)) return;
   __shared__ int s_found;
   const int tid = threadIdx.x;
@@ -2487,7 +2493,7 @@ __global__ __launch_bounds__(256) void repairLostPairs(
     const int pooled = s_pooled;
     for (int i = 0; i < pooled; ++i) {
       const int r = pool_row[i];
-      for (int c = tid; c < C; c += 256) E::store(result + (size_t)r * C + c, pool[(size_t)i * C + c]);
+      for (int c = tid; c < C; c += 256) E::store(result + (size_t)r * C + c, activated(pool[(size_t)i * C + c], relu));
     }
     __syncthreads();
   }
@@ -3780,7 +3786,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
   while (1 << shape.chunk_bits < chunks) ++shape.chunk_bits;
   while (1 << shape.group_bits < groups) ++shape.group_bits;
   const bool pad_rows = use_mfma && rowsNeedPadding(p.dtype, d.Q);
-  const ConvRows rows_of = {d.Q, pad_rows ? paddedRowBytes(p.dtype, d.Q) : d.Q * (int)sizeof(S), d.C, d.c_padded};
+  const ConvRows rows_of = {d.Q, pad_rows ? paddedRowBytes(p.dtype, d.Q) : d.Q * (int)sizeof(S), d.C, d.c_padded, p.relu};
   const void *rows_from = pad_rows ? ws.padded_rows : gathered;
   const PadRows pad = {static_cast<const char *>(gathered), static_cast<char *>(ws.padded_rows), d.Q * (int)sizeof(S),
                        rows_of.row_bytes, pad_rows ? d.n_src : 0, pad_rows ? gridFor((size_t)d.n_src, 1024) : 0};
@@ -3899,7 +3905,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
       gatherConvSimt<E><<<grid, 256, 0, lc.stream>>>(static_cast<const S *>(gathered), d.Q,
                                                   static_cast<const S *>(f.base), f.stride_k, sQ, sC,
                                                   entries, rows, p.K, inl, ws.dev_counts, d.C,
-                                                  ws.filled, result_rows);
+                                                  ws.filled, p.relu, result_rows);
       lc.end();
     }
     if (p.distinct_pairs || !own_map) continue;  // a map built ahead was checked when it was built
@@ -3909,7 +3915,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
         static_cast<const S *>(gathered), d.Q, static_cast<const S *>(f.base), f.stride_k, sQ, sC,
         p.indice_pairs, p.L, d.row_col, d.src_col, rows, d.n_src, p.K, row_base, inl, ws.dev_counts,
         ws.map, ws.filled, n_filled, ws.accepted, n_accepted, d.C,
-        RepairScratch{ws.shadow, ws.pool_row, ws.pool}, result_rows, run_if);
+        RepairScratch{ws.shadow, ws.pool_row, ws.pool}, p.relu, result_rows, run_if);
     lc.end();
   }
 }

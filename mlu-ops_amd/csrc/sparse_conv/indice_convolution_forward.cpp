@@ -242,6 +242,7 @@ mluOpStatus_t MLUOP_WIN_API mluOpIndiceConvolutionForward(
   ConvProblem p = makeProblem(features_desc, filters_desc, indice_pairs_desc, indice_num,
                               num_act_out, inverse, indice_pairs);
   p.distinct_pairs = handle->distinct_pairs_promised;
+  p.relu = handle->forward_relu;
   st = mluop::sparse_conv::takeRowMap(api, handle, announced_map, GatherDirection::kForward, &p);
   if (st != MLUOP_STATUS_SUCCESS) return st;
   // what this call overwrites is no pair tensor any more, whatever the handle noted there

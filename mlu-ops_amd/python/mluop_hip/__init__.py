@@ -127,6 +127,7 @@ SIGNATURES = {
     "mluOpExtSetSparseConvExtendedModes": (ctypes.c_int, [_vp, ctypes.c_int]),
     "mluOpExtSetDistinctPairsPromise": (ctypes.c_int, [_vp, ctypes.c_int]),
     "mluOpExtSetPairTails": (ctypes.c_int, [_vp, ctypes.c_int]),
+    "mluOpExtSetForwardRelu": (ctypes.c_int, [_vp, ctypes.c_int]),
     "mluOpExtGetVoxelizationHostCount": (ctypes.c_int, [_vp, _vp, ctypes.POINTER(ctypes.c_int32)]),
     "mluOpExtGetIndicePairsHostCounts": (ctypes.c_int, [_vp, _vp, ctypes.c_int, _i64p]),
     "mluOpExtGetRowMapSize": (ctypes.c_int, [_vp, ctypes.c_int64, ctypes.POINTER(ctypes.c_size_t)]),
@@ -231,6 +232,10 @@ class Handle:
     def set_extended_modes(self, enable):
         """Accept inverse = 1 and tagged filters_grad layouts, which the reference rejects."""
         check(lib().mluOpExtSetSparseConvExtendedModes(self.ptr, 1 if enable else 0))
+
+    def set_forward_relu(self, enable):
+        """mluOpExtSetForwardRelu: forward convolutions store negative results as zero."""
+        check(lib().mluOpExtSetForwardRelu(self.ptr, 1 if enable else 0))
 
     def promise_distinct_pairs(self, promised):
         """No offset of the rulebooks names a result row twice: skip the check for lost pairs."""
