@@ -1151,15 +1151,24 @@ __global__ __launch_bounds__(kBlock) void rbBitmapBlockSum(const unsigned long l
 }
 
 // Per bitmap word: number of marked cells before it (word_rank).  Every marked
-// cell is decoded to (n, d, h, w) and written at its rank.  A thread owns one word; where
-// a wavefront's 64 words hold many cells (a small dense grid) the wavefront decodes them
-// word by word, a lane per cell, instead of each lane walking its own word's bits.  Rows
-// of out_indices from the number of marked cells on are left as the caller passed them,
+// cell is decoded to (n, d, h, w) and written at its rank.  A thread owns one word, and the
+// wavefront takes the cells of its 64 words by their number, a lane each: the lane looks its
+// word up among the running counts and selects the bit, so neighbours write neighbouring rows
+// and no lane waits for a fuller word (a lane walking its own word's bits, or a wavefront
+// taking one word at a time: 14.6 us at 722 blocks of clustered cells, now 8.3).  A small
+// grid has few wavefronts and, behind some layers, most of its cells marked: gridDim.y
+// workgroups share the cells of a block (see decodeParts).  Rows of out_indices from the number of marked cells on are left as the caller passed them,
 // as the reference's decode kernel leaves them (normal_get_indice_pairs.cpp:1143-1150).
 // block_count holds the marked cells of every block of kWordsPerBlock words: either as
 // counted, then each workgroup sums the counts in front of its block itself and the last
 // one writes the total to num_act_out, or, for bitmaps of more blocks than that is worth,
 // already scanned (`scanned`, total already in num_act_out).
+// Workgroups that share a block's cells: about 3072 in all.  The kernel by blocks of 256 words, at
+// 1 / 2 / 4 / 8 / 16 a block: 13 blocks 15.0 us at 1, 5.2 at 16; 95 blocks 15.3 at 1, 5.9 at 8, 5.1 at
+// 16; 512 blocks 6.3 at 1, 5.0 at 2, 5.8 at 8; 722 blocks 5.6 to 12 at 2, 7 to 8.3 at 4, 8.8 at 8; 2888
+// blocks 10.6 at 1 with the word's own lane decoding, 8.7 at 1, 15 at 4 (every part ranks the words again).
+static int decodeParts(int n_blocks) { return n_blocks > 1536 ? 1 : n_blocks < 192 ? 16 : 3072 / n_blocks; }
+
 __global__ __launch_bounds__(kBlock) void rbRankAndDecode(GeomDev g,
                                                           const unsigned long long *bitmap,
                                                           size_t n_words,
@@ -1202,15 +1211,16 @@ __global__ __launch_bounds__(kBlock) void rbRankAndDecode(GeomDev g,
   for (int x = 0; x < kBlock / kWave; ++x)
     if (x < wave) rank += s_wsum[x];
   // the count of output cells, for the device and (pinned memory) for the host
-  if (!scanned && blockIdx.x == gridDim.x - 1 && threadIdx.x == kBlock - 1) {
+  const bool first_part = blockIdx.y == 0;
+  if (!scanned && first_part && blockIdx.x == gridDim.x - 1 && threadIdx.x == kBlock - 1) {
     *num_act_out = rank + mine;
     __hip_atomic_store(host_num_act_out, stampedWord(stamp, rank + mine), __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_SYSTEM);
   }
-  if (scanned && blockIdx.x == 0 && threadIdx.x == 0)
+  if (scanned && first_part && blockIdx.x == 0 && threadIdx.x == 0)
     __hip_atomic_store(host_num_act_out, stampedWord(stamp, *num_act_out), __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_SYSTEM);
-  if (w < n_words) word_rank[w] = (uint32_t)rank;
+  if (first_part && w < n_words) word_rank[w] = (uint32_t)rank;
   auto put = [&](size_t cell64, int r) {
     if (r >= out_rows) return;
     int cell = (int)cell64;
@@ -1224,23 +1234,34 @@ __global__ __launch_bounds__(kBlock) void rbRankAndDecode(GeomDev g,
     storeCoord(out_indices, r, o, aligned);
   };
   const int wave_cells = __shfl(incl, kWave - 1, kWave);
-  if (wave_cells > 4 * kWave) {
-    unsigned long long todo = __ballot(bits != 0ull);
-    const size_t w_first = w - lane;
-    while (todo) {
-      const int src = __ffsll((long long)todo) - 1;
-      todo &= todo - 1;
-      const unsigned long long b = __shfl(bits, src, kWave);
-      const int r0 = __shfl(rank, src, kWave);
-      if ((b >> lane) & 1ull) put((w_first + src) * 64 + lane, r0 + __popcll(b & ((1ull << lane) - 1ull)));
+  const size_t w_first = w - lane;
+  const int wave_rank = __shfl(rank, 0, kWave);
+  for (int c0 = (int)blockIdx.y * kWave; c0 < wave_cells; c0 += (int)gridDim.y * kWave) {
+    // the c-th cell: its word is behind all that end at or before it
+    const int c = c0 + lane;
+    int in = 0;
+#pragma unroll
+    for (int step = kWave / 2; step > 0; step >>= 1)
+      if (__shfl(incl, in + step - 1, kWave) <= c) in += step;
+    const unsigned long long b = __shfl(bits, in, kWave);
+    int left = c - __shfl(incl - mine, in, kWave), bit = 0;
+    uint32_t half = (uint32_t)b;
+    const int low = __popc(half);
+    if (left >= low) {
+      left -= low;
+      bit = 32;
+      half = (uint32_t)(b >> 32);
     }
-  } else {
-    unsigned long long b = bits;
-    while (b) {
-      const int bit = __ffsll((long long)b) - 1;
-      b &= b - 1;
-      put(w * 64 + bit, rank++);
+#pragma unroll
+    for (int width = 16; width > 0; width >>= 1) {
+      const int below = __popc(half & ((1u << width) - 1u));
+      if (left >= below) {
+        left -= below;
+        bit += width;
+        half >>= width;
+      }
     }
+    if (c < wave_cells) put((w_first + in) * 64 + bit, wave_rank + c);
   }
 }
 
@@ -1701,7 +1722,7 @@ hipError_t launchRegularRulebook(const LaunchCtx &lc, const RulebookGeom &g,
     lc.end();
   }
   lc.begin("rbRankAndDecode");
-  rbRankAndDecode<<<ws.n_bitmap_blocks, kBlock, 0, lc.stream>>>(d, ws.bitmap, ws.n_words, ws.block_sum,
+  rbRankAndDecode<<<dim3(ws.n_bitmap_blocks, decodeParts(ws.n_bitmap_blocks)), kBlock, 0, lc.stream>>>(d, ws.bitmap, ws.n_words, ws.block_sum,
                                                              scanned, ws.num_act_out, host_num_act_out,
                                                              report.stamp, ws.word_rank, out_indices, al_out, g.out_rows);
   lc.end();
