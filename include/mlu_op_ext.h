@@ -36,8 +36,7 @@ typedef enum {
   MLUOP_EXT_KERNEL_FILTER_STORES = 6,   /* 1: backward filter transposes its operands with element-sized
                                            LDS stores also for 2-byte types of 32 to 128 channels, where
                                            transposing LDS reads are the default */
-  MLUOP_EXT_KERNEL_TALL_TILES = 8,      /* gather kernel with tall tiles of result rows */
-  MLUOP_EXT_KERNEL_LISTS_ON_TRUST = 7   /* forward on a rulebook of this handle whose report (were the input
+  MLUOP_EXT_KERNEL_LISTS_ON_TRUST = 7,  /* forward on a rulebook of this handle whose report (were the input
                                            rows in cell order?) has not reached the host yet, as under graph
                                            capture or without any wait between the two calls.  -1: start on
                                            the pair lists and enqueue the row-map kernels behind them; the
@@ -45,6 +44,7 @@ typedef enum {
                                            work, the others return at once.  0: build the row map.  1: a test
                                            switch: the pair lists only; a call whose lists fail the check
                                            leaves its output as it was */
+  MLUOP_EXT_KERNEL_TALL_TILES = 16      /* gather kernel with tall tiles of result rows (8 is refused, as it always was) */
 } mluOpExtKernelChoice_t;
 
 mluOpStatus_t MLUOP_WIN_API mluOpExtSetKernelChoice(mluOpHandle_t handle,
