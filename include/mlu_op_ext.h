@@ -117,6 +117,17 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtGetIndicePairsHostCounts(mluOpHandle_t handl
 mluOpStatus_t MLUOP_WIN_API mluOpExtGetVoxelizationHostCount(mluOpHandle_t handle, const void *voxel_num,
                                                              int32_t *count);
 
+/* The order of voxels by their linear cell index (z * space[1] + y) * space[2] + x, and their cells in that
+ * order.  coors [voxels, 3] int32 (z, y, x) as mluOpVoxelization writes them; order [voxels] int64, the
+ * voxel at each place; indices [voxels, 4] int32 (batch_index, z, y, x) in order.  Equal cells are ordered
+ * by voxel; coordinates outside the space are ordered by their index all the same.  1 to 2^20 voxels
+ * (NOT_SUPPORTED above), workspace of the queried size.  No counterpart in the reference. */
+mluOpStatus_t MLUOP_WIN_API mluOpExtGetOrderVoxelsWorkspaceSize(int64_t voxels, const int64_t space[3],
+                                                                size_t *size);
+mluOpStatus_t MLUOP_WIN_API mluOpExtOrderVoxels(mluOpHandle_t handle, const void *coors, int64_t voxels,
+                                                const int64_t space[3], int32_t batch_index, void *workspace,
+                                                size_t workspace_size, void *order, void *indices);
+
 /* Row maps kept across calls.  mluOpIndiceConvolutionForward and ...BackwardData turn the pair
  * lists into a [K, rows] map (partner row of every result row at every offset, or -1) on every
  * call: the reference API (mlu_op.h:10321-10448, :9625-9773) hands them nothing else to keep.

@@ -61,6 +61,8 @@ namespace {
   X(mluOpExtSetDistinctPairsPromise)                       \
   X(mluOpExtSetPairTails)                                  \
   X(mluOpExtSetForwardRelu)                                \
+  X(mluOpExtGetOrderVoxelsWorkspaceSize)                   \
+  X(mluOpExtOrderVoxels)                                   \
   X(mluOpExtGetIndicePairsHostCounts)                      \
   X(mluOpExtGetVoxelizationHostCount)                      \
   X(mluOpExtGetRowMapSize)                                 \
@@ -621,6 +623,24 @@ std::vector<at::Tensor> voxelizationCut(bool guarded, const at::Tensor &points, 
   return r;
 }
 
+// Voxels in the order of their cells: (the voxel at each place, its (batch, z, y, x)).
+std::vector<at::Tensor> orderVoxels(bool guarded, const at::Tensor &coors, const Counts &space, int64_t batch_index) {
+  StreamHandle &h = streamHandle();
+  const OperatorLock lock(h);
+  const Buffers buffers(guarded, coors.device());
+  const int64_t n = coors.size(0);
+  const at::Tensor order = buffers.output({n}, at::kLong, "order");
+  const at::Tensor indices = buffers.output({n, 4}, at::kInt, "indices");
+  size_t bytes = 0;
+  check(api.mluOpExtGetOrderVoxelsWorkspaceSize(n, space.data(), &bytes), "mluOpExtGetOrderVoxelsWorkspaceSize");
+  const at::Tensor ws = buffers.workspace(bytes);
+  check(api.mluOpExtOrderVoxels(h.handle, coors.data_ptr(), n, space.data(), static_cast<int32_t>(batch_index),
+                                ws.data_ptr(), bytes, order.data_ptr(), indices.data_ptr()),
+        "mluOpExtOrderVoxels");
+  buffers.done("mluOpExtOrderVoxels");
+  return {order, indices};
+}
+
 std::vector<at::Tensor> scatterForward(mluOpHandle_t handle, const Buffers &buffers, const at::Tensor &feats,
                                        const at::Tensor &coors, mluOpReduceMode_t mode, int64_t rows) {
   const int64_t n = feats.size(0), c = feats.size(1);
@@ -764,6 +784,14 @@ PYBIND11_MODULE(_native, m) {
           }
           return py::make_tuple(r[0], r[1], r[2]);
         });
+  m.def("order_voxels", [](bool guarded, const at::Tensor &coors, const Counts &space, int64_t batch_index) {
+    std::vector<at::Tensor> r;
+    {
+      NoGil released;
+      r = orderVoxels(guarded, coors, space, batch_index);
+    }
+    return py::make_tuple(r[0], r[1]);
+  });
   m.def("dynamic_point_to_voxel_forward",
         [](uintptr_t handle, bool guarded, const at::Tensor &feats, const at::Tensor &coors, int mode, int64_t rows) {
           NoGil released;

@@ -233,6 +233,13 @@ class SparseInverseConv3d(_ConvBase):
         return SparseTensor(feats, rb.in_indices, rb.in_space, x.batch_size, x.rulebooks, distinct=rb.distinct)
 
 
+def _unwatched():
+    """Whether torch's calls are made by themselves: no tracing, no transform, no mode that sees them."""
+    return not (torch.jit.is_tracing() or torch.compiler.is_compiling() or
+                torch._C._len_torch_function_stack() or torch._C._len_torch_dispatch_stack() or
+                torch._C._functorch.peek_interpreter_stack() is not None)
+
+
 def _plain_call(m):
     """Whether calling module `m` comes to its class's forward and nothing else."""
     return not ("forward" in m.__dict__ or m._forward_hooks or m._forward_pre_hooks or
@@ -248,8 +255,7 @@ def _relu_in_store(conv, relu):
             conv.bias is None and _plain_call(conv) and _plain_call(relu) and
             # (behind guard bands a result is a view, which autograd does not let a ReLU overwrite)
             not (relu.inplace and _guarded()) and
-            not torch.jit.is_tracing() and not torch.compiler.is_compiling() and
-            not torch._C._len_torch_function_stack() and not torch._C._len_torch_dispatch_stack())
+            _unwatched())
 
 
 class SparseSequential(torch.nn.Sequential):
@@ -322,6 +328,16 @@ def mean_voxel_features(voxels, num_points_per_voxel):
     return voxels.sum(dim=1) / num_points_per_voxel.clamp(min=1).to(voxels.dtype).unsqueeze(1)
 
 
+def _ordered_by_library(coors, spatial_shape, batch_index):
+    """Whether the library's kernels order these voxels (five launches in place of some 20 of a sort and the
+    steps around it; voxelizer and 11-layer encoder, 120 000 voxels: 986 -> 865 us): what they accept, on
+    the current device, and no mode that watches torch's calls."""
+    return (coors.is_cuda and coors.dim() == 2 and coors.shape[1] == 3 and 1 < coors.shape[0] <= 1 << 20 and
+            coors.device.index == torch.cuda.current_device() and len(spatial_shape) == 3 and
+            all(0 < int(v) < 1 << 20 for v in spatial_shape) and -(1 << 31) <= int(batch_index) < 1 << 31 and
+            _unwatched())
+
+
 def sparse_tensor_from_voxels(features, coors, spatial_shape, batch_index=0, batch_size=1, order_by_cell=True):
     """SparseTensor of one cloud's voxels: indices (n, z, y, x) with n = batch_index.
 
@@ -332,6 +348,10 @@ def sparse_tensor_from_voxels(features, coors, spatial_shape, batch_index=0, bat
     table and the convolutions read as pair lists without a row map.  The rows of the returned
     tensor are a permutation of the voxelizer's; `order_by_cell=False` keeps its order."""
     coors = coors.to(torch.int32)
+    if order_by_cell and _ordered_by_library(coors, spatial_shape, batch_index):
+        order, indices = native().order_voxels(_guarded(), coors.contiguous(), [int(v) for v in spatial_shape],
+                                               int(batch_index))
+        return SparseTensor(features[order], indices, spatial_shape, batch_size, distinct=True)
     if order_by_cell and coors.shape[0] > 1:
         d, h, w = (int(v) for v in spatial_shape)
         key = (coors[:, 0].to(torch.int64) * h + coors[:, 1].to(torch.int64)) * w + coors[:, 2].to(torch.int64)
