@@ -209,12 +209,20 @@ class ConvDesc {
   mluOpSparseConvolutionDescriptor_t d_ = nullptr;
 };
 
-// `for_layer`: out_indices is cut to the active rows (and its tail left as allocated), and the
-// counts come back on the host.
+// The pair counts of a rulebook built on `handle`, as soon as they are there; false: not on file.
+bool hostCounts(mluOpHandle_t handle, const at::Tensor &pairs, Counts *counts) {
+  counts->assign(pairs.size(0), 0);
+  return pairs.numel() == 0 ||
+         api.mluOpExtGetIndicePairsHostCounts(handle, pairs.data_ptr(), static_cast<int>(pairs.size(0)),
+                                              counts->data()) == MLUOP_STATUS_SUCCESS;
+}
+
+// `for_layer`: out_indices is cut to the active rows (and its tail left as allocated), and with
+// `wait_counts` the counts come back on the host.
 Rulebook3 indicePairs(mluOpHandle_t handle, const Buffers &buffers, const at::Tensor &indices, int batch,
                       const Ints &input_space, const Ints &filter_space, const Ints &output_space, const Ints &pad,
                       const Ints &stride, const Ints &dilation, bool sub_m, std::optional<int64_t> out_rows,
-                      std::optional<at::Tensor> out_indices, bool for_layer, bool tails) {
+                      std::optional<at::Tensor> out_indices, bool for_layer, bool tails, bool wait_counts) {
   const int64_t L = indices.size(0);
   int64_t K = 1;
   for (int k : filter_space) K *= k;
@@ -256,10 +264,10 @@ Rulebook3 indicePairs(mluOpHandle_t handle, const Buffers &buffers, const at::Te
     r.num_act_out = n;
   }
   if (for_layer) {
-    r.counts.assign(K, 0);
     const bool empty = L == 0 || K == 0 || *out_rows == 0;
-    if (!empty && api.mluOpExtGetIndicePairsHostCounts(handle, r.pairs.data_ptr(), static_cast<int>(K),
-                                                       r.counts.data()) != MLUOP_STATUS_SUCCESS) {
+    if (empty) {
+      r.counts.assign(K, 0);
+    } else if (wait_counts && !hostCounts(handle, r.pairs, &r.counts)) {
       const at::Tensor host = r.indice_num.cpu();
       const int32_t *n = host.data_ptr<int32_t>();
       r.counts.assign(n, n + K);
@@ -724,18 +732,26 @@ PYBIND11_MODULE(_native, m) {
         [](uintptr_t handle, bool guarded, const at::Tensor &indices, int batch, const Ints &input_space,
            const Ints &filter_space, const Ints &output_space, const Ints &pad, const Ints &stride,
            const Ints &dilation, bool sub_m, std::optional<int64_t> out_rows, std::optional<at::Tensor> out_indices,
-           bool for_layer, bool tails) {
+           bool for_layer, bool tails, bool wait_counts) {
           Rulebook3 r;
           {
             NoGil released;
             const OperatorLock lock(asHandle(handle));
             r = indicePairs(asHandle(handle), Buffers(guarded, indices.device()), indices, batch, input_space,
                             filter_space, output_space, pad, stride, dilation, sub_m, out_rows, std::move(out_indices),
-                            for_layer, tails);
+                            for_layer, tails, wait_counts);
           }
-          py::object num = for_layer ? py::cast(r.counts) : py::cast(r.indice_num);
+          const bool counted = for_layer && r.counts.size() == static_cast<size_t>(r.pairs.size(0));
+          py::object num = counted ? py::cast(r.counts) : py::cast(r.indice_num);
           return py::make_tuple(r.pairs, r.out_indices, num, r.num_act_out);
         });
+  m.def("rulebook_counts", [](uintptr_t handle, const at::Tensor &pairs) -> std::optional<Counts> {
+    NoGil released;
+    const OperatorLock lock(asHandle(handle));
+    Counts counts;
+    if (!hostCounts(asHandle(handle), pairs, &counts)) return std::nullopt;
+    return counts;
+  });
   m.def("indice_conv_forward",
         [](uintptr_t handle, bool guarded, const at::Tensor &features, const at::Tensor &filters, int layout,
            const at::Tensor &pairs, const Counts &counts, int64_t num_act_out, bool sub_m, int64_t inverse,

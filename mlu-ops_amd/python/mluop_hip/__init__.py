@@ -452,7 +452,7 @@ def _guards_intact(call):
 
 
 def get_indice_pairs(handle, indices, batch, input_space, filter_space, output_space, pad, stride,
-                     dilation, sub_m, out_rows=None, out_indices=None, for_layer=False, tails=True):
+                     dilation, sub_m, out_rows=None, out_indices=None, for_layer=False, tails=True, wait_counts=True):
     """Builds the rulebook for `indices` (int32 [L, 4] device tensor).
 
     Returns (indice_pairs [K,2,L], out_indices [out_rows,4], indice_num [K] device int32,
@@ -461,13 +461,25 @@ def get_indice_pairs(handle, indices, batch, input_space, filter_space, output_s
     them alone (the reference decodes num_act_out rows, normal_get_indice_pairs.cpp:1143-1150).
 
     `for_layer=True` is the form the convolution operators go on with: out_indices cut to its
-    num_act_out rows and indice_num as host ints, waited for without draining the queue.
+    num_act_out rows and indice_num as host ints, waited for without draining the queue; with
+    `wait_counts=False` it stays on the device (unless there is nothing to count) and `rulebook_counts` takes it.
 
     `tails=False` leaves the slots of indice_pairs behind each offset's pairs as allocated instead of -1
     (mluOpExtSetPairTails), for callers who read no further than indice_num."""
     return native().get_indice_pairs(handle.ptr.value, _guarded(), indices, batch, _ints(input_space),
                                      _ints(filter_space), _ints(output_space), _ints(pad), _ints(stride),
-                                     _ints(dilation), bool(sub_m), out_rows, out_indices, for_layer, tails)
+                                     _ints(dilation), bool(sub_m), out_rows, out_indices, for_layer, tails,
+                                     wait_counts)
+
+
+def rulebook_counts(handle, indice_pairs, indice_num):
+    """Host ints of a rulebook that get_indice_pairs(..., for_layer=True, wait_counts=False) has built on `handle`,
+    as soon as its last kernel has stored them."""
+    counts = native().rulebook_counts(handle.ptr.value, indice_pairs)
+    if counts is None:  # no longer on file (the handle keeps 32 rulebooks), or too many offsets
+        _torch().cuda.synchronize(indice_num.device)
+        counts = indice_num.tolist()
+    return counts
 
 
 def _ints(values):
