@@ -44,7 +44,8 @@ typedef enum {
                                            work, the others return at once.  0: build the row map.  1: a test
                                            switch: the pair lists only; a call whose lists fail the check
                                            leaves its output as it was */
-  MLUOP_EXT_KERNEL_TALL_TILES = 16      /* gather kernel with tall tiles of result rows (8 is refused, as it always was) */
+  MLUOP_EXT_KERNEL_TALL_TILES = 16,     /* gather kernel with tall tiles of result rows (8 is refused, as it always was) */
+  MLUOP_EXT_KERNEL_SMALL_RULEBOOK = 17 /* submanifold rulebooks of up to 4096 rows in one launch */
 } mluOpExtKernelChoice_t;
 
 mluOpStatus_t MLUOP_WIN_API mluOpExtSetKernelChoice(mluOpHandle_t handle,

@@ -192,6 +192,7 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtSetKernelChoice(mluOpHandle_t handle,
     case MLUOP_EXT_KERNEL_SMALL_MAP_CHUNKS: c.small_map_chunks = value; break;
     case MLUOP_EXT_KERNEL_FILTER_STORES: c.filter_stores = value; break;
     case MLUOP_EXT_KERNEL_TALL_TILES: c.tall_tiles = value; break;
+    case MLUOP_EXT_KERNEL_SMALL_RULEBOOK: c.small_rulebook = value; break;
     case MLUOP_EXT_KERNEL_LISTS_ON_TRUST: c.lists_on_trust = value; break;
     default:
       MLUOP_LOG(ERROR) << "[mluOpExtSetKernelChoice] unknown kernel choice " << as_int;

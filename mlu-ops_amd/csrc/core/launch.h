@@ -58,6 +58,7 @@ struct KernelChoices {
   int small_map_chunks = -1;  // 1: row maps cover 2048 result rows at a time (the chunked path, on small inputs)
   int filter_stores = -1;   // 1: backward filter transposes with element-sized LDS stores also where transposing reads serve
   int tall_tiles = -1;      // the gather kernel of tall tiles
+  int small_rulebook = -1;  // 0: submanifold rulebooks of few rows take the launches of larger ones
   int lists_on_trust = -1;  // pair lists of unreported order: -1 lists with the row-map kernels behind, 0 row map, 1 lists only
 };
 

@@ -1580,6 +1580,129 @@ int offsetsPerSlice(int K) {
 
 size_t rulebookWorkspaceBytes(const RulebookGeom &g) { return carve(g, nullptr).bytes; }
 
+// A whole submanifold rulebook of unit strides and at most kSmallRows rows in one launch: a
+// workgroup an offset.  Each builds the table of all cells in LDS (slots hold the highest row of
+// a cell, the cells themselves stand beside it), looks up the partners of its offset for all rows and
+// places the pairs, which are at hand in row order.  Every workgroup builds the same table again, but that
+// takes less than handing it over: such a call is a chain of launches of 2 to 5 us each, whose
+// last word the host waits for, and here the chain is one kernel.
+// The wait for the counts included, us of the general launches against this one: 3x3x3 in cell order 64 rows
+// 25.3/16.4, 2048 27.7/18.2, 4096 28.4/22.9; in no order 64 27.7/16.0, 4096 34.9/22.5; 5x5x5 in no order 64
+// 40.2/16.9, 4096 49.3/24.5; one offset in cell order 64 21.9/15.0, 4096 23.0/23.9.  A table twice the rows
+// takes 37 at 4096: a wave goes on until its longest probe sequence ends.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallPer = 4;
+constexpr int kSmallRows = kSmallThreads * kSmallPer;
+constexpr uint32_t kSmallSlots = 4 * kSmallRows;
+// (the runs of hashCell serve a wave's probes from one line of memory; here neighbours are spread)
+__device__ __forceinline__ uint32_t smallSlot(uint32_t cell) { return (cell * 0x9E3779B1u) >> 18; }
+static_assert(kSmallSlots == 1u << (32 - 18), "a slot is the product's highest bits");
+__global__ __launch_bounds__(kSmallThreads) void rbSubmSmall(GeomDev g, const int32_t *indices, bool aligned,
+                                                             int32_t *out_indices, int out_rows, int32_t *pairs,
+                                                             int32_t *indice_num, RulebookReportTarget report) {
+  constexpr int kWaves = kSmallThreads / kWave;
+  static_assert(kSmallPer * kWaves == kWave, "one lane per count in the scan");
+  __shared__ int32_t s_row[kSmallSlots];
+  __shared__ uint32_t s_cell[kSmallRows];
+  __shared__ int s_first[kWave];
+  __shared__ int s_total;
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1), wave = tid >> 6;
+  const int k = blockIdx.x;
+#pragma unroll
+  for (uint32_t i = 0; i < kSmallSlots / kSmallThreads; ++i) s_row[i * kSmallThreads + tid] = -1;
+  int4 c[kSmallPer];
+  bool bad = false;
+#pragma unroll
+  for (int u = 0; u < kSmallPer; ++u) {
+    const int j = u * kSmallThreads + tid;
+    c[u] = make_int4(-1, 0, 0, 0);
+    if (j < g.L) c[u] = loadCoord(indices, j, aligned);
+  }
+#pragma unroll
+  for (int u = 0; u < kSmallPer; ++u) {
+    const int j = u * kSmallThreads + tid;
+    const bool in_range = (unsigned)c[u].x < (unsigned)g.batch && (unsigned)c[u].y < (unsigned)g.out[0] &&
+                          (unsigned)c[u].z < (unsigned)g.out[1] && (unsigned)c[u].w < (unsigned)g.out[2];
+    s_cell[j] = in_range ? (uint32_t)(((c[u].x * g.out[0] + c[u].y) * g.out[1] + c[u].z) * g.out[2] + c[u].w)
+                         : kEmptyKey;
+    // (the order of the rows is reported once)
+    if (k == 0 && j < g.L)
+      bad = bad || !in_range || (j > 0 && !coordBelow(loadCoord(indices, j - 1, aligned), c[u]));
+  }
+  for (int r = k * kSmallThreads + tid; r < out_rows; r += (int)gridDim.x * kSmallThreads)
+    storeCoord(out_indices, r, r < g.L ? loadCoord(indices, r, aligned) : make_int4(-1, -1, -1, -1), aligned);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kSmallPer; ++u) {
+    const int j = u * kSmallThreads + tid;
+    const uint32_t cell = s_cell[j];
+    if (cell == kEmptyKey) continue;
+    uint32_t slot = smallSlot(cell);
+    // (a slot only ever passes between rows of one cell; four times as many slots as rows: an empty one is reached)
+    while (true) {
+      const int old = atomicCAS(&s_row[slot], -1, j);
+      if (old == -1) break;
+      if (s_cell[old] == cell) {
+        atomicMax(&s_row[slot], j);
+        break;
+      }
+      slot = (slot + 1) & (kSmallSlots - 1);
+    }
+  }
+  const bool unordered = __syncthreads_or(bad) != 0;
+  if (k == 0 && tid == 0) fileReport(!unordered, report);
+  const int kd = k / (g.ks[1] * g.ks[2]), kh = k / g.ks[2] % g.ks[1], kw = k % g.ks[2];
+  int partner[kSmallPer], place[kSmallPer];
+#pragma unroll
+  for (int u = 0; u < kSmallPer; ++u) {
+    partner[u] = -1;
+    const int od = axisOut(c[u].y, g.pad[0], kd, g.dil[0], 1, g.by_stride[0], g.out[0]);
+    const int oh = axisOut(c[u].z, g.pad[1], kh, g.dil[1], 1, g.by_stride[1], g.out[1]);
+    const int ow = axisOut(c[u].w, g.pad[2], kw, g.dil[2], 1, g.by_stride[2], g.out[2]);
+    if ((unsigned)c[u].x < (unsigned)g.batch && (od | oh | ow) >= 0) {
+      const uint32_t cell = (uint32_t)(((c[u].x * g.out[0] + od) * g.out[1] + oh) * g.out[2] + ow);
+      uint32_t slot = smallSlot(cell);
+      while (true) {
+        const int row = s_row[slot];
+        if (row == -1) break;
+        if (s_cell[row] == cell) {
+          partner[u] = row;
+          break;
+        }
+        slot = (slot + 1) & (kSmallSlots - 1);
+      }
+    }
+    const unsigned long long found = __ballot(partner[u] >= 0);
+    place[u] = __popcll(found & ((1ull << lane) - 1ull));
+    if (lane == 0) s_first[u * kWaves + wave] = __popcll(found);
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const int mine = s_first[lane];
+    const int incl = waveInclusiveScan(mine);
+    s_first[lane] = incl - mine;
+    if (lane == kWave - 1) s_total = incl;
+  }
+  __syncthreads();
+  const int total = s_total;
+  if (tid == 0) fileCount(k, total, indice_num, report);
+  int32_t *in_col = pairs + (size_t)k * 2 * g.L, *out_col = in_col + g.L;
+#pragma unroll
+  for (int u = 0; u < kSmallPer; ++u) {
+    const int j = u * kSmallThreads + tid;
+    if (partner[u] >= 0) {
+      const int to = s_first[u * kWaves + wave] + place[u];
+      in_col[to] = j;
+      out_col[to] = partner[u];
+    }
+    if (g.fill_tails && j >= total && j < g.L) {
+      in_col[j] = -1;
+      out_col[j] = -1;
+    }
+  }
+}
+
 hipError_t launchSubmRulebook(const LaunchCtx &lc, const RulebookGeom &g, const int32_t *indices,
                               void *workspace, int32_t *indice_pairs, int32_t *out_indices,
                               int32_t *indice_num, const RulebookReportTarget &report) {
@@ -1591,6 +1714,13 @@ hipError_t launchSubmRulebook(const LaunchCtx &lc, const RulebookGeom &g, const 
   const bool unit_stride = g.stride[0] == 1 && g.stride[1] == 1 && g.stride[2] == 1 &&
                            g.ksize[0] <= 32 && g.ksize[1] <= 32 && g.ksize[2] <= 32 &&
                            g.K <= kMaxInlineOffsets;
+  if (unit_stride && g.L <= kSmallRows && lc.choices.small_rulebook != 0) {
+    lc.begin("rbSubmSmall");
+    rbSubmSmall<<<g.K, kSmallThreads, 0, lc.stream>>>(d, indices, al, out_indices, g.out_rows, indice_pairs, indice_num,
+                                                      report);
+    lc.end();
+    return hipGetLastError();
+  }
   bool mirror = unit_stride;
   for (int a = 0; a < 3; ++a)
     if (g.ksize[a] % 2 == 0 || 2 * g.pad[a] != g.dilation[a] * (g.ksize[a] - 1)) mirror = false;

@@ -224,7 +224,7 @@ class Handle:
 
     KERNEL_CHOICES = {"gather_simt": 0, "dense_tiles": 1, "wave_per_tile": 2, "flat_slice_sum": 3,
                       "flat_scatter": 4, "small_map_chunks": 5, "filter_stores": 6,
-                      "lists_on_trust": 7, "tall_tiles": 16}   # mluOpExtKernelChoice_t
+                      "lists_on_trust": 7, "tall_tiles": 16, "small_rulebook": 17}   # mluOpExtKernelChoice_t
 
     def set_kernel_choice(self, which, value):
         """mluOpExtSetKernelChoice: value None (the shape decides), False or True."""

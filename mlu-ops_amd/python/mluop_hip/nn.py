@@ -283,7 +283,7 @@ class SparseSequential(torch.nn.Sequential):
     convolutions that follow; built up front, the host runs ahead through all convolutions and the
     device stays busy.  The counts are waited for when the last rulebook is on its way: in between, only
     a strided layer's number of output rows is (waiting for each rulebook's counts before the next
-    left the device idle some 30 us a rulebook: seven of them, voxelizer and 11-layer encoder 865 -> 817 us)."""
+    left the device idle some 30 us a rulebook: seven of them; voxelizer and 11-layer encoder 865 -> 817 us)."""
 
     def plan(self, x):
         built = []
