@@ -21,12 +21,14 @@
 //  * gatherConvMfma   up to 128 channels on both sides, in MFMA blocks of 16 pairs.  Per offset the
 //    rows of a tile that have a partner are compacted, so MFMA work follows the number of
 //    pairs, not K x rows.  Each wave owns a column slice of the fp32 accumulator tile in LDS.
+//  * gatherConvTall   the same sums for rulebooks that are thinly filled: tiles of 256 or 512 rows by 64
+//    columns, with waves that only fetch beside those that multiply.
 //  * gatherConvWave   the same for results of up to 32 columns, one wavefront a tile.
 //  * gatherConvDense  rulebooks whose (tile, offset) pieces are well filled: accumulators in
 //    registers, all rows of a tile multiplied at every offset that has a pair there.
 //  * gatherConvSimt   any channel count, LDS-tiled FMA.
 // A row takes nothing from the filter of an offset at which it has no pair, in any of them, also
-// where that filter is not finite.
+// where that filter is not finite.  Forward stores its sums behind a ReLU where the caller asks for it.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

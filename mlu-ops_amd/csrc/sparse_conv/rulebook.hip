@@ -8,9 +8,10 @@
 // at the output coordinate (output row = that input row, the highest row index
 // wins for duplicated coordinates); regular mode keeps every valid pair and
 // numbers the distinct output cells in ascending linear order.  Inside one
-// offset, pairs are listed by ascending input row; unused tails are -1.
+// offset, pairs are listed by ascending input row; unused tails are -1 (unless the caller does without).
 //
 // Kernel set
+//   submanifold, up to 4096 rows at unit strides: one launch, a workgroup an offset (rbSubmSmall)
 //   submanifold:  prepare (copy out_indices, clear the hash table, write the sorted-cell
 //                 arrays and decide whether the rows are in strict cell order) -> insert
 //                 rows into the hash table (returns at once for rows in order) -> probe
