@@ -1068,7 +1068,7 @@ constexpr int kTallCols = 64;
 constexpr int kTallWaves = 4;  // multiplying waves, and as many fetching ones
 constexpr int kTallThreads = 2 * kTallWaves * 64;
 // Two workgroups of 256 rows share a CU, but for rows of 512 bytes, of which the second would leave
-// no room for a round.
+// no room for a round.  (Few rows run in half of the 256: tallHalfTiles.)
 constexpr int tallRows(int row_bytes) { return row_bytes >= 512 ? 512 : 256; }
 constexpr TallPlan tallPlan(int row_bytes) {
   const int rows = tallRows(row_bytes);
@@ -3563,14 +3563,20 @@ int tallGridX(int R, int tile_rows) { return ((R + tile_rows - 1) / tile_rows + 
 
 template <typename E, int Q, typename SRC>
 void launchTallInstance(const LaunchCtx &lc, const void *A, uint32_t a_size, const ConvRows &rows, const void *packed,
-                        const SRC &source, int R, int K, void *result) {
+                        const SRC &source, bool half_tiles, int R, int K, void *result) {
   constexpr int TR = tallRows(Q * (int)sizeof(typename E::storage));
-  const dim3 grid(tallGridX(R, TR), (rows.c + kTallCols - 1) / kTallCols);
-  lc.begin("gatherConvTall");
-  gatherConvTall<E, Q, kTallCols, TR, SRC><<<grid, kTallThreads, 0, lc.stream>>>(
-      static_cast<const typename E::storage *>(A), a_size, rows, static_cast<const typename E::storage *>(packed), source,
-      R, K, static_cast<typename E::storage *>(result));
-  lc.end();
+  const dim3 grid(tallGridX(R, half_tiles ? TR / 2 : TR), (rows.c + kTallCols - 1) / kTallCols);
+  auto launch = [&](auto kernel) {
+    lc.begin("gatherConvTall");
+    kernel<<<grid, kTallThreads, 0, lc.stream>>>(static_cast<const typename E::storage *>(A), a_size, rows,
+                                                 static_cast<const typename E::storage *>(packed), source, R, K,
+                                                 static_cast<typename E::storage *>(result));
+    lc.end();
+  };
+  if constexpr (SRC::kSegments && TR == 256) {
+    if (half_tiles) return launch(gatherConvTall<E, Q, kTallCols, TR / 2, SRC>);
+  }
+  launch(gatherConvTall<E, Q, kTallCols, TR, SRC>);
 }
 
 // Channels of the instance for rows of q_padded channels (16 channels of a 2-byte type are half a fragment,
@@ -3579,16 +3585,16 @@ int tallQ(ElemType t, int q_padded) { return t != ElemType::kFloat && q_padded <
 
 template <typename E, typename SRC>
 void launchTall(const LaunchCtx &lc, int q, const void *A, int n_src, const ConvRows &rows, const void *packed,
-                const SRC &source, int R, int K, void *result) {
+                const SRC &source, bool half_tiles, int R, int K, void *result) {
   const uint32_t a_size = (uint32_t)n_src * (uint32_t)rows.row_bytes;
   switch (q) {
     case 16:
       if constexpr (std::is_same<E, FloatElem>::value)
-        launchTallInstance<E, 16, SRC>(lc, A, a_size, rows, packed, source, R, K, result);
+        launchTallInstance<E, 16, SRC>(lc, A, a_size, rows, packed, source, half_tiles, R, K, result);
       break;
-    case 32: launchTallInstance<E, 32, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break;
-    case 64: launchTallInstance<E, 64, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break;
-    case 128: launchTallInstance<E, 128, SRC>(lc, A, a_size, rows, packed, source, R, K, result); break;
+    case 32: launchTallInstance<E, 32, SRC>(lc, A, a_size, rows, packed, source, half_tiles, R, K, result); break;
+    case 64: launchTallInstance<E, 64, SRC>(lc, A, a_size, rows, packed, source, half_tiles, R, K, result); break;
+    case 128: launchTallInstance<E, 128, SRC>(lc, A, a_size, rows, packed, source, half_tiles, R, K, result); break;
     default: break;
   }
 }
@@ -3604,6 +3610,21 @@ bool denseShapeOk(const ConvProblem &p, const GatherDims &d) {
   // (fp32 rows of more than 64 channels leave no room for two row groups a wave)
   if (p.dtype == ElemType::kFloat && d.Q > 64) return false;
   return (uint64_t)d.n_src * (uint64_t)paddedRowBytes(p.dtype, d.Q) < (uint64_t)kNoRow;
+}
+
+// Pair lists of so few rows that tiles of 128 do not outnumber the CUs run in those (tallHalfTiles): the
+// launch is one tile long then, and half a tile is half as many blocks.  us of gatherConvMfma / tiles of 256 /
+// of 128, fp16 64 -> 64, 128 -> 128 and fp32 64 -> 64:
+//   3x3x3 in boxes      4 k rows 15/18/12.9, 19/22/15.5, 28/35/23.2;    16 k 15/19/13.5, 21/24/17.2, 30/37/24.2
+//         strewn        16 k 13/14/11.9, 16/17/14.6, 23/24/20.5;        32 k 14/15/12.7, (22/19/21.0), 26/27/21.8
+//   5x5x5 in boxes      4 k 41/39/29.4, 57/51/37.9, 88/88/64.3;         16 k 42/47/33.6, 59/58/41.6, 91/99/66.8
+//   2x2x2 stride 2      12 k 11/13/10.4, 13/14/11.6, 17/20/15.4;        3x3x3 stride 2, 26 k 15/17/13.7, -, 28/31/23.2
+// With two tiles on some CUs the tall ones win or lose with the fill (45 k strewn 17.1/15.8/17.1, in boxes
+// 24/26/22.5), so gatherConvMfma stays there; over row maps tiles of 128 are no faster than it.
+constexpr int kTallFewRows = 128 * 256;  // times 64 result columns
+bool tallHalfTiles(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d) {
+  return lc.choices.tall_tiles < 0 && tallRows(d.q_padded * (int)elemSize(p.dtype)) == 256 &&
+         (int64_t)d.R * (d.c_padded / 64) <= kTallFewRows;
 }
 
 bool useTallKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d, bool lists) {
@@ -3628,6 +3649,7 @@ bool useTallKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &
   if (fill >= (p.K <= 8 ? 0.25 : 0.16)) return false;
   const bool long_rows = d.q_padded * (int)elemSize(p.dtype) > 256;
   if (lists) {
+    if (tallHalfTiles(lc, p, d)) return true;
     if (long_rows) return work >= 85000 && pairs >= 1.1 * d.R;
     return p.K > 32 || work >= 45000;
   }
@@ -3803,12 +3825,13 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
   const bool dense = use_mfma && useDenseKernel(lc, p, d);
   const bool tall = use_mfma && !dense && useTallKernel(lc, p, d, lists);
   const int tall_q = tallQ(p.dtype, d.q_padded);
+  const bool half_tiles = tall && lists && tallHalfTiles(lc, p, d);
   if (lists) {
     // Pair lists in order (as far as the caller knows: the first kernel checks): the
     // gather kernel reads them cut by tile, no row map.
     const int tile_cols = dense ? d.c_padded : mfmaTileCols(p, d);
     const int tile_rows = dense ? denseTileRows((int)sizeof(S), d.q_padded, d.c_padded, denseWide(p, d, d.R))
-                                : (tall ? tallRows(tall_q * (int)sizeof(S)) : mfmaTileRows(tile_cols));
+                                : (tall ? tallRows(tall_q * (int)sizeof(S)) / (half_tiles ? 2 : 1) : mfmaTileRows(tile_cols));
     int tile_shift = 0;
     while ((1 << tile_shift) < tile_rows) ++tile_shift;
     const int n_tiles = (d.R + tile_rows - 1) / tile_rows;
@@ -3845,7 +3868,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     if (dense)
       launchDense<E, SegmentSource>(lc, d.q_padded, denseWide(p, d, d.R), rows_from, d.n_src, rows_of, ws.packed, src, d.R, p.K, result);
     else if (tall)
-      launchTall<E, SegmentSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, src, d.R, p.K, result);
+      launchTall<E, SegmentSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, src, half_tiles, d.R, p.K, result);
     else if (tile_cols == d.c_padded && useWaveKernel(lc, p.dtype, d.q_padded, d.c_padded))
       launchWave<E>(lc, d.q_padded, rows_from, rows_of, ws.packed, src, d.R, p.K, result);
     else
@@ -3889,7 +3912,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
         launchDense<E, MapSource>(lc, d.q_padded, wide, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K, result_rows);
       } else if (tall) {
         n_filled = tallGridX(rows, tallRows(tall_q * (int)sizeof(S)));
-        launchTall<E, MapSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K, result_rows);
+        launchTall<E, MapSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, map, false, rows, p.K, result_rows);
       } else {
         n_filled = mfmaGridX(rows, tile_cols);
         launchMfma<E, MapSource>(lc, d.q_padded, tile_cols, rows_from, rows_of, ws.packed, map, rows, p.K, result_rows);

@@ -1,0 +1,46 @@
+"""Few result rows take the tall gather kernel's tiles of 128 rows: the bits of the pair-list kernel of short tiles in
+both directions, at row counts around its tiles and at the last row count that is one tile a CU."""
+import pytest
+
+from test_gpu_pair_lists import kernels_of
+from test_gpu_tall_tiles import make_case
+
+pytestmark = pytest.mark.gpu
+
+
+def both(handle, case, tall):
+    import mluop_hip as m
+    handle.set_kernel_choice("dense_tiles", False)
+    handle.set_kernel_choice("tall_tiles", tall)
+    try:
+        out, forward = kernels_of(handle, lambda: m.indice_conv_forward(
+            handle, case["x"], case["w"], m.LAYOUT_ARRAY, case["pairs"], case["num"], case["n_out"], case["sub_m"]))
+        dx, backward = kernels_of(handle, lambda: m.indice_conv_backward_data(
+            handle, case["dy"], case["w"], m.LAYOUT_ARRAY, case["pairs"], case["num"], case["sub_m"], case["ci"]))
+    finally:
+        handle.set_kernel_choice("dense_tiles", None)
+        handle.set_kernel_choice("tall_tiles", None)
+    return out, dx, "gatherConvTall" in forward, "gatherConvTall" in backward
+
+
+def few(rows, q, c, size):
+    q, c = (next(p for p in (16, 32, 64, 128) if p >= n) for n in (q, c))
+    return c >= 64 and q * size <= 256 and rows * (c // 64) <= 32768
+
+
+@pytest.mark.parametrize("ci,co", [(64, 64), (5, 128), (16, 64), (33, 100), (64, 128)])
+@pytest.mark.parametrize("dtype_name", ["float16", "bfloat16", "float32"])
+@pytest.mark.parametrize("ks,rows,space", [((3, 3, 3), 1, (9, 30, 40)), ((3, 3, 3), 127, (9, 30, 40)),
+                                           ((3, 3, 3), 129, (9, 30, 40)), ((3, 3, 3), 1100, (9, 30, 40)),
+                                           ((5, 5, 5), 700, (9, 30, 40)), ((3, 3, 3), 16384, (20, 160, 160)),
+                                           ((3, 3, 3), 16385, (20, 160, 160))])
+def test_bits_of_the_short_tiles(gpu_handle, ci, co, dtype_name, ks, rows, space):
+    import torch
+    print("tall, few rows", ci, co, dtype_name, ks, rows, flush=True)
+    case = make_case(gpu_handle, rows, space, ks, ci, co, dtype_name, False)
+    out, dx, forward, backward = both(gpu_handle, case, None)
+    ref_out, ref_dx, plain_f, plain_b = both(gpu_handle, case, False)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref_out) and torch.equal(dx, ref_dx) and not plain_f and not plain_b
+    size = 4 if dtype_name == "float32" else 2
+    assert forward == few(rows, ci, co, size) and backward == few(rows, co, ci, size)
