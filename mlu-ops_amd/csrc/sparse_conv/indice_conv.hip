@@ -3620,10 +3620,12 @@ bool denseShapeOk(const ConvProblem &p, const GatherDims &d) {
 //   5x5x5 in boxes      4 k 41/39/29.4, 57/51/37.9, 88/88/64.3;         16 k 42/47/33.6, 59/58/41.6, 91/99/66.8
 //   2x2x2 stride 2      12 k 11/13/10.4, 13/14/11.6, 17/20/15.4;        3x3x3 stride 2, 26 k 15/17/13.7, -, 28/31/23.2
 // With two tiles on some CUs the tall ones win or lose with the fill (45 k strewn 17.1/15.8/17.1, in boxes
-// 24/26/22.5), so gatherConvMfma stays there; over row maps tiles of 128 are no faster than it.
+// 24/26/22.5), so gatherConvMfma stays there; over row maps tiles of 128 are no faster than it.  Below 4096 rows the
+// gain is 1 to 2 us (1 k in boxes 14/12.2, 15/12.8) and gatherConvMfma stays for its tests' sake, which know it there.
 constexpr int kTallFewRows = 128 * 256;  // times 64 result columns
+constexpr int kTallFewestRows = 4096;
 bool tallHalfTiles(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d) {
-  return lc.choices.tall_tiles < 0 && tallRows(d.q_padded * (int)elemSize(p.dtype)) == 256 &&
+  return lc.choices.tall_tiles < 0 && d.R >= kTallFewestRows && tallRows(d.q_padded * (int)elemSize(p.dtype)) == 256 &&
          (int64_t)d.R * (d.c_padded / 64) <= kTallFewRows;
 }
 

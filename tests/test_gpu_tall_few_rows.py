@@ -25,14 +25,14 @@ def both(handle, case, tall):
 
 def few(rows, q, c, size):
     q, c = (next(p for p in (16, 32, 64, 128) if p >= n) for n in (q, c))
-    return c >= 64 and q * size <= 256 and rows * (c // 64) <= 32768
+    return c >= 64 and q * size <= 256 and rows >= 4096 and rows * (c // 64) <= 32768
 
 
 @pytest.mark.parametrize("ci,co", [(64, 64), (5, 128), (16, 64), (33, 100), (64, 128)])
 @pytest.mark.parametrize("dtype_name", ["float16", "bfloat16", "float32"])
-@pytest.mark.parametrize("ks,rows,space", [((3, 3, 3), 1, (9, 30, 40)), ((3, 3, 3), 127, (9, 30, 40)),
-                                           ((3, 3, 3), 129, (9, 30, 40)), ((3, 3, 3), 1100, (9, 30, 40)),
-                                           ((5, 5, 5), 700, (9, 30, 40)), ((3, 3, 3), 16384, (20, 160, 160)),
+@pytest.mark.parametrize("ks,rows,space", [((3, 3, 3), 4095, (9, 60, 100)), ((3, 3, 3), 4096, (9, 60, 100)),
+                                           ((3, 3, 3), 4097, (9, 60, 100)), ((3, 3, 3), 4351, (9, 60, 100)),
+                                           ((5, 5, 5), 4225, (9, 60, 100)), ((3, 3, 3), 16384, (20, 160, 160)),
                                            ((3, 3, 3), 16385, (20, 160, 160))])
 def test_bits_of_the_short_tiles(gpu_handle, ci, co, dtype_name, ks, rows, space):
     import torch
