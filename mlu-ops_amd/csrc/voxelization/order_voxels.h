@@ -12,8 +12,8 @@
 namespace mluop {
 namespace voxelization {
 
-// Most voxels one call accepts: voxels of one bucket are compared with each other, and coordinates
-// outside the grid all share one.
+// Most voxels one call accepts: a voxel of a crowded bucket is looked up in all its runs of 4096, and
+// coordinates outside the grid all share a bucket.
 constexpr int64_t kMaxOrderedVoxels = (int64_t)1 << 20;
 
 struct OrderShape {
