@@ -3620,13 +3620,22 @@ bool denseShapeOk(const ConvProblem &p, const GatherDims &d) {
 //   5x5x5 in boxes      4 k 41/39/29.4, 57/51/37.9, 88/88/64.3;         16 k 42/47/33.6, 59/58/41.6, 91/99/66.8
 //   2x2x2 stride 2      12 k 11/13/10.4, 13/14/11.6, 17/20/15.4;        3x3x3 stride 2, 26 k 15/17/13.7, -, 28/31/23.2
 // With two tiles on some CUs the tall ones win or lose with the fill (45 k strewn 17.1/15.8/17.1, in boxes
-// 24/26/22.5), so gatherConvMfma stays there; over row maps tiles of 128 are no faster than it.  Below 4096 rows the
-// gain is 1 to 2 us (1 k in boxes 14/12.2, 15/12.8) and gatherConvMfma stays for its tests' sake, which know it there.
+// 24/26/22.5), so gatherConvMfma stays there; over row maps tiles of 128 are no faster than it.
+// More than 32 offsets run in them from the first row on: with tiles of 256, which take all longer lists of so
+// many offsets, a layer of few rows is slower than one of more, and than gatherConvMfma at 63 offsets:
+//   5x5x5 in boxes      64 rows 37/26/25.7, 52/33/32.8, 78/57/56;       1 k 43/41/28.5, 59/52/37.0, 89/90/63.7
+//                       3 k 42/42/32.5, 57/53/37.7, 90/92/65.0
+//         strewn        128 rows 22/13/12.8, 24/13/12.3, 27/16/15.9;    2 k 36/32/25.5, 46/36/31.0, 70/63/52.7
+//   3x3x7 in boxes      64 rows 24/17/16.8, 32/21/20.3, 47/34/33.7;     3 k 26/29/20.7, 34/36/22.4, 53/62/37.0
+// Up to 32 offsets gatherConvMfma stays below 4096 rows.  These tiles are ahead there too (3x3x3 in boxes, 64 rows
+// 13/12/11.4, 16/13/13.1, 23/20/19.5; 1 k 14/18/12.8, 19/22/14.4, 27/35/21.5; 3 k 15/18/12.9, 19/21/15.1, 28/35/22.9), by 1 to
+// 6 us of a layer's 50 to 100: a lower line is open, and no measurement speaks for this one.
 constexpr int kTallFewRows = 128 * 256;  // times 64 result columns
-constexpr int kTallFewestRows = 4096;
+constexpr int kTallFewestRows = 4096;    // with up to kTallFewOffsets offsets
+constexpr int kTallFewOffsets = 32;
 bool tallHalfTiles(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d) {
-  return lc.choices.tall_tiles < 0 && d.R >= kTallFewestRows && tallRows(d.q_padded * (int)elemSize(p.dtype)) == 256 &&
-         (int64_t)d.R * (d.c_padded / 64) <= kTallFewRows;
+  return lc.choices.tall_tiles < 0 && (p.K > kTallFewOffsets || d.R >= kTallFewestRows) &&
+         tallRows(d.q_padded * (int)elemSize(p.dtype)) == 256 && (int64_t)d.R * (d.c_padded / 64) <= kTallFewRows;
 }
 
 bool useTallKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d, bool lists) {
@@ -3653,7 +3662,7 @@ bool useTallKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &
   if (lists) {
     if (tallHalfTiles(lc, p, d)) return true;
     if (long_rows) return work >= 85000 && pairs >= 1.1 * d.R;
-    return p.K > 32 || work >= 45000;
+    return p.K > kTallFewOffsets || work >= 45000;
   }
   return !long_rows && p.K <= 32 && d.q_padded >= 64 && work >= (d.c_padded == 128 ? 50000 : 80000);
 }
