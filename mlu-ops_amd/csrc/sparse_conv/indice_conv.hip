@@ -1720,11 +1720,10 @@ constexpr int kDenseMapBatch = 14;   // loads in flight per thread while a tile'
 // and SIMD.  Short rows: as many workgroups as registers and LDS allow.  Rows above 128 bytes: two
 // workgroups of four waves, of which one multiplies while the other builds its row map and waits for its
 // first rows (8.7 of a tile's 42 us at 128 -> 128 channels, with one workgroup of eight waves a CU); the ring
-// then holds one offset a phase at 128 columns instead of two, and every 128 rows load the filters again,
-// which costs more from about 220 000 rows on (`wide`: eight waves).  us, eight waves against twice four:
-//   fp16 128 -> 128   8 k rows 47/39, 30 k 52/42, 80 k 96/87, 150 k 161/147, 250 k 214/222
-//        128 -> 64    8 k 32/27, 80 k 70/71, 150 k 135/114, 250 k 171/161;  128 -> 32  30 k 42/28, 250 k 158/147
-//   fp32  64 -> 64    8 k 105/68, 30 k 114/70, 80 k 182/162, 150 k 280/271;  64 -> 128  30 k 218/127, 150 k 549/537
+// then holds one offset a phase at 128 columns instead of two, and every 128 rows load the filters again.
+// At 128 columns eight waves stay for some row counts (`wide`, denseWide).  us, eight waves against twice four:
+//   fp16 128 -> 64    8 k 32/27, 80 k 70/71, 150 k 135/114, 250 k 171/161;  128 -> 32  30 k 42/28, 250 k 158/147
+//   fp32  64 -> 64    8 k 105/68, 30 k 114/70, 80 k 182/162, 150 k 280/271
 enum class DenseRows { kByPhase, kStaged, kInPlace };  // how rows reach the operand registers
 struct DensePlan {
   int waves;        // per workgroup
@@ -3714,9 +3713,24 @@ bool useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims 
   return sheets && d.q_padded <= 32 && fill >= 0.2;
 }
 
-// Whether the kernel takes its wide tiles (densePlan).
+// Whether the kernel takes its wide tiles (densePlan).  Either shape has 256 rows on each of 256 CUs at a time,
+// so a launch takes rows / 65 536 rounds.  Up to half a CU's rows in the last round take the narrow tiles
+// half the time, and the wide ones that of a whole tile; in a round that is nearly full the narrow ones
+// pay for their phases of one offset and their second filters.  With more rounds the two come closer.  us of
+// gatherConvDense, wide / narrow, 27 offsets, by rounds:
+//   fp16 128 -> 128 scene   0.50 49/41, 0.60 49/50, 0.85 51/53, 1.00 53/56, 1.10 84/73, 1.40 96/88, 1.60 102/104,
+//                           2.00 104/113, 2.10 140/120, 2.60 142/141, 2.85 152/154, 3.30 203/180, 4.00 217/218
+//           strewn          0.50 45/41, 0.60 47/51, 1.10 93/82, 1.60 97/101, 2.00 104/113, 2.60 155/161, 3.00 163/181,
+//                           3.30 207/195, 4.00 225/229, 4.40 272/259, 4.70 271/288
+//           scene, row map  0.30 50/39, 0.60 53/55, 1.30 102/89, 1.85 113/117, 2.60 170/173, 2.85 174/188, 3.60 233/239
+//   bf16 96 -> 128 scene    0.50 50/42, 0.60 50/50, 1.00 52/54, 1.30 86/80, 1.60 88/91, 2.00 97/101, 2.60 141/131,
+//                           2.85 145/148, 3.30 168/161, 4.00 196/198
+//   fp32 64 -> 128 strewn   0.92 205/216, 1.04 392/320, 1.53 422/434, 2.06 630/559, 2.75 639/681
+// and a layer's training step on scenes, 128 -> 128, where the rows come from memory: 1.98 362/378, 2.90 523/527,
+// 3.43 619/589, 3.66 623/622, 3.79 632/648.
 bool denseWide(const ConvProblem &p, const GatherDims &d, int rows) {
-  return d.q_padded * (int)elemSize(p.dtype) > 128 && d.c_padded == 128 && rows >= 220000;
+  constexpr int kRound = 256 * 256;
+  return d.q_padded * (int)elemSize(p.dtype) > 128 && d.c_padded == 128 && (rows - 1) % kRound >= kRound * 2 / 3;
 }
 
 template <typename E, int Q, int C, typename SRC>

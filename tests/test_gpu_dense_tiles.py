@@ -1,12 +1,14 @@
-"""The dense gather kernel's two tile shapes for rows above 128 bytes: which one runs goes by the number of
-result rows, and both are held to sums in 64 bits, on either side of the line."""
+"""The dense gather kernel's two tile shapes for rows above 128 bytes: which one runs goes by how full the number of
+result rows leaves the last round of tiles (65 536 rows: wide from two thirds on), and both are held
+to sums in 64 bits, on either side of the lines."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("rows", [219_999, 220_000, 220_129])
+@pytest.mark.parametrize("rows", [219_999, 220_000, 220_129, 43_690, 43_691, 65_536, 65_537, 109_226, 109_227, 131_073,
+                                  196_608, 196_609])
 @pytest.mark.parametrize("dtype_name,ci,co", [("float16", 128, 128), ("bfloat16", 96, 65), ("float32", 64, 100)])
 @pytest.mark.parametrize("order", ["cell", "mixed"])
 def test_forward_on_either_side_of_the_wide_tiles(gpu_handle, rows, dtype_name, ci, co, order):
