@@ -89,12 +89,15 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtSetDistinctPairsPromise(mluOpHandle_t handle
 /* Whether mluOpGetIndicePairs sets the slots of indice_pairs behind each offset's indice_num pairs to -1 (the
  * default, and what the reference does).  0: it leaves them as they are, which saves most of a sparse
  * rulebook's writes; for callers who, like the indice-convolution operators, read no further than
- * indice_num.  Holds for the handle until changed. */
+ * indice_num.  Holds for the handle until changed.  The second call says which of the two is in force, for
+ * callers who change it for a while. */
 mluOpStatus_t MLUOP_WIN_API mluOpExtSetPairTails(mluOpHandle_t handle, int fill);
+mluOpStatus_t MLUOP_WIN_API mluOpExtGetPairTails(mluOpHandle_t handle, int *fill);
 
 /* mluOpIndiceConvolutionForward stores negative results as zero (NaN stays NaN) while this is on: the ReLU
  * behind a layer without a pass of its own over the result.  Off for a new handle; holds until changed. */
 mluOpStatus_t MLUOP_WIN_API mluOpExtSetForwardRelu(mluOpHandle_t handle, int enable);
+mluOpStatus_t MLUOP_WIN_API mluOpExtGetForwardRelu(mluOpHandle_t handle, int *enable);
 
 /* The pair counts of a rulebook on the host.  The convolution operators take indice_num as a host
  * array, so a caller has to bring the counts mluOpGetIndicePairs left in device memory over; a copy

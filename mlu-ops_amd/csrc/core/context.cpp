@@ -214,9 +214,23 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtSetForwardRelu(mluOpHandle_t handle, int ena
   return MLUOP_STATUS_SUCCESS;
 }
 
+mluOpStatus_t MLUOP_WIN_API mluOpExtGetForwardRelu(mluOpHandle_t handle, int *enable) {
+  PARAM_CHECK("[mluOpExtGetForwardRelu]", handle != NULL);
+  PARAM_CHECK("[mluOpExtGetForwardRelu]", enable != NULL);
+  *enable = handle->forward_relu ? 1 : 0;
+  return MLUOP_STATUS_SUCCESS;
+}
+
 mluOpStatus_t MLUOP_WIN_API mluOpExtSetPairTails(mluOpHandle_t handle, int fill) {
   PARAM_CHECK("[mluOpExtSetPairTails]", handle != NULL);
   handle->fill_pair_tails = fill != 0;
+  return MLUOP_STATUS_SUCCESS;
+}
+
+mluOpStatus_t MLUOP_WIN_API mluOpExtGetPairTails(mluOpHandle_t handle, int *fill) {
+  PARAM_CHECK("[mluOpExtGetPairTails]", handle != NULL);
+  PARAM_CHECK("[mluOpExtGetPairTails]", fill != NULL);
+  *fill = handle->fill_pair_tails ? 1 : 0;
   return MLUOP_STATUS_SUCCESS;
 }
 

@@ -60,7 +60,9 @@ namespace {
   X(mluOpExtSetSparseConvExtendedModes)                    \
   X(mluOpExtSetDistinctPairsPromise)                       \
   X(mluOpExtSetPairTails)                                  \
+  X(mluOpExtGetPairTails)                                  \
   X(mluOpExtSetForwardRelu)                                \
+  X(mluOpExtGetForwardRelu)                                \
   X(mluOpExtGetOrderVoxelsWorkspaceSize)                   \
   X(mluOpExtOrderVoxels)                                   \
   X(mluOpExtGetIndicePairsHostCounts)                      \
@@ -209,6 +211,25 @@ class ConvDesc {
   mluOpSparseConvolutionDescriptor_t d_ = nullptr;
 };
 
+// A setting of a handle has this value while this is there, and the caller's again afterwards.
+class Setting {
+ public:
+  using Get = mluOpStatus_t (*)(mluOpHandle_t, int *);
+  using Set = mluOpStatus_t (*)(mluOpHandle_t, int);
+  Setting(mluOpHandle_t handle, Get get, Set set, int value, const char *what) : handle_(handle), set_(set) {
+    check(get(handle, &before_), what);
+    check(set(handle, value), what);
+  }
+  ~Setting() { (void)set_(handle_, before_); }
+  Setting(const Setting &) = delete;
+  Setting &operator=(const Setting &) = delete;
+
+ private:
+  mluOpHandle_t handle_;
+  Set set_;
+  int before_ = 0;
+};
+
 // The pair counts of a rulebook built on `handle`, as soon as they are there; false: not on file.
 bool hostCounts(mluOpHandle_t handle, const at::Tensor &pairs, Counts *counts) {
   counts->assign(pairs.size(0), 0);
@@ -251,12 +272,14 @@ Rulebook3 indicePairs(mluOpHandle_t handle, const Buffers &buffers, const at::Te
   check(api.mluOpGetIndicePairsWorkspaceSize(handle, conv, d_in, d_pairs, d_out, d_num, &bytes),
         "mluOpGetIndicePairsWorkspaceSize");
   const at::Tensor ws = buffers.workspace(bytes);
-  if (!tails) check(api.mluOpExtSetPairTails(handle, 0), "mluOpExtSetPairTails");
-  const mluOpStatus_t built =
-      api.mluOpGetIndicePairs(handle, conv, d_in, indices.data_ptr(), ws.data_ptr(), bytes, d_pairs,
-                              r.pairs.data_ptr(), d_out, r.out_indices.data_ptr(), d_num, r.indice_num.data_ptr());
-  if (!tails) check(api.mluOpExtSetPairTails(handle, 1), "mluOpExtSetPairTails");
-  check(built, "mluOpGetIndicePairs");
+  {
+    std::optional<Setting> without;
+    if (!tails) without.emplace(handle, api.mluOpExtGetPairTails, api.mluOpExtSetPairTails, 0, "mluOpExtSetPairTails");
+    check(api.mluOpGetIndicePairs(handle, conv, d_in, indices.data_ptr(), ws.data_ptr(), bytes, d_pairs,
+                                  r.pairs.data_ptr(), d_out, r.out_indices.data_ptr(), d_num,
+                                  r.indice_num.data_ptr()),
+          "mluOpGetIndicePairs");
+  }
   r.num_act_out = L;
   if (!sub_m) {
     int n = 0;
@@ -505,22 +528,6 @@ struct LayerRulebook : torch::CustomClassHolder {
 };
 using LayerRulebookPtr = c10::intrusive_ptr<LayerRulebook>;
 
-// The handle's forward convolutions store negative results as zero while this is there.
-class ReluOn {
- public:
-  ReluOn(mluOpHandle_t handle, bool on) : handle_(on ? handle : nullptr) {
-    if (on) check(api.mluOpExtSetForwardRelu(handle, 1), "mluOpExtSetForwardRelu");
-  }
-  ~ReluOn() {
-    if (handle_ != nullptr) api.mluOpExtSetForwardRelu(handle_, 0);
-  }
-  ReluOn(const ReluOn &) = delete;
-  ReluOn &operator=(const ReluOn &) = delete;
-
- private:
-  mluOpHandle_t handle_;
-};
-
 struct IndiceConv : torch::autograd::Function<IndiceConv> {
   static at::Tensor forward(torch::autograd::AutogradContext *ctx, const at::Tensor &features,
                             const at::Tensor &weight, const LayerRulebookPtr &rb, bool inverse, bool share_row_maps,
@@ -538,7 +545,7 @@ struct IndiceConv : torch::autograd::Function<IndiceConv> {
     const void *map = share_row_maps ? rb->rowMap(h, buffers, inverse ? 0 : 1) : nullptr;
     // an inverse layer runs the partner layer's rulebook backwards: one output row per input
     // row of the partner
-    const ReluOn on(h.handle, relu);
+    const Setting stored(h.handle, api.mluOpExtGetForwardRelu, api.mluOpExtSetForwardRelu, relu, "mluOpExtSetForwardRelu");
     const at::Tensor out = inverse ? convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts,
                                                  rb->pairs.size(2), false, 1, map)
                                    : convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts,

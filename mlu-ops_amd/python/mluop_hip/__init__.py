@@ -127,7 +127,9 @@ SIGNATURES = {
     "mluOpExtSetSparseConvExtendedModes": (ctypes.c_int, [_vp, ctypes.c_int]),
     "mluOpExtSetDistinctPairsPromise": (ctypes.c_int, [_vp, ctypes.c_int]),
     "mluOpExtSetPairTails": (ctypes.c_int, [_vp, ctypes.c_int]),
+    "mluOpExtGetPairTails": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int)]),
     "mluOpExtSetForwardRelu": (ctypes.c_int, [_vp, ctypes.c_int]),
+    "mluOpExtGetForwardRelu": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int)]),
     "mluOpExtGetOrderVoxelsWorkspaceSize": (ctypes.c_int, [ctypes.c_int64, _vp, _vp]),
     "mluOpExtOrderVoxels": (ctypes.c_int, [_vp, _vp, ctypes.c_int64, _vp, ctypes.c_int32, _vp, ctypes.c_size_t, _vp, _vp]),
     "mluOpExtGetVoxelizationHostCount": (ctypes.c_int, [_vp, _vp, ctypes.POINTER(ctypes.c_int32)]),

@@ -628,6 +628,20 @@ def test_inverse_keeps_the_reference_status_until_switched_on(handle):
     assert m.lib().mluOpExtSetSparseConvExtendedModes(None, 1) == STATUS["MLUOP_STATUS_BAD_PARAM"]
 
 
+def test_settings_of_a_handle_can_be_asked_for(handle):
+    lib = m.lib()
+    for default, get, put in ((1, lib.mluOpExtGetPairTails, lib.mluOpExtSetPairTails),
+                              (0, lib.mluOpExtGetForwardRelu, lib.mluOpExtSetForwardRelu)):
+        value = ctypes.c_int(-1)
+        for now in (default, 0, 1, default):
+            if now != default or value.value >= 0:
+                assert put(handle.ptr, now) == 0
+            assert get(handle.ptr, ctypes.byref(value)) == 0 and value.value == now
+        assert get(handle.ptr, None) == STATUS["MLUOP_STATUS_BAD_PARAM"]
+        assert get(None, ctypes.byref(value)) == STATUS["MLUOP_STATUS_BAD_PARAM"]
+        assert put(None, 1) == STATUS["MLUOP_STATUS_BAD_PARAM"]
+
+
 def test_inverse_shape_checks(extended):
     K, L, n_in, ci, co = 8, 10, 6, 4, 5
     num = [3] * K

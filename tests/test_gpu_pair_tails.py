@@ -34,3 +34,46 @@ def test_lists_without_tails(gpu_handle, ks, stride, dilation, sub_m, shuffle, r
     for k, n in enumerate(num.cpu().tolist()):
         assert torch.equal(pairs[k, :, :n], bare[k, :, :n])
         assert (pairs[k, :, n:] == -1).all() and torch.equal(pairs[k], again[0][k])
+
+
+@pytest.mark.parametrize("own", [0, 1])
+def test_the_callers_settings_outlive_a_call(gpu_handle, own):
+    """A call and a layer that change a setting of the handle for themselves leave it as the caller had it."""
+    import ctypes
+    import torch
+    import mluop_hip as m
+    from mluop_hip import nn as spnn
+    lib, space, rows = m.lib(), (9, 18, 20), 500
+    idx = torch.from_numpy(random_voxels(np.random.default_rng(3), 1, space, rows, shuffle=False)).cuda()
+
+    def setting(handle, get):
+        value = ctypes.c_int(-1)
+        m.check(get(handle.ptr, ctypes.byref(value)))
+        return value.value
+
+    def build(handle, **kwargs):
+        return m.get_indice_pairs(handle, idx, 1, space, (3, 3, 3), space, [1] * 3, [1] * 3, [1] * 3, True, **kwargs)
+
+    m.check(lib.mluOpExtSetPairTails(gpu_handle.ptr, own))
+    try:
+        build(gpu_handle, tails=False)
+        assert setting(gpu_handle, lib.mluOpExtGetPairTails) == own
+        with pytest.raises(m.MluOpError):  # (output space of another size: refused)
+            m.get_indice_pairs(gpu_handle, idx, 1, space, (3, 3, 3), (9, 18, 21), [1] * 3, [1] * 3, [1] * 3, True,
+                               out_rows=rows, tails=False)
+        assert setting(gpu_handle, lib.mluOpExtGetPairTails) == own
+    finally:
+        m.check(lib.mluOpExtSetPairTails(gpu_handle.ptr, 1))
+
+    handle = spnn._handle()  # the layers' own: what is set on it does not reach into a layer without a ReLU
+    conv = spnn.SubMConv3d(16, 16, 3).cuda()
+    x = spnn.SparseTensor(torch.randn(rows, 16, device="cuda"), idx, space, 1, distinct=True)
+    with torch.no_grad():
+        plain = conv(x).features
+        handle.set_forward_relu(own)
+        try:
+            assert torch.equal(conv(x).features, plain)
+            assert torch.equal(spnn.SparseSequential(conv, torch.nn.ReLU())(x).features, plain.relu())
+            assert setting(handle, lib.mluOpExtGetForwardRelu) == own
+        finally:
+            handle.set_forward_relu(False)
