@@ -47,18 +47,20 @@ def share_row_maps(enable):
 
 
 class Rulebook:
-    """indice_pairs [K,2,L] (device; what lies behind an offset's indice_num pairs is not defined),
-    indice_num as host ints (where `indice_num_host` is the device tensor, those that the handle `built_on` has on
-    file, waited for when first asked for), out_indices, num_act_out."""
+    """indice_pairs [K,2,L] (device; -1 behind an offset's indice_num pairs, with `tails` off only once `pairs` has
+    been asked for: the operators read no further than the pairs), indice_num as host ints (where
+    `indice_num_host` is the device tensor, those that the handle `built_on` has on file, waited for when first
+    asked for), out_indices, num_act_out."""
 
     def __init__(self, pairs, out_indices, indice_num_host, num_act_out, filter_space, sub_m, out_space,
-                 in_indices=None, in_space=None, distinct=False, built_on=None):
+                 in_indices=None, in_space=None, distinct=False, built_on=None, tails=True):
         # the input coordinates were distinct: no offset names a result row twice, and the
         # operators may skip their check for such pairs (mluOpExtSetDistinctPairsPromise)
         self.distinct = distinct
         self.in_indices = in_indices  # what an inverse convolution over this rulebook gives back
         self.in_space = None if in_space is None else tuple(in_space)
-        self.pairs = pairs
+        self._pairs = pairs
+        self._tails = tails
         self.out_indices = out_indices
         self._indice_num = indice_num_host
         self._built_on = built_on
@@ -69,10 +71,23 @@ class Rulebook:
         self._for_operators = None
 
     @property
+    def pairs(self):
+        if not self._tails:
+            num = torch.tensor(self.indice_num, device=self._pairs.device).view(-1, 1, 1)
+            with torch.inference_mode(self._pairs.is_inference()):
+                self._pairs.masked_fill_(torch.arange(self._pairs.shape[2], device=num.device) >= num, -1)
+            self._tails = True
+        return self._pairs
+
+    @pairs.setter
+    def pairs(self, value):
+        self._pairs, self._tails = value, True
+
+    @property
     def indice_num(self):
         num = self._indice_num
         if isinstance(num, torch.Tensor):
-            self._indice_num = num = rulebook_counts(self._built_on, self.pairs, num)
+            self._indice_num = num = rulebook_counts(self._built_on, self._pairs, num)
         return num
 
     @indice_num.setter
@@ -82,7 +97,7 @@ class Rulebook:
     def for_operators(self):
         """What the native operators take of this rulebook; it holds the row maps they share."""
         if self._for_operators is None:
-            self._for_operators = native().LayerRulebook(self.pairs, self.indice_num, self.num_act_out,
+            self._for_operators = native().LayerRulebook(self._pairs, self.indice_num, self.num_act_out,
                                                          list(self.filter_space), self.sub_m, self.distinct)
         return self._for_operators
 
@@ -173,7 +188,7 @@ class _ConvBase(torch.nn.Module):
             self.stride, self.dilation, self.sub_m, for_layer=True, tails=False, wait_counts=wait_counts)
         rb = Rulebook(pairs, out_indices, num, n_out, self.kernel_size, self.sub_m,
                       out_space, in_indices=x.indices, in_space=x.spatial_shape, distinct=x.distinct,
-                      built_on=handle)
+                      built_on=handle, tails=False)
         if self.indice_key is not None:
             x.rulebooks[self.indice_key] = rb
         else:

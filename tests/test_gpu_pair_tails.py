@@ -77,3 +77,33 @@ def test_the_callers_settings_outlive_a_call(gpu_handle, own):
             assert setting(handle, lib.mluOpExtGetForwardRelu) == own
         finally:
             handle.set_forward_relu(False)
+
+
+@pytest.mark.parametrize("layer,rows", [("subm", 1), ("subm", 1300), ("strided", 700), ("network", 900)])
+@pytest.mark.parametrize("inference", [False, True])
+def test_the_pairs_of_a_layers_rulebook(gpu_handle, layer, rows, inference):
+    """Whoever asks a layer's rulebook for its pairs finds -1 behind them, as in the operator's own result."""
+    import torch
+    import mluop_hip as m
+    from mluop_hip import nn as spnn
+    print("layer's pairs", layer, rows, inference, flush=True)
+    space, ks = (9, 18, 20), 3
+    idx = torch.from_numpy(random_voxels(np.random.default_rng(rows), 1, space, rows, shuffle=True)).cuda()
+    conv = (spnn.SparseConv3d(16, 16, ks, stride=2, padding=1, indice_key="a") if layer == "strided"
+            else spnn.SubMConv3d(16, 16, ks, indice_key="a"))
+    net = (spnn.SparseSequential(conv, torch.nn.ReLU()) if layer == "network" else conv).cuda()
+    sub_m = layer != "strided"
+    ospace = list(space) if sub_m else out_space(space, [ks] * 3, [1] * 3, [2] * 3, [1] * 3)
+    want, _, num, _ = m.get_indice_pairs(gpu_handle, idx, 1, space, [ks] * 3, ospace, [1] * 3, [1 if sub_m else 2] * 3,
+                                         [1] * 3, sub_m)
+    poison = [torch.full((27, 2, rows), 7, dtype=torch.int32, device="cuda") for _ in range(4)]
+    torch.cuda.synchronize()
+    del poison   # (so that the layer's tensor is one that held something else)
+    with torch.inference_mode(inference):
+        x = spnn.SparseTensor(torch.randn(rows, 16, device="cuda"), idx, space, 1, distinct=True)
+        first = net(x).features
+    rb = x.rulebooks["a"]
+    assert rb.indice_num == [int(n) for n in num.cpu()]
+    assert torch.equal(rb.pairs, want)
+    with torch.no_grad():
+        assert torch.equal(net(x).features, first)
