@@ -270,19 +270,24 @@ def _unwatched():
                 torch._C._functorch.peek_interpreter_stack() is not None)
 
 
-def _plain_call(m):
-    """Whether calling module `m` comes to its class's forward and nothing else."""
-    return not ("forward" in m.__dict__ or m._forward_hooks or m._forward_pre_hooks or
-                m._backward_hooks or m._backward_pre_hooks or
-                torch.nn.modules.module._has_any_global_hook())
+_MODULE_CALL, _CONV_FORWARD, _RELU_FORWARD = torch.nn.Module.__call__, _ConvBase.forward, torch.nn.ReLU.forward
+
+
+def _plain_call(m, forward):
+    """Whether calling module `m` comes to the function `forward` and nothing else."""
+    return (type(m).forward is forward and type(m).__call__ is _MODULE_CALL and m._compiled_call_impl is None and
+            not ("forward" in m.__dict__ or m._forward_hooks or m._forward_pre_hooks or
+                 m._backward_hooks or m._backward_pre_hooks or
+                 torch.nn.modules.module._has_any_global_hook()))
 
 
 def _relu_in_store(conv, relu):
     """Whether the convolution `conv` can store what the module `relu` behind it would make of its result.
     Only where the layers' own calls would run and nobody could see the result in between: the library's
-    layer types without a bias, exactly torch.nn.ReLU, no hook, no mode that watches torch's calls."""
+    layer types without a bias, exactly torch.nn.ReLU, no hook, nothing compiled or put in a method's place, no
+    mode that watches torch's calls."""
     return (type(conv) in (SubMConv3d, SparseConv3d, SparseInverseConv3d) and type(relu) is torch.nn.ReLU and
-            conv.bias is None and _plain_call(conv) and _plain_call(relu) and
+            conv.bias is None and _plain_call(conv, _CONV_FORWARD) and _plain_call(relu, _RELU_FORWARD) and
             # (behind guard bands a result is a view, which autograd does not let a ReLU overwrite)
             not (relu.inplace and _guarded()) and
             _unwatched())

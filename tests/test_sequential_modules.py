@@ -1,0 +1,43 @@
+"""What SparseSequential may leave out: a ReLU goes into the convolution's store only where the modules' own calls would
+do the same and nothing else.  (Decisions of the host: no GPU.)"""
+import pytest
+import torch
+
+from mluop_hip import nn as spnn
+
+
+def pair():
+    return spnn.SubMConv3d(16, 16, 3), torch.nn.ReLU()
+
+
+def test_plain_modules():
+    for conv in (spnn.SubMConv3d(16, 16, 3), spnn.SparseConv3d(16, 16, 3), spnn.SparseInverseConv3d(16, 16, 3, "a")):
+        assert spnn._relu_in_store(conv, torch.nn.ReLU())
+
+
+@pytest.mark.parametrize("which", [0, 1])
+def test_a_compiled_module_is_called(which):
+    modules = pair()
+    modules[which].compile(backend="eager")
+    assert not spnn._relu_in_store(*modules)
+
+
+@pytest.mark.parametrize("owner,which", [(spnn.SubMConv3d, 0), (spnn._ConvBase, 0), (torch.nn.ReLU, 1)])
+def test_a_class_with_another_forward_is_called(owner, which, monkeypatch):
+    modules = pair()
+    real = owner.forward
+    monkeypatch.setattr(owner, "forward", lambda self, x: real(self, x))
+    assert not spnn._relu_in_store(*modules)
+    monkeypatch.undo()
+    assert spnn._relu_in_store(*modules)
+
+
+@pytest.mark.parametrize("which", [0, 1])
+def test_a_module_with_a_call_or_forward_of_its_own_is_called(which, monkeypatch):
+    modules = pair()
+    own = type(modules[which])
+    monkeypatch.setattr(own, "__call__", lambda self, x: torch.nn.Module.__call__(self, x), raising=False)
+    assert not spnn._relu_in_store(*modules)
+    monkeypatch.undo()
+    modules[which].forward = lambda x: x
+    assert not spnn._relu_in_store(*modules)
