@@ -317,7 +317,9 @@ class SparseSequential(torch.nn.Sequential):
         cells = x
         for m in self:
             if isinstance(m, SparseSequential):
-                cells = m._plan(cells, built)
+                # (a plan of the network's own is asked for as it is)
+                own = type(m).plan is not _SEQUENTIAL_PLAN or "plan" in m.__dict__
+                cells = m.plan(cells) if own else m._plan(cells, built)
             elif isinstance(m, _ConvBase):
                 if type(m) in (SubMConv3d, SparseConv3d):
                     rb = m._rulebook(cells, wait_counts=False)
@@ -347,6 +349,9 @@ class SparseSequential(torch.nn.Sequential):
             else:
                 x = x.replace_features(m(x.features))
         return x
+
+
+_SEQUENTIAL_PLAN = SparseSequential.plan
 
 
 class Voxelization(torch.nn.Module):

@@ -1,5 +1,6 @@
-"""What SparseSequential may leave out: a ReLU goes into the convolution's store only where the modules' own calls would
-do the same and nothing else.  (Decisions of the host: no GPU.)"""
+"""What SparseSequential may leave out: a ReLU goes into the convolution's store, and a nested network's rulebooks into
+the plan of the outer one, only where the modules' own calls would do the same and nothing else.  (Decisions of
+the host: no GPU.)"""
 import pytest
 import torch
 
@@ -41,3 +42,31 @@ def test_a_module_with_a_call_or_forward_of_its_own_is_called(which, monkeypatch
     monkeypatch.undo()
     modules[which].forward = lambda x: x
     assert not spnn._relu_in_store(*modules)
+
+
+class Cached(spnn.SparseSequential):
+    """A network with a way of its own to come to its rulebooks."""
+
+    def plan(self, x):
+        self.planned = getattr(self, "planned", 0) + 1
+        return x
+
+
+def empty_tensor():
+    return spnn.SparseTensor(torch.zeros(2, 16), torch.zeros(2, 4, dtype=torch.int32), (4, 4, 4), 1)
+
+
+@pytest.mark.parametrize("depth", [1, 2])
+def test_a_nested_networks_own_plan_is_called(depth):
+    inner = Cached(spnn.SubMConv3d(16, 16, 3), torch.nn.ReLU())
+    net = inner
+    for _ in range(depth):
+        net = spnn.SparseSequential(net)
+    net.plan(empty_tensor())
+    assert inner.planned == 1
+
+    plain, seen = spnn.SparseSequential(torch.nn.ReLU()), []
+    plain.plan = lambda x: (seen.append(x), x)[1]
+    outer = spnn.SparseSequential(plain)
+    x = empty_tensor()
+    assert outer.plan(x) is x and seen == [x]
