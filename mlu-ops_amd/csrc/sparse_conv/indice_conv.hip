@@ -688,8 +688,9 @@ __device__ __forceinline__ void storeColumns(typename E::storage *row, int col, 
 //       Lanes past the end of a short block repeat its first entry and
 //       accumulate into a spare row.
 template <typename E, int Q, int C, typename SRC>
-__global__ __launch_bounds__(mfmaThreads(C)) __attribute__((amdgpu_waves_per_eu(mfmaWavesPerSimd((int)sizeof(typename E::storage), Q, C),
-                                   mfmaWavesPerSimd((int)sizeof(typename E::storage), Q, C))))
+__global__ __launch_bounds__(mfmaThreads(C))
+    __attribute__((amdgpu_waves_per_eu(mfmaWavesPerSimd((int)sizeof(typename E::storage), Q, C),
+                                       mfmaWavesPerSimd((int)sizeof(typename E::storage), Q, C))))
 void gatherConvMfma(const typename E::storage *A, ConvRows rows, const typename E::storage *packedW,
                     SRC source, int R, int K, typename E::storage *result) {
   typedef typename E::vec8 vec8;
@@ -1836,7 +1837,8 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
         scanAllPairsForTile<E, NT>(A, conv.q, conv.row_bytes, source, K, r0, r_end, columns, c0, acc, CP);
         for (int i = tid; i < TR * CP; i += NT) {
           const int rr = i / CP, c = i % CP;
-          if (r0 + rr < R && c < columns) E::store(result + (size_t)(r0 + rr) * conv.c + c0 + c, activated(acc[i], conv.relu));
+          if (r0 + rr < R && c < columns)
+            E::store(result + (size_t)(r0 + rr) * conv.c + c0 + c, activated(acc[i], conv.relu));
         }
         __syncthreads();
       }
@@ -3627,8 +3629,8 @@ bool denseShapeOk(const ConvProblem &p, const GatherDims &d) {
 //         strewn        128 rows 22/13/12.8, 24/13/12.3, 27/16/15.9;    2 k 36/32/25.5, 46/36/31.0, 70/63/52.7
 //   3x3x7 in boxes      64 rows 24/17/16.8, 32/21/20.3, 47/34/33.7;     3 k 26/29/20.7, 34/36/22.4, 53/62/37.0
 // Up to 32 offsets gatherConvMfma stays below 4096 rows.  These tiles are ahead there too (3x3x3 in boxes, 64 rows
-// 13/12/11.4, 16/13/13.1, 23/20/19.5; 1 k 14/18/12.8, 19/22/14.4, 27/35/21.5; 3 k 15/18/12.9, 19/21/15.1, 28/35/22.9), by 1 to
-// 6 us of a layer's 50 to 100: a lower line is open, and no measurement speaks for this one.
+// 13/12/11.4, 16/13/13.1, 23/20/19.5; 1 k 14/18/12.8, 19/22/14.4, 27/35/21.5; 3 k 15/18/12.9, 19/21/15.1, 28/35/22.9),
+// by 1 to 6 us of a layer's 50 to 100: a lower line is open, and no measurement speaks for this one.
 constexpr int kTallFewRows = 128 * 256;  // times 64 result columns
 constexpr int kTallFewestRows = 4096;    // with up to kTallFewOffsets offsets
 constexpr int kTallFewOffsets = 32;
@@ -3740,8 +3742,8 @@ void launchDenseInstance(const LaunchCtx &lc, bool wide, const void *A, uint32_t
   constexpr int kElem = (int)sizeof(typename E::storage);
   auto launch = [&](auto wide_tag) {
     constexpr bool WIDE = decltype(wide_tag)::value;
-    gatherConvDense<E, Q, C, SRC, WIDE><<<denseGridX(R, denseTileRows(kElem, Q, C, WIDE)), 64 * densePlan(kElem, Q, C, WIDE).waves,
-                                          0, lc.stream>>>(
+    constexpr int kTileRows = denseTileRows(kElem, Q, C, WIDE), kThreads = 64 * densePlan(kElem, Q, C, WIDE).waves;
+    gatherConvDense<E, Q, C, SRC, WIDE><<<denseGridX(R, kTileRows), kThreads, 0, lc.stream>>>(
         static_cast<const typename E::storage *>(A), a_size, rows, static_cast<const typename E::storage *>(packed),
         source, R, K, static_cast<typename E::storage *>(result));
   };
@@ -3755,8 +3757,8 @@ void launchDenseInstance(const LaunchCtx &lc, bool wide, const void *A, uint32_t
 }
 
 template <typename E, typename SRC>
-void launchDense(const LaunchCtx &lc, int q_padded, bool wide, const void *A, int n_src, const ConvRows &rows, const void *packed,
-                 const SRC &source, int R, int K, void *result) {
+void launchDense(const LaunchCtx &lc, int q_padded, bool wide, const void *A, int n_src, const ConvRows &rows,
+                 const void *packed, const SRC &source, int R, int K, void *result) {
   const uint32_t a_size = (uint32_t)n_src * (uint32_t)rows.row_bytes;
 #define DENSE_INSTANCE(q, c) launchDenseInstance<E, q, c, SRC>(lc, wide, A, a_size, rows, packed, source, R, K, result)
 #define DENSE_BY_C(q)                       \
@@ -3856,7 +3858,8 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     // gather kernel reads them cut by tile, no row map.
     const int tile_cols = dense ? d.c_padded : mfmaTileCols(p, d);
     const int tile_rows = dense ? denseTileRows((int)sizeof(S), d.q_padded, d.c_padded, denseWide(p, d, d.R))
-                                : (tall ? tallRows(tall_q * (int)sizeof(S)) / (half_tiles ? 2 : 1) : mfmaTileRows(tile_cols));
+                          : tall ? tallRows(tall_q * (int)sizeof(S)) / (half_tiles ? 2 : 1)
+                                 : mfmaTileRows(tile_cols);
     int tile_shift = 0;
     while ((1 << tile_shift) < tile_rows) ++tile_shift;
     const int n_tiles = (d.R + tile_rows - 1) / tile_rows;
@@ -3891,9 +3894,11 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     src.sC = sC;
     src.counts = inl;
     if (dense)
-      launchDense<E, SegmentSource>(lc, d.q_padded, denseWide(p, d, d.R), rows_from, d.n_src, rows_of, ws.packed, src, d.R, p.K, result);
+      launchDense<E, SegmentSource>(lc, d.q_padded, denseWide(p, d, d.R), rows_from, d.n_src, rows_of, ws.packed, src,
+                                    d.R, p.K, result);
     else if (tall)
-      launchTall<E, SegmentSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, src, half_tiles, d.R, p.K, result);
+      launchTall<E, SegmentSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, src, half_tiles, d.R, p.K,
+                                   result);
     else if (tile_cols == d.c_padded && useWaveKernel(lc, p.dtype, d.q_padded, d.c_padded))
       launchWave<E>(lc, d.q_padded, rows_from, rows_of, ws.packed, src, d.R, p.K, result);
     else
@@ -3934,7 +3939,8 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
       if (dense) {
         const bool wide = denseWide(p, d, rows);
         n_filled = denseGridX(rows, denseTileRows((int)sizeof(S), d.q_padded, d.c_padded, wide));
-        launchDense<E, MapSource>(lc, d.q_padded, wide, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K, result_rows);
+        launchDense<E, MapSource>(lc, d.q_padded, wide, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K,
+                                  result_rows);
       } else if (tall) {
         n_filled = tallGridX(rows, tallRows(tall_q * (int)sizeof(S)));
         launchTall<E, MapSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, map, false, rows, p.K, result_rows);
@@ -4039,7 +4045,7 @@ bool transposingReads(const LaunchCtx &lc, const ConvProblem &p) {
          !rowsNeedPadding(p.dtype, p.Ci) && !rowsNeedPadding(p.dtype, p.Co);
 }
 
-// Workgroups of the walks (sliceOfWorkgroup), 0: slices.  As many as are resident at a time, so that all
+// Workgroups of the walks (walkOfWorkgroup), 0: slices.  As many as are resident at a time, so that all
 // of them are at about the same rows: 512 at 128 x 128 channels, 768 with 128 on one side, and from 1.5 M
 // pairs on, where a second round no longer shows, 1024.  Fewer pairs leave walks of a few steps.  us with the
 // sums, slices against walks of 512 / 768 / 1024 workgroups, scenes, 3x3x3, fp16:
@@ -4060,8 +4066,8 @@ int filterWalkers(const ConvProblem &p, long long pairs) {
 
 template <typename E, int CI, int CO>
 void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const SliceTable &tab,
-                              const SliceOrder &order, int slice_len, int shares, int total_slices, float *partial, const void *features,
-                              const void *output_grad, void *filters_grad) {
+                              const SliceOrder &order, int slice_len, int shares, int total_slices, float *partial,
+                              const void *features, const void *output_grad, void *filters_grad) {
   typedef typename E::storage S;
   constexpr bool kTransposingShape = sizeof(S) == 2 && CI >= 32 && CO >= 32;
   const bool transposing = kTransposingShape && transposingReads(lc, p);
@@ -4119,15 +4125,21 @@ void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const S
 
 template <typename E, int CI>
 void launchFilterMfmaByCo(const LaunchCtx &lc, const ConvProblem &p, const SliceTable &tab,
-                          const SliceOrder &order, int slice_len, int shares, int total_slices, float *partial, const void *features,
-                          const void *output_grad, void *filters_grad) {
+                          const SliceOrder &order, int slice_len, int shares, int total_slices, float *partial,
+                          const void *features, const void *output_grad, void *filters_grad) {
+#define FILTER_INSTANCE(co)                                                                                        \
+  case co:                                                                                                         \
+    launchFilterMfmaInstance<E, CI, co>(lc, p, tab, order, slice_len, shares, total_slices, partial, features,     \
+                                        output_grad, filters_grad);                                                \
+    break;
   switch (paddedChannels(p.Co)) {
-    case 16: launchFilterMfmaInstance<E, CI, 16>(lc, p, tab, order, slice_len, shares, total_slices, partial, features, output_grad, filters_grad); break;
-    case 32: launchFilterMfmaInstance<E, CI, 32>(lc, p, tab, order, slice_len, shares, total_slices, partial, features, output_grad, filters_grad); break;
-    case 64: launchFilterMfmaInstance<E, CI, 64>(lc, p, tab, order, slice_len, shares, total_slices, partial, features, output_grad, filters_grad); break;
-    case 128: launchFilterMfmaInstance<E, CI, 128>(lc, p, tab, order, slice_len, shares, total_slices, partial, features, output_grad, filters_grad); break;
+    FILTER_INSTANCE(16)
+    FILTER_INSTANCE(32)
+    FILTER_INSTANCE(64)
+    FILTER_INSTANCE(128)
     default: break;
   }
+#undef FILTER_INSTANCE
 }
 
 // Slice length from the real pair count: about kFilterMaxSlices workgroups
@@ -4200,13 +4212,19 @@ void launchFilterMfma(const LaunchCtx &lc, const ConvProblem &p, const FilterGra
             ++next[k];
           }
     }
+#define FILTER_BY_CO(ci)                                                                                           \
+  case ci:                                                                                                         \
+    launchFilterMfmaByCo<E, ci>(lc, p, tab, order, slice_len, shares, entries, ws.partial, features, output_grad,  \
+                                filters_grad);                                                                     \
+    break;
     switch (paddedChannels(p.Ci)) {
-      case 16: launchFilterMfmaByCo<E, 16>(lc, p, tab, order, slice_len, shares, entries, ws.partial, features, output_grad, filters_grad); break;
-      case 32: launchFilterMfmaByCo<E, 32>(lc, p, tab, order, slice_len, shares, entries, ws.partial, features, output_grad, filters_grad); break;
-      case 64: launchFilterMfmaByCo<E, 64>(lc, p, tab, order, slice_len, shares, entries, ws.partial, features, output_grad, filters_grad); break;
-      case 128: launchFilterMfmaByCo<E, 128>(lc, p, tab, order, slice_len, shares, entries, ws.partial, features, output_grad, filters_grad); break;
+      FILTER_BY_CO(16)
+      FILTER_BY_CO(32)
+      FILTER_BY_CO(64)
+      FILTER_BY_CO(128)
       default: break;
     }
+#undef FILTER_BY_CO
   }
 }
 

@@ -325,7 +325,8 @@ hipError_t launchOrderVoxels(const LaunchCtx &lc, const OrderShape &s, const int
   orderPlace<<<groups, kThreads, 0, lc.stream>>>(cells, ws.counts, ws.tiles, ws.slots, ws.keys, ws.ids);
   lc.end();
   lc.begin("orderSortRuns");
-  orderSortRuns<<<(int)((s.voxels + kRun - 1) / kRun), kRunThreads, 0, lc.stream>>>(ws.crowded, s.voxels, ws.keys, ws.ids);
+  const int runs = (int)((s.voxels + kRun - 1) / kRun);
+  orderSortRuns<<<runs, kRunThreads, 0, lc.stream>>>(ws.crowded, s.voxels, ws.keys, ws.ids);
   lc.end();
   const bool aligned = (reinterpret_cast<uintptr_t>(indices) & 15) == 0;
   lc.begin("orderRank");

@@ -505,8 +505,8 @@ hipError_t launchVoxelize(const LaunchCtx &lc, const VoxelizeShape &s, const flo
                      ((reinterpret_cast<uintptr_t>(points) | reinterpret_cast<uintptr_t>(voxels)) & 15) == 0;
   lc.begin("voxAssign");
   voxAssign<<<gridFor((size_t)n), kBlock, 0, lc.stream>>>(
-      points, voxel_size, coors_range, n, s.num_features, w.state, w.first_of, w.firsts, quads, s.max_points, s.max_voxels, voxels, coors, num_points_per_voxel,
-      voxel_num, host_voxel_num, stamp);
+      points, voxel_size, coors_range, n, s.num_features, w.state, w.first_of, w.firsts, quads, s.max_points,
+      s.max_voxels, voxels, coors, num_points_per_voxel, voxel_num, host_voxel_num, stamp);
   lc.end();
   return hipGetLastError();
 }
