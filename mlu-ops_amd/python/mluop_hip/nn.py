@@ -16,7 +16,7 @@ import math
 
 import torch
 
-from . import Handle, _guarded, get_indice_pairs, native, regular_output_space, rulebook_counts
+from . import Handle, _capturing, _guarded, get_indice_pairs, native, regular_output_space, rulebook_counts
 
 _handles = {}
 
@@ -73,10 +73,10 @@ class Rulebook:
     @property
     def pairs(self):
         if not self._tails:
-            num = torch.tensor(self.indice_num, device=self._pairs.device).view(-1, 1, 1)
             with torch.inference_mode(self._pairs.is_inference()):
-                self._pairs.masked_fill_(torch.arange(self._pairs.shape[2], device=num.device) >= num, -1)
-            self._tails = True
+                for of_offset, n in zip(self._pairs, self.indice_num):
+                    of_offset[:, n:].fill_(-1)
+            self._tails = not _capturing()   # (what is captured has not run)
         return self._pairs
 
     @pairs.setter

@@ -107,3 +107,29 @@ def test_the_pairs_of_a_layers_rulebook(gpu_handle, layer, rows, inference):
     assert torch.equal(rb.pairs, want)
     with torch.no_grad():
         assert torch.equal(net(x).features, first)
+
+
+def test_the_pairs_of_a_layers_rulebook_under_capture(gpu_handle):
+    """First asked for while a graph is captured: no copy from the host, and set for eager readers all the same."""
+    import torch
+    from mluop_hip import nn as spnn
+    space, rows = (9, 18, 20), 600
+    idx = torch.from_numpy(random_voxels(np.random.default_rng(8), 1, space, rows, shuffle=True)).cuda()
+    x = spnn.SparseTensor(torch.randn(rows, 16, device="cuda"), idx, space, 1, distinct=True)
+    rulebooks = []
+    for key in "ab":
+        spnn.SubMConv3d(16, 16, 3, indice_key=key).cuda()(x)
+        rulebooks.append(x.rulebooks[key])
+    torch.cuda.synchronize()
+    want = rulebooks[0].pairs.clone()
+    rulebooks[1]._pairs[:, :, -1] = torch.where(want[:, :, -1] == -1, 7, want[:, :, -1])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        seen = rulebooks[1].pairs + 1
+    assert torch.equal(rulebooks[1].pairs, want)
+    for _ in range(3):
+        seen.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(seen - 1, want)
