@@ -1683,135 +1683,238 @@ __global__ __launch_bounds__(64) void gatherConvWave(
 // When most rows of a tile have a partner at most offsets, compacting pairs buys
 // little and the fp32 accumulate in LDS (a 16-byte read-modify-write per lane and
 // 16 result columns, on arbitrary rows: bank conflicts) is what the kernels above
-// spend their time on.  Here a wave owns two groups of 16 result rows and all result
-// columns, and accumulates them in registers over all offsets: no accumulator traffic
-// at all.
+// spend their time on.  Here a wave owns groups of 16 result rows and accumulates them
+// in registers over all offsets: no accumulator traffic at all.  Two kernels, by the length of a
+// gathered row: gatherConvDense up to 64 bytes, gatherConvDenseStaged above.
 //
 // Rows are buffer loads: the row map holds byte offsets, a lane without a partner holds one
-// behind the tensor's end, and the hardware answers it with zeros without going to memory.  The
-// rows of the wave's next offsets travel while the current one is multiplied.
+// behind the tensor's end, and the hardware answers it with zeros without going to memory.
+// Both kernels multiply rows of zeros for the partners that are not there, which is nothing as long
+// as the filter is finite.  An offset whose filter is not (packFilter says so) is taken out of the
+// walk and multiplied by itself, its products added to the rows that have a partner there only.
+constexpr int kDenseChunk = 27;      // offsets whose row-map slice is resident in LDS at once
+constexpr int kDenseMapBatch = 14;   // loads in flight per thread while a tile's row map is read
+constexpr int kDenseRows = 128;      // of a tile
+constexpr int kDenseThreads = 256;
+constexpr int kDenseGroups = kDenseRows / 16;
+static_assert(kDenseChunk <= 32, "a chunk's offsets in one mask");
+
+// A tile's slice of the row map for a chunk of offsets.
+struct DenseMap {
+  uint32_t at[kDenseChunk][kDenseRows];  // where the partner row of (offset in chunk, tile row) begins, or kNoRow
+  int first[kDenseChunk], count[kDenseChunk];
+  int finite[kDenseChunk];       // the offset's filter holds no infinity and no NaN
+  uint32_t groups[kDenseChunk];  // the row groups that have a partner at the offset
+};
+
+// Fills the map for the offsets [kc, kc + kn), by the whole workgroup; ends in a barrier.  Returns the filled slots of
+// a MapSource that this thread has seen.
+template <typename SRC>
+__device__ __forceinline__ int fillDenseMap(DenseMap &map, const SRC &source, const unsigned long long *nonfinite,
+                                            int row_bytes, int tile, int r0, int R, int kc, int kn, int K) {
+  constexpr int TR = kDenseRows, NT = kDenseThreads;
+  const int tid = threadIdx.x, lane = tid & 63;
+  int slots = 0;
+  if (tid < kn) map.finite[tid] = nonfinite[kc + tid] != nonfinite[K];
+  if constexpr (SRC::kSegments) {
+    // The pairs of an offset that fall into this tile are one piece of its list, between
+    // two neighbouring entries of the cut table.
+    if (tid < kn) {
+      const int32_t *cut = source.cuts + (size_t)(kc + tid) * source.cut_stride + tile;
+      const int first = cut[0];
+      const int count = cut[1] - first;
+      map.first[tid] = first;
+      map.count[tid] = count < 0 ? 0 : (count > TR ? TR : count);
+    }
+    for (int i = tid; i < kn * TR; i += NT) (&map.at[0][0])[i] = kNoRow;
+    __syncthreads();
+    // a thread per (offset, pair of the piece): the partner goes to the result row's
+    // position.  A thread's loads of one batch are all requested before the first is
+    // used (a slot without a pair reads pair 0 of its offset and drops it).
+    if (source.L > 0) {
+      for (int base = tid; base < kn * TR; base += NT * kDenseMapBatch) {
+        int own[kDenseMapBatch], partner[kDenseMapBatch], at[kDenseMapBatch];
+#pragma unroll
+        for (int u = 0; u < kDenseMapBatch; ++u) {
+          const int slot = base + u * NT;
+          int kk = slot / TR;
+          const int q = slot % TR;
+          kk = kk < kn ? kk : kn - 1;
+          const bool live = slot < kn * TR && q < map.count[kk];
+          int p = live ? map.first[kk] + q : 0;
+          p = p < 0 ? 0 : (p < source.L ? p : source.L - 1);
+          const int32_t *list = source.pairs + (size_t)(kc + kk) * 2 * source.L;
+          own[u] = list[(size_t)source.row_col * source.L + p];
+          partner[u] = list[(size_t)source.src_col * source.L + p];
+          at[u] = live ? kk : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < kDenseMapBatch; ++u)
+          if (at[u] >= 0) map.at[at[u]][(own[u] - r0) & (TR - 1)] = (uint32_t)partner[u] * (uint32_t)row_bytes;
+      }
+    }
+  } else {
+    for (int base = tid; base < kn * TR; base += NT * kDenseMapBatch) {
+      int v[kDenseMapBatch];
+#pragma unroll
+      for (int u = 0; u < kDenseMapBatch; ++u) {
+        const int slot = base + u * NT;
+        int kk = slot / TR;
+        kk = kk < kn ? kk : kn - 1;
+        const int r = r0 + slot % TR;
+        v[u] = source.map[(size_t)(kc + kk) * R + (r < R ? r : R - 1)];
+        if (slot >= kn * TR || r >= R) v[u] = -1;
+      }
+#pragma unroll
+      for (int u = 0; u < kDenseMapBatch; ++u) {
+        const int slot = base + u * NT;
+        if (slot < kn * TR) map.at[slot / TR][slot % TR] = v[u] >= 0 ? (uint32_t)v[u] * (uint32_t)row_bytes : kNoRow;
+        slots += v[u] >= 0;
+      }
+    }
+  }
+  __syncthreads();
+  // which row groups have a partner at which offsets: a thread an (offset, group)
+  for (int base = 0; base < kn * kDenseGroups; base += NT) {
+    const int kk = (base + tid) / kDenseGroups, group = tid % kDenseGroups;
+    bool any = false;
+    if (kk < kn) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const u32x4 at = *reinterpret_cast<const u32x4 *>(&map.at[kk][group * 16 + q * 4]);
+        any = any | (at[0] != kNoRow) | (at[1] != kNoRow) | (at[2] != kNoRow) | (at[3] != kNoRow);
+      }
+    }
+    const unsigned long long m = __ballot(any);
+    if (kk < kn && group == 0) map.groups[kk] = (uint32_t)(m >> (lane & ~(kDenseGroups - 1))) & ((1u << kDenseGroups) - 1u);
+  }
+  __syncthreads();
+  return slots;
+}
+
+// A tile whose pair lists turned out to be out of order: fp32 rows where the row map would be, 16 columns at a time,
+// every pair looked at by every workgroup.
+template <typename E>
+__device__ __forceinline__ void denseTileOutOfOrder(DenseMap &map, const typename E::storage *A, const ConvRows &conv,
+                                                    const SegmentSource &source, int r0, int R, int K,
+                                                    typename E::storage *result) {
+  constexpr int TR = kDenseRows, NT = kDenseThreads, CP = 16;  // columns per pass
+  static_assert(CP <= kDenseChunk, "a pass of columns fits the row map");
+  float *acc = reinterpret_cast<float *>(&map.at[0][0]);
+  const int r_end = r0 + TR < R ? r0 + TR : R;
+  for (int c0 = 0; c0 < conv.c; c0 += CP) {
+    for (int i = threadIdx.x; i < TR * CP; i += NT) acc[i] = 0.f;
+    __syncthreads();
+    const int columns = conv.c - c0 < CP ? conv.c - c0 : CP;
+    scanAllPairsForTile<E, NT>(A, conv.q, conv.row_bytes, source, K, r0, r_end, columns, c0, acc, CP);
+    for (int i = threadIdx.x; i < TR * CP; i += NT) {
+      const int rr = i / CP, c = i % CP;
+      if (r0 + rr < R && c < columns)
+        E::store(result + (size_t)(r0 + rr) * conv.c + c0 + c, activated(acc[i], conv.relu));
+    }
+    __syncthreads();
+  }
+}
+
+// An offset whose filter is not finite: its products, added to the rows that have a partner there only.  `at`: the
+// map's entries of the wave's rows, `filter`: its first column block's fragments for lane 0.
+template <typename E, int G, int NB, int KB>
+__device__ __forceinline__ void addOffsetApart(float4v (&acc)[G][NB], __amdgpu_buffer_rsrc_t a_rows, const uint32_t *at_rows,
+                                               const char *filter, int row_bytes) {
+  typedef typename E::vec8 vec8;
+  int own = threadIdx.x & 63;  // (nothing of this rare loop is worked out ahead of it and held in registers)
+  asm volatile("" : "+v"(own));
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const uint32_t at = at_rows[g * 16 + (own & 15)];
+    vec8 row[KB];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const uint32_t piece = (uint32_t)(kb * 64 + (own >> 4) * 16);
+      row[kb] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(
+                                             a_rows, piece < (uint32_t)row_bytes ? at + piece : kNoRow, 0, 0));
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      float4v product = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        product = E::mfma(*reinterpret_cast<const vec8 *>(filter + (nb * KB + kb) * 1024 + own * 16), row[kb], product);
+      if (at != kNoRow) acc[g][nb] += product;  // (a lane's results are of its own row)
+      asm volatile("" ::: "memory");            // one block's fragments in registers at a time
+    }
+  }
+}
+
+// The filled slots of all threads, for the collision check; by the whole workgroup, behind its last use of the map.
+__device__ __forceinline__ void storeDenseSlots(DenseMap &map, int slots, int32_t *filled) {
+  __syncthreads();
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) slots += __shfl_xor(slots, d, kWave);
+  if ((threadIdx.x & 63) == 0) map.count[threadIdx.x >> 6] = slots;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int all = 0;
+    for (int w = 0; w < kDenseThreads / 64; ++w) all += map.count[w];
+    filled[blockIdx.x] = all;
+  }
+}
+
+// ---- rows of up to 64 bytes
+//
+// Operand-order loads take each such row whole, so rows come straight into the operand registers (lane (row,
+// quarter) loads 16 bytes) and whole phases of two offsets are in flight; nothing is skipped: a group
+// without rows multiplies zeros.  A wave owns two row groups and ALL result columns.
 // Filter.  The waves share an offset's filter: its fragments travel from global memory into a
 // ring of two LDS buffers, a phase of one or two offsets at a time, and every wave reads all of
 // them from there, once per offset for both its row groups.  One barrier per phase hands a
 // buffer over; it waits for LDS traffic only, and each wave waits for its own requests itself
 // (__syncthreads() would make every wave wait for all loads in flight).
-//
-// What bounds it differs with the row length, and so does the way of the rows (us for forward
-// at 80 k rows, 27 offsets, half the slots filled; in brackets one path for all lengths: 4 row
-// groups' filters read from LDS per offset by 4 waves, rows by plain loads):
-//   up to 64 bytes (16 channels: 37 us [42]): the loop itself.  Rows come straight into the
-//     operand registers (lane (row, quarter) loads 16 bytes), whole phases of two offsets are in
-//     flight, and nothing is skipped: a group without rows multiplies zeros.
-//   up to 128 bytes (64 channels: 88 us [101]): operand-order loads touch 16 rows of 64 bytes
-//     each, which the CU's address unit takes at a third of the rate of whole rows.  So rows come
-//     row by row into registers, go through LDS (pieces permuted so that operand reads meet no
-//     bank twice), and every request is spread between the multiplies.
-//   above (128 channels: 199 us [230]): the multiplies (130 us at the matrix cores' rate if
-//     nothing were skipped), and LDS, which carries the filter; rows through LDS as well measure
-//     217 us.  So rows go in operand order again, a chunk requested right behind its last use,
-//     and a wave multiplies only the groups that have a row
-//     at the offset.
-// All of them multiply rows of zeros for the partners that are not there, which is nothing as long
-// as the filter is finite.  An offset whose filter is not (packFilter says so) is taken out of the
-// walk and multiplied by itself, its products added to the rows that have a partner there only.
-constexpr int kDenseChunk = 27;      // offsets whose row-map slice is resident in LDS at once
-constexpr int kDenseMapBatch = 14;   // loads in flight per thread while a tile's row map is read
-
-// How an instance splits its work, from what a CU has: 160 KiB of LDS and 512 registers a lane
-// and SIMD.  Short rows: as many workgroups as registers and LDS allow.  Rows above 128 bytes: two
-// workgroups of four waves, of which one multiplies while the other builds its row map and waits for its
-// first rows (8.7 of a tile's 42 us at 128 -> 128 channels, with one workgroup of eight waves a CU); the ring
-// then holds one offset a phase at 128 columns instead of two, and every 128 rows load the filters again.
-// At 128 columns eight waves stay for some row counts (`wide`, denseWide).  us, eight waves against twice four:
-//   fp16 128 -> 64    8 k 32/27, 80 k 70/71, 150 k 135/114, 250 k 171/161;  128 -> 32  30 k 42/28, 250 k 158/147
-//   fp32  64 -> 64    8 k 105/68, 30 k 114/70, 80 k 182/162, 150 k 280/271
-enum class DenseRows { kByPhase, kStaged, kInPlace };  // how rows reach the operand registers
+// What bounds it is the loop itself (16 channels, 80 k rows, 27 offsets, half the slots filled: 37 us).  Rows through
+// LDS as below are no faster here (248 636 rows of a scene, with the filter's packing: 16 -> 16 38 us against 46,
+// 32 -> 32 47 against 47).
 struct DensePlan {
-  int waves;        // per workgroup
-  int groups;       // row groups (of 16) per wave
   int per_cu;       // workgroups a CU
   int offsets;      // offsets per phase
-  DenseRows rows;
 };
-constexpr DensePlan densePlan(int elem_bytes, int Q, int C, bool wide) {
-  const int nb = C / 16, kb = (Q * elem_bytes + 63) / 64;
-  const int row_bytes = Q * elem_bytes;
-  if (row_bytes <= 64) {
-    DensePlan p = {4, 2, 4, 2, DenseRows::kByPhase};
-    const int room = 160 * 1024 / 4 - kDenseChunk * 4 * p.groups * 16 * 4 - 1024;
-    if (p.groups * 4 * (nb + 2 * 2) + 4 * nb + 40 > 128) p.per_cu = 2;
-    if (p.per_cu == 4 && room < 4 * nb * kb * 1024) p.per_cu = 2;
-    return p;
-  }
-  if (row_bytes <= 128) {
-    DensePlan p = {4, 2, 2, 2, DenseRows::kStaged};
-    const int rows = p.waves * p.groups * 16;
-    const int room = 160 * 1024 / p.per_cu - kDenseChunk * rows * 4 - rows * row_bytes - 1024;
-    if (room < 4 * nb * kb * 1024) p.offsets = 1;
-    return p;
-  }
-  DensePlan p = wide ? DensePlan{8, 2, 1, 2, DenseRows::kInPlace} : DensePlan{4, 2, 2, 2, DenseRows::kInPlace};
-  const int room = 160 * 1024 / p.per_cu - kDenseChunk * p.waves * p.groups * 16 * 4 - 1024;
-  if (room < 4 * nb * kb * 1024) p.offsets = 1;
+constexpr DensePlan densePlan(int C) {
+  const int nb = C / 16, groups = 2;
+  DensePlan p = {4, 2};
+  const int room = 160 * 1024 / 4 - kDenseChunk * kDenseRows * 4 - 1024;
+  if (groups * 4 * (nb + 2 * 2) + 4 * nb + 40 > 128) p.per_cu = 2;
+  if (p.per_cu == 4 && room < 4 * nb * 1024) p.per_cu = 2;
   return p;
 }
-constexpr int denseWavesPerSimd(int elem_bytes, int Q, int C, bool wide) {
-  const DensePlan p = densePlan(elem_bytes, Q, C, wide);
-  return p.waves * p.per_cu / 4;
-}
-constexpr int denseTileRows(int elem_bytes, int Q, int C, bool wide) {
-  return densePlan(elem_bytes, Q, C, wide).waves * densePlan(elem_bytes, Q, C, wide).groups * 16;
-}
-// Where piece `piece` of a staged row lies in its row's bytes: rows lie a multiple of the bank
-// width apart, and the 16 rows whose same piece is read at once have to meet all banks.
-constexpr int denseRowSwizzle(int row_bytes, int row) {
-  return row_bytes >= 256 ? (row & 15) : ((row >> 1) & 7);
-}
 
-template <typename E, int Q, int C, typename SRC, bool WIDE>
-__global__ __launch_bounds__(64 * densePlan((int)sizeof(typename E::storage), Q, C, WIDE).waves)
-    __attribute__((amdgpu_waves_per_eu(denseWavesPerSimd((int)sizeof(typename E::storage), Q, C, WIDE),
-                                       denseWavesPerSimd((int)sizeof(typename E::storage), Q, C, WIDE))))
+template <typename E, int Q, int C, typename SRC>
+__global__ __launch_bounds__(kDenseThreads)
+    __attribute__((amdgpu_waves_per_eu(densePlan(C).per_cu, densePlan(C).per_cu)))
 void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows conv,
                      const typename E::storage *packedW, SRC source, int R, int K,
                      typename E::storage *result) {
   typedef typename E::vec8 vec8;
   typedef typename E::storage S;
-  constexpr DensePlan PLAN = densePlan((int)sizeof(S), Q, C, WIDE);
-  constexpr int WAVES = PLAN.waves;
-  constexpr bool kStaged = PLAN.rows == DenseRows::kStaged;
-  constexpr int G = PLAN.groups;
-  constexpr int TR = WAVES * G * 16;
-  constexpr int NT = WAVES * 64;
+  constexpr DensePlan PLAN = densePlan(C);
+  constexpr int WAVES = kDenseThreads / 64;
+  constexpr int G = kDenseGroups / WAVES;
   constexpr int NB = C / 16;                 // 16-column blocks, all of them in every wave
   constexpr int KC = kDenseChunk;
-  constexpr int KB = (Q + E::kChunk - 1) / E::kChunk;
-  constexpr int ROW_BYTES = Q * (int)sizeof(S);
-  constexpr int FRAGS = NB * KB;             // 1 KiB filter fragments per offset
+  constexpr int FRAGS = NB;                  // 1 KiB filter fragments per offset
   constexpr int W_BYTES = FRAGS * 1024;
   constexpr int OPP = PLAN.offsets;          // offsets per phase
   constexpr int BUF_FRAGS = OPP * FRAGS;
   constexpr int FPW = (BUF_FRAGS + WAVES - 1) / WAVES;
-  // kStaged: loads of 1 KiB per row group, and rows per load
-  constexpr int LPG = kStaged ? 16 * ROW_BYTES / 1024 : 1;
-  constexpr int RPL = kStaged ? 1024 / ROW_BYTES : 1;
-  static_assert(KC <= 32, "a chunk's offsets in one mask");
+  static_assert(Q <= E::kChunk, "one fragment a row");
 
   __shared__ __attribute__((aligned(1024))) char s_w[2 * BUF_FRAGS * 1024];
-  __shared__ __attribute__((aligned(1024))) char s_rows[kStaged ? TR * ROW_BYTES : 16];
-  __shared__ uint32_t s_map[KC][TR];  // where the partner row of (offset in chunk, tile row) begins, or kNoRow
-  __shared__ int s_has[KC];
-  __shared__ int s_first[KC];
-  __shared__ int s_finite[KC];        // the offset's filter holds no infinity and no NaN
-  __shared__ uint32_t s_offsets;      // offsets of the chunk that have a pair in this tile
-  __shared__ uint32_t s_apart;        // those of them whose filter is not finite (not among s_offsets)
+  __shared__ __attribute__((aligned(16))) DenseMap s_map;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tiles_per_xcd = gridDim.x >> 3;  // neighbouring tiles on one XCD, as above
   const int tile = (blockIdx.x & 7) * tiles_per_xcd + (blockIdx.x >> 3);
-  const int r0 = tile * TR;
+  const int r0 = tile * kDenseRows;
   if constexpr (!SRC::kSegments) {
     if (notWanted(source.run_if)) return;
   }
@@ -1822,26 +1925,8 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
     return;
   }
   if constexpr (SRC::kSegments) {
-    if (*source.verdict == source.ticket && source.leave_if_unordered) return;
     if (*source.verdict == source.ticket) {
-      // pair lists out of order: fp32 rows where the row map would be, 16 columns at a
-      // time, every pair looked at by every workgroup
-      float *acc = reinterpret_cast<float *>(&s_map[0][0]);
-      constexpr int CP = 16;  // columns per pass
-      static_assert(CP <= KC, "a pass of columns fits the row map");
-      const int r_end = r0 + TR < R ? r0 + TR : R;
-      for (int c0 = 0; c0 < conv.c; c0 += CP) {
-        for (int i = tid; i < TR * CP; i += NT) acc[i] = 0.f;
-        __syncthreads();
-        const int columns = conv.c - c0 < CP ? conv.c - c0 : CP;
-        scanAllPairsForTile<E, NT>(A, conv.q, conv.row_bytes, source, K, r0, r_end, columns, c0, acc, CP);
-        for (int i = tid; i < TR * CP; i += NT) {
-          const int rr = i / CP, c = i % CP;
-          if (r0 + rr < R && c < columns)
-            E::store(result + (size_t)(r0 + rr) * conv.c + c0 + c, activated(acc[i], conv.relu));
-        }
-        __syncthreads();
-      }
+      if (!source.leave_if_unordered) denseTileOutOfOrder<E>(s_map, A, conv, source, r0, R, K, result);
       return;
     }
   }
@@ -1853,16 +1938,8 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
       reinterpret_cast<const unsigned long long *>(reinterpret_cast<const char *>(packedW) + (size_t)K * W_BYTES);
   const uint32_t w_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)s_w;
   const int row_first = wave * (G * 16) + pair;  // this lane's row in its wave's first group
-  // Which 16 bytes of a row a lane asks for: its quarter, or in staged loads the piece that
-  // belongs where the lane writes.  Behind the row's own bytes: nowhere (zeros).
-  uint32_t piece_at[LPG];
-#pragma unroll
-  for (int j = 0; j < LPG; ++j) {
-    const int row = j * RPL + lane / (64 / RPL);
-    const int piece = kStaged ? (lane % (64 / RPL)) ^ denseRowSwizzle(ROW_BYTES, row) : quad;
-    piece_at[j] = piece * 16 < conv.row_bytes ? (uint32_t)piece * 16u : kNoRow;
-  }
-  char *const rows_lds = s_rows + wave * (G * 16) * (kStaged ? ROW_BYTES : 0);
+  // a lane's quarter of a row; behind the row's own bytes: nowhere (zeros)
+  const uint32_t piece_at = quad * 16 < conv.row_bytes ? (uint32_t)quad * 16u : kNoRow;
 
   float4v acc[G][NB];
 #pragma unroll
@@ -1874,109 +1951,15 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
   for (int kc = 0; kc < K; kc += KC) {
     const int kn = (K - kc) < KC ? (K - kc) : KC;
     __syncthreads();  // the chunk before is finished with s_map and the filter buffers
-    if constexpr (SRC::kSegments) {
-      // The pairs of an offset that fall into this tile are one piece of its list, between
-      // two neighbouring entries of the cut table.
-      if (tid < kn) {
-        const int32_t *cut = source.cuts + (size_t)(kc + tid) * source.cut_stride + tile;
-        const int first = cut[0];
-        int count = cut[1] - first;
-        count = count < 0 ? 0 : (count > TR ? TR : count);
-        s_first[tid] = first;
-        s_has[tid] = count;
-        s_finite[tid] = nonfinite[kc + tid] != nonfinite[K];
-      }
-      for (int i = tid; i < kn * TR; i += NT) (&s_map[0][0])[i] = kNoRow;
-      __syncthreads();
-      // a thread per (offset, pair of the piece): the partner goes to the result row's
-      // position.  A thread's loads of one batch are all requested before the first is
-      // used (a slot without a pair reads pair 0 of its offset and drops it).
-      if (source.L > 0) {
-        for (int base = tid; base < kn * TR; base += NT * kDenseMapBatch) {
-          int own[kDenseMapBatch], partner[kDenseMapBatch], at[kDenseMapBatch];
-#pragma unroll
-          for (int u = 0; u < kDenseMapBatch; ++u) {
-            const int slot = base + u * NT;
-            int kk = slot / TR;
-            const int q = slot % TR;
-            kk = kk < kn ? kk : kn - 1;
-            const bool live = slot < kn * TR && q < s_has[kk];
-            int p = live ? s_first[kk] + q : 0;
-            p = p < 0 ? 0 : (p < source.L ? p : source.L - 1);
-            const int32_t *list = source.pairs + (size_t)(kc + kk) * 2 * source.L;
-            own[u] = list[(size_t)source.row_col * source.L + p];
-            partner[u] = list[(size_t)source.src_col * source.L + p];
-            at[u] = live ? kk : -1;
-          }
-#pragma unroll
-          for (int u = 0; u < kDenseMapBatch; ++u)
-            if (at[u] >= 0) s_map[at[u]][(own[u] - r0) & (TR - 1)] = (uint32_t)partner[u] * (uint32_t)conv.row_bytes;
-        }
-      }
-    } else {
-      if (tid < kn) {
-        s_has[tid] = 0;
-        s_finite[tid] = nonfinite[kc + tid] != nonfinite[K];
-      }
-      __syncthreads();
-      for (int base = tid; base < kn * TR; base += NT * kDenseMapBatch) {
-        int v[kDenseMapBatch];
-#pragma unroll
-        for (int u = 0; u < kDenseMapBatch; ++u) {
-          const int slot = base + u * NT;
-          int kk = slot / TR;
-          kk = kk < kn ? kk : kn - 1;
-          const int r = r0 + slot % TR;
-          v[u] = source.map[(size_t)(kc + kk) * R + (r < R ? r : R - 1)];
-          if (slot >= kn * TR || r >= R) v[u] = -1;
-        }
-#pragma unroll
-        for (int u = 0; u < kDenseMapBatch; ++u) {
-          const int slot = base + u * NT;  // (a wave stays inside one offset)
-          if (slot < kn * TR) s_map[slot / TR][slot % TR] = v[u] >= 0 ? (uint32_t)v[u] * (uint32_t)conv.row_bytes : kNoRow;
-          const unsigned long long m = __ballot(v[u] >= 0);
-          if (m != 0ull && lane == 0) s_has[slot / TR] = 1;
-          slots += v[u] >= 0;
-        }
-      }
-    }
-    __syncthreads();
-    if (wave == 0) {
-      const bool has = lane < kn && s_has[lane < kn ? lane : 0] != 0;
-      const bool finite = s_finite[lane < kn ? lane : 0] != 0;
-      const unsigned long long m = __ballot(has && finite), apart = __ballot(has && !finite);
-      if (lane == 0) {
-        s_offsets = (uint32_t)m;
-        s_apart = (uint32_t)apart;
-      }
-    }
-    __syncthreads();
-    const uint32_t offsets = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_offsets);
-    for (uint32_t left = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_apart); left != 0; left &= left - 1) {
+    slots += fillDenseMap(s_map, source, nonfinite, conv.row_bytes, tile, r0, R, kc, kn, K);
+    const bool has = lane < kn && s_map.groups[lane < kn ? lane : 0] != 0;
+    const bool finite = s_map.finite[lane < kn ? lane : 0] != 0;
+    // offsets of the chunk that have a pair in this tile; those of them whose filter is not finite go by themselves
+    const uint32_t offsets = (uint32_t)__ballot(has && finite);
+    for (uint32_t left = (uint32_t)__ballot(has && !finite); left != 0; left &= left - 1) {
       const int kk = __builtin_ctz(left);
-      int own = lane;  // (nothing of this rare loop is worked out ahead of it and held in registers)
-      asm volatile("" : "+v"(own));
-      const char *const filter = reinterpret_cast<const char *>(packedW) + own * 16 + (size_t)(kc + kk) * W_BYTES;
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const uint32_t at = s_map[kk][wave * (G * 16) + g * 16 + (own & 15)];
-        vec8 row[KB];
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-          const uint32_t piece = (uint32_t)(kb * 64 + (own >> 4) * 16);
-          row[kb] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(
-                                                 a_rows, piece < (uint32_t)conv.row_bytes ? at + piece : kNoRow, 0, 0));
-        }
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          float4v product = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int kb = 0; kb < KB; ++kb)
-            product = E::mfma(*reinterpret_cast<const vec8 *>(filter + (nb * KB + kb) * 1024), row[kb], product);
-          if (at != kNoRow) acc[g][nb] += product;  // (a lane's results are of its own row)
-          asm volatile("" ::: "memory");            // one block's fragments in registers at a time
-        }
-      }
+      addOffsetApart<E, G, NB, 1>(acc, a_rows, &s_map.at[kk][wave * (G * 16)],
+                                  reinterpret_cast<const char *>(packedW) + (size_t)(kc + kk) * W_BYTES, conv.row_bytes);
     }
     if (offsets == 0) continue;
     // A phase: the OPP lowest offsets of `left` (fewer at the end), which are taken out of it.
@@ -2008,308 +1991,64 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
           requestToLds(fragment_of(phase, f), w_lds + (half * BUF_FRAGS + f) * 1024);
       }
     };
-    if constexpr (PLAN.rows == DenseRows::kByPhase) {
-      // Rows in one of two sets of registers, filters in one of two ring buffers.
-      vec8 rows_a[OPP][G], rows_b[OPP][G];
-      auto request_phase = [&](uint32_t phase, int half, vec8 (&rows)[OPP][G]) {
-        filters_to_lds(phase, half);
-        uint32_t left = phase;
-#pragma unroll
-        for (int o = 0; o < OPP; ++o) {
-          const bool there = left != 0;
-          const int kk = there ? __builtin_ctz(left) : 0;
-          left &= left - 1;
-#pragma unroll
-          for (int g = 0; g < G; ++g) {
-            const uint32_t at = there ? s_map[kk][row_first + g * 16] : kNoRow;
-            rows[o][g] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(
-                                                      a_rows, __builtin_elementwise_add_sat(at, piece_at[0]), 0, 0));
-          }
-        }
-      };
-      // Everything this wave has requested is there.  The rows pass through an empty statement
-      // that the compiler must take for their last writer: it then places its own wait for their
-      // loads here, and not in front of their first use, behind the next phase's requests, which
-      // it would wait for as well.
-      auto landed = [&](vec8 (&rows)[OPP][G]) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-        for (int o = 0; o < OPP; ++o)
-#pragma unroll
-          for (int g = 0; g < G; ++g) asm volatile("" : "+v"(rows[o][g]));
-      };
-      auto multiply_phase = [&](int half, const vec8 (&rows)[OPP][G]) {
-        const char *filters = s_w + half * BUF_FRAGS * 1024 + lane * 16;
-#pragma unroll
-        for (int o = 0; o < OPP; ++o)
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb) {
-            const vec8 w = *reinterpret_cast<const vec8 *>(filters + o * W_BYTES + nb * 1024);
-#pragma unroll
-            for (int g = 0; g < G; ++g) acc[g][nb] = E::mfma(w, rows[o][g], acc[g][nb]);
-          }
-      };
-      uint32_t left = offsets;
-      uint32_t phase = next_phase(left);
-      request_phase(phase, 0, rows_a);
-      landed(rows_a);
-      ldsBarrier();
-      while (true) {
-        phase = next_phase(left);
-        if (phase != 0) request_phase(phase, 1, rows_b);
-        multiply_phase(0, rows_a);
-        if (phase == 0) break;
-        landed(rows_b);
-        ldsBarrier();
-        phase = next_phase(left);
-        if (phase != 0) request_phase(phase, 0, rows_a);
-        multiply_phase(1, rows_b);
-        if (phase == 0) break;
-        landed(rows_a);
-        ldsBarrier();
-      }
-    } else if constexpr (PLAN.rows == DenseRows::kInPlace) {
-    // offsets at which the wave's first / second row group has a partner
-    uint32_t has_first = 0, has_second = 0;
-#pragma unroll 9
-    for (int kk = 0; kk < kn; ++kk) {
-      if (__ballot(s_map[kk][row_first] != kNoRow) != 0ull) has_first |= 1u << kk;
-      if (__ballot(s_map[kk][row_first + 16] != kNoRow) != 0ull) has_second |= 1u << kk;
-    }
-    has_first = (uint32_t)__builtin_amdgcn_readfirstlane((int)has_first);
-    has_second = (uint32_t)__builtin_amdgcn_readfirstlane((int)has_second);
-
-    // The wave's way through a phase: first the offsets at which both its groups have rows, then
-    // those of the first group alone, then the second's; each in ascending order.
-    struct Way {
-      uint32_t both, first, second;
-    };
-    auto way_through = [&](uint32_t phase) -> Way {
-      return Way{phase & has_first & has_second, phase & has_first & ~has_second, phase & has_second & ~has_first};
-    };
-    // The offset whose rows are requested next: one in front of the one that is multiplied.
-    uint32_t ahead_left = offsets;
-    Way ahead = {0, 0, 0};
-    auto next_ahead = [&]() -> int {
-      while ((ahead.both | ahead.first | ahead.second) == 0) {
-        if (ahead_left == 0) return -1;
-        ahead = way_through(next_phase(ahead_left));
-      }
-      const uint32_t from = ahead.both != 0 ? ahead.both : (ahead.first != 0 ? ahead.first : ahead.second);
-      const uint32_t taken = from & (0u - from);
-      ahead.both &= ~taken;  // (an offset is in one of the three masks)
-      ahead.first &= ~taken;
-      ahead.second &= ~taken;
-      return __builtin_ctz(taken);
-    };
-    // where this lane's rows of offset kk (none: -1) begin
-    auto locate_rows = [&](int kk, uint32_t (&at)[G]) {
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        at[g] = s_map[kk < 0 ? 0 : kk][row_first + g * 16];
-        at[g] = kk < 0 ? kNoRow : at[g];
-      }
-    };
-    // 16 bytes of a row: reduction chunk kb, this lane's quarter; zeros where the row ends before.
-    // (The chunk is part of the lane's own offset, not of the scalar one: the hardware compares the
-    // lane's offset with the tensor's length less the scalar offset, and a tensor of one short row
-    // is shorter than the last chunk's place in it.)
-    auto load_chunk = [&](uint32_t at, int kb) -> vec8 {
-      const uint32_t piece = (uint32_t)(kb * 64 + quad * 16);
-      const uint32_t from = piece < (uint32_t)conv.row_bytes ? at + piece : kNoRow;
-      return __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(a_rows, from, 0, 0));
-    };
-
-    vec8 rows[G][KB];
-    // one offset: the fragments at `wbuf` times the rows of the groups in MASK, while the rows of
-    // the wave's next offset are requested chunk by chunk behind their last use
-    auto multiply = [&](auto mask_tag, const char *wbuf) {
-      constexpr int MASK = decltype(mask_tag)::value;
-      uint32_t at[G];
-      locate_rows(next_ahead(), at);
-      vec8 w[2][NB];
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) w[0][nb] = *reinterpret_cast<const vec8 *>(wbuf + nb * KB * 1024);
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        if (kb + 1 < KB) {
-#pragma unroll
-          for (int nb = 0; nb < NB; ++nb)
-            w[(kb + 1) & 1][nb] = *reinterpret_cast<const vec8 *>(wbuf + (nb * KB + kb + 1) * 1024);
-        }
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          if ((MASK >> g) & 1) {
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) acc[g][nb] = E::mfma(w[kb & 1][nb], rows[g][kb], acc[g][nb]);
-          }
-        }
-#pragma unroll
-        for (int g = 0; g < G; ++g) rows[g][kb] = load_chunk(at[g], kb);
-        asm volatile("" ::: "memory");  // the requests stay here, an offset ahead of their use
-      }
-    };
-
-    uint32_t phases_left = offsets;
-    uint32_t phase = next_phase(phases_left);
-    filters_to_lds(phase, 0);
-    {
-      uint32_t at[G];
-      locate_rows(next_ahead(), at);
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-        for (int g = 0; g < G; ++g) rows[g][kb] = load_chunk(at[g], kb);
-    }
-    // (the filters are older than the rows)
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G * KB) : "memory");
-    ldsBarrier();
-    int half = 0;
-    while (true) {
-      // (every wave has left the other half of the ring)
-      const uint32_t phase_after = next_phase(phases_left);
-      if (phase_after != 0) filters_to_lds(phase_after, half ^ 1);
-      Way way = way_through(phase);
-      const bool took_part = (way.both | way.first | way.second) != 0;
-      const char *ring = s_w + half * OPP * W_BYTES + lane * 16;
-      auto filter_of = [&](int k) { return ring + __popc(phase & ((1u << k) - 1u)) * W_BYTES; };
-      for (; way.both != 0; way.both &= way.both - 1)
-        multiply(std::integral_constant<int, 3>(), filter_of(__builtin_ctz(way.both)));
-      for (; way.first != 0; way.first &= way.first - 1)
-        multiply(std::integral_constant<int, 1>(), filter_of(__builtin_ctz(way.first)));
-      for (; way.second != 0; way.second &= way.second - 1)
-        multiply(std::integral_constant<int, 2>(), filter_of(__builtin_ctz(way.second)));
-      if (phase_after == 0) break;
-      // the filters requested in front of this phase are older than the rows requested in it
-      if (took_part)
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(G * KB) : "memory");
-      else
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      ldsBarrier();
-      phase = phase_after;
-      half ^= 1;
-    }
-    } else {
-    // Where the rows of a phase's offsets begin, for this lane's share of the loads (a KiB each: whole
-    // lines of whole rows); behind the tensor where the phase has no such offset.
-    auto locate_rows = [&](uint32_t phase, uint32_t (&at)[OPP][G][LPG]) {
+    // Rows in one of two sets of registers, filters in one of two ring buffers.
+    vec8 rows_a[OPP][G], rows_b[OPP][G];
+    auto request_phase = [&](uint32_t phase, int half, vec8 (&rows)[OPP][G]) {
+      filters_to_lds(phase, half);
       uint32_t left = phase;
 #pragma unroll
       for (int o = 0; o < OPP; ++o) {
-        const uint32_t nowhere = left != 0 ? 0u : kNoRow;
-        const int kk = left != 0 ? __builtin_ctz(left) : 0;
+        const bool there = left != 0;
+        const int kk = there ? __builtin_ctz(left) : 0;
         left &= left - 1;
 #pragma unroll
-        for (int g = 0; g < G; ++g)
-#pragma unroll
-          for (int j = 0; j < LPG; ++j)
-            at[o][g][j] = s_map[kk][wave * (G * 16) + g * 16 + j * RPL + lane / (64 / RPL)] | nowhere;
-      }
-    };
-    auto request_row = [&](uint32_t at, int j) -> u32x4 {
-      return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                           a_rows, __builtin_elementwise_add_sat(at, piece_at[j]), 0, 0));
-    };
-    auto request_filter = [&](uint32_t phase, int t) -> u32x4 {
-      return *reinterpret_cast<const u32x4 *>(fragment_of(phase, (wave + t * WAVES) % BUF_FRAGS));
-    };
-    auto store_filter = [&](u32x4 v, int t, int half) {
-      *reinterpret_cast<u32x4 *>(s_w + (half * BUF_FRAGS + (wave + t * WAVES) % BUF_FRAGS) * 1024 + lane * 16) = v;
-    };
-    // One phase: its rows in `set` go through the wave's place in LDS into operand registers, and
-    // `set` is requested again for the phase after the next, as are the filters.  The requests are
-    // spread between the multiplies: made together they keep all waves waiting for the CU's
-    // address unit at the same time, with nothing left to multiply.  No load and no multiply
-    // depends on what the wave has to do: a wave without rows at an offset multiplies zeros,
-    // and the number of loads in flight is the same on every way through the loop, so that
-    // the compiler waits for exactly the ones it needs.
-    u32x4 filters[FPW];
-    auto take_phase = [&](uint32_t after_that, int half, u32x4 (&set)[OPP][G][LPG]) {
-      // steps of up to four column blocks of one chunk; a step's fragments are read while the
-      // step before is multiplied
-      constexpr int NS = NB < 4 ? NB : 4, PER = NB / NS, STEPS = KB * PER;
-      uint32_t at[OPP][G][LPG];
-      locate_rows(after_that, at);
-#pragma unroll
-      for (int o = 0; o < OPP; ++o) {
-#pragma unroll
-        for (int g = 0; g < G; ++g)
-#pragma unroll
-          for (int j = 0; j < LPG; ++j)
-            *reinterpret_cast<u32x4 *>(rows_lds + (g * LPG + j) * 1024 + lane * 16) = set[o][g][j];
-        const char *const wbuf = s_w + (half * BUF_FRAGS + o * FRAGS) * 1024 + lane * 16;
-        vec8 rows[2][G], w[2][NS];
-        auto read_step = [&](int step) {
-          const int kb = step / PER, nb0 = step % PER * NS;
-          if (step % PER == 0) {
-#pragma unroll
-            for (int g = 0; g < G; ++g)
-              rows[kb & 1][g] = *reinterpret_cast<const vec8 *>(
-                  rows_lds + (g * 16 + pair) * ROW_BYTES + (((kb * 4 + quad) ^ denseRowSwizzle(ROW_BYTES, pair)) * 16));
-          }
-#pragma unroll
-          for (int i = 0; i < NS; ++i)
-            w[step & 1][i] = *reinterpret_cast<const vec8 *>(wbuf + ((nb0 + i) * KB + kb) * 1024);
-        };
-        read_step(0);
-#pragma unroll
-        for (int step = 0; step < STEPS; ++step) {
-          if (step + 1 < STEPS) read_step(step + 1);
-          // this step's share of the requests
-#pragma unroll
-          for (int x = 0; x < G * LPG; ++x)
-            if (x * STEPS / (G * LPG) == step) set[o][x / LPG][x % LPG] = request_row(at[o][x / LPG][x % LPG], x % LPG);
-#pragma unroll
-          for (int t = 0; t < FPW; ++t)
-            if (t * (OPP * STEPS) / FPW == o * STEPS + step) {
-              store_filter(filters[t], t, half ^ 1);
-              filters[t] = request_filter(after_that, t);
-            }
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int i = 0; i < NS; ++i)
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-              float4v &sum = acc[g][step % PER * NS + i];
-              sum = E::mfma(w[step & 1][i], rows[(step / PER) & 1][g], sum);
-            }
+        for (int g = 0; g < G; ++g) {
+          const uint32_t at = there ? s_map.at[kk][row_first + g * 16] : kNoRow;
+          rows[o][g] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(
+                                                    a_rows, __builtin_elementwise_add_sat(at, piece_at), 0, 0));
         }
       }
-      ldsBarrier();
     };
-
-    u32x4 rows_a[OPP][G][LPG], rows_b[OPP][G][LPG];
+    // Everything this wave has requested is there.  The rows pass through an empty statement
+    // that the compiler must take for their last writer: it then places its own wait for their
+    // loads here, and not in front of their first use, behind the next phase's requests, which
+    // it would wait for as well.
+    auto landed = [&](vec8 (&rows)[OPP][G]) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int o = 0; o < OPP; ++o)
+#pragma unroll
+        for (int g = 0; g < G; ++g) asm volatile("" : "+v"(rows[o][g]));
+    };
+    auto multiply_phase = [&](int half, const vec8 (&rows)[OPP][G]) {
+      const char *filters = s_w + half * BUF_FRAGS * 1024 + lane * 16;
+#pragma unroll
+      for (int o = 0; o < OPP; ++o)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          const vec8 w = *reinterpret_cast<const vec8 *>(filters + o * W_BYTES + nb * 1024);
+#pragma unroll
+          for (int g = 0; g < G; ++g) acc[g][nb] = E::mfma(w, rows[o][g], acc[g][nb]);
+        }
+    };
     uint32_t left = offsets;
-    uint32_t p0 = next_phase(left), p1 = next_phase(left), p2 = 0;
-    {
-      auto request_phase = [&](uint32_t phase, u32x4 (&set)[OPP][G][LPG]) {
-        uint32_t at[OPP][G][LPG];
-        locate_rows(phase, at);
-#pragma unroll
-        for (int x = 0; x < OPP * G * LPG; ++x)
-          set[x / (G * LPG)][x / LPG % G][x % LPG] = request_row(at[x / (G * LPG)][x / LPG % G][x % LPG], x % LPG);
-      };
-#pragma unroll
-      for (int t = 0; t < FPW; ++t) filters[t] = request_filter(p0, t);
-      request_phase(p0, rows_a);
-#pragma unroll
-      for (int t = 0; t < FPW; ++t) store_filter(filters[t], t, 0);
-      asm volatile("" ::: "memory");
-#pragma unroll
-      for (int t = 0; t < FPW; ++t) filters[t] = request_filter(p1, t);
-      request_phase(p1, rows_b);
+    uint32_t phase = next_phase(left);
+    request_phase(phase, 0, rows_a);
+    landed(rows_a);
+    ldsBarrier();
+    while (true) {
+      phase = next_phase(left);
+      if (phase != 0) request_phase(phase, 1, rows_b);
+      multiply_phase(0, rows_a);
+      if (phase == 0) break;
+      landed(rows_b);
       ldsBarrier();
-    }
-    // (two phases a trip and one way out of the loop, at the price of an empty phase at the end of an
-    // odd number of them: with a second way out the compiler waits for all loads at the loop's head)
-    do {
-      p2 = next_phase(left);
-      take_phase(p2, 0, rows_a);
-      p0 = next_phase(left);
-      take_phase(p0, 1, rows_b);
-      p1 = p0;
-      p0 = p2;
-    } while (p0 != 0);
+      phase = next_phase(left);
+      if (phase != 0) request_phase(phase, 0, rows_a);
+      multiply_phase(1, rows_b);
+      if (phase == 0) break;
+      landed(rows_a);
+      ldsBarrier();
     }
   }
   // lane holds result columns 16*nb + 4*quad + (0..3) of row 16*g + pair of its wave's rows
@@ -2325,20 +2064,253 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
       storeColumns<E>(result + (size_t)r * conv.c, nb * 16 + quad * 4, conv.c, tmp);
     }
   }
+  if constexpr (!SRC::kSegments) storeDenseSlots(s_map, slots, source.filled);
+}
+
+// ---- rows above 64 bytes
+//
+// The waves of a workgroup split the result COLUMNS between them (below 64 columns the rows as well) and share the
+// tile's gathered rows: a phase's rows go from memory straight into one of two LDS buffers (16-byte loads in the
+// order of the rows, four or eight rows a load; their pieces permuted so that operand reads meet no bank
+// twice), while the phase before is multiplied, and every wave reads them from there.  A wave's filter
+// columns are its own: they come into registers, one phase ahead as well.  Row groups without a partner at
+// an offset are neither loaded nor multiplied.  Rows of 256 bytes take two phases an offset, half of their
+// channels each, so that three workgroups share a CU; what one of them waits for the others multiply through.
+//
+// What bounds it: instructions per phase and the CU's 64 bytes a clock from the L2, for rows (20 KB an offset
+// and tile at 128 channels, 0.6 of the groups present) and filters (32 KB).  Loads in operand order, 16 rows
+// of 64 bytes each, take the address unit 64 clocks a KiB, whole rows 20, which is why rows go through LDS.  us,
+// 248 636 rows of a scene, 27 offsets, with the filter's packing, this kernel / filters through LDS with
+// rows in operand order (128) or through registers and LDS (64):
+//   fp16 128 -> 128 167/210    64 -> 64 82/95
+// Of two offsets a phase (64 channels: 93), tiles of 256 rows (128: 233; 64: 123), whole rows of 256 bytes (185),
+// quarters (181) and 32 columns a wave at 64 (86) none is faster.
+struct StagedPlan {
+  int column_waves;   // waves side by side; the others are below each other
+  int column_blocks;  // of 16 result columns, of a wave
+  int parts;          // phases a row's channels are split over
+};
+constexpr StagedPlan stagedPlan(int elem_bytes, int Q, int C) {
+  return StagedPlan{C >= 64 ? 4 : (C >= 32 ? 2 : 1), C >= 128 ? 2 : 1, Q * elem_bytes >= 256 ? 2 : 1};
+}
+constexpr int kStagedPerCu = 3;  // workgroups a CU
+// Where piece `piece` of a staged row lies among its row's pieces: at piece ^ this.
+__device__ __forceinline__ int stagedSwizzle(int row) {
+  return (row >> 1) & 7;
+}
+
+// 16 bytes per lane from byte `offset` of a buffer straight into LDS (as requestToLds); zeros for offsets behind its
+// end.
+__device__ __forceinline__ void requestRowsToLds(u32x4 rows, uint32_t offset, uint32_t lds_address) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               :: "s"(lds_address), "v"(offset), "s"(rows) : "memory", "m0");
+}
+
+template <typename E, int Q, int C, typename SRC>
+__global__ __launch_bounds__(kDenseThreads) __attribute__((amdgpu_waves_per_eu(kStagedPerCu, kStagedPerCu)))
+void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRows conv,
+                           const typename E::storage *packedW, SRC source, int R, int K, typename E::storage *result) {
+  typedef typename E::vec8 vec8;
+  typedef typename E::storage S;
+  constexpr StagedPlan PLAN = stagedPlan((int)sizeof(S), Q, C);
+  constexpr int WAVES = kDenseThreads / 64;
+  constexpr int CW = PLAN.column_waves;
+  constexpr int NB = PLAN.column_blocks;         // of this wave
+  constexpr int G = kDenseGroups / (WAVES / CW);  // row groups of this wave
+  constexpr int KC = kDenseChunk;
+  constexpr int RB = Q * (int)sizeof(S);
+  constexpr int PARTS = PLAN.parts;
+  constexpr int SB = RB / PARTS;                 // bytes of a row staged in one phase
+  constexpr int KB = RB / 64;                    // fragments of a row
+  constexpr int KP = KB / PARTS;
+  constexpr int PPR = SB / 16;
+  constexpr int RPL = 1024 / SB;                 // rows a load of 1 KiB stages
+  constexpr int LPG = 16 / RPL;                  // loads a row group
+  constexpr int GPW = kDenseGroups / WAVES;      // row groups a wave stages
+  constexpr int BUFFER = kDenseRows * SB;
+  constexpr int W_BYTES = (C / 16) * KB * 1024;  // packed filter of an offset
+  static_assert(SB == 128 && CW * NB * 16 == C && WAVES % CW == 0, "split");
+
+  __shared__ __attribute__((aligned(1024))) char s_rows[2 * BUFFER];
+  __shared__ __attribute__((aligned(16))) DenseMap s_map;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tiles_per_xcd = gridDim.x >> 3;  // neighbouring tiles on one XCD, as above
+  const int tile = (blockIdx.x & 7) * tiles_per_xcd + (blockIdx.x >> 3);
+  const int r0 = tile * kDenseRows;
   if constexpr (!SRC::kSegments) {
-    // s_has is free again: the waves' slot counts meet there
-    __syncthreads();
-    int wave_slots = slots;
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) wave_slots += __shfl_xor(wave_slots, d, kWave);
-    if (lane == 0) s_has[wave] = wave_slots;
-    __syncthreads();
-    if (tid == 0) {
-      int all = 0;
-      for (int w = 0; w < WAVES; ++w) all += s_has[w];
-      source.filled[blockIdx.x] = all;
+    if (notWanted(source.run_if)) return;
+  }
+  if (r0 >= R) {
+    if constexpr (!SRC::kSegments) {
+      if (tid == 0) source.filled[blockIdx.x] = 0;
+    }
+    return;
+  }
+  if constexpr (SRC::kSegments) {
+    if (*source.verdict == source.ticket) {
+      if (!source.leave_if_unordered) denseTileOutOfOrder<E>(s_map, A, conv, source, r0, R, K, result);
+      return;
     }
   }
+  const int pair = lane & 15;
+  const int quad = lane >> 4;
+  const int first_group = wave / CW * G;          // this wave's rows,
+  const int first_block = wave % CW * NB;         // and columns
+  const int row_first = first_group * 16 + pair;  // this lane's row in the first group
+  const char *const w_base = reinterpret_cast<const char *>(packedW) + first_block * KB * 1024 + lane * 16;
+  const unsigned long long *const nonfinite =
+      reinterpret_cast<const unsigned long long *>(reinterpret_cast<const char *>(packedW) + (size_t)K * W_BYTES);
+  const uint32_t rows_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)s_rows;
+  // Where this lane's operand pieces of its wave's first row group lie.
+  const char *lane_rows[KP];
+#pragma unroll
+  for (int kb = 0; kb < KP; ++kb) lane_rows[kb] = s_rows + row_first * SB + ((kb * 4 + quad) ^ stagedSwizzle(pair)) * 16;
+  // Which piece of a row this lane stages, by load of a group.
+  const __amdgpu_buffer_rsrc_t a_rows = rowsBuffer(A, a_size);
+  const u32x4 rows_words = {(uint32_t)reinterpret_cast<uintptr_t>(A), (uint32_t)(reinterpret_cast<uintptr_t>(A) >> 32),
+                            a_size, 0x00020000u};  // (a_rows, as requestRowsToLds takes it)
+  uint32_t piece_of[PARTS][LPG];
+#pragma unroll
+  for (int part = 0; part < PARTS; ++part)
+#pragma unroll
+    for (int j = 0; j < LPG; ++j) {
+      const uint32_t piece = (uint32_t)((lane % PPR) ^ stagedSwizzle(j * RPL + lane / PPR)) * 16u + part * SB;
+      piece_of[part][j] = piece < (uint32_t)conv.row_bytes ? piece : kNoRow;
+    }
+
+  float4v acc[G][NB];
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[g][nb] = float4v{0.f, 0.f, 0.f, 0.f};
+  int slots = 0;  // filled map slots this thread staged
+
+  for (int kc = 0; kc < K; kc += KC) {
+    const int kn = (K - kc) < KC ? (K - kc) : KC;
+    __syncthreads();  // the chunk before is finished with s_map and the row buffers
+    slots += fillDenseMap(s_map, source, nonfinite, conv.row_bytes, tile, r0, R, kc, kn, K);
+    const int lane_groups = lane < kn ? (int)s_map.groups[lane] : 0;
+    const bool lane_finite = s_map.finite[lane < kn ? lane : 0] != 0;
+    // offsets of the chunk that have a pair in this tile; those of them whose filter is not finite go by themselves
+    const uint32_t offsets = (uint32_t)__ballot(lane_groups != 0 && lane_finite);
+    for (uint32_t left = (uint32_t)__ballot(lane_groups != 0 && !lane_finite); left != 0; left &= left - 1) {
+      const int kk = __builtin_ctz(left);
+      addOffsetApart<E, G, NB, KB>(
+          acc, a_rows, &s_map.at[kk][first_group * 16],
+          reinterpret_cast<const char *>(packedW) + (size_t)(kc + kk) * W_BYTES + first_block * KB * 1024, conv.row_bytes);
+    }
+    if (offsets == 0) continue;
+    // A phase is a part of one offset's channels.  kk < 0: none is left; nothing is staged and nothing multiplied.
+    uint32_t left = offsets;
+    auto next_offset = [&]() -> int {
+      const int kk = left != 0 ? __builtin_ctz(left) : -1;
+      left &= left - 1;
+      return kk;
+    };
+    auto groups_of = [&](int kk) -> uint32_t {
+      return kk < 0 ? 0u : (uint32_t)__builtin_amdgcn_readlane(lane_groups, kk);
+    };
+    typedef vec8 Filters[NB][KP];
+    // The row groups the wave stages straight into LDS, and its filter columns into registers.
+    auto request = [&](int kk, int part, int buffer, Filters &w) {
+      const int there = kk < 0 ? 0 : kk;
+      uint32_t at[GPW][LPG];  // (all places in the map are read before the first address is formed)
+#pragma unroll
+      for (int t = 0; t < GPW; ++t)
+#pragma unroll
+        for (int j = 0; j < LPG; ++j) at[t][j] = s_map.at[there][(wave + t * WAVES) * 16 + j * RPL + lane / PPR];
+      const char *const filter = w_base + (size_t)(kc + there) * W_BYTES;
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int kb = 0; kb < KP; ++kb)
+          w[nb][kb] = *reinterpret_cast<const vec8 *>(filter + (nb * KB + part * KP + kb) * 1024);
+#pragma unroll
+      for (int t = 0; t < GPW; ++t)
+#pragma unroll
+        for (int j = 0; j < LPG; ++j) {
+          at[t][j] = __builtin_elementwise_add_sat(at[t][j], piece_of[part][j]);
+          asm volatile("" : "+v"(at[t][j]));
+        }
+      const uint32_t groups = groups_of(kk) >> wave;
+#pragma unroll
+      for (int t = 0; t < GPW; ++t) {
+        if ((groups >> (t * WAVES) & 1u) == 0) continue;
+#pragma unroll
+        for (int j = 0; j < LPG; ++j)
+          requestRowsToLds(rows_words, at[t][j],
+                           rows_lds + (uint32_t)(buffer * BUFFER + ((wave + t * WAVES) * LPG + j) * 1024));
+      }
+    };
+    // Everything this wave has requested is there.  The filters pass through an empty statement that the
+    // compiler must take for their last writer: its own wait for their loads then lies here, and not in front
+    // of their first use, behind the next phase's requests, which it would wait for as well.
+    auto landed = [&](Filters &w) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int kb = 0; kb < KP; ++kb) asm volatile("" : "+v"(w[nb][kb]));
+    };
+    // (a group's rows are read while the group before is multiplied; those of a group without partners are what
+    // the buffer held before, and nobody multiplies them)
+    auto multiply = [&](int kk, int buffer, const Filters &w) {
+      const uint32_t groups = groups_of(kk) >> first_group;
+      vec8 row[2][KP];
+      auto read_group = [&](int g) {
+#pragma unroll
+        for (int kb = 0; kb < KP; ++kb)
+          row[g & 1][kb] = *reinterpret_cast<const vec8 *>(lane_rows[kb] + buffer * BUFFER + g * 16 * SB);
+      };
+      read_group(0);
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        if (g + 1 < G) read_group(g + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if ((groups >> g & 1u) == 0) continue;
+#pragma unroll
+        for (int kb = 0; kb < KP; ++kb)
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) acc[g][nb] = E::mfma(w[nb][kb], row[g & 1][kb], acc[g][nb]);
+      }
+    };
+    // (two phases a trip and one way out of the loop, at the price of an empty phase at the end of an
+    // odd number of them: with a second way out the compiler waits for all loads in front of every use)
+    Filters w_a, w_b;
+    int now = next_offset();
+    request(now, 0, 0, w_a);
+    landed(w_a);
+    ldsBarrier();
+    do {
+      const int after = PARTS == 2 ? now : next_offset();
+      request(after, PARTS - 1, 1, w_b);
+      multiply(now, 0, w_a);
+      landed(w_b);
+      ldsBarrier();
+      now = next_offset();
+      request(now, 0, 0, w_a);
+      multiply(after, 1, w_b);
+      landed(w_a);
+      ldsBarrier();
+    } while (now >= 0);
+  }
+  // lane holds result columns 16*nb + 4*quad + (0..3) of row 16*g + pair of its wave's rows
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int r = r0 + row_first + g * 16;
+    if (r >= R) continue;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      S tmp[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) E::store(&tmp[e], activated(acc[g][nb][e], conv.relu));
+      storeColumns<E>(result + (size_t)r * conv.c, (first_block + nb) * 16 + quad * 4, conv.c, tmp);
+    }
+  }
+  if constexpr (!SRC::kSegments) storeDenseSlots(s_map, slots, source.filled);
 }
 
 // ---- pairs that lost their map slot -----------------------------------------------
@@ -3485,7 +3457,7 @@ int mfmaGridX(int R, int tile_cols) {
   const int tr = mfmaTileRows(tile_cols);
   return ((R + tr - 1) / tr + 7) / 8 * 8;
 }
-int denseGridX(int R, int tile_rows) { return ((R + tile_rows - 1) / tile_rows + 7) / 8 * 8; }
+int denseGridX(int R) { return ((R + kDenseRows - 1) / kDenseRows + 7) / 8 * 8; }
 
 template <typename E, int Q, int C, typename SRC>
 void launchMfmaInstance(const LaunchCtx &lc, const void *A, const ConvRows &rows, const void *packed,
@@ -3715,52 +3687,25 @@ bool useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims 
   return sheets && d.q_padded <= 32 && fill >= 0.2;
 }
 
-// Whether the kernel takes its wide tiles (densePlan).  Either shape has 256 rows on each of 256 CUs at a time,
-// so a launch takes rows / 65 536 rounds.  Up to half a CU's rows in the last round take the narrow tiles
-// half the time, and the wide ones that of a whole tile; in a round that is nearly full the narrow ones
-// pay for their phases of one offset and their second filters.  With more rounds the two come closer.  us of
-// gatherConvDense, wide / narrow, 27 offsets, by rounds:
-//   fp16 128 -> 128 scene   0.50 49/41, 0.60 49/50, 0.85 51/53, 1.00 53/56, 1.10 84/73, 1.40 96/88, 1.60 102/104,
-//                           2.00 104/113, 2.10 140/120, 2.60 142/141, 2.85 152/154, 3.30 203/180, 4.00 217/218
-//           strewn          0.50 45/41, 0.60 47/51, 1.10 93/82, 1.60 97/101, 2.00 104/113, 2.60 155/161, 3.00 163/181,
-//                           3.30 207/195, 4.00 225/229, 4.40 272/259, 4.70 271/288
-//           scene, row map  0.30 50/39, 0.60 53/55, 1.30 102/89, 1.85 113/117, 2.60 170/173, 2.85 174/188, 3.60 233/239
-//   bf16 96 -> 128 scene    0.50 50/42, 0.60 50/50, 1.00 52/54, 1.30 86/80, 1.60 88/91, 2.00 97/101, 2.60 141/131,
-//                           2.85 145/148, 3.30 168/161, 4.00 196/198
-//   fp32 64 -> 128 strewn   0.92 205/216, 1.04 392/320, 1.53 422/434, 2.06 630/559, 2.75 639/681
-// and a layer's training step on scenes, 128 -> 128, where the rows come from memory: 1.98 362/378, 2.90 523/527,
-// 3.43 619/589, 3.66 623/622, 3.79 632/648.
-bool denseWide(const ConvProblem &p, const GatherDims &d, int rows) {
-  constexpr int kRound = 256 * 256;
-  return d.q_padded * (int)elemSize(p.dtype) > 128 && d.c_padded == 128 && (rows - 1) % kRound >= kRound * 2 / 3;
-}
-
 template <typename E, int Q, int C, typename SRC>
-void launchDenseInstance(const LaunchCtx &lc, bool wide, const void *A, uint32_t a_size, const ConvRows &rows,
+void launchDenseInstance(const LaunchCtx &lc, const void *A, uint32_t a_size, const ConvRows &rows,
                          const void *packed, const SRC &source, int R, int K, void *result) {
-  lc.begin("gatherConvDense");
-  constexpr int kElem = (int)sizeof(typename E::storage);
-  auto launch = [&](auto wide_tag) {
-    constexpr bool WIDE = decltype(wide_tag)::value;
-    constexpr int kTileRows = denseTileRows(kElem, Q, C, WIDE), kThreads = 64 * densePlan(kElem, Q, C, WIDE).waves;
-    gatherConvDense<E, Q, C, SRC, WIDE><<<denseGridX(R, kTileRows), kThreads, 0, lc.stream>>>(
+  auto launch = [&](auto kernel) {
+    lc.begin("gatherConvDense");
+    kernel<<<denseGridX(R), kDenseThreads, 0, lc.stream>>>(
         static_cast<const typename E::storage *>(A), a_size, rows, static_cast<const typename E::storage *>(packed),
         source, R, K, static_cast<typename E::storage *>(result));
+    lc.end();
   };
-  if constexpr (Q * kElem > 128 && C == 128) {
-    if (wide) launch(std::true_type());
-    else launch(std::false_type());
-  } else {
-    launch(std::false_type());
-  }
-  lc.end();
+  if constexpr (Q * (int)sizeof(typename E::storage) > 64) launch(gatherConvDenseStaged<E, Q, C, SRC>);
+  else launch(gatherConvDense<E, Q, C, SRC>);
 }
 
 template <typename E, typename SRC>
-void launchDense(const LaunchCtx &lc, int q_padded, bool wide, const void *A, int n_src, const ConvRows &rows,
+void launchDense(const LaunchCtx &lc, int q_padded, const void *A, int n_src, const ConvRows &rows,
                  const void *packed, const SRC &source, int R, int K, void *result) {
   const uint32_t a_size = (uint32_t)n_src * (uint32_t)rows.row_bytes;
-#define DENSE_INSTANCE(q, c) launchDenseInstance<E, q, c, SRC>(lc, wide, A, a_size, rows, packed, source, R, K, result)
+#define DENSE_INSTANCE(q, c) launchDenseInstance<E, q, c, SRC>(lc, A, a_size, rows, packed, source, R, K, result)
 #define DENSE_BY_C(q)                       \
   switch (rows.c_padded) {                  \
     case 16: DENSE_INSTANCE(q, 16); break;  \
@@ -3857,7 +3802,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     // Pair lists in order (as far as the caller knows: the first kernel checks): the
     // gather kernel reads them cut by tile, no row map.
     const int tile_cols = dense ? d.c_padded : mfmaTileCols(p, d);
-    const int tile_rows = dense ? denseTileRows((int)sizeof(S), d.q_padded, d.c_padded, denseWide(p, d, d.R))
+    const int tile_rows = dense ? kDenseRows
                           : tall ? tallRows(tall_q * (int)sizeof(S)) / (half_tiles ? 2 : 1)
                                  : mfmaTileRows(tile_cols);
     int tile_shift = 0;
@@ -3894,8 +3839,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     src.sC = sC;
     src.counts = inl;
     if (dense)
-      launchDense<E, SegmentSource>(lc, d.q_padded, denseWide(p, d, d.R), rows_from, d.n_src, rows_of, ws.packed, src,
-                                    d.R, p.K, result);
+      launchDense<E, SegmentSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, src, d.R, p.K, result);
     else if (tall)
       launchTall<E, SegmentSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, src, half_tiles, d.R, p.K,
                                    result);
@@ -3937,10 +3881,8 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
       if (own_map) n_accepted = launchScatterRowMap(lc, p, d, ws, inl, max_count, row_base, rows, run_if);
       const MapSource map = {entries, ws.filled, run_if};
       if (dense) {
-        const bool wide = denseWide(p, d, rows);
-        n_filled = denseGridX(rows, denseTileRows((int)sizeof(S), d.q_padded, d.c_padded, wide));
-        launchDense<E, MapSource>(lc, d.q_padded, wide, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K,
-                                  result_rows);
+        n_filled = denseGridX(rows);
+        launchDense<E, MapSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K, result_rows);
       } else if (tall) {
         n_filled = tallGridX(rows, tallRows(tall_q * (int)sizeof(S)));
         launchTall<E, MapSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, map, false, rows, p.K, result_rows);
