@@ -17,6 +17,9 @@
 //   5 rankFlags        bitmap of the cells' first points with prefix sums: the voxel number of a cell
 //                      is the number of first points in front of its own
 //   6 voxAssign        in point order: copies points and coordinates, writes the counts
+// Clouds of up to kFewPoints points take three launches instead (voxTagPoints, voxRankFew, voxAssign): every
+// bucket's workgroup picks its points out of all of them, and every workgroup of the last one counts the
+// first points itself.
 // Integer atomics only (LDS counts and table insertion): the outputs are the same bits on
 // every run.
 //
@@ -31,6 +34,7 @@
 #include <hip/hip_runtime.h>
 
 #include "core/device_sort.h"
+#include "core/wave_scan.h"
 
 #include "voxelization/voxelize.h"
 
@@ -117,6 +121,11 @@ __device__ inline u64 cellKey(const Cell &c) {
 // A grid of fewer than 2^32 - 1 cells (the same for every thread) has 32-bit keys; in a larger
 // one the cell of a partitioned point is worked out again from the point.
 __device__ inline bool smallGrid(u64 cells) { return cells < 0xffffffffull; }
+
+__device__ inline u64 gridCells(const float *__restrict__ voxel_size, const float *__restrict__ range) {
+  return (u64)axisCells(range[2], range[5], voxel_size[2]) * (u64)axisCells(range[1], range[4], voxel_size[1]) *
+         (u64)axisCells(range[0], range[3], voxel_size[0]);
+}
 
 // Up to four regions of 32-bit words cleared by one launch.
 constexpr int kClearRegions = 4;
@@ -225,7 +234,8 @@ template <int THREADS, int SLOTS, typename TABLE>
 __device__ __forceinline__ bool rankBucket(const TABLE &t, const u64 *__restrict__ entries, uint32_t count,
                            const float *__restrict__ points, const float *__restrict__ voxel_size,
                            const float *__restrict__ range, int num_features, bool small_grid, uint32_t max_points,
-                           volatile uint16_t *s_owner, uint32_t *__restrict__ state, uint32_t *__restrict__ first_of) {
+                           volatile uint16_t *s_owner, uint32_t *__restrict__ state, uint32_t *__restrict__ first_of,
+                           uint8_t *first_flags = nullptr) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (TABLE::kFills && tid == 0) *t.used = 0;
   for (uint32_t s = tid; s < t.slots; s += THREADS) {
@@ -280,7 +290,8 @@ __device__ __forceinline__ bool rankBucket(const TABLE &t, const u64 *__restrict
       open &= ~same;
     }
     uint32_t before = 0;
-    for (int w = 0; w < (THREADS / 64); ++w) {
+    const uint32_t waves = (count - base + 63) / 64;  // that have points
+    for (int w = 0; w < (int)(waves < THREADS / 64 ? waves : THREADS / 64); ++w) {
       if (wave == w && live && rank == 0) {
         before = t.counts[slot];
         t.counts[slot] = before + group;
@@ -297,7 +308,10 @@ __device__ __forceinline__ bool rankBucket(const TABLE &t, const u64 *__restrict
   __syncthreads();
   for (uint32_t s = tid; s < t.slots; s += THREADS) {
     const uint32_t c = t.counts[s];
-    if (c != 0) state[t.firsts[s]] = kIsFirst | (c < max_points ? c : max_points);
+    if (c == 0) continue;
+    const uint32_t first = t.firsts[s];
+    state[first] = kIsFirst | (c < max_points ? c : max_points);
+    if (first_flags != nullptr) first_flags[first] = 1;  // (a bit each, set by atomics, took 5 us at 23 k points)
   }
   return true;
 }
@@ -306,39 +320,185 @@ __device__ __forceinline__ bool rankBucket(const TABLE &t, const u64 *__restrict
 // rank in the cell for another point it keeps, whose first_of[i] is the first one; 0 otherwise.
 // A bucket of any number of points is ranked in LDS as long as its cells fit there, which those of a
 // crowded cell do; the table in device memory takes several times as long.
+//
+// The ranks of one bucket's `count` points, `entries` in point order.  `wide_at`: where the bucket's share of the
+// region in device memory begins.
+template <int THREADS, int SLOTS>
+__device__ __forceinline__ void rankCells(const float *__restrict__ points, const float *__restrict__ voxel_size,
+                                          const float *__restrict__ range, int num_features, uint32_t max_points,
+                                          const u64 *__restrict__ entries, uint32_t count, size_t wide_at, u64 *wide_keys,
+                                          uint32_t *wide_counts, uint32_t *wide_firsts, uint32_t *__restrict__ state,
+                                          uint32_t *__restrict__ first_of, uint8_t *first_flags, bool small_grid) {
+  __shared__ uint32_t s_keys[SLOTS], s_counts[SLOTS], s_firsts[SLOTS];
+  __shared__ uint16_t s_owner[SLOTS];
+  __shared__ uint32_t s_used;
+  if (small_grid) {
+    if (__builtin_expect(count <= SLOTS / 2, 1)) {
+      LdsTable<false> t = {s_keys, s_counts, s_firsts, 64, nullptr};
+      while (t.slots < 2 * count) t.slots <<= 1;
+      rankBucket<THREADS, SLOTS>(t, entries, count, points, voxel_size, range, num_features, true, max_points, s_owner,
+                                 state, first_of, first_flags);
+      return;
+    }
+    const LdsTable<true> t = {s_keys, s_counts, s_firsts, SLOTS, &s_used};
+    if (rankBucket<THREADS, SLOTS>(t, entries, count, points, voxel_size, range, num_features, true, max_points, s_owner,
+                                   state, first_of, first_flags))
+      return;
+  }
+  // the bucket's share of the region: the largest power of two within three slots a point
+  const WideTable t = {wide_keys + wide_at, wide_counts + wide_at, wide_firsts + wide_at, 1u << (31 - __clz(3 * count)),
+                       nullptr};
+  rankBucket<THREADS, SLOTS>(t, entries, count, points, voxel_size, range, num_features, small_grid, max_points, s_owner,
+                             state, first_of, first_flags);
+}
+
 template <int THREADS, int SLOTS>
 __global__ __launch_bounds__(THREADS) void voxRankInCells(
     const float *__restrict__ points, const float *__restrict__ voxel_size, const float *__restrict__ range,
     int num_features, uint32_t max_points, const u64 *__restrict__ grouped, const uint32_t *__restrict__ bucket_start,
     const uint32_t *__restrict__ totals, u64 *wide_keys, uint32_t *wide_counts, uint32_t *wide_firsts,
     uint32_t *__restrict__ state, uint32_t *__restrict__ first_of) {
-  __shared__ uint32_t s_keys[SLOTS], s_counts[SLOTS], s_firsts[SLOTS];
-  __shared__ uint16_t s_owner[SLOTS];
-  __shared__ uint32_t s_used;
   const uint32_t count = totals[blockIdx.x];
   if (count == 0) return;
   const uint32_t start = bucket_start[blockIdx.x];
-  const bool small_grid =
-      smallGrid((u64)axisCells(range[2], range[5], voxel_size[2]) * (u64)axisCells(range[1], range[4], voxel_size[1]) *
-                (u64)axisCells(range[0], range[3], voxel_size[0]));
-  if (small_grid) {
-    if (__builtin_expect(count <= SLOTS / 2, 1)) {
-      LdsTable<false> t = {s_keys, s_counts, s_firsts, 64, nullptr};
-      while (t.slots < 2 * count) t.slots <<= 1;
-      rankBucket<THREADS, SLOTS>(t, grouped + start, count, points, voxel_size, range, num_features, true, max_points,
-                                 s_owner, state, first_of);
-      return;
-    }
-    const LdsTable<true> t = {s_keys, s_counts, s_firsts, SLOTS, &s_used};
-    if (rankBucket<THREADS, SLOTS>(t, grouped + start, count, points, voxel_size, range, num_features, true, max_points,
-                                   s_owner, state, first_of))
-      return;
+  rankCells<THREADS, SLOTS>(points, voxel_size, range, num_features, max_points, grouped + start, count,
+                            3 * (size_t)start, wide_keys, wide_counts, wide_firsts, state, first_of, nullptr,
+                            smallGrid(gridCells(voxel_size, range)));
+}
+
+// ---- few points ---------------------------------------------------------------------------
+//
+// A cloud of one sweep is a chain of launches that start cold and hold a handful of workgroups: the partition
+// alone took three of them, 16 of the six launches' 29 us at 23 k points.  Here a point is tagged with its
+// bucket, one byte, and every bucket's workgroup, one a CU, reads all tags (sixteen a load) and puts its own points
+// in order by prefix sums.  Three launches, 3.1 + 8.6 + 5.4 us at 23 k points.  What the tags and the first points'
+// flags cost grows with the points.  us of the layer's call, six launches / three: 5 k points 36.6/25.8, 12 k 38.8/28.4,
+// 23 k 39.1/29.1, 40 k 40.2/32.0, 65 k 41.3/39.1, which is where the line lies.
+constexpr int kFewPoints = 1 << 16;
+constexpr uint32_t kFewBuckets = 255;
+constexpr uint32_t kFewNone = 255;                     // the tag of a point outside the grid
+constexpr int kFewThreads = 512;
+constexpr int kFewTags = 16 * kFewThreads;             // tags the workgroup reads in a round
+constexpr int kFewRounds = kFewPoints / kFewTags;
+constexpr int kFewListed = 1024;                       // points of a bucket that are listed in LDS
+static_assert(kFewRounds % 2 == 0 && kFewTags < 1 << 16, "two rounds' counts in one word");
+
+// (multiples of whole rounds: the tags behind the last point are kFewNone)
+inline size_t fewTags(int64_t n) { return ((size_t)n + kFewTags - 1) / kFewTags * kFewTags; }
+
+// A point a thread in the first `point_blocks` workgroups; the others clear.
+__global__ __launch_bounds__(kBlock) void voxTagPoints(const float *__restrict__ points,
+                                                       const float *__restrict__ voxel_size,
+                                                       const float *__restrict__ range, int n, int num_features,
+                                                       int point_blocks, int tags_end, uint32_t *__restrict__ keys,
+                                                       uint8_t *__restrict__ tags, ClearRegions clear) {
+  if ((int)blockIdx.x >= point_blocks) {
+    clearRegions(clear, blockIdx.x - point_blocks, gridDim.x - point_blocks);
+    return;
   }
-  // the bucket's share of the region: the largest power of two within three slots a point
-  const size_t at = 3 * (size_t)start;
-  const WideTable t = {wide_keys + at, wide_counts + at, wide_firsts + at, 1u << (31 - __clz(3 * count)), nullptr};
-  rankBucket<THREADS, SLOTS>(t, grouped + start, count, points, voxel_size, range, num_features, small_grid, max_points,
-                             s_owner, state, first_of);
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= tags_end) return;
+  uint32_t tag = kFewNone;
+  if (i < n) {
+    const Cell c = cellOfPoint(points + (size_t)i * num_features, voxel_size, range);
+    if (c.cz >= 0) {
+      const u64 key = cellKey(c);
+      tag = __umulhi((uint32_t)mix64(key), kFewBuckets);
+      keys[i] = (uint32_t)key;
+    }
+  }
+  tags[i] = (uint8_t)tag;
+}
+
+// Bit 7 of every byte of `word` that is `byte`.
+__device__ __forceinline__ uint32_t bytesEqual(uint32_t word, uint32_t byte) {
+  const uint32_t x = word ^ (byte * 0x01010101u);
+  return ~(((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x | 0x7f7f7f7fu);
+}
+
+// *cursor (cleared before): points of the buckets that have taken their places in `grouped`, in no particular order:
+// those with more points than the list in LDS holds.
+__global__ __launch_bounds__(kFewThreads) void voxRankFew(
+    const float *__restrict__ points, const float *__restrict__ voxel_size, const float *__restrict__ range, int n,
+    int num_features, uint32_t max_points, const uint32_t *__restrict__ keys, const uint8_t *__restrict__ tags,
+    uint32_t *cursor, u64 *grouped, u64 *wide_keys, uint32_t *wide_counts, uint32_t *wide_firsts,
+    uint32_t *__restrict__ state, uint32_t *__restrict__ first_of, uint8_t *__restrict__ first_flags) {
+  constexpr int kWaves = kFewThreads / 64;
+  __shared__ uint32_t s_wave[kFewRounds / 2][kWaves];
+  __shared__ u64 s_list[kFewListed];
+  __shared__ uint32_t s_start;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t bucket = blockIdx.x;
+  const int rounds = (n + kFewTags - 1) / kFewTags;
+  const bool small_grid = smallGrid(gridCells(voxel_size, range));
+  uint4 t[kFewRounds];
+#pragma unroll
+  for (int r = 0; r < kFewRounds; ++r) {
+    t[r] = make_uint4(~0u, ~0u, ~0u, ~0u);
+    if (r < rounds) t[r] = reinterpret_cast<const uint4 *>(tags)[(size_t)r * kFewThreads + tid];
+  }
+  uint32_t match[kFewRounds];        // bit 4 q + b: byte b of word q is one of the bucket's
+  uint32_t before[kFewRounds / 2];   // two rounds a word: matches of the threads before, in the wave
+#pragma unroll
+  for (int r = 0; r < kFewRounds; ++r) {
+    match[r] = 0;
+    if (r < rounds) {
+      const uint32_t words[4] = {t[r].x, t[r].y, t[r].z, t[r].w};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t eq = bytesEqual(words[q], bucket) >> 7;
+        match[r] |= ((eq | eq >> 7 | eq >> 14 | eq >> 21) & 15u) << (4 * q);
+      }
+    }
+    if (r % 2 == 1) {
+      const uint32_t mine = (uint32_t)__popc(match[r - 1]) | (uint32_t)__popc(match[r]) << 16;
+      uint32_t incl = 0;
+      if (r - 1 < rounds) incl = (uint32_t)waveInclusiveScan((int)mine);
+      before[r / 2] = incl - mine;
+      if (lane == 63) s_wave[r / 2][wave] = incl;
+    }
+  }
+  __syncthreads();
+  uint32_t count = 0, first[kFewRounds];
+#pragma unroll
+  for (int r = 0; r < kFewRounds; ++r) {
+    const int shift = r % 2 * 16;
+    first[r] = before[r / 2] >> shift & 0xffffu;
+    if (r < rounds) {
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        if (w == wave) first[r] += count;
+        count += s_wave[r / 2][w] >> shift & 0xffffu;
+      }
+    }
+  }
+  if (count == 0) return;
+  // (grids whose keys need 64 bits take a table in device memory, for which a bucket needs its place there)
+  const bool listed = count <= (uint32_t)kFewListed && small_grid;
+  if (!listed) {
+    if (tid == 0) s_start = atomicAdd(cursor, count);
+    __syncthreads();
+  }
+  const uint32_t start = listed ? 0u : s_start;
+#pragma unroll
+  for (int r = 0; r < kFewRounds; ++r) {
+    uint32_t to = first[r];
+    for (uint32_t left = match[r]; left != 0; left &= left - 1) {
+      const uint32_t i = (uint32_t)(r * kFewTags + tid * 16 + __ffs((int)left) - 1);
+      const u64 entry = (u64)i << 32 | keys[i];
+      if (listed) s_list[to++] = entry;
+      else grouped[start + to++] = entry;
+    }
+  }
+  __syncthreads();
+  if (!listed) {
+    rankCells<kFewThreads, 2048>(points, voxel_size, range, num_features, max_points, grouped + start, count,
+                                 3 * (size_t)start, wide_keys, wide_counts, wide_firsts, state, first_of, first_flags,
+                                 small_grid);
+    return;
+  }
+  rankCells<kFewThreads, 2048>(points, voxel_size, range, num_features, max_points, s_list, count, 0, wide_keys,
+                               wide_counts, wide_firsts, state, first_of, first_flags, true);
 }
 
 // ---- voxel numbers -----------------------------------------------------------------------
@@ -356,14 +516,67 @@ struct FirstPoints {
   __device__ bool flagged(int64_t i) const { return (state[i] & kIsFirst) != 0; }
 };
 
+// First points in front of a point, from a byte a point (few points): every workgroup counts all of them.
+struct FewFirsts {
+  const uint4 *flags;
+  int pieces;  // of 16 points
+};
+struct FewSums {
+  static constexpr int kPer = kFewPoints / 16 / kBlock;  // pieces a thread sums up
+  uint32_t piece[kFewPoints / 16];
+  uint32_t wave[kBlock / 64];
+  __device__ static uint32_t sum(uint4 f) { return (uint32_t)(__popc(f.x) + __popc(f.y) + __popc(f.z) + __popc(f.w)); }
+  __device__ uint32_t add(const FewFirsts &f) {
+    const int tid = threadIdx.x;
+    uint4 flags[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      flags[u] = make_uint4(0, 0, 0, 0);
+      if (u * kBlock < f.pieces) flags[u] = f.flags[min(u * kBlock + tid, f.pieces - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < kPer; ++u)
+      piece[u * kBlock + tid] = u * kBlock + tid < f.pieces ? sum(flags[u]) : 0u;
+    __syncthreads();
+    const int per = (f.pieces + kBlock - 1) / kBlock, first = tid * per;
+    uint32_t mine = 0, all = 0;
+    for (int u = 0; u < per; ++u) mine += piece[first + u];
+    const uint32_t incl = (uint32_t)waveInclusiveScan((int)mine);
+    if ((tid & 63) == 63) wave[tid >> 6] = incl;
+    __syncthreads();
+    uint32_t run = incl - mine;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; ++w) {
+      run += w < (tid >> 6) ? wave[w] : 0u;
+      all += wave[w];
+    }
+    for (int u = 0; u < per; ++u) {
+      const uint32_t c = piece[first + u];
+      piece[first + u] = run;
+      run += c;
+    }
+    __syncthreads();
+    return all;
+  }
+  __device__ uint32_t before(const FewFirsts &f, uint32_t i) const {
+    const uint4 flags = f.flags[i >> 4];
+    const u64 lo = (u64)flags.y << 32 | flags.x, hi = (u64)flags.w << 32 | flags.z;
+    const int bits = (int)(i & 7) * 8;
+    const u64 below = (1ull << bits) - 1ull;
+    const bool upper = (i & 8) != 0;
+    return piece[i >> 4] + (uint32_t)__popcll((upper ? hi : lo) & below) + (upper ? (uint32_t)__popcll(lo) : 0u);
+  }
+};
+
 // Point i of the cloud.
+template <typename FIRSTS, typename SUMS>
 __global__ __launch_bounds__(kBlock) void voxAssign(
     const float *__restrict__ points, const float *__restrict__ voxel_size, const float *__restrict__ range, int64_t n,
     int num_features, const uint32_t *__restrict__ state, const uint32_t *__restrict__ first_of,
-    device_sort::FlagRanks firsts, bool quads, int max_points, int max_voxels,
+    FIRSTS firsts, bool quads, int max_points, int max_voxels,
     float *__restrict__ voxels, int32_t *__restrict__ coors, int32_t *__restrict__ num_points_per_voxel,
     int32_t *__restrict__ voxel_num, u64 *host_voxel_num, u64 stamp) {
-  __shared__ device_sort::FlagSums s_sums;
+  __shared__ SUMS s_sums;
   const int tid = threadIdx.x;
   const int64_t i = (int64_t)blockIdx.x * kBlock + tid;
   const uint32_t st = i < n ? state[i] : 0u;
@@ -398,6 +611,12 @@ __global__ __launch_bounds__(kBlock) void voxAssign(
 struct Workspace {
   u64 *tagged, *grouped, *wide_keys;
   uint32_t *state, *first_of, *counters, *bucket_start, *wide_counts, *wide_firsts;
+  // few points: cleared with `state`, in front of which they lie
+  uint8_t *first_flags;
+  uint32_t *cursor;
+  uint32_t *cleared;
+  size_t clear_words;
+  uint8_t *tags;
   device_sort::FlagRanks firsts;
   size_t total;
 };
@@ -419,7 +638,14 @@ Workspace carve(void *base, const VoxelizeShape &s) {
   Workspace w;
   w.tagged = longs(n);
   w.grouped = longs(n);
-  w.state = words(n);
+  const bool few = s.num_points <= kFewPoints;
+  const size_t flag_words = few ? (n + 15) / 16 * 4 : 0;
+  w.clear_words = flag_words + (few ? 1 : 0) + n;
+  w.cleared = words(w.clear_words);
+  w.first_flags = reinterpret_cast<uint8_t *>(w.cleared);
+  w.state = w.cleared + flag_words;
+  w.cursor = w.state + n;
+  w.tags = reinterpret_cast<uint8_t *>(take(few ? fewTags(s.num_points) : 0));
   w.first_of = words(n);
   w.counters = words(device_sort::counterWords(s.num_points, bucketsFor(s.num_points)));
   w.bucket_start = words(kMaxDigits);
@@ -459,12 +685,36 @@ hipError_t launchVoxelize(const LaunchCtx &lc, const VoxelizeShape &s, const flo
   clear.words[1] = (size_t)s.max_voxels * 3;
   clear.base[2] = reinterpret_cast<uint32_t *>(num_points_per_voxel);
   clear.words[2] = (size_t)s.max_voxels;
-  clear.base[3] = w.state;
-  clear.words[3] = (size_t)n;
+  clear.base[3] = w.cleared;
+  clear.words[3] = w.clear_words;
   size_t most = 0;
   for (int g = 0; g < kClearRegions; ++g) most = clear.words[g] > most ? clear.words[g] : most;
   const size_t clear_blocks = most / (4 * kTileThreads) + 1;
+  const bool quads = s.num_features == 4 &&
+                     ((reinterpret_cast<uintptr_t>(points) | reinterpret_cast<uintptr_t>(voxels)) & 15) == 0;
   hipError_t e;
+  if (n <= kFewPoints) {
+    uint32_t *keys = reinterpret_cast<uint32_t *>(w.tagged);
+    const int tags_end = (int)fewTags(n), point_blocks = gridFor((size_t)tags_end);
+    lc.begin("voxTagPoints");
+    voxTagPoints<<<point_blocks + (int)(clear_blocks < 1024 ? clear_blocks : 1024), kBlock, 0, lc.stream>>>(
+        points, voxel_size, coors_range, (int)n, s.num_features, point_blocks, tags_end, keys, w.tags, clear);
+    lc.end();
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    lc.begin("voxRankFew");
+    voxRankFew<<<kFewBuckets, kFewThreads, 0, lc.stream>>>(
+        points, voxel_size, coors_range, (int)n, s.num_features, (uint32_t)s.max_points, keys, w.tags, w.cursor, w.grouped,
+        w.wide_keys, w.wide_counts, w.wide_firsts, w.state, w.first_of, w.first_flags);
+    lc.end();
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    const FewFirsts firsts = {reinterpret_cast<const uint4 *>(w.first_flags), (int)((n + 15) / 16)};
+    lc.begin("voxAssign");
+    voxAssign<FewFirsts, FewSums><<<gridFor((size_t)n), kBlock, 0, lc.stream>>>(
+        points, voxel_size, coors_range, n, s.num_features, w.state, w.first_of, firsts, quads, s.max_points,
+        s.max_voxels, voxels, coors, num_points_per_voxel, voxel_num, host_voxel_num, stamp);
+    lc.end();
+    return hipGetLastError();
+  }
   lc.begin("voxCountBuckets");
   voxCountBuckets<<<tiles + (int)(clear_blocks < 1024 ? clear_blocks : 1024), kTileThreads, 0, lc.stream>>>(
       points, voxel_size, coors_range, n, s.num_features, buckets, rounds, tiles, w.tagged, hist, clear);
@@ -501,10 +751,8 @@ hipError_t launchVoxelize(const LaunchCtx &lc, const VoxelizeShape &s, const flo
   lc.end();
   if (e != hipSuccess) return e;
 
-  const bool quads = s.num_features == 4 &&
-                     ((reinterpret_cast<uintptr_t>(points) | reinterpret_cast<uintptr_t>(voxels)) & 15) == 0;
   lc.begin("voxAssign");
-  voxAssign<<<gridFor((size_t)n), kBlock, 0, lc.stream>>>(
+  voxAssign<device_sort::FlagRanks, device_sort::FlagSums><<<gridFor((size_t)n), kBlock, 0, lc.stream>>>(
       points, voxel_size, coors_range, n, s.num_features, w.state, w.first_of, w.firsts, quads, s.max_points,
       s.max_voxels, voxels, coors, num_points_per_voxel, voxel_num, host_voxel_num, stamp);
   lc.end();
