@@ -240,6 +240,20 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtSetDistinctPairsPromise(mluOpHandle_t handle
   return MLUOP_STATUS_SUCCESS;
 }
 
+mluOpStatus_t MLUOP_WIN_API mluOpExtSetSinglePairsPromise(mluOpHandle_t handle, int column) {
+  PARAM_CHECK("[mluOpExtSetSinglePairsPromise]", handle != NULL);
+  PARAM_CHECK("[mluOpExtSetSinglePairsPromise]", column >= -1 && column <= 1);
+  handle->single_pairs_column = column;
+  return MLUOP_STATUS_SUCCESS;
+}
+
+mluOpStatus_t MLUOP_WIN_API mluOpExtGetSinglePairsPromise(mluOpHandle_t handle, int *column) {
+  PARAM_CHECK("[mluOpExtGetSinglePairsPromise]", handle != NULL);
+  PARAM_CHECK("[mluOpExtGetSinglePairsPromise]", column != NULL);
+  *column = handle->single_pairs_column;
+  return MLUOP_STATUS_SUCCESS;
+}
+
 mluOpStatus_t MLUOP_WIN_API mluOpExtGetKernelTimingCount(mluOpHandle_t handle, int *count) {
   PARAM_CHECK("[mluOpExtGetKernelTimingCount]", handle != NULL);
   PARAM_CHECK("[mluOpExtGetKernelTimingCount]", count != NULL);

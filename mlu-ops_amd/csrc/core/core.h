@@ -43,6 +43,9 @@ struct mluOpContext {
   // (mluOpExtSetDistinctPairsPromise): forward and backward data then skip the
   // check that finds and adds such pairs.
   bool distinct_pairs_promised = false;
+  // The pair column of which the caller promised that it names every row once, over all offsets together; -1: neither
+  // (mluOpExtSetSinglePairsPromise).
+  int single_pairs_column = -1;
   // rulebooks set the pair slots behind each offset's pairs to -1 (mluOpExtSetPairTails)
   bool fill_pair_tails = true;
   // forward convolutions store negative results as zero (mluOpExtSetForwardRelu)

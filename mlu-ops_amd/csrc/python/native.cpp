@@ -59,6 +59,8 @@ namespace {
   X(mluOpDynamicPointToVoxelBackward)                      \
   X(mluOpExtSetSparseConvExtendedModes)                    \
   X(mluOpExtSetDistinctPairsPromise)                       \
+  X(mluOpExtSetSinglePairsPromise)                         \
+  X(mluOpExtGetSinglePairsPromise)                         \
   X(mluOpExtSetPairTails)                                  \
   X(mluOpExtGetPairTails)                                  \
   X(mluOpExtSetForwardRelu)                                \
@@ -475,6 +477,7 @@ struct LayerRulebook : torch::CustomClassHolder {
   Counts counts, filter_space;
   int64_t num_act_out = 0;
   bool sub_m = false, distinct = false;
+  bool single = false;  // every input row is in one pair at most
 
   ~LayerRulebook() override {
     for (const auto &[key, map] : row_maps_)
@@ -545,6 +548,8 @@ struct IndiceConv : torch::autograd::Function<IndiceConv> {
     const void *map = share_row_maps ? rb->rowMap(h, buffers, inverse ? 0 : 1) : nullptr;
     // an inverse layer runs the partner layer's rulebook backwards: one output row per input
     // row of the partner
+    const Setting single(h.handle, api.mluOpExtGetSinglePairsPromise, api.mluOpExtSetSinglePairsPromise, rb->single ? 0 : -1,
+                         "mluOpExtSetSinglePairsPromise");
     const Setting stored(h.handle, api.mluOpExtGetForwardRelu, api.mluOpExtSetForwardRelu, relu, "mluOpExtSetForwardRelu");
     const at::Tensor out = inverse ? convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts,
                                                  rb->pairs.size(2), false, 1, map)
@@ -573,6 +578,8 @@ struct IndiceConv : torch::autograd::Function<IndiceConv> {
     check(api.mluOpExtSetDistinctPairsPromise(h.handle, rb->distinct), "mluOpExtSetDistinctPairsPromise");
     const Buffers buffers(ctx->saved_data["guarded"].toBool(), x.device());
     const bool sub_m = !inverse && rb->sub_m;
+    const Setting single(h.handle, api.mluOpExtGetSinglePairsPromise, api.mluOpExtSetSinglePairsPromise, rb->single ? 0 : -1,
+                         "mluOpExtSetSinglePairsPromise");
     if (ctx->needs_input_grad(0)) {
       const void *map =
           ctx->saved_data["share_row_maps"].toBool() ? rb->rowMap(h, buffers, inverse ? 1 : 0) : nullptr;
@@ -834,7 +841,7 @@ PYBIND11_MODULE(_native, m) {
 
   py::class_<LayerRulebook, LayerRulebookPtr>(m, "LayerRulebook")
       .def(py::init([](const at::Tensor &pairs, Counts counts, int64_t num_act_out, Counts filter_space, bool sub_m,
-                       bool distinct) {
+                       bool distinct, bool single) {
         auto rb = c10::make_intrusive<LayerRulebook>();
         rb->pairs = pairs;
         rb->counts = std::move(counts);
@@ -842,8 +849,11 @@ PYBIND11_MODULE(_native, m) {
         rb->filter_space = std::move(filter_space);
         rb->sub_m = sub_m;
         rb->distinct = distinct;
+        rb->single = single;
         return rb;
-      }))
+      }),
+           py::arg("pairs"), py::arg("counts"), py::arg("num_act_out"), py::arg("filter_space"), py::arg("sub_m"),
+           py::arg("distinct"), py::arg("single") = false)
       .def("row_maps", &LayerRulebook::rowMaps, "(handle, pair column) of the row maps its calls have built.");
   m.def("indice_conv", [](const at::Tensor &features, const at::Tensor &weight, const LayerRulebookPtr &rulebook,
                           bool inverse, bool share_row_maps, bool guarded, bool relu) {

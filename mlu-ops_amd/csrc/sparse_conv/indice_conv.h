@@ -49,6 +49,8 @@ struct ConvProblem {
   bool inverse = false;
   // The caller promised that no offset names a result row twice: no check for lost pairs.
   bool distinct_pairs = false;
+  // The caller promised that no result row is in two pairs, over all offsets together.
+  bool single_pairs = false;
   // Forward: negative results are stored as zero.
   bool relu = false;
   // Forward and backward data: the [K, rows] row map of exactly this rulebook and direction,

@@ -403,9 +403,18 @@ __device__ __forceinline__ void padRows(const PadRows &pad) {
   }
 }
 
+// `elems` words set to `value` by 16-byte stores from a 16-byte boundary on.
+__device__ __forceinline__ void fillWords(int32_t *words, size_t elems, int32_t value, int block, int blocks) {
+  const size_t quads = elems / 4;
+  int4 *dst = reinterpret_cast<int4 *>(words);
+  for (size_t i = (size_t)block * 256 + threadIdx.x; i < quads; i += (size_t)blocks * 256)
+    dst[i] = make_int4(value, value, value, value);
+  if (block == 0 && threadIdx.x < (elems & 3)) words[quads * 4 + threadIdx.x] = value;
+}
+
 // One launch for the independent preparations of the MFMA path on a row map: the first pad.blocks
-// workgroups copy the gathered rows to padded ones, the next fill_blocks set the row map to -1
-// (16-byte stores), the others repack the filter.
+// workgroups copy the gathered rows to padded ones, the next fill_blocks set the row map to -1, the others
+// repack the filter.
 template <typename E>
 __global__ __launch_bounds__(256) void fillMapPackFilter(PadRows pad, int32_t *map, size_t map_elems,
                                                          int fill_blocks,
@@ -421,11 +430,29 @@ __global__ __launch_bounds__(256) void fillMapPackFilter(PadRows pad, int32_t *m
   }
   const int block = (int)blockIdx.x - pad.blocks;
   if (block < fill_blocks) {
-    const size_t quads = map_elems / 4;
-    int4 *dst = reinterpret_cast<int4 *>(map);
-    for (size_t i = (size_t)block * 256 + threadIdx.x; i < quads; i += (size_t)fill_blocks * 256)
-      dst[i] = make_int4(-1, -1, -1, -1);
-    if (block == 0 && threadIdx.x < (map_elems & 3)) map[quads * 4 + threadIdx.x] = -1;
+    fillWords(map, map_elems, -1, block, fill_blocks);
+    return;
+  }
+  packFilter<E>(W, sK, sQ, sC, K, shape, packed, ticket, block - fill_blocks,
+                (int)gridDim.x - pad.blocks - fill_blocks);
+}
+
+// The same in front of gatherConvSingle: fill_blocks workgroups set the result of `elems` elements to zero, where some
+// of its rows are in no pair.
+template <typename E>
+__global__ __launch_bounds__(256) void clearResultPackFilter(PadRows pad, typename E::storage *result, size_t elems,
+                                                             int fill_blocks, const typename E::storage *W, int64_t sK,
+                                                             int64_t sQ, int64_t sC, int K, FilterShape shape,
+                                                             typename E::storage *packed, unsigned long long ticket) {
+  if ((int)blockIdx.x < pad.blocks) {
+    padRows<typename E::storage>(pad);
+    return;
+  }
+  const int block = (int)blockIdx.x - pad.blocks;
+  if (block < fill_blocks) {
+    constexpr int kPerWord = 4 / (int)sizeof(typename E::storage);
+    fillWords(reinterpret_cast<int32_t *>(result), elems / kPerWord, 0, block, fill_blocks);
+    if (elems % kPerWord != 0 && block == 0 && threadIdx.x == 0) result[elems - 1] = typename E::storage(0);
     return;
   }
   packFilter<E>(W, sK, sQ, sC, K, shape, packed, ticket, block - fill_blocks,
@@ -2313,6 +2340,118 @@ void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRo
   if constexpr (!SRC::kSegments) storeDenseSlots(s_map, slots, source.filled);
 }
 
+// ---- result rows in one pair each -------------------------------------------------------
+//
+// Where no result row is in two pairs (the input rows of a 2x2x2 layer with stride 2, for its input's gradient and for
+// the inverse layer) there is nothing to add up: a workgroup multiplies `singlePairs` pairs of ONE offset, whatever
+// rows they belong to, and stores the products.  Its blocks are full, its filter is one, and it needs no sums in
+// LDS and no cut table.  The waves split columns and rows as in the dense kernel above; rows go straight into LDS.
+// What bounds it is the chain of three dependent loads (pairs, rows, results) of workgroups that live for 5 us, and
+// memory.  us of the gather kernel alone, 2x2x2 stride 2, the list kernels / this one: fp32 96 -> 64 of 200 000 rows
+// 76/39, bf16 128 -> 96 of 100 000 31/16, fp16 128 -> 64 of 150 000 24/15, 64 -> 64 of 100 000 15/10, 32 -> 16 9.8/5.8.
+constexpr int singlePairs(int row_bytes) { return row_bytes >= 512 ? 64 : 128; }
+constexpr int singlePieceAt(int row_bytes, int row, int piece) {
+  if (row_bytes >= 256) return piece ^ (row & 15);
+  if (row_bytes == 128) return piece ^ (row >> 1 & 7);
+  const int r = row >> 2 & 3;  // 0 2 3 1: the 16 rows whose pieces are read together meet all banks
+  return piece ^ (r << 1 & 2) ^ (r >> 1 & 1) * 3;
+}
+
+template <typename E, int Q, int C>
+__global__ __launch_bounds__(kDenseThreads) void gatherConvSingle(
+    const typename E::storage *A, uint32_t a_size, ConvRows conv, const typename E::storage *packedW,
+    const int32_t *__restrict__ pairs, int L, int row_col, int src_col, OffsetCounts counts, OffsetBlocks blocks, int K,
+    int R, int n_src, typename E::storage *result) {
+  typedef typename E::vec8 vec8;
+  typedef typename E::storage S;
+  constexpr int WAVES = kDenseThreads / 64;
+  constexpr int RB = Q * (int)sizeof(S) < 64 ? 64 : Q * (int)sizeof(S);
+  constexpr int T = singlePairs(RB);
+  constexpr int CW = stagedPlan((int)sizeof(S), Q, C).column_waves, NB = stagedPlan((int)sizeof(S), Q, C).column_blocks;
+  constexpr int GROUPS = T / 16;
+  constexpr int G = GROUPS / (WAVES / CW);
+  constexpr int KB = RB / 64;
+  constexpr int PPR = RB / 16;
+  constexpr int RPL = 1024 / RB;  // rows a load of 1 KiB stages
+  constexpr int LPG = 16 / RPL;
+  __shared__ __attribute__((aligned(1024))) char s_rows[T * RB];
+  __shared__ uint32_t s_src[T];  // where a pair's gathered row begins, or kNoRow
+  __shared__ int s_row[T];       // its result row, or -1
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int pair = lane & 15, quad = lane >> 4;
+  int lo = 0, hi = K - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (blocks.first[mid] <= (int)blockIdx.x) lo = mid; else hi = mid - 1;
+  }
+  const int k = lo, p0 = ((int)blockIdx.x - blocks.first[k]) * T;
+  if (tid < T) {
+    int row = -1, src = 0;
+    if (p0 + tid < counts.n[k]) {
+      const int32_t *const list = pairs + (size_t)k * 2 * L + p0 + tid;
+      row = list[(size_t)row_col * L];
+      src = list[(size_t)src_col * L];
+    }
+    const bool there = (unsigned)row < (unsigned)R && (unsigned)src < (unsigned)n_src;
+    s_src[tid] = there ? (uint32_t)src * (uint32_t)conv.row_bytes : kNoRow;
+    s_row[tid] = there ? row : -1;
+  }
+  const int first_group = wave / CW * G, first_block = wave % CW * NB;
+  const char *const filter =
+      reinterpret_cast<const char *>(packedW) + (size_t)(k * (C / 16) + first_block) * KB * 1024 + lane * 16;
+  vec8 w[NB][KB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) w[nb][kb] = *reinterpret_cast<const vec8 *>(filter + (nb * KB + kb) * 1024);
+  ldsBarrier();
+  const u32x4 rows_words = {(uint32_t)reinterpret_cast<uintptr_t>(A), (uint32_t)(reinterpret_cast<uintptr_t>(A) >> 32),
+                            a_size, 0x00020000u};
+  const uint32_t rows_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)s_rows;
+#pragma unroll
+  for (int t = 0; t < GROUPS / WAVES; ++t) {
+    uint32_t at[LPG];
+#pragma unroll
+    for (int j = 0; j < LPG; ++j) {
+      const int row = (wave + t * WAVES) * 16 + j * RPL + lane / PPR;
+      // (the swizzle is its own inverse)
+      const uint32_t piece = (uint32_t)singlePieceAt(RB, row & 15, lane % PPR) * 16u;
+      at[j] = __builtin_elementwise_add_sat(s_src[row], piece < (uint32_t)conv.row_bytes ? piece : kNoRow);
+    }
+#pragma unroll
+    for (int j = 0; j < LPG; ++j) asm volatile("" : "+v"(at[j]));
+#pragma unroll
+    for (int j = 0; j < LPG; ++j)
+      requestRowsToLds(rows_words, at[j], rows_lds + (uint32_t)(((wave + t * WAVES) * LPG + j) * 1024));
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  ldsBarrier();
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int in_tile = (first_group + g) * 16 + pair;
+    const char *const rows = s_rows + in_tile * RB;
+    vec8 row[KB];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+      row[kb] = *reinterpret_cast<const vec8 *>(rows + singlePieceAt(RB, pair, kb * 4 + quad) * 16);
+    const int to = s_row[in_tile];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      float4v product = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) product = E::mfma(w[nb][kb], row[kb], product);
+      if (to < 0) continue;
+      // (a sum that starts from zero, as in the other kernels: a product of -0 is stored as 0)
+      S tmp[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) E::store(&tmp[e], activated(0.f + product[e], conv.relu));
+      storeColumns<E>(result + (size_t)to * conv.c, (first_block + nb) * 16 + quad * 4, conv.c, tmp);
+    }
+  }
+}
+
 // ---- pairs that lost their map slot -----------------------------------------------
 // Runs behind every gather kernel and returns at once when the kernels found as many
 // filled map slots as there are pairs inside their tensors (always, for a rulebook built
@@ -3726,6 +3865,46 @@ void launchDense(const LaunchCtx &lc, int q_padded, const void *A, int n_src, co
 #undef DENSE_INSTANCE
 }
 
+template <typename E, int Q, int C>
+void launchSingleInstance(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d, const OffsetCounts &inl,
+                          const void *A, const ConvRows &rows, const void *packed, void *result) {
+  constexpr int RB = Q * (int)sizeof(typename E::storage) < 64 ? 64 : Q * (int)sizeof(typename E::storage);
+  OffsetBlocks ob;
+  int blocks = 0;
+  for (int k = 0; k < kMaxInlineK; ++k) {
+    ob.first[k] = blocks;
+    if (k < p.K) blocks += (inl.n[k] + singlePairs(RB) - 1) / singlePairs(RB);
+  }
+  if (blocks == 0) return;
+  lc.begin("gatherConvSingle");
+  gatherConvSingle<E, Q, C><<<blocks, kDenseThreads, 0, lc.stream>>>(
+      static_cast<const typename E::storage *>(A), (uint32_t)d.n_src * (uint32_t)rows.row_bytes, rows,
+      static_cast<const typename E::storage *>(packed), p.indice_pairs, p.L, d.row_col, d.src_col, inl, ob, p.K, d.R,
+      d.n_src, static_cast<typename E::storage *>(result));
+  lc.end();
+}
+
+template <typename E>
+void launchSingle(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d, const OffsetCounts &inl, const void *A,
+                  const ConvRows &rows, const void *packed, void *result) {
+#define SINGLE_INSTANCE(q, c) launchSingleInstance<E, q, c>(lc, p, d, inl, A, rows, packed, result)
+#define SINGLE_BY_C(q)                       \
+  switch (d.c_padded) {                      \
+    case 16: SINGLE_INSTANCE(q, 16); break;  \
+    case 32: SINGLE_INSTANCE(q, 32); break;  \
+    case 64: SINGLE_INSTANCE(q, 64); break;  \
+    default: SINGLE_INSTANCE(q, 128); break; \
+  }
+  switch (d.q_padded) {
+    case 16: SINGLE_BY_C(16) break;
+    case 32: SINGLE_BY_C(32) break;
+    case 64: SINGLE_BY_C(64) break;
+    default: SINGLE_BY_C(128) break;
+  }
+#undef SINGLE_BY_C
+#undef SINGLE_INSTANCE
+}
+
 // Row maps are built on the flat grid from this many workgroups of the per-offset grid on.
 constexpr int kFlatScatterFromBlocks = 16384;
 
@@ -3787,6 +3966,20 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
   const PadRows pad = {static_cast<const char *>(gathered), static_cast<char *>(ws.padded_rows), d.Q * (int)sizeof(S),
                        rows_of.row_bytes, pad_rows ? d.n_src : 0, pad_rows ? gridFor((size_t)d.n_src, 1024) : 0};
   const size_t frags = (size_t)p.K * groups * chunks * 64;
+  if (p.single_pairs && use_mfma && p.row_map == nullptr && p.K <= kMaxInlineK &&
+      (uint64_t)d.n_src * (uint64_t)rows_of.row_bytes < (uint64_t)kNoRow) {
+    int64_t pairs = 0;
+    for (int k = 0; k < p.K; ++k) pairs += inl.n[k];
+    const size_t elems = pairs < d.R ? (size_t)d.R * d.C : 0;  // to be cleared: some rows are in no pair
+    const int fill_blocks = elems > 0 ? gridFor(elems * sizeof(S) / 16 + 1, 2048) : 0;
+    lc.begin("clearResultPackFilter");
+    clearResultPackFilter<E><<<pad.blocks + fill_blocks + gridFor(frags, 512), 256, 0, lc.stream>>>(
+        pad, static_cast<S *>(result), elems, fill_blocks, static_cast<const S *>(f.base), f.stride_k, sQ, sC, p.K, shape,
+        static_cast<S *>(ws.packed), p.ticket);
+    lc.end();
+    launchSingle<E>(lc, p, d, inl, rows_from, rows_of, ws.packed, result);
+    return;
+  }
   const bool single_chunk = p.row_map == nullptr && ws.map_rows >= d.R && lc.choices.small_map_chunks != 1;
   // Pair lists whose order nobody has reported yet: the call starts on them all the same,
   // and the row-map kernels are enqueued behind, each of them told to return at once unless

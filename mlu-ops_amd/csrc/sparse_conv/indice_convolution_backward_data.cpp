@@ -299,6 +299,7 @@ mluOpStatus_t MLUOP_WIN_API mluOpIndiceConvolutionBackwardData(
   ConvProblem p = makeProblem(output_grad_desc, filters_desc, indice_pairs_desc, input_grad_desc,
                               indice_num, inverse, indice_pairs);
   p.distinct_pairs = handle->distinct_pairs_promised;
+  p.single_pairs = handle->single_pairs_column == (p.inverse ? 1 : 0);
   st = mluop::sparse_conv::takeRowMap(api, handle, announced_map, GatherDirection::kBackwardData, &p);
   if (st != MLUOP_STATUS_SUCCESS) return st;
   // what this call overwrites is no pair tensor any more, whatever the handle noted there

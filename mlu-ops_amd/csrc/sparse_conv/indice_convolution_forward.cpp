@@ -243,6 +243,7 @@ mluOpStatus_t MLUOP_WIN_API mluOpIndiceConvolutionForward(
                               num_act_out, inverse, indice_pairs);
   p.distinct_pairs = handle->distinct_pairs_promised;
   p.relu = handle->forward_relu;
+  p.single_pairs = handle->single_pairs_column == (p.inverse ? 0 : 1);
   st = mluop::sparse_conv::takeRowMap(api, handle, announced_map, GatherDirection::kForward, &p);
   if (st != MLUOP_STATUS_SUCCESS) return st;
   // what this call overwrites is no pair tensor any more, whatever the handle noted there

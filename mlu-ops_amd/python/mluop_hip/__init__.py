@@ -128,6 +128,8 @@ SIGNATURES = {
     "mluOpExtSetDistinctPairsPromise": (ctypes.c_int, [_vp, ctypes.c_int]),
     "mluOpExtSetPairTails": (ctypes.c_int, [_vp, ctypes.c_int]),
     "mluOpExtGetPairTails": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int)]),
+    "mluOpExtSetSinglePairsPromise": (ctypes.c_int, [_vp, ctypes.c_int]),
+    "mluOpExtGetSinglePairsPromise": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int)]),
     "mluOpExtSetForwardRelu": (ctypes.c_int, [_vp, ctypes.c_int]),
     "mluOpExtGetForwardRelu": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int)]),
     "mluOpExtGetOrderVoxelsWorkspaceSize": (ctypes.c_int, [ctypes.c_int64, _vp, _vp]),
@@ -240,6 +242,10 @@ class Handle:
     def set_forward_relu(self, enable):
         """mluOpExtSetForwardRelu: forward convolutions store negative results as zero."""
         check(lib().mluOpExtSetForwardRelu(self.ptr, 1 if enable else 0))
+
+    def promise_single_pairs(self, column):
+        """mluOpExtSetSinglePairsPromise: this pair column names every row once (None: no promise)."""
+        check(lib().mluOpExtSetSinglePairsPromise(self.ptr, -1 if column is None else column))
 
     def promise_distinct_pairs(self, promised):
         """No offset of the rulebooks names a result row twice: skip the check for lost pairs."""

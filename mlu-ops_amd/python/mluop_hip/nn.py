@@ -53,10 +53,13 @@ class Rulebook:
     asked for), out_indices, num_act_out."""
 
     def __init__(self, pairs, out_indices, indice_num_host, num_act_out, filter_space, sub_m, out_space,
-                 in_indices=None, in_space=None, distinct=False, built_on=None, tails=True):
+                 in_indices=None, in_space=None, distinct=False, built_on=None, tails=True, single=False):
         # the input coordinates were distinct: no offset names a result row twice, and the
         # operators may skip their check for such pairs (mluOpExtSetDistinctPairsPromise)
         self.distinct = distinct
+        # no input row is in two pairs: a kernel that reaches no further than its stride (the gradient of such a
+        # layer's input, and its inverse, multiply full tiles of pairs: mluOpExtSetSinglePairsPromise)
+        self.single = single
         self.in_indices = in_indices  # what an inverse convolution over this rulebook gives back
         self.in_space = None if in_space is None else tuple(in_space)
         self._pairs = pairs
@@ -98,7 +101,8 @@ class Rulebook:
         """What the native operators take of this rulebook; it holds the row maps they share."""
         if self._for_operators is None:
             self._for_operators = native().LayerRulebook(self._pairs, self.indice_num, self.num_act_out,
-                                                         list(self.filter_space), self.sub_m, self.distinct)
+                                                         list(self.filter_space), self.sub_m, self.distinct,
+                                                         self.single)
         return self._for_operators
 
     @property
@@ -188,7 +192,9 @@ class _ConvBase(torch.nn.Module):
             self.stride, self.dilation, self.sub_m, for_layer=True, tails=False, wait_counts=wait_counts)
         rb = Rulebook(pairs, out_indices, num, n_out, self.kernel_size, self.sub_m,
                       out_space, in_indices=x.indices, in_space=x.spatial_shape, distinct=x.distinct,
-                      built_on=handle, tails=False)
+                      built_on=handle, tails=False,
+                      single=not self.sub_m and all((k - 1) * d < s for k, d, s in
+                                                    zip(self.kernel_size, self.dilation, self.stride)))
         if self.indice_key is not None:
             x.rulebooks[self.indice_key] = rb
         else:
