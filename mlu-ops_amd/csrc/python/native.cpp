@@ -14,6 +14,7 @@
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
 
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <optional>
@@ -303,9 +304,11 @@ Rulebook3 indicePairs(mluOpHandle_t handle, const Buffers &buffers, const at::Te
   return r;
 }
 
+// `counts_of`: the pair counts; it may wait for them, and is asked once all that needs none of them is done.
+template <typename COUNTS_OF>
 at::Tensor convForward(mluOpHandle_t handle, const Buffers &buffers, const at::Tensor &features,
                        const at::Tensor &filters, mluOpTensorLayout_t layout, const at::Tensor &pairs,
-                       const Counts &counts, int64_t num_act_out, bool sub_m, int64_t inverse,
+                       COUNTS_OF &&counts_of, int64_t num_act_out, bool sub_m, int64_t inverse,
                        const void *row_map) {
   const mluOpDataType_t code = dtypeCode(features.scalar_type());
   const int64_t co = filters.size(layout == MLUOP_LAYOUT_ARRAY ? 4 : 0);
@@ -315,10 +318,12 @@ at::Tensor convForward(mluOpHandle_t handle, const Buffers &buffers, const at::T
   const TensorDesc d_pairs(MLUOP_LAYOUT_ARRAY, MLUOP_DTYPE_INT32, pairs.sizes());
   const TensorDesc d_out(MLUOP_LAYOUT_ARRAY, code, out.sizes());
   size_t bytes = 0;
-  check(api.mluOpGetIndiceConvolutionForwardWorkspaceSize(handle, d_x, d_w, d_pairs, d_out, counts.data(),
+  // (the workspace is as large for one number of pairs as for another)
+  check(api.mluOpGetIndiceConvolutionForwardWorkspaceSize(handle, d_x, d_w, d_pairs, d_out, Counts(pairs.size(0)).data(),
                                                           num_act_out, inverse, sub_m, &bytes),
         "mluOpGetIndiceConvolutionForwardWorkspaceSize");
   const at::Tensor ws = buffers.workspace(bytes);
+  const Counts &counts = counts_of();
   if (row_map != nullptr) check(api.mluOpExtUseRowMap(handle, row_map), "mluOpExtUseRowMap");
   check(api.mluOpIndiceConvolutionForward(handle, d_x, features.data_ptr(), d_w, filters.data_ptr(), d_pairs,
                                           pairs.data_ptr(), counts.data(), num_act_out, inverse, sub_m,
@@ -474,10 +479,31 @@ class OperatorLock {
 // outputs, 0: its inputs).  They live as long as this object, which a pending backward pass holds.
 struct LayerRulebook : torch::CustomClassHolder {
   at::Tensor pairs;
-  Counts counts, filter_space;
+  Counts filter_space;
   int64_t num_act_out = 0;
   bool sub_m = false, distinct = false;
   bool single = false;  // every input row is in one pair at most
+
+  void setCounts(Counts counts) { counts_ = std::move(counts); }
+  // They are on the device yet, in `indice_num`, and with the handle that built the rulebook.
+  void setCountsPending(const at::Tensor &indice_num, mluOpHandle_t built_on) {
+    indice_num_ = indice_num;
+    built_on_ = built_on;
+    pending_ = true;
+  }
+
+  // The pair counts, waited for on first use: a layer's output, workspace and descriptors are made while the device
+  // builds its rulebook.  `held` is locked; where the rulebook was built on another handle, takeCountsFrom has
+  // been called before that.  (No two handles are ever locked together, and counts_mutex_ only inside one's lock.)
+  const Counts &counts(mluOpHandle_t held) {
+    if (pending_.load(std::memory_order_acquire)) takeCounts(held);
+    return counts_;
+  }
+  void takeCountsFromOther(mluOpHandle_t own) {
+    if (!pending_.load(std::memory_order_acquire) || built_on_ == own) return;
+    const OperatorLock lock(built_on_);
+    takeCounts(built_on_);
+  }
 
   ~LayerRulebook() override {
     for (const auto &[key, map] : row_maps_)
@@ -507,7 +533,7 @@ struct LayerRulebook : torch::CustomClassHolder {
     size_t bytes = 0;
     check(api.mluOpExtGetRowMapSize(d_pairs, rows, &bytes), "mluOpExtGetRowMapSize");
     const at::Tensor map = buffers.output({static_cast<int64_t>(bytes)}, at::kByte, "row map");
-    check(api.mluOpExtBuildRowMap(h.handle, d_pairs, pairs.data_ptr(), counts.data(), rows, source_rows, column,
+    check(api.mluOpExtBuildRowMap(h.handle, d_pairs, pairs.data_ptr(), counts(h.handle).data(), rows, source_rows, column,
                                   map.data_ptr(), bytes, nullptr),
           "mluOpExtBuildRowMap");
     buffers.done("mluOpExtBuildRowMap");
@@ -525,6 +551,27 @@ struct LayerRulebook : torch::CustomClassHolder {
   }
 
  private:
+  void takeCounts(mluOpHandle_t built_on) {
+    const std::lock_guard<std::mutex> lock(counts_mutex_);
+    if (!pending_.load(std::memory_order_relaxed)) return;
+    Counts counts;
+    if (!hostCounts(built_on, pairs, &counts)) {
+      // no longer on file (the handle keeps 32 rulebooks), or too many offsets
+      const c10::DeviceGuard guard(pairs.device());
+      if (hipDeviceSynchronize() != hipSuccess) throw std::runtime_error("waiting for a rulebook's pair counts failed");
+      const at::Tensor host = indice_num_.cpu();
+      const int32_t *n = host.data_ptr<int32_t>();
+      counts.assign(n, n + host.numel());
+    }
+    counts_ = std::move(counts);
+    pending_.store(false, std::memory_order_release);
+  }
+
+  Counts counts_;
+  at::Tensor indice_num_;
+  mluOpHandle_t built_on_ = nullptr;
+  std::atomic<bool> pending_{false};
+  std::mutex counts_mutex_;
   using Key = std::pair<StreamHandle *, int>;
   std::mutex maps_mutex_;  // never held while anything else is waited for
   std::map<Key, at::Tensor> row_maps_;
@@ -542,18 +589,20 @@ struct IndiceConv : torch::autograd::Function<IndiceConv> {
     ctx->saved_data["guarded"] = guarded;
     ctx->saved_data["relu"] = relu;
     StreamHandle &h = streamHandle();
+    rb->takeCountsFromOther(h.handle);
     const OperatorLock lock(h);
     check(api.mluOpExtSetDistinctPairsPromise(h.handle, rb->distinct), "mluOpExtSetDistinctPairsPromise");
     const Buffers buffers(guarded, x.device());
+    const auto counts_of = [&]() -> const Counts & { return rb->counts(h.handle); };
     const void *map = share_row_maps ? rb->rowMap(h, buffers, inverse ? 0 : 1) : nullptr;
     // an inverse layer runs the partner layer's rulebook backwards: one output row per input
     // row of the partner
     const Setting single(h.handle, api.mluOpExtGetSinglePairsPromise, api.mluOpExtSetSinglePairsPromise, rb->single ? 0 : -1,
                          "mluOpExtSetSinglePairsPromise");
     const Setting stored(h.handle, api.mluOpExtGetForwardRelu, api.mluOpExtSetForwardRelu, relu, "mluOpExtSetForwardRelu");
-    const at::Tensor out = inverse ? convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts,
+    const at::Tensor out = inverse ? convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, counts_of,
                                                  rb->pairs.size(2), false, 1, map)
-                                   : convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts,
+                                   : convForward(h.handle, buffers, x, w, MLUOP_LAYOUT_ARRAY, rb->pairs, counts_of,
                                                  rb->num_act_out, rb->sub_m, 0, map);
     if (relu)
       ctx->save_for_backward({x, w, out});
@@ -574,6 +623,7 @@ struct IndiceConv : torch::autograd::Function<IndiceConv> {
     const bool relu = ctx->saved_data["relu"].toBool();
     const at::Tensor dy = (relu ? at::threshold_backward(grads[0], saved[2], 0) : grads[0]).contiguous();
     StreamHandle &h = streamHandle();
+    rb->takeCountsFromOther(h.handle);
     const OperatorLock lock(h);
     check(api.mluOpExtSetDistinctPairsPromise(h.handle, rb->distinct), "mluOpExtSetDistinctPairsPromise");
     const Buffers buffers(ctx->saved_data["guarded"].toBool(), x.device());
@@ -583,12 +633,12 @@ struct IndiceConv : torch::autograd::Function<IndiceConv> {
     if (ctx->needs_input_grad(0)) {
       const void *map =
           ctx->saved_data["share_row_maps"].toBool() ? rb->rowMap(h, buffers, inverse ? 1 : 0) : nullptr;
-      out[0] = convBackwardData(h.handle, buffers, dy, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts, sub_m,
+      out[0] = convBackwardData(h.handle, buffers, dy, w, MLUOP_LAYOUT_ARRAY, rb->pairs, rb->counts(h.handle), sub_m,
                                 x.size(1), inverse, x.size(0), map);
     }
     if (ctx->needs_input_grad(1))
-      out[1] = convBackwardFilter(h.handle, buffers, x, dy, rb->pairs, rb->counts, rb->filter_space, sub_m, inverse,
-                                  true, MLUOP_LAYOUT_ARRAY);
+      out[1] = convBackwardFilter(h.handle, buffers, x, dy, rb->pairs, rb->counts(h.handle), rb->filter_space, sub_m,
+                                  inverse, true, MLUOP_LAYOUT_ARRAY);
     return out;
   }
 };
@@ -773,7 +823,8 @@ PYBIND11_MODULE(_native, m) {
           NoGil released;
           const OperatorLock lock(asHandle(handle));
           return convForward(asHandle(handle), Buffers(guarded, features.device()), features, filters,
-                             static_cast<mluOpTensorLayout_t>(layout), pairs, counts, num_act_out, sub_m, inverse,
+                             static_cast<mluOpTensorLayout_t>(layout), pairs,
+                             [&]() -> const Counts & { return counts; }, num_act_out, sub_m, inverse,
                              reinterpret_cast<const void *>(row_map));
         });
   m.def("indice_conv_backward_data",
@@ -840,11 +891,14 @@ PYBIND11_MODULE(_native, m) {
         });
 
   py::class_<LayerRulebook, LayerRulebookPtr>(m, "LayerRulebook")
-      .def(py::init([](const at::Tensor &pairs, Counts counts, int64_t num_act_out, Counts filter_space, bool sub_m,
-                       bool distinct, bool single) {
+      .def(py::init([](const at::Tensor &pairs, std::optional<Counts> counts, int64_t num_act_out, Counts filter_space,
+                       bool sub_m, bool distinct, bool single, std::optional<at::Tensor> indice_num, uintptr_t built_on) {
         auto rb = c10::make_intrusive<LayerRulebook>();
         rb->pairs = pairs;
-        rb->counts = std::move(counts);
+        if (counts)
+          rb->setCounts(std::move(*counts));
+        else
+          rb->setCountsPending(indice_num.value(), asHandle(built_on));
         rb->num_act_out = num_act_out;
         rb->filter_space = std::move(filter_space);
         rb->sub_m = sub_m;
@@ -853,7 +907,8 @@ PYBIND11_MODULE(_native, m) {
         return rb;
       }),
            py::arg("pairs"), py::arg("counts"), py::arg("num_act_out"), py::arg("filter_space"), py::arg("sub_m"),
-           py::arg("distinct"), py::arg("single") = false)
+           py::arg("distinct"), py::arg("single") = false, py::arg("indice_num") = std::nullopt, py::arg("built_on") = 0,
+           "With counts None, `indice_num` holds them on the device and the handle at `built_on` has built the rulebook.")
       .def("row_maps", &LayerRulebook::rowMaps, "(handle, pair column) of the row maps its calls have built.");
   m.def("indice_conv", [](const at::Tensor &features, const at::Tensor &weight, const LayerRulebookPtr &rulebook,
                           bool inverse, bool share_row_maps, bool guarded, bool relu) {

@@ -1,0 +1,92 @@
+"""Layers take a rulebook's pair counts when they run: when the handle has them on file no longer, on another
+stream than the rulebook's, and from several threads at once."""
+import threading
+
+import numpy as np
+import pytest
+
+from spconv_cases import random_voxels
+
+pytestmark = pytest.mark.gpu
+
+SPACE = (9, 40, 40)
+
+
+def setup(rows, seed=0):
+    import torch
+    from mluop_hip import nn as spnn
+    torch.manual_seed(seed)
+    idx = torch.from_numpy(random_voxels(np.random.default_rng(seed), 1, SPACE, rows)).cuda()
+    layer = spnn.SubMConv3d(8, 16, 3, indice_key="k").cuda()
+    x = spnn.SparseTensor(torch.randn(rows, 8, device="cuda", requires_grad=True), idx, SPACE, 1, distinct=True)
+    waited = spnn.SparseTensor(x.features, idx, SPACE, 1, distinct=True)
+    assert isinstance(layer._rulebook(waited)._indice_num, list)
+    want = layer(waited).features
+    grads = torch.autograd.grad(want.sum(), [x.features, layer.weight])
+    torch.cuda.synchronize()
+    return layer, x, want.detach(), grads
+
+
+def pending(layer, x):
+    import torch
+    rb = layer._rulebook(x, wait_counts=False)
+    assert isinstance(rb._indice_num, torch.Tensor)
+    return rb
+
+
+def check(layer, x, want, grads):
+    import torch
+    y = layer(x).features
+    assert torch.equal(y, want)
+    for g, w in zip(torch.autograd.grad(y.sum(), [x.features, layer.weight]), grads):
+        assert torch.equal(g, w)
+
+
+@pytest.mark.parametrize("rows", [1, 700, 6000])
+@pytest.mark.parametrize("others", [0, 40])
+def test_counts_taken_by_the_operator(rows, others):
+    from mluop_hip import nn as spnn
+    layer, x, want, grads = setup(rows)
+    rb = pending(layer, x)
+    more = [pending(spnn.SubMConv3d(8, 16, 3).cuda(),
+                    spnn.SparseTensor(x.features, x.indices, SPACE, 1, distinct=True)) for _ in range(others)]
+    check(layer, x, want, grads)
+    assert rb.indice_num[13] == rows and all(r.indice_num == rb.indice_num for r in more)
+
+
+def test_on_another_stream():
+    import torch
+    layer, x, want, grads = setup(3000)
+    pending(layer, x)
+    other = torch.cuda.Stream()
+    other.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(other):
+        check(layer, x, want, grads)
+    torch.cuda.current_stream().wait_stream(other)
+
+
+def test_from_several_threads():
+    import torch
+    for seed in range(5):
+        layer, x, want, grads = setup(2500, seed)
+        pending(layer, x)
+        main = torch.cuda.current_stream()
+        streams = [torch.cuda.Stream() for _ in range(3)] + [main]
+        errors = []
+
+        def work(stream):
+            try:
+                with torch.cuda.stream(stream):
+                    if stream is not main:
+                        stream.wait_stream(main)
+                    for _ in range(3):
+                        assert torch.equal(layer(x).features.detach(), want)
+            except Exception as e:  # noqa: BLE001
+                errors.append(e)
+        threads = [threading.Thread(target=work, args=(s,)) for s in streams]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        torch.cuda.synchronize()
+        assert not errors, errors
