@@ -3080,6 +3080,10 @@ __global__ __launch_bounds__(256) void backwardFilterMfma(
 // receives channel j of the four pairs.  Two such reads are one operand fragment.  No
 // element-sized stores, no registers for staging, one barrier per step.
 //
+// A row is asked for by the place where it begins, worked out once when the pair's index is staged: a buffer load answers
+// a pair that is not there with zeros, and a load costs one addition in front of it (a 64-bit address and a choice
+// of a row of zeros were ten operations each, some 80 a step).  us with the sums, 248 636 rows of a scene, before / now:
+// 128 x 128 161/147, 64 x 64 71/67, 32 x 32 58/53 (with the steps unrolled by two 162, 70, 54).
 // A row's 16-byte pieces are stored permuted (piece ^ f(pair)), since rows lie a
 // multiple of the bank width apart: f spreads the eight pairs that half a wavefront
 // reads at once over all 64 banks.  Waves are laid out 2 x 2 over the blocks of dW[k].
@@ -3114,8 +3118,9 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
 
   __shared__ __attribute__((aligned(1024))) char s_x[2][SP * RBX];
   __shared__ __attribute__((aligned(1024))) char s_y[2][SP * RBY];
-  __shared__ int s_in[2][kIndexChunk];   // row indices of a chunk of pairs, and of the chunk after
-  __shared__ int s_out[2][kIndexChunk];
+  // where the rows of a chunk of pairs begin, and of the chunk after; kNoRow: a pair that is not there
+  __shared__ uint32_t s_in[2][kIndexChunk];
+  __shared__ uint32_t s_out[2][kIndexChunk];
 
   const FilterRun run = runOfWorkgroup(tab, order, total_slices, slice_len, shares);
   if (run.k < 0) return;
@@ -3128,7 +3133,12 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
   const int32_t *out_col = pairs + ((size_t)k * 2 + 1 - x_col) * L;
   const uint32_t x_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)&s_x[0][0];
   const uint32_t y_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)&s_y[0][0];
-  const char *zero_row = reinterpret_cast<const char *>(kZeroRow);
+  const uint32_t x_length = (uint32_t)rows.ci * 2u, y_length = (uint32_t)rows.co * 2u;  // bytes; zeros behind them
+  auto words_of = [](const void *base, uint32_t bytes) {
+    return u32x4{(uint32_t)reinterpret_cast<uintptr_t>(base), (uint32_t)(reinterpret_cast<uintptr_t>(base) >> 32), bytes,
+                 0x00020000u};
+  };
+  const u32x4 x_words = words_of(X, (uint32_t)n_in * x_length), y_words = words_of(dY, (uint32_t)n_out * y_length);
 
   float4v acc[AB][BB];
 #pragma unroll
@@ -3138,50 +3148,62 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
 
   // One step's rows into a buffer: wave-load t of an operand covers 1 KiB of the buffer, lane
   // l its bytes [16 l, 16 l + 16), i.e. a fixed (pair, place) of the step.  Wave w issues
-  // loads w, w + 4, ...: `locate` reads all row indices first and forms the addresses (one
-  // LDS latency a step, not one a load), `request` issues load u of the wave's XM + YM.
+  // loads w, w + 4, ...; all places are read first (one LDS latency a step, not one a load).
   constexpr int XM = (XN + 3) / 4, YM = (YN + 3) / 4;
-  struct StepLoads {
-    const char *from[XM + YM];
-  };
-  // (live == false: a step that is not there; every lane then reads the row of zeros, so
-  // that the requests need no branch around them)
-  auto locate = [&](int step, bool live, StepLoads &loads) {
-    const int *in = s_in[(step / kChunkSteps) & 1] + (step % kChunkSteps) * SP;
-    const int *out = s_out[(step / kChunkSteps) & 1] + (step % kChunkSteps) * SP;
-    int row[XM + YM];
+  uint32_t x_piece[XM], y_piece[YM];  // the piece of its row that a lane asks for, by load
 #pragma unroll
-    for (int u = 0; u < XM; ++u) row[u] = in[((wave + u * 4) * 1024 + lane * 16) / RBX];
+  for (int u = 0; u < XM; ++u) {
+    const int byte = (wave + u * 4) * 1024 + lane * 16;
+    x_piece[u] = (uint32_t)(((byte % RBX) / 16) ^ filterRowSwizzle(RBX, byte / RBX)) * 16u;
+    if (x_piece[u] >= x_length) x_piece[u] = kNoRow;
+  }
 #pragma unroll
-    for (int u = 0; u < YM; ++u) row[XM + u] = out[((wave + u * 4) * 1024 + lane * 16) / RBY];
+  for (int u = 0; u < YM; ++u) {
+    const int byte = (wave + u * 4) * 1024 + lane * 16;
+    y_piece[u] = (uint32_t)(((byte % RBY) / 16) ^ filterRowSwizzle(RBY, byte / RBY)) * 16u;
+    if (y_piece[u] >= y_length) y_piece[u] = kNoRow;
+  }
+  auto request_step = [&](int step, int buffer) {
+    const uint32_t *in = s_in[(step / kChunkSteps) & 1] + (step % kChunkSteps) * SP;
+    const uint32_t *out = s_out[(step / kChunkSteps) & 1] + (step % kChunkSteps) * SP;
+    uint32_t at_x[XM], at_y[YM];
 #pragma unroll
-    for (int u = 0; u < XM + YM; ++u) {
-      const bool is_x = u < XM;
-      const int row_bytes = is_x ? RBX : RBY;
-      const int byte = (wave + (is_x ? u : u - XM) * 4) * 1024 + lane * 16;
-      const int piece = ((byte % row_bytes) / 16) ^ filterRowSwizzle(row_bytes, byte / row_bytes);
-      const char *from = reinterpret_cast<const char *>(is_x ? (const void *)X : (const void *)dY);
-      const int length = (is_x ? rows.ci : rows.co) * 2;  // bytes; zeros behind them
-      loads.from[u] =
-          (live && row[u] >= 0 && piece * 16 < length ? from + (size_t)row[u] * length : zero_row) + piece * 16;
+    for (int u = 0; u < XM; ++u) at_x[u] = in[((wave + u * 4) * 1024 + lane * 16) / RBX % SP];
+#pragma unroll
+    for (int u = 0; u < YM; ++u) at_y[u] = out[((wave + u * 4) * 1024 + lane * 16) / RBY % SP];
+#pragma unroll
+    for (int u = 0; u < XM; ++u) {
+      at_x[u] = __builtin_elementwise_add_sat(at_x[u], x_piece[u]);
+      asm volatile("" : "+v"(at_x[u]));
     }
-  };
-  auto request = [&](const StepLoads &loads, int u, int buffer) {
-    if (u < XM) {
-      const int t = wave + u * 4;
-      if (XN % 4 == 0 || t < XN) requestToLds(loads.from[u], x_lds + buffer * (SP * RBX) + t * 1024);
-    } else if (u < XM + YM) {
-      const int t = wave + (u - XM) * 4;
-      if (YN % 4 == 0 || t < YN) requestToLds(loads.from[u], y_lds + buffer * (SP * RBY) + t * 1024);
+#pragma unroll
+    for (int u = 0; u < YM; ++u) {
+      at_y[u] = __builtin_elementwise_add_sat(at_y[u], y_piece[u]);
+      asm volatile("" : "+v"(at_y[u]));
     }
+#pragma unroll
+    for (int u = 0; u < XM; ++u)
+      if (XN % 4 == 0 || wave + u * 4 < XN)
+        requestRowsToLds(x_words, at_x[u], x_lds + (uint32_t)(buffer * (SP * RBX) + (wave + u * 4) * 1024));
+#pragma unroll
+    for (int u = 0; u < YM; ++u)
+      if (YN % 4 == 0 || wave + u * 4 < YN)
+        requestRowsToLds(y_words, at_y[u], y_lds + (uint32_t)(buffer * (SP * RBY) + (wave + u * 4) * 1024));
   };
-  // fragment of block `block` (16 channels) for the 32 pairs from `pair0` on: lane (c, kq)
-  // receives pairs pair0 + 8 kq + (0..7) of channel 16 block + c
+  // fragment of block `block` (16 channels) for 32 pairs: lane (c, kq) receives the pairs 8 kq + (0..7) of channel
+  // 16 block + c
   const int sub = lane & 15, kq = lane >> 4;
-  auto fragment = [&](const char *buffer, int row_bytes, int block, int pair0) -> vec8 {
-    const int pair = pair0 + 8 * kq + (sub >> 2);  // the four pairs after it have the same swizzle
+  auto fragment_place = [&](int row_bytes, int block) -> int {
+    const int pair = 8 * kq + (sub >> 2);  // the four pairs after it, and those 32 on, have the same swizzle
     const int place = (block * 2 + ((sub & 3) >> 1)) ^ filterRowSwizzle(row_bytes, pair);
-    const char *at = buffer + pair * row_bytes + place * 16 + (sub & 1) * 8;
+    return pair * row_bytes + place * 16 + (sub & 1) * 8;
+  };
+  const char *x_frag[AB], *y_frag[BB];  // in the first buffer
+#pragma unroll
+  for (int a = 0; a < AB; ++a) x_frag[a] = &s_x[0][0] + fragment_place(RBX, wa * AB + a);
+#pragma unroll
+  for (int b = 0; b < BB; ++b) y_frag[b] = &s_y[0][0] + fragment_place(RBY, wb * BB + b);
+  auto fragment = [&](const char *at, int row_bytes) -> vec8 {
     const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
         (__attribute__((address_space(3))) v4i16 *)(at));
     const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
@@ -3211,8 +3233,8 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
     for (int u = 0; u < IPT; ++u) {
       int i = idx_in[u], o = idx_out[u];
       if ((unsigned)i >= (unsigned)n_in || (unsigned)o >= (unsigned)n_out) i = o = -1;
-      s_in[chunk & 1][u * 256 + tid] = i;
-      s_out[chunk & 1][u * 256 + tid] = o;
+      s_in[chunk & 1][u * 256 + tid] = i < 0 ? kNoRow : (uint32_t)i * x_length;
+      s_out[chunk & 1][u * 256 + tid] = o < 0 ? kNoRow : (uint32_t)o * y_length;
     }
   };
 
@@ -3220,10 +3242,7 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
   fetch_indices(0);
   store_indices(0);
   __syncthreads();
-  StepLoads next_rows;
-  locate(0, true, next_rows);
-#pragma unroll
-  for (int u = 0; u < XM + YM; ++u) request(next_rows, u, 0);
+  request_step(0, 0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   ldsBarrier();
   for (int step = 0; step < steps; ++step) {
@@ -3233,24 +3252,23 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
     // in LDS one barrier before the chunk's last step asks for the next chunk's first rows
     const bool chunk_follows = (chunk + 1) * kChunkSteps < steps;
     if (in_chunk == 0 && chunk_follows) fetch_indices(chunk + 1);
-    const bool ahead = step + 1 < steps;
-    locate(ahead ? step + 1 : step, ahead, next_rows);
-    const char *bx = s_x[cur], *by = s_y[cur];
-    // (all requests first: they have one step's multiplies to land)
-#pragma unroll
-    for (int u = 0; u < XM + YM; ++u) request(next_rows, u, cur ^ 1);
+    // (all requests first: they have one step's multiplies to land; the other workgroups' requests wait for these
+    // multiplies)
+    if (step + 1 < steps) request_step(step + 1, cur ^ 1);
+    __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int kb = 0; kb < SP / 32; ++kb) {
       vec8 bfr[BB];
 #pragma unroll
-      for (int b = 0; b < BB; ++b) bfr[b] = fragment(by, RBY, wb * BB + b, kb * 32);
+      for (int b = 0; b < BB; ++b) bfr[b] = fragment(y_frag[b] + cur * (SP * RBY) + kb * 32 * RBY, RBY);
 #pragma unroll
       for (int a = 0; a < AB; ++a) {
-        const vec8 afr = fragment(bx, RBX, wa * AB + a, kb * 32);
+        const vec8 afr = fragment(x_frag[a] + cur * (SP * RBX) + kb * 32 * RBX, RBX);
 #pragma unroll
         for (int b = 0; b < BB; ++b) acc[a][b] = E::mfma(afr, bfr[b], acc[a][b]);
       }
     }
+    __builtin_amdgcn_s_setprio(0);
     if (in_chunk == kChunkSteps - 2 && chunk_follows) store_indices(chunk + 1);
     // the next step's rows have landed, and every wave has left this step's buffers
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -4176,8 +4194,11 @@ GradLayout gradLayout(const ConvProblem &p) {
 
 // Rows whose operands the backward filter can transpose with LDS reads.
 bool transposingReads(const LaunchCtx &lc, const ConvProblem &p) {
+  // (rows are addressed with 32-bit byte offsets)
+  const uint64_t x_bytes = (uint64_t)(p.inverse ? p.num_out : p.L) * (uint64_t)p.Ci * 2;
+  const uint64_t y_bytes = (uint64_t)(p.inverse ? p.L : p.num_out) * (uint64_t)p.Co * 2;
   return p.dtype != ElemType::kFloat && p.Ci > 16 && p.Co > 16 && lc.choices.filter_stores != 1 &&
-         !rowsNeedPadding(p.dtype, p.Ci) && !rowsNeedPadding(p.dtype, p.Co);
+         !rowsNeedPadding(p.dtype, p.Ci) && !rowsNeedPadding(p.dtype, p.Co) && x_bytes < kNoRow && y_bytes < kNoRow;
 }
 
 // Workgroups of the walks (walkOfWorkgroup), 0: slices.  As many as are resident at a time, so that all
