@@ -3286,6 +3286,217 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaTr(
             acc[a][b][v];
 }
 
+// The same for fp32, where an operand is one element a lane and needs no transposition: rows as they are in LDS, four-byte
+// reads.  The pairs of a multiply are those of backwardFilterMfma (4 kq + s of 16 pairs), whose bits it gives.  The four
+// rows a multiply reads at once have to meet all banks: a row's 64-byte chunks are permuted by bits 2 and 3 of its
+// pair, and of rows of 128 bytes every second four stand in each other's places.  A wave's blocks of 16 channels are every
+// second one, so that the two waves of a side share those that a row has; the multiplies of blocks that it does not have
+// are left out (all operands are read in front of them: a branch between reads and multiplies made small layers slower).
+// Bound by the multiplies from 96 channels on (128 x 128: 223 us of them at the 144 TFLOP/s this instruction reaches) and by
+// a step's round trip below.  us with the sums, 100 000-row scene, 0.98 M pairs, backwardFilterMfma / this:
+//   32 x 32  53/41   48 x 48  137/66   64 x 64  141/92   68 x 36  247/106   64 x 96  260/133   96 x 96  377/211
+//   32 x 128  190/106   128 x 128  362/300          and 3 000 rows, 20 000 pairs: 32 x 32  22/18   96 x 96  108/71
+constexpr int floatRowChunk(int row_bytes, int pair) { return row_bytes >= 256 ? pair >> 2 & 3 : pair >> 3 & 1; }
+constexpr int floatRowSlot(int row_bytes, int pair) { return row_bytes >= 256 ? pair : pair ^ (pair >> 2 & 1); }
+// Where the row of pair 4 kq + q lies behind that of pair 4 kq.
+__device__ __forceinline__ int floatStepPlace(int row_bytes, int q, int kq) {
+  return row_bytes >= 256 ? q * row_bytes : (floatRowSlot(row_bytes, 4 * kq + q) - floatRowSlot(row_bytes, 4 * kq)) * row_bytes;
+}
+
+template <int CI, int CO, bool WHOLE>
+__global__ __launch_bounds__(256) void backwardFilterMfmaRows(
+    const float *X, const float *dY, FilterGradRows lengths, const int32_t *pairs, int L,
+    int x_col, int n_in, int n_out, int K, SliceTable tab, SliceOrder order, int total_slices,
+    int slice_len, int shares, float *partial) {
+  constexpr int SP = 32;
+  static_assert(CI % 32 == 0 && CO % 32 == 0 && CI <= 128 && CO <= 128, "two row and column blocks per wave pair");
+  constexpr int kIndexChunk = kFilterWalkChunk;
+  const FilterGradRows rows = WHOLE ? FilterGradRows{CI, CO} : lengths;
+  constexpr int kChunkSteps = kIndexChunk / SP;
+  constexpr int RBX = CI * 4, RBY = CO * 4;     // bytes per row
+  constexpr int XN = SP * RBX / 1024;           // 1 KiB wave-loads per step
+  constexpr int YN = SP * RBY / 1024;
+  constexpr int AB = CI / 32, BB = CO / 32;     // 16-row / 16-column blocks per wave
+
+  __shared__ __attribute__((aligned(1024))) char s_x[2][SP * RBX];
+  __shared__ __attribute__((aligned(1024))) char s_y[2][SP * RBY];
+  // where the rows of a chunk of pairs begin, and of the chunk after; kNoRow: a pair that is not there
+  __shared__ uint32_t s_in[2][kIndexChunk];
+  __shared__ uint32_t s_out[2][kIndexChunk];
+
+  const FilterRun run = runOfWorkgroup(tab, order, total_slices, slice_len, shares);
+  if (run.k < 0) return;
+  const int k = run.k;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wa = wave >> 1, wb = wave & 1;
+  const int32_t *in_col = pairs + ((size_t)k * 2 + x_col) * L;
+  const int32_t *out_col = pairs + ((size_t)k * 2 + 1 - x_col) * L;
+  const uint32_t x_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)&s_x[0][0];
+  const uint32_t y_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)&s_y[0][0];
+  const uint32_t x_length = (uint32_t)rows.ci * 4u, y_length = (uint32_t)rows.co * 4u;  // bytes; zeros behind them
+  auto words_of = [](const void *base, uint32_t bytes) {
+    return u32x4{(uint32_t)reinterpret_cast<uintptr_t>(base), (uint32_t)(reinterpret_cast<uintptr_t>(base) >> 32), bytes,
+                 0x00020000u};
+  };
+  const u32x4 x_words = words_of(X, (uint32_t)n_in * x_length), y_words = words_of(dY, (uint32_t)n_out * y_length);
+
+  // blocks of 16 channels that the rows have, of this wave's (every second one: a wave has no more than the other)
+  const int blocks_a = WHOLE ? AB : ((rows.ci + 15) / 16 - wa + 1) / 2;
+  const int blocks_b = WHOLE ? BB : ((rows.co + 15) / 16 - wb + 1) / 2;
+  float4v acc[AB][BB];
+#pragma unroll
+  for (int a = 0; a < AB; ++a)
+#pragma unroll
+    for (int b = 0; b < BB; ++b) acc[a][b] = float4v{0.f, 0.f, 0.f, 0.f};
+
+  // One step's rows into a buffer: wave-load t of an operand covers 1 KiB of the buffer, lane
+  // l its bytes [16 l, 16 l + 16), i.e. a fixed (pair, place) of the step.  Wave w issues
+  // loads w, w + 4, ...; all places are read first (one LDS latency a step, not one a load).
+  constexpr int XM = (XN + 3) / 4, YM = (YN + 3) / 4;
+  uint32_t x_piece[XM], y_piece[YM];  // the piece of its row that a lane asks for, by load
+#pragma unroll
+  for (int u = 0; u < XM; ++u) {
+    const int byte = (wave + u * 4) * 1024 + lane * 16;
+    x_piece[u] = (uint32_t)((byte % RBX / 16) ^ floatRowChunk(RBX, floatRowSlot(RBX, byte / RBX % SP)) * 4) * 16u;
+    if (x_piece[u] >= x_length) x_piece[u] = kNoRow;
+  }
+#pragma unroll
+  for (int u = 0; u < YM; ++u) {
+    const int byte = (wave + u * 4) * 1024 + lane * 16;
+    y_piece[u] = (uint32_t)((byte % RBY / 16) ^ floatRowChunk(RBY, floatRowSlot(RBY, byte / RBY % SP)) * 4) * 16u;
+    if (y_piece[u] >= y_length) y_piece[u] = kNoRow;
+  }
+  auto request_step = [&](int step, int buffer) {
+    const uint32_t *in = s_in[(step / kChunkSteps) & 1] + (step % kChunkSteps) * SP;
+    const uint32_t *out = s_out[(step / kChunkSteps) & 1] + (step % kChunkSteps) * SP;
+    uint32_t at_x[XM], at_y[YM];
+#pragma unroll
+    for (int u = 0; u < XM; ++u) at_x[u] = in[floatRowSlot(RBX, ((wave + u * 4) * 1024 + lane * 16) / RBX % SP)];
+#pragma unroll
+    for (int u = 0; u < YM; ++u) at_y[u] = out[floatRowSlot(RBY, ((wave + u * 4) * 1024 + lane * 16) / RBY % SP)];
+#pragma unroll
+    for (int u = 0; u < XM; ++u) {
+      at_x[u] = __builtin_elementwise_add_sat(at_x[u], x_piece[u]);
+      asm volatile("" : "+v"(at_x[u]));
+    }
+#pragma unroll
+    for (int u = 0; u < YM; ++u) {
+      at_y[u] = __builtin_elementwise_add_sat(at_y[u], y_piece[u]);
+      asm volatile("" : "+v"(at_y[u]));
+    }
+#pragma unroll
+    for (int u = 0; u < XM; ++u)
+      if (XN % 4 == 0 || wave + u * 4 < XN)
+        requestRowsToLds(x_words, at_x[u], x_lds + (uint32_t)(buffer * (SP * RBX) + (wave + u * 4) * 1024));
+#pragma unroll
+    for (int u = 0; u < YM; ++u)
+      if (YN % 4 == 0 || wave + u * 4 < YN)
+        requestRowsToLds(y_words, at_y[u], y_lds + (uint32_t)(buffer * (SP * RBY) + (wave + u * 4) * 1024));
+  };
+  // Element of lane (c, kq) for MFMA step s of 16 pairs: channel 16 block + c of pair 4 kq + s.  (Slots and chunks are
+  // permuted by bits 2 and 3 of the pair: the same for all s and for the next 16 pairs.)
+  const int sub = lane & 15, kq = lane >> 4;
+  auto place_of = [&](int row_bytes, int block) -> int {
+    return (floatRowSlot(row_bytes, 4 * kq) - 4 * kq) * row_bytes + 4 * kq * row_bytes +
+           (block ^ floatRowChunk(row_bytes, 4 * kq)) * 64 + sub * 4;
+  };
+  const char *x_frag[AB], *y_frag[BB];  // in the first buffer
+#pragma unroll
+  for (int a = 0; a < AB; ++a) x_frag[a] = &s_x[0][0] + place_of(RBX, wa + 2 * a);
+#pragma unroll
+  for (int b = 0; b < BB; ++b) y_frag[b] = &s_y[0][0] + place_of(RBY, wb + 2 * b);
+
+  // Row indices of chunk c: four pairs a thread, checked; -1 marks a pair that is not there.
+  constexpr int IPT = kIndexChunk / 256;
+  int idx_in[IPT], idx_out[IPT];
+  auto fetch_indices = [&](int chunk) {
+#pragma unroll
+    for (int u = 0; u < IPT; ++u) {
+      const int at = run.at(chunk * kIndexChunk + u * 256 + tid);
+      int i = -1, o = -1;
+      if (at < run.end) {
+        i = in_col[at];
+        o = out_col[at];
+      }
+      idx_in[u] = i;
+      idx_out[u] = o;
+    }
+  };
+  auto store_indices = [&](int chunk) {
+#pragma unroll
+    for (int u = 0; u < IPT; ++u) {
+      int i = idx_in[u], o = idx_out[u];
+      if ((unsigned)i >= (unsigned)n_in || (unsigned)o >= (unsigned)n_out) i = o = -1;
+      s_in[chunk & 1][u * 256 + tid] = i < 0 ? kNoRow : (uint32_t)i * x_length;
+      s_out[chunk & 1][u * 256 + tid] = o < 0 ? kNoRow : (uint32_t)o * y_length;
+    }
+  };
+
+  const int steps = run.length / SP;
+  fetch_indices(0);
+  store_indices(0);
+  __syncthreads();
+  request_step(0, 0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  ldsBarrier();
+  for (int step = 0; step < steps; ++step) {
+    const int cur = step & 1;
+    const int in_chunk = step % kChunkSteps, chunk = step / kChunkSteps;
+    // the chunk after this one: its indices are requested at the chunk's first step and are
+    // in LDS one barrier before the chunk's last step asks for the next chunk's first rows
+    const bool chunk_follows = (chunk + 1) * kChunkSteps < steps;
+    if (in_chunk == 0 && chunk_follows) fetch_indices(chunk + 1);
+    // (all requests first: they have one step's multiplies to land; the other workgroups' requests wait for these
+    // multiplies)
+    if (step + 1 < steps) request_step(step + 1, cur ^ 1);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int kb = 0; kb < SP / 16; ++kb) {
+      // (slot of pair 4 kq + q: with short rows bit 0 is flipped for half of the lanes)
+      const int x_at = cur * (SP * RBX) + kb * 16 * RBX, y_at = cur * (SP * RBY) + kb * 16 * RBY;
+      float xs[4][AB], ys[4][BB];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+#pragma unroll
+        for (int a = 0; a < AB; ++a)
+          xs[q][a] = *reinterpret_cast<const float *>(x_frag[a] + x_at + floatStepPlace(RBX, q, kq));
+#pragma unroll
+        for (int b = 0; b < BB; ++b)
+          ys[q][b] = *reinterpret_cast<const float *>(y_frag[b] + y_at + floatStepPlace(RBY, q, kq));
+      }
+      // (a row's missing blocks are zeros in LDS; their multiplies are left out)
+#pragma unroll
+      for (int a = 0; a < AB; ++a) {
+        if (a >= blocks_a) break;
+#pragma unroll
+        for (int b = 0; b < BB; ++b) {
+          if (b >= blocks_b) break;
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(xs[q][a], ys[q][b], acc[a][b], 0, 0, 0);
+        }
+      }
+    }
+    __builtin_amdgcn_s_setprio(0);
+    if (in_chunk == kChunkSteps - 2 && chunk_follows) store_indices(chunk + 1);
+    // the next step's rows have landed, and every wave has left this step's buffers
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    ldsBarrier();
+  }
+  // lane holds rows 4*(lane/16)+v, column lane%16 of every 16 x 16 block
+  float *const sums = partial + (size_t)run.tile * CI * CO;
+#pragma unroll
+  for (int a = 0; a < AB; ++a)
+#pragma unroll
+    for (int b = 0; b < BB; ++b)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        sums[(size_t)((wa + 2 * a) * 16 + 4 * (lane >> 4) + v) * CO + (wb + 2 * b) * 16 + (lane & 15)] =
+            acc[a][b][v];
+}
+
 // dW[k] = sum of the offset's partial tiles, rounded once.  A block adds 256
 // consecutive elements (four per lane): wave g of 16 takes the slices g, g+16, ...
 // in eight independent running sums, the sums are combined pairwise in a fixed
@@ -4192,13 +4403,14 @@ GradLayout gradLayout(const ConvProblem &p) {
   return g;
 }
 
-// Rows whose operands the backward filter can transpose with LDS reads.
+// Rows that the backward filter reads into LDS as they are: 2-byte operands are transposed by LDS reads, fp32 ones need
+// no transposition.
 bool transposingReads(const LaunchCtx &lc, const ConvProblem &p) {
   // (rows are addressed with 32-bit byte offsets)
-  const uint64_t x_bytes = (uint64_t)(p.inverse ? p.num_out : p.L) * (uint64_t)p.Ci * 2;
-  const uint64_t y_bytes = (uint64_t)(p.inverse ? p.L : p.num_out) * (uint64_t)p.Co * 2;
-  return p.dtype != ElemType::kFloat && p.Ci > 16 && p.Co > 16 && lc.choices.filter_stores != 1 &&
-         !rowsNeedPadding(p.dtype, p.Ci) && !rowsNeedPadding(p.dtype, p.Co) && x_bytes < kNoRow && y_bytes < kNoRow;
+  const uint64_t x_bytes = (uint64_t)(p.inverse ? p.num_out : p.L) * (uint64_t)p.Ci * elemSize(p.dtype);
+  const uint64_t y_bytes = (uint64_t)(p.inverse ? p.L : p.num_out) * (uint64_t)p.Co * elemSize(p.dtype);
+  return p.Ci > 16 && p.Co > 16 && lc.choices.filter_stores != 1 && !rowsNeedPadding(p.dtype, p.Ci) &&
+         !rowsNeedPadding(p.dtype, p.Co) && x_bytes < kNoRow && y_bytes < kNoRow;
 }
 
 // Workgroups of the walks (walkOfWorkgroup), 0: slices.  As many as are resident at a time, so that all
@@ -4225,11 +4437,11 @@ void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const S
                               const SliceOrder &order, int slice_len, int shares, int total_slices, float *partial,
                               const void *features, const void *output_grad, void *filters_grad) {
   typedef typename E::storage S;
-  constexpr bool kTransposingShape = sizeof(S) == 2 && CI >= 32 && CO >= 32;
+  constexpr bool kTransposingShape = CI >= 32 && CO >= 32;
   const bool transposing = kTransposingShape && transposingReads(lc, p);
   const FilterGradRows rows = {p.Ci, p.Co};
   const int grid = shares > 0 ? shares * total_slices : (total_slices + 7) / 8 * 8;
-  lc.begin(transposing ? "backwardFilterMfmaTr" : "backwardFilterMfma");
+  lc.begin(!transposing ? "backwardFilterMfma" : (sizeof(S) == 4 ? "backwardFilterMfmaRows" : "backwardFilterMfmaTr"));
   if (total_slices > 0) {
     const bool whole = p.Ci == CI && p.Co == CO;
     auto kernel = backwardFilterMfma<E, CI, CO, false>;
@@ -4241,9 +4453,14 @@ void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const S
       // share a CU then, which pays when the slices are long (network 64 x 64: 101 -> 88 us;
       // on slices of a few steps the shorter steps only add barriers: config 4 23.7 -> 25.3 us).
       const bool short_steps = CI + CO < 256 && slice_len >= 2048;
-      auto tr = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32, false> : backwardFilterMfmaTr<E, CI, CO, 64, false>;
-      if (whole)
-        tr = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32, true> : backwardFilterMfmaTr<E, CI, CO, 64, true>;
+      auto tr = kernel;
+      if constexpr (sizeof(S) == 4) {
+        tr = whole ? backwardFilterMfmaRows<CI, CO, true> : backwardFilterMfmaRows<CI, CO, false>;
+      } else {
+        tr = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32, false> : backwardFilterMfmaTr<E, CI, CO, 64, false>;
+        if (whole)
+          tr = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32, true> : backwardFilterMfmaTr<E, CI, CO, 64, true>;
+      }
       if (transposing)
         tr<<<grid, 256, 0, lc.stream>>>(
             static_cast<const S *>(features), static_cast<const S *>(output_grad), rows, p.indice_pairs, p.L,
