@@ -4533,10 +4533,18 @@ void launchFilterMfma(const LaunchCtx &lc, const ConvProblem &p, const FilterGra
       max_slices = kFilterMaxSlicesManyOffsets;
     int slice_len = (int)((total + max_slices - 1) / max_slices);
     slice_len = (slice_len + kFilterStepPairs - 1) / kFilterStepPairs * kFilterStepPairs;
-    // A slice has fixed costs (the first rows' round trip, a Ci x Co fp32 tile written and summed
-    // again): few pairs are not cut finer than this, at the price of idle CUs (config 5b, 128 x
-    // 128, 400 000 pairs: 56 -> 46 us at 1024; config 2, 32 x 32, 205 000 pairs: 22.5 -> 19 us at 512).
-    const int least = paddedChannels(p.Ci) * paddedChannels(p.Co) >= 128 * 128 ? 1024 : 512;
+    // A slice has fixed costs (the first rows' round trip, a Ci x Co fp32 tile written and summed again), and a slice's
+    // steps follow each other: few pairs are cut into about 192 slices and no finer than 256 pairs, nor, however many
+    // the pairs are, finer than 1024 at 128 x 128 channels and 512 below, at the price of idle CUs.  fp32, whose
+    // multiplies take eight times as long, is cut to 256 at once.  us with the sums, slices of 256 / 512 / 1024 pairs:
+    //   fp16  128 x 128   20 000 pairs 22/24/29   91 000 32/29/31   277 000 41/42/37      64 x 64  20 000 14/15/18   91 000 17/16/18
+    //   fp32  128 x 128   20 000 pairs 37/53/88   91 000 58/60/91   277 000 122/131/151   64 x 64  20 000 18/24/35   91 000 25/32/36
+    const int most = paddedChannels(p.Ci) * paddedChannels(p.Co) >= 128 * 128 ? 1024 : 512;
+    int least = 256;
+    if (p.dtype != ElemType::kFloat) {
+      const int spread = (int)((total + 191) / 192 < most ? (total + 191) / 192 : most);
+      least = spread < 256 ? 256 : (spread + kFilterStepPairs - 1) / kFilterStepPairs * kFilterStepPairs;
+    }
     if (slice_len < least) slice_len = least;
     // Walks instead of slices, and the workgroups an offset's share of its list is walked by: one each,
     // the others to the offsets whose walks are longest.
