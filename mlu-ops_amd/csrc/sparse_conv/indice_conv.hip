@@ -2133,6 +2133,12 @@ __device__ __forceinline__ void requestRowsToLds(u32x4 rows, uint32_t offset, ui
                :: "s"(lds_address), "v"(offset), "s"(rows) : "memory", "m0");
 }
 
+// The same with 4 bytes per lane.
+__device__ __forceinline__ void requestWordsToLds(u32x4 words, uint32_t offset, uint32_t lds_address) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+               :: "s"(lds_address), "v"(offset), "s"(words) : "memory", "m0");
+}
+
 template <typename E, int Q, int C, typename SRC>
 __global__ __launch_bounds__(kDenseThreads) __attribute__((amdgpu_waves_per_eu(kStagedPerCu, kStagedPerCu)))
 void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRows conv,
@@ -3070,23 +3076,21 @@ __global__ __launch_bounds__(256) void backwardFilterMfma(
   }
 }
 
-// The same product for 2-byte elements, 17 to 128 channels on both sides and rows of whole
-// 16-byte pieces (an LDS request takes one), with the
-// transposition done by the LDS read itself.  The gathered rows go from global memory
-// straight into LDS as they are ([pair][channel], 16 bytes per lane, a pair without a
-// valid row reads a row of zeros), one step of 64 (or 32) pairs ahead into the other of two
-// buffers, and `ds_read_b64_tr_b16` hands a lane four consecutive pairs of one channel:
-// within 16 lanes, lane i supplies the address of 4 channels of pair i / 4 and lane j
-// receives channel j of the four pairs.  Two such reads are one operand fragment.  No
-// element-sized stores, no registers for staging, one barrier per step.
+// The same product for 17 to 128 channels on both sides and rows of whole 16-byte pieces (an LDS request takes one).  The
+// gathered rows go from global memory straight into LDS as they are ([pair][channel], 16 bytes per lane), one step of SP
+// pairs ahead into the other of two buffers.  No registers for staging, one barrier per step.  (Bound by what a step
+// takes besides its multiplies, not by memory's latency: three, four or five buffers with as many steps under way gave the
+// same times or, where fewer workgroups fit a CU, longer ones.)
 //
 // A row is asked for by the place where it begins, worked out once when the pair's index is staged: a buffer load answers
-// a pair that is not there with zeros, and a load costs one addition in front of it (a 64-bit address and a choice
-// of a row of zeros were ten operations each, some 80 a step).  us with the sums, 248 636 rows of a scene, before / now:
-// 128 x 128 161/147, 64 x 64 71/67, 32 x 32 58/53 (with the steps unrolled by two 162, 70, 54).
-// A row's 16-byte pieces are stored permuted (piece ^ f(pair)), since rows lie a
-// multiple of the bank width apart: f spreads the eight pairs that half a wavefront
-// reads at once over all 64 banks.  Waves are laid out 2 x 2 over the blocks of dW[k].
+// a pair that is not there with zeros, and a load costs one addition in front of it (with a 64-bit address and a choice
+// of a row of zeros, ten operations each, 128 x 128 channels of a 248 636-row scene took 161 us with the sums and not 147).
+//
+// 2-byte elements are transposed by the LDS read itself: `ds_read_b64_tr_b16` hands a lane four consecutive pairs of one
+// channel; within 16 lanes, lane i supplies the address of 4 channels of pair i / 4 and lane j receives channel j of the
+// four pairs.  Two such reads are one operand fragment.  A row's 16-byte pieces are stored permuted (piece ^ f(pair)),
+// since rows lie a multiple of the bank width apart: f spreads the eight pairs that half a wavefront reads at once over
+// all 64 banks.
 constexpr int filterRowSwizzle(int row_bytes, int pair) {
   return row_bytes == 256 ? (((pair & 1) << 1) | ((pair & 2) << 1) | (pair & 8))
        : row_bytes == 128 ? ((pair & 2) | ((pair & 8) >> 1))
@@ -3094,204 +3098,10 @@ constexpr int filterRowSwizzle(int row_bytes, int pair) {
                           : 0;
 }
 
-template <typename E, int CI, int CO, int SP, bool WHOLE>
-__global__ __launch_bounds__(256) void backwardFilterMfmaTr(
-    const typename E::storage *X, const typename E::storage *dY, FilterGradRows lengths, const int32_t *pairs, int L,
-    int x_col, int n_in, int n_out, int K, SliceTable tab, SliceOrder order, int total_slices,
-    int slice_len, int shares, float *partial) {
-  typedef typename E::vec8 vec8;
-  typedef typename E::storage S;
-  typedef short v4i16 __attribute__((ext_vector_type(4)));
-  typedef short v8i16 __attribute__((ext_vector_type(8)));
-  static_assert(sizeof(S) == 2 && E::kChunk == 32, "2-byte elements, 32 pairs per fragment");
-  static_assert(CI % 32 == 0 && CO % 32 == 0 && CI <= 128 && CO <= 128, "two row and column blocks per wave pair");
-  // two chunks of row indices: with 128 channels on both sides the buffers leave 16 KiB of
-  // half a CU's LDS
-  constexpr int kIndexChunk = kFilterWalkChunk;
-  const FilterGradRows rows = WHOLE ? FilterGradRows{CI, CO} : lengths;
-  constexpr int kChunkSteps = kIndexChunk / SP;
-  constexpr int RBX = CI * 2, RBY = CO * 2;     // bytes per row
-  constexpr int XN = SP * RBX / 1024;           // 1 KiB wave-loads per step
-  constexpr int YN = SP * RBY / 1024;
-  constexpr int AB = CI / 32, BB = CO / 32;     // 16-row / 16-column blocks per wave
-  static_assert(SP == 32 || SP == 64, "one or two fragments per step");
-
-  __shared__ __attribute__((aligned(1024))) char s_x[2][SP * RBX];
-  __shared__ __attribute__((aligned(1024))) char s_y[2][SP * RBY];
-  // where the rows of a chunk of pairs begin, and of the chunk after; kNoRow: a pair that is not there
-  __shared__ uint32_t s_in[2][kIndexChunk];
-  __shared__ uint32_t s_out[2][kIndexChunk];
-
-  const FilterRun run = runOfWorkgroup(tab, order, total_slices, slice_len, shares);
-  if (run.k < 0) return;
-  const int k = run.k;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wa = wave >> 1, wb = wave & 1;
-  const int32_t *in_col = pairs + ((size_t)k * 2 + x_col) * L;
-  const int32_t *out_col = pairs + ((size_t)k * 2 + 1 - x_col) * L;
-  const uint32_t x_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)&s_x[0][0];
-  const uint32_t y_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)&s_y[0][0];
-  const uint32_t x_length = (uint32_t)rows.ci * 2u, y_length = (uint32_t)rows.co * 2u;  // bytes; zeros behind them
-  auto words_of = [](const void *base, uint32_t bytes) {
-    return u32x4{(uint32_t)reinterpret_cast<uintptr_t>(base), (uint32_t)(reinterpret_cast<uintptr_t>(base) >> 32), bytes,
-                 0x00020000u};
-  };
-  const u32x4 x_words = words_of(X, (uint32_t)n_in * x_length), y_words = words_of(dY, (uint32_t)n_out * y_length);
-
-  float4v acc[AB][BB];
-#pragma unroll
-  for (int a = 0; a < AB; ++a)
-#pragma unroll
-    for (int b = 0; b < BB; ++b) acc[a][b] = float4v{0.f, 0.f, 0.f, 0.f};
-
-  // One step's rows into a buffer: wave-load t of an operand covers 1 KiB of the buffer, lane
-  // l its bytes [16 l, 16 l + 16), i.e. a fixed (pair, place) of the step.  Wave w issues
-  // loads w, w + 4, ...; all places are read first (one LDS latency a step, not one a load).
-  constexpr int XM = (XN + 3) / 4, YM = (YN + 3) / 4;
-  uint32_t x_piece[XM], y_piece[YM];  // the piece of its row that a lane asks for, by load
-#pragma unroll
-  for (int u = 0; u < XM; ++u) {
-    const int byte = (wave + u * 4) * 1024 + lane * 16;
-    x_piece[u] = (uint32_t)(((byte % RBX) / 16) ^ filterRowSwizzle(RBX, byte / RBX)) * 16u;
-    if (x_piece[u] >= x_length) x_piece[u] = kNoRow;
-  }
-#pragma unroll
-  for (int u = 0; u < YM; ++u) {
-    const int byte = (wave + u * 4) * 1024 + lane * 16;
-    y_piece[u] = (uint32_t)(((byte % RBY) / 16) ^ filterRowSwizzle(RBY, byte / RBY)) * 16u;
-    if (y_piece[u] >= y_length) y_piece[u] = kNoRow;
-  }
-  auto request_step = [&](int step, int buffer) {
-    const uint32_t *in = s_in[(step / kChunkSteps) & 1] + (step % kChunkSteps) * SP;
-    const uint32_t *out = s_out[(step / kChunkSteps) & 1] + (step % kChunkSteps) * SP;
-    uint32_t at_x[XM], at_y[YM];
-#pragma unroll
-    for (int u = 0; u < XM; ++u) at_x[u] = in[((wave + u * 4) * 1024 + lane * 16) / RBX % SP];
-#pragma unroll
-    for (int u = 0; u < YM; ++u) at_y[u] = out[((wave + u * 4) * 1024 + lane * 16) / RBY % SP];
-#pragma unroll
-    for (int u = 0; u < XM; ++u) {
-      at_x[u] = __builtin_elementwise_add_sat(at_x[u], x_piece[u]);
-      asm volatile("" : "+v"(at_x[u]));
-    }
-#pragma unroll
-    for (int u = 0; u < YM; ++u) {
-      at_y[u] = __builtin_elementwise_add_sat(at_y[u], y_piece[u]);
-      asm volatile("" : "+v"(at_y[u]));
-    }
-#pragma unroll
-    for (int u = 0; u < XM; ++u)
-      if (XN % 4 == 0 || wave + u * 4 < XN)
-        requestRowsToLds(x_words, at_x[u], x_lds + (uint32_t)(buffer * (SP * RBX) + (wave + u * 4) * 1024));
-#pragma unroll
-    for (int u = 0; u < YM; ++u)
-      if (YN % 4 == 0 || wave + u * 4 < YN)
-        requestRowsToLds(y_words, at_y[u], y_lds + (uint32_t)(buffer * (SP * RBY) + (wave + u * 4) * 1024));
-  };
-  // fragment of block `block` (16 channels) for 32 pairs: lane (c, kq) receives the pairs 8 kq + (0..7) of channel
-  // 16 block + c
-  const int sub = lane & 15, kq = lane >> 4;
-  auto fragment_place = [&](int row_bytes, int block) -> int {
-    const int pair = 8 * kq + (sub >> 2);  // the four pairs after it, and those 32 on, have the same swizzle
-    const int place = (block * 2 + ((sub & 3) >> 1)) ^ filterRowSwizzle(row_bytes, pair);
-    return pair * row_bytes + place * 16 + (sub & 1) * 8;
-  };
-  const char *x_frag[AB], *y_frag[BB];  // in the first buffer
-#pragma unroll
-  for (int a = 0; a < AB; ++a) x_frag[a] = &s_x[0][0] + fragment_place(RBX, wa * AB + a);
-#pragma unroll
-  for (int b = 0; b < BB; ++b) y_frag[b] = &s_y[0][0] + fragment_place(RBY, wb * BB + b);
-  auto fragment = [&](const char *at, int row_bytes) -> vec8 {
-    const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (__attribute__((address_space(3))) v4i16 *)(at));
-    const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (__attribute__((address_space(3))) v4i16 *)(at + 4 * row_bytes));
-    const v8i16 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-    return __builtin_bit_cast(vec8, both);
-  };
-
-  // Row indices of chunk c: four pairs a thread, checked; -1 marks a pair that is not there.
-  constexpr int IPT = kIndexChunk / 256;
-  int idx_in[IPT], idx_out[IPT];
-  auto fetch_indices = [&](int chunk) {
-#pragma unroll
-    for (int u = 0; u < IPT; ++u) {
-      const int at = run.at(chunk * kIndexChunk + u * 256 + tid);
-      int i = -1, o = -1;
-      if (at < run.end) {
-        i = in_col[at];
-        o = out_col[at];
-      }
-      idx_in[u] = i;
-      idx_out[u] = o;
-    }
-  };
-  auto store_indices = [&](int chunk) {
-#pragma unroll
-    for (int u = 0; u < IPT; ++u) {
-      int i = idx_in[u], o = idx_out[u];
-      if ((unsigned)i >= (unsigned)n_in || (unsigned)o >= (unsigned)n_out) i = o = -1;
-      s_in[chunk & 1][u * 256 + tid] = i < 0 ? kNoRow : (uint32_t)i * x_length;
-      s_out[chunk & 1][u * 256 + tid] = o < 0 ? kNoRow : (uint32_t)o * y_length;
-    }
-  };
-
-  const int steps = run.length / SP;
-  fetch_indices(0);
-  store_indices(0);
-  __syncthreads();
-  request_step(0, 0);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  ldsBarrier();
-  for (int step = 0; step < steps; ++step) {
-    const int cur = step & 1;
-    const int in_chunk = step % kChunkSteps, chunk = step / kChunkSteps;
-    // the chunk after this one: its indices are requested at the chunk's first step and are
-    // in LDS one barrier before the chunk's last step asks for the next chunk's first rows
-    const bool chunk_follows = (chunk + 1) * kChunkSteps < steps;
-    if (in_chunk == 0 && chunk_follows) fetch_indices(chunk + 1);
-    // (all requests first: they have one step's multiplies to land; the other workgroups' requests wait for these
-    // multiplies)
-    if (step + 1 < steps) request_step(step + 1, cur ^ 1);
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int kb = 0; kb < SP / 32; ++kb) {
-      vec8 bfr[BB];
-#pragma unroll
-      for (int b = 0; b < BB; ++b) bfr[b] = fragment(y_frag[b] + cur * (SP * RBY) + kb * 32 * RBY, RBY);
-#pragma unroll
-      for (int a = 0; a < AB; ++a) {
-        const vec8 afr = fragment(x_frag[a] + cur * (SP * RBX) + kb * 32 * RBX, RBX);
-#pragma unroll
-        for (int b = 0; b < BB; ++b) acc[a][b] = E::mfma(afr, bfr[b], acc[a][b]);
-      }
-    }
-    __builtin_amdgcn_s_setprio(0);
-    if (in_chunk == kChunkSteps - 2 && chunk_follows) store_indices(chunk + 1);
-    // the next step's rows have landed, and every wave has left this step's buffers
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    ldsBarrier();
-  }
-  // lane holds rows 4*(lane/16)+v, column lane%16 of every 16 x 16 block
-  float *const sums = partial + (size_t)run.tile * CI * CO;
-#pragma unroll
-  for (int a = 0; a < AB; ++a)
-#pragma unroll
-    for (int b = 0; b < BB; ++b)
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        sums[(size_t)((wa * AB + a) * 16 + 4 * (lane >> 4) + v) * CO + (wb * BB + b) * 16 + (lane & 15)] =
-            acc[a][b][v];
-}
-
-// The same for fp32, where an operand is one element a lane and needs no transposition: rows as they are in LDS, four-byte
-// reads.  The pairs of a multiply are those of backwardFilterMfma (4 kq + s of 16 pairs), whose bits it gives.  The four
-// rows a multiply reads at once have to meet all banks: a row's 64-byte chunks are permuted by bits 2 and 3 of its
-// pair, and of rows of 128 bytes every second four stand in each other's places.  A wave's blocks of 16 channels are every
-// second one, so that the two waves of a side share those that a row has; the multiplies of blocks that it does not have
-// are left out (all operands are read in front of them: a branch between reads and multiplies made small layers slower).
+// An fp32 operand is one element a lane and needs no transposition: four-byte reads.  The pairs of a multiply are those of
+// backwardFilterMfma (4 kq + s of 16 pairs), whose bits it gives.  The four rows a multiply reads at once have to meet
+// all banks: a row's 64-byte chunks are permuted by bits 2 and 3 of its pair, and of rows of 128 bytes every second
+// four stand in each other's places.
 // Bound by the multiplies from 96 channels on (128 x 128: 223 us of them at the 144 TFLOP/s this instruction reaches) and by
 // a step's round trip below.  us with the sums, 100 000-row scene, 0.98 M pairs, backwardFilterMfma / this:
 //   32 x 32  53/41   48 x 48  137/66   64 x 64  141/92   68 x 36  247/106   64 x 96  260/133   96 x 96  377/211
@@ -3303,26 +3113,34 @@ __device__ __forceinline__ int floatStepPlace(int row_bytes, int q, int kq) {
   return row_bytes >= 256 ? q * row_bytes : (floatRowSlot(row_bytes, 4 * kq + q) - floatRowSlot(row_bytes, 4 * kq)) * row_bytes;
 }
 
-template <int CI, int CO, bool WHOLE>
-__global__ __launch_bounds__(256) void backwardFilterMfmaRows(
-    const float *X, const float *dY, FilterGradRows lengths, const int32_t *pairs, int L,
+// Waves are laid out 2 x 2 over the blocks of dW[k], each with every second block of a side, so that the two waves of a
+// side share the blocks that a row has.
+template <typename E, int CI, int CO, int SP, bool WHOLE>
+__global__ __launch_bounds__(256) void backwardFilterRows(
+    const typename E::storage *X, const typename E::storage *dY, FilterGradRows lengths, const int32_t *pairs, int L,
     int x_col, int n_in, int n_out, int K, SliceTable tab, SliceOrder order, int total_slices,
     int slice_len, int shares, float *partial) {
-  constexpr int SP = 32;
+  typedef typename E::vec8 vec8;
+  typedef short v4i16 __attribute__((ext_vector_type(4)));
+  typedef short v8i16 __attribute__((ext_vector_type(8)));
+  constexpr int kSize = (int)sizeof(typename E::storage);
+  constexpr bool kFloat = kSize == 4;
   static_assert(CI % 32 == 0 && CO % 32 == 0 && CI <= 128 && CO <= 128, "two row and column blocks per wave pair");
-  constexpr int kIndexChunk = kFilterWalkChunk;
-  const FilterGradRows rows = WHOLE ? FilterGradRows{CI, CO} : lengths;
+  static_assert(SP == 32 || SP == 64, "whole fragments, and whole steps in what a workgroup is given");
+  constexpr int kIndexChunk = kFilterWalkChunk;  // a pair a thread
   constexpr int kChunkSteps = kIndexChunk / SP;
-  constexpr int RBX = CI * 4, RBY = CO * 4;     // bytes per row
-  constexpr int XN = SP * RBX / 1024;           // 1 KiB wave-loads per step
-  constexpr int YN = SP * RBY / 1024;
-  constexpr int AB = CI / 32, BB = CO / 32;     // 16-row / 16-column blocks per wave
+  static_assert(kIndexChunk == 256 && kChunkSteps > 2, "indices land in time (see the loop)");
+  const FilterGradRows rows = WHOLE ? FilterGradRows{CI, CO} : lengths;
+  constexpr int RBX = CI * kSize, RBY = CO * kSize;  // bytes per row
+  constexpr int XN = SP * RBX / 1024;                // 1 KiB wave-loads per step, x first
+  constexpr int LOADS = XN + SP * RBY / 1024;
+  constexpr int MOST = (LOADS + 3) / 4;              // a wave's
+  constexpr int AB = CI / 32, BB = CO / 32;          // 16-row / 16-column blocks per wave
 
   __shared__ __attribute__((aligned(1024))) char s_x[2][SP * RBX];
   __shared__ __attribute__((aligned(1024))) char s_y[2][SP * RBY];
-  // where the rows of a chunk of pairs begin, and of the chunk after; kNoRow: a pair that is not there
-  __shared__ uint32_t s_in[2][kIndexChunk];
-  __shared__ uint32_t s_out[2][kIndexChunk];
+  // where the x rows and the y rows of a chunk of pairs begin, and of the chunk after; kNoRow: a pair that is not there
+  __shared__ __attribute__((aligned(1024))) uint32_t s_at[2][2][kIndexChunk];
 
   const FilterRun run = runOfWorkgroup(tab, order, total_slices, slice_len, shares);
   if (run.k < 0) return;
@@ -3331,18 +3149,19 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaRows(
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wa = wave >> 1, wb = wave & 1;
-  const int32_t *in_col = pairs + ((size_t)k * 2 + x_col) * L;
-  const int32_t *out_col = pairs + ((size_t)k * 2 + 1 - x_col) * L;
-  const uint32_t x_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)&s_x[0][0];
-  const uint32_t y_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)&s_y[0][0];
-  const uint32_t x_length = (uint32_t)rows.ci * 4u, y_length = (uint32_t)rows.co * 4u;  // bytes; zeros behind them
+  auto lds_of = [](const void *at) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)at; };
   auto words_of = [](const void *base, uint32_t bytes) {
     return u32x4{(uint32_t)reinterpret_cast<uintptr_t>(base), (uint32_t)(reinterpret_cast<uintptr_t>(base) >> 32), bytes,
                  0x00020000u};
   };
+  const uint32_t x_lds = lds_of(&s_x[0][0]), y_lds = lds_of(&s_y[0][0]);
+  const uint32_t index_lds = lds_of(&s_at[0][0][0]) + (uint32_t)wave * 256u;
+  const uint32_t x_length = (uint32_t)(rows.ci * kSize), y_length = (uint32_t)(rows.co * kSize);  // zeros behind them
   const u32x4 x_words = words_of(X, (uint32_t)n_in * x_length), y_words = words_of(dY, (uint32_t)n_out * y_length);
+  const u32x4 in_words = words_of(pairs + ((size_t)k * 2 + x_col) * L, (uint32_t)L * 4u);
+  const u32x4 out_words = words_of(pairs + ((size_t)k * 2 + 1 - x_col) * L, (uint32_t)L * 4u);
 
-  // blocks of 16 channels that the rows have, of this wave's (every second one: a wave has no more than the other)
+  // blocks of 16 channels that the rows have, of this wave's
   const int blocks_a = WHOLE ? AB : ((rows.ci + 15) / 16 - wa + 1) / 2;
   const int blocks_b = WHOLE ? BB : ((rows.co + 15) / 16 - wb + 1) / 2;
   float4v acc[AB][BB];
@@ -3351,139 +3170,153 @@ __global__ __launch_bounds__(256) void backwardFilterMfmaRows(
 #pragma unroll
     for (int b = 0; b < BB; ++b) acc[a][b] = float4v{0.f, 0.f, 0.f, 0.f};
 
-  // One step's rows into a buffer: wave-load t of an operand covers 1 KiB of the buffer, lane
-  // l its bytes [16 l, 16 l + 16), i.e. a fixed (pair, place) of the step.  Wave w issues
-  // loads w, w + 4, ...; all places are read first (one LDS latency a step, not one a load).
-  constexpr int XM = (XN + 3) / 4, YM = (YN + 3) / 4;
-  uint32_t x_piece[XM], y_piece[YM];  // the piece of its row that a lane asks for, by load
+  // One step's rows into a buffer: a wave-load covers 1 KiB of it, lane l its bytes [16 l, 16 l + 16), i.e. a fixed (pair,
+  // place) of the step.  Wave w issues loads w, w + 4, ...; all places are read first (one LDS latency a step,
+  // not one a load).
+  uint32_t piece[MOST];  // the piece of its row that a lane asks for, by load
+  int pair_of[MOST];     // and the pair, in s_at[chunk & 1]
+  bool of_x[MOST];
 #pragma unroll
-  for (int u = 0; u < XM; ++u) {
-    const int byte = (wave + u * 4) * 1024 + lane * 16;
-    x_piece[u] = (uint32_t)((byte % RBX / 16) ^ floatRowChunk(RBX, floatRowSlot(RBX, byte / RBX % SP)) * 4) * 16u;
-    if (x_piece[u] >= x_length) x_piece[u] = kNoRow;
-  }
-#pragma unroll
-  for (int u = 0; u < YM; ++u) {
-    const int byte = (wave + u * 4) * 1024 + lane * 16;
-    y_piece[u] = (uint32_t)((byte % RBY / 16) ^ floatRowChunk(RBY, floatRowSlot(RBY, byte / RBY % SP)) * 4) * 16u;
-    if (y_piece[u] >= y_length) y_piece[u] = kNoRow;
+  for (int u = 0; u < MOST; ++u) {
+    of_x[u] = u * 4 + 3 < XN || (u * 4 < XN && wave + u * 4 < XN);
+    const int row_bytes = of_x[u] ? RBX : RBY;
+    const int byte = ((of_x[u] ? 0 : -XN) + wave + u * 4) * 1024 + lane * 16;
+    const int slot = byte / row_bytes % SP;
+    const int pair = kFloat ? floatRowSlot(row_bytes, slot) : slot;
+    const int moved = kFloat ? floatRowChunk(row_bytes, pair) * 4 : filterRowSwizzle(row_bytes, pair);
+    piece[u] = (uint32_t)((byte % row_bytes / 16) ^ moved) * 16u;
+    if (piece[u] >= (of_x[u] ? x_length : y_length)) piece[u] = kNoRow;
+    pair_of[u] = (of_x[u] ? 0 : kIndexChunk) + pair;
   }
   auto request_step = [&](int step, int buffer) {
-    const uint32_t *in = s_in[(step / kChunkSteps) & 1] + (step % kChunkSteps) * SP;
-    const uint32_t *out = s_out[(step / kChunkSteps) & 1] + (step % kChunkSteps) * SP;
-    uint32_t at_x[XM], at_y[YM];
+    const uint32_t *at_step = &s_at[(step / kChunkSteps) & 1][0][(step % kChunkSteps) * SP];
+    uint32_t at[MOST];
 #pragma unroll
-    for (int u = 0; u < XM; ++u) at_x[u] = in[floatRowSlot(RBX, ((wave + u * 4) * 1024 + lane * 16) / RBX % SP)];
+    for (int u = 0; u < MOST; ++u) at[u] = at_step[pair_of[u]];
 #pragma unroll
-    for (int u = 0; u < YM; ++u) at_y[u] = out[floatRowSlot(RBY, ((wave + u * 4) * 1024 + lane * 16) / RBY % SP)];
-#pragma unroll
-    for (int u = 0; u < XM; ++u) {
-      at_x[u] = __builtin_elementwise_add_sat(at_x[u], x_piece[u]);
-      asm volatile("" : "+v"(at_x[u]));
+    for (int u = 0; u < MOST; ++u) {
+      at[u] = __builtin_elementwise_add_sat(at[u], piece[u]);
+      asm volatile("" : "+v"(at[u]));
     }
 #pragma unroll
-    for (int u = 0; u < YM; ++u) {
-      at_y[u] = __builtin_elementwise_add_sat(at_y[u], y_piece[u]);
-      asm volatile("" : "+v"(at_y[u]));
+    for (int u = 0; u < MOST; ++u) {
+      if (LOADS % 4 != 0 && wave + u * 4 >= LOADS) break;
+      if (of_x[u])
+        requestRowsToLds(x_words, at[u], x_lds + (uint32_t)(buffer * (SP * RBX) + (wave + u * 4) * 1024));
+      else
+        requestRowsToLds(y_words, at[u], y_lds + (uint32_t)(buffer * (SP * RBY) + (wave + u * 4 - XN) * 1024));
     }
-#pragma unroll
-    for (int u = 0; u < XM; ++u)
-      if (XN % 4 == 0 || wave + u * 4 < XN)
-        requestRowsToLds(x_words, at_x[u], x_lds + (uint32_t)(buffer * (SP * RBX) + (wave + u * 4) * 1024));
-#pragma unroll
-    for (int u = 0; u < YM; ++u)
-      if (YN % 4 == 0 || wave + u * 4 < YN)
-        requestRowsToLds(y_words, at_y[u], y_lds + (uint32_t)(buffer * (SP * RBY) + (wave + u * 4) * 1024));
   };
-  // Element of lane (c, kq) for MFMA step s of 16 pairs: channel 16 block + c of pair 4 kq + s.  (Slots and chunks are
-  // permuted by bits 2 and 3 of the pair: the same for all s and for the next 16 pairs.)
+
+  // Operand fragments: of 32 pairs of 2-byte elements, where lane (c, kq) receives the pairs 8 kq + (0..7) of channel
+  // 16 block + c, or, element by element, of 16 pairs in fp32, where multiply s takes its pair 4 kq + s.  (What is
+  // permuted by pair is the same for the four pairs and for the next fragment.)
   const int sub = lane & 15, kq = lane >> 4;
-  auto place_of = [&](int row_bytes, int block) -> int {
-    return (floatRowSlot(row_bytes, 4 * kq) - 4 * kq) * row_bytes + 4 * kq * row_bytes +
-           (block ^ floatRowChunk(row_bytes, 4 * kq)) * 64 + sub * 4;
+  auto fragment_place = [&](int row_bytes, int block) -> int {
+    if (kFloat)
+      return floatRowSlot(row_bytes, 4 * kq) * row_bytes + (block ^ floatRowChunk(row_bytes, 4 * kq)) * 64 + sub * 4;
+    const int pair = 8 * kq + (sub >> 2);
+    const int place = (block * 2 + ((sub & 3) >> 1)) ^ filterRowSwizzle(row_bytes, pair);
+    return pair * row_bytes + place * 16 + (sub & 1) * 8;
   };
   const char *x_frag[AB], *y_frag[BB];  // in the first buffer
 #pragma unroll
-  for (int a = 0; a < AB; ++a) x_frag[a] = &s_x[0][0] + place_of(RBX, wa + 2 * a);
+  for (int a = 0; a < AB; ++a) x_frag[a] = &s_x[0][0] + fragment_place(RBX, wa + 2 * a);
 #pragma unroll
-  for (int b = 0; b < BB; ++b) y_frag[b] = &s_y[0][0] + place_of(RBY, wb + 2 * b);
-
-  // Row indices of chunk c: four pairs a thread, checked; -1 marks a pair that is not there.
-  constexpr int IPT = kIndexChunk / 256;
-  int idx_in[IPT], idx_out[IPT];
-  auto fetch_indices = [&](int chunk) {
+  for (int b = 0; b < BB; ++b) y_frag[b] = &s_y[0][0] + fragment_place(RBY, wb + 2 * b);
+  auto fragment = [&](const char *at, int row_bytes) -> vec8 {
+    const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) v4i16 *)(at));
+    const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) v4i16 *)(at + 4 * row_bytes));
+    const v8i16 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    return __builtin_bit_cast(vec8, both);
+  };
+  auto multiply = [&](int buffer) {
+    const int x_at = buffer * (SP * RBX), y_at = buffer * (SP * RBY);
+    if constexpr (kFloat) {
 #pragma unroll
-    for (int u = 0; u < IPT; ++u) {
-      const int at = run.at(chunk * kIndexChunk + u * 256 + tid);
-      int i = -1, o = -1;
-      if (at < run.end) {
-        i = in_col[at];
-        o = out_col[at];
+      for (int kb = 0; kb < SP / 16; ++kb) {
+        float xs[4][AB], ys[4][BB];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+#pragma unroll
+          for (int a = 0; a < AB; ++a)
+            xs[q][a] = *reinterpret_cast<const float *>(x_frag[a] + x_at + kb * 16 * RBX + floatStepPlace(RBX, q, kq));
+#pragma unroll
+          for (int b = 0; b < BB; ++b)
+            ys[q][b] = *reinterpret_cast<const float *>(y_frag[b] + y_at + kb * 16 * RBY + floatStepPlace(RBY, q, kq));
+        }
+        // (the blocks that a row does not have are zeros in LDS; their multiplies are left out, behind the reads: a branch
+        // between reads and multiplies made small layers slower)
+#pragma unroll
+        for (int a = 0; a < AB; ++a) {
+          if (a >= blocks_a) break;
+#pragma unroll
+          for (int b = 0; b < BB; ++b) {
+            if (b >= blocks_b) break;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(xs[q][a], ys[q][b], acc[a][b], 0, 0, 0);
+          }
+        }
       }
-      idx_in[u] = i;
-      idx_out[u] = o;
+    } else {
+#pragma unroll
+      for (int kb = 0; kb < SP / 32; ++kb) {
+        vec8 bfr[BB];
+#pragma unroll
+        for (int b = 0; b < BB; ++b) bfr[b] = fragment(y_frag[b] + y_at + kb * 32 * RBY, RBY);
+#pragma unroll
+        for (int a = 0; a < AB; ++a) {
+          const vec8 afr = fragment(x_frag[a] + x_at + kb * 32 * RBX, RBX);
+#pragma unroll
+          for (int b = 0; b < BB; ++b) acc[a][b] = E::mfma(afr, bfr[b], acc[a][b]);
+        }
+      }
     }
   };
-  auto store_indices = [&](int chunk) {
-#pragma unroll
-    for (int u = 0; u < IPT; ++u) {
-      int i = idx_in[u], o = idx_out[u];
-      if ((unsigned)i >= (unsigned)n_in || (unsigned)o >= (unsigned)n_out) i = o = -1;
-      s_in[chunk & 1][u * 256 + tid] = i < 0 ? kNoRow : (uint32_t)i * x_length;
-      s_out[chunk & 1][u * 256 + tid] = o < 0 ? kNoRow : (uint32_t)o * y_length;
-    }
+
+  // A chunk's indices: a thread's own, to LDS as they are; then checked, and places where they stood.
+  auto request_indices = [&](int chunk) {
+    const uint32_t at = (uint32_t)run.at(chunk * kIndexChunk + tid) * 4u;  // (behind the list: zeros, checked below)
+    const uint32_t to = index_lds + (uint32_t)(chunk & 1) * (2 * kIndexChunk * 4);
+    requestWordsToLds(in_words, at, to);
+    requestWordsToLds(out_words, at, to + kIndexChunk * 4);
+  };
+  auto place_indices = [&](int chunk) {
+    uint32_t &in = s_at[chunk & 1][0][tid], &out = s_at[chunk & 1][1][tid];
+    const uint32_t i = in, o = out;
+    const bool there = run.at(chunk * kIndexChunk + tid) < run.end && i < (uint32_t)n_in && o < (uint32_t)n_out;
+    in = there ? i * x_length : kNoRow;
+    out = there ? o * y_length : kNoRow;
   };
 
   const int steps = run.length / SP;
-  fetch_indices(0);
-  store_indices(0);
-  __syncthreads();
-  request_step(0, 0);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  ldsBarrier();
+  if (steps > 0) {
+    request_indices(0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    place_indices(0);
+    ldsBarrier();
+    request_step(0, 0);
+  }
   for (int step = 0; step < steps; ++step) {
     const int cur = step & 1;
+    // this step's rows have landed, and every wave has left the buffers of the step before
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    ldsBarrier();
+    // The chunk after this one: its indices are requested at the chunk's first step (the places they come over were last
+    // read two steps before) and are places one barrier before the chunk's last step asks for the next one's first rows.
     const int in_chunk = step % kChunkSteps, chunk = step / kChunkSteps;
-    // the chunk after this one: its indices are requested at the chunk's first step and are
-    // in LDS one barrier before the chunk's last step asks for the next chunk's first rows
     const bool chunk_follows = (chunk + 1) * kChunkSteps < steps;
-    if (in_chunk == 0 && chunk_follows) fetch_indices(chunk + 1);
+    if (in_chunk == 0 && chunk_follows) request_indices(chunk + 1);
     // (all requests first: they have one step's multiplies to land; the other workgroups' requests wait for these
     // multiplies)
     if (step + 1 < steps) request_step(step + 1, cur ^ 1);
     __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int kb = 0; kb < SP / 16; ++kb) {
-      // (slot of pair 4 kq + q: with short rows bit 0 is flipped for half of the lanes)
-      const int x_at = cur * (SP * RBX) + kb * 16 * RBX, y_at = cur * (SP * RBY) + kb * 16 * RBY;
-      float xs[4][AB], ys[4][BB];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-#pragma unroll
-        for (int a = 0; a < AB; ++a)
-          xs[q][a] = *reinterpret_cast<const float *>(x_frag[a] + x_at + floatStepPlace(RBX, q, kq));
-#pragma unroll
-        for (int b = 0; b < BB; ++b)
-          ys[q][b] = *reinterpret_cast<const float *>(y_frag[b] + y_at + floatStepPlace(RBY, q, kq));
-      }
-      // (a row's missing blocks are zeros in LDS; their multiplies are left out)
-#pragma unroll
-      for (int a = 0; a < AB; ++a) {
-        if (a >= blocks_a) break;
-#pragma unroll
-        for (int b = 0; b < BB; ++b) {
-          if (b >= blocks_b) break;
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(xs[q][a], ys[q][b], acc[a][b], 0, 0, 0);
-        }
-      }
-    }
+    multiply(cur);
     __builtin_amdgcn_s_setprio(0);
-    if (in_chunk == kChunkSteps - 2 && chunk_follows) store_indices(chunk + 1);
-    // the next step's rows have landed, and every wave has left this step's buffers
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    ldsBarrier();
+    if (in_chunk == kChunkSteps - 2 && chunk_follows) place_indices(chunk + 1);
   }
   // lane holds rows 4*(lane/16)+v, column lane%16 of every 16 x 16 block
   float *const sums = partial + (size_t)run.tile * CI * CO;
@@ -4449,17 +4282,16 @@ void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const S
       if (whole) kernel = backwardFilterMfma<E, CI, CO, true>;
     }
     if constexpr (kTransposingShape) {
-      // Steps of 32 pairs halve the row buffers: below 128 x 128 channels more workgroups
-      // share a CU then, which pays when the slices are long (network 64 x 64: 101 -> 88 us;
-      // on slices of a few steps the shorter steps only add barriers: config 4 23.7 -> 25.3 us).
-      const bool short_steps = CI + CO < 256 && slice_len >= 2048;
-      auto tr = kernel;
-      if constexpr (sizeof(S) == 4) {
-        tr = whole ? backwardFilterMfmaRows<CI, CO, true> : backwardFilterMfmaRows<CI, CO, false>;
-      } else {
-        tr = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32, false> : backwardFilterMfmaTr<E, CI, CO, 64, false>;
-        if (whole)
-          tr = short_steps ? backwardFilterMfmaTr<E, CI, CO, 32, true> : backwardFilterMfmaTr<E, CI, CO, 64, true>;
+      // fp32 takes steps of 32 pairs, 2-byte types of 64, half as many barriers; with 128 channels on a side those
+      // leave two or three workgroups' buffers on a CU, and where a workgroup has many steps the shorter ones, with
+      // four, are faster.  us with the sums, fp16, steps of 32 / 64, 3.0 M pairs: 32 x 32 55/39   32 x 64 62/50
+      // 64 x 64 67/57   32 x 128 73/83   64 x 128 89/100   128 x 128 135/142; 0.98 M pairs: 32 x 32 28/23   64 x 64 35/31
+      // 64 x 128 43/41   128 x 128 67/59.  fp32, 0.98 M: 64 x 64 86/98   128 x 128 302/317
+      auto tr = backwardFilterRows<E, CI, CO, 32, false>;
+      if (whole) tr = backwardFilterRows<E, CI, CO, 32, true>;
+      if constexpr (sizeof(S) == 2) {
+        const bool short_steps = (CI == 128 || CO == 128) && slice_len >= 2048;
+        if (!short_steps) tr = whole ? backwardFilterRows<E, CI, CO, 64, true> : backwardFilterRows<E, CI, CO, 64, false>;
       }
       if (transposing)
         tr<<<grid, 256, 0, lc.stream>>>(
