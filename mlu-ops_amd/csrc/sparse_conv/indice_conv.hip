@@ -1086,25 +1086,43 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rowsBuffer(const void *base, u
 // blocks takes about 0.4 us, and the launch lasts as long as its heaviest tile (28 us, mean 16).
 // Rounds are padded to whole trips of the loops, which have one way out each: with a second one the
 // compiler waits for all loads in flight at the loop's head.
+//
+// Tiles of 512 rows of a 2-byte type (tallTileRows) halve the filters a row costs and fill their blocks better (0.69 of
+// the pairs of a block instead of 0.48 at the 5x5x5 shape).  They leave a CU one workgroup, and a round is a chain of LDS
+// round trips: so eight waves multiply, as two teams that take the rounds in turn.  A team reads its round's
+// rows and adds its last products while the other multiplies, and the other way round: two barriers a round of a team,
+// one a round of the tile, and sums still change in the order of the blocks.
+// 449 -> 360 us at the 5x5x5 shape; 409 without the teams.  Of the 360 some 60 are tiles' beginnings and ends; without
+// the requests of filters and rows 317 are left, so the rest is the rounds' chains.  (Twice as many rounds under way, sums
+// by LDS additions without return (2680 us), or entries of one word: none faster.)  At 256 rows teams gave 2 %.
 struct TallPlan {
   int per_cu;      // workgroups a CU
   int blocks;      // blocks of 16 pairs a round
   int ahead;       // rounds whose rows and filters travel in registers
   int max_blocks;  // blocks whose entries are in LDS at once
+  bool teams;      // the multiplying waves are two teams
+  int multipliers; // multiplying waves
 };
 constexpr int kTallCols = 64;
-constexpr int kTallWaves = 4;  // multiplying waves, and as many fetching ones
-constexpr int kTallThreads = 2 * kTallWaves * 64;
+constexpr int kTallFetchers = 4;  // fetching waves
 // Two workgroups of 256 rows share a CU, but for rows of 512 bytes, of which the second would leave
-// no room for a round.  (Few rows run in half of the 256: tallHalfTiles.)
+// no room for a round.  (Few rows run in half of the 256, many offsets in twice as many: tallTileRows.)
 constexpr int tallRows(int row_bytes) { return row_bytes >= 512 ? 512 : 256; }
-constexpr TallPlan tallPlan(int row_bytes) {
-  const int rows = tallRows(row_bytes);
-  TallPlan p = {rows == 256 ? 2 : 1, 1, 4, 0};
+// (Tiles of 128 rows take the plan of 256.)
+constexpr TallPlan tallPlan(int elem_bytes, int row_bytes, int tile_rows) {
+  const int rows = tile_rows == 512 ? 512 : 256;
+  TallPlan p = {rows == 256 ? 2 : 1, 1, 4, 0, elem_bytes == 2 && rows == 512, 4};
+  if (p.teams) p.multipliers = 8;
   p.blocks = (rows == 256 ? 4096 : 8192) / (16 * row_bytes);
   const int left = 160 * 1024 / p.per_cu - (rows + 1) * kTallCols * 4 - 2 * p.blocks * 16 * row_bytes - 256;
   p.max_blocks = left / 98 / (p.ahead * p.blocks) * (p.ahead * p.blocks);
   return p;
+}
+constexpr int tallThreads(int elem_bytes, int row_bytes, int tile_rows) {
+  return (tallPlan(elem_bytes, row_bytes, tile_rows).multipliers + kTallFetchers) * 64;
+}
+constexpr int tallWavesPerSimd(int elem_bytes, int row_bytes, int tile_rows) {
+  return tallPlan(elem_bytes, row_bytes, tile_rows).per_cu * tallThreads(elem_bytes, row_bytes, tile_rows) / 256;
 }
 // Where 16-byte piece `piece` of staged row `row` lies: piece ^ this.
 constexpr int tallRowSwizzle(int row_bytes, int row) {
@@ -1112,18 +1130,22 @@ constexpr int tallRowSwizzle(int row_bytes, int row) {
 }
 
 template <typename E, int Q, int C, int TR, typename SRC>
-__global__ __launch_bounds__(kTallThreads)
-    __attribute__((amdgpu_waves_per_eu(2 * tallPlan(Q * (int)sizeof(typename E::storage)).per_cu,
-                                       2 * tallPlan(Q * (int)sizeof(typename E::storage)).per_cu)))
+__global__ __launch_bounds__(tallThreads((int)sizeof(typename E::storage), Q * (int)sizeof(typename E::storage), TR))
+    __attribute__((amdgpu_waves_per_eu(
+        tallWavesPerSimd((int)sizeof(typename E::storage), Q * (int)sizeof(typename E::storage), TR),
+        tallWavesPerSimd((int)sizeof(typename E::storage), Q * (int)sizeof(typename E::storage), TR))))
 void gatherConvTall(const typename E::storage *A, uint32_t a_size, ConvRows rows, const typename E::storage *packedW,
                     SRC source, int R, int K, typename E::storage *result) {
   typedef typename E::vec8 vec8;
   typedef typename E::storage S;
   constexpr int ROW_BYTES = Q * (int)sizeof(S);
-  constexpr TallPlan PLAN = tallPlan(ROW_BYTES);
-  constexpr int NT = kTallThreads;
-  constexpr int FW = kTallWaves;
-  constexpr int NB = C / 16 / kTallWaves;    // column blocks of a multiplying wave
+  constexpr TallPlan PLAN = tallPlan((int)sizeof(S), ROW_BYTES, TR);
+  constexpr int MW = PLAN.multipliers;
+  constexpr int FW = kTallFetchers;
+  constexpr int NT = (MW + FW) * 64;
+  constexpr bool kTeams = PLAN.teams;
+  constexpr int TW = kTeams ? MW / 2 : MW;   // waves of a team
+  constexpr int NB = C / 16 / TW;            // column blocks of a multiplying wave
   constexpr int KB = ROW_BYTES / 64;         // operand fragments per row
   constexpr int G = PLAN.blocks;
   constexpr int U = PLAN.ahead;
@@ -1148,7 +1170,7 @@ void gatherConvTall(const typename E::storage *A, uint32_t a_size, ConvRows rows
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const bool fetcher = wave >= kTallWaves;
+  const bool fetcher = wave >= MW;
   const int tiles_per_xcd = gridDim.x >> 3;  // neighbouring tiles on one XCD, as above
   const int tile = (blockIdx.x & 7) * tiles_per_xcd + (blockIdx.x >> 3);
   const int r0 = tile * TR;
@@ -1196,7 +1218,7 @@ void gatherConvTall(const typename E::storage *A, uint32_t a_size, ConvRows rows
   const int quad = lane >> 4;
   const __amdgpu_buffer_rsrc_t a_rows = rowsBuffer(A, a_size);
   const char *const b_base = reinterpret_cast<const char *>(packedW) +
-                             ((size_t)(col_group * GROUPS + (wave & 3) * NB) * KB * 64 + lane) * 16;
+                             ((size_t)(col_group * GROUPS + wave % TW * NB) * KB * 64 + lane) * 16;
   const uint32_t bytes_per_offset = (uint32_t)(rows.c_padded / 16) * KB * 1024;  // packed W[k]
 
   for (int kc = 0; kc < (in_order ? K : 0);) {
@@ -1305,7 +1327,7 @@ void gatherConvTall(const typename E::storage *A, uint32_t a_size, ConvRows rows
     if (n_blocks == 0) continue;
     // B
     if (fetcher) {
-      const int ftid = tid - kTallWaves * 64;
+      const int ftid = tid - MW * 64;
       u32x4 piece[U][NI];
       auto request_round = [&](int round, u32x4 (&to)[NI]) {
 #pragma unroll
@@ -1337,6 +1359,92 @@ void gatherConvTall(const typename E::storage *A, uint32_t a_size, ConvRows rows
           ldsBarrier();  // round r + j is there, and nobody reads the round before any more
         }
       }
+      if constexpr (kTeams) {  // (the phases behind the last round's first)
+        ldsBarrier();
+        ldsBarrier();
+      }
+    } else if constexpr (kTeams) {
+      constexpr int UT = U / 2;  // of a team's rounds, whose filters travel in registers
+      const int team = wave / TW, part = wave % TW;
+      vec8 w[UT][G][KB][NB];
+      auto request_filters = [&](const int (&ks)[G], vec8 (&to)[G][KB][NB]) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const char *const bk = b_base + (size_t)__builtin_amdgcn_readfirstlane(ks[g]) * bytes_per_offset;
+#pragma unroll
+          for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) to[g][kb][nb] = *reinterpret_cast<const vec8 *>(bk + (nb * KB + kb) * 1024);
+        }
+      };
+      // (round t of the team)
+      auto offsets_of = [&](int t, int (&ks)[G]) {
+        const int r = t * 2 + team < n_rounds ? t * 2 + team : n_rounds - 1;
+#pragma unroll
+        for (int g = 0; g < G; ++g) ks[g] = s_k[r * G + g];
+      };
+      int ks[G], own[G];
+#pragma unroll
+      for (int j = 0; j < UT; ++j) {
+        offsets_of(j, ks);
+        request_filters(ks, w[j]);
+        asm volatile("" ::: "memory");
+      }
+      offsets_of(UT, ks);
+      float4v prod[G][NB];
+      // one block after the other, since blocks of different offsets may meet in a row
+      auto add_block = [&](int g) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+          // lane holds result columns 4 * piece + (0..3) of its pair
+          const int piece = (part * NB + nb) * 4 + quad;
+          float4v *const sum = reinterpret_cast<float4v *>(s_acc) + own[g] * (C / 4) + (piece ^ (own[g] & 15));
+          float4v old = *sum;
+          old += prod[g][nb];
+          *sum = old;
+        }
+      };
+#pragma unroll
+      for (int g = 0; g < G; ++g) own[g] = TR;
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) prod[g][nb] = float4v{0.f, 0.f, 0.f, 0.f};
+      if (team == 1) ldsBarrier();
+      const char *const stage = s_stage + team * ROUND;
+      for (int t = 0; t < n_rounds / 2; t += UT) {
+#pragma unroll
+        for (int j = 0; j < UT; ++j) {
+          ldsBarrier();  // the round is there, and the other team has added the round between
+          vec8 a[G][KB];
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+              a[g][kb] = *reinterpret_cast<const vec8 *>(stage + (g * 16 + pair) * ROW_BYTES +
+                                                         (((kb * 4 + quad) ^ tallRowSwizzle(ROW_BYTES, pair)) * 16));
+            add_block(g);
+          }
+#pragma unroll
+          for (int g = 0; g < G; ++g) own[g] = s_row[(((t + j) * 2 + team) * G + g) * 16 + pair];
+          ldsBarrier();
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) prod[g][nb] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+              for (int nb = 0; nb < NB; ++nb) prod[g][nb] = E::mfma(w[j][g][kb][nb], a[g][kb], prod[g][nb]);
+          }
+          request_filters(ks, w[j]);
+          offsets_of(t + j + UT + 1, ks);
+        }
+      }
+      ldsBarrier();
+#pragma unroll
+      for (int g = 0; g < G; ++g) add_block(g);
+      if (team == 0) ldsBarrier();
     } else {
       vec8 w[U][G][KB][NB];
       // filters of a round whose blocks have the offsets ks
@@ -3737,20 +3845,23 @@ int tallGridX(int R, int tile_rows) { return ((R + tile_rows - 1) / tile_rows + 
 
 template <typename E, int Q, typename SRC>
 void launchTallInstance(const LaunchCtx &lc, const void *A, uint32_t a_size, const ConvRows &rows, const void *packed,
-                        const SRC &source, bool half_tiles, int R, int K, void *result) {
-  constexpr int TR = tallRows(Q * (int)sizeof(typename E::storage));
-  const dim3 grid(tallGridX(R, half_tiles ? TR / 2 : TR), (rows.c + kTallCols - 1) / kTallCols);
-  auto launch = [&](auto kernel) {
+                        const SRC &source, int tile_rows, int R, int K, void *result) {
+  constexpr int S = (int)sizeof(typename E::storage);
+  constexpr int TR = tallRows(Q * S);
+  auto launch = [&](auto kernel, int threads) {
+    const dim3 grid(tallGridX(R, tile_rows), (rows.c + kTallCols - 1) / kTallCols);
     lc.begin("gatherConvTall");
-    kernel<<<grid, kTallThreads, 0, lc.stream>>>(static_cast<const typename E::storage *>(A), a_size, rows,
-                                                 static_cast<const typename E::storage *>(packed), source, R, K,
-                                                 static_cast<typename E::storage *>(result));
+    kernel<<<grid, threads, 0, lc.stream>>>(static_cast<const typename E::storage *>(A), a_size, rows,
+                                            static_cast<const typename E::storage *>(packed), source, R, K,
+                                            static_cast<typename E::storage *>(result));
     lc.end();
   };
   if constexpr (SRC::kSegments && TR == 256) {
-    if (half_tiles) return launch(gatherConvTall<E, Q, kTallCols, TR / 2, SRC>);
+    if (tile_rows == 128) return launch(gatherConvTall<E, Q, kTallCols, 128, SRC>, tallThreads(S, Q * S, 128));
+    if constexpr (S == 2)
+      if (tile_rows == 512) return launch(gatherConvTall<E, Q, kTallCols, 512, SRC>, tallThreads(S, Q * S, 512));
   }
-  launch(gatherConvTall<E, Q, kTallCols, TR, SRC>);
+  launch(gatherConvTall<E, Q, kTallCols, TR, SRC>, tallThreads(S, Q * S, TR));
 }
 
 // Channels of the instance for rows of q_padded channels (16 channels of a 2-byte type are half a fragment,
@@ -3759,16 +3870,16 @@ int tallQ(ElemType t, int q_padded) { return t != ElemType::kFloat && q_padded <
 
 template <typename E, typename SRC>
 void launchTall(const LaunchCtx &lc, int q, const void *A, int n_src, const ConvRows &rows, const void *packed,
-                const SRC &source, bool half_tiles, int R, int K, void *result) {
+                const SRC &source, int tile_rows, int R, int K, void *result) {
   const uint32_t a_size = (uint32_t)n_src * (uint32_t)rows.row_bytes;
   switch (q) {
     case 16:
       if constexpr (std::is_same<E, FloatElem>::value)
-        launchTallInstance<E, 16, SRC>(lc, A, a_size, rows, packed, source, half_tiles, R, K, result);
+        launchTallInstance<E, 16, SRC>(lc, A, a_size, rows, packed, source, tile_rows, R, K, result);
       break;
-    case 32: launchTallInstance<E, 32, SRC>(lc, A, a_size, rows, packed, source, half_tiles, R, K, result); break;
-    case 64: launchTallInstance<E, 64, SRC>(lc, A, a_size, rows, packed, source, half_tiles, R, K, result); break;
-    case 128: launchTallInstance<E, 128, SRC>(lc, A, a_size, rows, packed, source, half_tiles, R, K, result); break;
+    case 32: launchTallInstance<E, 32, SRC>(lc, A, a_size, rows, packed, source, tile_rows, R, K, result); break;
+    case 64: launchTallInstance<E, 64, SRC>(lc, A, a_size, rows, packed, source, tile_rows, R, K, result); break;
+    case 128: launchTallInstance<E, 128, SRC>(lc, A, a_size, rows, packed, source, tile_rows, R, K, result); break;
     default: break;
   }
 }
@@ -3810,6 +3921,21 @@ constexpr int kTallFewOffsets = 32;
 bool tallHalfTiles(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d) {
   return lc.choices.tall_tiles < 0 && (p.K > kTallFewOffsets || d.R >= kTallFewestRows) &&
          tallRows(d.q_padded * (int)elemSize(p.dtype)) == 256 && (int64_t)d.R * (d.c_padded / 64) <= kTallFewRows;
+}
+
+// Rows of a tall tile.  Many offsets of short lists (the filters of 125 at 128 x 128 channels are 4 MB, and every tile reads
+// them): 512 rows with two teams of multiplying waves, for 2-byte types and rows of 65 channels up; one of 33 to 64 still
+// gains, one of 32 does not.  us of tiles of 256 / 512 rows, fp16, surfaces, 5x5x5:
+//   128 -> 128   400 k rows 449/360   200 k 246/212   50 k 73/54      128 -> 64   400 k 235/193   50 k 54/50
+//    96 -> 96    400 k rows 410/349   100 k 138/117                    64 -> 64   400 k 165/150   100 k 71/65   50 k 43/42
+//    32 -> 64    400 k rows 139/142   50 k 37/41
+//   3x3x3, clustered: 128 -> 128  400 k 243/232   200 k 117/118;  64 -> 64  400 k 99/104   60 k 23/25;  uniform, 200 k:
+//   128 -> 128  69/78;  2x2x2 stride 2, 177 k rows: 128 -> 128  55/60: up to 32 offsets stay with 256.
+int tallTileRows(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d, int tall_q, bool lists) {
+  const int row_bytes = tall_q * (int)elemSize(p.dtype);
+  if (lists && tallHalfTiles(lc, p, d)) return 128;
+  if (lists && p.K > kTallFewOffsets && elemSize(p.dtype) == 2 && row_bytes >= 128) return 512;
+  return tallRows(row_bytes);
 }
 
 bool useTallKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d, bool lists) {
@@ -4052,13 +4178,13 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
   const bool dense = use_mfma && useDenseKernel(lc, p, d);
   const bool tall = use_mfma && !dense && useTallKernel(lc, p, d, lists);
   const int tall_q = tallQ(p.dtype, d.q_padded);
-  const bool half_tiles = tall && lists && tallHalfTiles(lc, p, d);
+  const int tall_rows = tall ? tallTileRows(lc, p, d, tall_q, lists) : 0;
   if (lists) {
     // Pair lists in order (as far as the caller knows: the first kernel checks): the
     // gather kernel reads them cut by tile, no row map.
     const int tile_cols = dense ? d.c_padded : mfmaTileCols(p, d);
     const int tile_rows = dense ? kDenseRows
-                          : tall ? tallRows(tall_q * (int)sizeof(S)) / (half_tiles ? 2 : 1)
+                          : tall ? tall_rows
                                  : mfmaTileRows(tile_cols);
     int tile_shift = 0;
     while ((1 << tile_shift) < tile_rows) ++tile_shift;
@@ -4096,7 +4222,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     if (dense)
       launchDense<E, SegmentSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, src, d.R, p.K, result);
     else if (tall)
-      launchTall<E, SegmentSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, src, half_tiles, d.R, p.K,
+      launchTall<E, SegmentSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, src, tall_rows, d.R, p.K,
                                    result);
     else if (tile_cols == d.c_padded && useWaveKernel(lc, p.dtype, d.q_padded, d.c_padded))
       launchWave<E>(lc, d.q_padded, rows_from, rows_of, ws.packed, src, d.R, p.K, result);
@@ -4139,8 +4265,9 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
         n_filled = denseGridX(rows);
         launchDense<E, MapSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K, result_rows);
       } else if (tall) {
-        n_filled = tallGridX(rows, tallRows(tall_q * (int)sizeof(S)));
-        launchTall<E, MapSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, map, false, rows, p.K, result_rows);
+        n_filled = tallGridX(rows, tall_rows);
+        launchTall<E, MapSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, map, tall_rows, rows, p.K,
+                                 result_rows);
       } else {
         n_filled = mfmaGridX(rows, tile_cols);
         launchMfma<E, MapSource>(lc, d.q_padded, tile_cols, rows_from, rows_of, ws.packed, map, rows, p.K, result_rows);
