@@ -1363,6 +1363,17 @@ void gatherConvTall(const typename E::storage *A, uint32_t a_size, ConvRows rows
         ldsBarrier();
         ldsBarrier();
       }
+    } else if (col_group * C + wave % TW * NB * 16 >= rows.c) {
+      // no result column of this wave's: its part of the barriers (the other workgroup gets its CU's pipes: fp32
+      // 64 -> 96, 2x2x2 stride 2 of 200 000 rows, 74 -> 70 us)
+      for (int r = 0; r < n_rounds; r += U) {
+#pragma unroll
+        for (int j = 0; j < U; ++j) ldsBarrier();
+      }
+      if constexpr (kTeams) {
+        ldsBarrier();
+        ldsBarrier();
+      }
     } else if constexpr (kTeams) {
       constexpr int UT = U / 2;  // of a team's rounds, whose filters travel in registers
       const int team = wave / TW, part = wave % TW;
@@ -2461,8 +2472,9 @@ void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRo
 // rows they belong to, and stores the products.  Its blocks are full, its filter is one, and it needs no sums in
 // LDS and no cut table.  The waves split columns and rows as in the dense kernel above; rows go straight into LDS.
 // What bounds it is the chain of three dependent loads (pairs, rows, results) of workgroups that live for 5 us, and
-// memory.  us of the gather kernel alone, 2x2x2 stride 2, the list kernels / this one: fp32 96 -> 64 of 200 000 rows
-// 76/39, bf16 128 -> 96 of 100 000 31/16, fp16 128 -> 64 of 150 000 24/15, 64 -> 64 of 100 000 15/10, 32 -> 16 9.8/5.8.
+// memory; in fp32 the multiplies, of which those behind a row's end are left out (39 -> 35 us with 96 channels in tiles of
+// 128).  us of the gather kernel alone, 2x2x2 stride 2, the list kernels / this one: fp32 96 -> 64 of 200 000 rows
+// 76/35, bf16 128 -> 96 of 100 000 31/16, fp16 128 -> 64 of 150 000 24/15, 64 -> 64 of 100 000 15/10, 32 -> 16 9.8/5.8.
 constexpr int singlePairs(int row_bytes) { return row_bytes >= 512 ? 64 : 128; }
 constexpr int singlePieceAt(int row_bytes, int row, int piece) {
   if (row_bytes >= 256) return piece ^ (row & 15);
@@ -2555,7 +2567,8 @@ __global__ __launch_bounds__(kDenseThreads) void gatherConvSingle(
     for (int nb = 0; nb < NB; ++nb) {
       float4v product = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) product = E::mfma(w[nb][kb], row[kb], product);
+      for (int kb = 0; kb < KB; ++kb)
+        if (kb * 64 < conv.row_bytes) product = E::mfma(w[nb][kb], row[kb], product);
       if (to < 0) continue;
       // (a sum that starts from zero, as in the other kernels: a product of -0 is stored as 0)
       S tmp[4];
