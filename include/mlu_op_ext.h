@@ -141,6 +141,14 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtOrderVoxels(mluOpHandle_t handle, const void
                                                 const int64_t space[3], int32_t batch_index, void *workspace,
                                                 size_t workspace_size, void *order, void *indices);
 
+/* The mean of every voxel's points: voxels [num_voxels, max_points, features] fp32, contiguous, as mluOpVoxelization
+ * writes them (all slots are summed: those behind a voxel's points hold zeros), num_points_per_voxel
+ * [num_voxels] int32, below one taken as one; mean [num_voxels, features] fp32.  One launch, no workspace, no
+ * wait.  No counterpart in the reference. */
+mluOpStatus_t MLUOP_WIN_API mluOpExtMeanVoxelPoints(mluOpHandle_t handle, const void *voxels,
+                                                    const void *num_points_per_voxel, int64_t num_voxels,
+                                                    int32_t max_points, int32_t features, void *mean);
+
 /* Row maps kept across calls.  mluOpIndiceConvolutionForward and ...BackwardData turn the pair
  * lists into a [K, rows] map (partner row of every result row at every offset, or -1) on every
  * call: the reference API (mlu_op.h:10321-10448, :9625-9773) hands them nothing else to keep.

@@ -68,6 +68,7 @@ namespace {
   X(mluOpExtGetForwardRelu)                                \
   X(mluOpExtGetOrderVoxelsWorkspaceSize)                   \
   X(mluOpExtOrderVoxels)                                   \
+  X(mluOpExtMeanVoxelPoints)                               \
   X(mluOpExtGetIndicePairsHostCounts)                      \
   X(mluOpExtGetVoxelizationHostCount)                      \
   X(mluOpExtGetRowMapSize)                                 \
@@ -713,6 +714,20 @@ std::vector<at::Tensor> orderVoxels(bool guarded, const at::Tensor &coors, const
   return {order, indices};
 }
 
+// Mean of every voxel's points: [V, max_points, F] fp32 -> [V, F].
+at::Tensor meanVoxelPoints(bool guarded, const at::Tensor &voxels, const at::Tensor &counts) {
+  StreamHandle &h = streamHandle();
+  const OperatorLock lock(h);
+  const Buffers buffers(guarded, voxels.device());
+  const at::Tensor mean = buffers.output({voxels.size(0), voxels.size(2)}, at::kFloat, "mean");
+  check(api.mluOpExtMeanVoxelPoints(h.handle, voxels.data_ptr(), counts.data_ptr(), voxels.size(0),
+                                    static_cast<int32_t>(voxels.size(1)), static_cast<int32_t>(voxels.size(2)),
+                                    mean.data_ptr()),
+        "mluOpExtMeanVoxelPoints");
+  buffers.done("mluOpExtMeanVoxelPoints");
+  return mean;
+}
+
 std::vector<at::Tensor> scatterForward(mluOpHandle_t handle, const Buffers &buffers, const at::Tensor &feats,
                                        const at::Tensor &coors, mluOpReduceMode_t mode, int64_t rows) {
   const int64_t n = feats.size(0), c = feats.size(1);
@@ -872,6 +887,10 @@ PYBIND11_MODULE(_native, m) {
       r = orderVoxels(guarded, coors, space, batch_index);
     }
     return py::make_tuple(r[0], r[1]);
+  });
+  m.def("mean_voxel_points", [](bool guarded, const at::Tensor &voxels, const at::Tensor &counts) {
+    NoGil released;
+    return meanVoxelPoints(guarded, voxels, counts);
   });
   m.def("dynamic_point_to_voxel_forward",
         [](uintptr_t handle, bool guarded, const at::Tensor &feats, const at::Tensor &coors, int mode, int64_t rows) {

@@ -134,6 +134,7 @@ SIGNATURES = {
     "mluOpExtGetForwardRelu": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int)]),
     "mluOpExtGetOrderVoxelsWorkspaceSize": (ctypes.c_int, [ctypes.c_int64, _vp, _vp]),
     "mluOpExtOrderVoxels": (ctypes.c_int, [_vp, _vp, ctypes.c_int64, _vp, ctypes.c_int32, _vp, ctypes.c_size_t, _vp, _vp]),
+    "mluOpExtMeanVoxelPoints": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, _vp]),
     "mluOpExtGetVoxelizationHostCount": (ctypes.c_int, [_vp, _vp, ctypes.POINTER(ctypes.c_int32)]),
     "mluOpExtGetIndicePairsHostCounts": (ctypes.c_int, [_vp, _vp, ctypes.c_int, _i64p]),
     "mluOpExtGetRowMapSize": (ctypes.c_int, [_vp, ctypes.c_int64, ctypes.POINTER(ctypes.c_size_t)]),

@@ -400,7 +400,22 @@ class Voxelization(torch.nn.Module):
 
 def mean_voxel_features(voxels, num_points_per_voxel):
     """Mean of the points of every voxel (mmcv's HardSimpleVFE): [V, max_points, F] -> [V, F]."""
+    if _mean_by_library(voxels, num_points_per_voxel):
+        return native().mean_voxel_points(_guarded(), voxels, num_points_per_voxel)
     return voxels.sum(dim=1) / num_points_per_voxel.clamp(min=1).to(voxels.dtype).unsqueeze(1)
+
+
+def _mean_by_library(voxels, counts):
+    """Whether the library's kernel takes the means (one launch in place of four; voxelizer and 11-layer encoder, 120 000
+    voxels: 746 -> 713 us): what it accepts, on the current device, without a gradient to record and no mode that
+    watches torch's calls."""
+    return (type(voxels) is torch.Tensor and type(counts) is torch.Tensor and voxels.is_cuda and counts.is_cuda and
+            voxels.dtype == torch.float32 and counts.dtype == torch.int32 and voxels.dim() == 3 and counts.dim() == 1 and
+            counts.shape[0] == voxels.shape[0] and 0 < voxels.numel() < 1 << 31 and
+            voxels.is_contiguous() and counts.is_contiguous() and not voxels.is_conj() and not voxels.is_neg() and
+            voxels.device.index == torch.cuda.current_device() and counts.device == voxels.device and
+            not (torch.is_grad_enabled() and voxels.requires_grad) and
+            torch.autograd.forward_ad.unpack_dual(voxels).tangent is None and _unwatched())
 
 
 def _ordered_by_library(coors, spatial_shape, batch_index):
