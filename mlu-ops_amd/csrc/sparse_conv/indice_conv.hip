@@ -2229,6 +2229,8 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
 // 248 636 rows of a scene, 27 offsets, with the filter's packing, this kernel / filters through LDS with
 // rows in operand order (128) or through registers and LDS (64):
 //   fp16 128 -> 128 167/210    64 -> 64 82/95
+// OFFSETS: an offset's product is a chain of its own, added to the row's sum when it is whole, as the pair-list kernels
+// add: their bits (128 -> 128 takes the registers of two workgroups a CU for it; useDenseKernel has both sides' times).
 // Of two offsets a phase (64 channels: 93), tiles of 256 rows (128: 233; 64: 123), whole rows of 256 bytes (185),
 // quarters (181) and 32 columns a wave at 64 (86) none is faster.
 struct StagedPlan {
@@ -2239,7 +2241,8 @@ struct StagedPlan {
 constexpr StagedPlan stagedPlan(int elem_bytes, int Q, int C) {
   return StagedPlan{C >= 64 ? 4 : (C >= 32 ? 2 : 1), C >= 128 ? 2 : 1, Q * elem_bytes >= 256 ? 2 : 1};
 }
-constexpr int kStagedPerCu = 3;  // workgroups a CU
+// Workgroups a CU.
+constexpr int stagedPerCu(int Q, int C, bool offsets) { return offsets && Q == 128 && C == 128 ? 2 : 3; }
 // Where piece `piece` of a staged row lies among its row's pieces: at piece ^ this.
 __device__ __forceinline__ int stagedSwizzle(int row) {
   return (row >> 1) & 7;
@@ -2258,8 +2261,9 @@ __device__ __forceinline__ void requestWordsToLds(u32x4 words, uint32_t offset, 
                :: "s"(lds_address), "v"(offset), "s"(words) : "memory", "m0");
 }
 
-template <typename E, int Q, int C, typename SRC>
-__global__ __launch_bounds__(kDenseThreads) __attribute__((amdgpu_waves_per_eu(kStagedPerCu, kStagedPerCu)))
+template <typename E, int Q, int C, bool OFFSETS, typename SRC>
+__global__ __launch_bounds__(kDenseThreads)
+    __attribute__((amdgpu_waves_per_eu(stagedPerCu(Q, C, OFFSETS), stagedPerCu(Q, C, OFFSETS))))
 void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRows conv,
                            const typename E::storage *packedW, SRC source, int R, int K, typename E::storage *result) {
   typedef typename E::vec8 vec8;
@@ -2338,6 +2342,7 @@ void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRo
   for (int g = 0; g < G; ++g)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[g][nb] = float4v{0.f, 0.f, 0.f, 0.f};
+  float4v held[OFFSETS && PARTS > 1 ? G : 1][OFFSETS && PARTS > 1 ? NB : 1];  // an offset's product, of its first part
   int slots = 0;  // filled map slots this thread staged
 
   for (int kc = 0; kc < K; kc += KC) {
@@ -2409,7 +2414,7 @@ void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRo
     };
     // (a group's rows are read while the group before is multiplied; those of a group without partners are what
     // the buffer held before, and nobody multiplies them)
-    auto multiply = [&](int kk, int buffer, const Filters &w) {
+    auto multiply = [&](int kk, int part, int buffer, const Filters &w) {
       const uint32_t groups = groups_of(kk) >> first_group;
       vec8 row[2][KP];
       auto read_group = [&](int g) {
@@ -2423,10 +2428,21 @@ void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRo
         if (g + 1 < G) read_group(g + 1);
         __builtin_amdgcn_sched_barrier(0);
         if ((groups >> g & 1u) == 0) continue;
+        if constexpr (OFFSETS) {
 #pragma unroll
-        for (int kb = 0; kb < KP; ++kb)
+          for (int nb = 0; nb < NB; ++nb) {
+            float4v product = part > 0 ? held[g][nb] : float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int nb = 0; nb < NB; ++nb) acc[g][nb] = E::mfma(w[nb][kb], row[g & 1][kb], acc[g][nb]);
+            for (int kb = 0; kb < KP; ++kb) product = E::mfma(w[nb][kb], row[g & 1][kb], product);
+            if (part == PARTS - 1) acc[g][nb] += product;
+            else held[g][nb] = product;
+          }
+        } else {
+#pragma unroll
+          for (int kb = 0; kb < KP; ++kb)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) acc[g][nb] = E::mfma(w[nb][kb], row[g & 1][kb], acc[g][nb]);
+        }
       }
     };
     // (two phases a trip and one way out of the loop, at the price of an empty phase at the end of an
@@ -2439,12 +2455,12 @@ void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRo
     do {
       const int after = PARTS == 2 ? now : next_offset();
       request(after, PARTS - 1, 1, w_b);
-      multiply(now, 0, w_a);
+      multiply(now, 0, 0, w_a);
       landed(w_b);
       ldsBarrier();
       now = next_offset();
       request(now, 0, 0, w_a);
-      multiply(after, 1, w_b);
+      multiply(after, PARTS - 1, 1, w_b);
       landed(w_a);
       ldsBarrier();
     } while (now >= 0);
@@ -3980,9 +3996,15 @@ bool useTallKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &
   return !long_rows && p.K <= 32 && d.q_padded >= 64 && work >= (d.c_padded == 128 ? 50000 : 80000);
 }
 
-bool useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d) {
-  if (!denseShapeOk(p, d)) return false;
-  if (lc.choices.dense_tiles >= 0) return lc.choices.dense_tiles == 1;
+// Shapes of gatherConvDenseStaged that add up by offset.
+constexpr bool denseByOffsetShape(int elem_bytes, int Q, int C) { return elem_bytes == 2 && Q >= 64 && C >= 64; }
+
+// How the register-accumulating kernel adds up, if it is used: all products of a row in one chain, or each offset's by
+// itself, as the pair-list kernels do.
+enum class DenseSums { kNone, kChain, kByOffset };
+
+DenseSums useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d, bool lists) {
+  if (!denseShapeOk(p, d) || lc.choices.dense_tiles == 0) return DenseSums::kNone;
   // What the kernel costs goes with the (tile, offset) pieces that hold a pair at all, what
   // the pair-list kernels cost with the pairs.  Measured on 150000 rows, 3x3x3, as the share of all
   // (row, offset) slots that hold a pair from which the kernel wins, with us of the pair-list kernels
@@ -4018,18 +4040,37 @@ bool useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims 
   // (the largest count is the centre offset of a submanifold convolution: left out)
   const double mean_rest = p.K > 1 ? (pairs - largest) / (p.K - 1) : 0.0;
   const bool sheets = mean_rest > 0 && second >= 1.5 * mean_rest;
+  bool chain;
   if (p.dtype != ElemType::kFloat) {
-    if (sheets) return fill >= (d.q_padded >= 64 && d.c_padded == 64 ? 0.085 : 0.05);
-    return fill >= (d.q_padded <= 32 ? 0.17 : 0.27);
+    chain = fill >= (sheets ? (d.q_padded >= 64 && d.c_padded == 64 ? 0.085 : 0.05) : (d.q_padded <= 32 ? 0.17 : 0.27));
+  } else if (d.c_padded <= 32) {
+    chain = fill >= (sheets ? 0.06 : 0.35);
+  } else if (d.c_padded == 64) {
+    chain = fill >= (sheets ? 0.18 : 0.5);
+  } else {
+    chain = sheets && d.q_padded <= 32 && fill >= 0.2;
   }
-  if (d.c_padded <= 32) return fill >= (sheets ? 0.06 : 0.35);
-  if (d.c_padded == 64) return fill >= (sheets ? 0.18 : 0.5);
-  return sheets && d.q_padded <= 32 && fill >= 0.2;
+  // Fewer pairs, 2-byte rows of more than 64 bytes: with each offset's product by itself, which gives the pair-list
+  // kernels' bits, so that a layer's results do not depend on this line.  Filled sheets show less in a strided layer's
+  // counts, in which strewn voxels differ by a few per cent.  us of the pair-list kernels / this one, fp16, 3x3x3:
+  //   stride 2 on scenes, 0.18 to 0.20 filled (second count 1.11 to 1.27 of the mean)
+  //     64 -> 64    5 k rows 38/30   37 k 37/33   69 k 52/37   110 k 78/55   168 k 79/60
+  //     64 -> 128   11 k 34/37   19 k 35/37   37 k 46/43   69 k 68/50   168 k 119/82
+  //     128 -> 64   5 k 51/39   69 k 74/53   110 k 116/80       128 -> 128  11 k 48/49   37 k 66/64   69 k 96/84   110 k 142/107
+  //   strewn, or stride 2 on what layers have thickened (1.02 to 1.06)
+  //     64 -> 128   50 k rows 0.21 43/44   0.24 47/45   151 k 0.22 101/82   150 k 0.17 84/81   0.21 88/82   16 k 0.21 25/37
+  //     64 -> 64    125 k 0.20 51/58   150 k 0.21 61/60         128 -> 128  125 k 0.20 115/127   150 k 0.21 131/153
+  const bool uneven = second >= 1.1 * mean_rest;
+  const bool by_offset = !chain && lists && denseByOffsetShape((int)elemSize(p.dtype), d.q_padded, d.c_padded) &&
+                         fill >= 0.16 &&
+                         (uneven ? d.c_padded == 64 || d.R >= 30000 : d.q_padded == 64 && d.c_padded == 128 && d.R >= 50000);
+  if (by_offset) return DenseSums::kByOffset;
+  return chain || lc.choices.dense_tiles == 1 ? DenseSums::kChain : DenseSums::kNone;
 }
 
 template <typename E, int Q, int C, typename SRC>
 void launchDenseInstance(const LaunchCtx &lc, const void *A, uint32_t a_size, const ConvRows &rows,
-                         const void *packed, const SRC &source, int R, int K, void *result) {
+                         const void *packed, const SRC &source, bool by_offset, int R, int K, void *result) {
   auto launch = [&](auto kernel) {
     lc.begin("gatherConvDense");
     kernel<<<denseGridX(R), kDenseThreads, 0, lc.stream>>>(
@@ -4037,15 +4078,18 @@ void launchDenseInstance(const LaunchCtx &lc, const void *A, uint32_t a_size, co
         source, R, K, static_cast<typename E::storage *>(result));
     lc.end();
   };
-  if constexpr (Q * (int)sizeof(typename E::storage) > 64) launch(gatherConvDenseStaged<E, Q, C, SRC>);
+  if constexpr (SRC::kSegments && denseByOffsetShape((int)sizeof(typename E::storage), Q, C)) {
+    if (by_offset) return launch(gatherConvDenseStaged<E, Q, C, true, SRC>);
+  }
+  if constexpr (Q * (int)sizeof(typename E::storage) > 64) launch(gatherConvDenseStaged<E, Q, C, false, SRC>);
   else launch(gatherConvDense<E, Q, C, SRC>);
 }
 
 template <typename E, typename SRC>
 void launchDense(const LaunchCtx &lc, int q_padded, const void *A, int n_src, const ConvRows &rows,
-                 const void *packed, const SRC &source, int R, int K, void *result) {
+                 const void *packed, const SRC &source, bool by_offset, int R, int K, void *result) {
   const uint32_t a_size = (uint32_t)n_src * (uint32_t)rows.row_bytes;
-#define DENSE_INSTANCE(q, c) launchDenseInstance<E, q, c, SRC>(lc, A, a_size, rows, packed, source, R, K, result)
+#define DENSE_INSTANCE(q, c) launchDenseInstance<E, q, c, SRC>(lc, A, a_size, rows, packed, source, by_offset, R, K, result)
 #define DENSE_BY_C(q)                       \
   switch (rows.c_padded) {                  \
     case 16: DENSE_INSTANCE(q, 16); break;  \
@@ -4188,7 +4232,8 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
   // instead).  Worth it only where the row map is a single chunk of four launches.
   const bool speculate = p.list_trust == ListTrust::kUnknown && single_chunk && lc.choices.lists_on_trust != 0;
   const bool lists = use_mfma && listsUsable(p, d) && (p.list_trust == ListTrust::kInOrder || speculate);
-  const bool dense = use_mfma && useDenseKernel(lc, p, d);
+  const DenseSums dense_sums = use_mfma ? useDenseKernel(lc, p, d, lists) : DenseSums::kNone;
+  const bool dense = dense_sums != DenseSums::kNone;
   const bool tall = use_mfma && !dense && useTallKernel(lc, p, d, lists);
   const int tall_q = tallQ(p.dtype, d.q_padded);
   const int tall_rows = tall ? tallTileRows(lc, p, d, tall_q, lists) : 0;
@@ -4233,7 +4278,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     src.sC = sC;
     src.counts = inl;
     if (dense)
-      launchDense<E, SegmentSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, src, d.R, p.K, result);
+      launchDense<E, SegmentSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, src, dense_sums == DenseSums::kByOffset, d.R, p.K, result);
     else if (tall)
       launchTall<E, SegmentSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, src, tall_rows, d.R, p.K,
                                    result);
@@ -4276,7 +4321,8 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
       const MapSource map = {entries, ws.filled, run_if};
       if (dense) {
         n_filled = denseGridX(rows);
-        launchDense<E, MapSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, map, rows, p.K, result_rows);
+        launchDense<E, MapSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, map, false, rows, p.K,
+                                  result_rows);
       } else if (tall) {
         n_filled = tallGridX(rows, tall_rows);
         launchTall<E, MapSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, map, tall_rows, rows, p.K,
