@@ -21,11 +21,13 @@
 //  * gatherConvMfma   up to 128 channels on both sides, in MFMA blocks of 16 pairs.  Per offset the
 //    rows of a tile that have a partner are compacted, so MFMA work follows the number of
 //    pairs, not K x rows.  Each wave owns a column slice of the fp32 accumulator tile in LDS.
-//  * gatherConvTall   the same sums for rulebooks that are thinly filled: tiles of 256 or 512 rows by 64
+//  * gatherConvTall   the same sums for rulebooks that are thinly filled: tiles of 128 to 512 rows by 64
 //    columns, with waves that only fetch beside those that multiply.
 //  * gatherConvWave   the same for results of up to 32 columns, one wavefront a tile.
 //  * gatherConvDense  rulebooks whose (tile, offset) pieces are well filled: accumulators in
 //    registers, all rows of a tile multiplied at every offset that has a pair there.
+//    gatherConvDenseStaged  the same with rows above 64 bytes brought through LDS.
+//  * gatherConvSingle result rows in one pair each: the products of one offset's pairs, stored as they are.
 //  * gatherConvSimt   any channel count, LDS-tiled FMA.
 // A row takes nothing from the filter of an offset at which it has no pair, in any of them, also
 // where that filter is not finite.  Forward stores its sums behind a ReLU where the caller asks for it.
@@ -2229,10 +2231,10 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
 // 248 636 rows of a scene, 27 offsets, with the filter's packing, this kernel / filters through LDS with
 // rows in operand order (128) or through registers and LDS (64):
 //   fp16 128 -> 128 167/210    64 -> 64 82/95
-// OFFSETS: an offset's product is a chain of its own, added to the row's sum when it is whole, as the pair-list kernels
-// add: their bits (128 -> 128 takes the registers of two workgroups a CU for it; useDenseKernel has both sides' times).
 // Of two offsets a phase (64 channels: 93), tiles of 256 rows (128: 233; 64: 123), whole rows of 256 bytes (185),
 // quarters (181) and 32 columns a wave at 64 (86) none is faster.
+// OFFSETS: an offset's product is a chain of its own, added to the row's sum when it is whole, as the pair-list kernels
+// add: their bits (128 -> 128 takes the registers of two workgroups a CU for it; useDenseKernel has both sides' times).
 struct StagedPlan {
   int column_waves;   // waves side by side; the others are below each other
   int column_blocks;  // of 16 result columns, of a wave
@@ -3921,7 +3923,7 @@ bool useWaveKernel(const LaunchCtx &lc, ElemType t, int Q, int C) {
 // The register-accumulating kernel addresses the gathered tensor with 32-bit byte offsets: tensors of
 // 2 GiB and more take the pair-list kernels.
 bool denseShapeOk(const ConvProblem &p, const GatherDims &d) {
-  // (fp32 rows of more than 64 channels leave no room for two row groups a wave)
+  // (fp32 rows of more than 64 channels have no instance)
   if (p.dtype == ElemType::kFloat && d.Q > 64) return false;
   return (uint64_t)d.n_src * (uint64_t)paddedRowBytes(p.dtype, d.Q) < (uint64_t)kNoRow;
 }
@@ -4013,9 +4015,12 @@ DenseSums useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const Gather
   //   fp16   16 -> 16                  0.18 (0.15: 24/26, 0.27: 31/26)       0.045 (0.04: 18/19, 0.05: 23/19)
   //          32 -> 32                  0.18 (0.15: 28/31, 0.27: 36/30)       0.045 (0.04: 20/21, 0.05: 27/20)
   //          16, 32 -> 64              0.14 (0.13: 39/41, 0.18: 47/41)       0.06  (0.05: 31/29, 0.10: 46/32)
-  //          64 -> 64                  0.25 (0.22: 59/63, 0.27: 66/62)       0.09  (0.07: 39/47, 0.10: 52/48)
-  //          64 -> 128                 0.22 (0.18: 79/84, 0.27: 98/83)       0.05  (0.04: 51/56, 0.05: 59/54)
-  //          128 -> 128                0.27 (0.22: 132/149, 0.31: 165/150)   0.055 (0.04: 67/75, 0.07: 91/91)
+  // Rows of 2-byte types above 64 bytes, since they go through LDS, are ahead around 0.2 strewn and below 0.18 in thinned scenes;
+  // the lines stayed, so that no layer's sums changed, and below them each offset's product goes by itself (see below):
+  //          64 -> 64                  0.27 (0.26: 69/56, 0.31: 77/57)      0.085 (0.18: 50/46, 0.26: 74/54, 0.35: 121/72)
+  //          64 -> 128                 0.27 (0.26: 102/87, 0.31: 118/81)    0.05  (0.18: 77/59, 0.26: 109/72, 0.35: 178/96)
+  //          128 -> 64                 0.27 (0.26: 98/86, 0.31: 111/87)     0.085 (0.18: 70/70, 0.26: 109/80, 0.35: 187/110)
+  //          128 -> 128                0.27 (0.26: 149/131, 0.31: 170/133)  0.05  (0.18: 108/92, 0.26: 159/115, 0.35: 258/160)
   //   fp32   16 -> 16, 32              0.3  (0.22: 46/54, 0.4: 66/54)        0.05  (0.04: 26/31, 0.07: 49/38)
   //          32 -> 32                  0.4  (0.31: 81/95, 0.5: 114/95)       0.065 (0.05: 46/57, 0.10: 95/72)
   //          32 -> 64                  0.5  (0.4: 138/160, 0.5: 160/159)     0.15  (0.11: 111/125, 0.17: 138/129)
