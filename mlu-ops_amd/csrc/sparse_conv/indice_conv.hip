@@ -4246,9 +4246,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     // Pair lists in order (as far as the caller knows: the first kernel checks): the
     // gather kernel reads them cut by tile, no row map.
     const int tile_cols = dense ? d.c_padded : mfmaTileCols(p, d);
-    const int tile_rows = dense ? kDenseRows
-                          : tall ? tall_rows
-                                 : mfmaTileRows(tile_cols);
+    const int tile_rows = dense ? kDenseRows : tall ? tall_rows : mfmaTileRows(tile_cols);
     int tile_shift = 0;
     while ((1 << tile_shift) < tile_rows) ++tile_shift;
     const int n_tiles = (d.R + tile_rows - 1) / tile_rows;
@@ -4283,7 +4281,8 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     src.sC = sC;
     src.counts = inl;
     if (dense)
-      launchDense<E, SegmentSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, src, dense_sums == DenseSums::kByOffset, d.R, p.K, result);
+      launchDense<E, SegmentSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, src,
+                                    dense_sums == DenseSums::kByOffset, d.R, p.K, result);
     else if (tall)
       launchTall<E, SegmentSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, src, tall_rows, d.R, p.K,
                                    result);
@@ -4300,7 +4299,10 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
   // gather kernel for those rows, checked for lost pairs, and filled again for the next rows.
   int chunk_rows = own_map ? ws.map_rows : d.R;
   if (own_map && lc.choices.small_map_chunks == 1 && chunk_rows > kRepairPoolRows) chunk_rows = kRepairPoolRows;
-  const int tile_cols = use_mfma && !dense ? mfmaTileCols(p, d) : d.c_padded;
+  // (what goes by pair lists only: sums by offset, and tall tiles of another height than the row maps')
+  const bool map_dense = dense_sums == DenseSums::kChain;
+  const int map_tall_rows = tallRows(tall_q * (int)sizeof(S));
+  const int tile_cols = use_mfma && !map_dense ? mfmaTileCols(p, d) : d.c_padded;
   for (int row_base = 0; row_base < d.R; row_base += chunk_rows) {
     const int rows = d.R - row_base < chunk_rows ? d.R - row_base : chunk_rows;
     const size_t map_elems = (size_t)p.K * rows;
@@ -4324,13 +4326,13 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
       }
       if (own_map) n_accepted = launchScatterRowMap(lc, p, d, ws, inl, max_count, row_base, rows, run_if);
       const MapSource map = {entries, ws.filled, run_if};
-      if (dense) {
+      if (map_dense) {
         n_filled = denseGridX(rows);
         launchDense<E, MapSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, map, false, rows, p.K,
                                   result_rows);
       } else if (tall) {
-        n_filled = tallGridX(rows, tall_rows);
-        launchTall<E, MapSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, map, tall_rows, rows, p.K,
+        n_filled = tallGridX(rows, map_tall_rows);
+        launchTall<E, MapSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, map, map_tall_rows, rows, p.K,
                                  result_rows);
       } else {
         n_filled = mfmaGridX(rows, tile_cols);

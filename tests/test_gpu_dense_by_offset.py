@@ -60,3 +60,22 @@ def test_bits_of_the_pair_list_kernels(gpu_handle, ci, co, space, dtype_name, fi
         assert torch.equal(torch.isfinite(a), torch.isfinite(b)) and not bool(torch.isfinite(a).all())
         error = (a.double() - b.double())[:, keep].abs().max()
         assert float(error) <= 2.0 ** (-7 if dtype_name == "bfloat16" else -10) * float(b[:, keep].double().abs().max())
+
+
+def test_lists_that_are_not_in_order(gpu_handle):
+    """Pairs the library has not seen, out of order: taken in order on trust first, then by the row map."""
+    import torch
+    import mluop_hip as m
+    ks, ci, co = (3, 3, 3), 64, 64
+    idx = floors_and_walls(SMALL, 0.37, 5)
+    pairs, num, n_out = gpu_rulebook(gpu_handle, idx, 1, SMALL, ks, [1, 1, 1], [2, 2, 2], [1, 1, 1], False)
+    rng = np.random.default_rng(6)
+    x = torch.from_numpy(rng.standard_normal((idx.shape[0], ci)).astype(np.float32)).cuda().half()
+    w = torch.from_numpy((rng.standard_normal(ks + (ci, co)) / 40).astype(np.float32)).cuda().half()
+    host = pairs.cpu().numpy().copy()
+    for k, n in enumerate(num):
+        order = rng.permutation(n)
+        host[k, :, :n] = host[k][:, :n][:, order]
+    ref = m.indice_conv_forward(gpu_handle, x, w, m.LAYOUT_ARRAY, pairs, num, n_out, False)
+    out = m.indice_conv_forward(gpu_handle, x, w, m.LAYOUT_ARRAY, torch.from_numpy(host).cuda(), num, n_out, False)
+    assert torch.equal(out, ref)  # (no two pairs of an offset share a row: the sums' order is the offsets')
