@@ -6,6 +6,7 @@ import pytest
 
 from spconv_cases import round_to, to_torch
 from test_gpu_pair_lists import gpu_rulebook, kernels_of
+from test_gpu_tall_teams import with_and_without_a_wait
 
 pytestmark = pytest.mark.gpu
 
@@ -62,20 +63,18 @@ def test_bits_of_the_pair_list_kernels(gpu_handle, ci, co, space, dtype_name, fi
         assert float(error) <= 2.0 ** (-7 if dtype_name == "bfloat16" else -10) * float(b[:, keep].double().abs().max())
 
 
-def test_lists_that_are_not_in_order(gpu_handle):
-    """Pairs the library has not seen, out of order: taken in order on trust first, then by the row map."""
+def test_row_map_behind_lists_on_trust():
+    """Rows out of order: the row map's kernel adds in the same order, whether the host knew or launched on trust."""
     import torch
     import mluop_hip as m
-    ks, ci, co = (3, 3, 3), 64, 64
+    ks, channels = (3, 3, 3), 64
     idx = floors_and_walls(SMALL, 0.37, 5)
-    pairs, num, n_out = gpu_rulebook(gpu_handle, idx, 1, SMALL, ks, [1, 1, 1], [2, 2, 2], [1, 1, 1], False)
     rng = np.random.default_rng(6)
-    x = torch.from_numpy(rng.standard_normal((idx.shape[0], ci)).astype(np.float32)).cuda().half()
-    w = torch.from_numpy((rng.standard_normal(ks + (ci, co)) / 40).astype(np.float32)).cuda().half()
-    host = pairs.cpu().numpy().copy()
-    for k, n in enumerate(num):
-        order = rng.permutation(n)
-        host[k, :, :n] = host[k][:, :n][:, order]
-    ref = m.indice_conv_forward(gpu_handle, x, w, m.LAYOUT_ARRAY, pairs, num, n_out, False)
-    out = m.indice_conv_forward(gpu_handle, x, w, m.LAYOUT_ARRAY, torch.from_numpy(host).cuda(), num, n_out, False)
-    assert torch.equal(out, ref)  # (no two pairs of an offset share a row: the sums' order is the offsets')
+    idx = np.ascontiguousarray(idx[rng.permutation(len(idx))])
+    x = torch.from_numpy(rng.standard_normal((idx.shape[0], channels)).astype(np.float32)).cuda().half()
+    w = torch.from_numpy((rng.standard_normal(ks + (channels, channels)) / 40).astype(np.float32)).cuda().half()
+    ((want, known), (got, trusted)), fill = with_and_without_a_wait(m.make_handle_on_current_stream(), idx, SMALL, ks, 2, x, w)
+    assert 0.16 <= fill < 0.27, fill
+    assert "packFilterCutPairLists" not in known and "gatherConvDense" not in known, known
+    assert "packFilterCutPairLists" in trusted and trusted.count("gatherConvDense") == 1, trusted
+    assert torch.equal(got, want)

@@ -4,7 +4,8 @@ tiles, none and a few rows of them, and the fallback for lists that are not in o
 import numpy as np
 import pytest
 
-from spconv_cases import check_close, from_torch
+from spconv_cases import check_close, from_torch, random_voxels
+from test_gpu_pair_lists import kernels_of
 from test_gpu_tall_tiles import both_directions, check, make_case
 import sparse_conv_oracle as oracle
 
@@ -20,22 +21,16 @@ def test_bits_of_the_short_tiles(gpu_handle, ci, co, dtype_name, rows, space):
     check(gpu_handle, make_case(gpu_handle, rows, space, (3, 3, 5), ci, co, dtype_name, False), (True, True))
 
 
-@pytest.mark.parametrize("foreign", [False, True])
-def test_lists_that_are_not_in_order(gpu_handle, foreign):
-    """Pairs written over after the library saw them in order, and pairs it has not seen: those are taken in order on
-    trust, with the row map's kernels, whose tiles have another height, behind them."""
+def test_lists_that_are_not_in_order(gpu_handle):
     import torch
-    rows, space, ks, channels = 5000, (12, 24, 24), (3, 3, 5), 64  # (more than a grid rounded up to eight tiles covers)
+    rows, space, ks, channels = 1100, (8, 16, 16), (3, 3, 5), 64
     case = make_case(gpu_handle, rows, space, ks, channels, channels, "float16", False)
     pairs = case["pairs"].cpu().numpy().copy()
     rng = np.random.default_rng(3)
     for k, n in enumerate(case["num"]):
         order = rng.permutation(n)
         pairs[k, :, :n] = pairs[k][:, :n][:, order]
-    if foreign:
-        case["pairs"] = torch.from_numpy(pairs).cuda()
-    else:
-        case["pairs"].copy_(torch.from_numpy(pairs))
+    case["pairs"].copy_(torch.from_numpy(pairs))
     out, dx, ran = both_directions(gpu_handle, case, True)
     torch.cuda.synchronize()
     assert ran == (True, True)
@@ -44,3 +39,55 @@ def test_lists_that_are_not_in_order(gpu_handle, foreign):
     check_close(from_torch(out), ref, "float16", "tall teams")
     ref = oracle.backward_data(case["host"]["dy"], w_k, pairs, case["num"])
     check_close(from_torch(dx), ref, "float16", "tall teams")
+
+
+def with_and_without_a_wait(handle, idx, space, ks, stride, x, w):
+    """Forward on a rulebook whose report is there, and on one whose report is not: (result, kernels) of each.  Rows that are not
+    in order run over the row map then, behind list kernels that were launched on trust and return."""
+    import torch
+    import mluop_hip as m
+    sub_m = stride == 1
+    pad = [k // 2 for k in ks]
+    out_space = list(space) if sub_m else [(s + 2 * p - k) // stride + 1 for s, p, k in zip(space, pad, ks)]
+    idx = torch.from_numpy(idx).cuda()
+
+    def rulebook():
+        return m.get_indice_pairs(handle, idx, 1, space, ks, out_space, pad, [stride] * 3, [1, 1, 1], sub_m)
+
+    pairs, _, num, n_out = rulebook()
+    torch.cuda.synchronize()
+    num = [int(v) for v in num.cpu()]
+    got = [kernels_of(handle, lambda: m.indice_conv_forward(handle, x, w, m.LAYOUT_ARRAY, pairs, num, n_out, sub_m))]
+    torch.cuda.synchronize()
+    guard_bytes, m.GUARD_BYTES = m.GUARD_BYTES, 0  # (checked after a wait)
+    try:
+        busy = torch.ones((4096, 4096), device="cuda")
+
+        def call():
+            a = busy
+            for _ in range(6):  # a few milliseconds in front of the rulebook
+                a = (a @ a) * 1e-4
+            return m.indice_conv_forward(handle, x, w, m.LAYOUT_ARRAY, rulebook()[0], num, n_out, sub_m)
+        got.append(kernels_of(handle, call))
+        torch.cuda.synchronize()
+    finally:
+        m.GUARD_BYTES = guard_bytes
+    return got, sum(num) / n_out / len(num)
+
+
+def test_row_map_behind_lists_on_trust():
+    """The row map's tiles are of 256 rows (5000 rows: more than a grid for 512, rounded up to eight tiles, covers)."""
+    import torch
+    import mluop_hip as m
+    space, ks = (12, 24, 24), (3, 3, 5)
+    rng = np.random.default_rng(8)
+    idx = random_voxels(rng, 1, space, 5000, shuffle=True)
+    x = torch.from_numpy(rng.standard_normal((5000, 64)).astype(np.float32)).cuda().half()
+    w = torch.from_numpy((rng.standard_normal(ks + (64, 64)) / 50).astype(np.float32)).cuda().half()
+    handle = m.make_handle_on_current_stream()
+    handle.set_kernel_choice("dense_tiles", False)
+    handle.set_kernel_choice("tall_tiles", True)
+    ((want, known), (got, trusted)), _ = with_and_without_a_wait(handle, idx, space, ks, 1, x, w)
+    assert "packFilterCutPairLists" not in known and "gatherConvTall" in known, known
+    assert "packFilterCutPairLists" in trusted and trusted.count("gatherConvTall") == 2, trusted
+    assert torch.equal(got, want)
