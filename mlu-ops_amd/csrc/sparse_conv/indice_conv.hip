@@ -4477,13 +4477,13 @@ void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const S
     if constexpr (kTransposingShape) {
       // fp32 takes steps of 32 pairs, 2-byte types of 64, half as many barriers; with 128 channels on a side those
       // leave two or three workgroups' buffers on a CU, and where a workgroup has many steps the shorter ones, with
-      // four, are faster.  us with the sums, fp16, steps of 32 / 64, 3.0 M pairs: 32 x 32 55/39   32 x 64 62/50
+      // four, are faster (in walks: slices of 125 offsets, 1.6 M pairs, 128 x 128, 141/131).  us with the sums, fp16, steps of 32 / 64, 3.0 M pairs: 32 x 32 55/39   32 x 64 62/50
       // 64 x 64 67/57   32 x 128 73/83   64 x 128 89/100   128 x 128 135/142; 0.98 M pairs: 32 x 32 28/23   64 x 64 35/31
       // 64 x 128 43/41   128 x 128 67/59.  fp32, 0.98 M: 64 x 64 86/98   128 x 128 302/317
       auto tr = backwardFilterRows<E, CI, CO, 32, false>;
       if (whole) tr = backwardFilterRows<E, CI, CO, 32, true>;
       if constexpr (sizeof(S) == 2) {
-        const bool short_steps = (CI == 128 || CO == 128) && slice_len >= 2048;
+        const bool short_steps = (CI == 128 || CO == 128) && shares > 0 && slice_len >= 2048;
         if (!short_steps) tr = whole ? backwardFilterRows<E, CI, CO, 64, true> : backwardFilterRows<E, CI, CO, 64, false>;
       }
       if (transposing)
