@@ -656,6 +656,14 @@ Workspace carve(void *base, const VoxelizeShape &s) {
   w.wide_counts = words(3 * n);
   w.wide_firsts = words(3 * n);
   w.total = off + 256;
+  if (!few) {
+    // a workspace that is large enough for a cloud is so for every smaller one, also across the line above, below
+    // which the tags and flags come on top (65 536 points need what 67 300 would)
+    VoxelizeShape most_few = s;
+    most_few.num_points = kFewPoints;
+    const size_t few_total = carve(nullptr, most_few).total;
+    if (w.total < few_total) w.total = few_total;
+  }
   return w;
 }
 

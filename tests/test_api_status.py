@@ -376,6 +376,23 @@ def test_voxelization_null_arguments(handle):
     free_descs(*descs)
 
 
+def test_voxelization_workspace_of_a_larger_cloud(handle):
+    """A workspace made for the largest cloud serves every smaller one, on either side of the line between the
+    voxelizer's two ways (65 536 points)."""
+    f, i = "MLUOP_DTYPE_FLOAT", "MLUOP_DTYPE_INT32"
+    last = 0
+    for n in [1, 2, 63, 64, 65, 4095, 4096, 8191, 8192, 8193, 60000, 65535, 65536, 65537,
+              *range(65540, 70000, 9), 200000]:
+        descs = [make_desc(T("MLUOP_LAYOUT_ARRAY", dt, d)) for dt, d in
+                 ((f, [n, 4]), (f, [3]), (f, [6]), (f, [50, 3, 4]), (i, [50, 3]), (i, [50]), (i, [1]))]
+        size = ctypes.c_size_t(0)
+        assert m.lib().mluOpGetVoxelizationWorkspaceSize(handle.ptr, descs[0], descs[1], descs[2], 3, 50, 3, True,
+                                                         descs[3], descs[4], descs[5], descs[6], ctypes.byref(size)) == 0
+        assert size.value >= last, (n, size.value, last)
+        last = size.value
+        free_descs(*descs)
+
+
 def test_dynamic_point_to_voxel_forward_null_arguments(handle):
     """api_gtest/src/gtest/dynamic_point_to_voxel_forward/dynamic_point_to_voxel_forward.cpp:326-500 and
     dynamic_point_to_voxel_forward_workspace.cpp:101-140."""
