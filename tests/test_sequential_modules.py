@@ -52,6 +52,24 @@ class Cached(spnn.SparseSequential):
         return x
 
 
+class Given(spnn.SubMConv3d):
+    """A layer with a way of its own to come to its rulebook."""
+
+    def _rulebook(self, x):
+        return x.rulebooks["given"]
+
+
+@pytest.mark.parametrize("how", ["class", "instance"])
+def test_a_layers_own_rulebook_is_asked_for(how, monkeypatch):
+    monkeypatch.setattr(spnn._IndiceConv, "apply", staticmethod(lambda features, weight, rb, *a, **k: features + rb))
+    x = empty_tensor()
+    x.rulebooks["given"] = 3.0
+    layer = Given(16, 16, 3) if how == "class" else spnn.SubMConv3d(16, 16, 3)
+    if how == "instance":
+        layer._rulebook = lambda x: x.rulebooks["given"]
+    assert torch.equal(layer(x).features, x.features + 3.0)
+
+
 def empty_tensor():
     return spnn.SparseTensor(torch.zeros(2, 16), torch.zeros(2, 4, dtype=torch.int32), (4, 4, 4), 1)
 
