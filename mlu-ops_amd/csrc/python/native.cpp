@@ -11,6 +11,7 @@
 #include <torch/extension.h>
 
 #include <ATen/hip/HIPContext.h>
+#include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <dlfcn.h>
 
@@ -35,6 +36,7 @@ namespace {
 #define MLUOP_NATIVE_FUNCTIONS(X)                          \
   X(mluOpCreate)                                           \
   X(mluOpSetQueue)                                         \
+  X(mluOpGetQueue)                                         \
   X(mluOpGetErrorString)                                   \
   X(mluOpCreateTensorDescriptor)                           \
   X(mluOpSetTensorDescriptor_v2)                           \
@@ -455,6 +457,12 @@ StreamHandle &streamHandle() {
   return h;
 }
 
+bool isStreamHandle(mluOpHandle_t handle) {
+  StreamHandles &all = streamHandles();
+  const std::lock_guard<std::mutex> lock(all.mutex);
+  return all.by_handle.count(handle) > 0;
+}
+
 // Held for one operator on `handle`, without the GIL (a buffer in guard mode takes it).
 class OperatorLock {
  public:
@@ -471,6 +479,24 @@ class OperatorLock {
  private:
   std::unique_lock<std::mutex> lock_;
 };
+
+// The pair counts of a rulebook built on `handle` (held by the caller), in `indice_num` on the device: as soon as they
+// are there, or, where they are no longer on file (the handle keeps 32 rulebooks) or too many, behind what the
+// rulebook's own stream holds.  (A handle of the caller's own may have been given another stream since.)
+Counts takeHostCounts(mluOpHandle_t handle, const at::Tensor &pairs, const at::Tensor &indice_num) {
+  Counts counts;
+  if (hostCounts(handle, pairs, &counts)) return counts;
+  mluOpQueue_t queue = nullptr;
+  check(api.mluOpGetQueue(handle, &queue), "mluOpGetQueue");
+  const c10::hip::HIPStreamGuard own(
+      c10::hip::getStreamFromExternal(reinterpret_cast<hipStream_t>(queue), pairs.device().index()));
+  if (!isStreamHandle(handle) && hipDeviceSynchronize() != hipSuccess)
+    throw std::runtime_error("waiting for a rulebook's pair counts failed");
+  const at::Tensor host = indice_num.cpu();
+  const int32_t *n = host.data_ptr<int32_t>();
+  counts.assign(n, n + host.numel());
+  return counts;
+}
 
 // ---- the layers' autograd node -------------------------------------------------------------
 
@@ -555,16 +581,7 @@ struct LayerRulebook : torch::CustomClassHolder {
   void takeCounts(mluOpHandle_t built_on) {
     const std::lock_guard<std::mutex> lock(counts_mutex_);
     if (!pending_.load(std::memory_order_relaxed)) return;
-    Counts counts;
-    if (!hostCounts(built_on, pairs, &counts)) {
-      // no longer on file (the handle keeps 32 rulebooks), or too many offsets
-      const c10::DeviceGuard guard(pairs.device());
-      if (hipDeviceSynchronize() != hipSuccess) throw std::runtime_error("waiting for a rulebook's pair counts failed");
-      const at::Tensor host = indice_num_.cpu();
-      const int32_t *n = host.data_ptr<int32_t>();
-      counts.assign(n, n + host.numel());
-    }
-    counts_ = std::move(counts);
+    counts_ = takeHostCounts(built_on, pairs, indice_num_);
     pending_.store(false, std::memory_order_release);
   }
 
@@ -824,12 +841,10 @@ PYBIND11_MODULE(_native, m) {
           py::object num = counted ? py::cast(r.counts) : py::cast(r.indice_num);
           return py::make_tuple(r.pairs, r.out_indices, num, r.num_act_out);
         });
-  m.def("rulebook_counts", [](uintptr_t handle, const at::Tensor &pairs) -> std::optional<Counts> {
+  m.def("rulebook_counts", [](uintptr_t handle, const at::Tensor &pairs, const at::Tensor &indice_num) {
     NoGil released;
     const OperatorLock lock(asHandle(handle));
-    Counts counts;
-    if (!hostCounts(asHandle(handle), pairs, &counts)) return std::nullopt;
-    return counts;
+    return takeHostCounts(asHandle(handle), pairs, indice_num);
   });
   m.def("indice_conv_forward",
         [](uintptr_t handle, bool guarded, const at::Tensor &features, const at::Tensor &filters, int layout,

@@ -483,12 +483,9 @@ def get_indice_pairs(handle, indices, batch, input_space, filter_space, output_s
 
 def rulebook_counts(handle, indice_pairs, indice_num):
     """Host ints of a rulebook that get_indice_pairs(..., for_layer=True, wait_counts=False) has built on `handle`,
-    as soon as its last kernel has stored them."""
-    counts = native().rulebook_counts(handle.ptr.value, indice_pairs)
-    if counts is None:  # no longer on file (the handle keeps 32 rulebooks), or too many offsets
-        _torch().cuda.synchronize(indice_num.device)
-        counts = indice_num.tolist()
-    return counts
+    as soon as its last kernel has stored them; where they are no longer on file (the handle keeps 32 rulebooks), or are
+    too many, copied behind what the rulebook's stream holds."""
+    return native().rulebook_counts(handle.ptr.value, indice_pairs, indice_num)
 
 
 def _ints(values):

@@ -65,6 +65,38 @@ def test_on_another_stream():
     torch.cuda.current_stream().wait_stream(other)
 
 
+@pytest.mark.parametrize("asked_by", ["operator", "python"])
+@pytest.mark.parametrize("why", ["too many offsets", "no longer on file"])
+def test_counts_that_are_copied_wait_for_no_other_stream(asked_by, why):
+    import torch
+    from mluop_hip import nn as spnn
+    idx = torch.from_numpy(random_voxels(np.random.default_rng(3), 1, SPACE, 500)).cuda()
+    x = spnn.SparseTensor(torch.randn(500, 8, device="cuda"), idx, SPACE, 1, distinct=True)
+    size = 9 if why == "too many offsets" else 3  # (the handle keeps 343 counts of a rulebook)
+    layer = spnn.SubMConv3d(8, 16, size).cuda()
+    with torch.no_grad():
+        want = layer(spnn.SparseTensor(x.features, idx, SPACE, 1, distinct=True)).features
+        rb = pending(layer, x)
+        if why == "no longer on file":
+            for _ in range(40):
+                pending(spnn.SubMConv3d(8, 16, 3), spnn.SparseTensor(x.features, idx, SPACE, 1, distinct=True))
+        torch.cuda.synchronize()
+        a, busy = torch.ones(4096, 4096, device="cuda"), torch.cuda.Stream()
+        busy.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(busy):
+            for _ in range(200):  # about 1 ms each
+                b = a @ a
+            done = busy.record_event()
+        if asked_by == "operator":
+            got = layer(x).features
+        else:
+            assert rb.indice_num[size ** 3 // 2] == 500
+        assert not done.query(), "waited for a stream that has nothing to do with the rulebook"
+        assert asked_by == "python" or torch.equal(got, want)
+        torch.cuda.synchronize()
+        del b
+
+
 def test_from_several_threads():
     import torch
     for seed in range(5):
