@@ -532,6 +532,15 @@ struct LayerRulebook : torch::CustomClassHolder {
     takeCounts(built_on_);
   }
 
+  // The same for a caller who holds no lock.
+  const Counts &takenCounts() {
+    if (pending_.load(std::memory_order_acquire)) {
+      const OperatorLock lock(built_on_);
+      takeCounts(built_on_);
+    }
+    return counts_;
+  }
+
   ~LayerRulebook() override {
     for (const auto &[key, map] : row_maps_)
       if (map.defined()) key.first->forgetRowMap(map.data_ptr());
@@ -943,6 +952,10 @@ PYBIND11_MODULE(_native, m) {
            py::arg("pairs"), py::arg("counts"), py::arg("num_act_out"), py::arg("filter_space"), py::arg("sub_m"),
            py::arg("distinct"), py::arg("single") = false, py::arg("indice_num") = std::nullopt, py::arg("built_on") = 0,
            "With counts None, `indice_num` holds them on the device and the handle at `built_on` has built the rulebook.")
+      .def("counts", [](const LayerRulebookPtr &rulebook) {
+        NoGil released;
+        return rulebook->takenCounts();
+      }, "The pair counts, waited for unless a call has taken them.")
       .def("row_maps", &LayerRulebook::rowMaps, "(handle, pair column) of the row maps its calls have built.");
   m.def("indice_conv", [](const at::Tensor &features, const at::Tensor &weight, const LayerRulebookPtr &rulebook,
                           bool inverse, bool share_row_maps, bool guarded, bool relu) {

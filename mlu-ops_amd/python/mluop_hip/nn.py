@@ -90,7 +90,9 @@ class Rulebook:
     def indice_num(self):
         num = self._indice_num
         if isinstance(num, torch.Tensor):
-            self._indice_num = num = rulebook_counts(self._built_on, self._pairs, num)
+            # (an operator may have taken them: the handle need not have them on file any more)
+            self._indice_num = num = (rulebook_counts(self._built_on, self._pairs, num) if self._for_operators is None
+                                      else self._for_operators.counts())
         return num
 
     @indice_num.setter

@@ -97,6 +97,28 @@ def test_counts_that_are_copied_wait_for_no_other_stream(asked_by, why):
         del b
 
 
+def test_counts_that_an_operator_took_are_not_asked_for_again():
+    """Neither behind other rulebooks' nor while a graph is captured, which allows no wait."""
+    import torch
+    from mluop_hip import nn as spnn
+    layer, x, want, grads = setup(3000)
+    rb = pending(layer, x)
+    check(layer, x, want, grads)
+    for _ in range(40):
+        pending(spnn.SubMConv3d(8, 16, 3), spnn.SparseTensor(x.features, x.indices, SPACE, 1, distinct=True))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        pairs = rb.pairs
+    counts = rb.indice_num
+    assert counts[13] == 3000 and isinstance(counts, list)
+    for _ in range(3):
+        pairs.fill_(7)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all((p[:, n:] == -1).all() and (p[:, :n] == 7).all() for p, n in zip(pairs, counts))
+
+
 def test_from_several_threads():
     import torch
     for seed in range(5):
