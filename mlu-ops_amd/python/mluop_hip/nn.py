@@ -335,13 +335,19 @@ class SparseSequential(torch.nn.Sequential):
             if isinstance(m, SparseSequential):
                 # (a plan of the network's own is asked for as it is)
                 own = type(m).plan is not _SEQUENTIAL_PLAN or "plan" in m.__dict__
+                if own:  # (it may build any number)
+                    for rb in built:
+                        rb.indice_num
                 cells = m.plan(cells) if own else m._plan(cells, built)
             elif isinstance(m, _ConvBase):
                 if type(m) in (SubMConv3d, SparseConv3d):
                     rb = m._rulebook(cells, wait_counts=False)
-                    built.append(rb)
                 else:
                     rb = m._rulebook(cells)
+                if isinstance(rb, Rulebook) and rb not in built:
+                    built.append(rb)
+                    if len(built) > _PENDING:
+                        built[-1 - _PENDING].indice_num
                 indices, space, distinct = m._cells_after(cells, rb)
                 if indices is not cells.indices:
                     # (features are not looked at while planning: a view of the right height)
@@ -356,6 +362,9 @@ class SparseSequential(torch.nn.Sequential):
             built = []
             try:
                 self._plan(x, built)
+                for rb in built:
+                    if len(rb._pairs) > _COUNTED:
+                        rb.indice_num
             except BaseException:
                 for rb in built:
                     rb.indice_num
@@ -377,6 +386,10 @@ class SparseSequential(torch.nn.Sequential):
 
 
 _SEQUENTIAL_PLAN = SparseSequential.plan
+# How many rulebooks of a plan may have their pair counts outstanding, and of how many offsets: a handle has those of 32
+# rulebooks of up to 343 on file, and others are copied, behind whatever convolutions are enqueued by then (40 layers:
+# the device was drained eight times).
+_PENDING, _COUNTED = 16, 343
 
 
 class Voxelization(torch.nn.Module):

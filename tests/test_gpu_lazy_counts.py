@@ -119,6 +119,71 @@ def test_counts_that_an_operator_took_are_not_asked_for_again():
         assert all((p[:, n:] == -1).all() and (p[:, :n] == 7).all() for p, n in zip(pairs, counts))
 
 
+def watch(seen):
+    """Notes copies to the host and layers' results in the order in which they are made."""
+    import torch
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            result = func(*args, **(kwargs or {}))
+            if isinstance(result, torch.Tensor):
+                if result.device.type == "cpu" and isinstance(args[0], torch.Tensor) and args[0].is_cuda:
+                    seen.append("copy")
+                elif func is torch.ops.aten.empty.memory_format and result.dtype == torch.float32:
+                    seen.append("result")
+            return result
+    return Watch()
+
+
+def many_layers(layers, form, size=lambda i: 3):
+    import torch
+    from mluop_hip import nn as spnn
+    torch.manual_seed(0)
+    idx = torch.from_numpy(random_voxels(np.random.default_rng(1), 1, SPACE, 900)).cuda()
+    feats = torch.randn(900, 8, device="cuda")
+    convs = [spnn.SubMConv3d(8, 8, size(i)).cuda() for i in range(layers)]
+    inner = type("Inner", (Planned, spnn.SparseSequential), {}) if form.endswith("own") else spnn.SparseSequential
+    net = spnn.SparseSequential(*convs) if form == "flat" else spnn.SparseSequential(*convs[:5], inner(*convs[5:]))
+    return net, convs, feats, lambda: spnn.SparseTensor(feats, idx, SPACE, 1, distinct=True)
+
+
+class Planned:
+    """A network's own plan (put in front of SparseSequential below)."""
+
+    def plan(self, x):
+        return super().plan(x)
+
+
+@pytest.mark.parametrize("layers", [11, 33, 40])
+@pytest.mark.parametrize("form", ["flat", "nested", "nested with a plan of its own"])
+def test_networks_of_many_rulebooks_copy_no_counts(layers, form):
+    """A handle keeps the counts of 32 rulebooks: they are all taken before they leave."""
+    import torch
+    net, convs, feats, tensor = many_layers(layers, form)
+    seen = []
+    with torch.no_grad():
+        want = tensor()
+        for conv in convs:
+            want = conv(want)
+        torch.cuda.synchronize()
+        with watch(seen):
+            assert torch.ones(3, device="cuda").cpu().shape == (3,) and "copy" in seen  # (it sees them)
+            seen.clear()
+            got = net(tensor())
+    assert "copy" not in seen and seen.count("result") == layers, seen
+    assert torch.equal(got.features, want.features)
+
+
+def test_counts_of_many_offsets_are_copied_in_front_of_the_convolutions():
+    import torch
+    net, convs, feats, tensor = many_layers(6, "flat", lambda i: 9 if i % 2 else 3)
+    seen = []
+    with torch.no_grad(), watch(seen):
+        net(tensor())
+    assert seen == ["copy"] * 3 + ["result"] * 6
+
+
 def test_from_several_threads():
     import torch
     for seed in range(5):
