@@ -86,12 +86,14 @@ mluOpStatus_t MLUOP_WIN_API mluOpExtSetSparseConvExtendedModes(mluOpHandle_t han
  * all but one of such pairs.  Off by default. */
 mluOpStatus_t MLUOP_WIN_API mluOpExtSetDistinctPairsPromise(mluOpHandle_t handle, int promised);
 
-/* A caller can promise that one pair column (0 or 1) names no row twice, over all offsets together: the input rows
- * of a strided layer whose kernel reaches no further than its stride are in one pair each.
- * mluOpIndiceConvolutionForward and mluOpIndiceConvolutionBackwardData calls whose result rows that column names
- * then multiply full tiles of pairs and store the products, with nothing to add up; a rulebook that breaks the
- * promise keeps one pair's product in such a row.  -1, the value of a new handle: no promise.  Holds until
- * changed; the second call says which is in force. */
+/* A caller can promise that one pair column (0 or 1) names rows of the result only and none of them twice, over all
+ * offsets together: the input rows of a strided layer whose kernel reaches no further than its stride are in
+ * one pair each.  mluOpIndiceConvolutionForward and mluOpIndiceConvolutionBackwardData calls whose result rows
+ * that column names then multiply full tiles of pairs and store the products, with nothing to add up.  Rows in no pair
+ * are zero, and so is the row of a pair whose other column names no row.  Where a rulebook breaks the promise, a row
+ * named twice may hold any mixture of its pairs' products, from run to run another, and a row in no pair may keep what
+ * the memory held before.  -1, the value of a new handle: no promise.  Holds until changed; the second call
+ * says which is in force. */
 mluOpStatus_t MLUOP_WIN_API mluOpExtSetSinglePairsPromise(mluOpHandle_t handle, int column);
 mluOpStatus_t MLUOP_WIN_API mluOpExtGetSinglePairsPromise(mluOpHandle_t handle, int *column);
 

@@ -2519,7 +2519,7 @@ __global__ __launch_bounds__(kDenseThreads) void gatherConvSingle(
   constexpr int RPL = 1024 / RB;  // rows a load of 1 KiB stages
   constexpr int LPG = 16 / RPL;
   __shared__ __attribute__((aligned(1024))) char s_rows[T * RB];
-  __shared__ uint32_t s_src[T];  // where a pair's gathered row begins, or kNoRow
+  __shared__ uint32_t s_src[T];  // where a pair's gathered row begins; kNoRow: the pair adds nothing
   __shared__ int s_row[T];       // its result row, or -1
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -2538,9 +2538,8 @@ __global__ __launch_bounds__(kDenseThreads) void gatherConvSingle(
       row = list[(size_t)row_col * L];
       src = list[(size_t)src_col * L];
     }
-    const bool there = (unsigned)row < (unsigned)R && (unsigned)src < (unsigned)n_src;
-    s_src[tid] = there ? (uint32_t)src * (uint32_t)conv.row_bytes : kNoRow;
-    s_row[tid] = there ? row : -1;
+    s_src[tid] = (unsigned)src < (unsigned)n_src ? (uint32_t)src * (uint32_t)conv.row_bytes : kNoRow;
+    s_row[tid] = (unsigned)row < (unsigned)R ? row : -1;
   }
   const int first_group = wave / CW * G, first_block = wave % CW * NB;
   const char *const filter =
@@ -2581,6 +2580,7 @@ __global__ __launch_bounds__(kDenseThreads) void gatherConvSingle(
     for (int kb = 0; kb < KB; ++kb)
       row[kb] = *reinterpret_cast<const vec8 *>(rows + singlePieceAt(RB, pair, kb * 4 + quad) * 16);
     const int to = s_row[in_tile];
+    const bool adds = s_src[in_tile] != kNoRow;  // (a row of zeros times a filter that is not finite is not zero)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
       float4v product = {0.f, 0.f, 0.f, 0.f};
@@ -2591,7 +2591,7 @@ __global__ __launch_bounds__(kDenseThreads) void gatherConvSingle(
       // (a sum that starts from zero, as in the other kernels: a product of -0 is stored as 0)
       S tmp[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) E::store(&tmp[e], activated(0.f + product[e], conv.relu));
+      for (int e = 0; e < 4; ++e) E::store(&tmp[e], activated(adds ? 0.f + product[e] : 0.f, conv.relu));
       storeColumns<E>(result + (size_t)to * conv.c, (first_block + nb) * 16 + quad * 4, conv.c, tmp);
     }
   }

@@ -72,6 +72,51 @@ def test_same_numbers_as_without_the_promise(gpu_handle, rows, ks, stride, dtype
     assert ((ref.double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("relu", [False, True])
+@pytest.mark.parametrize("dtype_name,q,c", [("float16", 64, 96), ("float32", 40, 24), ("bfloat16", 128, 128)])
+@pytest.mark.parametrize("finite", [True, False])
+def test_partners_out_of_range_give_zero_rows(gpu_handle, dtype_name, q, c, finite, relu):
+    """Every row is in a pair, so that nothing clears the result, and some pairs' other row does not exist.  (The
+    kernel looks at every index before it uses it.)"""
+    import torch
+    import mluop_hip as m
+    rows, ks, stride = 1500, (1, 1, 1), (1, 1, 1)
+    pairs, counts, n_out = rulebook(gpu_handle, rows, ks, stride)
+    assert counts == [rows] and n_out == rows
+    out_of_range = {3: -1, 64: n_out, 200: 1 << 30, 1499: -(1 << 31)}
+    for at, value in out_of_range.items():
+        pairs[0, 1, at] = value
+    bad = pairs[0, 0, list(out_of_range)].long()
+    dtype = getattr(torch, dtype_name)
+    x = torch.randn((n_out, q), device="cuda").to(dtype)
+    w = torch.randn((1, 1, 1, q, c), device="cuda").to(dtype)
+    if not finite:
+        w[0, 0, 0, 5, 7], w[0, 0, 0, 6, 1] = float("inf"), float("nan")
+    gpu_handle.set_extended_modes(True)
+    gpu_handle.promise_single_pairs(0)
+    gpu_handle.set_forward_relu(relu)
+    try:
+        torch.full((rows, c), 7.0, device="cuda", dtype=dtype)  # (what the allocator hands out next is not zero)
+        got = m.indice_conv_forward(gpu_handle, x, w, m.LAYOUT_ARRAY, pairs, counts, rows, False, inverse=1)
+    finally:
+        gpu_handle.set_forward_relu(False)
+        gpu_handle.promise_single_pairs(None)
+        gpu_handle.set_extended_modes(False)
+    assert (got[bad] == 0).all()
+    good = torch.ones(rows, dtype=torch.bool, device="cuda")
+    good[bad] = False
+    partner = torch.zeros(rows, dtype=torch.int64, device="cuda")
+    keep = good[pairs[0, 0].long()]
+    partner[pairs[0, 0].long()[keep]] = pairs[0, 1].long()[keep]
+    want = x[partner].double() @ w[0, 0, 0].double()
+    want = want.clamp(min=0) if relu else want
+    size = x[partner].double().abs() @ w[0, 0, 0].double().abs()
+    rounding = {"float16": 2.0 ** -11, "bfloat16": 2.0 ** -8, "float32": 2.0 ** -24}[dtype_name]
+    ok = (got.double() - want).abs() <= 2.0 ** -24 * q * size + rounding * want.abs() + 2.0 ** -25
+    same = (got.double() == want) | (got.isnan() & want.isnan())  # (infinities and NaN)
+    assert (ok | same)[good].all()
+
+
 def test_relu_in_the_store(gpu_handle):
     import torch
     import mluop_hip as m
