@@ -3254,6 +3254,12 @@ __device__ __forceinline__ int floatStepPlace(int row_bytes, int q, int kq) {
 
 // Waves are laid out 2 x 2 over the blocks of dW[k], each with every second block of a side, so that the two waves of a
 // side share the blocks that a row has.
+// The place of a row that is not there: behind the end of every tensor (transposingReads) and, with a row's
+// pieces added, below 2^32, so that the tensors may be twice as long as the gathered ones of the kernels above (2-byte output
+// gradients of more than 2 GiB, which the kernel that stages rows through registers would take: 128 x 128 channels,
+// 3.0 M pairs, 331 us, this one 224).
+constexpr uint32_t kNoPlace = 0xfffffe00u;
+
 template <typename E, int CI, int CO, int SP, bool WHOLE>
 __global__ __launch_bounds__(256) void backwardFilterRows(
     const typename E::storage *X, const typename E::storage *dY, FilterGradRows lengths, const int32_t *pairs, int L,
@@ -3278,7 +3284,7 @@ __global__ __launch_bounds__(256) void backwardFilterRows(
 
   __shared__ __attribute__((aligned(1024))) char s_x[2][SP * RBX];
   __shared__ __attribute__((aligned(1024))) char s_y[2][SP * RBY];
-  // where the x rows and the y rows of a chunk of pairs begin, and of the chunk after; kNoRow: a pair that is not there
+  // where the x rows and the y rows of a chunk of pairs begin, and of the chunk after; kNoPlace: a pair that is not there
   __shared__ __attribute__((aligned(1024))) uint32_t s_at[2][2][kIndexChunk];
 
   const FilterRun run = runOfWorkgroup(tab, order, total_slices, slice_len, shares);
@@ -3324,7 +3330,7 @@ __global__ __launch_bounds__(256) void backwardFilterRows(
     const int pair = kFloat ? floatRowSlot(row_bytes, slot) : slot;
     const int moved = kFloat ? floatRowChunk(row_bytes, pair) * 4 : filterRowSwizzle(row_bytes, pair);
     piece[u] = (uint32_t)((byte % row_bytes / 16) ^ moved) * 16u;
-    if (piece[u] >= (of_x[u] ? x_length : y_length)) piece[u] = kNoRow;
+    if (piece[u] >= (of_x[u] ? x_length : y_length)) piece[u] = kNoPlace;
     pair_of[u] = (of_x[u] ? 0 : kIndexChunk) + pair;
   }
   auto request_step = [&](int step, int buffer) {
@@ -3334,7 +3340,8 @@ __global__ __launch_bounds__(256) void backwardFilterRows(
     for (int u = 0; u < MOST; ++u) at[u] = at_step[pair_of[u]];
 #pragma unroll
     for (int u = 0; u < MOST; ++u) {
-      at[u] = __builtin_elementwise_add_sat(at[u], piece[u]);
+      // (a piece behind the row's end is nowhere, wherever the row begins)
+      at[u] = WHOLE ? at[u] + piece[u] : __builtin_elementwise_min(__builtin_elementwise_add_sat(at[u], piece[u]), kNoPlace);
       asm volatile("" : "+v"(at[u]));
     }
 #pragma unroll
@@ -3427,8 +3434,8 @@ __global__ __launch_bounds__(256) void backwardFilterRows(
     uint32_t &in = s_at[chunk & 1][0][tid], &out = s_at[chunk & 1][1][tid];
     const uint32_t i = in, o = out;
     const bool there = run.at(chunk * kIndexChunk + tid) < run.end && i < (uint32_t)n_in && o < (uint32_t)n_out;
-    in = there ? i * x_length : kNoRow;
-    out = there ? o * y_length : kNoRow;
+    in = there ? i * x_length : kNoPlace;
+    out = there ? o * y_length : kNoPlace;
   };
 
   const int steps = run.length / SP;
@@ -4432,11 +4439,11 @@ GradLayout gradLayout(const ConvProblem &p) {
 // Rows that the backward filter reads into LDS as they are: 2-byte operands are transposed by LDS reads, fp32 ones need
 // no transposition.
 bool transposingReads(const LaunchCtx &lc, const ConvProblem &p) {
-  // (rows are addressed with 32-bit byte offsets)
+  // (rows are addressed with 32-bit byte offsets; the API's tensors have less than 2^31 elements)
   const uint64_t x_bytes = (uint64_t)(p.inverse ? p.num_out : p.L) * (uint64_t)p.Ci * elemSize(p.dtype);
   const uint64_t y_bytes = (uint64_t)(p.inverse ? p.L : p.num_out) * (uint64_t)p.Co * elemSize(p.dtype);
   return p.Ci > 16 && p.Co > 16 && lc.choices.filter_stores != 1 && !rowsNeedPadding(p.dtype, p.Ci) &&
-         !rowsNeedPadding(p.dtype, p.Co) && x_bytes < kNoRow && y_bytes < kNoRow;
+         !rowsNeedPadding(p.dtype, p.Co) && x_bytes <= kNoPlace && y_bytes <= kNoPlace;
 }
 
 // Workgroups of the walks (walkOfWorkgroup), 0: slices.  As many as are resident at a time, so that all
