@@ -425,10 +425,12 @@ def mean_voxel_features(voxels, num_points_per_voxel):
 def _mean_by_library(voxels, counts):
     """Whether the library's kernel takes the means (one launch in place of four; voxelizer and 11-layer encoder, 120 000
     voxels: 746 -> 713 us): what it accepts, on the current device, without a gradient to record and no mode that
-    watches torch's calls."""
+    watches torch's calls.  It sums a voxel's points one after the other, torch's reduction of many points side by
+    side.  us, torch / the library: 1000 voxels of 64 features, 100 points 22/8, 200 points 24/34, 400 34/66; 10 000 of 4
+    features, 100 points 22/9, 128 20/16, 200 23/30; 30 of 16 features, 1000 points 26/61, 4000 35/635."""
     return (type(voxels) is torch.Tensor and type(counts) is torch.Tensor and voxels.is_cuda and counts.is_cuda and
             voxels.dtype == torch.float32 and counts.dtype == torch.int32 and voxels.dim() == 3 and counts.dim() == 1 and
-            counts.shape[0] == voxels.shape[0] and 0 < voxels.numel() < 1 << 31 and
+            voxels.shape[1] <= 128 and counts.shape[0] == voxels.shape[0] and 0 < voxels.numel() < 1 << 31 and
             voxels.is_contiguous() and counts.is_contiguous() and not voxels.is_conj() and not voxels.is_neg() and
             voxels.device.index == torch.cuda.current_device() and counts.device == voxels.device and
             not (torch.is_grad_enabled() and voxels.requires_grad) and

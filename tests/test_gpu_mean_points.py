@@ -42,6 +42,19 @@ def test_against_float64(monkeypatch, features, points, voxels, skew):
     assert bool(((got.double() - ref).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("points", [127, 128, 129, 4000])
+def test_many_points_a_voxel_stay_with_torch(monkeypatch, points):
+    """(whose reduction takes them side by side: 30 voxels of 4000 points in 35 us, one after the other in 635)"""
+    import torch
+    from mluop_hip import nn as spnn
+    x = torch.randn(30, points, 16, device="cuda")
+    counts = torch.full((30,), points, device="cuda", dtype=torch.int32)
+    got, native = launched(monkeypatch, lambda: spnn.mean_voxel_features(x, counts))
+    assert native == (points <= 128)
+    bound = (points + 1) * 2.0 ** -24 * x.double().abs().mean(dim=1)
+    assert bool(((got.double() - x.double().mean(dim=1)).abs() <= bound).all())
+
+
 def test_what_stays_with_torch(monkeypatch):
     import torch
     from mluop_hip import nn as spnn
