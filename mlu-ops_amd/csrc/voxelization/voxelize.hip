@@ -199,20 +199,21 @@ struct BucketedPoints {
 
 constexpr uint32_t kIsFirst = 0x80000000u;
 
-// Cells of a bucket in LDS (32-bit keys).  FILLS: the bucket has more points than the table has
+// Cells of a bucket in LDS.  FILLS: the bucket has more points than the table has
 // slots to spare, and so perhaps more cells.
-template <bool FILLS>
+template <bool FILLS, typename KEY = uint32_t>
 struct LdsTable {
-  uint32_t *keys, *counts, *firsts;
+  KEY *keys;
+  uint32_t *counts, *firsts;
   uint32_t slots;  // a power of two
   uint32_t *used;  // slots taken so far (FILLS)
   static constexpr bool kFills = FILLS;
-  typedef uint32_t Key;
-  static constexpr Key kEmpty = 0xffffffffu;
+  typedef KEY Key;
+  static constexpr Key kEmpty = ~Key(0);
   __device__ static void cleared() {}
 };
-// The same in device memory, for buckets of more cells than the LDS table holds and for grids whose
-// keys need 64 bits.
+// The same in device memory, for buckets of more cells than the LDS table holds and, but for small buckets of few
+// points, for grids whose keys need 64 bits.
 struct WideTable {
   u64 *keys;
   uint32_t *counts, *firsts;
@@ -322,16 +323,27 @@ __device__ __forceinline__ bool rankBucket(const TABLE &t, const u64 *__restrict
 // crowded cell do; the table in device memory takes several times as long.
 //
 // The ranks of one bucket's `count` points, `entries` in point order.  `wide_at`: where the bucket's share of the
-// region in device memory begins.
-template <int THREADS, int SLOTS>
+// region in device memory begins.  LONG_KEYS: the keys in LDS have room for 64 bits, which up to SLOTS / 2 points need.
+template <int THREADS, int SLOTS, bool LONG_KEYS>
 __device__ __forceinline__ void rankCells(const float *__restrict__ points, const float *__restrict__ voxel_size,
                                           const float *__restrict__ range, int num_features, uint32_t max_points,
                                           const u64 *__restrict__ entries, uint32_t count, size_t wide_at, u64 *wide_keys,
                                           uint32_t *wide_counts, uint32_t *wide_firsts, uint32_t *__restrict__ state,
                                           uint32_t *__restrict__ first_of, uint8_t *first_flags, bool small_grid) {
-  __shared__ uint32_t s_keys[SLOTS], s_counts[SLOTS], s_firsts[SLOTS];
+  __shared__ u64 s_long_keys[LONG_KEYS ? SLOTS : SLOTS / 2];
+  __shared__ uint32_t s_counts[SLOTS], s_firsts[SLOTS];
   __shared__ uint16_t s_owner[SLOTS];
   __shared__ uint32_t s_used;
+  uint32_t *const s_keys = reinterpret_cast<uint32_t *>(s_long_keys);
+  if constexpr (LONG_KEYS) {
+    if (!small_grid && count <= SLOTS / 2) {
+      LdsTable<false, u64> t = {s_long_keys, s_counts, s_firsts, 64, nullptr};
+      while (t.slots < 2 * count) t.slots <<= 1;
+      rankBucket<THREADS, SLOTS>(t, entries, count, points, voxel_size, range, num_features, false, max_points, s_owner,
+                                 state, first_of, first_flags);
+      return;
+    }
+  }
   if (small_grid) {
     if (__builtin_expect(count <= SLOTS / 2, 1)) {
       LdsTable<false> t = {s_keys, s_counts, s_firsts, 64, nullptr};
@@ -361,9 +373,9 @@ __global__ __launch_bounds__(THREADS) void voxRankInCells(
   const uint32_t count = totals[blockIdx.x];
   if (count == 0) return;
   const uint32_t start = bucket_start[blockIdx.x];
-  rankCells<THREADS, SLOTS>(points, voxel_size, range, num_features, max_points, grouped + start, count,
-                            3 * (size_t)start, wide_keys, wide_counts, wide_firsts, state, first_of, nullptr,
-                            smallGrid(gridCells(voxel_size, range)));
+  rankCells<THREADS, SLOTS, false>(points, voxel_size, range, num_features, max_points, grouped + start, count,
+                                   3 * (size_t)start, wide_keys, wide_counts, wide_firsts, state, first_of, nullptr,
+                                   smallGrid(gridCells(voxel_size, range)));
 }
 
 // ---- few points ---------------------------------------------------------------------------
@@ -381,6 +393,7 @@ constexpr int kFewThreads = 512;
 constexpr int kFewTags = 16 * kFewThreads;             // tags the workgroup reads in a round
 constexpr int kFewRounds = kFewPoints / kFewTags;
 constexpr int kFewListed = 1024;                       // points of a bucket that are listed in LDS
+constexpr uint32_t kFewSlots = 2048;                   // of the table of its cells there
 static_assert(kFewRounds % 2 == 0 && kFewTags < 1 << 16, "two rounds' counts in one word");
 
 // (multiples of whole rounds: the tags behind the last point are kFewNone)
@@ -473,8 +486,10 @@ __global__ __launch_bounds__(kFewThreads) void voxRankFew(
     }
   }
   if (count == 0) return;
-  // (grids whose keys need 64 bits take a table in device memory, for which a bucket needs its place there)
-  const bool listed = count <= (uint32_t)kFewListed && small_grid;
+  // (what is listed is ranked in LDS, also in grids whose keys need 64 bits: with a table in device memory the three kernels
+  // took 76 us there at 23 k points, those of the six launches take 63, these 25)
+  const bool listed = count <= (uint32_t)kFewListed;
+  static_assert(kFewListed <= kFewSlots / 2, "listed points have a table in LDS");
   if (!listed) {
     if (tid == 0) s_start = atomicAdd(cursor, count);
     __syncthreads();
@@ -492,13 +507,13 @@ __global__ __launch_bounds__(kFewThreads) void voxRankFew(
   }
   __syncthreads();
   if (!listed) {
-    rankCells<kFewThreads, 2048>(points, voxel_size, range, num_features, max_points, grouped + start, count,
-                                 3 * (size_t)start, wide_keys, wide_counts, wide_firsts, state, first_of, first_flags,
-                                 small_grid);
+    rankCells<kFewThreads, kFewSlots, true>(points, voxel_size, range, num_features, max_points, grouped + start, count,
+                                            3 * (size_t)start, wide_keys, wide_counts, wide_firsts, state, first_of,
+                                            first_flags, small_grid);
     return;
   }
-  rankCells<kFewThreads, 2048>(points, voxel_size, range, num_features, max_points, s_list, count, 0, wide_keys,
-                               wide_counts, wide_firsts, state, first_of, first_flags, true);
+  rankCells<kFewThreads, kFewSlots, true>(points, voxel_size, range, num_features, max_points, s_list, count, 0, wide_keys,
+                                          wide_counts, wide_firsts, state, first_of, first_flags, small_grid);
 }
 
 // ---- voxel numbers -----------------------------------------------------------------------

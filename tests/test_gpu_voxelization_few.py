@@ -63,3 +63,23 @@ def test_crowded_cells_beyond_the_range(gpu_handle, max_points, grid):
     for n in (FEW - 3000, len(pts)):
         assert_same(run_gpu(gpu_handle, pts[:n], vs, cr, max_points, 40000),
                     sorted_voxelization(pts[:n], vs, cr, max_points, 40000))
+
+
+@pytest.mark.parametrize("cells", [1, 32, 33, 510, 512, 514, 1026, 3000])
+def test_buckets_of_grids_with_64_bit_keys(gpu_handle, cells):
+    """Cells of one bucket, twice each, in a grid of 2^33 cells: the table in LDS has 64-bit keys there, and those of whole
+    rounds differ in their upper halves only."""
+    rng = np.random.default_rng(cells)
+    side = 2048
+    keys = np.unique(rng.integers(0, side ** 3, 400 * cells + 2000))
+    keys = np.concatenate([keys, keys[keys < 1 << 32] + (1 << 32)])
+    keys = rng.permutation(np.unique(keys[tag_of(keys) == 5]))[:cells]
+    assert len(keys) == cells and keys.max() < side ** 3
+    keys = np.concatenate([keys, keys])
+    rng.shuffle(keys)
+    pts = np.stack([keys % side, keys // side % side, keys // side ** 2, keys], 1).astype(np.float32)
+    pts[:, :3] += 0.5
+    vs, cr = [1.0, 1.0, 1.0], [0.0, 0.0, 0.0, float(side), float(side), float(side)]
+    print("voxelization, long keys", cells, flush=True)
+    for max_points in (1, 3):
+        assert_same(run_gpu(gpu_handle, pts, vs, cr, max_points, 6000), sorted_voxelization(pts, vs, cr, max_points, 6000))
