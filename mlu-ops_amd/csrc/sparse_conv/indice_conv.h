@@ -49,6 +49,9 @@ struct ConvProblem {
   bool inverse = false;
   // The caller promised that no offset names a result row twice: no check for lost pairs.
   bool distinct_pairs = false;
+  // Neighbouring result rows gather from all over the tensor, as far as the host knows (speed only: the rulebook's input
+  // rows were in no order).
+  bool scattered = false;
   // The caller promised that no result row is in two pairs, over all offsets together.
   bool single_pairs = false;
   // Forward: negative results are stored as zero.

@@ -2245,6 +2245,7 @@ void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows con
 //   fp16 128 -> 128 167/210    64 -> 64 82/95
 // Of two offsets a phase (64 channels: 93), tiles of 256 rows (128: 233; 64: 123), whole rows of 256 bytes (185),
 // quarters (181) and 32 columns a wave at 64 (86) none is faster.
+// A phase of two pieces (DEPTH) is for few tiles and for rows in no order: denseDepth.
 // OFFSETS: an offset's product is a chain of its own, added to the row's sum when it is whole, as the pair-list kernels
 // add: their bits (128 -> 128 takes the registers of two workgroups a CU for it; useDenseKernel has both sides' times).
 struct StagedPlan {
@@ -2256,7 +2257,9 @@ constexpr StagedPlan stagedPlan(int elem_bytes, int Q, int C) {
   return StagedPlan{C >= 64 ? 4 : (C >= 32 ? 2 : 1), C >= 128 ? 2 : 1, Q * elem_bytes >= 256 ? 2 : 1};
 }
 // Workgroups a CU.
-constexpr int stagedPerCu(int Q, int C, bool offsets) { return offsets && Q == 128 && C == 128 ? 2 : 3; }
+constexpr int stagedPerCu(int Q, int C, bool offsets, int depth) {
+  return depth == 2 || (offsets && Q == 128 && C == 128) ? 2 : 3;
+}
 // Where piece `piece` of a staged row lies among its row's pieces: at piece ^ this.
 __device__ __forceinline__ int stagedSwizzle(int row) {
   return (row >> 1) & 7;
@@ -2275,9 +2278,9 @@ __device__ __forceinline__ void requestWordsToLds(u32x4 words, uint32_t offset, 
                :: "s"(lds_address), "v"(offset), "s"(words) : "memory", "m0");
 }
 
-template <typename E, int Q, int C, bool OFFSETS, typename SRC>
+template <typename E, int Q, int C, bool OFFSETS, int DEPTH, typename SRC>
 __global__ __launch_bounds__(kDenseThreads)
-    __attribute__((amdgpu_waves_per_eu(stagedPerCu(Q, C, OFFSETS), stagedPerCu(Q, C, OFFSETS))))
+    __attribute__((amdgpu_waves_per_eu(stagedPerCu(Q, C, OFFSETS, DEPTH), stagedPerCu(Q, C, OFFSETS, DEPTH))))
 void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRows conv,
                            const typename E::storage *packedW, SRC source, int R, int K, typename E::storage *result) {
   typedef typename E::vec8 vec8;
@@ -2301,7 +2304,7 @@ void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRo
   constexpr int W_BYTES = (C / 16) * KB * 1024;  // packed filter of an offset
   static_assert(SB == 128 && CW * NB * 16 == C && WAVES % CW == 0, "split");
 
-  __shared__ __attribute__((aligned(1024))) char s_rows[2 * BUFFER];
+  __shared__ __attribute__((aligned(1024))) char s_rows[2 * DEPTH * BUFFER];
   __shared__ __attribute__((aligned(16))) DenseMap s_map;
 
   const int tid = threadIdx.x;
@@ -2374,7 +2377,8 @@ void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRo
           reinterpret_cast<const char *>(packedW) + (size_t)(kc + kk) * W_BYTES + first_block * KB * 1024, conv.row_bytes);
     }
     if (offsets == 0) continue;
-    // A phase is a part of one offset's channels.  kk < 0: none is left; nothing is staged and nothing multiplied.
+    // A piece is a part of one offset's channels, a phase DEPTH pieces.  kk < 0: no offset is left; nothing is staged and
+    // nothing multiplied.
     uint32_t left = offsets;
     auto next_offset = [&]() -> int {
       const int kk = left != 0 ? __builtin_ctz(left) : -1;
@@ -2416,15 +2420,25 @@ void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRo
                            rows_lds + (uint32_t)(buffer * BUFFER + ((wave + t * WAVES) * LPG + j) * 1024));
       }
     };
+    // Piece `first` + j of the trip's 2 * DEPTH, each with a buffer of its own; `before`: the offset of the piece in front.
+    auto request_phase = [&](auto first, int before, int (&of)[DEPTH], Filters (&w)[DEPTH]) {
+#pragma unroll
+      for (int j = 0; j < DEPTH; ++j) {
+        of[j] = (first + j) % PARTS == 0 ? next_offset() : (j > 0 ? of[j - 1] : before);
+        request(of[j], (first + j) % PARTS, first + j, w[j]);
+      }
+    };
     // Everything this wave has requested is there.  The filters pass through an empty statement that the
     // compiler must take for their last writer: its own wait for their loads then lies here, and not in front
     // of their first use, behind the next phase's requests, which it would wait for as well.
-    auto landed = [&](Filters &w) {
+    auto landed = [&](Filters (&w)[DEPTH]) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
+      for (int j = 0; j < DEPTH; ++j)
 #pragma unroll
-        for (int kb = 0; kb < KP; ++kb) asm volatile("" : "+v"(w[nb][kb]));
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+          for (int kb = 0; kb < KP; ++kb) asm volatile("" : "+v"(w[j][nb][kb]));
     };
     // (a group's rows are read while the group before is multiplied; those of a group without partners are what
     // the buffer held before, and nobody multiplies them)
@@ -2461,23 +2475,27 @@ void gatherConvDenseStaged(const typename E::storage *A, uint32_t a_size, ConvRo
     };
     // (two phases a trip and one way out of the loop, at the price of an empty phase at the end of an
     // odd number of them: with a second way out the compiler waits for all loads in front of every use)
-    Filters w_a, w_b;
-    int now = next_offset();
-    request(now, 0, 0, w_a);
+    auto multiply_phase = [&](auto first, const int (&of)[DEPTH], const Filters (&w)[DEPTH]) {
+#pragma unroll
+      for (int j = 0; j < DEPTH; ++j) multiply(of[j], (first + j) % PARTS, first + j, w[j]);
+    };
+    constexpr std::integral_constant<int, 0> kEven{};
+    constexpr std::integral_constant<int, DEPTH> kOdd{};
+    Filters w_a[DEPTH], w_b[DEPTH];
+    int now[DEPTH], after[DEPTH];
+    request_phase(kEven, -1, now, w_a);
     landed(w_a);
     ldsBarrier();
     do {
-      const int after = PARTS == 2 ? now : next_offset();
-      request(after, PARTS - 1, 1, w_b);
-      multiply(now, 0, 0, w_a);
+      request_phase(kOdd, now[DEPTH - 1], after, w_b);
+      multiply_phase(kEven, now, w_a);
       landed(w_b);
       ldsBarrier();
-      now = next_offset();
-      request(now, 0, 0, w_a);
-      multiply(after, PARTS - 1, 1, w_b);
+      request_phase(kEven, -1, now, w_a);
+      multiply_phase(kOdd, after, w_b);
       landed(w_a);
       ldsBarrier();
-    } while (now >= 0);
+    } while (now[0] >= 0);
   }
   // lane holds result columns 16*nb + 4*quad + (0..3) of row 16*g + pair of its wave's rows
 #pragma unroll
@@ -4092,9 +4110,30 @@ DenseSums useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const Gather
   return chain || lc.choices.dense_tiles == 1 ? DenseSums::kChain : DenseSums::kNone;
 }
 
+// Pieces of a phase of gatherConvDenseStaged, 2-byte types: one or two.  Two halve the round trips that follow each other
+// in a tile, and leave a CU two workgroups instead of three: for launches of few tiles, and for rows strewn over memory
+// (`scattered`), whose two halves are then fetched together.  Row maps of 128 result columns take two always (their kernel
+// needs the registers of two workgroups).  us with the filter's packing, one / two pieces, 3x3x3, 0.19 to 0.38 filled:
+//   lists, rows in order    64 -> 16   1 k rows 24.9/22.2  20 k 23.0/21.6  120 k 40/39  250 k 65/69
+//                           128 -> 32  1 k 37/31.5  20 k 31/31  50 k 39/36  120 k 63/61  250 k 100/106
+//                           64 -> 64   1 k 27.4/25.4  8 k 26.7/25.8  20 k 26.5/26.4  50 k 30.4/30.7  250 k 75/84
+//                           128 -> 64  1 k 39/35  8 k 37.7/35.8  20 k 35.6/36.9  50 k 43/44  250 k 112/126
+//                           128 -> 128 1 k 45/43  8 k 43.9/45.4  250 k 157/171
+//   lists, rows in no order 64 -> 16   1 k 26/23  20 k 26/23  120 k 56/48  300 k 107/104     64 -> 64  1 k 28/26  20 k 29/27
+//                           120 k 59/56  300 k 115/120     128 -> 64  20 k 42/38  120 k 94/88  300 k 190/193
+//   row maps, no order      64 -> 64   8 k 41/37  120 k 90/85  300 k 161/162   128 -> 128  20 k 71/59  120 k 170/150  300 k 358/322
+//   row maps, rows in order 64 -> 64   1 k 25/23  20 k 24.5/24.4  300 k 78/88   128 -> 128  20 k 47/45  300 k 223/204
+int denseDepth(bool lists, bool scattered, int q_padded, int c_padded, int rows) {
+  if (c_padded == 128) return lists ? 1 : 2;
+  if (!lists && scattered) return 2;
+  if (c_padded <= 32) return scattered || rows <= 131072 ? 2 : 1;
+  return rows <= (scattered ? 131072 : (q_padded == 64 ? 32768 : 10000)) ? 2 : 1;
+}
+
 template <typename E, int Q, int C, typename SRC>
 void launchDenseInstance(const LaunchCtx &lc, const void *A, uint32_t a_size, const ConvRows &rows,
-                         const void *packed, const SRC &source, bool by_offset, int R, int K, void *result) {
+                         const void *packed, const SRC &source, bool by_offset, bool scattered, int R, int K,
+                         void *result) {
   auto launch = [&](auto kernel) {
     lc.begin("gatherConvDense");
     kernel<<<denseGridX(R), kDenseThreads, 0, lc.stream>>>(
@@ -4103,17 +4142,25 @@ void launchDenseInstance(const LaunchCtx &lc, const void *A, uint32_t a_size, co
     lc.end();
   };
   if constexpr (SRC::kSegments && denseByOffsetShape((int)sizeof(typename E::storage), Q, C)) {
-    if (by_offset) return launch(gatherConvDenseStaged<E, Q, C, true, SRC>);
+    if (by_offset) return launch(gatherConvDenseStaged<E, Q, C, true, 1, SRC>);
   }
-  if constexpr (Q * (int)sizeof(typename E::storage) > 64) launch(gatherConvDenseStaged<E, Q, C, false, SRC>);
-  else launch(gatherConvDense<E, Q, C, SRC>);
+  if constexpr (Q * (int)sizeof(typename E::storage) > 64) {
+    if constexpr (sizeof(typename E::storage) == 2 && !(SRC::kSegments && C == 128)) {
+      if (C == 128 || denseDepth(SRC::kSegments, scattered, Q, C, R) == 2)
+        return launch(gatherConvDenseStaged<E, Q, C, false, 2, SRC>);
+    }
+    if constexpr (sizeof(typename E::storage) == 4 || SRC::kSegments || C < 128)
+      launch(gatherConvDenseStaged<E, Q, C, false, 1, SRC>);
+  } else {
+    launch(gatherConvDense<E, Q, C, SRC>);
+  }
 }
 
 template <typename E, typename SRC>
 void launchDense(const LaunchCtx &lc, int q_padded, const void *A, int n_src, const ConvRows &rows,
-                 const void *packed, const SRC &source, bool by_offset, int R, int K, void *result) {
+                 const void *packed, const SRC &source, bool by_offset, bool scattered, int R, int K, void *result) {
   const uint32_t a_size = (uint32_t)n_src * (uint32_t)rows.row_bytes;
-#define DENSE_INSTANCE(q, c) launchDenseInstance<E, q, c, SRC>(lc, A, a_size, rows, packed, source, by_offset, R, K, result)
+#define DENSE_INSTANCE(q, c) launchDenseInstance<E, q, c, SRC>(lc, A, a_size, rows, packed, source, by_offset, scattered, R, K, result)
 #define DENSE_BY_C(q)                       \
   switch (rows.c_padded) {                  \
     case 16: DENSE_INSTANCE(q, 16); break;  \
@@ -4301,7 +4348,7 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
     src.counts = inl;
     if (dense)
       launchDense<E, SegmentSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, src,
-                                    dense_sums == DenseSums::kByOffset, d.R, p.K, result);
+                                    dense_sums == DenseSums::kByOffset, p.scattered, d.R, p.K, result);
     else if (tall)
       launchTall<E, SegmentSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, src, tall_rows, d.R, p.K,
                                    result);
@@ -4347,8 +4394,8 @@ void launchGatherTyped(const LaunchCtx &lc, const ConvProblem &p, const GatherDi
       const MapSource map = {entries, ws.filled, run_if};
       if (map_dense) {
         n_filled = denseGridX(rows);
-        launchDense<E, MapSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, map, false, rows, p.K,
-                                  result_rows);
+        launchDense<E, MapSource>(lc, d.q_padded, rows_from, d.n_src, rows_of, ws.packed, map, false,
+                                  p.list_trust != ListTrust::kInOrder || p.scattered, rows, p.K, result_rows);
       } else if (tall) {
         n_filled = tallGridX(rows, map_tall_rows);
         launchTall<E, MapSource>(lc, tall_q, rows_from, d.n_src, rows_of, ws.packed, map, map_tall_rows, rows, p.K,

@@ -58,17 +58,16 @@ void consultRulebookNotes(mluOpContext *handle, int row_column, ConvProblem *p) 
   for (int slot = 0; slot < mluOpContext::kRulebookNotes; ++slot) {
     const mluOpContext::RulebookNote &note = handle->rulebook_notes[slot];
     if (note.pairs != p->indice_pairs || note.K != p->K || note.L != p->L) continue;
-    if (row_column == 0) {
-      p->list_trust = ListTrust::kInOrder;
-      return;
-    }
     const unsigned long long report = __atomic_load_n(handle->rulebook_reports + slot, __ATOMIC_ACQUIRE);
-    if (report >> 32 != (note.stamp & 0xffffffffull)) {
-      // not arrived (or never sent: a captured rulebook files none)
+    // (false: not arrived, or never sent: a captured rulebook files none)
+    const bool arrived = report >> 32 == (note.stamp & 0xffffffffull), in_order = (uint32_t)report != 0;
+    p->scattered = arrived && !in_order;
+    if (row_column == 0)
+      p->list_trust = ListTrust::kInOrder;
+    else if (!arrived)
       p->list_trust = ListTrust::kUnknown;
-      return;
-    }
-    p->list_trust = (uint32_t)report != 0 ? ListTrust::kInOrder : ListTrust::kNone;
+    else
+      p->list_trust = in_order ? ListTrust::kInOrder : ListTrust::kNone;
     return;
   }
 }
