@@ -35,6 +35,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <cmath>
 #include <type_traits>
 
 #include "core/wave_scan.h"
@@ -4093,19 +4094,30 @@ DenseSums useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const Gather
     chain = sheets && d.q_padded <= 32 && fill >= 0.2;
   }
   // Fewer pairs, 2-byte rows of more than 64 bytes: with each offset's product by itself, which gives the pair-list
-  // kernels' bits, so that a layer's results do not depend on this line.  Filled sheets show less in a strided layer's
-  // counts, in which strewn voxels differ by a few per cent.  us of the pair-list kernels / this one, fp16, 3x3x3:
-  //   stride 2 on scenes, 0.18 to 0.20 filled (second count 1.11 to 1.27 of the mean)
-  //     64 -> 64    5 k rows 38/30   37 k 37/33   69 k 52/37   110 k 78/55   168 k 79/60
-  //     64 -> 128   11 k 34/37   19 k 35/37   37 k 46/43   69 k 68/50   168 k 119/82
-  //     128 -> 64   5 k 51/39   69 k 74/53   110 k 116/80       128 -> 128  11 k 48/49   37 k 66/64   69 k 96/84   110 k 142/107
-  //   strewn, or stride 2 on what layers have thickened (1.02 to 1.06)
-  //     64 -> 128   50 k rows 0.21 43/44   0.24 47/45   151 k 0.22 101/82   150 k 0.17 84/81   0.21 88/82   16 k 0.21 25/37
-  //     64 -> 64    125 k 0.20 51/58   150 k 0.21 61/60         128 -> 128  125 k 0.20 115/127   150 k 0.21 131/153
-  const bool uneven = second >= 1.1 * mean_rest;
+  // kernels' bits, so that a layer's results do not depend on this line.  It pays where some tiles hold far more pairs
+  // than others: filled sheets, which show less in a strided layer's counts.  Strewn voxels differ in theirs as chance
+  // has it, by some square roots of the count (1 500 rows: the second count 1.11 of the mean).  Up to 27 offsets: of 125, 5 k
+  // strewn rows 64 -> 64 take 71/101.  us of the pair-list kernels / this one with the filter's packing, fp16, 3x3x3:
+  //   stride 2 on scenes, 0.16 to 0.20 filled (second count 1.11 to 1.27 of the mean)
+  //     64 -> 64    5 k rows 38/30   38 k 40/33   60 k 48/35   110 k 78/55   168 k 79/60
+  //     128 -> 64   5 k 51/39   38 k 56/45   60 k 69/46   110 k 116/80
+  //     64 -> 128   11 k 34/37   19 k 35/37   38 k 43/42   60 k 58/43   168 k 119/82
+  //     128 -> 128  11 k 48/49   38 k 59/61   60 k 80/60   110 k 142/107        96 -> 96  38 k 58/62
+  //   stride 2 on even walls and floors, 0.19 filled (1.17 to 1.35, by which the host cannot tell them from scenes; at
+  //   0.23 filled the two are level from 2.5 k rows on)
+  //     64 -> 64    0.8 k 25/29   2.5 k 27/29   7 k 28/30   28 k 30/31   51 k 34/33      128 -> 64   2.5 k 34/39   28 k 39/40   51 k 46/45
+  //   strewn (1.02 to 1.39 at few rows), 64 -> 64 and 128 -> 64
+  //     300 rows 0.18 24/30, 31/42   1 500 0.20 25/31, 31/42   16 k 0.21 26/31, 33/42   120 k 0.22 51/57, 70/82
+  //   64 -> 128, strewn     50 k rows 0.18 41/44  0.22 44/44  0.25 47/44   120 k 0.18 70/73  0.21 74/75  0.25 81/76
+  //                         160 k 0.18 87/82   250 k 0.18 136/121   16 k 0.21 25/37
+  //   64 -> 128, stride 2 on what layers have thickened (1.02)    56 k 0.18 48/44   90 k 0.18 63/53   185 k 0.20 104/97
+  //              2x2x2, stride 2 (1.00 to 1.03)    42 k 0.24 25/25   104 k 0.24 38/39   117 k 0.27 51/40   155 k 0.24 49/44
+  const bool uneven = second >= 1.1 * mean_rest && second >= mean_rest + 4.0 * std::sqrt(mean_rest);
+  const bool strided = largest < 0.9 * d.R;  // (a submanifold layer has every row in its centre)
+  const double from = uneven ? (d.c_padded == 64 ? 1300 : d.q_padded == 64 ? 30000 : 50000) : p.K > 8 ? 50000 : 100000;
   const bool by_offset = !chain && lists && denseByOffsetShape((int)elemSize(p.dtype), d.q_padded, d.c_padded) &&
-                         fill >= 0.16 &&
-                         (uneven ? d.c_padded == 64 || d.R >= 30000 : d.q_padded == 64 && d.c_padded == 128 && d.R >= 50000);
+                         p.K <= 27 && fill >= 0.16 && d.R >= from &&
+                         (uneven || (d.q_padded == 64 && d.c_padded == 128 && (strided || fill >= 0.22)));
   if (by_offset) return DenseSums::kByOffset;
   return chain || lc.choices.dense_tiles == 1 ? DenseSums::kChain : DenseSums::kNone;
 }
@@ -4115,6 +4127,7 @@ DenseSums useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const Gather
 // (`scattered`), whose two halves are then fetched together.  Row maps of 128 result columns take two always (their kernel
 // needs the registers of two workgroups).  us with the filter's packing, one / two pieces, 3x3x3, 0.19 to 0.38 filled:
 //   lists, rows in order    64 -> 16   1 k rows 24.9/22.2  20 k 23.0/21.6  120 k 40/39  250 k 65/69
+//                           64 -> 32   1 k 25.5/23  20 k 23.6/23.5  50 k 26.0/27.0
 //                           128 -> 32  1 k 37/31.5  20 k 31/31  50 k 39/36  120 k 63/61  250 k 100/106
 //                           64 -> 64   1 k 27.4/25.4  8 k 26.7/25.8  20 k 26.5/26.4  50 k 30.4/30.7  250 k 75/84
 //                           128 -> 64  1 k 39/35  8 k 37.7/35.8  20 k 35.6/36.9  50 k 43/44  250 k 112/126
@@ -4125,9 +4138,9 @@ DenseSums useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const Gather
 //   row maps, rows in order 64 -> 64   1 k 25/23  20 k 24.5/24.4  300 k 78/88   128 -> 128  20 k 47/45  300 k 223/204
 int denseDepth(bool lists, bool scattered, int q_padded, int c_padded, int rows) {
   if (c_padded == 128) return lists ? 1 : 2;
-  if (!lists && scattered) return 2;
-  if (c_padded <= 32) return scattered || rows <= 131072 ? 2 : 1;
-  return rows <= (scattered ? 131072 : (q_padded == 64 ? 32768 : 10000)) ? 2 : 1;
+  if (scattered) return !lists || c_padded <= 32 || rows <= 131072 ? 2 : 1;
+  if (c_padded == 64) return rows <= (q_padded == 64 ? 32768 : 10000) ? 2 : 1;
+  return rows <= (q_padded == 64 && c_padded == 32 ? 32768 : 131072) ? 2 : 1;
 }
 
 template <typename E, int Q, int C, typename SRC>
