@@ -46,6 +46,12 @@ def share_row_maps(enable):
     _share_row_maps = bool(enable)
 
 
+# How many rulebooks of a plan may have their pair counts outstanding, and of how many offsets: a handle has those of 32
+# rulebooks of up to 343 on file, and others are copied, behind whatever convolutions are enqueued by then (40 layers:
+# the device was drained eight times).
+_PENDING, _COUNTED = 16, 343
+
+
 class Rulebook:
     """indice_pairs [K,2,L] (device; -1 behind an offset's indice_num pairs, with `tails` off only once `pairs` has
     been asked for: the operators read no further than the pairs), indice_num as host ints (where
@@ -69,6 +75,7 @@ class Rulebook:
         self._built_on = built_on
         self.num_act_out = num_act_out
         self.filter_space = tuple(filter_space)
+        self.counts_are_copied = math.prod(self.filter_space) > _COUNTED
         self.sub_m = sub_m
         self.out_space = tuple(out_space)
         self._for_operators = None
@@ -363,7 +370,7 @@ class SparseSequential(torch.nn.Sequential):
             try:
                 self._plan(x, built)
                 for rb in built:
-                    if len(rb._pairs) > _COUNTED:
+                    if rb.counts_are_copied:
                         rb.indice_num
             except BaseException:
                 for rb in built:
@@ -386,10 +393,6 @@ class SparseSequential(torch.nn.Sequential):
 
 
 _SEQUENTIAL_PLAN = SparseSequential.plan
-# How many rulebooks of a plan may have their pair counts outstanding, and of how many offsets: a handle has those of 32
-# rulebooks of up to 343 on file, and others are copied, behind whatever convolutions are enqueued by then (40 layers:
-# the device was drained eight times).
-_PENDING, _COUNTED = 16, 343
 
 
 class Voxelization(torch.nn.Module):
