@@ -4000,11 +4000,32 @@ bool tallHalfTiles(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &
 //    32 -> 64    400 k rows 139/142   50 k 37/41
 //   3x3x3, clustered: 128 -> 128  400 k 243/232   200 k 117/118;  64 -> 64  400 k 99/104   60 k 23/25;  uniform, 200 k:
 //   128 -> 128  69/78;  2x2x2 stride 2, 177 k rows: 128 -> 128  55/60: up to 32 offsets stay with 256.
+// A CU has one such tile at a time and nothing to do in its round trips, and a launch lasts as long as its heaviest tile:
+// fewer workgroups than half the CUs, or many pairs a row, favour two tiles of 256.  us, 5x5x5, by pairs a row, with the
+// filter's packing:
+//   by workgroups  128 -> 64, gradient of stride 2 (15 pairs)  98 workgroups 105/132   196 200/164   390 373/324
+//                  128 -> 64, stride 2 of a scene (5 to 8)     116 113/145   258 236/235   374 276/288   839 526/468
+//                  128 -> 64, stride 2 of surfaces (1)         140 61/44     265 89/78     96 -> 96, scene (4)  140 108/136
+//                  64 -> 128, surfaces (2) 80 42/39   196 53/44    stride 2 of a thinned scene (3) 106 43/48
+//   64 channels    64 -> 64   surfaces (3) 391 workgroups 110/103   clustered (8) 391 152/152  (11) 782 311/296
+//                             stride 2, strewn (2.6) 559 100/95   thinned scene (3.6) 422 109/117   scene (7) 839 355/368
+//                             gradient of stride 2 (15) 391 193/213         64 -> 128  782 305/328
+//                  64 -> 128  stride 2, strewn (2.6) 1118 163/150  thinned scene (4) 316 89/100   scene (6) 516 214/230
 int tallTileRows(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d, int tall_q, bool lists) {
   const int row_bytes = tall_q * (int)elemSize(p.dtype);
   if (lists && tallHalfTiles(lc, p, d)) return 128;
-  if (lists && p.K > kTallFewOffsets && elemSize(p.dtype) == 2 && row_bytes >= 128) return 512;
-  return tallRows(row_bytes);
+  if (!lists || p.K <= kTallFewOffsets || elemSize(p.dtype) != 2 || row_bytes < 128) return tallRows(row_bytes);
+  if (lc.choices.tall_tiles == 1) return 512;
+  double pairs = 0, largest = 0;
+  for (int k = 0; k < p.K; ++k) {
+    pairs += (double)p.indice_num[k];
+    largest = (double)p.indice_num[k] > largest ? (double)p.indice_num[k] : largest;
+  }
+  const int64_t workgroups = ((int64_t)d.R + 511) / 512 * (d.c_padded / kTallCols);
+  const bool submanifold = largest >= 0.9 * d.R;  // (every row is in the centre's pairs)
+  const int64_t enough = pairs < 2.2 * d.R ? 64 : pairs < 4.0 * d.R || row_bytes < 256 ? 128 : 160;
+  const bool tall = workgroups >= enough && (row_bytes >= 256 || submanifold || pairs < 3.0 * d.R);
+  return tall ? 512 : tallRows(row_bytes);
 }
 
 bool useTallKernel(const LaunchCtx &lc, const ConvProblem &p, const GatherDims &d, bool lists) {
