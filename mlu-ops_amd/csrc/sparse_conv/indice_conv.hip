@@ -3919,7 +3919,7 @@ void launchTallInstance(const LaunchCtx &lc, const void *A, uint32_t a_size, con
   constexpr int TR = tallRows(Q * S);
   auto launch = [&](auto kernel, int threads) {
     const dim3 grid(tallGridX(R, tile_rows), (rows.c + kTallCols - 1) / kTallCols);
-    lc.begin("gatherConvTall");
+    lc.begin(tile_rows == 512 && TR == 256 ? "gatherConvTall512" : "gatherConvTall");
     kernel<<<grid, threads, 0, lc.stream>>>(static_cast<const typename E::storage *>(A), a_size, rows,
                                             static_cast<const typename E::storage *>(packed), source, R, K,
                                             static_cast<typename E::storage *>(result));
@@ -4169,7 +4169,7 @@ void launchDenseInstance(const LaunchCtx &lc, const void *A, uint32_t a_size, co
                          const void *packed, const SRC &source, bool by_offset, bool scattered, int R, int K,
                          void *result) {
   auto launch = [&](auto kernel) {
-    lc.begin("gatherConvDense");
+    lc.begin(by_offset ? "gatherConvDenseByOffset" : "gatherConvDense");
     kernel<<<denseGridX(R), kDenseThreads, 0, lc.stream>>>(
         static_cast<const typename E::storage *>(A), a_size, rows, static_cast<const typename E::storage *>(packed),
         source, R, K, static_cast<typename E::storage *>(result));

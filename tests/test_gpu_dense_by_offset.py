@@ -51,7 +51,7 @@ def test_bits_of_the_pair_list_kernels(gpu_handle, ci, co, space, dtype_name, fi
                 gpu_handle, x, w, m.LAYOUT_ARRAY, pairs, num, n_out, False))
         finally:
             gpu_handle.set_kernel_choice("dense_tiles", None)
-        assert ("gatherConvDense" in names) != lists, names
+        assert ("gatherConvDenseByOffset" in names) != lists and "gatherConvDense" not in names, names
     a, b = got[False], got[True]
     if finite:
         assert torch.equal(a, b)
@@ -75,6 +75,24 @@ def test_row_map_behind_lists_on_trust():
     w = torch.from_numpy((rng.standard_normal(ks + (channels, channels)) / 40).astype(np.float32)).cuda().half()
     ((want, known), (got, trusted)), fill = with_and_without_a_wait(m.make_handle_on_current_stream(), idx, space, ks, 1, x, w)
     assert 0.16 <= fill < 0.27, fill
-    assert "packFilterCutPairLists" not in known and "gatherConvDense" not in known, known
-    assert "packFilterCutPairLists" in trusted and trusted.count("gatherConvDense") == 1, trusted
+    dense = {"gatherConvDense", "gatherConvDenseByOffset"}
+    assert "packFilterCutPairLists" not in known and not dense & set(known), known
+    assert "packFilterCutPairLists" in trusted and [n for n in trusted if n in dense] == ["gatherConvDenseByOffset"], trusted
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("rows,density", [(300, 0.18), (700, 0.25), (1500, 0.2), (6000, 0.2)])
+@pytest.mark.parametrize("ks", [(3, 3, 3), (5, 5, 5)])
+def test_strewn_voxels_stay_with_the_pair_lists(gpu_handle, rows, density, ks):
+    """Their counts differ by chance, by a tenth of the mean and more at few rows; and 125 offsets, whatever they differ by."""
+    import torch
+    import mluop_hip as m
+    rng = np.random.default_rng(rows)
+    side = int(round((rows / density) ** (1 / 3)))
+    cells = np.sort(rng.choice(side ** 3, rows, replace=False))
+    idx = np.stack([0 * cells, cells // side ** 2, cells // side % side, cells % side], 1).astype(np.int32)
+    pairs, num, n_out = gpu_rulebook(gpu_handle, idx, 1, (side,) * 3, ks, [k // 2 for k in ks], [1, 1, 1], [1, 1, 1], True)
+    x = torch.randn((rows, 64), device="cuda").half()
+    w = torch.randn(ks + (64, 64), device="cuda").half()
+    _, names = kernels_of(gpu_handle, lambda: m.indice_conv_forward(gpu_handle, x, w, m.LAYOUT_ARRAY, pairs, num, n_out, True))
+    assert not any(n.startswith("gatherConvDense") for n in names), names

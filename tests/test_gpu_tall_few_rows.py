@@ -20,7 +20,7 @@ def both(handle, case, tall):
     finally:
         handle.set_kernel_choice("dense_tiles", None)
         handle.set_kernel_choice("tall_tiles", None)
-    return out, dx, "gatherConvTall" in forward, "gatherConvTall" in backward
+    return (out, dx) + tuple("gatherConvTall" in names or "gatherConvTall512" in names for names in (forward, backward))
 
 
 def few(rows, q, c, size):

@@ -18,7 +18,40 @@ pytestmark = pytest.mark.gpu
                                         (2049, (12, 20, 24))])
 def test_bits_of_the_short_tiles(gpu_handle, ci, co, dtype_name, rows, space):
     print("tall teams", ci, co, dtype_name, rows, flush=True)
-    check(gpu_handle, make_case(gpu_handle, rows, space, (3, 3, 5), ci, co, dtype_name, False), (True, True))
+    case = make_case(gpu_handle, rows, space, (3, 3, 5), ci, co, dtype_name, False)
+    check(gpu_handle, case, (True, True))
+    both_directions(gpu_handle, case, True)
+    assert all("gatherConvTall512" in names for names in case["kernels"]), case["kernels"]
+
+
+@pytest.mark.parametrize("ci,co,rows,forward,backward", [
+    (64, 64, 65025, True, True),       # 128 workgroups
+    (64, 64, 65024, False, False),     # 127
+    (128, 64, 65025, True, True),      # two groups of columns backward
+    (64, 128, 32600, True, False),     # 128 and 64 workgroups
+    (64, 32, 65025, None, False),      # (results of up to 32 columns have another kernel; rows of 32 channels stay with 256)
+])
+def test_by_workgroups(gpu_handle, ci, co, rows, forward, backward):
+    """Which tiles a layer of 45 offsets takes by itself, and the same bits with either."""
+    import torch
+    import mluop_hip as m
+    print("tall teams by workgroups", ci, co, rows, flush=True)
+    case = make_case(gpu_handle, rows, (20, 240, 240) if rows > 40000 else (20, 180, 180), (3, 3, 5), ci, co, "float16", False)
+    assert 2.2 < sum(case["num"]) / rows < 4  # pairs a row
+    got = {}
+    for tall in (None, False):
+        gpu_handle.set_kernel_choice("tall_tiles", tall)
+        try:
+            got[tall] = [kernels_of(gpu_handle, call) for call in (
+                lambda: m.indice_conv_forward(gpu_handle, case["x"], case["w"], m.LAYOUT_ARRAY, case["pairs"], case["num"],
+                                              rows, True),
+                lambda: m.indice_conv_backward_data(gpu_handle, case["dy"], case["w"], m.LAYOUT_ARRAY, case["pairs"],
+                                                    case["num"], True, ci))]
+        finally:
+            gpu_handle.set_kernel_choice("tall_tiles", None)
+    for (a, names), (b, short), tall in zip(got[None], got[False], (forward, backward)):
+        assert torch.equal(a, b) and "gatherConvTall512" not in short
+        assert tall is None or ("gatherConvTall512" in names) == tall and ("gatherConvTall" in names) == (not tall), names
 
 
 def test_lists_that_are_not_in_order(gpu_handle):
@@ -33,7 +66,7 @@ def test_lists_that_are_not_in_order(gpu_handle):
     case["pairs"].copy_(torch.from_numpy(pairs))
     out, dx, ran = both_directions(gpu_handle, case, True)
     torch.cuda.synchronize()
-    assert ran == (True, True)
+    assert ran == (True, True) and all("gatherConvTall512" in names for names in case["kernels"])
     w_k = from_torch(case["w"]).reshape(45, channels, channels)
     ref = oracle.forward(case["host"]["x"], w_k, pairs, case["num"], case["n_out"])
     check_close(from_torch(out), ref, "float16", "tall teams")
@@ -88,6 +121,6 @@ def test_row_map_behind_lists_on_trust():
     handle.set_kernel_choice("dense_tiles", False)
     handle.set_kernel_choice("tall_tiles", True)
     ((want, known), (got, trusted)), _ = with_and_without_a_wait(handle, idx, space, ks, 1, x, w)
-    assert "packFilterCutPairLists" not in known and "gatherConvTall" in known, known
-    assert "packFilterCutPairLists" in trusted and trusted.count("gatherConvTall") == 2, trusted
+    assert "packFilterCutPairLists" not in known and "gatherConvTall" in known and "gatherConvTall512" not in known, known
+    assert "packFilterCutPairLists" in trusted and "gatherConvTall512" in trusted and "gatherConvTall" in trusted, trusted
     assert torch.equal(got, want)

@@ -25,7 +25,8 @@ def both_directions(handle, case, tall):
     finally:
         for which in ("dense_tiles", "wave_per_tile", "tall_tiles"):
             handle.set_kernel_choice(which, None)
-    return out, dx, ("gatherConvTall" in forward, "gatherConvTall" in backward)
+    case["kernels"] = forward, backward
+    return out, dx, tuple("gatherConvTall" in names or "gatherConvTall512" in names for names in case["kernels"])
 
 
 def make_case(handle, rows, space, ks, ci, co, dtype_name, shuffle, stride=1):
