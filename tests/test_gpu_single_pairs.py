@@ -16,6 +16,8 @@ def rulebook(handle, rows, ks, stride, repeated=False):
     rng = np.random.default_rng(rows + ks[0])
     space = (9, 21, 31)
     cells = rng.choice(space[0] * space[1] * space[2], rows, replace=repeated)
+    if rows == 1:
+        cells[:] = 0  # (whatever the stride, some output reaches the first cell)
     idx = np.stack([0 * cells, cells // (21 * 31), cells // 31 % 21, cells % 31], axis=1).astype(np.int32)
     out = [(s - k) // t + 1 for s, k, t in zip(space, ks, stride)]
     pairs, _, num, n_out = m.get_indice_pairs(handle, torch.from_numpy(idx).cuda(), 1, space, ks, out, [0, 0, 0],
@@ -34,8 +36,7 @@ def test_same_numbers_as_without_the_promise(gpu_handle, rows, ks, stride, dtype
     import mluop_hip as m
     print("single pairs", rows, ks, stride, dtype_name, q, c, inverse, flush=True)
     pairs, counts, n_out = rulebook(gpu_handle, rows, ks, stride, repeated=rows == 1000 and max(ks) > 1)
-    if n_out == 0:
-        pytest.skip("no output cell")
+    assert n_out > 0
     dtype = getattr(torch, dtype_name)
     g = torch.Generator(device="cuda").manual_seed(rows)
     x = torch.randn((n_out, q), generator=g, device="cuda").to(dtype)
@@ -134,6 +135,53 @@ def test_relu_in_the_store(gpu_handle):
         gpu_handle.promise_single_pairs(None)
         gpu_handle.set_extended_modes(False)
     assert torch.equal(got, plain.clamp(min=0)) and (plain < 0).any()
+
+
+@pytest.mark.parametrize("backward", [False, True])
+@pytest.mark.parametrize("dtype_name,q,c", [("float16", 64, 64), ("bfloat16", 33, 128), ("float32", 48, 20)])
+def test_the_other_column(gpu_handle, backward, dtype_name, q, c):
+    """Column 1 names the rows of a plain layer's result and of an inverse layer's gradient; calls whose result rows the
+    other column names stay with the ordinary kernels."""
+    import torch
+    import mluop_hip as m
+    rows, ks, stride = 900, (1, 1, 1), (1, 1, 1)
+    pairs, counts, n_out = rulebook(gpu_handle, rows, ks, stride)
+    dtype = getattr(torch, dtype_name)
+    x = torch.randn((rows, q), device="cuda").to(dtype)
+    w = torch.randn((1, 1, 1) + ((c, q) if backward else (q, c)), device="cuda").to(dtype)
+
+    def run(other=False):
+        # the layer and its inverse: which of them has its result rows in column 1 depends on the direction
+        inverse = int(backward != other)
+        gpu_handle.set_kernel_timing(True)
+        if backward:
+            y = m.indice_conv_backward_data(gpu_handle, x, w, m.LAYOUT_ARRAY, pairs, counts, False, c, inverse=inverse,
+                                            rows=rows)
+        else:
+            y = m.indice_conv_forward(gpu_handle, x, w, m.LAYOUT_ARRAY, pairs, counts, rows, False, inverse=inverse)
+        torch.cuda.synchronize()
+        names = [n for n, _ in gpu_handle.kernel_timings()]
+        gpu_handle.set_kernel_timing(False)
+        return y, names
+    gpu_handle.set_extended_modes(True)
+    try:
+        ref, plain = run()
+        gpu_handle.promise_single_pairs(1)
+        got, names = run()
+        _, others = run(other=True)
+    finally:
+        gpu_handle.promise_single_pairs(None)
+        gpu_handle.set_extended_modes(False)
+    assert "gatherConvSingle" in names and "gatherConvSingle" not in plain + others, (names, plain, others)
+    want = torch.zeros((rows, c), dtype=torch.float64, device="cuda")
+    f = w[0, 0, 0].double().T if backward else w[0, 0, 0].double()
+    source = pairs[0, 0].long()
+    want[pairs[0, 1].long()] = x[source].double() @ f
+    size = torch.zeros_like(want)
+    size[pairs[0, 1].long()] = x[source].double().abs() @ f.abs()
+    rounding = {"float16": 2.0 ** -11, "bfloat16": 2.0 ** -8, "float32": 2.0 ** -24}[dtype_name]
+    bound = 2.0 ** -24 * q * size + rounding * want.abs() + 2.0 ** -25
+    assert ((got.double() - want).abs() <= bound).all() and ((ref.double() - want).abs() <= bound).all()
 
 
 def test_layers_promise_what_their_geometry_says():
