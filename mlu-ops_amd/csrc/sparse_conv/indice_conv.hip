@@ -2015,42 +2015,31 @@ __device__ __forceinline__ void storeDenseSlots(DenseMap &map, int slots, int32_
 // quarter) loads 16 bytes) and whole phases of two offsets are in flight; nothing is skipped: a group
 // without rows multiplies zeros.  A wave owns two row groups and ALL result columns.
 // Filter.  The waves share an offset's filter: its fragments travel from global memory into a
-// ring of two LDS buffers, a phase of one or two offsets at a time, and every wave reads all of
+// ring of two LDS buffers, a phase of two offsets at a time, and every wave reads all of
 // them from there, once per offset for both its row groups.  One barrier per phase hands a
 // buffer over; it waits for LDS traffic only, and each wave waits for its own requests itself
 // (__syncthreads() would make every wave wait for all loads in flight).
 // What bounds it is the loop itself (16 channels, 80 k rows, 27 offsets, half the slots filled: 37 us).  Rows through
 // LDS as below are no faster here (248 636 rows of a scene, with the filter's packing: 16 -> 16 38 us against 46,
 // 32 -> 32 47 against 47).
-struct DensePlan {
-  int per_cu;       // workgroups a CU
-  int offsets;      // offsets per phase
-};
-constexpr DensePlan densePlan(int C) {
-  const int nb = C / 16, groups = 2;
-  DensePlan p = {4, 2};
-  const int room = 160 * 1024 / 4 - kDenseChunk * kDenseRows * 4 - 1024;
-  if (groups * 4 * (nb + 2 * 2) + 4 * nb + 40 > 128) p.per_cu = 2;
-  if (p.per_cu == 4 && room < 4 * nb * 1024) p.per_cu = 2;
-  return p;
-}
+// Workgroups a CU: sums of two row groups and eight column blocks take the registers of two.
+constexpr int densePerCu(int C) { return C >= 128 ? 2 : 4; }
 
 template <typename E, int Q, int C, typename SRC>
 __global__ __launch_bounds__(kDenseThreads)
-    __attribute__((amdgpu_waves_per_eu(densePlan(C).per_cu, densePlan(C).per_cu)))
+    __attribute__((amdgpu_waves_per_eu(densePerCu(C), densePerCu(C))))
 void gatherConvDense(const typename E::storage *A, uint32_t a_size, ConvRows conv,
                      const typename E::storage *packedW, SRC source, int R, int K,
                      typename E::storage *result) {
   typedef typename E::vec8 vec8;
   typedef typename E::storage S;
-  constexpr DensePlan PLAN = densePlan(C);
   constexpr int WAVES = kDenseThreads / 64;
   constexpr int G = kDenseGroups / WAVES;
   constexpr int NB = C / 16;                 // 16-column blocks, all of them in every wave
   constexpr int KC = kDenseChunk;
   constexpr int FRAGS = NB;                  // 1 KiB filter fragments per offset
   constexpr int W_BYTES = FRAGS * 1024;
-  constexpr int OPP = PLAN.offsets;          // offsets per phase
+  constexpr int OPP = 2;                     // offsets per phase
   constexpr int BUF_FRAGS = OPP * FRAGS;
   constexpr int FPW = (BUF_FRAGS + WAVES - 1) / WAVES;
   static_assert(Q <= E::kChunk, "one fragment a row");
@@ -4074,12 +4063,18 @@ DenseSums useDenseKernel(const LaunchCtx &lc, const ConvProblem &p, const Gather
   //   fp16   16 -> 16                  0.18 (0.15: 24/26, 0.27: 31/26)       0.045 (0.04: 18/19, 0.05: 23/19)
   //          32 -> 32                  0.18 (0.15: 28/31, 0.27: 36/30)       0.045 (0.04: 20/21, 0.05: 27/20)
   //          16, 32 -> 64              0.14 (0.13: 39/41, 0.18: 47/41)       0.06  (0.05: 31/29, 0.10: 46/32)
-  // Rows of 2-byte types above 64 bytes, since they go through LDS, are ahead around 0.2 strewn and below 0.18 in thinned scenes;
-  // the lines stayed, so that no layer's sums changed, and below them each offset's product goes by itself (see below):
+  // Rows of 2-byte types above 64 bytes, since they go through LDS, are ahead around 0.2 strewn; the lines stayed, so that no
+  // layer's sums changed, and below them each offset's product goes by itself (see below):
   //          64 -> 64                  0.27 (0.26: 69/56, 0.31: 77/57)      0.085 (0.18: 50/46, 0.26: 74/54, 0.35: 121/72)
   //          64 -> 128                 0.27 (0.26: 102/87, 0.31: 118/81)    0.05  (0.18: 77/59, 0.26: 109/72, 0.35: 178/96)
   //          128 -> 64                 0.27 (0.26: 98/86, 0.31: 111/87)     0.085 (0.18: 70/70, 0.26: 109/80, 0.35: 187/110)
   //          128 -> 128                0.27 (0.26: 149/131, 0.31: 170/133)  0.05  (0.18: 108/92, 0.26: 159/115, 0.35: 258/160)
+  // The line of 64 result columns on scenes dates from pair-list kernels without tall tiles, which are ahead of this one
+  // up to 0.16 filled (64 -> 64) and 0.18 (128 -> 64): thinned scenes, us of those / this,
+  //   64 -> 64    5 k rows 0.09 20/26  0.14 23/27  0.18 27/27    20 k 0.12 22/27  0.17 28/27  0.24 33/27
+  //               45 k 0.08 25/30  0.15 33/30    100 k 0.09 25/30  0.12 37/34  0.145 41/45  0.18 51/45
+  //   128 -> 64   5 k 0.09 22/37  0.18 35/37  0.24 44/39    20 k 0.12 25/36  0.19 38/35    45 k 0.15 39/40  0.20 44/42
+  //               100 k 0.145 51/65  0.18 69/66  0.26 87/65
   //   fp32   16 -> 16, 32              0.3  (0.22: 46/54, 0.4: 66/54)        0.05  (0.04: 26/31, 0.07: 49/38)
   //          32 -> 32                  0.4  (0.31: 81/95, 0.5: 114/95)       0.065 (0.05: 46/57, 0.10: 95/72)
   //          32 -> 64                  0.5  (0.4: 138/160, 0.5: 160/159)     0.15  (0.11: 111/125, 0.17: 138/129)
@@ -4577,9 +4572,10 @@ void launchFilterMfmaInstance(const LaunchCtx &lc, const ConvProblem &p, const S
     if constexpr (kTransposingShape) {
       // fp32 takes steps of 32 pairs, 2-byte types of 64, half as many barriers; with 128 channels on a side those
       // leave two or three workgroups' buffers on a CU, and where a workgroup has many steps the shorter ones, with
-      // four, are faster (in walks: slices of 125 offsets, 1.6 M pairs, 128 x 128, 141/131).  us with the sums, fp16, steps of 32 / 64, 3.0 M pairs: 32 x 32 55/39   32 x 64 62/50
-      // 64 x 64 67/57   32 x 128 73/83   64 x 128 89/100   128 x 128 135/142; 0.98 M pairs: 32 x 32 28/23   64 x 64 35/31
-      // 64 x 128 43/41   128 x 128 67/59.  fp32, 0.98 M: 64 x 64 86/98   128 x 128 302/317
+      // four, are faster (in walks: slices of 125 offsets, 1.6 M pairs, 128 x 128, 141/131).  us with the sums, fp16,
+      // steps of 32 / 64:
+      //   3.0 M pairs   32 x 32 55/39   32 x 64 62/50   64 x 64 67/57   32 x 128 73/83   64 x 128 89/100   128 x 128 135/142
+      //   0.98 M pairs  32 x 32 28/23   64 x 64 35/31   64 x 128 43/41   128 x 128 67/59;  fp32  64 x 64 86/98   128 x 128 302/317
       auto tr = backwardFilterRows<E, CI, CO, 32, false>;
       if (whole) tr = backwardFilterRows<E, CI, CO, 32, true>;
       if constexpr (sizeof(S) == 2) {
