@@ -67,34 +67,43 @@ def test_on_another_stream():
 
 @pytest.mark.parametrize("asked_by", ["operator", "python"])
 @pytest.mark.parametrize("why", ["too many offsets", "no longer on file"])
-def test_counts_that_are_copied_wait_for_no_other_stream(asked_by, why):
+def test_counts_that_are_copied_wait_for_no_other_stream(monkeypatch, asked_by, why):
+    """(Streams share four hardware queues, and behind another stream's work in one of them everybody waits: so with several
+    streams in turn, and one that goes on behind the counts is enough.)"""
     import torch
+    import mluop_hip
     from mluop_hip import nn as spnn
+    monkeypatch.setattr(mluop_hip, "GUARD_BYTES", 0)  # (guards are checked after a wait for the device)
     idx = torch.from_numpy(random_voxels(np.random.default_rng(3), 1, SPACE, 500)).cuda()
-    x = spnn.SparseTensor(torch.randn(500, 8, device="cuda"), idx, SPACE, 1, distinct=True)
+    features = torch.randn(500, 8, device="cuda")
     size = 9 if why == "too many offsets" else 3  # (the handle keeps 343 counts of a rulebook)
     layer = spnn.SubMConv3d(8, 16, size).cuda()
+    a = torch.ones(4096, 4096, device="cuda")
     with torch.no_grad():
-        want = layer(spnn.SparseTensor(x.features, idx, SPACE, 1, distinct=True)).features
-        rb = pending(layer, x)
-        if why == "no longer on file":
-            for _ in range(40):
-                pending(spnn.SubMConv3d(8, 16, 3), spnn.SparseTensor(x.features, idx, SPACE, 1, distinct=True))
-        torch.cuda.synchronize()
-        a, busy = torch.ones(4096, 4096, device="cuda"), torch.cuda.Stream()
-        busy.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(busy):
-            for _ in range(200):  # about 1 ms each
-                b = a @ a
-            done = busy.record_event()
-        if asked_by == "operator":
-            got = layer(x).features
-        else:
-            assert rb.indice_num[size ** 3 // 2] == 500
-        assert not done.query(), "waited for a stream that has nothing to do with the rulebook"
-        assert asked_by == "python" or torch.equal(got, want)
-        torch.cuda.synchronize()
-        del b
+        want = layer(spnn.SparseTensor(features, idx, SPACE, 1, distinct=True)).features
+        for attempt in range(12):
+            x = spnn.SparseTensor(features, idx, SPACE, 1, distinct=True)
+            rb = pending(layer, x)
+            if why == "no longer on file":
+                for _ in range(40):
+                    pending(spnn.SubMConv3d(8, 16, 3), spnn.SparseTensor(features, idx, SPACE, 1, distinct=True))
+            torch.cuda.synchronize()
+            busy = torch.cuda.Stream()
+            with torch.cuda.stream(busy):
+                for _ in range(200):  # about 1 ms each
+                    a @ a
+                done = busy.record_event()
+            if asked_by == "operator":
+                got = layer(x).features
+            else:
+                assert rb.indice_num[size ** 3 // 2] == 500
+            went_on = not done.query()
+            torch.cuda.synchronize()
+            assert asked_by == "python" or torch.equal(got, want)
+            print("attempt", attempt, "the other stream is still busy:", went_on, flush=True)
+            if went_on:
+                return
+    raise AssertionError("waited for streams that have nothing to do with the rulebook")
 
 
 def test_counts_that_an_operator_took_are_not_asked_for_again():
