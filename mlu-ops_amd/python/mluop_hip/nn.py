@@ -213,6 +213,10 @@ class _ConvBase(torch.nn.Module):
             x.rulebooks[("planned", id(self))] = rb
         return rb
 
+    def _plain_rulebook(self):
+        """Whether `_rulebook` takes `wait_counts`: it is the library's, and not one put in its place."""
+        return getattr(self._rulebook, "__func__", None) in (_ConvBase._rulebook, SparseInverseConv3d._rulebook)
+
     def _cells_after(self, x, rb):
         """(indices, spatial shape, distinct) of this layer's result on `x`, from the rulebook alone."""
         if self.sub_m:
@@ -234,10 +238,8 @@ class _ConvBase(torch.nn.Module):
 
     def _convolve(self, x, **store):
         # (the counts are waited for in the operator, behind what the host has to do there: 60 000 rows, 48 -> 48
-        # channels 53 -> 48 us, a training step of 3001 rows 109 -> 99; a `_rulebook` put in the library's place is
-        # asked as it always was)
-        own = getattr(self._rulebook, "__func__", None) not in (_ConvBase._rulebook, SparseInverseConv3d._rulebook)
-        rb = self._rulebook(x) if own else self._rulebook(x, wait_counts=False)
+        # channels 53 -> 48 us, a training step of 3001 rows 109 -> 99)
+        rb = self._rulebook(x, wait_counts=False) if self._plain_rulebook() else self._rulebook(x)
         feats, weight = x.features, self.weight.to(x.features.dtype)
         feats = _IndiceConv.apply(feats, weight, rb, self.inverse, **store)
         if self.bias is not None:
@@ -347,7 +349,7 @@ class SparseSequential(torch.nn.Sequential):
                         rb.indice_num
                 cells = m.plan(cells) if own else m._plan(cells, built)
             elif isinstance(m, _ConvBase):
-                if type(m) in (SubMConv3d, SparseConv3d):
+                if type(m) in (SubMConv3d, SparseConv3d) and m._plain_rulebook():
                     rb = m._rulebook(cells, wait_counts=False)
                 else:
                     rb = m._rulebook(cells)

@@ -60,14 +60,16 @@ class Given(spnn.SubMConv3d):
 
 
 @pytest.mark.parametrize("how", ["class", "instance"])
-def test_a_layers_own_rulebook_is_asked_for(how, monkeypatch):
+@pytest.mark.parametrize("in_network", [False, True])
+def test_a_layers_own_rulebook_is_asked_for(how, in_network, monkeypatch):
     monkeypatch.setattr(spnn._IndiceConv, "apply", staticmethod(lambda features, weight, rb, *a, **k: features + rb))
     x = empty_tensor()
     x.rulebooks["given"] = 3.0
     layer = Given(16, 16, 3) if how == "class" else spnn.SubMConv3d(16, 16, 3)
     if how == "instance":
         layer._rulebook = lambda x: x.rulebooks["given"]
-    assert torch.equal(layer(x).features, x.features + 3.0)
+    net = spnn.SparseSequential(layer) if in_network else layer
+    assert torch.equal(net(x).features, x.features + 3.0)
 
 
 def empty_tensor():
