@@ -98,7 +98,7 @@ def with_and_without_a_wait(handle, idx, space, ks, stride, x, w):
 
         def call():
             a = busy
-            for _ in range(6):  # a few milliseconds in front of the rulebook
+            for _ in range(40):  # some 40 milliseconds in front of the rulebook
                 a = (a @ a) * 1e-4
             return m.indice_conv_forward(handle, x, w, m.LAYOUT_ARRAY, rulebook()[0], num, n_out, sub_m)
         got.append(kernels_of(handle, call))
